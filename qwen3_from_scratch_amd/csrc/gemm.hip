@@ -3,12 +3,11 @@
 #include "gates.h"
 
 // ---------------------------------------------------------------------------
-// float32: plain fused multiply-adds, no matrix-core mode of reduced precision.
-// A block of 256 threads computes a 64 x 64 tile of out; each thread a 4 x 4
-// patch, summing over k in ascending order, so an output element's value does
-// not depend on which rows share its batch. The same kernel with bfloat16
-// operands (read one by one, summed in float32) serves bfloat16 products of any
-// size that no matrix-core kernel takes: an inner size that is no multiple of 8.
+// Plain fused multiply-adds for any size: float32 products whose inner size is no multiple of 4 (or whose
+// operands lie at odd addresses), and bfloat16 ones of any size that no matrix-core kernel takes, an inner
+// size that is no multiple of 8 (read one by one, summed in float32). A block of 256 threads computes a
+// 64 x 64 tile of out; each thread a 4 x 4 patch, summing over k in ascending order, so an output element's
+// value does not depend on which rows share its batch.
 // ---------------------------------------------------------------------------
 #define F32_BM 64
 #define F32_BN 64
@@ -93,6 +92,139 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const IN* __restrict__ a,
 
 
 // ---------------------------------------------------------------------------
+// float32 on the matrix cores (v_mfma_f32_16x16x4_f32: float32 operands, products and sums, no mode of
+// reduced precision). Four wavefronts, two by two, share a tile of 32 WM x 32 WN of out; a wavefront has
+// WM x WN accumulators of 16 x 16. Stages of CHUNKS x 16 k pass through shared memory in two buffers; the
+// next stage (AHEAD 1) or two (AHEAD 2) are in registers or on their way there while one is multiplied.
+// Within a chunk lane group g holds k = 4 g .. 4 g + 3 as one 16-byte read and step s multiplies the four
+// k = 4 g + s: the order of a sum is the same for every tile size, row and column, so a value does not depend
+// on what stands beside it. A row's piece g sits at place g ^ (row / 4) % 4, so that the 16 rows that are read
+// together lie in all banks. The weight is the first operand: a lane then holds four neighbouring columns.
+//
+// Large products are bound by the matrix pipe (157 TFLOP/s nominal, 128 the vendor library's 4,096 cubed), small
+// ones by the wait for a stage, which is why the smallest tile takes 128 k at a time, two stages ahead (with one
+// stage of 32 k in flight 336 x 1,024 x 4,096 took 86 us instead of 53). Weights from memory, microseconds, the
+// multiply-adds above / this: 336 rows of 4,096 x 1,024, 1,024 x 2,048, 8,192 x 1,024 and 1,024 x 4,096 79 / 37,
+// 139 / 28, 109 / 71, 269 / 53; 20 rows 72 / 12, 140 / 20, 73 / 13, 272 / 36; 2,048 rows 242 / 146, 156 / 81,
+// 455 / 285 (121 TFLOP/s), 304 / 157. The error against 64 bits is the same.
+// ---------------------------------------------------------------------------
+typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+
+template <int WM, int WN, int CHUNKS, int AHEAD>
+__global__ __launch_bounds__(256) void gemm_f32_mma_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                           float* __restrict__ out, int M, int N, int K, int tiles_m,
+                                                           int tiles) {
+  constexpr int BM = 32 * WM, BN = 32 * WN;       // rows and columns of a block's tile
+  constexpr int BK = 16 * CHUNKS, PIECES = BK / 4;
+  constexpr int XT = BM * PIECES / 256, WT = BN * PIECES / 256;   // 16-byte pieces a thread moves per stage
+  __shared__ float4 sx[2][CHUNKS][BM * 4], sw[2][CHUNKS][BN * 4];   // [buffer][chunk of 16 k][row and place]
+  // a chiplet's blocks (every eighth) take neighbouring tiles, those of one weight tile together
+  const int share = (tiles + 7) / 8;
+  const int tile = ((int)blockIdx.x & 7) * share + ((int)blockIdx.x >> 3);
+  if (((int)blockIdx.x >> 3) >= share || tile >= tiles) return;
+  const int m0 = tile % tiles_m * BM, n0 = tile / tiles_m * BN;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int col = lane & 15, grp = lane >> 4;
+  const int wm = (wave & 1) * 16 * WM, wn = (wave >> 1) * 16 * WN;
+
+  float4 xv[AHEAD][XT], wv[AHEAD][WT];
+  auto load = [&](int set, int k0) {
+    const int k = k0 + 4 * (t % PIECES);
+#pragma unroll
+    for (int j = 0; j < XT; ++j) {
+      const int m = m0 + (t + 256 * j) / PIECES;
+      xv[set][j] = m < M && k < K ? *reinterpret_cast<const float4*>(x + (size_t)m * K + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+#pragma unroll
+    for (int j = 0; j < WT; ++j) {
+      const int n = n0 + (t + 256 * j) / PIECES;
+      wv[set][j] = n < N && k < K ? *reinterpret_cast<const float4*>(w + (size_t)n * K + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+  };
+  auto store = [&](int set, int buffer) {
+    const int piece = t % PIECES;
+#pragma unroll
+    for (int j = 0; j < XT; ++j) {
+      const int row = (t + 256 * j) / PIECES;
+      sx[buffer][piece >> 2][row * 4 + ((piece & 3) ^ ((row >> 2) & 3))] = xv[set][j];
+    }
+#pragma unroll
+    for (int j = 0; j < WT; ++j) {
+      const int row = (t + 256 * j) / PIECES;
+      sw[buffer][piece >> 2][row * 4 + ((piece & 3) ^ ((row >> 2) & 3))] = wv[set][j];
+    }
+  };
+  f32x4_t acc[WM][WN];
+#pragma unroll
+  for (int i = 0; i < WM; ++i)
+#pragma unroll
+    for (int j = 0; j < WN; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  const int stages = (K + BK - 1) / BK;
+  load(0, 0);
+  if (AHEAD == 2 && stages > 1) load(AHEAD - 1, BK);
+  store(0, 0);
+  __syncthreads();
+  for (int first = 0; first < stages; first += 2)
+#pragma unroll
+    for (int buffer = 0; buffer < 2; ++buffer) {
+      const int st = first + buffer;
+      if (st >= stages) break;
+      if (st + AHEAD < stages) load(AHEAD == 2 ? buffer : 0, (st + AHEAD) * BK);
+#pragma unroll
+      for (int c = 0; c < CHUNKS; ++c) {
+        f32x4_t xr[WM], wr[WN];
+#pragma unroll
+        for (int i = 0; i < WM; ++i) {
+          const int row = wm + 16 * i + col;
+          xr[i] = *reinterpret_cast<const f32x4_t*>(&sx[buffer][c][row * 4 + (grp ^ ((row >> 2) & 3))]);
+        }
+#pragma unroll
+        for (int j = 0; j < WN; ++j) {
+          const int row = wn + 16 * j + col;
+          wr[j] = *reinterpret_cast<const f32x4_t*>(&sw[buffer][c][row * 4 + (grp ^ ((row >> 2) & 3))]);
+        }
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+          for (int i = 0; i < WM; ++i)
+#pragma unroll
+            for (int j = 0; j < WN; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wr[j][s], xr[i][s], acc[i][j], 0, 0, 0);
+      }
+      // (the other buffer's readers have passed the barrier before this stage)
+      if (st + 1 < stages) store(AHEAD == 2 ? buffer ^ 1 : 0, buffer ^ 1);
+      __syncthreads();
+    }
+#pragma unroll
+  for (int i = 0; i < WM; ++i) {
+    const int m = m0 + wm + 16 * i + col;
+    if (m >= M) continue;
+#pragma unroll
+    for (int j = 0; j < WN; ++j) {
+      const int n = n0 + wn + 16 * j + 4 * grp;
+      float* o = out + (size_t)m * N + n;
+      if (N % 4 == 0) {
+        if (n < N) *reinterpret_cast<f32x4_t*>(o) = acc[i][j];
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < N) o[e] = acc[i][j][e];
+      }
+    }
+  }
+}
+
+template <int WM, int WN, int CHUNKS, int AHEAD>
+static int launch_f32_mma(const void* x, const void* w, void* out, int M, int N, int K, hipStream_t stream) {
+  const long tiles_m = (M + 32 * WM - 1) / (32 * WM), tiles = tiles_m * ((N + 32 * WN - 1) / (32 * WN));
+  if (tiles > (1l << 30)) return Q3_ERR_UNSUPPORTED;
+  hipLaunchKernelGGL((gemm_f32_mma_kernel<WM, WN, CHUNKS, AHEAD>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(256), 0, stream,
+                     (const float*)x, (const float*)w, (float*)out, M, N, K, (int)tiles_m, (int)tiles);
+  return q3_launch_status();
+}
+
+// ---------------------------------------------------------------------------
 // bfloat16 with at most 16 rows (and, for small weights, a few groups of 16 rows, each a set of
 // blocks of its own: q3_linear_tiled): a weight-streaming kernel. Every weight is
 // read once from HBM and that read is the cost; the matrix cores do the sums
@@ -114,7 +246,6 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const IN* __restrict__ a,
 // outputs are two (gate, up) pairs.
 // ---------------------------------------------------------------------------
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
-typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 
 union Pack16 {
   uint4 u;
@@ -599,6 +730,17 @@ extern "C" int q3_linear(const void* x, const void* weight, void* out, int M, in
         hipLaunchKernelGGL(gemm_f32_few_rows_kernel<16>, few, dim3(256), 0, stream, (const float*)x,
                            (const float*)weight, (float*)out, M, N, K);
       return q3_launch_status();
+    }
+    if (K % 4 == 0 && (((size_t)x | (size_t)weight | (size_t)out) & 15) == 0) {
+      // The largest tile that gives every CU two blocks (of 32 x 64, one and a half): 1,024 x 8,192 x 1,024 (512 tiles
+      // of 128 x 128) takes 146 us in these, 168 in 64 x 64; 600 rows (320 tiles) 142 and 111. 450 x 4,096 x 1,024
+      // (512 tiles of 64 x 64) 44 in these, 50 in 32 x 64; 336 rows (384) 43 and 37. 201 rows of it (448 tiles of
+      // 32 x 64) 27 in these, 31 in 32 x 32; 128 rows (256) 19 and 17.
+      const long m32 = (M + 31) / 32, n32 = (N + 31) / 32;
+      if ((m32 + 3) / 4 * ((n32 + 3) / 4) >= 512) return launch_f32_mma<4, 4, 2, 1>(x, weight, out, M, N, K, stream);
+      if ((m32 + 1) / 2 * ((n32 + 1) / 2) >= 512) return launch_f32_mma<2, 2, 4, 1>(x, weight, out, M, N, K, stream);
+      if (m32 * ((n32 + 1) / 2) >= 384) return launch_f32_mma<1, 2, 4, 1>(x, weight, out, M, N, K, stream);
+      return launch_f32_mma<1, 1, 8, 2>(x, weight, out, M, N, K, stream);
     }
     const dim3 grid((N + F32_BN - 1) / F32_BN, (M + F32_BM - 1) / F32_BM);
     if (grid.y > 65535) return Q3_ERR_UNSUPPORTED;
