@@ -151,6 +151,172 @@ static int launch_general(const void* q, int q_stride, void* out, const void* k_
   return q3_launch_status();
 }
 
+#if !defined(Q3_SCORE_CAP) && !defined(Q3_POOLED) && !defined(Q3_SIGMOID) && !defined(Q3_SPAN)
+#define Q3_F32_MMA 1
+// ---------------------------------------------------------------------------
+// float32 on the matrix cores (v_mfma_f32_16x16x4_f32, float32 throughout as in the kernel above), for pages of a
+// multiple of 16 and at most 16 query heads a key head. A block of eight wavefronts serves 16 rows, a
+// (token, query head of the group) pair each, so that a group's heads share every key; wavefront w
+// walks the 16-key tiles t with t % 8 = w, counted from the sequence's first key, with maximum, sum and result
+// of its own, and the eight are joined in a fixed order: a row's sums depend neither on how the sequence was cut
+// into steps nor on the rows beside it.
+//
+//   S^T (keys x rows) = K . Q^T, O^T (d x rows) += V^T . P^T: the row is the lane's low four bits in both.
+//
+// Lane group g holds d = 16 c + 4 g .. + 3 of its key and of its row as one 16-byte load each and step s multiplies
+// the four d = 16 c + 4 g + s; it then has the scores of keys 4 g .. 4 g + 3, which the values' 16-byte loads (the
+// cache is transposed within the page) match in the same way. Nothing passes through shared memory but the
+// eight results at the end.
+//
+// Bound by the wait for keys and values from the L2 and by the chain from scores to probabilities; the kernel
+// above, 16 rows of one head a block, read two numbers from shared memory per multiply-add. Two prompts of 111 and
+// 222 tokens beside three single tokens behind up to 150, 16 heads over 8 of 128: 177 us there, 22 here.
+// ---------------------------------------------------------------------------
+typedef __attribute__((ext_vector_type(4))) float f32_four;
+
+__device__ __forceinline__ f32_four load_four(const float* p) { return *reinterpret_cast<const f32_four*>(p); }
+
+template <int D>
+__global__ __launch_bounds__(512) void attn_f32_mma_kernel(
+    const float* __restrict__ q, int q_stride, float* __restrict__ out, const float* __restrict__ k_cache,
+    const float* __restrict__ v_cache, int num_pages, const int* __restrict__ block_table, int bt_stride,
+    const int* __restrict__ cu_q, const int* __restrict__ kv_lens, int Hq, int Hkv, int page, float scale, int window,
+    const float* __restrict__ sink, int tokens_per_block) {
+  constexpr int C = D / 16, LD = D + 4;
+  __shared__ float part[4][16][LD], sh_m[8][16], sh_l[8][16];
+  const int b = blockIdx.z, g_kv = blockIdx.y, G = Hq / Hkv;
+  const int q0 = cu_q[b], q_len = cu_q[b + 1] - q0;
+  const int t0 = blockIdx.x * tokens_per_block;
+  if (t0 >= q_len) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int col = lane & 15, grp = lane >> 4;
+  const int first_pos = kv_lens[b] - q_len;
+  const int tokens = min(tokens_per_block, q_len - t0), rows = tokens * G;
+  const bool my_row = col < rows;
+  const int my_pos = my_row ? first_pos + t0 + col / G : -1;
+
+  f32_four qr[C], acc[C];
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    qr[c] = f32_four{0.f, 0.f, 0.f, 0.f};
+    acc[c] = f32_four{0.f, 0.f, 0.f, 0.f};
+    if (my_row)
+      qr[c] = load_four(q + (size_t)(q0 + t0 + col / G) * q_stride + (size_t)(g_kv * G + col % G) * D + 16 * c + 4 * grp);
+  }
+  float m_run = -INFINITY, l_run = 0.f;
+
+  const int k_end = first_pos + t0 + tokens;      // one past the last key any row sees
+  const int begin = window > 0 ? max(0, first_pos + t0 - window + 1) / 16 : 0;
+  const int end = (k_end + 15) / 16;
+  for (int tile = begin + ((wave - begin) & 7); tile < end; tile += 8) {
+    const int key0 = 16 * tile;
+    const int pg = block_table[(size_t)b * bt_stride + key0 / page];
+    const bool there = pg >= 0 && pg < num_pages;   // (a page given back counts as zeros; nobody sees it)
+    const size_t base = ((size_t)(there ? pg : 0) * Hkv + g_kv) * page * D;
+    const float* kp = k_cache + base + (size_t)(key0 % page + col) * D + 4 * grp;
+    const float* vp = v_cache + base + (size_t)col * page + key0 % page + 4 * grp;
+    f32_four kr[C], vr[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) kr[c] = there ? load_four(kp + 16 * c) : f32_four{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < C; ++c) vr[c] = there ? load_four(vp + (size_t)16 * c * page) : f32_four{0.f, 0.f, 0.f, 0.f};
+    f32_four s4 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s4 = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[c][i], qr[c][i], s4, 0, 0, 0);
+    const int my_key = key0 + 4 * grp;
+    if (key0 + 16 > k_end) {                        // what lies behind the sequence's end may be anything
+#pragma unroll
+      for (int c = 0; c < C; ++c)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (my_key + i >= k_end) vr[c][i] = 0.f;
+    }
+    float sc[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const bool seen = my_key + i <= my_pos && !(window > 0 && my_pos - (my_key + i) >= window);
+      sc[i] = seen ? s4[i] * scale : -INFINITY;
+    }
+    const float m_new = fmaxf(m_run, quad_rows_max(fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]))));
+    float alpha = 1.f, p[4] = {0.f, 0.f, 0.f, 0.f};
+    if (m_new > -INFINITY) {
+      alpha = expf(m_run - m_new);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) p[i] = expf(sc[i] - m_new);
+    }
+    l_run = l_run * alpha + ((p[0] + p[1]) + (p[2] + p[3]));
+    m_run = m_new;
+#pragma unroll
+    for (int c = 0; c < C; ++c) acc[c] *= alpha;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int c = 0; c < C; ++c) acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(vr[c][i], p[i], acc[c], 0, 0, 0);
+  }
+
+  // the eight results are joined: every wavefront brings its own to the common maximum, four are added to
+  // the other four, and the four sums in their order
+  l_run = quad_rows_sum(l_run);
+  if (grp == 0) {
+    sh_m[wave][col] = m_run;
+    sh_l[wave][col] = l_run;
+  }
+  __syncthreads();
+  float top = sh_m[0][col];
+#pragma unroll
+  for (int w = 1; w < 8; ++w) top = fmaxf(top, sh_m[w][col]);
+  const float factor = m_run > -INFINITY ? expf(m_run - top) : 0.f;
+#pragma unroll
+  for (int half = 1; half >= 0; --half) {
+    if ((wave >> 2) == half) {
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        f32_four* place = reinterpret_cast<f32_four*>(&part[wave & 3][col][16 * c + 4 * grp]);
+        const f32_four mine = acc[c] * factor;
+        *place = half ? mine : *place + mine;
+      }
+    }
+    __syncthreads();
+  }
+  for (int idx = tid; idx < rows * C * 4; idx += 512) {
+    const int r = idx / (C * 4), d = idx % (C * 4) * 4;
+    const int head = g_kv * G + r % G;
+    float m = sh_m[0][r];
+#pragma unroll
+    for (int w = 1; w < 8; ++w) m = fmaxf(m, sh_m[w][r]);
+    float total = 0.f;
+#pragma unroll
+    for (int w = 0; w < 8; ++w) total += sh_m[w][r] > -INFINITY ? sh_l[w][r] * expf(sh_m[w][r] - m) : 0.f;
+    if (sink) total += expf(sink[head] - m);
+    const f32_four sum = (load_four(&part[0][r][d]) + load_four(&part[1][r][d])) +
+                         (load_four(&part[2][r][d]) + load_four(&part[3][r][d]));
+    *reinterpret_cast<f32_four*>(out + (size_t)(q0 + t0 + r / G) * ((size_t)Hq * D) + (size_t)head * D + d) = sum * (1.f / total);
+  }
+}
+
+// Whether that kernel takes a call.
+static bool f32_mma_takes(const void* q, int q_stride, const void* out, const void* k_cache, const void* v_cache, int Hq,
+                          int Hkv, int D, int page) {
+  return (D == 16 || D == 32 || D == 64 || D == 128) && page % 16 == 0 && Hq / Hkv <= 16 && Hkv <= 65535 &&
+         q_stride % 4 == 0 && (((size_t)q | (size_t)out | (size_t)k_cache | (size_t)v_cache) & 15) == 0;
+}
+
+template <int D>
+static int launch_f32_mma(const void* q, int q_stride, void* out, const void* k_cache, const void* v_cache, int num_pages,
+                          const int* block_table, int bt_stride, const int* cu_q, const int* kv_lens, int B, int Hq,
+                          int Hkv, int page, float scale, int window, int max_q_len, const float* sink,
+                          hipStream_t stream) {
+  const int tokens_per_block = 16 / (Hq / Hkv);
+  const dim3 grid((max_q_len + tokens_per_block - 1) / tokens_per_block, Hkv, B);
+  hipLaunchKernelGGL(attn_f32_mma_kernel<D>, grid, dim3(512), 0, stream, (const float*)q, q_stride, (float*)out,
+                     (const float*)k_cache, (const float*)v_cache, num_pages, block_table, bt_stride, cu_q, kv_lens, Hq, Hkv,
+                     page, scale, window, sink, tokens_per_block);
+  return q3_launch_status();
+}
+#endif
+
 
 // ---------------------------------------------------------------------------
 // The matrix-core kernels: bfloat16, head size 64 or 128, page size a multiple
@@ -2112,6 +2278,19 @@ extern "C" int q3_paged_attention(const void* q, int q_stride, void* out, const 
   }
 #if defined(Q3_SCORE_CAP) || defined(Q3_POOLED) || defined(Q3_SIGMOID)
   return Q3_ERR_UNSUPPORTED;      // these builds have the matrix-core kernels only
+#endif
+#ifdef Q3_F32_MMA
+  if (dtype == Q3_F32 && f32_mma_takes(q, q_stride, out, k_cache, v_cache, Hq, Hkv, D, page)) {
+#define Q3_F32_MMA_LAUNCH(DD)                                                                                           \
+  if (D == DD)                                                                                                          \
+  return launch_f32_mma<DD>(q, q_stride, out, k_cache, v_cache, num_pages, block_table, bt_stride, cu_q, kv_lens, B, Hq, \
+                            Hkv, page, scale, window, max_q_len, sink, stream)
+    Q3_F32_MMA_LAUNCH(16);
+    Q3_F32_MMA_LAUNCH(32);
+    Q3_F32_MMA_LAUNCH(64);
+    Q3_F32_MMA_LAUNCH(128);
+#undef Q3_F32_MMA_LAUNCH
+  }
 #endif
   Q3_DISPATCH_DTYPE(dtype, TT, return launch_general<TT>(q, q_stride, out, k_cache, v_cache, num_pages,
                                                         block_table, bt_stride, cu_q, kv_lens, B, Hq, Hkv,
