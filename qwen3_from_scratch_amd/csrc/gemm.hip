@@ -96,17 +96,18 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const IN* __restrict__ a,
 // reduced precision). Four wavefronts, two by two, share a tile of 32 WM x 32 WN of out; a wavefront has
 // WM x WN accumulators of 16 x 16. Stages of CHUNKS x 16 k pass through shared memory in two buffers; the
 // next stage (AHEAD 1) or two (AHEAD 2) are in registers or on their way there while one is multiplied.
-// Within a chunk lane group g holds k = 4 g .. 4 g + 3 as one 16-byte read and step s multiplies the four
-// k = 4 g + s: the order of a sum is the same for every tile size, row and column, so a value does not depend
-// on what stands beside it. A row's piece g sits at place g ^ (row / 4) % 4, so that the 16 rows that are read
-// together lie in all banks. The weight is the first operand: a lane then holds four neighbouring columns.
+// Step s of a chunk multiplies k = 4 s + g, g the lane group, and the instruction adds its four products one after the
+// other: every sum runs over k in ascending order, as in the kernel above and with its bits, so a value does not depend
+// on the tile or on what stands beside it. A lane group's four numbers of a row are one piece, read in 16 bytes (and
+// written one by one); piece g sits at place g ^ (row / 4) % 4, so that the 16 rows that are read together lie in all
+// banks. The weight is the first operand: a lane then holds four neighbouring columns.
 //
 // Large products are bound by the matrix pipe (157 TFLOP/s nominal, 128 the vendor library's 4,096 cubed), small
 // ones by the wait for a stage, which is why the smallest tile takes 128 k at a time, two stages ahead (with one
 // stage of 32 k in flight 336 x 1,024 x 4,096 took 86 us instead of 53). Weights from memory, microseconds, the
-// multiply-adds above / this: 336 rows of 4,096 x 1,024, 1,024 x 2,048, 8,192 x 1,024 and 1,024 x 4,096 79 / 37,
-// 139 / 28, 109 / 71, 269 / 53; 20 rows 72 / 12, 140 / 20, 73 / 13, 272 / 36; 2,048 rows 242 / 146, 156 / 81,
-// 455 / 285 (121 TFLOP/s), 304 / 157. The error against 64 bits is the same.
+// multiply-adds above / this: 336 rows of 4,096 x 1,024, 1,024 x 2,048, 8,192 x 1,024 and 1,024 x 4,096 78 / 36,
+// 139 / 28, 109 / 71, 269 / 54; 20 rows 72 / 12, 140 / 20, 73 / 13, 272 / 37; 2,048 rows 243 / 154, 154 / 80,
+// 459 / 303 (113 TFLOP/s), 307 / 155.
 // ---------------------------------------------------------------------------
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 
@@ -117,7 +118,8 @@ __global__ __launch_bounds__(256) void gemm_f32_mma_kernel(const float* __restri
   constexpr int BM = 32 * WM, BN = 32 * WN;       // rows and columns of a block's tile
   constexpr int BK = 16 * CHUNKS, PIECES = BK / 4;
   constexpr int XT = BM * PIECES / 256, WT = BN * PIECES / 256;   // 16-byte pieces a thread moves per stage
-  __shared__ float4 sx[2][CHUNKS][BM * 4], sw[2][CHUNKS][BN * 4];   // [buffer][chunk of 16 k][row and place]
+  // [buffer][chunk of 16 k][row and place]; the place more shifts the chunks' numbers of one row into different banks
+  __shared__ float4 sx[2][CHUNKS][BM * 4 + 1], sw[2][CHUNKS][BN * 4 + 1];
   // a chiplet's blocks (every eighth) take neighbouring tiles, those of one weight tile together
   const int share = (tiles + 7) / 8;
   const int tile = ((int)blockIdx.x & 7) * share + ((int)blockIdx.x >> 3);
@@ -141,18 +143,20 @@ __global__ __launch_bounds__(256) void gemm_f32_mma_kernel(const float* __restri
       wv[set][j] = n < N && k < K ? *reinterpret_cast<const float4*>(w + (size_t)n * K + k) : make_float4(0.f, 0.f, 0.f, 0.f);
     }
   };
+  auto scatter = [&](float4* rows, int row, int q, const float4& v) {   // k = 4 q .. 4 q + 3 of a chunk: number q of four pieces
+    float* p = reinterpret_cast<float*>(rows + row * 4) + q;
+    const int turn = (row >> 2) & 3;
+    p[4 * (0 ^ turn)] = v.x;
+    p[4 * (1 ^ turn)] = v.y;
+    p[4 * (2 ^ turn)] = v.z;
+    p[4 * (3 ^ turn)] = v.w;
+  };
   auto store = [&](int set, int buffer) {
     const int piece = t % PIECES;
 #pragma unroll
-    for (int j = 0; j < XT; ++j) {
-      const int row = (t + 256 * j) / PIECES;
-      sx[buffer][piece >> 2][row * 4 + ((piece & 3) ^ ((row >> 2) & 3))] = xv[set][j];
-    }
+    for (int j = 0; j < XT; ++j) scatter(sx[buffer][piece >> 2], (t + 256 * j) / PIECES, piece & 3, xv[set][j]);
 #pragma unroll
-    for (int j = 0; j < WT; ++j) {
-      const int row = (t + 256 * j) / PIECES;
-      sw[buffer][piece >> 2][row * 4 + ((piece & 3) ^ ((row >> 2) & 3))] = wv[set][j];
-    }
+    for (int j = 0; j < WT; ++j) scatter(sw[buffer][piece >> 2], (t + 256 * j) / PIECES, piece & 3, wv[set][j]);
   };
   f32x4_t acc[WM][WN];
 #pragma unroll
@@ -732,12 +736,12 @@ extern "C" int q3_linear(const void* x, const void* weight, void* out, int M, in
       return q3_launch_status();
     }
     if (K % 4 == 0 && (((size_t)x | (size_t)weight | (size_t)out) & 15) == 0) {
-      // The largest tile that gives every CU two blocks (of 32 x 64, one and a half): 1,024 x 8,192 x 1,024 (512 tiles
-      // of 128 x 128) takes 146 us in these, 168 in 64 x 64; 600 rows (320 tiles) 142 and 111. 450 x 4,096 x 1,024
-      // (512 tiles of 64 x 64) 44 in these, 50 in 32 x 64; 336 rows (384) 43 and 37. 201 rows of it (448 tiles of
-      // 32 x 64) 27 in these, 31 in 32 x 32; 128 rows (256) 19 and 17.
+      // The largest tile that leaves every CU two blocks at a time (64 x 128: two rounds of them; 32 x 64: one and a
+      // half blocks): 2,048 x 8,192 x 1,024 (2,048 tiles of 64 x 128) takes 303 us in these, 320 in 64 x 64; 600 rows of
+      // it (640) 125 and 110. 450 x 4,096 x 1,024 (512 tiles of 64 x 64) 43 in these, 50 in 32 x 64; 336 rows (384) 41 and
+      // 36. 201 rows of it (448 tiles of 32 x 64) 26 in these, 30 in 32 x 32; 128 rows (256) 19 and 17.
       const long m32 = (M + 31) / 32, n32 = (N + 31) / 32;
-      if ((m32 + 3) / 4 * ((n32 + 3) / 4) >= 512) return launch_f32_mma<4, 4, 2, 1>(x, weight, out, M, N, K, stream);
+      if ((m32 + 1) / 2 * ((n32 + 3) / 4) >= 1024) return launch_f32_mma<2, 4, 2, 1>(x, weight, out, M, N, K, stream);
       if ((m32 + 1) / 2 * ((n32 + 1) / 2) >= 512) return launch_f32_mma<2, 2, 4, 1>(x, weight, out, M, N, K, stream);
       if (m32 * ((n32 + 1) / 2) >= 384) return launch_f32_mma<1, 2, 4, 1>(x, weight, out, M, N, K, stream);
       return launch_f32_mma<1, 1, 8, 2>(x, weight, out, M, N, K, stream);

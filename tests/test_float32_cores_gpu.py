@@ -9,7 +9,7 @@ from test_kernels_gpu import _ops, _paged_case, _rand
 pytestmark = pytest.mark.gpu
 
 
-# every tile size of the dispatch (32 x 32, 32 x 64, 64 x 64, 128 x 128), rows and columns that end inside a tile, inner
+# every tile size of the dispatch (32 x 32, 32 x 64, 64 x 64, 64 x 128), rows and columns that end inside a tile, inner
 # sizes shorter than a stage, that end inside one, and of every number of stages from one to four
 @pytest.mark.parametrize("M,N,K", [(17, 1, 4), (31, 33, 20), (32, 64, 128), (33, 130, 132), (100, 1027, 260), (70, 6150, 64),
                                    (129, 6146, 68), (500, 4098, 100), (1030, 8130, 36), (2050, 4100, 388)])
@@ -21,7 +21,11 @@ def test_linear_float32_many_rows(M, N, K):
     # a chain of K additions: at most K roundings of half a unit in the last place of the sum of the magnitudes
     bound = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
     assert bool(((got.double() - want).abs() <= bound).all())
-    # a row's values do not depend on its neighbours, nor on the tile size that their number picks
+    # a row's values do not depend on its neighbours, nor on the tile size that their number picks; and the sums run in
+    # the order of the kernel for odd addresses, with the same bits
+    flat = torch.empty(M * K + 1, device="cuda")
+    flat[1:] = x.view(-1)
+    assert torch.equal(ops.linear(flat[1:].view(M, K), w), got)
     for part in (x[:17], x[M - 17:], x[:max(17, M // 3)]):
         first = part.storage_offset() // K
         assert torch.equal(ops.linear(part.contiguous(), w), got[first:first + part.shape[0]])
