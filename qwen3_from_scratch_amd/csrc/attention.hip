@@ -525,7 +525,7 @@ __device__ __forceinline__ Pack16 softmax_step(const f32x4_t (&s)[2], bool full,
   if (!full) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const int key = key0 + 16 * (j >> 2) + 4 * grp + (j & 3);
+      const int key = key0 + 8 * grp + j;      // see TileAddr
       bool seen = key <= row_pos;
       if (span_hides(window, row_pos, key)) seen = false;
       if (!seen) v[j] = -INFINITY;
@@ -565,41 +565,9 @@ __device__ __forceinline__ Pack16 softmax_step(const f32x4_t (&s)[2], bool full,
 #endif
 }
 
-// Where the two 16-key blocks of the tile that starts at key0 lie in the caches
-// (nullptr for a block past the sequence's end or in a page given back), from
-// this lane's point of view: its K row and its V^T row.
-struct TileAddr {
-  const bf16_t* k[2];
-  const bf16_t* v[2];
-};
-
-__device__ __forceinline__ TileAddr tile_addr(const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
-                                              int num_pages, const int* __restrict__ bt_row, int Hkv, int g_kv,
-                                              int page, int D, int DV, int key0, int kv_len) {
-  const int lane = threadIdx.x & 63;
-  const int col = lane & 15, grp = lane >> 4;
-  TileAddr t;
-#pragma unroll
-  for (int kb = 0; kb < 2; ++kb) {
-    const int kbase = key0 + 16 * kb;
-    t.k[kb] = nullptr;
-    t.v[kb] = nullptr;
-    if (kbase < kv_len) {
-      const int pg = bt_row[kbase / page];
-      if (pg >= 0 && pg < num_pages) {
-        const int slot0 = kbase % page;
-        t.k[kb] = k_cache + (((size_t)pg * Hkv + g_kv) * page + slot0 + col) * D + 8 * grp;
-        t.v[kb] = v_cache + (((size_t)pg * Hkv + g_kv) * DV + col) * page + slot0 + 4 * grp;
-      }
-    }
-  }
-  return t;
-}
-
-// The same in two halves, for a block that does not have the sequence's length in hand yet:
-// the table entries of a tile's two blocks of 16 keys (-1 where the table has none: entries past
-// a sequence's pages are -1), and the addresses from them. Keys past the sequence's end inside
-// its last page hold anything; the caller masks them.
+// The block-table entries of the two halves (16 keys each) of the tile that starts at key0: -1 where the table
+// has none (entries past a sequence's pages are -1) and for a page given back. The same in all lanes of a
+// wavefront, whose tile it is: they are read and multiplied as scalars.
 struct TilePages {
   int pg[2];
 };
@@ -607,73 +575,92 @@ struct TilePages {
 __device__ __forceinline__ TilePages tile_pages(const int* __restrict__ bt_row, int bt_stride, int page, int key0) {
   TilePages p;
 #pragma unroll
-  for (int kb = 0; kb < 2; ++kb) {
-    const int entry = (key0 + 16 * kb) / page;
-    p.pg[kb] = entry < bt_stride ? bt_row[entry] : -1;
+  for (int h = 0; h < 2; ++h) {
+    const int entry = (key0 + 16 * h) / page;
+    p.pg[h] = entry < bt_stride ? bt_row[entry] : -1;
   }
   return p;
 }
 
-__device__ __forceinline__ TileAddr tile_addr_of(const TilePages& p, const bf16_t* __restrict__ k_cache,
-                                                 const bf16_t* __restrict__ v_cache, int num_pages, int Hkv, int g_kv,
-                                                 int page, int D, int DV, int key0) {
+// Where a lane's pieces of a tile begin. The tile's 32 keys go over the rows of the two score products so that a
+// lane, whose scores are rows 4 g .. 4 g + 3 of either, gets eight neighbouring keys, 8 g .. 8 g + 7: row m of product
+// kb is key 8 (m / 4) + 4 kb + m % 4. The values of those keys are then one 16-byte load per 16 columns. A half
+// that is not there points at the cache's first page, so that no load waits behind a branch (with the loads
+// guarded one by one, the compiler waited for each before it asked for the next: 4,000 of the 17,000 cycles a
+// block took for one request over 1,100 keys), and `there` says whose loads count.
+struct TileAddr {
+  const bf16_t* k;   // the lane's key row of product 0, from element 8 g on; product 1's is four keys on
+  const bf16_t* v;   // the lane's first value row, from key 8 g on; its others are 16 rows apart
+  int there;         // a bit per half
+};
+
+__device__ __forceinline__ TileAddr tile_addr(const TilePages& p, const bf16_t* __restrict__ k_cache,
+                                              const bf16_t* __restrict__ v_cache, int num_pages, int Hkv, int g_kv,
+                                              int page, int D, int DV, int key0) {
   const int lane = threadIdx.x & 63;
   const int col = lane & 15, grp = lane >> 4;
+  size_t kh[2], vh[2];
   TileAddr t;
+  t.there = 0;
 #pragma unroll
-  for (int kb = 0; kb < 2; ++kb) {
-    t.k[kb] = nullptr;
-    t.v[kb] = nullptr;
-    const int pg = p.pg[kb];
-    if (pg >= 0 && pg < num_pages) {
-      const int slot0 = (key0 + 16 * kb) % page;
-      t.k[kb] = k_cache + (((size_t)pg * Hkv + g_kv) * page + slot0 + col) * D + 8 * grp;
-      t.v[kb] = v_cache + (((size_t)pg * Hkv + g_kv) * DV + col) * page + slot0 + 4 * grp;
-    }
+  for (int h = 0; h < 2; ++h) {
+    const bool there = p.pg[h] >= 0 && p.pg[h] < num_pages;
+    const size_t head = (size_t)(there ? p.pg[h] : 0) * Hkv + g_kv;
+    const int slot0 = (key0 + 16 * h) & (page - 1);
+    kh[h] = (head * page + slot0) * D;
+    vh[h] = head * DV * page + slot0;
+    t.there |= there ? 1 << h : 0;
   }
+  t.k = k_cache + (col >> 3 ? kh[1] : kh[0]) + (unsigned)((8 * ((col >> 2) & 1) + (col & 3)) * D + 8 * grp);
+  t.v = v_cache + (grp >> 1 ? vh[1] : vh[0]) + (unsigned)(col * page + 8 * (grp & 1));
   return t;
 }
 
-// The K operands of a tile: [key block][d step].
-template <int D>
-__device__ __forceinline__ void load_keys(Pack16 (&a)[2][D / 32], const TileAddr& t) {
+// A tile's operands in a wavefront's registers: keys [product][d step], values per 16 output columns.
+template <int D, int DV>
+struct TileRegs {
+  Pack16 k[2][D / 32];
+  Pack16 v[DV / 16];
+  TileAddr at;
+};
+
+template <int D, int DV>
+__device__ __forceinline__ void load_keys(TileRegs<D, DV>& r, const TileAddr& t) {
+  r.at = t;
 #pragma unroll
   for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-    for (int i = 0; i < D / 32; ++i) {
-      if (t.k[kb])
-        a[kb][i].u = *reinterpret_cast<const uint4*>(t.k[kb] + 32 * i);
-      else
-        a[kb][i].u = make_uint4(0, 0, 0, 0);
-    }
+    for (int i = 0; i < D / 32; ++i) r.k[kb][i].u = *reinterpret_cast<const uint4*>(t.k + 4 * D * kb + 32 * i);
+}
+
+template <int D, int DV>
+__device__ __forceinline__ void load_values(TileRegs<D, DV>& r, int page) {
+#pragma unroll
+  for (int nb = 0; nb < DV / 16; ++nb) r.v[nb].u = *reinterpret_cast<const uint4*>(r.at.v + (size_t)(16 * nb) * page);
 }
 
 // Scores, softmax update and value accumulation of one 32-key tile for QB
-// blocks of 16 rows, with the tile's K operands already in registers. row_pos[qb]:
+// blocks of 16 rows, with the tile's operands in registers. row_pos[qb]:
 // position of this lane's row, below zero for a row that does not exist. m, l:
-// running maximum (log2 domain) and this lane's share of the running sum. The
-// value loads are issued first and meet the probabilities after the softmax.
-// The V^T operands of a tile, one per block of 16 output columns.
-template <int D>
-__device__ __forceinline__ void load_values(Pack16 (&vt)[D / 16], const TileAddr& t, int page) {
-#pragma unroll
-  for (int nb = 0; nb < D / 16; ++nb)
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
-      if (t.v[kb])
-        vt[nb].h[kb] = *reinterpret_cast<const uint2*>(t.v[kb] + (size_t)16 * nb * page);
-      else
-        vt[nb].h[kb] = make_uint2(0, 0);
-    }
-}
-
+// running maximum (log2 domain) and this lane's share of the running sum.
 template <int D, int QB, int DV = D>
-__device__ __forceinline__ void attend_tile(const Pack16 (&qreg)[QB][D / 32], const Pack16 (&a)[2][D / 32],
-                                            Pack16 (&vt)[DV / 16], int key0, int kv_len,
+__device__ __forceinline__ void attend_tile(const Pack16 (&qreg)[QB][D / 32], TileRegs<D, DV>& r, int key0, int kv_len,
                                             const int (&row_pos)[QB], row_spans_t<QB> window, score_scale_t scale_log2,
                                             f32x4_t (&acc)[QB][DV / 16], float (&m_run)[QB], float (&l_run)[QB]) {
   const int lane = threadIdx.x & 63;
-  const int grp = lane >> 4;
+  const int col = lane & 15, grp = lane >> 4;
+  if (r.at.there != 3) {            // a half without a page counts as zeros (rare, and the same for all lanes)
+    if (!((r.at.there >> (col >> 3)) & 1)) {
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int i = 0; i < D / 32; ++i) r.k[kb][i].u = make_uint4(0, 0, 0, 0);
+    }
+    if (!((r.at.there >> (grp >> 1)) & 1)) {
+#pragma unroll
+      for (int nb = 0; nb < DV / 16; ++nb) r.v[nb].u = make_uint4(0, 0, 0, 0);
+    }
+  }
   f32x4_t s[QB][2];
 #pragma unroll
   for (int kb = 0; kb < 2; ++kb)
@@ -682,7 +669,7 @@ __device__ __forceinline__ void attend_tile(const Pack16 (&qreg)[QB][D / 32], co
       f32x4_t c = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int i = 0; i < D / 32; ++i)
-        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[kb][i].v, qreg[qb][i].v, c, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(r.k[kb][i].v, qreg[qb][i].v, c, 0, 0, 0);
       s[qb][kb] = c;
     }
   Pack16 p[QB];
@@ -695,198 +682,47 @@ __device__ __forceinline__ void attend_tile(const Pack16 (&qreg)[QB][D / 32], co
     for (int nb = 0; nb < DV / 16; ++nb)
 #pragma unroll
       for (int j = 0; j < 8; ++j)
-        if (key0 + 16 * (j >> 2) + 4 * grp + (j & 3) >= kv_len) vt[nb].e[j] = (__bf16)0.f;
+        if (key0 + 8 * grp + j >= kv_len) r.v[nb].e[j] = (__bf16)0.f;
   }
 #pragma unroll
   for (int nb = 0; nb < DV / 16; ++nb)
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb)
-      acc[qb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt[nb].v, p[qb].v, acc[qb][nb], 0, 0, 0);
+      acc[qb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(r.v[nb].v, p[qb].v, acc[qb][nb], 0, 0, 0);
 }
 
-// All tiles first, first + step, ... below last for one wavefront: the value loads of a
-// tile and the key loads of the next one are issued before the tile's arithmetic. The
-// first tile's keys are loaded by the caller (`first_tile_keys`), who may have other work
-// to do while they travel.
-template <int D>
-__device__ __forceinline__ TileAddr first_tile_keys(Pack16 (&a_cur)[2][D / 32], const bf16_t* __restrict__ k_cache,
-                                                    const bf16_t* __restrict__ v_cache, int num_pages,
-                                                    const int* __restrict__ bt_row, int Hkv, int g_kv, int page,
-                                                    int first, int last, int kv_len) {
-  TileAddr t{};
-  if (first >= last) return t;
-  t = tile_addr(k_cache, v_cache, num_pages, bt_row, Hkv, g_kv, page, D, D, first * FAST_TILE, kv_len);
-  load_keys<D>(a_cur, t);
-  return t;
-}
-
-template <int D, int QB>
-__device__ __forceinline__ void attend_tiles(const Pack16 (&qreg)[QB][D / 32], Pack16 (&a_cur)[2][D / 32],
-                                             TileAddr t_cur, const bf16_t* __restrict__ k_cache,
-                                             const bf16_t* __restrict__ v_cache, int num_pages,
-                                             const int* __restrict__ bt_row, int Hkv, int g_kv, int page, int first,
-                                             int last, int step, int kv_len, const int (&row_pos)[QB],
-                                             row_spans_t<QB> window, score_scale_t scale_log2, f32x4_t (&acc)[QB][D / 16], float (&m_run)[QB],
-                                             float (&l_run)[QB]) {
+// A wavefront's walk over tiles first, first + step, ... below last. The caller has asked for the first tile
+// (`even`) and has the second one's table entries (`p_nxt`); every turn asks for the next tile's keys and values, a
+// whole tile before they are used, and for the table entries of the one after. The two sets of registers
+// change places by the code being there twice: copied, the next tile's would have to be waited for first. Behind
+// the last tile a turn asks for the cache's first page, as in TileAddr, rather than branch around its loads.
+// (Keys of 192 numbers leave no registers for a second tile's values: VALUES_AHEAD false asks for a tile's own
+// at the beginning of its turn.)
+template <int D, int DV, bool VALUES_AHEAD, typename Pages, typename Addr, typename Attend>
+__device__ __forceinline__ void walk_tiles(TileRegs<D, DV>& even, TileRegs<D, DV>& odd, TilePages p_nxt, int first, int last,
+                                           int step, int page, Pages pages_of, Addr addr_of, Attend attend) {
   if (first >= last) return;
-  Pack16 a_nxt[2][D / 32], vt[D / 16];
-  for (int t = first; t < last; t += step) {
-    load_values<D>(vt, t_cur, page);
-    const bool more = t + step < last;
-    if (more) {
-      t_cur = tile_addr(k_cache, v_cache, num_pages, bt_row, Hkv, g_kv, page, D, D, (t + step) * FAST_TILE, kv_len);
-      load_keys<D>(a_nxt, t_cur);
-    }
-    attend_tile<D, QB>(qreg, a_cur, vt, t * FAST_TILE, kv_len, row_pos, window, scale_log2, acc, m_run, l_run);
-    if (more) {
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int i = 0; i < D / 32; ++i) a_cur[kb][i] = a_nxt[kb][i];
-    }
-  }
-}
-
-// The same walk for a wavefront whose tiles are known before the sequence's length is (tiles
-// first, first + step, ... of the whole sequence): the caller has the first tile's keys on their
-// and values on their way (`a_cur`, `v_cur`) and the second tile's table entries asked for (`p_nxt`);
-// every turn asks for the table entries two tiles ahead, so that no key load waits for a table load.
-template <int D, int QB>
-__device__ __forceinline__ void attend_tiles_ahead(const Pack16 (&qreg)[QB][D / 32], Pack16 (&a_cur)[2][D / 32],
-                                                   Pack16 (&v_cur)[D / 16], TilePages p_nxt,
-                                                   const bf16_t* __restrict__ k_cache,
-                                                   const bf16_t* __restrict__ v_cache, int num_pages,
-                                                   const int* __restrict__ bt_row, int bt_stride, int Hkv, int g_kv,
-                                                   int page, int first, int last, int step, int kv_len,
-                                                   const int (&row_pos)[QB], row_spans_t<QB> window,
-                                                   score_scale_t scale_log2, f32x4_t (&acc)[QB][D / 16],
-                                                   float (&m_run)[QB], float (&l_run)[QB]) {
-  if (first >= last) return;
-  // a tile's keys and values are asked for together, a whole tile before they are used: a
-  // wavefront with two or three tiles (few requests, each over a few thousand keys) then waits
-  // for memory once per tile, not twice
-  Pack16 a_nxt[2][D / 32], v_nxt[D / 16];
-  for (int t = first; t < last; t += step) {
-    const bool more = t + step < last;
-    if (more) {
-      const TileAddr t_nxt = tile_addr_of(p_nxt, k_cache, v_cache, num_pages, Hkv, g_kv, page, D, D, (t + step) * FAST_TILE);
-      load_keys<D>(a_nxt, t_nxt);
-      load_values<D>(v_nxt, t_nxt, page);
-      p_nxt = tile_pages(bt_row, bt_stride, page, (t + 2 * step) * FAST_TILE);
-    }
-    attend_tile<D, QB>(qreg, a_cur, v_cur, t * FAST_TILE, kv_len, row_pos, window, scale_log2, acc, m_run, l_run);
-    if (more) {
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int i = 0; i < D / 32; ++i) a_cur[kb][i] = a_nxt[kb][i];
-#pragma unroll
-      for (int nb = 0; nb < D / 16; ++nb) v_cur[nb] = v_nxt[nb];
-    }
-  }
-}
-
-#ifdef Q3_POOLED
-// Both sources of a wavefront's rows as one sequence of tiles: of tiles first, first + step, ... below
-// last, those before `run_tiles` are runs', the others tokens' from tile `tile_lo` on. As in
-// attend_tiles_ahead a tile's keys and values are asked for a whole tile before they are used and its
-// table entries two tiles before.
-template <int D>
-__device__ __forceinline__ void attend_both(const Pack16 (&qreg)[1][D / 32], const bf16_t* __restrict__ k_cache,
-                                            const bf16_t* __restrict__ v_cache, int num_pages,
-                                            const int* __restrict__ bt_row, int bt_stride, const RunSource& runs,
-                                            const int* __restrict__ run_row, int Hkv, int g_kv, int page, int first,
-                                            int last, int step, int run_tiles, int tile_lo, int kv_len,
-                                            const int (&row_pos)[1], int window, score_scale_t scale_log2,
-                                            f32x4_t (&acc)[1][D / 16], float (&m_run)[1], float (&l_run)[1]) {
-  if (first >= last) return;
-  const int run_pos = runs_seen(row_pos[0], window, runs.pool) - 1, run_count = kv_len / runs.pool;
-  auto key_of = [&](int s) { return (s < run_tiles ? s : tile_lo + s - run_tiles) * FAST_TILE; };
-  auto pages_of = [&](int s) {
-    return s < run_tiles ? tile_pages(run_row, runs.stride, page, key_of(s)) : tile_pages(bt_row, bt_stride, page, key_of(s));
+  if (first + step >= last) p_nxt.pg[0] = p_nxt.pg[1] = -1;
+  int t = first;
+  auto turn = [&](TileRegs<D, DV>& cur, TileRegs<D, DV>& nxt) {
+    if constexpr (!VALUES_AHEAD) load_values(cur, page);
+    load_keys(nxt, addr_of(p_nxt, t + step));
+    if constexpr (VALUES_AHEAD) load_values(nxt, page);
+    if (t + 2 * step < last)
+      p_nxt = pages_of(t + 2 * step);
+    else
+      p_nxt.pg[0] = p_nxt.pg[1] = -1;
+    attend(cur, t);
+    t += step;
+    if (t < last) return true;
+    // (the way out meets the way back to the loop's head in the compiler's form of it: loads left open here
+    // would be waited for there, in each turn)
+    __builtin_amdgcn_s_waitcnt(0x0f70);     // vmcnt(0)
+    return false;
   };
-  auto addr_of = [&](const TilePages& p, int s) {
-    const bool run = s < run_tiles;
-    return tile_addr_of(p, run ? runs.k : k_cache, run ? runs.v : v_cache, run ? runs.num_pages : num_pages, Hkv, g_kv, page,
-                        D, D, key_of(s));
-  };
-  Pack16 a_cur[2][D / 32], v_cur[D / 16], a_nxt[2][D / 32], v_nxt[D / 16];
-  {
-    const TileAddr t = addr_of(pages_of(first), first);
-    load_keys<D>(a_cur, t);
-    load_values<D>(v_cur, t, page);
-  }
-  TilePages p_nxt = pages_of(first + step);
-  for (int s = first; s < last; s += step) {
-    const bool more = s + step < last;
-    if (more) {
-      const TileAddr t = addr_of(p_nxt, s + step);
-      load_keys<D>(a_nxt, t);
-      load_values<D>(v_nxt, t, page);
-      p_nxt = pages_of(s + 2 * step);
-    }
-    const bool run = s < run_tiles;
-    int pos[1] = {run ? run_pos : row_pos[0]};
-    attend_tile<D, 1>(qreg, a_cur, v_cur, key_of(s), run ? run_count : kv_len, pos, run ? 0 : window, scale_log2, acc, m_run,
-                      l_run);
-    if (more) {
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int i = 0; i < D / 32; ++i) a_cur[kb][i] = a_nxt[kb][i];
-#pragma unroll
-      for (int nb = 0; nb < D / 16; ++nb) v_cur[nb] = v_nxt[nb];
-    }
+  while (turn(even, odd) && turn(odd, even)) {
   }
 }
-#endif
-
-#ifdef Q3_SPAN
-// A wavefront's rows over a sequence of tiles of which those before `keep_tiles` are the sequence's first and
-// the others begin at tile `tile_lo`: tiles first, first + step, ... below last of it. As above a tile's keys
-// and values are asked for a whole tile before they are used and its table entries two tiles before.
-template <int D, int DV>
-__device__ __forceinline__ void attend_span(const Pack16 (&qreg)[1][D / 32], const bf16_t* __restrict__ k_cache,
-                                            const bf16_t* __restrict__ v_cache, int num_pages,
-                                            const int* __restrict__ bt_row, int bt_stride, int Hkv, int g_kv, int page,
-                                            int first, int last, int step, int keep_tiles, int tile_lo, int kv_len,
-                                            const int (&row_pos)[1], RowSpans<1> span, score_scale_t scale_log2,
-                                            f32x4_t (&acc)[1][DV / 16], float (&m_run)[1], float (&l_run)[1]) {
-  if (first >= last) return;
-  auto key_of = [&](int s) { return (s < keep_tiles ? s : tile_lo + s - keep_tiles) * FAST_TILE; };
-  auto addr_of = [&](const TilePages& p, int s) {
-    return tile_addr_of(p, k_cache, v_cache, num_pages, Hkv, g_kv, page, D, DV, key_of(s));
-  };
-  // (keys of 192 numbers leave no registers for a second tile's values: those are asked for a turn later)
-  constexpr bool VALUES_AHEAD = D <= 128;
-  Pack16 a_cur[2][D / 32], v_cur[DV / 16], a_nxt[2][D / 32], v_nxt[VALUES_AHEAD ? DV / 16 : 1];
-  TileAddr t_cur = addr_of(tile_pages(bt_row, bt_stride, page, key_of(first)), first);
-  load_keys<D>(a_cur, t_cur);
-  if constexpr (VALUES_AHEAD) load_values<DV>(v_cur, t_cur, page);
-  TilePages p_nxt = tile_pages(bt_row, bt_stride, page, key_of(first + step));
-  for (int s = first; s < last; s += step) {
-    const bool more = s + step < last;
-    if constexpr (!VALUES_AHEAD) load_values<DV>(v_cur, t_cur, page);
-    if (more) {
-      t_cur = addr_of(p_nxt, s + step);
-      load_keys<D>(a_nxt, t_cur);
-      if constexpr (VALUES_AHEAD) load_values<DV>(v_nxt, t_cur, page);
-      p_nxt = tile_pages(bt_row, bt_stride, page, key_of(s + 2 * step));
-    }
-    attend_tile<D, 1, DV>(qreg, a_cur, v_cur, key_of(s), kv_len, row_pos, span, scale_log2, acc, m_run, l_run);
-    if (more) {
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int i = 0; i < D / 32; ++i) a_cur[kb][i] = a_nxt[kb][i];
-      if constexpr (VALUES_AHEAD) {
-#pragma unroll
-        for (int nb = 0; nb < DV / 16; ++nb) v_cur[nb] = v_nxt[nb];
-      }
-    }
-  }
-}
-#endif
 
 // ---- sequences with few rows (q_len * G <= 16): decoding ---------------------
 // grid (splits, Hkv, B), 256 threads. The four wavefronts of a block take the
@@ -903,11 +739,15 @@ __device__ __forceinline__ void attend_span(const Pack16 (&qreg)[1][D / 32], con
 // block reads the new position from the cache: they read what earlier steps wrote, so no
 // read waits for a write.
 // Without a window (AHEAD) a wavefront's tiles are every (4 x splits)-th of the whole sequence,
-// so its first tile is known before the sequence's length is, and a tile's keys and values
-// travel together, one tile ahead of their use. Measured at batch 8 over 2,100 keys: 25.2 us
-// with the merge against 26.0 before; with 2, 4, 16, 32 splits instead of 8: 33, 27, 31, 48 us;
-// one request: 14 us (16 or 32 splits), which is what two launches and their chains of
-// dependent loads (length, table entry, keys; then the partial results) cost with no data at all.
+// so its first tile is known before the sequence's length is.
+// Bound by the keys' and values' bytes for many requests and by the chain of dependent loads for few: table entry
+// and length, then keys, values and the rotation's row together, then the merges; whatever needs none of these
+// (query rows, norm weights, the new key and value) is asked for before them.
+// Before, with each load behind a branch of its own, the first tile's value loads one after the other, and a wait for
+// the whole next tile at the end of every turn, against now, with the merge, microseconds, keys and values from
+// memory (8 key heads of 128): one request over 1,100 keys 13.7 and 11.4; eight over 2,060 24.9 and 22.7; 20 over 512 to
+// 1,030 25.2 and 22.1; 64 over 2,060 111 and 107 (5.0 TB/s; a plain read reaches 5.8); 33 over 700 35.5 and 32.3.
+// Eight wavefronts a block in place of two parts: 15 us for the first, which is three more.
 struct DecodePrep {
   const void* q_weight;  // (D,) or null: no norm
   const void* k_weight;
@@ -918,12 +758,46 @@ struct DecodePrep {
   bf16_t* v_cache;
 };
 
+// Eight numbers as they lie in memory, loaded before they are needed.
+template <typename W>
+struct Raw8 {
+  uint4 r[sizeof(W) / 2];
+};
+template <typename W>
+__device__ __forceinline__ Raw8<W> load_raw8(const W* p) {
+  Raw8<W> x;
+#pragma unroll
+  for (int i = 0; i < (int)sizeof(W) / 2; ++i) x.r[i] = reinterpret_cast<const uint4*>(p)[i];
+  return x;
+}
+__device__ __forceinline__ void unpack8(const Raw8<bf16_t>& x, float (&o)[8]) {
+  Half8 h;
+  h.u = x.r[0];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) o[i] = bf16_to_float(h.e[i]);
+}
+__device__ __forceinline__ void unpack8(const Raw8<float>& x, float (&o)[8]) {
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    o[4 * i] = __uint_as_float(x.r[i].x);
+    o[4 * i + 1] = __uint_as_float(x.r[i].y);
+    o[4 * i + 2] = __uint_as_float(x.r[i].z);
+    o[4 * i + 3] = __uint_as_float(x.r[i].w);
+  }
+}
+
+template <typename W>
+__device__ __forceinline__ void arrived(const Raw8<W>& x) {
+#pragma unroll
+  for (int i = 0; i < (int)sizeof(W) / 2; ++i) asm volatile("" ::"v"(x.r[i].x), "v"(x.r[i].w));
+}
+
 // One query row's operand registers from its raw values: lane (col, grp) holds elements
 // 32 i + 8 grp + j; the pairs (d, d + D / 2) are registers i and i + D / 64 of the same lane.
 // The sums take the order of the preparation kernel's butterfly (its lane c = 4 i + grp).
 template <int D, typename W>
-__device__ __forceinline__ void prepare_query(Pack16 (&qreg)[D / 32], const W* weight, float eps,
-                                              const float* table_row, int grp) {
+__device__ __forceinline__ void prepare_query(Pack16 (&qreg)[D / 32], bool norm, const Raw8<W> (&weight)[D / 32], float eps,
+                                              bool turn, const Raw8<float> (&table)[D / 32]) {
   constexpr int HI = D / 64;
   float a[HI][8], b[HI][8];
 #pragma unroll
@@ -933,7 +807,7 @@ __device__ __forceinline__ void prepare_query(Pack16 (&qreg)[D / 32], const W* w
       a[i][j] = (float)qreg[i].e[j];
       b[i][j] = (float)qreg[i + HI].e[j];
     }
-  if (weight != nullptr) {
+  if (norm) {
     float ss = pairs_sum_of_squares(a[0], b[0]);
     if constexpr (HI == 2) ss += pairs_sum_of_squares(a[1], b[1]);
     ss += __shfl_xor(ss, 32, 64);
@@ -942,17 +816,17 @@ __device__ __forceinline__ void prepare_query(Pack16 (&qreg)[D / 32], const W* w
 #pragma unroll
     for (int i = 0; i < HI; ++i) {
       float wa[8], wb[8];
-      load_weights8<W>(weight + 32 * i + 8 * grp, wa);
-      load_weights8<W>(weight + D / 2 + 32 * i + 8 * grp, wb);
+      unpack8(weight[i], wa);
+      unpack8(weight[i + HI], wb);
       pairs_normalise(a[i], b[i], scale, wa, wb);
     }
   }
-  if (table_row != nullptr) {
+  if (turn) {
 #pragma unroll
     for (int i = 0; i < HI; ++i) {
       float cs[8], sn[8];
-      load_weights8<float>(table_row + 32 * i + 8 * grp, cs);
-      load_weights8<float>(table_row + D / 2 + 32 * i + 8 * grp, sn);
+      unpack8(table[i], cs);
+      unpack8(table[i + HI], sn);
       pairs_rotate(a[i], b[i], cs, sn);
     }
   }
@@ -965,86 +839,70 @@ __device__ __forceinline__ void prepare_query(Pack16 (&qreg)[D / 32], const W* w
     }
 }
 
-// The new key of head g_kv (the first D / 16 lanes of the block's last wavefront, as the
-// preparation kernel's lanes) and the new value (the first D / 16 lanes of the wavefront
-// before it) of the token whose raw row is `row`, into
-// slot pos % page of `pg` (if there is such a page) and, as the cache's rounded numbers, into
-// shared memory.
+// The new key of a head (the first D / 16 lanes of the block's last wavefront, as the preparation kernel's lanes)
+// or the new value (those of the wavefront before it), `raw` in pieces c and c + D / 16, into slot `slot` of `pg` (if
+// there is such a page) and, as the cache's rounded numbers, into shared memory.
 template <int D, typename W>
-__device__ __forceinline__ void store_new_key_value(const bf16_t* row, int Hq, int Hkv, int g_kv, const W* k_weight,
-                                                    float eps, const float* table_row, bf16_t* k_cache,
-                                                    bf16_t* v_cache, int pg, int page, int slot, float* sh_k,
-                                                    float* sh_v) {
+__device__ __forceinline__ void store_new_key(Half8 (&raw)[2], int c, bool norm, const Raw8<W> (&weight)[2], float eps,
+                                              bool turn, const Raw8<float> (&table)[2], bf16_t* k_cache, int pg, int Hkv,
+                                              int g_kv, int page, int slot, float* sh_k) {
   constexpr int LPH = D / 16, HALF = D / 2;
-  const int t = threadIdx.x;
-  if (t >= 192 && t < 192 + LPH) {
-    const int c = t - 192;
-    const bf16_t* src = row + (size_t)(Hq + g_kv) * D;
-    Half8 x1, x2;
-    x1.u = *reinterpret_cast<const uint4*>(src + 8 * c);
-    x2.u = *reinterpret_cast<const uint4*>(src + HALF + 8 * c);
-    float a[8], b[8];
+  float a[8], b[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    a[i] = bf16_to_float(raw[0].e[i]);
+    b[i] = bf16_to_float(raw[1].e[i]);
+  }
+  if (norm) {
+    float ss = pairs_sum_of_squares(a, b);
+#pragma unroll
+    for (int off = LPH / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
+    float wa[8], wb[8];
+    unpack8(weight[0], wa);
+    unpack8(weight[1], wb);
+    pairs_normalise(a, b, head_norm_scale(ss, D, eps), wa, wb);
+  }
+  if (turn) {
+    float cs[8], sn[8];
+    unpack8(table[0], cs);
+    unpack8(table[1], sn);
+    pairs_rotate(a, b, cs, sn);
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    raw[0].e[i] = float_to_bf16(a[i]);
+    raw[1].e[i] = float_to_bf16(b[i]);
+    sh_k[8 * c + i] = bf16_to_float(raw[0].e[i]);
+    sh_k[HALF + 8 * c + i] = bf16_to_float(raw[1].e[i]);
+  }
+  if (pg >= 0) {
+    bf16_t* dst = k_cache + (((size_t)pg * Hkv + g_kv) * page + slot) * D;
+    *reinterpret_cast<uint4*>(dst + 8 * c) = raw[0].u;
+    *reinterpret_cast<uint4*>(dst + HALF + 8 * c) = raw[1].u;
+  }
+}
+
+template <int D>
+__device__ __forceinline__ void store_new_value(const Half8 (&raw)[2], int c, bf16_t* v_cache, int pg, int Hkv, int g_kv,
+                                                int page, int slot, float* sh_v) {
+  constexpr int HALF = D / 2;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    sh_v[8 * c + i] = bf16_to_float(raw[0].e[i]);
+    sh_v[HALF + 8 * c + i] = bf16_to_float(raw[1].e[i]);
+  }
+  if (pg >= 0) {
+    bf16_t* o = v_cache + ((size_t)pg * Hkv + g_kv) * D * page + slot;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      a[i] = bf16_to_float(x1.e[i]);
-      b[i] = bf16_to_float(x2.e[i]);
-    }
-    if (k_weight != nullptr) {
-      float ss = pairs_sum_of_squares(a, b);
-#pragma unroll
-      for (int off = LPH / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
-      float wa[8], wb[8];
-      load_weights8<W>(k_weight + 8 * c, wa);
-      load_weights8<W>(k_weight + HALF + 8 * c, wb);
-      pairs_normalise(a, b, head_norm_scale(ss, D, eps), wa, wb);
-    }
-    if (table_row != nullptr) {
-      float cs[8], sn[8];
-      load_weights8<float>(table_row + 8 * c, cs);
-      load_weights8<float>(table_row + HALF + 8 * c, sn);
-      pairs_rotate(a, b, cs, sn);
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      x1.e[i] = float_to_bf16(a[i]);
-      x2.e[i] = float_to_bf16(b[i]);
-      sh_k[8 * c + i] = bf16_to_float(x1.e[i]);
-      sh_k[HALF + 8 * c + i] = bf16_to_float(x2.e[i]);
-    }
-    if (pg >= 0) {
-      bf16_t* dst = k_cache + (((size_t)pg * Hkv + g_kv) * page + slot) * D;
-      *reinterpret_cast<uint4*>(dst + 8 * c) = x1.u;
-      *reinterpret_cast<uint4*>(dst + HALF + 8 * c) = x2.u;
-    }
-  } else if (t >= 128 && t < 128 + LPH) {
-    const int c = t - 128;
-    const bf16_t* src = row + (size_t)(Hq + Hkv + g_kv) * D;
-    Half8 x1, x2;
-    x1.u = *reinterpret_cast<const uint4*>(src + 8 * c);
-    x2.u = *reinterpret_cast<const uint4*>(src + HALF + 8 * c);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      sh_v[8 * c + i] = bf16_to_float(x1.e[i]);
-      sh_v[HALF + 8 * c + i] = bf16_to_float(x2.e[i]);
-    }
-    if (pg >= 0) {
-      bf16_t* o = v_cache + ((size_t)pg * Hkv + g_kv) * D * page + slot;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        o[(size_t)(8 * c + i) * page] = x1.e[i];
-        o[(size_t)(HALF + 8 * c + i) * page] = x2.e[i];
-      }
+      o[(size_t)(8 * c + i) * page] = raw[0].e[i];
+      o[(size_t)(HALF + 8 * c + i) * page] = raw[1].e[i];
     }
   }
 }
 
-// (with two sources the kernel would take a few registers more than leave room for two blocks a CU, which
-// takes a third longer from two splits on)
-#if defined(Q3_POOLED) || defined(Q3_SPAN)
+// (left alone the compiler takes more registers than leave room for two wavefronts a SIMD)
 #define Q3_DECODE_WAVES __attribute__((amdgpu_waves_per_eu(2)))
-#else
-#define Q3_DECODE_WAVES
-#endif
 template <int D, bool PREP, typename W, bool AHEAD, int DV = D>
 __global__ __launch_bounds__(256) Q3_DECODE_WAVES void attn_decode_kernel(
     const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, const bf16_t* __restrict__ k_cache,
@@ -1052,6 +910,7 @@ __global__ __launch_bounds__(256) Q3_DECODE_WAVES void attn_decode_kernel(
     const int* __restrict__ cu_q, const int* __restrict__ kv_lens, int Hq, int Hkv, int page, score_scale_t scale_log2,
     span_t window, int splits, float* __restrict__ ws_acc, float* __restrict__ ws_ml, DecodePrep prep,
     const float* __restrict__ sink Q3_BIAS_PARAM Q3_RUNS_PARAM Q3_GATE_PARAM) {
+  constexpr int WAVES = 4;
   const int b = blockIdx.z, g_kv = blockIdx.y, split = blockIdx.x;
   const int G = Hq / Hkv;
   // a step of single tokens (PREP): sequence b's token is row b, and nothing is read to know it
@@ -1059,28 +918,51 @@ __global__ __launch_bounds__(256) Q3_DECODE_WAVES void attn_decode_kernel(
   const int q_len = PREP ? 1 : cu_q[b + 1] - q0;
   if (q_len <= 0 || q_len * G > 16) return;  // the other kernel's sequence
   const int* bt_row = block_table + (size_t)b * bt_stride;
-  // Without a window a wavefront's tiles are first, first + step, ... of the whole sequence, known
-  // before its length is: the table entries and then the keys of the first tile are asked for
-  // beside the length, not after it.
-  // (AHEAD: the host launches this form when there is no window.)
-  constexpr bool ahead = AHEAD;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, grp = lane >> 4;
+  const int rows = q_len * G;
+  // Without a window (AHEAD: the host launches this form then) a wavefront's tiles are first, first + step, ...
+  // of the whole sequence, known before its length is: the table entries are asked for beside the length.
   const int kv_len = kv_lens[b];
-  const int wave_of_block = threadIdx.x >> 6;
-  const int ahead_first = split * 4 + wave_of_block, ahead_step = 4 * splits;
-  Pack16 a_first[2][D / 32], v_first[ahead ? D / 16 : 1];
-  TileAddr t_first{};
-  TilePages p_second{};
-  if constexpr (ahead) {
-    t_first = tile_addr_of(tile_pages(bt_row, bt_stride, page, ahead_first * FAST_TILE), k_cache, v_cache, num_pages,
-                           Hkv, g_kv, page, D, D, ahead_first * FAST_TILE);
-    load_keys<D>(a_first, t_first);
-    load_values<D>(v_first, t_first, page);
+  const int ahead_first = split * WAVES + wave, ahead_step = WAVES * splits;
+  TilePages p_first{}, p_second{};
+  if constexpr (AHEAD) {
+    p_first = tile_pages(bt_row, bt_stride, page, ahead_first * FAST_TILE);
     p_second = tile_pages(bt_row, bt_stride, page, (ahead_first + ahead_step) * FAST_TILE);
   }
-  if (PREP && (q_len != 1 || kv_len < 1)) {
+  // the new key is not in the cache yet: the last split's block brings it
+  const bool fresh = PREP && prep.k_cache != nullptr;
+  const bool brings_new = fresh && split == splits - 1;  // uniform in the block
+
+  Pack16 qreg[1][D / 32];
+#pragma unroll
+  for (int i = 0; i < D / 32; ++i) {
+    const int row = min(col, rows - 1);       // rows that do not exist load the last one's and are zeroed
+    qreg[0][i].u = *reinterpret_cast<const uint4*>(q + (size_t)(q0 + row / G) * q_stride + (size_t)(g_kv * G + row % G) * D +
+                                                  32 * i + 8 * grp);
+  }
+  constexpr int LPH = D / 16;
+  Raw8<W> q_weight[D / 32] = {}, k_weight[2] = {};
+  Half8 fresh_raw[2];
+  const bool norm = PREP && prep.q_weight != nullptr;
+  const bool lends_key = brings_new && wave == WAVES - 1, lends_value = brings_new && wave == WAVES - 2;
+  const int piece = lane & (LPH - 1);
+  if constexpr (PREP) {
+    if (norm) {
+#pragma unroll
+      for (int i = 0; i < D / 32; ++i) q_weight[i] = load_raw8(static_cast<const W*>(prep.q_weight) + 32 * i + 8 * grp);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) k_weight[i] = load_raw8(static_cast<const W*>(prep.k_weight) + i * D / 2 + 8 * piece);
+    }
+    const bf16_t* src = q + (size_t)q0 * q_stride + (size_t)(Hq + (lends_value ? Hkv : 0) + g_kv) * D + 8 * piece;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) fresh_raw[i].u = *reinterpret_cast<const uint4*>(src + i * D / 2);
+  }
+
+  if (PREP && kv_len < 1) {
     // not a step of single tokens (the host sends no such row): the row's output is zero, and
     // the merge finds an empty share in this block's place, not whatever the workspace held
-    for (int i = threadIdx.x; i < q_len * G * D; i += blockDim.x) {
+    for (int i = threadIdx.x; i < rows * D; i += blockDim.x) {
       const int r = i / D, d = i - r * D;
       if (splits == 1) {
         out[(size_t)(q0 + r / G) * Hq * D + (size_t)(g_kv * G + r % G) * D + d] = float_to_bf16(0.f);
@@ -1095,29 +977,19 @@ __global__ __launch_bounds__(256) Q3_DECODE_WAVES void attn_decode_kernel(
     }
     return;
   }
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int col = lane & 15, grp = lane >> 4;
-  const int rows = q_len * G;
   const int first_pos = kv_len - q_len;
-  // the new key is not in the cache yet: the last split's block brings it
-  const bool fresh = PREP && prep.k_cache != nullptr;
-  const bool brings_new = fresh && split == splits - 1;  // uniform in the block
-  const float* table_row = nullptr;
+  Raw8<float> q_table[D / 32] = {}, k_table[2] = {};
+  bool turn = false;
   if constexpr (PREP) {
-    if (prep.table != nullptr && first_pos < prep.max_pos) table_row = prep.table + (size_t)first_pos * D;
-  }
-  __shared__ float sh_k[PREP ? D : 1], sh_v[PREP ? D : 1];
-
-  Pack16 qreg[1][D / 32];
+    turn = prep.table != nullptr && first_pos < prep.max_pos;
+    if (turn) {
+      const float* table_row = prep.table + (size_t)first_pos * D;
 #pragma unroll
-  for (int i = 0; i < D / 32; ++i) {
-    if (col < rows)
-      qreg[0][i].u = *reinterpret_cast<const uint4*>(q + (size_t)(q0 + col / G) * q_stride +
-                                                    (size_t)(g_kv * G + col % G) * D + 32 * i + 8 * grp);
-    else
-      qreg[0][i].u = make_uint4(0, 0, 0, 0);
+      for (int i = 0; i < D / 32; ++i) q_table[i] = load_raw8(table_row + 32 * i + 8 * grp);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) k_table[i] = load_raw8(table_row + i * D / 2 + 8 * piece);
+    }
   }
-
   // with a fresh key the cache is read up to the position before it: the rows then stand one
   // position earlier for the masks, and the window, which counts the new key, is one shorter
   const int kv_seen = fresh ? kv_len - 1 : kv_len;
@@ -1134,45 +1006,93 @@ __global__ __launch_bounds__(256) Q3_DECODE_WAVES void attn_decode_kernel(
   int tile_hi = (kv_seen + FAST_TILE - 1) / FAST_TILE;
   if (fresh && window == 1) tile_hi = tile_lo;  // the new key alone is visible
 #endif
+  // the sequence of tiles that the splits share out, and what this wavefront takes of it
 #if defined(Q3_SPAN)
-  // the first keys' tiles come first in the sequence of tiles that the splits share out
-  const int keep_tiles = min((window.keep + FAST_TILE - 1) / FAST_TILE, tile_lo);
-  const int all_tiles = keep_tiles + tile_hi - tile_lo;
-  const int per_split = (all_tiles + splits - 1) / splits;
-  const int s0 = min(split * per_split, all_tiles), s1 = min(s0 + per_split, all_tiles);
-  (void)t_first;
+  // the first keys' tiles come first
+  const int front = min((window.keep + FAST_TILE - 1) / FAST_TILE, tile_lo);
 #elif defined(Q3_POOLED)
-  // the runs' tiles come first in the sequence of tiles that the splits share out
-  const int run_tiles = (runs_seen(first_pos + q_len - 1, window, runs.pool) + FAST_TILE - 1) / FAST_TILE;
-  const int all_tiles = run_tiles + max(tile_hi - tile_lo, 0);
-  const int per_split = (all_tiles + splits - 1) / splits;
-  const int s0 = min(split * per_split, all_tiles), s1 = min(s0 + per_split, all_tiles);
-  (void)t_first;
+  // the runs' tiles come first
+  const int front = (runs_seen(first_pos + q_len - 1, window, runs.pool) + FAST_TILE - 1) / FAST_TILE;
+  const int run_pos = runs_seen(row_pos[0], window, runs.pool) - 1, run_count = kv_seen / runs.pool;
+  const int* run_row = runs.table + (size_t)b * runs.stride;
 #else
-  const int per_split = (max(tile_hi - tile_lo, 0) + splits - 1) / splits;
-  const int t0 = tile_lo + split * per_split;
-  const int t1 = min(tile_hi, t0 + per_split);
+  constexpr int front = 0;
 #endif
-#if !defined(Q3_POOLED) && !defined(Q3_SPAN)
-  // the first tile's keys are on their way while the query rows are prepared
-  if constexpr (!ahead)
-    t_first = first_tile_keys<D>(a_first, k_cache, v_cache, num_pages, bt_row, Hkv, g_kv, page, t0 + wave, t1, kv_seen);
+  const int all_tiles = front + max(tile_hi - tile_lo, 0);
+  const int per_split = (all_tiles + splits - 1) / splits;
+  const int first = AHEAD ? ahead_first : min(split * per_split, all_tiles) + wave;
+  const int last = AHEAD ? tile_hi : min(min(split * per_split, all_tiles) + per_split, all_tiles);
+  const int step = AHEAD ? ahead_step : WAVES;
+  auto key_of = [&](int t) {
+    if constexpr (AHEAD) return t * FAST_TILE;
+    return (t < front ? t : tile_lo + t - front) * FAST_TILE;
+  };
+  auto pages_of = [&](int t) {
+#ifdef Q3_POOLED
+    if (t < front) return tile_pages(run_row, runs.stride, page, key_of(t));
 #endif
+    return tile_pages(bt_row, bt_stride, page, key_of(t));
+  };
+  auto addr_of = [&](const TilePages& p, int t) {
+#ifdef Q3_POOLED
+    if (t < front) return tile_addr(p, runs.k, runs.v, runs.num_pages, Hkv, g_kv, page, D, D, key_of(t));
+#endif
+    return tile_addr(p, k_cache, v_cache, num_pages, Hkv, g_kv, page, D, DV, key_of(t));
+  };
+  constexpr bool VALUES_AHEAD = D <= 128;
+  TileRegs<D, DV> even, odd;
+  if constexpr (!AHEAD) {
+    if (first < last) {
+      p_first = pages_of(first);
+      p_second = pages_of(first + step);
+    } else {
+      p_first.pg[0] = p_first.pg[1] = -1;
+    }
+  }
+  // (a wavefront without a tile asks for the cache's first page and never looks at it)
+  load_keys(even, AHEAD || first < last ? addr_of(p_first, first) : tile_addr(p_first, k_cache, v_cache, num_pages, Hkv, g_kv, page, D, DV, 0));
+  if constexpr (VALUES_AHEAD) load_values(even, page);
+  __builtin_amdgcn_sched_barrier(0);     // the loads above are on their way before anything waits for them
+
+  __shared__ float sh_k[PREP ? D : 1], sh_v[PREP ? D : 1];
+  if (col >= rows) {
+#pragma unroll
+    for (int i = 0; i < D / 32; ++i) qreg[0][i].u = make_uint4(0, 0, 0, 0);
+  }
   float m_new = -INFINITY;  // in the last wavefront: the new key's score for this lane's row
   if constexpr (PREP) {
-    prepare_query<D, W>(qreg[0], static_cast<const W*>(prep.q_weight), prep.eps, table_row, grp);
-    if (brings_new) {
+    prepare_query<D, W>(qreg[0], norm, q_weight, prep.eps, turn, q_table);
+    // Whatever was loaded here has arrived in all wavefronts, used or not: with loads left open on one of the ways to
+    // the walk below the compiler waits for every load at its head, in each of its turns.
+#pragma unroll
+    for (int i = 0; i < D / 32; ++i) {
+      arrived(q_weight[i]);
+      arrived(q_table[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      asm volatile("" ::"v"(fresh_raw[i].u.x), "v"(fresh_raw[i].u.w));
+      arrived(k_weight[i]);
+      arrived(k_table[i]);
+    }
+    if (lends_key || lends_value) {
       // the last two wavefronts, which have the fewest tiles, lend a few lanes: the key and the
-      // value into the cache for later steps, and into shared memory for this one (the value
-      // is read after the barriers of the merge, the key after the barrier below)
+      // value into the cache for later steps, and into shared memory for this one (the key is read by the
+      // wavefront that wrote it, the value after the merge's barriers)
       const int blk = first_pos / page;
       int pg = blk < bt_stride ? bt_row[blk] : -1;
       if (pg >= num_pages) pg = -1;
-      store_new_key_value<D, W>(q + (size_t)q0 * q_stride, Hq, Hkv, g_kv, static_cast<const W*>(prep.k_weight),
-                                prep.eps, table_row, prep.k_cache, prep.v_cache, pg, page, first_pos % page, sh_k,
-                                sh_v);
-      __syncthreads();  // the key is in shared memory for all lanes that read it (brings_new is the block's)
-      if (wave == 3) {
+      if (lane < LPH) {
+        if (lends_key)
+          store_new_key<D, W>(fresh_raw, piece, norm, k_weight, prep.eps, turn, k_table, prep.k_cache, pg, Hkv, g_kv, page,
+                              first_pos % page, sh_k);
+        else
+          store_new_value<D>(fresh_raw, piece, prep.v_cache, pg, Hkv, g_kv, page, first_pos % page, sh_v);
+      }
+      if (lends_key) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         float dot = 0.f;
 #pragma unroll
         for (int i = 0; i < D / 32; ++i)
@@ -1193,21 +1113,18 @@ __global__ __launch_bounds__(256) Q3_DECODE_WAVES void attn_decode_kernel(
 #else
   float m_run[1] = {-INFINITY}, l_run[1] = {0.f};
 #endif
-#if defined(Q3_SPAN)
-  attend_span<D, DV>(qreg, k_cache, v_cache, num_pages, bt_row, bt_stride, Hkv, g_kv, page, s0 + wave, s1, 4, keep_tiles,
-                     tile_lo, kv_seen, row_pos, win, scale_log2, acc, m_run, l_run);
-#elif defined(Q3_POOLED)
-  attend_both<D>(qreg, k_cache, v_cache, num_pages, bt_row, bt_stride, runs, runs.table + (size_t)b * runs.stride, Hkv, g_kv,
-                 page, s0 + wave, s1, 4, run_tiles, tile_lo, kv_seen, row_pos, win, scale_log2, acc, m_run, l_run);
+  walk_tiles<D, DV, VALUES_AHEAD>(even, odd, p_second, first, last, step, page, pages_of, addr_of,
+                                  [&](TileRegs<D, DV>& r, int t) {
+#ifdef Q3_POOLED
+                                    const bool run = t < front;
+                                    const int pos[1] = {run ? run_pos : row_pos[0]};
+                                    attend_tile<D, 1, DV>(qreg, r, key_of(t), run ? run_count : kv_seen, pos, run ? 0 : win,
+                                                          scale_log2, acc, m_run, l_run);
 #else
-  if constexpr (ahead)
-    attend_tiles_ahead<D, 1>(qreg, a_first, v_first, p_second, k_cache, v_cache, num_pages, bt_row, bt_stride, Hkv,
-                             g_kv, page, ahead_first, tile_hi, ahead_step, kv_seen, row_pos, win, scale_log2, acc,
-                             m_run, l_run);
-  else
-    attend_tiles<D, 1>(qreg, a_first, t_first, k_cache, v_cache, num_pages, bt_row, Hkv, g_kv, page, t0 + wave, t1, 4,
-                       kv_seen, row_pos, win, scale_log2, acc, m_run, l_run);
+                                    attend_tile<D, 1, DV>(qreg, r, key_of(t), kv_seen, row_pos, win, scale_log2, acc, m_run,
+                                                          l_run);
 #endif
+                                  });
 #ifdef Q3_SIGMOID
   m_run[0] = 0.f;
 #endif
@@ -1217,58 +1134,63 @@ __global__ __launch_bounds__(256) Q3_DECODE_WAVES void attn_decode_kernel(
   l += __shfl_xor(l, 16, 64);
   l += __shfl_xor(l, 32, 64);
 
-  // the merge of the four wavefronts, and of the new key as a fifth contribution of one key:
+  // the merge of the wavefronts, and of the new key as one more contribution of one key:
   // its score is its maximum, its sum is one, its accumulator is the value itself
-  __shared__ float sh_m[5][16], sh_l[4][16];
-  __shared__ float sh_acc[4][16][DV + 4];
+  __shared__ float sh_m[WAVES + 1][16], sh_l[WAVES][16];
+  __shared__ __attribute__((aligned(16))) float sh_acc[4][16][DV + 4];
   if (grp == 0) {
     sh_m[wave][col] = m_run[0];
     sh_l[wave][col] = l;
   }
-  if (wave == 3 && grp == 0) sh_m[4][col] = m_new;
+  if (wave == WAVES - 1 && grp == 0) sh_m[WAVES][col] = m_new;
   __syncthreads();
-  float m_all = fmaxf(fmaxf(sh_m[0][col], sh_m[1][col]), fmaxf(sh_m[2][col], sh_m[3][col]));
-  m_all = fmaxf(m_all, sh_m[4][col]);
+  float m_all = sh_m[0][col];
+#pragma unroll
+  for (int w = 1; w <= WAVES; ++w) m_all = fmaxf(m_all, sh_m[w][col]);
   const float w_mine = m_run[0] > -INFINITY ? exp2f(m_run[0] - m_all) : 0.f;
   if (col < rows) {
 #pragma unroll
     for (int nb = 0; nb < DV / 16; ++nb)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) sh_acc[wave][col][16 * nb + 4 * grp + j] = acc[0][nb][j] * w_mine;
+      *reinterpret_cast<f32x4_t*>(&sh_acc[wave][col][16 * nb + 4 * grp]) = acc[0][nb] * w_mine;
   }
   __syncthreads();
-  // 256 threads: thread -> (row = t / 16, d = t % 16 + 16 k)
-  const int r = threadIdx.x >> 4, dd = threadIdx.x & 15;
-  if (r >= rows) return;
-  const float m5 = sh_m[4][r];
-  const float mr = fmaxf(fmaxf(fmaxf(sh_m[0][r], sh_m[1][r]), fmaxf(sh_m[2][r], sh_m[3][r])), m5);
-  const float w5 = m5 > -INFINITY ? exp2f(m5 - mr) : 0.f;
-  float lr = w5;
+  // a thread takes four neighbouring columns of a row
+  for (int idx = threadIdx.x; idx < rows * (DV / 4); idx += 64 * WAVES) {
+    const int r = idx / (DV / 4), d = idx % (DV / 4) * 4;
+    const float m5 = sh_m[WAVES][r];
+    float mr = m5;
 #pragma unroll
-  for (int w = 0; w < 4; ++w) lr += sh_m[w][r] > -INFINITY ? sh_l[w][r] * exp2f(sh_m[w][r] - mr) : 0.f;
-  const int token = q0 + r / G, head = g_kv * G + r % G;
-  if (splits == 1) {
-    // a sink joins the denominator once, as 2^(sink log2(e) - maximum): here, or in the merge of the splits
+    for (int w = 0; w < WAVES; ++w) mr = fmaxf(mr, sh_m[w][r]);
+    const float w5 = m5 > -INFINITY ? exp2f(m5 - mr) : 0.f;
+    float lr = w5;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) lr += sh_m[w][r] > -INFINITY ? sh_l[w][r] * exp2f(sh_m[w][r] - mr) : 0.f;
+    f32x4_t o = *reinterpret_cast<const f32x4_t*>(&sh_acc[0][r][d]);
+#pragma unroll
+    for (int w = 1; w < 4; ++w) o += *reinterpret_cast<const f32x4_t*>(&sh_acc[w][r][d]);
+    if (PREP && w5 > 0.f) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] += sh_v[d + e] * w5;
+    }
+    const int token = q0 + r / G, head = g_kv * G + r % G;
+    if (splits == 1) {
+      // a sink joins the denominator once, as 2^(sink log2(e) - maximum): here, or in the merge of the splits
 #ifdef Q3_SIGMOID
-    const float inv = 1.f;
+      const float inv = 1.f;
 #else
-    const float inv = 1.f / (sink ? lr + exp2f(sink[head] * 1.4426950408889634f - mr) : lr);
+      const float inv = 1.f / (sink ? lr + exp2f(sink[head] * 1.4426950408889634f - mr) : lr);
 #endif
-    for (int d = dd; d < DV; d += 16) {
-      float o = sh_acc[0][r][d] + sh_acc[1][r][d] + sh_acc[2][r][d] + sh_acc[3][r][d];
-      if (PREP && w5 > 0.f) o += sh_v[d] * w5;
-      out[(size_t)token * Hq * DV + (size_t)head * DV + d] = float_to_bf16(o * inv Q3_OPEN(token, head, DV, d));
-    }
-  } else {
-    const size_t slot = (((size_t)b * Hkv + g_kv) * splits + split) * 16 + r;
-    for (int d = dd; d < DV; d += 16) {
-      float o = sh_acc[0][r][d] + sh_acc[1][r][d] + sh_acc[2][r][d] + sh_acc[3][r][d];
-      if (PREP && w5 > 0.f) o += sh_v[d] * w5;
-      ws_acc[slot * DV + d] = o;
-    }
-    if (dd == 0) {
-      ws_ml[slot * 2] = mr;
-      ws_ml[slot * 2 + 1] = lr;
+      union {
+        uint2 u;
+        bf16_t e[4];
+      } pk;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) pk.e[e] = float_to_bf16(o[e] * inv Q3_OPEN(token, head, DV, d + e));
+      *reinterpret_cast<uint2*>(out + (size_t)token * Hq * DV + (size_t)head * DV + d) = pk.u;
+    } else {
+      const size_t slot = (((size_t)b * Hkv + g_kv) * splits + split) * 16 + r;
+      *reinterpret_cast<f32x4_t*>(ws_acc + slot * DV + d) = o;
+      if (d == 0) *reinterpret_cast<float2*>(ws_ml + slot * 2) = make_float2(mr, lr);
     }
   }
 }

@@ -1661,23 +1661,34 @@ def span_sizes(heads, kv_heads, dim, vdim, page, dtype):
 
 
 def _splits(B, Hkv, max_kv_len):
-    """Into how many blocks a sequence's keys are split when a step has few rows per sequence:
-    until the chip is full, two blocks a compute unit and no more (the blocks beyond 512 run when
-    the others have ended: 24 requests of 8 key heads over 768 keys take 27 us in two parts and 31
-    in three, 12 requests over 2,000 keys 30 us in five parts and 35 in six); beyond 32 parts the
-    merge costs more than the split gains. Two corrections to that, both measured with 8 key heads
-    of 128: with 8,192 keys or more a block's work dwarfs its start and what counts is that the
-    blocks come in even rounds, so at least eight parts are taken up to 384 (sequence, key head)
-    pairs and four beyond (33 sequences over 8,200 keys: 257 us whole, 199 in eight parts; 40: 272
-    and 232; 24: 156 in two parts, 143 in eight; 48: 295 whole, 274 in four; over 32,000 keys 955
-    and 713, 1,022 and 832, 557 and 511, 1,110 and 1,018); and 257 to 320 pairs over fewer keys are
-    split in three (33 sequences over 2,100 keys: 78 us whole, 70 in three; 40: 85 and 78; from 48
-    sequences on one part is the fastest there)."""
+    """Into how many blocks a sequence's keys are split when a step has few rows per sequence. Measured with
+    8 key heads of 128, keys and values from memory, contexts all alike and spread over a quarter to the whole of
+    the longest, in microseconds with the merge:
+
+    - up to 256 keys a block has two tiles a wavefront and the merge costs more than a split gains (1 to 24
+      requests 9 to 12 whole, 11 to 18 in parts); up to 512 only where few blocks run (one request 11.2 and
+      10.9 in eight, four 12.8 and 12.2, eight 13.1 and 15.8);
+    - beyond that one block a compute unit (a second one shares the memory's rate and its merge is longer): eight
+      requests over 2,000 keys 22.5 in four parts, 23.2 in eight, 27.1 in two; two over 4,000 15.6 in sixteen, 18.8 in
+      24; twelve over 2,000 29.7 in two, 35.3 in three; twenty over 1,000 24.5 whole, 27.3 in three; one over
+      8,000 15.5 in 32 and 17.3 in sixteen, over 1,000 11.4 in either;
+    - where that leaves a sequence whole, long contexts are as a rule uneven ones and the longest would be waited
+      for: 20 requests over 1,000 to 4,000 keys 61.6 whole, 54.4 in three (all over 4,000: 71.7 and 72.2), 24
+      66.7 and 63.2; over 2,000 to 8,000 115.6 whole, 89.0 in six, 122 and 108;
+    - with 8,192 keys or more a block's work dwarfs its start and what counts is that the blocks come in even rounds:
+      at least eight parts up to 384 (sequence, key head) pairs and four beyond (33 sequences over 8,200 keys: 257
+      whole, 199 in eight parts; 48: 295 whole, 274 in four; over 32,000 keys 955 and 713, 1,110 and 1,018);
+    - 257 to 320 pairs, a little more than a block each: 36 requests over 2,000 keys 79.5 whole, 72.9 in three (over
+      1,000 44.3 and 44.6); from 48 requests on one part is the fastest there."""
     pairs = B * Hkv
-    splits = max(1, min(max_kv_len // 64, 512 // pairs, 32))
+    if max_kv_len <= 256:
+        return 1
+    if max_kv_len <= 512:
+        return max_kv_len // 64 if pairs <= 32 else 1
+    splits = max(1, min(max_kv_len // 64, 256 // pairs, 32 if max_kv_len >= 4096 else 16))
     if max_kv_len >= 8192 and pairs < 512:
         splits = max(splits, 8 if pairs <= 384 else 4)
-    elif 256 < pairs <= 320 and max_kv_len >= 1024:
+    elif (max_kv_len >= 4096 and 128 < pairs <= 192) or (max_kv_len >= 2048 and 256 < pairs <= 320):
         splits = 3
     return splits
 
