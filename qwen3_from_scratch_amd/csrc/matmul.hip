@@ -54,6 +54,7 @@ constexpr size_t WORKSPACE_BYTES = 128u << 20;
 constexpr size_t EVICT_BYTES = 512u << 20;     // twice the 256 MB last-level cache (the tuner's)
 constexpr size_t PARTIALS_BYTES = 128u << 20;  // float32 partial products of the hand-written kernel's K shares
 constexpr size_t STAGING_BYTES = 64u << 20;
+constexpr int FUSED_ROWS_LIMIT = 640;         // rows of a product that carries a norm (128 but for small weights)
 constexpr int EVICT_BLOCKS = 2048, EVICT_THREADS = 256;
 constexpr int MAX_CANDIDATES = 64;
 constexpr int LIBRARY = -1;                    // a Choice's `own` when the library serves the size
@@ -250,10 +251,27 @@ Choice plain_by_rule(int M, int N, int K) {
 // the fewest shares to fill the chip), unless the tiles come to a little more than a whole number of rounds over
 // the 256 CUs and leave most of them idle in the last one: then the library's product with the norm's work in a
 // kernel behind it (for KIND_RESIDUAL: declined, the caller's plain product and the norm's own kernel).
+// 129 to 640 rows (small weights): 64 x 128 tiles while they fit the chip in one round, in three stages (four blocks a
+// CU; five where more than 256 rows share K out), then 128 x 128, then the library. The products alone, us, three
+// stages / five / 128 x 128 / library: 201 rows of 4,096 x 1,024 10.5 / 11.1 / 14.0 / 12.0, of 8,192 x 1,024 11.1 / 11.7 /
+// 14.4 / 13.5, of 1,024 x 4,096 in eight shares 13.3 / 13.8 / 16.5; 400 rows of the last, in four, 17.4 / 15.7 / 16.7; 400
+// of 8,192 x 1,024 (448 tiles) 16.4 / 20.6 / 15.5 / 15.5; 532 of it (320 tiles of 128 x 128) 23.3 / 29.4 / 20.9 / 17.4.
 Choice fused_by_rule(int kind, int M, int N, int K) {
   (void)kind;
   Choice c;
   if (g_kernels == KERNELS_LIBRARY) return c;
+  if (M > 128) {
+    const long small = (long)((M + 63) / 64) * ((N + 127) / 128), large = (long)((M + 127) / 128) * ((N + 127) / 128);
+    if (small > 256 && large > 256 && g_kernels == KERNELS_BOTH) return c;
+    c.own = small > 256 ? 1 : 5;
+    c.splits = tiles::splits_that_fill(c.own, M, N, K);
+    if (c.own == 5 && c.splits > 1 && M > 256) {
+      c.own = 8;
+      c.splits = tiles::splits_that_fill(8, M, N, K);
+    }
+    if ((size_t)c.splits * ((M + 7) / 8 * 8) * N * sizeof(float) > PARTIALS_BYTES) c.splits = 1;
+    return c;
+  }
   c.own = 8;
   c.splits = tiles::splits_that_fill(8, M, N, K);
   if ((size_t)c.splits * ((M + 7) / 8 * 8) * N * sizeof(float) > PARTIALS_BYTES) c.splits = 1;
@@ -530,7 +548,7 @@ extern "C" int q3_matmul_init() {
   return set_up(g_devices[device]);
 }
 
-// Products of up to 256 rows that carry a norm, by the hand-written tiled kernel (the few-row kernel of
+// Products of up to 640 rows that carry a norm, by the hand-written tiled kernel (the few-row kernel of
 // gemm.hip does the same for up to 16 rows, or 64 of a small weight, and is faster there; the callers' policy decides which rows come
 // here). x (M, K) and w (N, K) bfloat16, K a multiple of 64, N of 4.
 //
@@ -542,7 +560,7 @@ extern "C" int q3_matmul_init() {
 extern "C" int q3_tiles_scaled(const void* x, const void* w, void* out, int M, int N, int K, int out_dtype,
                                int epilogue, const float* sums, int chunks, int sums_stride, float eps, int width,
                                void* stream_) {
-  if (!x || !w || !out || !sums || M < 1 || M > 256 || N % 4 || !tiles::takes(M, N, K)) return Q3_ERR_BAD_ARGUMENT;
+  if (!x || !w || !out || !sums || M < 1 || M > FUSED_ROWS_LIMIT || N % 4 || !tiles::takes(M, N, K)) return Q3_ERR_BAD_ARGUMENT;
   if (chunks < 1 || sums_stride < M || width != K) return Q3_ERR_BAD_ARGUMENT;
   const bool swiglu = epilogue == tiles::EPI_SWIGLU;
   if (!swiglu && epilogue != tiles::EPI_PLAIN) return Q3_ERR_BAD_ARGUMENT;
@@ -611,7 +629,7 @@ extern "C" int q3_tiles_residual(const void* x, const void* w, int M, int N, int
                                  const void* norm_weight, int norm_weight_dtype, void* values, float* sums,
                                  int sums_stride, void* stream_) {
   if (!x || !w || !residual || !norm_weight || !values || !sums || sums_stride < M) return Q3_ERR_BAD_ARGUMENT;
-  if (M < 1 || M > 256 || N % 4 || !tiles::takes(M, N, K)) return Q3_ERR_BAD_ARGUMENT;
+  if (M < 1 || M > FUSED_ROWS_LIMIT || N % 4 || !tiles::takes(M, N, K)) return Q3_ERR_BAD_ARGUMENT;
   if (norm_weight_dtype != Q3_BF16 && norm_weight_dtype != Q3_F32) return Q3_ERR_BAD_ARGUMENT;
   hipStream_t stream = (hipStream_t)stream_;
   std::lock_guard<std::mutex> hold(g_lock);

@@ -1815,15 +1815,26 @@ def _row_sums_args(unscaled, M, K):
 
 
 FUSED_ROWS_FEW, FUSED_ROWS_MOST = FEW_ROWS, 128
+FUSED_ROWS_SMALL = 640          # and of a small weight
+SMALL_WEIGHT_LEAST = 2 << 20    # (a few hundred rows of a weight smaller than this were not measured)
+
+
+def fused_rows_most(weight):
+    """Up to how many rows the tiled kernel carries a norm for a product with `weight`: 128 (beyond that the vendor
+    library's products with the norms as kernels of their own are faster), or 640 for a weight of 2 to 18 MB. There the
+    norm's kernel, the activation's and a product's second one cost more than the products' difference: a prompt of the
+    0.6B shape in one step, 3.49 ms at 136 to 256 rows and 3.71 at 512 with the kernels apart, 2.80 to 2.83 and 2.91 so;
+    level at 640 (3.71, 3.58), 3.91 against 3.94 at 768. The 8B shape (33 to 201 MB) 6.93 apart and 8.34 so at 136."""
+    size = weight.numel() * weight.element_size()
+    return FUSED_ROWS_SMALL if SMALL_WEIGHT_LEAST <= size <= SMALL_WEIGHT_BYTES else FUSED_ROWS_MOST
 
 
 def fused_rows_take(weight, M):
     """Whether the tiled kernel carries a norm for `M` rows of a product with `weight` (N, K):
-    more than 16 rows, at most 128 (beyond that the vendor library's products with the norms as
-    kernels of their own are faster), bfloat16, K a multiple of 64 and N of 4. (Where the few-row
+    more than 16 rows, at most `fused_rows_most`, bfloat16, K a multiple of 64 and N of 4. (Where the few-row
     kernel takes the rows too, a small weight's 17 to 32 or 64, that one is used.)"""
-    return (FUSED_ROWS_FEW < M <= FUSED_ROWS_MOST and weight.dtype == torch.bfloat16 and weight.dim() == 2
-            and weight.shape[1] % 64 == 0 and weight.shape[0] % 4 == 0 and weight.is_contiguous())
+    return (FUSED_ROWS_FEW < M <= FUSED_ROWS_SMALL and M <= fused_rows_most(weight) and weight.dtype == torch.bfloat16
+            and weight.dim() == 2 and weight.shape[1] % 64 == 0 and weight.shape[0] % 4 == 0 and weight.is_contiguous())
 
 
 def _tiles_scaled(x, weight, out, unscaled, swiglu, what):
@@ -1913,7 +1924,7 @@ def linear(x, weight, out_dtype=None, out=None, tiled=None, unscaled=None):
     if unscaled is not None and x.dtype == torch.bfloat16 and fused_rows_take(weight, M):
         return _tiles_scaled(x, weight, out, unscaled, False, "linear")
     _need(unscaled is None, "unscaled rows need bfloat16 and few rows with a tiled weight (few_rows_limit), or 17 to "
-          "128 rows with an inner size that is a multiple of 64")
+          "128 rows (640 of a small weight, fused_rows_most) with an inner size that is a multiple of 64")
     if M and x.dtype == torch.bfloat16 and not library("gemm").q3_linear_is_skinny(M, N, K, 1):
         # bfloat16 products with many rows go to the vendor library (hipBLASLt), as the
         # reference's engine uses its vendor library for them, or to the hand-written tiled
@@ -1996,7 +2007,7 @@ def linear_swiglu(x, weight, tiled=None, unscaled=None, kind="silu"):
         out = torch.empty((M, N // 2), dtype=x.dtype, device=x.device)
         return _tiles_scaled(x, weight, out, unscaled, True, "linear_swiglu")
     _need(unscaled is None, "unscaled rows need bfloat16 and few rows with a tiled weight (few_rows_limit), or 17 to "
-          "128 rows with an inner size that is a multiple of 64")
+          "128 rows (640 of a small weight, fused_rows_most) with an inner size that is a multiple of 64")
     if M and library("gemm").q3_linear_is_skinny(M, N, K, _DT[x.dtype]):
         out = torch.empty((M, N // 2), dtype=x.dtype, device=x.device)
         _check(library("gemm").q3_linear_swiglu(_ptr(x), _ptr(weight), _ptr(out), M, N, K, _DT[x.dtype], _stream()),
@@ -2018,7 +2029,7 @@ def linear_residual_norm(x, weight, tiled, residual, norm_weight):
 
     Up to `few_rows_limit(weight)` rows, with the weight's tiled copy and N a multiple of 16, it
     is the few-row kernel's epilogue (P = N / 16, partial sums of 16 columns). With more rows, up
-    to 128 (`fused_rows_take`; `tiled` is not used), the tiled kernel's partial products are added
+    to 128 or 640 (`fused_rows_take`; `tiled` is not used), the tiled kernel's partial products are added
     by a second kernel that does the same (P = ceil(N / 1024)). There the result is None, and
     nothing was done, for a size at which the plain product (`linear`) followed by the norm's own
     kernel is the faster way."""
@@ -2043,7 +2054,7 @@ def linear_residual_norm(x, weight, tiled, residual, norm_weight):
         _check(status, "linear_residual_norm")
         return values, sums
     _need(few, "bfloat16, a tiled weight with a width that is a multiple of 16 and no more rows than few_rows_limit, "
-          "or 17 to 128 rows with an inner size that is a multiple of 64")
+          "or 17 to 128 rows (640 of a small weight, fused_rows_most) with an inner size that is a multiple of 64")
     sums = torch.empty((N // 16, sums_stride(M)), dtype=torch.float32, device=x.device)
     _check(library("gemm").q3_linear_tiled(
         _ptr(x), _ptr(tiled), _ptr(values), M, N, K, 1, 2, None, 0, ctypes.c_float(0.0), 0,

@@ -93,6 +93,10 @@ class PagedAttention(Part):
     def takes_unscaled(self):
         return self.qkv is not None and self.qkv.fuses
 
+    @property
+    def unscaled_rows_most(self):
+        return self.qkv.fused_rows_most
+
     def forward(self, x, batch, cache, sink=None):
         Hq, Hkv, D = self.num_heads, self.num_kv_heads, self.head_dim
         qkv = self.qkv.forward(x)

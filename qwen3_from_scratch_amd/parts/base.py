@@ -91,7 +91,8 @@ class Part:
     # A model with a part that does not declare this is run without graphs.
     graph_safe = False
     # the norm fusion of steps with few rows (see NormSink, UnscaledRows): whether forward()
-    # takes `sink=`, and whether it takes UnscaledRows for its input
+    # takes `sink=`, and whether it takes UnscaledRows for its input (of up to `unscaled_rows_most`
+    # rows, where a part has that; `ops.FUSED_ROWS_MOST` otherwise)
     feeds_sink = False
     takes_unscaled = False
     # a part that works on a request's tokens in runs of fixed length (a mixer that keeps its

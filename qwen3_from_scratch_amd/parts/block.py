@@ -41,6 +41,9 @@ class PreNormBlock(Part):
         self.feed_forward = feed_forward
         self.mixer_norm = mixer_norm
         self.feed_forward_norm = feed_forward_norm
+        for norm, reader in ((mixer_norm, mixer), (feed_forward_norm, feed_forward)):
+            if hasattr(norm, "sink_for"):
+                norm.reader = reader        # up to how many rows it takes unscaled is its weight's matter
 
     def entry_norm(self):
         """The norm a preceding block may fuse into its last product (see

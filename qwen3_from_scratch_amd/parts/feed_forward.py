@@ -53,6 +53,10 @@ class SwiGLU(Part):
     def takes_unscaled(self):
         return self.gate_up is not None and self.gate_up.fuses
 
+    @property
+    def unscaled_rows_most(self):
+        return self.gate_up.fused_rows_most
+
     def forward(self, x, batch=None, sink=None):
         h = self.gate_up.forward_swiglu(x, self.activation)
         return self.down.forward(h) if sink is None else self.down.forward_into(h, sink)

@@ -49,10 +49,15 @@ class LinearWeight:
     def fuses(self):
         """Whether steps of few rows go through kernels whose epilogues carry the
         norm fusion, UnscaledRows in, a NormSink out: up to 16 rows (32 or 64 for a
-        small weight) the few-row kernel on the tiled copy, up to 128 the tiled
+        small weight) the few-row kernel on the tiled copy, up to 128 (or 640) the tiled
         matrix-core kernel. A
         reader of UnscaledRows must have output rows in steps of 4."""
         return self.tiled is not None and self.weight.shape[0] % 4 == 0
+
+    @property
+    def fused_rows_most(self):
+        """Up to how many rows those kernels take UnscaledRows for this weight."""
+        return ops.fused_rows_most(self.weight)
 
     def forward_into(self, x, sink):
         """x @ W^T added into the sink's residual and prepared for its norm, as

@@ -31,6 +31,7 @@ class RMSNorm(Part):
         self.leaf = leaf            # the tensor's name below the prefix; "" if it is the prefix itself
         self.offset = float(offset)
         self.weight = None
+        self.reader = None          # the part that reads this norm's result, if the block says so
 
     def tensors(self):
         return {self._name(self.leaf): TensorShape((self.size,), "scale" if self.offset == 0.0 else "bias")}
@@ -63,12 +64,13 @@ class RMSNorm(Part):
     def sink_for(self, x):
         """A NormSink for the residual `x` if this step may have the addition
         and this norm fused into the neighbouring products (bfloat16 with
-        tiled matrices; at most 16 rows and a width in steps of 16, or up to
-        128 rows and a width in steps of 64), else None."""
+        tiled matrices; at most 16 rows and a width in steps of 16, or a width in steps of 64 and up to
+        128 rows, or as many as the part that reads this norm says), else None."""
         rows = x.shape[0]
         if self.precision.act != torch.bfloat16 or not self.precision.tiled or self.weight is None:
             return None
-        if not 1 <= rows <= ops.FUSED_ROWS_MOST or self.size % (16 if rows <= ops.FUSED_ROWS_FEW else 64):
+        most = getattr(self.reader, "unscaled_rows_most", ops.FUSED_ROWS_MOST)
+        if not 1 <= rows <= most or self.size % (16 if rows <= ops.FUSED_ROWS_FEW else 64):
             return None
         return NormSink(x, self.weight, self.eps, self.size)
 

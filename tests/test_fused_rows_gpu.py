@@ -1,0 +1,52 @@
+"""Products of 129 to 640 rows of a small weight that carry a norm, and the steps that are made of them."""
+
+import pytest
+import torch
+
+from test_kernels_gpu import _ops, test_linear_residual_norm_and_unscaled_rows_beyond_sixteen as _fused_products
+
+pytestmark = pytest.mark.gpu
+
+
+# rows at both ends of the range and of a tile; a writer that shares K out and one that does not; readers whose tiles fit
+# the chip in one round of 64 x 128, of 128 x 128, and of neither
+@pytest.mark.parametrize("M,H,K,N2", [(129, 1024, 2048, 4096), (256, 1024, 4096, 8192), (257, 1024, 4096, 8192),
+                                      (400, 1088, 1024, 8000), (640, 1024, 4096, 8192), (640, 2048, 4096, 2560)])
+@pytest.mark.parametrize("norm_dtype", [torch.float32, torch.bfloat16])
+def test_products_that_carry_a_norm(M, H, K, N2, norm_dtype):
+    _fused_products(M, H, K, N2, norm_dtype)
+
+
+def test_rows_and_weights_that_take_part():
+    ops = _ops()
+    small, large, tiny = (torch.empty(n, 1024, dtype=torch.bfloat16, device="cuda") for n in (8192, 10240, 512))
+    assert [ops.fused_rows_take(small, m) for m in (16, 17, 128, 129, 640, 641)] == [False, True, True, True, True, False]
+    assert [ops.fused_rows_take(w, 129) for w in (large, tiny)] == [False, False]
+
+
+@pytest.mark.parametrize("inner", [4096, 8192])       # 8,192: the gate and up product is too large, its neighbours are not
+def test_prompts_whole_and_in_portions(inner):
+    from qwen3_from_scratch_amd.config import ModelConfig
+    from qwen3_from_scratch_amd.engine import ModelRunner, StepEntry, random_model
+
+    config = ModelConfig.from_dict(dict(
+        architectures=["Qwen3ForCausalLM"], vocab_size=2048, hidden_size=1024, hidden_act="silu", num_hidden_layers=3,
+        max_position_embeddings=2048, num_attention_heads=16, num_key_value_heads=8, head_dim=128,
+        intermediate_size=inner, rms_norm_eps=1e-6, rope_theta=1e6, tie_word_embeddings=False))
+    runner = ModelRunner(random_model(config, device="cuda:0", seed=3, std=0.02), 16, 100, 2)
+    tokens = torch.randint(0, 2048, (641,), generator=torch.Generator().manual_seed(4)).tolist()
+
+    def logits(cuts):
+        at = 0
+        for n in cuts:
+            out = runner.step([StepEntry("r", tokens[at:at + n], [n - 1])])
+            at += n
+        out = out.clone()
+        runner.finish("r")
+        return out
+
+    for M in (129, 300, 640, 641):
+        whole = logits([M])
+        portions = logits([100] * (M // 100) + [M % 100 or 100][:1] * bool(M % 100))
+        # two bfloat16 ways through three layers: a few roundings of 2^-9 each
+        assert float((whole - portions).norm() / portions.norm()) < 2e-2, M
