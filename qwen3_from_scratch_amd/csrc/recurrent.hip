@@ -533,30 +533,61 @@ __device__ inline int chunks_before(const int* __restrict__ cu, int b) {
   return n;
 }
 
-// la of the chunk's rows into shared memory (one thread; 64 additions), returns nothing.
-__device__ inline void chunk_decays(float* la, const float* __restrict__ ld, long ld_row, int h, int row0, int len) {
-  if (threadIdx.x == 0) {
-    float run = 0.f;
-    for (int s = 0; s < Q3_CHUNK; ++s) {
-      if (s < len) run += ld[(size_t)(row0 + s) * ld_row + h];
-      la[s] = run;
-    }
+// la of the chunk's rows, added up in order by one wavefront from a lane each (the caller's first; a loop of loads is
+// 64 round trips), and behind them, if asked for, exp(la_last - la_s), zero past the chunk's end.
+__device__ inline void chunk_decays(float* la, float* left, const float* __restrict__ ld, long ld_row, int h, int row0, int len) {
+  if (threadIdx.x >= 64) return;
+  const int lane = threadIdx.x;
+  const float own = lane < len ? ld[(size_t)(row0 + lane) * ld_row + h] : 0.f;
+  float run = 0.f, mine = 0.f;
+#pragma unroll
+  for (int s = 0; s < Q3_CHUNK; ++s) {
+    run += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(own), s));
+    if (lane == s) mine = run;
+  }
+  la[lane] = mine;
+  if (left) left[lane] = lane < len ? expf(run - mine) : 0.f;      // (the rows past the end add nothing: run is la_last)
+}
+
+// The chunk kernels' products run on the matrix cores (v_mfma_f32_16x16x4_f32: float32 operands and sums, one k after
+// the other, with the bits of a loop of multiply-adds). A wavefront's operands are single numbers from shared memory,
+// 16 neighbouring ones of four rows (row stride 16 more than a multiple of 64 numbers) or one number of sixteen rows
+// for four neighbouring k (row stride 4 more): either way all 64 banks. The columns are the first operand, so that a
+// lane holds four neighbouring columns of one row of the result.
+typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+#define Q3_ROW16 80      // row strides of a 64-wide slice in the two layouts
+#define Q3_ROW4 68
+
+__device__ inline float4 load_four(const float* p, int there, bool whole) {   // p[0 .. 3], of which `there` exist
+  if (whole) return there > 0 ? *reinterpret_cast<const float4*>(p) : make_float4(0.f, 0.f, 0.f, 0.f);
+  return make_float4(there > 0 ? p[0] : 0.f, there > 1 ? p[1] : 0.f, there > 2 ? p[2] : 0.f, there > 3 ? p[3] : 0.f);
+}
+__device__ inline void store_four(float* p, const f32x4_t& v, int there, bool whole) {
+  if (whole) {
+    if (there > 0) *reinterpret_cast<f32x4_t*>(p) = v;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (e < there) p[e] = v[e];
   }
 }
 
 // grid (chunks of the longest sequence, H * dv tiles of 64, B); 256 threads. U[i][j] = sum_s
 // exp(la_last - la_s) k_s[i] v_s[j] for the tile's 64 columns j, into `sums` (chunk, H, d, dv); the chunk's
-// whole decay exp(la_last) into `decays` (chunk, H). All threads bring k and v into shared memory; then eight
-// threads for every eight rows of d form 8 x 8 numbers each from 16-byte reads, four reads for 64 multiply-adds.
+// whole decay exp(la_last) into `decays` (chunk, H). d up to 64 MT; a wavefront takes 16 MT rows i.
+//
+// Bound by the passage of k, v and the sums through the caches (48 KB in, 32 KB out per block at d 128). 2,048 tokens,
+// 64 heads of 64 columns, d 128: 136 us with 8 x 8 multiply-adds a thread and one thread adding up the decays, 50 now.
+template <int MT>
 __global__ void __launch_bounds__(256) chunk_state_kernel(const float* __restrict__ k, const float* __restrict__ v,
                                                           const float* __restrict__ ld, long ld_row,
                                                           const int* __restrict__ cu, float* __restrict__ sums,
                                                           float* __restrict__ decays, int H, int hpg, int d, int dv) {
+  constexpr int KS = 64 * MT + 16;
   extern __shared__ __attribute__((aligned(16))) float lds[];
-  const int dp = (d + 7) / 8 * 8;           // rows of 8: the last ones may be zeros
-  float* kw = lds;                          // (64, dp)
-  float* vt = kw + Q3_CHUNK * dp;           // (64, 64)
-  __shared__ float la[Q3_CHUNK];
+  float* kw = lds;                          // (64, KS)
+  float* vt = kw + Q3_CHUNK * KS;           // (64, Q3_ROW16)
+  __shared__ float la[Q3_CHUNK], left[Q3_CHUNK];
   const int b = blockIdx.z;
   const int tiles = (dv + 63) / 64;
   const int h = blockIdx.y / tiles, tile = blockIdx.y % tiles;
@@ -567,70 +598,68 @@ __global__ void __launch_bounds__(256) chunk_state_kernel(const float* __restric
   const int len = n - c * Q3_CHUNK < Q3_CHUNK ? n - c * Q3_CHUNK : Q3_CHUNK;
   const int chunk = chunks_before(cu, b) + c;
   const int G = H / hpg, g = h / hpg;
-  chunk_decays(la, ld, ld_row, h, row0, len);
+  const int t = threadIdx.x;
+  const bool whole_k = d % 4 == 0 && ((size_t)k & 15) == 0;
+  const bool whole_v = dv % 4 == 0 && (((size_t)v | (size_t)sums) & 15) == 0;
+  const int pieces = (d + 3) / 4;           // of four numbers in a row of k
+  float4 gk[4 * MT], gv[4];
+#pragma unroll
+  for (int u = 0; u < 4 * MT; ++u) {
+    const int e = t + 256 * u, s = e / pieces, i = 4 * (e - s * pieces);
+    gk[u] = load_four(k + ((size_t)(row0 + s) * G + g) * d + i, s < len ? d - i : 0, whole_k);
+  }
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int e = t + 256 * u, s = e / 16, j = tile * 64 + 4 * (e % 16);
+    gv[u] = load_four(v + ((size_t)(row0 + s) * H + h) * dv + j, s < len ? dv - j : 0, whole_v);
+  }
+  chunk_decays(la, left, ld, ld_row, h, row0, len);
   __syncthreads();
-  const float last = la[len - 1];
-  // sixteen loads a thread are asked for before the first is used (a loop of single loads is a chain of round trips)
-  for (int e0 = threadIdx.x; e0 < Q3_CHUNK * dp; e0 += 256 * 16) {
-    float got[16];
 #pragma unroll
-    for (int u = 0; u < 16; ++u) {
-      const int e = e0 + 256 * u;
-      const int s = e / dp, i = e % dp;
-      got[u] = (e < Q3_CHUNK * dp && s < len && i < d) ? k[((size_t)(row0 + s) * G + g) * d + i] : 0.f;
-    }
-#pragma unroll
-    for (int u = 0; u < 16; ++u) {
-      const int e = e0 + 256 * u;
-      if (e < Q3_CHUNK * dp) kw[e] = e / dp < len ? got[u] * expf(last - la[e / dp]) : 0.f;
+  for (int u = 0; u < 4 * MT; ++u) {
+    const int e = t + 256 * u, s = e / pieces, i = 4 * (e - s * pieces);
+    if (s < Q3_CHUNK) {
+      const float w = left[s];
+      *reinterpret_cast<float4*>(kw + s * KS + i) = make_float4(gk[u].x * w, gk[u].y * w, gk[u].z * w, gk[u].w * w);
     }
   }
-  {
-    float got[16];
 #pragma unroll
-    for (int u = 0; u < 16; ++u) {
-      const int e = threadIdx.x + 256 * u;
-      const int s = e / 64, j = tile * 64 + e % 64;
-      got[u] = (s < len && j < dv) ? v[((size_t)(row0 + s) * H + h) * dv + j] : 0.f;
-    }
-#pragma unroll
-    for (int u = 0; u < 16; ++u) vt[threadIdx.x + 256 * u] = got[u];
+  for (int u = 0; u < 4; ++u) {
+    const int e = t + 256 * u;
+    *reinterpret_cast<float4*>(vt + (e / 16) * Q3_ROW16 + 4 * (e % 16)) = gv[u];
   }
   __syncthreads();
-  // (d up to 256: 32 groups of eight rows, eight threads each)
-  const int ti = threadIdx.x / 8, tj = threadIdx.x % 8;      // rows 8 ti .., columns 8 tj ..
-  if (8 * ti < dp) {
-    float acc[8][8];
+  const int lane = t & 63, wave = t >> 6, col = lane & 15, grp = lane >> 4;
+  f32x4_t acc[MT][4];
 #pragma unroll
-    for (int r = 0; r < 8; ++r)
+  for (int m = 0; m < MT; ++m)
 #pragma unroll
-      for (int x = 0; x < 8; ++x) acc[r][x] = 0.f;
-    for (int s = 0; s < len; ++s) {
-      const float4 k0 = *reinterpret_cast<const float4*>(kw + s * dp + 8 * ti);
-      const float4 k1 = *reinterpret_cast<const float4*>(kw + s * dp + 8 * ti + 4);
-      const float4 v0 = *reinterpret_cast<const float4*>(vt + s * 64 + 8 * tj);
-      const float4 v1 = *reinterpret_cast<const float4*>(vt + s * 64 + 8 * tj + 4);
-      const float kk[8] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w};
-      const float vv[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+    for (int x = 0; x < 4; ++x) acc[m][x] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int s0 = 0; s0 < Q3_CHUNK; s0 += 4) {
+    float vv[4], kk[MT];
 #pragma unroll
-      for (int r = 0; r < 8; ++r)
+    for (int x = 0; x < 4; ++x) vv[x] = vt[(s0 + grp) * Q3_ROW16 + 16 * x + col];
 #pragma unroll
-        for (int x = 0; x < 8; ++x) acc[r][x] += kk[r] * vv[x];
-    }
-    float* dst = sums + ((size_t)chunk * H + h) * d * dv;
+    for (int m = 0; m < MT; ++m) kk[m] = kw[(s0 + grp) * KS + 16 * (wave * MT + m) + col];
 #pragma unroll
-    for (int r = 0; r < 8; ++r) {
-      const int i = 8 * ti + r;
-      if (i < d) {
+    for (int m = 0; m < MT; ++m)
 #pragma unroll
-        for (int x = 0; x < 8; ++x) {
-          const int j = tile * 64 + 8 * tj + x;
-          if (j < dv) dst[(size_t)i * dv + j] = acc[r][x];
-        }
+      for (int x = 0; x < 4; ++x) acc[m][x] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[x], kk[m], acc[m][x], 0, 0, 0);
+  }
+  float* dst = sums + ((size_t)chunk * H + h) * d * dv;
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    const int i = 16 * (wave * MT + m) + col;
+    if (i < d) {
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const int j = tile * 64 + 16 * x + 4 * grp;
+        store_four(dst + (size_t)i * dv + j, acc[m][x], dv - j, whole_v);
       }
     }
   }
-  if (tile == 0 && threadIdx.x == 0) decays[(size_t)chunk * H + h] = expf(last);
+  if (tile == 0 && t == 0) decays[(size_t)chunk * H + h] = expf(la[len - 1]);
 }
 
 // grid (d * dv / 256, H, B): one number of the state per thread, through the sequence's chunks in
@@ -657,75 +686,85 @@ __global__ void chunk_scan_kernel(float* __restrict__ sums, const float* __restr
   *mine = S;
 }
 
+// A slice of 64 numbers of 64 rows (from column `from` of `width`, rows `row_stride` apart) on its way: four pieces a thread.
+__device__ inline void load_slice(float4 (&got)[4], const float* __restrict__ rows, size_t row_stride, int count, int from,
+                                  int width) {
+  const bool whole = width % 4 == 0 && row_stride % 4 == 0 && ((size_t)rows & 15) == 0;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int e = threadIdx.x + 256 * u, s = e / 16, i = from + 4 * (e % 16);
+    got[u] = load_four(rows + s * row_stride + i, s < count ? width - i : 0, whole);
+  }
+}
+__device__ inline void store_slice(float* to, int row, const float4 (&got)[4]) {
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int e = threadIdx.x + 256 * u;
+    *reinterpret_cast<float4*>(to + (e / 16) * row + 4 * (e % 16)) = got[u];
+  }
+}
+
 // grid (chunks of the longest sequence, groups, B): the chunk's raw products q_t . k_s (64 x 64), over d in
 // slices of 64 through shared memory, into `scores` (chunk, group, t, s). They are the same for all heads of a
-// group and all tiles of a head's columns, which only weigh them with their own decays.
+// group and all tiles of a head's columns, which only weigh them with their own decays. A wavefront takes 16 rows t.
 __global__ void __launch_bounds__(256) chunk_scores_kernel(const float* __restrict__ q, const float* __restrict__ k,
                                                            const int* __restrict__ cu, float* __restrict__ scores, int G,
                                                            int d) {
-  __shared__ float one[Q3_CHUNK * 65];
-  __shared__ float two[Q3_CHUNK * 65];
+  __shared__ __attribute__((aligned(16))) float one[Q3_CHUNK * Q3_ROW4], two[Q3_CHUNK * Q3_ROW4];
   const int b = blockIdx.z, g = blockIdx.y, c = blockIdx.x;
   const int start = cu[b], n = cu[b + 1] - start;
   if (c * Q3_CHUNK >= n) return;
   const int row0 = start + c * Q3_CHUNK;
   const int len = n - c * Q3_CHUNK < Q3_CHUNK ? n - c * Q3_CHUNK : Q3_CHUNK;
   const int chunk = chunks_before(cu, b) + c;
-  const int tt = threadIdx.x / 16, tj = threadIdx.x % 16;
-  float acc[4][4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, grp = lane >> 4;
+  const float *qr = q + ((size_t)row0 * G + g) * d, *kr = k + ((size_t)row0 * G + g) * d;
+  float4 gq[4], gk[4];
+  load_slice(gq, qr, (size_t)G * d, len, 0, d);
+  load_slice(gk, kr, (size_t)G * d, len, 0, d);
+  f32x4_t acc[4];
 #pragma unroll
-  for (int r = 0; r < 4; ++r)
-#pragma unroll
-    for (int x = 0; x < 4; ++x) acc[r][x] = 0.f;
+  for (int x = 0; x < 4; ++x) acc[x] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   for (int i0 = 0; i0 < d; i0 += 64) {
     __syncthreads();
-    {
-      float gq[16], gk[16];
-#pragma unroll
-      for (int u = 0; u < 16; ++u) {
-        const int e = threadIdx.x + 256 * u;
-        const int s = e / 64, i = i0 + e % 64;
-        const bool in = s < len && i < d;
-        gq[u] = in ? q[((size_t)(row0 + s) * G + g) * d + i] : 0.f;
-        gk[u] = in ? k[((size_t)(row0 + s) * G + g) * d + i] : 0.f;
-      }
-#pragma unroll
-      for (int u = 0; u < 16; ++u) {
-        const int e = threadIdx.x + 256 * u;
-        one[(e / 64) * 65 + e % 64] = gq[u];
-        two[(e / 64) * 65 + e % 64] = gk[u];
-      }
-    }
+    store_slice(one, Q3_ROW4, gq);
+    store_slice(two, Q3_ROW4, gk);
     __syncthreads();
-    for (int i = 0; i < 64; ++i) {
-      float qv[4], kv[4];
+    if (i0 + 64 < d) {
+      load_slice(gq, qr, (size_t)G * d, len, i0 + 64, d);
+      load_slice(gk, kr, (size_t)G * d, len, i0 + 64, d);
+    }
+#pragma unroll 4
+    for (int i = 0; i < 64; i += 4) {
+      const float qv = one[(16 * wave + col) * Q3_ROW4 + i + grp];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) qv[r] = one[(tt + 16 * r) * 65 + i];
-#pragma unroll
-      for (int x = 0; x < 4; ++x) kv[x] = two[(4 * tj + x) * 65 + i];
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int x = 0; x < 4; ++x) acc[r][x] += qv[r] * kv[x];
+      for (int x = 0; x < 4; ++x)
+        acc[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(two[(16 * x + col) * Q3_ROW4 + i + grp], qv, acc[x], 0, 0, 0);
     }
   }
-  float* dst = scores + ((size_t)chunk * G + g) * Q3_CHUNK * Q3_CHUNK;
+  float* dst = scores + ((size_t)chunk * G + g) * Q3_CHUNK * Q3_CHUNK + (16 * wave + col) * Q3_CHUNK;
 #pragma unroll
-  for (int r = 0; r < 4; ++r)
-    *reinterpret_cast<float4*>(dst + (tt + 16 * r) * Q3_CHUNK + 4 * tj) = make_float4(acc[r][0], acc[r][1], acc[r][2], acc[r][3]);
+  for (int x = 0; x < 4; ++x) *reinterpret_cast<f32x4_t*>(dst + 16 * x + 4 * grp) = acc[x];
 }
 
 // grid as chunk_state_kernel. A[t][s] = scores[t][s] exp(la_t - la_s) for s <= t; then
-// o[t][j] = sum_s A[t][s] v_s[j] + exp(la_t) sum_i q_t[i] S[i][j] with S the state before the chunk (from `sums`),
-// in slices of 64 over i through shared memory.
+// o[t][j] = exp(la_t) sum_i q_t[i] S[i][j] + sum_s A[t][s] v_s[j] with S the state before the chunk (from `sums`),
+// in slices of 64 over i through shared memory, the next slice (behind the last: v) on its way to registers meanwhile.
+// `skip_x` (rows of `skip_stride`; Mamba-2): o[t][j] += skip[h] x_t[h dv + j], D x in the recurrence's terms.
+// A wavefront takes 16 rows t.
+//
+// Bound like chunk_state_kernel (q, S, v and the scores in, the results out): the same rows 112 us before and 15 for a
+// kernel of its own that added D x, 82 now.
+template <typename TA>
 __global__ void __launch_bounds__(256) chunk_output_kernel(const float* __restrict__ q, const float* __restrict__ scores,
                                                            const float* __restrict__ v, const float* __restrict__ ld,
                                                            long ld_row, const int* __restrict__ cu,
                                                            const float* __restrict__ sums, float* __restrict__ out, int H,
-                                                           int hpg, int d, int dv) {
-  __shared__ float A[Q3_CHUNK * Q3_CHUNK];       // (t, s)
-  __shared__ float one[Q3_CHUNK * 65];           // a slice of q, rows padded to 65
-  __shared__ float two[Q3_CHUNK * 64];           // a slice of S, then of v
+                                                           int hpg, int d, int dv, const TA* __restrict__ skip_x,
+                                                           long skip_stride, const float* __restrict__ skip) {
+  __shared__ __attribute__((aligned(16))) float A[Q3_CHUNK * Q3_ROW4];       // (t, s)
+  __shared__ __attribute__((aligned(16))) float one[Q3_CHUNK * Q3_ROW4];     // a slice of q
+  __shared__ __attribute__((aligned(16))) float two[Q3_CHUNK * Q3_ROW16];    // a slice of S, then v
   __shared__ float la[Q3_CHUNK];
   const int b = blockIdx.z;
   const int tiles = (dv + 63) / 64;
@@ -737,97 +776,72 @@ __global__ void __launch_bounds__(256) chunk_output_kernel(const float* __restri
   const int len = n - c * Q3_CHUNK < Q3_CHUNK ? n - c * Q3_CHUNK : Q3_CHUNK;
   const int chunk = chunks_before(cu, b) + c;
   const int G = H / hpg, g = h / hpg;
-  chunk_decays(la, ld, ld_row, h, row0, len);
-  __syncthreads();
-  const int tt = threadIdx.x / 16, tj = threadIdx.x % 16;      // rows tt + 16 r, columns 4 tj .. 4 tj + 3
-  float acc[4][4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, grp = lane >> 4;
+  const float* qr = q + ((size_t)row0 * G + g) * d;
+  const float* S = sums + ((size_t)chunk * H + h) * d * dv;
   const float* raw = scores + ((size_t)chunk * G + g) * Q3_CHUNK * Q3_CHUNK;
+  float4 gq[4], gs[4], ga[4];
+  load_slice(gq, qr, (size_t)G * d, len, 0, d);
+  load_slice(gs, S, dv, d, tile * 64, dv);
+  load_slice(ga, raw, Q3_CHUNK, Q3_CHUNK, 0, Q3_CHUNK);
+  chunk_decays(la, nullptr, ld, ld_row, h, row0, len);
+  __syncthreads();
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int t = tt + 16 * r;
-    const float4 sc = *reinterpret_cast<const float4*>(raw + t * Q3_CHUNK + 4 * tj);
-    const float got[4] = {sc.x, sc.y, sc.z, sc.w};
+  for (int u = 0; u < 4; ++u) {
+    const int e = threadIdx.x + 256 * u, t = e / 16, s = 4 * (e % 16);
+    const float at = la[t], got[4] = {ga[u].x, ga[u].y, ga[u].z, ga[u].w};
+    float4 w;
+    w.x = (s <= t && t < len) ? got[0] * expf(at - la[s]) : 0.f;
+    w.y = (s + 1 <= t && t < len) ? got[1] * expf(at - la[s + 1]) : 0.f;
+    w.z = (s + 2 <= t && t < len) ? got[2] * expf(at - la[s + 2]) : 0.f;
+    w.w = (s + 3 <= t && t < len) ? got[3] * expf(at - la[s + 3]) : 0.f;
+    *reinterpret_cast<float4*>(A + t * Q3_ROW4 + s) = w;
+  }
+  f32x4_t acc[4];
+#pragma unroll
+  for (int x = 0; x < 4; ++x) acc[x] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int my_row = 16 * wave + col;
+  auto multiply = [&](const float* rows) {
+#pragma unroll 4
+    for (int i = 0; i < 64; i += 4) {
+      const float r = rows[my_row * Q3_ROW4 + i + grp];
+#pragma unroll
+      for (int x = 0; x < 4; ++x)
+        acc[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(two[(i + grp) * Q3_ROW16 + 16 * x + col], r, acc[x], 0, 0, 0);
+    }
+  };
+  for (int i0 = 0; i0 < d; i0 += 64) {
+    if (i0) __syncthreads();
+    store_slice(one, Q3_ROW4, gq);
+    store_slice(two, Q3_ROW16, gs);
+    __syncthreads();
+    if (i0 + 64 < d) {
+      load_slice(gq, qr, (size_t)G * d, len, i0 + 64, d);
+      load_slice(gs, S + (size_t)(i0 + 64) * dv, dv, d - i0 - 64, tile * 64, dv);
+    } else {
+      load_slice(gs, v + ((size_t)row0 * H + h) * dv, (size_t)H * dv, len, tile * 64, dv);
+    }
+    multiply(one);
+  }
+  const float grow = expf(la[my_row]);
+#pragma unroll
+  for (int x = 0; x < 4; ++x) acc[x] *= grow;
+  __syncthreads();
+  store_slice(two, Q3_ROW16, gs);
+  __syncthreads();
+  multiply(A);
+  if (my_row < len) {
+    const bool whole = dv % 4 == 0 && ((size_t)out & 15) == 0;
 #pragma unroll
     for (int x = 0; x < 4; ++x) {
-      const int s = 4 * tj + x;
-      A[t * Q3_CHUNK + s] = (s <= t && t < len) ? got[x] * expf(la[t] - la[s]) : 0.f;
-      acc[r][x] = 0.f;
-    }
-  }
-  // the state's share: exp(la_t) q_t S, a slice of 64 of d at a time
-  const float* S = sums + ((size_t)chunk * H + h) * d * dv;
-  for (int i0 = 0; i0 < d; i0 += 64) {
-    __syncthreads();
-    {
-      float gq[16], gs[16];
+      const int j = tile * 64 + 16 * x + 4 * grp;
+      if (skip_x) {
+        const TA* at = skip_x + (size_t)(row0 + my_row) * skip_stride + (size_t)h * dv + j;
 #pragma unroll
-      for (int u = 0; u < 16; ++u) {
-        const int e = threadIdx.x + 256 * u;
-        const int s = e / 64, i = i0 + e % 64;
-        gq[u] = (s < len && i < d) ? q[((size_t)(row0 + s) * G + g) * d + i] : 0.f;
-        const int si = i0 + e / 64, j = tile * 64 + e % 64;
-        gs[u] = (si < d && j < dv) ? S[(size_t)si * dv + j] : 0.f;
+        for (int e = 0; e < 4; ++e)
+          if (j + e < dv) acc[x][e] += skip[h] * to_float(at[e]);
       }
-#pragma unroll
-      for (int u = 0; u < 16; ++u) {
-        const int e = threadIdx.x + 256 * u;
-        one[(e / 64) * 65 + e % 64] = gq[u];
-        two[e] = gs[u];
-      }
-    }
-    __syncthreads();
-    for (int i = 0; i < 64; ++i) {
-      const float4 sv = *reinterpret_cast<const float4*>(two + i * 64 + 4 * tj);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float qv = one[(tt + 16 * r) * 65 + i];
-        acc[r][0] += qv * sv.x;
-        acc[r][1] += qv * sv.y;
-        acc[r][2] += qv * sv.z;
-        acc[r][3] += qv * sv.w;
-      }
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const float grow = expf(la[tt + 16 * r]);
-#pragma unroll
-    for (int x = 0; x < 4; ++x) acc[r][x] *= grow;
-  }
-  // the chunk's own share: A v
-  __syncthreads();
-  {
-    float gv[16];
-#pragma unroll
-    for (int u = 0; u < 16; ++u) {
-      const int e = threadIdx.x + 256 * u;
-      const int s = e / 64, j = tile * 64 + e % 64;
-      gv[u] = (s < len && j < dv) ? v[((size_t)(row0 + s) * H + h) * dv + j] : 0.f;
-    }
-#pragma unroll
-    for (int u = 0; u < 16; ++u) two[threadIdx.x + 256 * u] = gv[u];
-  }
-  __syncthreads();
-  for (int s = 0; s < len; ++s) {
-    const float4 vv = *reinterpret_cast<const float4*>(two + s * 64 + 4 * tj);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float a = A[(tt + 16 * r) * Q3_CHUNK + s];
-      acc[r][0] += a * vv.x;
-      acc[r][1] += a * vv.y;
-      acc[r][2] += a * vv.z;
-      acc[r][3] += a * vv.w;
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int t = tt + 16 * r;
-    if (t < len) {
-#pragma unroll
-      for (int x = 0; x < 4; ++x) {
-        const int j = tile * 64 + 4 * tj + x;
-        if (j < dv) out[((size_t)(row0 + t) * H + h) * dv + j] = acc[r][x];
-      }
+      store_four(out + ((size_t)(row0 + my_row) * H + h) * dv + j, acc[x], dv - j, whole);
     }
   }
 }
@@ -866,15 +880,6 @@ __global__ void mamba2_prepare_kernel(const TA* __restrict__ xbc, const TA* __re
     kf[(size_t)t * G * N + e] = to_float(row[H * P + e]);
     qf[(size_t)t * G * N + e] = to_float(row[H * P + G * N + e]);
   }
-}
-
-// y += D x after the three kernels.
-template <typename TA>
-__global__ void mamba2_skip_kernel(const TA* __restrict__ xbc, const float* __restrict__ d_skip, float* __restrict__ y,
-                                   int H, int P, int C) {
-  const int t = blockIdx.x;
-  for (int e = threadIdx.x; e < H * P; e += blockDim.x)
-    y[(size_t)t * H * P + e] += d_skip[e / P] * to_float(xbc[(size_t)t * C + e]);
 }
 
 // Retention's rows for the three kernels: q and k turned by the position (k times k_scale), v as float32.
@@ -926,27 +931,39 @@ extern "C" long q3_chunked_workspace(int T, int B, int H, int G, int d, int dv) 
   return 2L * T * G * d + (long)T * H * dv + (long)T * H + chunks * H * ((long)d * dv + 1) + chunks * G * Q3_CHUNK * Q3_CHUNK;
 }
 
-static int launch_chunks(const float* qf, const float* kf, const float* vf, const float* ld, long ld_row, float* sums,
-                         float* decays, float* scores, float* state, long state_stride, const int* slots, const int* cu, float* out,
-                         int B, int max_q_len, int H, int hpg, int d, int dv, hipStream_t stream) {
-  const int chunks = (max_q_len + Q3_CHUNK - 1) / Q3_CHUNK;
-  const int tiles = (dv + 63) / 64;
-  const dim3 grid(chunks, H * tiles, B);
-  const int dp = (d + 7) / 8 * 8;
-  const size_t lds = (size_t)(Q3_CHUNK * dp + Q3_CHUNK * 64) * sizeof(float);
+template <int MT>
+static int launch_chunk_states(const float* kf, const float* vf, const float* ld, long ld_row, const int* cu, float* sums,
+                               float* decays, dim3 grid, int H, int hpg, int d, int dv, hipStream_t stream) {
+  const size_t lds = (size_t)Q3_CHUNK * (64 * MT + 16 + Q3_ROW16) * sizeof(float);
   if (lds > 64 * 1024) {
-    // 64 rows of more than 192 numbers and the values' tile pass the 64 KB a launch may ask for unasked
-    const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(chunk_state_kernel),
+    // (from keys of 129 numbers on) more than the 64 KB a launch may ask for unasked
+    const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(chunk_state_kernel<MT>),
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (allowed != hipSuccess) return (int)allowed;
   }
-  hipLaunchKernelGGL(chunk_state_kernel, grid, dim3(256), lds, stream, kf, vf, ld, ld_row, cu, sums, decays, H, hpg, d,
-                     dv);
+  hipLaunchKernelGGL(chunk_state_kernel<MT>, grid, dim3(256), lds, stream, kf, vf, ld, ld_row, cu, sums, decays, H, hpg, d, dv);
+  return q3_launch_status();
+}
+
+// `skip_x`, `skip_stride`, `skip`: see chunk_output_kernel. d up to 256.
+template <typename TA>
+static int launch_chunks(const float* qf, const float* kf, const float* vf, const float* ld, long ld_row, float* sums,
+                         float* decays, float* scores, float* state, long state_stride, const int* slots, const int* cu, float* out,
+                         int B, int max_q_len, int H, int hpg, int d, int dv, const TA* skip_x, long skip_stride,
+                         const float* skip, hipStream_t stream) {
+  const int chunks = (max_q_len + Q3_CHUNK - 1) / Q3_CHUNK;
+  const int tiles = (dv + 63) / 64;
+  const dim3 grid(chunks, H * tiles, B);
+  const int status =
+      d <= 64 ? launch_chunk_states<1>(kf, vf, ld, ld_row, cu, sums, decays, grid, H, hpg, d, dv, stream)
+      : d <= 128 ? launch_chunk_states<2>(kf, vf, ld, ld_row, cu, sums, decays, grid, H, hpg, d, dv, stream)
+                 : launch_chunk_states<4>(kf, vf, ld, ld_row, cu, sums, decays, grid, H, hpg, d, dv, stream);
+  if (status) return status;
   hipLaunchKernelGGL(chunk_scan_kernel, dim3((d * dv + 255) / 256, H, B), dim3(256), 0, stream, sums, decays, state,
                      state_stride, slots, cu, H, d * dv);
   hipLaunchKernelGGL(chunk_scores_kernel, dim3(chunks, H / hpg, B), dim3(256), 0, stream, qf, kf, cu, scores, H / hpg, d);
-  hipLaunchKernelGGL(chunk_output_kernel, grid, dim3(256), 0, stream, qf, scores, vf, ld, ld_row, cu, sums, out, H, hpg, d,
-                     dv);
+  hipLaunchKernelGGL(chunk_output_kernel<TA>, grid, dim3(256), 0, stream, qf, scores, vf, ld, ld_row, cu, sums, out, H, hpg, d,
+                     dv, skip_x, skip_stride, skip);
   return q3_launch_status();
 }
 
@@ -961,18 +978,15 @@ extern "C" int q3_mamba2_chunked(const void* xbc, const void* dt, long dt_stride
   float* qf = scores + (size_t)(T / Q3_CHUNK + B) * G * Q3_CHUNK * Q3_CHUNK;
   float* kf = qf + (size_t)T * G * N;
   float* vf = kf + (size_t)T * G * N;
-  float* ld = vf + (size_t)T * H * P;
-  float* sums = ld + (size_t)T * H;
-  float* decays = sums + (size_t)(T / Q3_CHUNK + B) * H * N * P;
+  float* sums = vf + (size_t)T * H * P;      // before what comes in single numbers
+  float* ld = sums + (size_t)(T / Q3_CHUNK + B) * H * N * P;
+  float* decays = ld + (size_t)T * H;
   Q3_DISPATCH_DTYPE(act_dtype, TA,
                     hipLaunchKernelGGL(mamba2_prepare_kernel<TA>, dim3(T), dim3(256), (size_t)H * sizeof(float), stream, (const TA*)xbc,
                                        (const TA*)dt, dt_stride, dt_bias, a_log, qf, kf, vf, ld, H, P, N, G));
-  const int status = launch_chunks(qf, kf, vf, ld, H, sums, decays, scores, state, state_stride, slots, cu, y, B, max_q_len, H,
-                                   H / G, N, P, stream);
-  if (status) return status;
-  Q3_DISPATCH_DTYPE(act_dtype, TA,
-                    hipLaunchKernelGGL(mamba2_skip_kernel<TA>, dim3(T), dim3(256), 0, stream, (const TA*)xbc, d_skip, y,
-                                       H, P, H * P + 2 * G * N));
+  Q3_DISPATCH_DTYPE(act_dtype, TA, return launch_chunks<TA>(qf, kf, vf, ld, H, sums, decays, scores, state, state_stride, slots,
+                                                            cu, y, B, max_q_len, H, H / G, N, P, (const TA*)xbc,
+                                                            (long)H * P + 2 * G * N, d_skip, stream));
   return q3_launch_status();
 }
 
@@ -990,14 +1004,13 @@ extern "C" int q3_retention_chunked(const void* rows, const float* inv_freq, int
   float* qf = scores + (size_t)(T / Q3_CHUNK + B) * H * Q3_CHUNK * Q3_CHUNK;
   float* kf = qf + (size_t)T * H * dim;
   float* vf = kf + (size_t)T * H * dim;
-  float* ld = vf + (size_t)T * H * vdim;          // unused stretch: the decays are one number per head
-  float* sums = ld + (size_t)T * H;
+  float* sums = vf + (size_t)T * H * vdim;
   float* decays = sums + (size_t)(T / Q3_CHUNK + B) * H * dim * vdim;
   Q3_DISPATCH_DTYPE(act_dtype, TA,
                     hipLaunchKernelGGL(retention_prepare_kernel<TA>, dim3(T), dim3(256), 0, stream, (const TA*)rows,
                                        inv_freq, half, positions, k_scale, qf, kf, vf, H, dim, vdim));
-  const int status = launch_chunks(qf, kf, vf, log_decays, 0, sums, decays, scores, state, state_stride, slots, cu, scratch_out,
-                                   B, max_q_len, H, 1, dim, vdim, stream);
+  const int status = launch_chunks<float>(qf, kf, vf, log_decays, 0, sums, decays, scores, state, state_stride, slots, cu,
+                                          scratch_out, B, max_q_len, H, 1, dim, vdim, nullptr, 0, nullptr, stream);
   if (status) return status;
   const int threads = vdim >= 256 ? 256 : (vdim >= 128 ? 128 : 64);
   Q3_DISPATCH_DTYPE(act_dtype, TA,
