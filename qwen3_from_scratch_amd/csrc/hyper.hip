@@ -115,6 +115,96 @@ __global__ void hyper_norm_kernel(float* __restrict__ x, const TA* __restrict__ 
   for (int j = threadIdx.x; j < W; j += blockDim.x) dst[j] = from_float<TA>((u_row[j] - mean) * inv * weight[j]);
 }
 
+// Four neighbouring numbers of either type in one access.
+__device__ inline void load_quad(const float* p, float (&v)[4]) {
+  const float4 a = *reinterpret_cast<const float4*>(p);
+  v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w;
+}
+__device__ inline void load_quad(const bf16_t* p, float (&v)[4]) {
+  union {
+    uint2 u;
+    bf16_t e[4];
+  } a;
+  a.u = *reinterpret_cast<const uint2*>(p);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = bf16_to_float(a.e[i]);
+}
+__device__ inline void store_quad(float* p, const float (&v)[4]) {
+  *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
+}
+__device__ inline void store_quad(bf16_t* p, const float (&v)[4]) {
+  union {
+    uint2 u;
+    bf16_t e[4];
+  } a;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) a.e[i] = float_to_bf16(v[i]);
+  *reinterpret_cast<uint2*>(p) = a.u;
+}
+
+// The same with four columns a thread and the whole row in a block (W a multiple of four up to 4,096, sixteen-byte
+// rows, STREAMS streams): the streams, what enters them, the tables and the norm's weight are all asked for at once and
+// u stays in registers. Few rows are bound by latency, where the kernel above waits for a table, a column of u and a
+// weight in turn: 8 rows of four streams of 2,048 take 4.9 us, there 9.0. Many are bound by memory: 2,048 such rows
+// (84 MB read, 76 written) 28 us, 5.7 TB/s, there 31. Other numbers of streams, widths and addresses stay with it.
+template <typename TA, int STREAMS>
+__global__ void __launch_bounds__(1024) hyper_norm_row_kernel(float* __restrict__ x, const TA* __restrict__ delta,
+                                                              const float* __restrict__ mix, const float* __restrict__ write,
+                                                              const float* __restrict__ read, const float* __restrict__ weight,
+                                                              const int* __restrict__ rows, TA* __restrict__ out, int W,
+                                                              float eps, int write_back) {
+  __shared__ float scratch[17];
+  const int r = blockIdx.x;
+  const size_t src = rows ? (size_t)rows[r] : (size_t)r;
+  const bool live = 4 * threadIdx.x < (unsigned)W;
+  const int j = live ? 4 * threadIdx.x : 0;      // a thread past the end reads column 0 and adds nothing
+  float* xs = x + src * STREAMS * W;
+  float4 old[STREAMS];
+#pragma unroll
+  for (int s = 0; s < STREAMS; ++s) old[s] = *reinterpret_cast<const float4*>(xs + (size_t)s * W + j);
+  const float4 w4 = out ? *reinterpret_cast<const float4*>(weight + j) : make_float4(0.f, 0.f, 0.f, 0.f);
+  float take[STREAMS];
+#pragma unroll
+  for (int s = 0; s < STREAMS; ++s) take[s] = read ? read[s] : 1.f;
+  float u[4] = {0.f, 0.f, 0.f, 0.f};
+  if (delta) {
+    float d[4], m[STREAMS * STREAMS], put[STREAMS];
+    load_quad(delta + src * W + j, d);
+#pragma unroll
+    for (int s = 0; s < STREAMS * STREAMS; ++s) m[s] = mix[s];
+#pragma unroll
+    for (int s = 0; s < STREAMS; ++s) put[s] = write[s];
+#pragma unroll
+    for (int t = 0; t < STREAMS; ++t) {
+      float v[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < STREAMS; ++s) {
+        const float by = m[s * STREAMS + t];
+        v[0] += by * old[s].x, v[1] += by * old[s].y, v[2] += by * old[s].z, v[3] += by * old[s].w;
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[e] += put[t] * d[e];
+        u[e] += take[t] * v[e];
+      }
+      if (write_back && live) *reinterpret_cast<float4*>(xs + (size_t)t * W + j) = make_float4(v[0], v[1], v[2], v[3]);
+    }
+  } else {
+#pragma unroll
+    for (int s = 0; s < STREAMS; ++s)
+      u[0] += take[s] * old[s].x, u[1] += take[s] * old[s].y, u[2] += take[s] * old[s].z, u[3] += take[s] * old[s].w;
+  }
+  if (!out) return;
+  const float mean = block_sum(live ? (u[0] + u[1]) + (u[2] + u[3]) : 0.f, scratch) / (float)W;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) u[e] -= mean;
+  const float inv =
+      rsqrtf(block_sum(live ? (u[0] * u[0] + u[1] * u[1]) + (u[2] * u[2] + u[3] * u[3]) : 0.f, scratch) / (float)W + eps);
+  if (!live) return;
+  const float v[4] = {u[0] * inv * w4.x, u[1] * inv * w4.y, u[2] * inv * w4.z, u[3] * inv * w4.w};
+  store_quad(out + (size_t)r * W + j, v);
+}
+
 // One block per (token, part): v = y * silu(gate); out = v * rsqrt(mean(v^2) + eps) * weight over
 // the part's `size` numbers. y float32 (T, inner); gate rows `gate_stride` apart.
 template <typename TA>
@@ -138,6 +228,32 @@ __global__ void gated_rmsnorm_kernel(const float* __restrict__ y, const TA* __re
     const float g = to_float(gr[j]);
     dst[j] = from_float<TA>(yr[j] * (g / (1.f + expf(-g))) * inv * w[j]);
   }
+}
+
+// The same with four numbers a thread and a whole part in a block (parts of a multiple of four up to 4,096, sixteen-byte
+// rows): every number is read, and its gate formed, once, where the kernel above does both twice and in a loop that waits
+// for each number: a part of 4,096 takes 4.8 us for 8 rows (there 14.5) and 17.9 for 2,048 rows (there 27; 67 MB,
+// bound by memory).
+template <typename TA>
+__global__ void __launch_bounds__(1024) gated_rmsnorm_row_kernel(const float* __restrict__ y, const TA* __restrict__ gate,
+                                                                 long gate_stride, const float* __restrict__ weight,
+                                                                 TA* __restrict__ out, int inner, int size, float eps) {
+  __shared__ float scratch[17];
+  const int t = blockIdx.x, part = blockIdx.y;
+  const bool live = 4 * threadIdx.x < (unsigned)size;
+  const size_t at = (size_t)part * size + (live ? 4 * threadIdx.x : 0);
+  float v[4], g[4], w[4];
+  load_quad(y + (size_t)t * inner + at, v);
+  load_quad(gate + (size_t)t * gate_stride + at, g);
+  load_quad(weight + at, w);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] *= g[e] / (1.f + expf(-g[e]));
+  const float sq = (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
+  const float inv = rsqrtf(block_sum(live ? sq : 0.f, scratch) / (float)size + eps);
+  if (!live) return;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = v[e] * inv * w[e];
+  store_quad(out + (size_t)t * inner + at, v);
 }
 
 template <typename TA>
@@ -165,7 +281,15 @@ extern "C" int q3_hyper_norm(float* x, const void* delta, const float* mix, cons
   if ((size_t)W * sizeof(float) > 60 * 1024) return Q3_ERR_UNSUPPORTED;
   if (delta && (!mix || !write)) return Q3_ERR_BAD_ARGUMENT;
   if (out && !weight) return Q3_ERR_BAD_ARGUMENT;
-  if (W % 4 == 0)
+  const size_t act_quad = act_dtype == Q3_F32 ? 15 : 7;
+  if (W % 4 == 0 && W <= 4096 && (S == 2 || S == 4) && (((size_t)x | (size_t)weight) & 15) == 0 &&
+      (((size_t)delta | (size_t)out) & act_quad) == 0) {
+    const dim3 threads((W / 4 + 63) / 64 * 64);
+    Q3_DISPATCH_DTYPE(act_dtype, TA,
+                      hipLaunchKernelGGL((S == 2 ? hyper_norm_row_kernel<TA, 2> : hyper_norm_row_kernel<TA, 4>), dim3(n_out),
+                                         threads, 0, stream, x, (const TA*)delta, mix, write, read, weight, rows, (TA*)out, W,
+                                         eps, write_back));
+  } else if (W % 4 == 0)
     Q3_DISPATCH_DTYPE(act_dtype, TA,
                       hipLaunchKernelGGL((hyper_norm_kernel<TA, 4>), dim3(n_out), dim3(W >= 2048 ? 512 : threads_for(W / 2)),
                                          (size_t)W * sizeof(float), stream, x, (const TA*)delta, mix, write, read, weight,
@@ -182,6 +306,14 @@ extern "C" int q3_gated_rmsnorm(const float* y, const void* gate, long gate_stri
                                 int T, int inner, int parts, float eps, int act_dtype, hipStream_t stream) {
   if (T <= 0 || inner <= 0 || parts <= 0 || inner % parts || parts > 65535) return Q3_ERR_BAD_ARGUMENT;
   const int size = inner / parts;
+  const size_t act_quad = act_dtype == Q3_F32 ? 15 : 7;
+  if (size % 4 == 0 && size <= 4096 && gate_stride % 4 == 0 && (((size_t)y | (size_t)weight) & 15) == 0 &&
+      (((size_t)gate | (size_t)out) & act_quad) == 0) {
+    Q3_DISPATCH_DTYPE(act_dtype, TA,
+                      hipLaunchKernelGGL(gated_rmsnorm_row_kernel<TA>, dim3(T, parts), dim3((size / 4 + 63) / 64 * 64), 0,
+                                         stream, y, (const TA*)gate, gate_stride, weight, (TA*)out, inner, size, eps));
+    return q3_launch_status();
+  }
   Q3_DISPATCH_DTYPE(act_dtype, TA,
                     hipLaunchKernelGGL(gated_rmsnorm_kernel<TA>, dim3(T, parts), dim3(threads_for(size)), 0, stream, y,
                                        (const TA*)gate, gate_stride, weight, (TA*)out, inner, size, eps));
