@@ -301,124 +301,6 @@ __global__ void __launch_bounds__(64) mamba2_scan_kernel(
   }
 }
 
-// ---- the recurrent unit's gates ----
-// out[g, t, b * bw + o] = sigmoid(bias[g, b, o] + sum_i w[g, b, i, o] * u[t, b * bw + i]) for the
-// two gates g, block-diagonal over `blocks` parts of bw numbers. A block of threads forms 64 tokens
-// by 64 outputs of one part and gate, over the inputs in slices of 64 that go through shared
-// memory (asked for in batches, as everywhere here); a thread holds 4 x 4 of them.
-#define Q3_GATE_TOKENS 8
-__global__ void __launch_bounds__(256) block_gates_kernel(const float* __restrict__ u, const float* __restrict__ w,
-                                                          const float* __restrict__ bias, float* __restrict__ out, int T,
-                                                          int width, int bw, int out_tiles) {
-  __shared__ float one[64 * 65];           // (token, input), rows padded
-  __shared__ __attribute__((aligned(16))) float two[64 * 64];           // (input, output)
-  const int t0 = blockIdx.x * 64;
-  const int b = blockIdx.y / out_tiles, o0 = (blockIdx.y % out_tiles) * 64, g = blockIdx.z;
-  const int blocks = width / bw;
-  const float* wb = w + ((size_t)g * blocks + b) * bw * bw;
-  const int tt = threadIdx.x / 16, tj = threadIdx.x % 16;      // tokens tt + 16 r, outputs 4 tj .. 4 tj + 3
-  float acc[4][4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r)
-#pragma unroll
-    for (int x = 0; x < 4; ++x) acc[r][x] = 0.f;
-  for (int i0 = 0; i0 < bw; i0 += 64) {
-    __syncthreads();
-    {
-      float gu[16], gw[16];
-#pragma unroll
-      for (int k = 0; k < 16; ++k) {
-        const int e = threadIdx.x + 256 * k;
-        const int s = e / 64, c = e % 64;
-        gu[k] = (t0 + s < T && i0 + c < bw) ? u[(size_t)(t0 + s) * width + b * bw + i0 + c] : 0.f;
-        gw[k] = (i0 + s < bw && o0 + c < bw) ? wb[(size_t)(i0 + s) * bw + o0 + c] : 0.f;
-      }
-#pragma unroll
-      for (int k = 0; k < 16; ++k) {
-        const int e = threadIdx.x + 256 * k;
-        one[(e / 64) * 65 + e % 64] = gu[k];
-        two[e] = gw[k];
-      }
-    }
-    __syncthreads();
-    for (int i = 0; i < 64; ++i) {
-      const float4 wv = *reinterpret_cast<const float4*>(two + i * 64 + 4 * tj);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float uv = one[(tt + 16 * r) * 65 + i];
-        acc[r][0] += uv * wv.x;
-        acc[r][1] += uv * wv.y;
-        acc[r][2] += uv * wv.z;
-        acc[r][3] += uv * wv.w;
-      }
-    }
-  }
-#pragma unroll
-  for (int x = 0; x < 4; ++x) {
-    const int o = o0 + 4 * tj + x;
-    if (o < bw) {
-      const float start = bias[((size_t)g * blocks + b) * bw + o];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int t = t0 + tt + 16 * r;
-        if (t < T) out[((size_t)g * T + t) * width + b * bw + o] = sigmoid_value(start + acc[r][x]);
-      }
-    }
-  }
-}
-
-// The same for steps of few rows, where the kernel above leaves most of the chip idle: a block
-// takes 64 outputs of one part and gate for eight tokens, its four quarters of threads each a
-// quarter of the inputs; the quarters' sums meet in shared memory in a fixed order.
-__global__ void __launch_bounds__(256) block_gates_few_kernel(const float* __restrict__ u, const float* __restrict__ w,
-                                                              const float* __restrict__ bias, float* __restrict__ out,
-                                                              int T, int width, int bw, int out_tiles) {
-  extern __shared__ float su[];          // (Q3_GATE_TOKENS, bw), then (4, 64, Q3_GATE_TOKENS) partial sums
-  float* part = su + Q3_GATE_TOKENS * bw;
-  const int t0 = blockIdx.x * Q3_GATE_TOKENS;
-  const int b = blockIdx.y / out_tiles, tile = blockIdx.y % out_tiles, g = blockIdx.z;
-  const int blocks = width / bw;
-  for (int i = threadIdx.x; i < Q3_GATE_TOKENS * bw; i += 256) {
-    const int tt = i / bw, e = i % bw;
-    su[i] = t0 + tt < T ? u[(size_t)(t0 + tt) * width + b * bw + e] : 0.f;
-  }
-  __syncthreads();
-  const int lane = threadIdx.x & 63, quarter = threadIdx.x >> 6;
-  const int o = tile * 64 + lane;
-  const int each = (bw + 3) / 4;
-  const int i0 = quarter * each, i1 = i0 + each < bw ? i0 + each : bw;
-  float acc[Q3_GATE_TOKENS];
-#pragma unroll
-  for (int tt = 0; tt < Q3_GATE_TOKENS; ++tt) acc[tt] = 0.f;
-  if (o < bw) {
-    const float* wb = w + ((size_t)g * blocks + b) * bw * bw + o;
-    // eight weights at a time, all asked for before any is used: the loop is a chain of memory round trips otherwise
-    for (int i = i0; i < i1; i += 8) {
-      float wv[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) wv[j] = i + j < i1 ? wb[(size_t)(i + j) * bw] : 0.f;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int at = i + j < i1 ? i + j : i0;
-#pragma unroll
-        for (int tt = 0; tt < Q3_GATE_TOKENS; ++tt) acc[tt] += wv[j] * su[tt * bw + at];
-      }
-    }
-  }
-#pragma unroll
-  for (int tt = 0; tt < Q3_GATE_TOKENS; ++tt) part[(quarter * 64 + lane) * Q3_GATE_TOKENS + tt] = acc[tt];
-  __syncthreads();
-  if (quarter == 0 && o < bw) {
-    const float start = bias[((size_t)g * blocks + b) * bw + o];
-#pragma unroll
-    for (int tt = 0; tt < Q3_GATE_TOKENS; ++tt) {
-      float total = start;
-      for (int qtr = 0; qtr < 4; ++qtr) total += part[(qtr * 64 + lane) * Q3_GATE_TOKENS + tt];
-      if (t0 + tt < T) out[((size_t)g * T + t0 + tt) * width + b * bw + o] = sigmoid_value(total);
-    }
-  }
-}
-
 // ---- the recurrent unit's recurrence ----
 // Per (sequence, channel): log a = -rate r, a = exp(log a), S = a S + sqrt(1 - a^2) i u (1 - a^2 as
 // -expm1(2 log a)), out = S * gelu_tanh(y + y_bias). gates = [r | i], each (T, width).
@@ -533,12 +415,16 @@ __device__ inline int chunks_before(const int* __restrict__ cu, int b) {
   return n;
 }
 
-// la of the chunk's rows, added up in order by one wavefront from a lane each (the caller's first; a loop of loads is
-// 64 round trips), and behind them, if asked for, exp(la_last - la_s), zero past the chunk's end.
-__device__ inline void chunk_decays(float* la, float* left, const float* __restrict__ ld, long ld_row, int h, int row0, int len) {
-  if (threadIdx.x >= 64) return;
-  const int lane = threadIdx.x;
-  const float own = lane < len ? ld[(size_t)(row0 + lane) * ld_row + h] : 0.f;
+// la of the chunk's rows, added up in order from a lane's `own` each (asked for before the caller's other loads; a loop
+// of loads is 64 round trips), and behind them, if asked for, exp(la_last - la_s), zero past the chunk's end. All
+// wavefronts do the same and write the same: behind a branch for one of them its wait would be for every load in flight.
+__device__ inline float own_decay(const float* __restrict__ ld, long ld_row, int h, int row0, int len) {
+  const int s = (int)(threadIdx.x & 63) < len ? threadIdx.x & 63 : 0;
+  return ld[(size_t)(row0 + s) * ld_row + h];
+}
+__device__ inline void chunk_decays(float* la, float* left, float own, int len) {
+  const int lane = threadIdx.x & 63;
+  own = lane < len ? own : 0.f;
   float run = 0.f, mine = 0.f;
 #pragma unroll
   for (int s = 0; s < Q3_CHUNK; ++s) {
@@ -551,16 +437,74 @@ __device__ inline void chunk_decays(float* la, float* left, const float* __restr
 
 // The chunk kernels' products run on the matrix cores (v_mfma_f32_16x16x4_f32: float32 operands and sums, one k after
 // the other, with the bits of a loop of multiply-adds). A wavefront's operands are single numbers from shared memory,
-// 16 neighbouring ones of four rows (row stride 16 more than a multiple of 64 numbers) or one number of sixteen rows
-// for four neighbouring k (row stride 4 more): either way all 64 banks. The columns are the first operand, so that a
-// lane holds four neighbouring columns of one row of the result.
+// 16 neighbouring ones of four rows (rows of 64 whose 16-wide quarters are swapped by the row, column_at) or one number
+// of sixteen rows for four neighbouring k (row stride 4 more than 64): either way all 64 banks. The columns are the
+// first operand, so that a lane holds four neighbouring columns of one row of the result.
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
-#define Q3_ROW16 80      // row strides of a 64-wide slice in the two layouts
 #define Q3_ROW4 68
 
-__device__ inline float4 load_four(const float* p, int there, bool whole) {   // p[0 .. 3], of which `there` exist
-  if (whole) return there > 0 ? *reinterpret_cast<const float4*>(p) : make_float4(0.f, 0.f, 0.f, 0.f);
-  return make_float4(there > 0 ? p[0] : 0.f, there > 1 ? p[1] : 0.f, there > 2 ? p[2] : 0.f, there > 3 ? p[3] : 0.f);
+// acc[x] += what 64 numbers k of the lane's row (r, k neighbouring) and of 16 x + col give; `columns` is a slice whose rows are k
+// (row stride 64, the 16-wide quarters of row k swapped by k % 4: see column_at). The next step's operands are asked for
+// before this step's products.
+__device__ inline int column_at(int k, int j) { return 64 * k + (j ^ (16 * (k & 3))); }
+__device__ inline void multiply_slice(f32x4_t (&acc)[4], const float* columns, const float* r, int col, int grp) {
+  const float* at[4];       // of k = grp; the lane's k are those that leave grp, so that the swap stays the same
+#pragma unroll
+  for (int x = 0; x < 4; ++x) at[x] = columns + column_at(grp, 16 * x + col);
+  float mine = r[grp], other[4];
+#pragma unroll
+  for (int x = 0; x < 4; ++x) other[x] = at[x][0];
+#pragma unroll
+  for (int k = 0; k < 64; k += 4) {
+    float next = 0.f, following[4] = {0.f, 0.f, 0.f, 0.f};
+    if (k + 4 < 64) {
+      next = r[k + 4 + grp];
+#pragma unroll
+      for (int x = 0; x < 4; ++x) following[x] = at[x][64 * (k + 4)];
+    }
+#pragma unroll
+    for (int x = 0; x < 4; ++x) acc[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(other[x], mine, acc[x], 0, 0, 0);
+    mine = next;
+#pragma unroll
+    for (int x = 0; x < 4; ++x) other[x] = following[x];
+  }
+}
+
+// Four numbers of a row of `width` from column i on. WHOLE (widths of a multiple of four, sixteen-byte rows): one access.
+// A load never waits behind a branch (the compiler drains all loads in flight there): past the end it reads the row's
+// first numbers, and `kept_four` puts zeros in their place where the numbers are used.
+template <bool WHOLE>
+__device__ inline float4 load_four(const float* __restrict__ row, int i, int width) {
+  if (WHOLE) return *reinterpret_cast<const float4*>(row + (i < width ? i : 0));
+  return make_float4(row[i < width ? i : 0], row[i + 1 < width ? i + 1 : 0], row[i + 2 < width ? i + 2 : 0],
+                     row[i + 3 < width ? i + 3 : 0]);
+}
+// The same of either type, left as it comes until it is used.
+template <typename TA>
+struct Four {
+  TA of[4];
+  template <bool WHOLE>
+  __device__ void load(const TA* __restrict__ row, int i, int width) {
+    if constexpr (WHOLE) {
+      typedef typename std::conditional<sizeof(TA) == 2, uint2, uint4>::type Raw;
+      union {
+        Raw raw;
+        TA of[4];
+      } got;
+      got.raw = *reinterpret_cast<const Raw*>(row + (i < width ? i : 0));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) of[e] = got.of[e];
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) of[e] = row[i + e < width ? i + e : 0];
+    }
+  }
+};
+template <bool WHOLE>
+__device__ inline float4 kept_four(const float4& v, int i, int width, bool row) {
+  const int there = row ? width - i : 0;
+  if (WHOLE) return make_float4(there > 0 ? v.x : 0.f, there > 0 ? v.y : 0.f, there > 0 ? v.z : 0.f, there > 0 ? v.w : 0.f);
+  return make_float4(there > 0 ? v.x : 0.f, there > 1 ? v.y : 0.f, there > 2 ? v.z : 0.f, there > 3 ? v.w : 0.f);
 }
 __device__ inline void store_four(float* p, const f32x4_t& v, int there, bool whole) {
   if (whole) {
@@ -572,21 +516,50 @@ __device__ inline void store_four(float* p, const f32x4_t& v, int there, bool wh
   }
 }
 
+// A slice of 64 numbers of 64 rows (from column `from` of `width`, rows `row_stride` apart, the first `count` >= 1 of which
+// exist) on its way, four pieces a thread, and into shared memory.
+template <bool WHOLE>
+__device__ inline void load_slice(float4 (&got)[4], const float* __restrict__ rows, size_t row_stride, int count, int from,
+                                  int width) {
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int e = threadIdx.x + 256 * u, s = e / 16;
+    got[u] = load_four<WHOLE>(rows + (s < count ? s : 0) * row_stride, from + 4 * (e % 16), width);
+  }
+}
+template <bool WHOLE>
+__device__ inline void store_columns(float* to, const float4 (&got)[4], int count, int from, int width) {   // as column_at
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int e = threadIdx.x + 256 * u, s = e / 16, i = 4 * (e % 16);
+    *reinterpret_cast<float4*>(to + column_at(s, i)) = kept_four<WHOLE>(got[u], from + i, width, s < count);
+  }
+}
+template <bool WHOLE>
+__device__ inline void store_slice(float* to, int row, const float4 (&got)[4], int count, int from, int width) {
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int e = threadIdx.x + 256 * u, s = e / 16, i = 4 * (e % 16);
+    *reinterpret_cast<float4*>(to + s * row + i) = kept_four<WHOLE>(got[u], from + i, width, s < count);
+  }
+}
+
 // grid (chunks of the longest sequence, H * dv tiles of 64, B); 256 threads. U[i][j] = sum_s
 // exp(la_last - la_s) k_s[i] v_s[j] for the tile's 64 columns j, into `sums` (chunk, H, d, dv); the chunk's
 // whole decay exp(la_last) into `decays` (chunk, H). d up to 64 MT; a wavefront takes 16 MT rows i.
 //
 // Bound by the passage of k, v and the sums through the caches (48 KB in, 32 KB out per block at d 128). 2,048 tokens,
-// 64 heads of 64 columns, d 128: 136 us with 8 x 8 multiply-adds a thread and one thread adding up the decays, 50 now.
-template <int MT>
+// 64 heads of 64 columns, d 128: 136 us with 8 x 8 multiply-adds a thread and one thread adding up the decays, 48 with loads
+// that each waited behind a branch and padded rows (two blocks a compute unit), 41 now.
+template <int MT, bool WHOLE>
 __global__ void __launch_bounds__(256) chunk_state_kernel(const float* __restrict__ k, const float* __restrict__ v,
                                                           const float* __restrict__ ld, long ld_row,
                                                           const int* __restrict__ cu, float* __restrict__ sums,
                                                           float* __restrict__ decays, int H, int hpg, int d, int dv) {
-  constexpr int KS = 64 * MT + 16;
+  constexpr int KS = 64 * MT;
   extern __shared__ __attribute__((aligned(16))) float lds[];
-  float* kw = lds;                          // (64, KS)
-  float* vt = kw + Q3_CHUNK * KS;           // (64, Q3_ROW16)
+  float* kw = lds;                          // (64, KS) and (64, 64), the quarters of every 64 numbers swapped as in column_at
+  float* vt = kw + Q3_CHUNK * KS;
   __shared__ float la[Q3_CHUNK], left[Q3_CHUNK];
   const int b = blockIdx.z;
   const int tiles = (dv + 63) / 64;
@@ -599,35 +572,27 @@ __global__ void __launch_bounds__(256) chunk_state_kernel(const float* __restric
   const int chunk = chunks_before(cu, b) + c;
   const int G = H / hpg, g = h / hpg;
   const int t = threadIdx.x;
-  const bool whole_k = d % 4 == 0 && ((size_t)k & 15) == 0;
-  const bool whole_v = dv % 4 == 0 && (((size_t)v | (size_t)sums) & 15) == 0;
   const int pieces = (d + 3) / 4;           // of four numbers in a row of k
   float4 gk[4 * MT], gv[4];
+  const float own = own_decay(ld, ld_row, h, row0, len);
 #pragma unroll
   for (int u = 0; u < 4 * MT; ++u) {
     const int e = t + 256 * u, s = e / pieces, i = 4 * (e - s * pieces);
-    gk[u] = load_four(k + ((size_t)(row0 + s) * G + g) * d + i, s < len ? d - i : 0, whole_k);
+    gk[u] = load_four<WHOLE>(k + ((size_t)(row0 + (s < len ? s : 0)) * G + g) * d, i, d);
   }
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int e = t + 256 * u, s = e / 16, j = tile * 64 + 4 * (e % 16);
-    gv[u] = load_four(v + ((size_t)(row0 + s) * H + h) * dv + j, s < len ? dv - j : 0, whole_v);
-  }
-  chunk_decays(la, left, ld, ld_row, h, row0, len);
+  load_slice<WHOLE>(gv, v + ((size_t)row0 * H + h) * dv, (size_t)H * dv, len, tile * 64, dv);
+  __builtin_amdgcn_sched_barrier(0);        // all loads go out before the first is waited for
+  chunk_decays(la, left, own, len);
   __syncthreads();
 #pragma unroll
   for (int u = 0; u < 4 * MT; ++u) {
     const int e = t + 256 * u, s = e / pieces, i = 4 * (e - s * pieces);
-    if (s < Q3_CHUNK) {
-      const float w = left[s];
-      *reinterpret_cast<float4*>(kw + s * KS + i) = make_float4(gk[u].x * w, gk[u].y * w, gk[u].z * w, gk[u].w * w);
-    }
+    const float w = left[s < Q3_CHUNK ? s : 0];
+    const float4 kept = kept_four<WHOLE>(gk[u], i, d, s < len);
+    if (s < Q3_CHUNK)
+      *reinterpret_cast<float4*>(kw + s * KS + (i ^ (16 * (s & 3)))) = make_float4(kept.x * w, kept.y * w, kept.z * w, kept.w * w);
   }
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int e = t + 256 * u;
-    *reinterpret_cast<float4*>(vt + (e / 16) * Q3_ROW16 + 4 * (e % 16)) = gv[u];
-  }
+  store_columns<WHOLE>(vt, gv, len, tile * 64, dv);
   __syncthreads();
   const int lane = t & 63, wave = t >> 6, col = lane & 15, grp = lane >> 4;
   f32x4_t acc[MT][4];
@@ -639,9 +604,9 @@ __global__ void __launch_bounds__(256) chunk_state_kernel(const float* __restric
   for (int s0 = 0; s0 < Q3_CHUNK; s0 += 4) {
     float vv[4], kk[MT];
 #pragma unroll
-    for (int x = 0; x < 4; ++x) vv[x] = vt[(s0 + grp) * Q3_ROW16 + 16 * x + col];
+    for (int x = 0; x < 4; ++x) vv[x] = vt[column_at(grp, 16 * x + col) + 64 * s0];
 #pragma unroll
-    for (int m = 0; m < MT; ++m) kk[m] = kw[(s0 + grp) * KS + 16 * (wave * MT + m) + col];
+    for (int m = 0; m < MT; ++m) kk[m] = kw[(s0 + grp) * KS + ((16 * (wave * MT + m) + col) ^ (16 * grp))];
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -655,7 +620,7 @@ __global__ void __launch_bounds__(256) chunk_state_kernel(const float* __restric
 #pragma unroll
       for (int x = 0; x < 4; ++x) {
         const int j = tile * 64 + 16 * x + 4 * grp;
-        store_four(dst + (size_t)i * dv + j, acc[m][x], dv - j, whole_v);
+        store_four(dst + (size_t)i * dv + j, acc[m][x], dv - j, WHOLE);
       }
     }
   }
@@ -686,27 +651,10 @@ __global__ void chunk_scan_kernel(float* __restrict__ sums, const float* __restr
   *mine = S;
 }
 
-// A slice of 64 numbers of 64 rows (from column `from` of `width`, rows `row_stride` apart) on its way: four pieces a thread.
-__device__ inline void load_slice(float4 (&got)[4], const float* __restrict__ rows, size_t row_stride, int count, int from,
-                                  int width) {
-  const bool whole = width % 4 == 0 && row_stride % 4 == 0 && ((size_t)rows & 15) == 0;
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int e = threadIdx.x + 256 * u, s = e / 16, i = from + 4 * (e % 16);
-    got[u] = load_four(rows + s * row_stride + i, s < count ? width - i : 0, whole);
-  }
-}
-__device__ inline void store_slice(float* to, int row, const float4 (&got)[4]) {
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int e = threadIdx.x + 256 * u;
-    *reinterpret_cast<float4*>(to + (e / 16) * row + 4 * (e % 16)) = got[u];
-  }
-}
-
 // grid (chunks of the longest sequence, groups, B): the chunk's raw products q_t . k_s (64 x 64), over d in
 // slices of 64 through shared memory, into `scores` (chunk, group, t, s). They are the same for all heads of a
 // group and all tiles of a head's columns, which only weigh them with their own decays. A wavefront takes 16 rows t.
+template <bool WHOLE>
 __global__ void __launch_bounds__(256) chunk_scores_kernel(const float* __restrict__ q, const float* __restrict__ k,
                                                            const int* __restrict__ cu, float* __restrict__ scores, int G,
                                                            int d) {
@@ -720,20 +668,21 @@ __global__ void __launch_bounds__(256) chunk_scores_kernel(const float* __restri
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, grp = lane >> 4;
   const float *qr = q + ((size_t)row0 * G + g) * d, *kr = k + ((size_t)row0 * G + g) * d;
   float4 gq[4], gk[4];
-  load_slice(gq, qr, (size_t)G * d, len, 0, d);
-  load_slice(gk, kr, (size_t)G * d, len, 0, d);
+  load_slice<WHOLE>(gq, qr, (size_t)G * d, len, 0, d);
+  load_slice<WHOLE>(gk, kr, (size_t)G * d, len, 0, d);
   f32x4_t acc[4];
 #pragma unroll
   for (int x = 0; x < 4; ++x) acc[x] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   for (int i0 = 0; i0 < d; i0 += 64) {
     __syncthreads();
-    store_slice(one, Q3_ROW4, gq);
-    store_slice(two, Q3_ROW4, gk);
+    store_slice<WHOLE>(one, Q3_ROW4, gq, len, i0, d);
+    store_slice<WHOLE>(two, Q3_ROW4, gk, len, i0, d);
     __syncthreads();
     if (i0 + 64 < d) {
-      load_slice(gq, qr, (size_t)G * d, len, i0 + 64, d);
-      load_slice(gk, kr, (size_t)G * d, len, i0 + 64, d);
+      load_slice<WHOLE>(gq, qr, (size_t)G * d, len, i0 + 64, d);
+      load_slice<WHOLE>(gk, kr, (size_t)G * d, len, i0 + 64, d);
     }
+    __builtin_amdgcn_sched_barrier(0);      // the loads go out before the products
 #pragma unroll 4
     for (int i = 0; i < 64; i += 4) {
       const float qv = one[(16 * wave + col) * Q3_ROW4 + i + grp];
@@ -753,9 +702,10 @@ __global__ void __launch_bounds__(256) chunk_scores_kernel(const float* __restri
 // `skip_x` (rows of `skip_stride`; Mamba-2): o[t][j] += skip[h] x_t[h dv + j], D x in the recurrence's terms.
 // A wavefront takes 16 rows t.
 //
-// Bound like chunk_state_kernel (q, S, v and the scores in, the results out): the same rows 112 us before and 15 for a
-// kernel of its own that added D x, 82 now.
-template <typename TA>
+// Bound like chunk_state_kernel (q, S, v and the scores in, the results out): the same rows 112 us with multiply-adds and
+// 15 for a kernel of its own that added D x, 82 with loads that waited behind branches (x for D x the longest chain of
+// them), 48 now.
+template <typename TA, bool WHOLE>
 __global__ void __launch_bounds__(256) chunk_output_kernel(const float* __restrict__ q, const float* __restrict__ scores,
                                                            const float* __restrict__ v, const float* __restrict__ ld,
                                                            long ld_row, const int* __restrict__ cu,
@@ -764,8 +714,8 @@ __global__ void __launch_bounds__(256) chunk_output_kernel(const float* __restri
                                                            long skip_stride, const float* __restrict__ skip) {
   __shared__ __attribute__((aligned(16))) float A[Q3_CHUNK * Q3_ROW4];       // (t, s)
   __shared__ __attribute__((aligned(16))) float one[Q3_CHUNK * Q3_ROW4];     // a slice of q
-  __shared__ __attribute__((aligned(16))) float two[Q3_CHUNK * Q3_ROW16];    // a slice of S, then v
-  __shared__ float la[Q3_CHUNK];
+  __shared__ __attribute__((aligned(16))) float two[Q3_CHUNK * 64];          // a slice of S, then v
+  __shared__ __attribute__((aligned(16))) float la[Q3_CHUNK];
   const int b = blockIdx.z;
   const int tiles = (dv + 63) / 64;
   const int h = blockIdx.y / tiles, tile = blockIdx.y % tiles;
@@ -781,69 +731,188 @@ __global__ void __launch_bounds__(256) chunk_output_kernel(const float* __restri
   const float* S = sums + ((size_t)chunk * H + h) * d * dv;
   const float* raw = scores + ((size_t)chunk * G + g) * Q3_CHUNK * Q3_CHUNK;
   float4 gq[4], gs[4], ga[4];
-  load_slice(gq, qr, (size_t)G * d, len, 0, d);
-  load_slice(gs, S, dv, d, tile * 64, dv);
-  load_slice(ga, raw, Q3_CHUNK, Q3_CHUNK, 0, Q3_CHUNK);
-  chunk_decays(la, nullptr, ld, ld_row, h, row0, len);
+  const float own = own_decay(ld, ld_row, h, row0, len);
+  load_slice<true>(ga, raw, Q3_CHUNK, Q3_CHUNK, 0, Q3_CHUNK);
+  load_slice<WHOLE>(gq, qr, (size_t)G * d, len, 0, d);
+  load_slice<WHOLE>(gs, S, dv, d, tile * 64, dv);
+  __builtin_amdgcn_sched_barrier(0);        // all loads go out before the first is waited for
+  chunk_decays(la, nullptr, own, len);
   __syncthreads();
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     const int e = threadIdx.x + 256 * u, t = e / 16, s = 4 * (e % 16);
-    const float at = la[t], got[4] = {ga[u].x, ga[u].y, ga[u].z, ga[u].w};
-    float4 w;
-    w.x = (s <= t && t < len) ? got[0] * expf(at - la[s]) : 0.f;
-    w.y = (s + 1 <= t && t < len) ? got[1] * expf(at - la[s + 1]) : 0.f;
-    w.z = (s + 2 <= t && t < len) ? got[2] * expf(at - la[s + 2]) : 0.f;
-    w.w = (s + 3 <= t && t < len) ? got[3] * expf(at - la[s + 3]) : 0.f;
-    *reinterpret_cast<float4*>(A + t * Q3_ROW4 + s) = w;
+    const float4 las = *reinterpret_cast<const float4*>(la + s);
+    const float at = la[t], got[4] = {ga[u].x, ga[u].y, ga[u].z, ga[u].w}, from[4] = {las.x, las.y, las.z, las.w};
+    float w[4];
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      const bool kept = s + x <= t && t < len;
+      const float grown = expf(kept ? at - from[x] : 0.f);      // (of the others' differences none is taken: no branch)
+      w[x] = kept ? got[x] * grown : 0.f;
+    }
+    *reinterpret_cast<float4*>(A + t * Q3_ROW4 + s) = make_float4(w[0], w[1], w[2], w[3]);
   }
   f32x4_t acc[4];
 #pragma unroll
   for (int x = 0; x < 4; ++x) acc[x] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   const int my_row = 16 * wave + col;
-  auto multiply = [&](const float* rows) {
-#pragma unroll 4
-    for (int i = 0; i < 64; i += 4) {
-      const float r = rows[my_row * Q3_ROW4 + i + grp];
-#pragma unroll
-      for (int x = 0; x < 4; ++x)
-        acc[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(two[(i + grp) * Q3_ROW16 + 16 * x + col], r, acc[x], 0, 0, 0);
-    }
-  };
   for (int i0 = 0; i0 < d; i0 += 64) {
     if (i0) __syncthreads();
-    store_slice(one, Q3_ROW4, gq);
-    store_slice(two, Q3_ROW16, gs);
+    store_slice<WHOLE>(one, Q3_ROW4, gq, len, i0, d);
+    store_columns<WHOLE>(two, gs, d - i0, tile * 64, dv);
     __syncthreads();
     if (i0 + 64 < d) {
-      load_slice(gq, qr, (size_t)G * d, len, i0 + 64, d);
-      load_slice(gs, S + (size_t)(i0 + 64) * dv, dv, d - i0 - 64, tile * 64, dv);
+      load_slice<WHOLE>(gq, qr, (size_t)G * d, len, i0 + 64, d);
+      load_slice<WHOLE>(gs, S + (size_t)(i0 + 64) * dv, dv, d - i0 - 64, tile * 64, dv);
     } else {
-      load_slice(gs, v + ((size_t)row0 * H + h) * dv, (size_t)H * dv, len, tile * 64, dv);
+      load_slice<WHOLE>(gs, v + ((size_t)row0 * H + h) * dv, (size_t)H * dv, len, tile * 64, dv);
     }
-    multiply(one);
+    __builtin_amdgcn_sched_barrier(0);      // the loads go out before the products
+    multiply_slice(acc, two, one + my_row * Q3_ROW4, col, grp);
   }
   const float grow = expf(la[my_row]);
 #pragma unroll
   for (int x = 0; x < 4; ++x) acc[x] *= grow;
   __syncthreads();
-  store_slice(two, Q3_ROW16, gs);
+  store_columns<WHOLE>(two, gs, len, tile * 64, dv);
   __syncthreads();
-  multiply(A);
+  Four<TA> skipped[4];
+  float by = 0.f;
+  if (skip_x) {
+    const TA* at = skip_x + (size_t)(row0 + (my_row < len ? my_row : 0)) * skip_stride + (size_t)h * dv;
+#pragma unroll
+    for (int x = 0; x < 4; ++x) skipped[x].template load<WHOLE>(at, tile * 64 + 16 * x + 4 * grp, dv);
+    by = skip[h];
+  }
+  multiply_slice(acc, two, A + my_row * Q3_ROW4, col, grp);
   if (my_row < len) {
     const bool whole = dv % 4 == 0 && ((size_t)out & 15) == 0;
 #pragma unroll
     for (int x = 0; x < 4; ++x) {
       const int j = tile * 64 + 16 * x + 4 * grp;
       if (skip_x) {
-        const TA* at = skip_x + (size_t)(row0 + my_row) * skip_stride + (size_t)h * dv + j;
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (j + e < dv) acc[x][e] += skip[h] * to_float(at[e]);
+        for (int e = 0; e < 4; ++e) acc[x][e] += by * to_float(skipped[x].of[e]);      // (past dv: not stored)
       }
       store_four(out + ((size_t)(row0 + my_row) * H + h) * dv + j, acc[x], dv - j, whole);
     }
   }
+}
+
+// ---- the recurrent unit's gates ----
+// out[g, t, b * bw + o] = sigmoid(bias[g, b, o] + sum_i w[g, b, i, o] * u[t, b * bw + i]) for the
+// two gates g, block-diagonal over `blocks` parts of bw numbers. A block of threads forms 64 tokens by 64 outputs of
+// one part and gate, over the inputs in slices of 64 that go through shared memory as in the kernels above, the next
+// slice on its way to registers meanwhile; a wavefront takes 16 tokens.
+//
+// Bound by the matrix cores' float32 rate and the slices' passage: 2,048 tokens of 8 parts of 256 (4.3 GFLOP) in
+// 54 us, 89 with 4 x 4 multiply-adds a thread; 512 tokens 17 us (there 31), 128 tokens 10 (25).
+template <bool WHOLE>
+__global__ void __launch_bounds__(256) block_gates_kernel(const float* __restrict__ u, const float* __restrict__ w,
+                                                          const float* __restrict__ bias, float* __restrict__ out, int T,
+                                                          int width, int bw, int out_tiles) {
+  __shared__ __attribute__((aligned(16))) float one[64 * Q3_ROW4];      // (token, input)
+  __shared__ __attribute__((aligned(16))) float two[64 * 64];           // (input, output)
+  const int t0 = blockIdx.x * 64;
+  const int b = blockIdx.y / out_tiles, o0 = (blockIdx.y % out_tiles) * 64, g = blockIdx.z;
+  const int blocks = width / bw;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, grp = lane >> 4;
+  const float* ub = u + (size_t)t0 * width + b * bw;
+  const float* wb = w + ((size_t)g * blocks + b) * bw * bw;
+  float4 gu[4], gw[4], start[4];
+  const float* own_bias = bias + ((size_t)g * blocks + b) * bw;
+#pragma unroll
+  for (int x = 0; x < 4; ++x) start[x] = load_four<WHOLE>(own_bias, o0 + 16 * x + 4 * grp, bw);
+  load_slice<WHOLE>(gu, ub, width, T - t0, 0, bw);
+  load_slice<WHOLE>(gw, wb, bw, bw, o0, bw);
+  f32x4_t acc[4];
+#pragma unroll
+  for (int x = 0; x < 4; ++x) acc[x] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int i0 = 0; i0 < bw; i0 += 64) {
+    if (i0) __syncthreads();
+    store_slice<WHOLE>(one, Q3_ROW4, gu, T - t0, i0, bw);
+    store_columns<WHOLE>(two, gw, bw - i0, o0, bw);
+    __syncthreads();
+    if (i0 + 64 < bw) {
+      load_slice<WHOLE>(gu, ub, width, T - t0, i0 + 64, bw);
+      load_slice<WHOLE>(gw, wb + (size_t)(i0 + 64) * bw, bw, bw - i0 - 64, o0, bw);
+    }
+    __builtin_amdgcn_sched_barrier(0);      // the loads go out before the products
+    multiply_slice(acc, two, one + (16 * wave + col) * Q3_ROW4, col, grp);
+  }
+  const int t = t0 + 16 * wave + col;
+  if (t >= T) return;
+  const bool whole = bw % 4 == 0 && ((size_t)out & 15) == 0;
+#pragma unroll
+  for (int x = 0; x < 4; ++x) {
+    const int o = o0 + 16 * x + 4 * grp;
+    acc[x][0] = sigmoid_value(start[x].x + acc[x][0]);
+    acc[x][1] = sigmoid_value(start[x].y + acc[x][1]);
+    acc[x][2] = sigmoid_value(start[x].z + acc[x][2]);
+    acc[x][3] = sigmoid_value(start[x].w + acc[x][3]);
+    store_four(out + ((size_t)g * T + t) * width + b * bw + o, acc[x], bw - o, whole);
+  }
+}
+
+// The same for steps of few rows, where the weights' passage is the work: a block takes 16 outputs of one part and gate
+// for 16 tokens, each of its wavefronts a quarter of every 256 inputs, straight from memory: 16 rows of 64 bytes a load
+// of weights, all loads of a turn asked for before the first is used. The four sums meet in shared memory in a fixed
+// order. In a matrix step lane group k holds input 16 q + 4 k + e (q, e the step's), so that u comes four at a time.
+//
+// 8 tokens of 8 parts of 256 (4.2 MB of weights) 4.3 us, 15 with eight tokens and 64 outputs a block and a quarter of the
+// inputs a thread. Its work is weights and inputs from the caches, 1 / 16 of it per token, that of the kernel above
+// nearly constant up to some hundred tokens (10 us at a part of 256, 28 at 1,024): at a width of 2,048 they cross
+// between 48 (9.0 and 9.7 us) and 64 tokens (10.8 and 9.8), at 4,096 below 32 (34.8 and 28.5), at 1,536 behind 64 (38.3
+// and 39.8).
+#define Q3_GATES_FEW (96 * 1024)      // tokens times width
+__global__ void __launch_bounds__(256) block_gates_few_kernel(const float* __restrict__ u, const float* __restrict__ w,
+                                                              const float* __restrict__ bias, float* __restrict__ out,
+                                                              int T, int width, int bw, int out_tiles) {
+  __shared__ __attribute__((aligned(16))) float part[4][64][4];
+  const int t0 = blockIdx.x * 16;
+  const int b = blockIdx.y / out_tiles, o0 = (blockIdx.y % out_tiles) * 16, g = blockIdx.z;
+  const int blocks = width / bw;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, grp = lane >> 4;
+  const bool token = t0 + col < T, output = o0 + col < bw;
+  const float* ub = u + (size_t)(token ? t0 + col : 0) * width + b * bw;
+  const float* wb = w + ((size_t)g * blocks + b) * bw * bw + (output ? o0 + col : 0);
+  const bool whole = bw % 4 == 0 && ((size_t)u & 15) == 0;      // (width is a multiple of bw)
+  // a thread's own output and token at the end: lane 16 (o / 4) + t of the products, number o % 4
+  const int t = threadIdx.x >> 4, o = threadIdx.x & 15;
+  const bool mine = t0 + t < T && o0 + o < bw;
+  float total = bias[((size_t)g * blocks + b) * bw + (mine ? o0 + o : 0)];
+  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+  for (int i0 = 64 * wave; i0 < bw; i0 += 256) {
+    float wv[4][4], uv[4][4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int i = i0 + 16 * q + 4 * grp;
+      // inputs past the end: a place that exists, and zeros behind the load
+#pragma unroll
+      for (int e = 0; e < 4; ++e) wv[q][e] = wb[(size_t)(i + e < bw ? i + e : 0) * bw];
+      if (whole) {
+        const float4 four = *reinterpret_cast<const float4*>(ub + (i < bw ? i : 0));
+        uv[q][0] = four.x, uv[q][1] = four.y, uv[q][2] = four.z, uv[q][3] = four.w;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) uv[q][e] = ub[i + e < bw ? i + e : 0];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int i = i0 + 16 * q + 4 * grp;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(output && i + e < bw ? wv[q][e] : 0.f, token && i + e < bw ? uv[q][e] : 0.f,
+                                                   acc, 0, 0, 0);
+    }
+  }
+  *reinterpret_cast<f32x4_t*>(part[wave][lane]) = acc;
+  __syncthreads();
+  if (!mine) return;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) total += part[k][16 * (o / 4) + t][o % 4];
+  out[((size_t)g * T + t0 + t) * width + b * bw + o0 + o] = sigmoid_value(total);
 }
 
 // What the three kernels need of Mamba-2's rows: step = softplus(dt + dt_bias); ld = -exp(A_log) step;
@@ -931,23 +1000,23 @@ extern "C" long q3_chunked_workspace(int T, int B, int H, int G, int d, int dv) 
   return 2L * T * G * d + (long)T * H * dv + (long)T * H + chunks * H * ((long)d * dv + 1) + chunks * G * Q3_CHUNK * Q3_CHUNK;
 }
 
-template <int MT>
+template <int MT, bool WHOLE>
 static int launch_chunk_states(const float* kf, const float* vf, const float* ld, long ld_row, const int* cu, float* sums,
                                float* decays, dim3 grid, int H, int hpg, int d, int dv, hipStream_t stream) {
-  const size_t lds = (size_t)Q3_CHUNK * (64 * MT + 16 + Q3_ROW16) * sizeof(float);
+  const size_t lds = (size_t)Q3_CHUNK * (64 * MT + 64) * sizeof(float);
   if (lds > 64 * 1024) {
     // (from keys of 129 numbers on) more than the 64 KB a launch may ask for unasked
-    const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(chunk_state_kernel<MT>),
+    const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>((chunk_state_kernel<MT, WHOLE>)),
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (allowed != hipSuccess) return (int)allowed;
   }
-  hipLaunchKernelGGL(chunk_state_kernel<MT>, grid, dim3(256), lds, stream, kf, vf, ld, ld_row, cu, sums, decays, H, hpg, d, dv);
+  hipLaunchKernelGGL((chunk_state_kernel<MT, WHOLE>), grid, dim3(256), lds, stream, kf, vf, ld, ld_row, cu, sums, decays, H, hpg, d, dv);
   return q3_launch_status();
 }
 
 // `skip_x`, `skip_stride`, `skip`: see chunk_output_kernel. d up to 256.
-template <typename TA>
-static int launch_chunks(const float* qf, const float* kf, const float* vf, const float* ld, long ld_row, float* sums,
+template <typename TA, bool WHOLE>
+static int launch_whole_chunks(const float* qf, const float* kf, const float* vf, const float* ld, long ld_row, float* sums,
                          float* decays, float* scores, float* state, long state_stride, const int* slots, const int* cu, float* out,
                          int B, int max_q_len, int H, int hpg, int d, int dv, const TA* skip_x, long skip_stride,
                          const float* skip, hipStream_t stream) {
@@ -955,16 +1024,29 @@ static int launch_chunks(const float* qf, const float* kf, const float* vf, cons
   const int tiles = (dv + 63) / 64;
   const dim3 grid(chunks, H * tiles, B);
   const int status =
-      d <= 64 ? launch_chunk_states<1>(kf, vf, ld, ld_row, cu, sums, decays, grid, H, hpg, d, dv, stream)
-      : d <= 128 ? launch_chunk_states<2>(kf, vf, ld, ld_row, cu, sums, decays, grid, H, hpg, d, dv, stream)
-                 : launch_chunk_states<4>(kf, vf, ld, ld_row, cu, sums, decays, grid, H, hpg, d, dv, stream);
+      d <= 64 ? launch_chunk_states<1, WHOLE>(kf, vf, ld, ld_row, cu, sums, decays, grid, H, hpg, d, dv, stream)
+      : d <= 128 ? launch_chunk_states<2, WHOLE>(kf, vf, ld, ld_row, cu, sums, decays, grid, H, hpg, d, dv, stream)
+                 : launch_chunk_states<4, WHOLE>(kf, vf, ld, ld_row, cu, sums, decays, grid, H, hpg, d, dv, stream);
   if (status) return status;
   hipLaunchKernelGGL(chunk_scan_kernel, dim3((d * dv + 255) / 256, H, B), dim3(256), 0, stream, sums, decays, state,
                      state_stride, slots, cu, H, d * dv);
-  hipLaunchKernelGGL(chunk_scores_kernel, dim3(chunks, H / hpg, B), dim3(256), 0, stream, qf, kf, cu, scores, H / hpg, d);
-  hipLaunchKernelGGL(chunk_output_kernel<TA>, grid, dim3(256), 0, stream, qf, scores, vf, ld, ld_row, cu, sums, out, H, hpg, d,
+  hipLaunchKernelGGL(chunk_scores_kernel<WHOLE>, dim3(chunks, H / hpg, B), dim3(256), 0, stream, qf, kf, cu, scores, H / hpg, d);
+  hipLaunchKernelGGL((chunk_output_kernel<TA, WHOLE>), grid, dim3(256), 0, stream, qf, scores, vf, ld, ld_row, cu, sums, out, H, hpg, d,
                      dv, skip_x, skip_stride, skip);
   return q3_launch_status();
+}
+
+// Rows that can be read sixteen bytes at a time, or not.
+template <typename TA>
+static int launch_chunks(const float* qf, const float* kf, const float* vf, const float* ld, long ld_row, float* sums,
+                         float* decays, float* scores, float* state, long state_stride, const int* slots, const int* cu, float* out,
+                         int B, int max_q_len, int H, int hpg, int d, int dv, const TA* skip_x, long skip_stride,
+                         const float* skip, hipStream_t stream) {
+  const bool whole = d % 4 == 0 && dv % 4 == 0 && (((size_t)qf | (size_t)kf | (size_t)vf | (size_t)sums | (size_t)skip_x) & 15) == 0 &&
+                     skip_stride % 4 == 0;
+  return (whole ? launch_whole_chunks<TA, true> : launch_whole_chunks<TA, false>)(
+      qf, kf, vf, ld, ld_row, sums, decays, scores, state, state_stride, slots, cu, out, B, max_q_len, H, hpg, d, dv, skip_x,
+      skip_stride, skip, stream);
 }
 
 extern "C" int q3_mamba2_chunked(const void* xbc, const void* dt, long dt_stride, const float* dt_bias,
@@ -1203,18 +1285,17 @@ extern "C" int q3_block_gates(const float* u, const float* w, const float* bias,
   if (T <= 0 || width <= 0 || blocks <= 0 || width % blocks || blocks > 65535) return Q3_ERR_BAD_ARGUMENT;
   const int bw = width / blocks;
   if (bw > 1536) return Q3_ERR_UNSUPPORTED;
-  if (T <= 96) {
-    const int out_tiles = (bw + 63) / 64;
-    if ((long)blocks * out_tiles > 65535) return Q3_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL(block_gates_few_kernel, dim3((T + Q3_GATE_TOKENS - 1) / Q3_GATE_TOKENS, blocks * out_tiles, 2),
-                       dim3(256), (size_t)(Q3_GATE_TOKENS * bw + 4 * 64 * Q3_GATE_TOKENS) * sizeof(float), stream, u, w,
-                       bias, out, T, width, bw, out_tiles);
+  if ((long)T * width <= Q3_GATES_FEW && (long)blocks * ((bw + 15) / 16) <= 65535) {
+    const int out_tiles = (bw + 15) / 16;
+    hipLaunchKernelGGL(block_gates_few_kernel, dim3((T + 15) / 16, blocks * out_tiles, 2), dim3(256), 0, stream, u, w, bias,
+                       out, T, width, bw, out_tiles);
     return q3_launch_status();
   }
   const int out_tiles = (bw + 63) / 64;
   if ((long)blocks * out_tiles > 65535) return Q3_ERR_UNSUPPORTED;
-  hipLaunchKernelGGL(block_gates_kernel, dim3((T + 63) / 64, blocks * out_tiles, 2), dim3(256), 0, stream, u, w, bias, out,
-                     T, width, bw, out_tiles);
+  const bool whole = bw % 4 == 0 && (((size_t)u | (size_t)w | (size_t)bias) & 15) == 0;
+  hipLaunchKernelGGL((whole ? block_gates_kernel<true> : block_gates_kernel<false>), dim3((T + 63) / 64, blocks * out_tiles, 2),
+                     dim3(256), 0, stream, u, w, bias, out, T, width, bw, out_tiles);
   return q3_launch_status();
 }
 

@@ -40,3 +40,36 @@ def test_gated_rmsnorm_rows(dtype, n, groups, off):
     gate = _rand(g, 3, n + 12, dtype=dtype)[:, off:off + n]
     _close(ops.gated_rmsnorm(y, gate, weight, groups, 1e-6, dtype), twin.gated_rmsnorm(y, gate, weight, groups, 1e-6, dtype),
            _tol(dtype))
+
+
+@pytest.mark.parametrize("T,width,blocks", [(1, 64, 1), (17, 60, 2), (16, 1536, 1), (48, 2048, 8), (49, 2048, 8), (65, 2048, 2),
+                                            (1970, 50, 2), (130, 1020, 15), (70, 3070, 2)])
+def test_block_gates_both_ways(T, width, blocks):
+    g = _gen(T + width)
+    bw = width // blocks
+    u, weights, biases = _rand(g, T, width), _rand(g, 2, blocks, bw, bw, scale=bw ** -0.5), _rand(g, 2, blocks, bw)
+    z = torch.stack([u.double().view(T, blocks, bw)[:, b] @ weights[:, b].double() for b in range(blocks)], 2)
+    want = torch.sigmoid(z + biases.double()[:, None]).reshape(2, T, width)
+    # a sigmoid's slope is at most 1/4: a quarter of the error of a float32 sum of 1,536 products, whose partial sums are
+    # of size 1 and drift by sqrt(1536) halves of 2^-23 (0.6e-6 in all); a few times that
+    assert float((ops.block_gates(u, weights, biases).double() - want).abs().max()) < 4e-6
+    aside = torch.empty(T * width + 1, device=DEV)[1:].view(T, width).copy_(u)      # rows that begin on four bytes
+    assert float((ops.block_gates(aside, weights, biases).double() - want).abs().max()) < 4e-6
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("H,P,N,G,lengths", [(2, 64, 64, 1, [64, 65]), (2, 62, 65, 2, [127, 1]), (3, 68, 132, 1, [70, 63]),
+                                             (1, 3, 1, 1, [66]), (2, 130, 256, 2, [129])])
+def test_chunks_of_whole_and_broken_rows(dtype, H, P, N, G, lengths):
+    """Keys of up to 64, 128 and 256 numbers, rows read four numbers at a time and one by one, chunks of one row."""
+    g = _gen(H * P + N)
+    T = sum(lengths)
+    xbc, dt = _rand(g, T, H * P + 2 * G * N, dtype=dtype), _rand(g, T, H, dtype=dtype)
+    dt_bias, a_log, skip = _rand(g, H), _rand(g, H, scale=0.5), _rand(g, H)
+    cu, _, slots = _step(lengths, [1, 0][:len(lengths)])
+    full = _rand(g, 2, H * N * P, scale=0.3)
+    a, b = full.clone(), full.clone()
+    assert max(lengths) >= ops.CHUNKED_FROM
+    got = ops.mamba2_scan(xbc, dt, dt_bias, a_log, skip, a, slots, cu, H, P, N, G, max_q_len=max(lengths))
+    _close(got, twin.mamba2_scan(xbc, dt, dt_bias, a_log, skip, b, slots, cu, H, P, N, G), 3e-5)
+    _close(a, b, 3e-5)
