@@ -248,59 +248,6 @@ __global__ void conv_tail_kernel(const TI* __restrict__ x, long x_stride, const 
   for (int k = 0; k < taps - 1; ++k) tail[(size_t)k * C + c] = keep[k];
 }
 
-// ---- Mamba-2 ----
-// One wavefront per (sequence, head, 64 columns of the head's vdim): lane p keeps column p of the
-// state S (N x vdim) in registers and walks the sequence's tokens in order:
-//   dt = softplus(dt_raw + dt_bias),  S = exp(-exp(A_log) dt) S + dt B x_p,  y_p = sum_n S[n] C[n] + D x_p.
-// xbc rows are [x: H P | B: G N | C: G N]; B and C of the head's group go through shared memory.
-template <typename TA, int NMAX>
-__global__ void __launch_bounds__(64) mamba2_scan_kernel(
-    const TA* __restrict__ xbc, const TA* __restrict__ dt, long dt_stride, const float* __restrict__ dt_bias,
-    const float* __restrict__ a_log, const float* __restrict__ d_skip, float* __restrict__ state, long state_stride,
-    const int* __restrict__ slots, const int* __restrict__ cu, float* __restrict__ y, int H, int P, int N, int G) {
-  __shared__ float sB[NMAX], sC[NMAX];
-  const int lane = threadIdx.x;
-  const int p = blockIdx.x * 64 + lane;
-  const int h = blockIdx.y, b = blockIdx.z;
-  const int start = cu[b], end = cu[b + 1];
-  if (end <= start) return;
-  const int g = h / (H / G);
-  const int C = H * P + 2 * G * N;
-  const bool live = p < P;
-  float* mine = state + (size_t)slots[b] * state_stride + (size_t)h * N * P + p;
-  float S[NMAX];
-#pragma unroll
-  for (int n = 0; n < NMAX; ++n) S[n] = (live && n < N) ? mine[(size_t)n * P] : 0.f;
-  const float rate = expf(a_log[h]), shift = dt_bias[h], skip = d_skip[h];
-  for (int t = start; t < end; ++t) {
-    const TA* row = xbc + (size_t)t * C;
-    for (int n = lane; n < N; n += 64) {
-      sB[n] = to_float(row[H * P + g * N + n]);
-      sC[n] = to_float(row[H * P + G * N + g * N + n]);
-    }
-    __syncthreads();
-    const float step = softplus_value(to_float(dt[(size_t)t * dt_stride + h]) + shift);
-    const float decay = expf(-rate * step);
-    const float xv = live ? to_float(row[h * P + p]) : 0.f;
-    const float push = step * xv;
-    float acc = 0.f;
-#pragma unroll
-    for (int n = 0; n < NMAX; ++n) {
-      if (n < N) {
-        S[n] = decay * S[n] + sB[n] * push;
-        acc += S[n] * sC[n];
-      }
-    }
-    if (live) y[(size_t)t * H * P + h * P + p] = acc + skip * xv;
-    __syncthreads();
-  }
-  if (live) {
-#pragma unroll
-    for (int n = 0; n < NMAX; ++n)
-      if (n < N) mine[(size_t)n * P] = S[n];
-  }
-}
-
 // ---- the recurrent unit's recurrence ----
 // Per (sequence, channel): log a = -rate r, a = exp(log a), S = a S + sqrt(1 - a^2) i u (1 - a^2 as
 // -expm1(2 log a)), out = S * gelu_tanh(y + y_bias). gates = [r | i], each (T, width).
@@ -328,72 +275,6 @@ __global__ void rglru_scan_kernel(const float* __restrict__ u, const float* __re
     out[at] = from_float<TO>(S * branch);
   }
   *mine = S;
-}
-
-// ---- retention ----
-// One block per (sequence, head, 256 columns of the head's vdim), thread v keeps column v of S
-// (dim x vdim) in registers. Rows of the input are [q: H dim | k: H dim | v: H vdim | g: H vdim]. Per
-// token q and k turn by the position (pairs (i, i + half) of their first 2 * half numbers, angle =
-// position * inv_freq[i]), k times k_scale; S = decay S + k v^T, o = S^T q, left as float32 in
-// `raw` (T, H vdim): the division by the head's root mean square and the gate follow in
-// retention_finish_kernel.
-template <typename TA, int DMAX>
-__global__ void __launch_bounds__(256) retention_scan_kernel(
-    const TA* __restrict__ rows, const float* __restrict__ inv_freq, int half, const int* __restrict__ positions,
-    const float* __restrict__ decays, float k_scale, float* __restrict__ state, long state_stride,
-    const int* __restrict__ slots, const int* __restrict__ cu, float* __restrict__ raw, int H, int dim, int vdim) {
-  __shared__ float sq[DMAX], sk[DMAX];
-  const int slices = (vdim + 255) / 256;
-  const int h = blockIdx.x / slices;
-  const int v = (blockIdx.x % slices) * 256 + threadIdx.x;
-  const int b = blockIdx.y;
-  const int start = cu[b], end = cu[b + 1];
-  if (end <= start) return;
-  const bool live = v < vdim;
-  const int hd = H * dim, hv = H * vdim;
-  const size_t width = 2 * (size_t)hd + 2 * (size_t)hv;
-  float* mine = state + (size_t)slots[b] * state_stride + (size_t)h * dim * vdim + v;
-  float S[DMAX];
-#pragma unroll
-  for (int n = 0; n < DMAX; ++n) S[n] = (live && n < dim) ? mine[(size_t)n * vdim] : 0.f;
-  const float decay = decays[h];
-  for (int t = start; t < end; ++t) {
-    const TA* row = rows + (size_t)t * width;
-    const TA* q = row + h * dim;
-    const TA* k = row + hd + h * dim;
-    const float pos = (float)positions[t];
-    __syncthreads();
-    for (int j = threadIdx.x; j < dim; j += 256) {
-      float qv = to_float(q[j]), kv = to_float(k[j]);
-      if (j < 2 * half) {
-        const bool first = j < half;
-        const int partner = first ? j + half : j - half;
-        const float angle = pos * inv_freq[first ? j : j - half];
-        const float c = cosf(angle), s = sinf(angle);
-        const float qp = to_float(q[partner]), kp = to_float(k[partner]);
-        qv = first ? qv * c - qp * s : qv * c + qp * s;
-        kv = first ? kv * c - kp * s : kv * c + kp * s;
-      }
-      sq[j] = qv;
-      sk[j] = kv * k_scale;
-    }
-    __syncthreads();
-    const float vv = live ? to_float(row[2 * hd + h * vdim + v]) : 0.f;
-    float acc = 0.f;
-#pragma unroll
-    for (int n = 0; n < DMAX; ++n) {
-      if (n < dim) {
-        S[n] = decay * S[n] + sk[n] * vv;
-        acc += S[n] * sq[n];
-      }
-    }
-    if (live) raw[(size_t)t * hv + h * vdim + v] = acc;
-  }
-  if (live) {
-#pragma unroll
-    for (int n = 0; n < DMAX; ++n)
-      if (n < dim) mine[(size_t)n * vdim] = S[n];
-  }
 }
 
 // ---- recurrences with a decayed outer-product state, many tokens at a time ----
@@ -797,6 +678,174 @@ __global__ void __launch_bounds__(256) chunk_output_kernel(const float* __restri
       store_four(out + ((size_t)(row0 + my_row) * H + h) * dv + j, acc[x], dv - j, whole);
     }
   }
+}
+
+// ---- Mamba-2 and retention, a row at a time ----
+// A block of 256 threads per (sequence, head, 64 columns of the head's vdim) keeps the columns' state (up to 16 EACH rows n
+// of vdim) in registers and walks the sequence's tokens in order. A thread holds four neighbouring columns of the rows
+// `group`, `group` + 16 and so on, so that the state comes and goes in accesses of four numbers, all in flight at once and
+// behind the first token's; each following token's row is on its way while its predecessor is worked off. The groups'
+// shares of a result meet by lane exchanges and then, from the four wavefronts, in shared memory.
+//
+// Few tokens are bound by the state's passage. 8 sequences of one token: Mamba-2's 64 heads of 128 x 64 (17 MB in, 17 out)
+// 9.4 us, 16.9 with a wavefront per 64 columns and a column a thread; retention's 8 heads of 128 x 256 (8.4 MB and 8.4)
+// 6.6 us, 17.2 with a block per 256 columns.
+template <int EACH, bool WHOLE>
+struct StateColumns {
+  float S[EACH][4];
+  __device__ void load(const float* __restrict__ state, int rows, int width, int group, int column) {
+    float4 got[EACH];
+#pragma unroll
+    for (int k = 0; k < EACH; ++k) {
+      const int n = group + 16 * k;
+      got[k] = load_four<WHOLE>(state + (size_t)(n < rows ? n : 0) * width, column, width);
+    }
+#pragma unroll
+    for (int k = 0; k < EACH; ++k) {
+      const float4 kept = kept_four<WHOLE>(got[k], column, width, group + 16 * k < rows);
+      S[k][0] = kept.x, S[k][1] = kept.y, S[k][2] = kept.z, S[k][3] = kept.w;
+    }
+  }
+  __device__ void store(float* __restrict__ state, int rows, int width, int group, int column) const {
+#pragma unroll
+    for (int k = 0; k < EACH; ++k) {
+      const int n = group + 16 * k;
+      if (n < rows) store_four(state + (size_t)n * width + column, f32x4_t{S[k][0], S[k][1], S[k][2], S[k][3]}, width - column, WHOLE);
+    }
+  }
+  // S = decay S + key push, and what the rows of the wavefront give of sum_n S[n] query[n] into part[wave]; `keys` and
+  // `queries` hold zeros past the rows that exist.
+  __device__ void step(float decay, const float* keys, const float* queries, const float (&push)[4], int group, float (*part)[64]) {
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < EACH; ++k) {
+      const float key = keys[group + 16 * k], query = queries[group + 16 * k];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        S[k][e] = decay * S[k][e] + key * push[e];
+        acc[e] += S[k][e] * query;
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      acc[e] += __shfl_xor(acc[e], 16);
+      acc[e] += __shfl_xor(acc[e], 32);
+    }
+    if ((threadIdx.x & 63) < 16)
+      *reinterpret_cast<float4*>(part[threadIdx.x >> 6] + 4 * (threadIdx.x & 15)) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+  }
+};
+
+// step = softplus(dt + dt_bias), S = exp(-exp(A_log) step) S + step B x_p, y_p = sum_n S[n] C[n] + D x_p. xbc rows are
+// [x: H P | B: G N | C: G N].
+template <typename TA, int EACH, bool WHOLE>
+__global__ void __launch_bounds__(256) mamba2_scan_kernel(
+    const TA* __restrict__ xbc, const TA* __restrict__ dt, long dt_stride, const float* __restrict__ dt_bias,
+    const float* __restrict__ a_log, const float* __restrict__ d_skip, float* __restrict__ state, long state_stride,
+    const int* __restrict__ slots, const int* __restrict__ cu, float* __restrict__ y, int H, int P, int N, int G) {
+  __shared__ float sB[16 * EACH], sC[16 * EACH];
+  __shared__ __attribute__((aligned(16))) float part[4][64];
+  const int tid = threadIdx.x, group = tid >> 4;
+  const int column = blockIdx.x * 64 + 4 * (tid & 15), own = blockIdx.x * 64 + (tid & 63);
+  const int h = blockIdx.y, b = blockIdx.z;
+  const int start = cu[b], end = cu[b + 1];
+  if (end <= start) return;
+  const int g = h / (H / G);
+  const int C = H * P + 2 * G * N;
+  const int at_b = H * P + g * N + (tid < N ? tid : 0);
+  const TA* row = xbc + (size_t)start * C;
+  TA rb = row[at_b], rc = row[at_b + G * N], ro = row[h * P + (own < P ? own : 0)], rd = dt[(size_t)start * dt_stride + h];
+  Four<TA> rx;
+  rx.template load<false>(row + h * P, column, P);
+  const float rate = expf(a_log[h]), shift = dt_bias[h], skip = d_skip[h];
+  float* mine = state + (size_t)slots[b] * state_stride + (size_t)h * N * P;
+  StateColumns<EACH, WHOLE> at;
+  at.load(mine, N, P, group, column);
+  for (int t = start; t < end; ++t) {
+    if (tid < 16 * EACH) {
+      sB[tid] = tid < N ? to_float(rb) : 0.f;
+      sC[tid] = tid < N ? to_float(rc) : 0.f;
+    }
+    const float step = softplus_value(to_float(rd) + shift);
+    const float decay = expf(-rate * step), x_own = to_float(ro);
+    float push[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) push[e] = step * to_float(rx.of[e]);
+    __syncthreads();
+    if (t + 1 < end) {
+      row = xbc + (size_t)(t + 1) * C;
+      rb = row[at_b], rc = row[at_b + G * N], ro = row[h * P + (own < P ? own : 0)], rd = dt[(size_t)(t + 1) * dt_stride + h];
+      rx.template load<false>(row + h * P, column, P);
+    }
+    at.step(decay, sB, sC, push, group, part);
+    __syncthreads();
+    if (tid < 64 && own < P)
+      y[((size_t)t * H + h) * P + own] = ((part[0][tid] + part[1][tid]) + (part[2][tid] + part[3][tid])) + skip * x_own;
+  }
+  at.store(mine, N, P, group, column);
+}
+
+// Rows of the input are [q: H dim | k: H dim | v: H vdim | g: H vdim]. Per token q and k turn by the position (pairs
+// (i, i + half) of their first 2 * half numbers, angle = position * inv_freq[i]), k times k_scale; S = decay S + k v^T,
+// o = S^T q, left as float32 in `raw` (T, H vdim): the division by the head's root mean square and the gate follow in
+// retention_finish_kernel.
+template <typename TA, int EACH, bool WHOLE>
+__global__ void __launch_bounds__(256) retention_scan_kernel(
+    const TA* __restrict__ rows, const float* __restrict__ inv_freq, int half, const int* __restrict__ positions,
+    const float* __restrict__ decays, float k_scale, float* __restrict__ state, long state_stride,
+    const int* __restrict__ slots, const int* __restrict__ cu, float* __restrict__ raw, int H, int dim, int vdim) {
+  __shared__ float sq[16 * EACH], sk[16 * EACH];
+  __shared__ __attribute__((aligned(16))) float part[4][64];
+  const int tid = threadIdx.x, group = tid >> 4;
+  const int tiles = (vdim + 63) / 64;
+  const int h = blockIdx.x / tiles, tile = blockIdx.x % tiles, b = blockIdx.y;
+  const int column = tile * 64 + 4 * (tid & 15), own = tile * 64 + (tid & 63);
+  const int start = cu[b], end = cu[b + 1];
+  if (end <= start) return;
+  const int hd = H * dim, hv = H * vdim;
+  const size_t width = 2 * (size_t)hd + 2 * (size_t)hv;
+  const int j = tid < dim ? tid : 0;
+  const bool turned = j < 2 * half, first = j < half;
+  const int partner = turned ? (first ? j + half : j - half) : j;
+  const float freq = half ? inv_freq[turned ? (first ? j : j - half) : 0] : 0.f;
+  const TA* row = rows + (size_t)start * width + h * dim;
+  TA rq = row[j], rqp = row[partner], rk = row[hd + j], rkp = row[hd + partner];
+  int position = positions[start];
+  Four<TA> rv;
+  rv.template load<false>(rows + (size_t)start * width + 2 * hd + h * vdim, column, vdim);
+  const float decay = decays[h];
+  float* mine = state + (size_t)slots[b] * state_stride + (size_t)h * dim * vdim;
+  StateColumns<EACH, WHOLE> at;
+  at.load(mine, dim, vdim, group, column);
+  for (int t = start; t < end; ++t) {
+    float qv = to_float(rq), kv = to_float(rk);
+    if (turned) {
+      const float angle = (float)position * freq;
+      const float c = cosf(angle), s = sinf(angle);
+      const float qp = to_float(rqp), kp = to_float(rkp);
+      qv = first ? qv * c - qp * s : qv * c + qp * s;
+      kv = first ? kv * c - kp * s : kv * c + kp * s;
+    }
+    if (tid < 16 * EACH) {
+      sq[tid] = tid < dim ? qv : 0.f;
+      sk[tid] = tid < dim ? kv * k_scale : 0.f;
+    }
+    float push[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) push[e] = to_float(rv.of[e]);
+    __syncthreads();
+    if (t + 1 < end) {
+      row = rows + (size_t)(t + 1) * width + h * dim;
+      rq = row[j], rqp = row[partner], rk = row[hd + j], rkp = row[hd + partner];
+      position = positions[t + 1];
+      rv.template load<false>(rows + (size_t)(t + 1) * width + 2 * hd + h * vdim, column, vdim);
+    }
+    at.step(decay, sk, sq, push, group, part);
+    __syncthreads();
+    if (tid < 64 && own < vdim)
+      raw[(size_t)t * hv + h * vdim + own] = (part[0][tid] + part[1][tid]) + (part[2][tid] + part[3][tid]);
+  }
+  at.store(mine, dim, vdim, group, column);
 }
 
 // ---- the recurrent unit's gates ----
@@ -1258,14 +1307,15 @@ static int launch_mamba2(const void* xbc, const void* dt, long dt_stride, const 
                          const float* d_skip, float* state, long state_stride, const int* slots, const int* cu, float* y,
                          int B, int H, int P, int N, int G, hipStream_t stream) {
   const dim3 grid((P + 63) / 64, H, B);
-#define Q3_MAMBA(NMAX)                                                                                              \
-  hipLaunchKernelGGL((mamba2_scan_kernel<TA, NMAX>), grid, dim3(64), 0, stream, (const TA*)xbc, (const TA*)dt,      \
-                     dt_stride, dt_bias, a_log, d_skip, state, state_stride, slots, cu, y, H, P, N, G)
-  if (N <= 16) Q3_MAMBA(16);
-  else if (N <= 32) Q3_MAMBA(32);
-  else if (N <= 64) Q3_MAMBA(64);
-  else if (N <= 128) Q3_MAMBA(128);
-  else Q3_MAMBA(256);
+  const bool whole = P % 4 == 0 && state_stride % 4 == 0 && ((size_t)state & 15) == 0;
+#define Q3_MAMBA(EACH)                                                                                                    \
+  hipLaunchKernelGGL((whole ? mamba2_scan_kernel<TA, EACH, true> : mamba2_scan_kernel<TA, EACH, false>), grid, dim3(256), \
+                     0, stream, (const TA*)xbc, (const TA*)dt, dt_stride, dt_bias, a_log, d_skip, state, state_stride,    \
+                     slots, cu, y, H, P, N, G)
+  if (N <= 32) Q3_MAMBA(2);
+  else if (N <= 64) Q3_MAMBA(4);
+  else if (N <= 128) Q3_MAMBA(8);
+  else Q3_MAMBA(16);
 #undef Q3_MAMBA
   return q3_launch_status();
 }
@@ -1315,14 +1365,16 @@ template <typename TA>
 static int launch_retention(const void* rows, const float* inv_freq, int half, const int* positions, const float* decays,
                             float k_scale, float eps, float* state, long state_stride, const int* slots, const int* cu,
                             void* out, float* raw, int T, int B, int H, int dim, int vdim, hipStream_t stream) {
-  const dim3 grid(H * ((vdim + 255) / 256), B);
-#define Q3_RETENTION(DMAX)                                                                                            \
-  hipLaunchKernelGGL((retention_scan_kernel<TA, DMAX>), grid, dim3(256), 0, stream, (const TA*)rows, inv_freq, half,  \
-                     positions, decays, k_scale, state, state_stride, slots, cu, raw, H, dim, vdim)
-  if (dim <= 32) Q3_RETENTION(32);
-  else if (dim <= 64) Q3_RETENTION(64);
-  else if (dim <= 128) Q3_RETENTION(128);
-  else Q3_RETENTION(256);
+  const dim3 grid(H * ((vdim + 63) / 64), B);
+  const bool whole = vdim % 4 == 0 && state_stride % 4 == 0 && ((size_t)state & 15) == 0;
+#define Q3_RETENTION(EACH)                                                                                            \
+  hipLaunchKernelGGL((whole ? retention_scan_kernel<TA, EACH, true> : retention_scan_kernel<TA, EACH, false>), grid,  \
+                     dim3(256), 0, stream, (const TA*)rows, inv_freq, half, positions, decays, k_scale, state,        \
+                     state_stride, slots, cu, raw, H, dim, vdim)
+  if (dim <= 32) Q3_RETENTION(2);
+  else if (dim <= 64) Q3_RETENTION(4);
+  else if (dim <= 128) Q3_RETENTION(8);
+  else Q3_RETENTION(16);
 #undef Q3_RETENTION
   const int threads = vdim >= 256 ? 256 : (vdim >= 128 ? 128 : 64);
   hipLaunchKernelGGL(retention_finish_kernel<TA>, dim3(T, H), dim3(threads), 0, stream, raw, (const TA*)rows, eps,

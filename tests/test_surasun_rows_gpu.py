@@ -73,3 +73,21 @@ def test_chunks_of_whole_and_broken_rows(dtype, H, P, N, G, lengths):
     got = ops.mamba2_scan(xbc, dt, dt_bias, a_log, skip, a, slots, cu, H, P, N, G, max_q_len=max(lengths))
     _close(got, twin.mamba2_scan(xbc, dt, dt_bias, a_log, skip, b, slots, cu, H, P, N, G), 3e-5)
     _close(a, b, 3e-5)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("rows,width,off", [(1, 1, 0), (16, 64, 0), (33, 68, 0), (64, 62, 0), (65, 130, 3), (128, 64, 2), (256, 256, 4)])
+@pytest.mark.parametrize("lengths", [[1, 1], [8, 3]])
+def test_state_walked_row_by_row(dtype, rows, width, off, lengths):
+    """Sequences of one token and of several, states of rows and widths around the kernel's 16 EACH rows and 64 columns,
+    on sixteen bytes or not."""
+    g = _gen(rows * width + off)
+    T, H = sum(lengths), 2
+    cu, _, slots = _step(lengths, [2, 0])
+    full = _rand(g, 3, H * rows * width + off, scale=0.3)
+    xbc, dt = _rand(g, T, H * width + 2 * rows, dtype=dtype), _rand(g, T, H, dtype=dtype)
+    dt_bias, a_log, skip = _rand(g, H), _rand(g, H, scale=0.5), _rand(g, H)
+    a, b = full.clone(), full.clone()
+    got = ops.mamba2_scan(xbc, dt, dt_bias, a_log, skip, a[:, off:], slots, cu, H, width, rows, 1, max_q_len=max(lengths))
+    _close(got, twin.mamba2_scan(xbc, dt, dt_bias, a_log, skip, b[:, off:], slots, cu, H, width, rows, 1), 3e-5)
+    _close(a, b, 3e-5)
