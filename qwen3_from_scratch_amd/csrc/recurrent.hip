@@ -62,10 +62,9 @@ __global__ void causal_conv_kernel(const TI* __restrict__ x, long x_stride, cons
   }
 }
 
-// Eight channels a thread in 16-byte accesses, for steps of many rows: the thread walks `rows_each`
-// rows with its last taps - 1 inputs in registers, so every input is read once; where a row is a
-// sequence's first (or the thread's first), the inputs before it come from the rows above or from
-// the sequence's tail. Needs C and the rows' stride in steps of eight and 16-byte aligned rows.
+// Eight channels a thread in 16-byte accesses, for steps of many rows: the thread takes a tile of rows with the last
+// taps - 1 inputs before them, which come from the rows above or, where a row is a sequence's first, from the
+// sequence's tail. Needs C and the rows' stride in steps of eight and 16-byte aligned rows.
 __device__ inline void load8(const bf16_t* p, float (&v)[8]) {
   union {
     uint4 u;
@@ -93,68 +92,108 @@ __device__ inline void store8(float* p, const float (&v)[8]) {
   *reinterpret_cast<float4*>(p + 4) = make_float4(v[4], v[5], v[6], v[7]);
 }
 
+// Eight numbers as they come, made float32 where they are used: made so where they are loaded, each load waits.
+template <typename TI>
+struct Eight;
+template <>
+struct Eight<bf16_t> {
+  uint4 raw;
+  __device__ void load(const bf16_t* p) { raw = *reinterpret_cast<const uint4*>(p); }
+  __device__ void get(float (&v)[8]) const {
+    const unsigned w[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[2 * i] = __uint_as_float(w[i] << 16), v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+  }
+};
+template <>
+struct Eight<float> {
+  float4 a, b;
+  __device__ void load(const float* p) { a = *reinterpret_cast<const float4*>(p), b = *reinterpret_cast<const float4*>(p + 4); }
+  __device__ void get(float (&v)[8]) const {
+    v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
+  }
+};
+
+// A thread's tile is Q3_CONV_TILE rows. TAPS 4: that many, and a thread takes its channels' taps straight from memory; 0:
+// up to Q3_TAPS_MOST, through shared memory. Bound by memory and the taps' passage: 2,048 rows of 4,352 bfloat16 channels and 4 taps (36 MB) 22 us, 37 with an input's wait before
+// each next one and taps that 32 lanes read from one bank of shared memory.
 #define Q3_CONV_TILE 8
-template <typename TI, typename TO>
+template <typename TI, typename TO, int TAPS>
 __global__ void __launch_bounds__(64) causal_conv_wide_kernel(const TI* __restrict__ x, long x_stride, const float* __restrict__ in_bias,
                                         const float* __restrict__ w, const float* __restrict__ bias,
                                         const float* __restrict__ state, long state_stride,
                                         const int* __restrict__ slots, const int* __restrict__ cu,
-                                        const int* __restrict__ seq_index, TO* __restrict__ out, int T, int C, int taps,
-                                        int act, int rows_each) {
-  // the block's taps lie side by side in memory (64 threads x 8 channels x taps): in through shared memory
-  __shared__ __attribute__((aligned(16))) float taps_of_block[64 * 8 * Q3_TAPS_MOST];
+                                        const int* __restrict__ seq_index, TO* __restrict__ out, int T, int C, int any_taps,
+                                        int act) {
+  constexpr int MOST = TAPS ? TAPS : Q3_TAPS_MOST;
+  const int taps = TAPS ? TAPS : any_taps;
   const int first = blockIdx.y * 64 * 8;
-  const int held = C - first < 64 * 8 ? C - first : 64 * 8;
-  {
-    // 2 * taps loads of 16 bytes a thread, all asked for before the first is stored
-    const float4* src = reinterpret_cast<const float4*>(w + (size_t)first * taps);
-    const int pieces = held * taps / 4;
-    float4 got[2 * Q3_TAPS_MOST];
+  const int c0 = first + threadIdx.x * 8 < C ? first + threadIdx.x * 8 : first;      // (a thread past the end only helps with the taps)
+  const int t0 = blockIdx.x * Q3_CONV_TILE;
+  const int t1 = t0 + Q3_CONV_TILE < T ? t0 + Q3_CONV_TILE : T;
+  const int seq = seq_index[t0], start = cu[seq];
+  const bool one_sequence = seq == seq_index[t1 - 1];
+  float tap[MOST][8];
+  if constexpr (TAPS == 4) {
 #pragma unroll
-    for (int k = 0; k < 2 * Q3_TAPS_MOST; ++k)
-      got[k] = (k < 2 * taps && threadIdx.x + 64 * k < pieces) ? src[threadIdx.x + 64 * k] : make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-    for (int k = 0; k < 2 * Q3_TAPS_MOST; ++k)
-      if (k < 2 * taps && threadIdx.x + 64 * k < pieces) reinterpret_cast<float4*>(taps_of_block)[threadIdx.x + 64 * k] = got[k];
+    for (int e = 0; e < 8; ++e) {
+      const float4 own = *reinterpret_cast<const float4*>(w + (size_t)(c0 + e) * 4);
+      tap[3][e] = own.x, tap[2][e] = own.y, tap[1][e] = own.z, tap[0][e] = own.w;
+    }
   }
-  __syncthreads();
-  const int c0 = first + threadIdx.x * 8;
-  if (c0 >= C) return;
-  float tap[Q3_TAPS_MOST][8], base[8], add[8], win[Q3_TAPS_MOST - 1][8];
+  // the usual case, all rows of one sequence: every input the rows need is asked for at once, behind
+  // no branch, rows t0 - (MOST - 1) .. t1 - 1; rows that do not exist (or precede the sequence) are read as one that does
+  Eight<TI> raw[Q3_CONV_TILE + MOST - 1];
+  if (one_sequence) {
+#pragma unroll
+    for (int i = 0; i < Q3_CONV_TILE + MOST - 1; ++i) {
+      int row = t0 - (MOST - 1) + i;
+      row = row < start ? start : (row < t1 ? row : t1 - 1);
+      raw[i].load(x + (size_t)row * x_stride + c0);
+    }
+  }
+  float base[8], add[8];
   load8(bias + c0, base);
 #pragma unroll
   for (int e = 0; e < 8; ++e) add[e] = 0.f;
   if (in_bias) load8(in_bias + c0, add);
+  __builtin_amdgcn_sched_barrier(0);      // all loads go out before the first is waited for
+  if constexpr (TAPS == 0) {
+    // the block's taps lie side by side in memory (64 threads x 8 channels x taps); the loads past their end read the
+    // first again, into a place that nothing reads
+    __shared__ __attribute__((aligned(16))) float taps_of_block[64 * 8 * MOST];
+    const float4* src = reinterpret_cast<const float4*>(w + (size_t)first * taps);
+    const int pieces = (C - first < 64 * 8 ? C - first : 64 * 8) * taps / 4;
+    float4 got[2 * MOST];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
+    for (int k = 0; k < 2 * MOST; ++k) got[k] = src[(int)threadIdx.x + 64 * k < pieces ? threadIdx.x + 64 * k : 0];
 #pragma unroll
-    for (int j = 0; j < Q3_TAPS_MOST; ++j)
-      tap[j][e] = j < taps ? taps_of_block[(threadIdx.x * 8 + e) * taps + taps - 1 - j] : 0.f;
+    for (int k = 0; k < 2 * MOST; ++k) reinterpret_cast<float4*>(taps_of_block)[threadIdx.x + 64 * k] = got[k];
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+#pragma unroll
+      for (int j = 0; j < MOST; ++j) tap[j][e] = j < taps ? taps_of_block[(threadIdx.x * 8 + e) * taps + taps - 1 - j] : 0.f;
+    }
   }
-  const int t0 = blockIdx.x * rows_each;
-  const int t1 = t0 + rows_each < T ? t0 + rows_each : T;
-  if (rows_each == Q3_CONV_TILE && seq_index[t0] == seq_index[t1 - 1]) {
-    // the usual case, all rows of one sequence: every input the rows need is asked for at once (one wait
-    // instead of a chain of them), rows t0 - (taps - 1) .. t1 - 1 at in[Q3_TAPS_MOST - taps ..]
-    const int b = seq_index[t0];
-    const int start = cu[b];
-    const float* tail = state + (size_t)slots[b] * state_stride;
-    float in[Q3_CONV_TILE + Q3_TAPS_MOST - 1][8];
+  if (first + (int)threadIdx.x * 8 >= C) return;
+  if (one_sequence) {
+    float in[Q3_CONV_TILE + MOST - 1][8];
 #pragma unroll
-    for (int i = 0; i < Q3_CONV_TILE + Q3_TAPS_MOST - 1; ++i) {
-      const int row = t0 - (Q3_TAPS_MOST - 1) + i;
-      if (i >= Q3_TAPS_MOST - taps && row < t1) {
-        if (row >= start) {
-          load8(x + (size_t)row * x_stride + c0, in[i]);
+    for (int i = 0; i < Q3_CONV_TILE + MOST - 1; ++i) {
+      raw[i].get(in[i]);
 #pragma unroll
-          for (int e = 0; e < 8; ++e) in[i][e] += add[e];
-        } else {
+      for (int e = 0; e < 8; ++e) in[i][e] += add[e];
+    }
+    if (t0 - (taps - 1) < start) {
+      const float* tail = state + (size_t)slots[seq] * state_stride;
+#pragma unroll
+      for (int i = 0; i < MOST - 1; ++i) {
+        const int row = t0 - (MOST - 1) + i;
+        if (i >= MOST - taps && row < start) {
 #pragma unroll
           for (int e = 0; e < 8; ++e) in[i][e] = tail[(size_t)(taps - 1 - (start - row)) * C + c0 + e];
         }
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) in[i][e] = 0.f;
       }
     }
 #pragma unroll
@@ -164,10 +203,10 @@ __global__ void __launch_bounds__(64) causal_conv_wide_kernel(const TI* __restri
 #pragma unroll
         for (int e = 0; e < 8; ++e) acc[e] = base[e];
 #pragma unroll
-        for (int j = 0; j < Q3_TAPS_MOST; ++j)
+        for (int j = 0; j < MOST; ++j)
           if (j < taps) {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) acc[e] += tap[j][e] * in[r + Q3_TAPS_MOST - 1 - j][e];
+            for (int e = 0; e < 8; ++e) acc[e] += tap[j][e] * in[r + MOST - 1 - j][e];
           }
         if (act == 1) {
 #pragma unroll
@@ -178,13 +217,14 @@ __global__ void __launch_bounds__(64) causal_conv_wide_kernel(const TI* __restri
     }
     return;
   }
+  float win[MOST - 1][8];
   for (int t = t0; t < t1; ++t) {
     const int b = seq_index[t];
     const int start = cu[b];
     if (t == t0 || t == start) {
       const float* tail = state + (size_t)slots[b] * state_stride;
 #pragma unroll
-      for (int j = 0; j < Q3_TAPS_MOST - 1; ++j) {
+      for (int j = 0; j < MOST - 1; ++j) {
         if (j < taps - 1) {
           const int src = t - 1 - j;
           if (src >= start) {
@@ -206,7 +246,7 @@ __global__ void __launch_bounds__(64) causal_conv_wide_kernel(const TI* __restri
       acc[e] = base[e] + tap[0][e] * cur[e];
     }
 #pragma unroll
-    for (int j = 0; j < Q3_TAPS_MOST - 1; ++j)
+    for (int j = 0; j < MOST - 1; ++j)
       if (j < taps - 1) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) acc[e] += tap[j + 1][e] * win[j][e];
@@ -217,7 +257,7 @@ __global__ void __launch_bounds__(64) causal_conv_wide_kernel(const TI* __restri
     }
     store8(out + (size_t)t * C + c0, acc);
 #pragma unroll
-    for (int j = Q3_TAPS_MOST - 2; j > 0; --j) {
+    for (int j = MOST - 2; j > 0; --j) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) win[j][e] = win[j - 1][e];
     }
@@ -1281,12 +1321,12 @@ extern "C" int q3_causal_conv(const void* x, long x_stride, const float* in_bias
       (x_stride * in_size) % 16 == 0 && (C * out_size) % 16 == 0 && ((size_t)bias % 16) == 0 && ((size_t)w % 16) == 0 &&
       (!in_bias || ((size_t)in_bias % 16) == 0)) {
     const int wide_threads = 64;       // the kernel's shared memory is sized for this
-    const int wide_rows = Q3_CONV_TILE;
+    const dim3 tiles((T + Q3_CONV_TILE - 1) / Q3_CONV_TILE, (C / 8 + wide_threads - 1) / wide_threads);
     Q3_DISPATCH_DTYPE(in_dtype, TI, Q3_DISPATCH_DTYPE(out_dtype, TO, {
-                        hipLaunchKernelGGL((causal_conv_wide_kernel<TI, TO>),
-                                           dim3((T + wide_rows - 1) / wide_rows, (C / 8 + wide_threads - 1) / wide_threads),
-                                           dim3(wide_threads), 0, stream, (const TI*)x, x_stride, in_bias, w, bias, state,
-                                           state_stride, slots, cu, seq_index, (TO*)out, T, C, taps, act, wide_rows);
+                        hipLaunchKernelGGL((taps == 4 ? causal_conv_wide_kernel<TI, TO, 4>
+                                                      : causal_conv_wide_kernel<TI, TO, 0>),
+                                           tiles, dim3(wide_threads), 0, stream, (const TI*)x, x_stride, in_bias, w, bias,
+                                           state, state_stride, slots, cu, seq_index, (TO*)out, T, C, taps, act);
                       }));
   } else
   Q3_DISPATCH_DTYPE(in_dtype, TI, Q3_DISPATCH_DTYPE(out_dtype, TO, {

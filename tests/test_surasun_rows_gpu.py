@@ -91,3 +91,61 @@ def test_state_walked_row_by_row(dtype, rows, width, off, lengths):
     got = ops.mamba2_scan(xbc, dt, dt_bias, a_log, skip, a[:, off:], slots, cu, H, width, rows, 1, max_q_len=max(lengths))
     _close(got, twin.mamba2_scan(xbc, dt, dt_bias, a_log, skip, b[:, off:], slots, cu, H, width, rows, 1), 3e-5)
     _close(a, b, 3e-5)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("C,taps,lengths", [(8, 4, [256]), (520, 4, [1, 2, 255]), (512, 4, [263, 1]), (520, 8, [259]), (1024, 1, [256])])
+def test_causal_conv_tiles(dtype, C, taps, lengths):
+    """Tiles of eight rows whole and broken, of one sequence and of two, the exact taps and any number."""
+    g = _gen(C + taps)
+    x = _rand(g, sum(lengths), C, dtype=dtype)
+    weight, bias, add = _rand(g, C, taps), _rand(g, C), _rand(g, C)
+    cu, seq, slots = _step(lengths, [4, 0, 2][:len(lengths)])
+    full = _rand(g, 5, max(1, (taps - 1) * C))
+    for in_bias in (None, add):
+        a, b = full.clone(), full.clone()
+        state_a, state_b = a[:, :(taps - 1) * C], b[:, :(taps - 1) * C]
+        _close(ops.causal_conv(x, weight, bias, state_a, slots, cu, seq, "silu", dtype, in_bias, max_q_len=max(lengths)),
+               twin.causal_conv(x, weight, bias, state_b, slots, cu, seq, "silu", dtype, in_bias), _tol(dtype))
+        _close(a, b, 1e-6)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("H,G,dim,vdim,half,off", [(2, 1, 2, 1, 1, 0), (30, 2, 128, 128, 32, 0), (32, 2, 128, 64, 64, 0), (4, 4, 66, 512, 16, 2),
+                                                   (4, 4, 64, 516, 0, 0), (4, 2, 64, 64, 16, 1)])
+@pytest.mark.parametrize("transposed", [False, True])
+def test_capped_preparation_rows(dtype, H, G, dim, vdim, half, off, transposed):
+    """Rows that the registers hold (up to 4,096 numbers of q and k, 2,048 of v) and the next larger, on eight bytes or
+    not, a page that is missing, no cache."""
+    g = _gen(H * dim + vdim + off)
+    T, page = 5, 16
+    n = H * dim + G * dim + G * vdim
+    rows = _rand(g, T, n + off + n % 2)[:, off:off + n]
+    bias, qw, kw = _rand(g, n), _rand(g, H * dim), _rand(g, G * dim)
+    inv_freq = torch.rand(half, generator=g).to(DEV) if half else None
+    as_int = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    positions, seq, table = as_int([0, 17, 40, 3, 15]), as_int([0, 0, 0, 1, 1]), as_int([[2, 0, 3], [-1, 1, 1]])
+    def caches():
+        shape = (4, G, vdim, page) if transposed else (4, G, page, vdim)
+        return torch.zeros(4, G, page, dim, dtype=dtype, device=DEV), torch.zeros(shape, dtype=dtype, device=DEV)
+    for b in (bias, None):
+        mine, other = caches(), caches()
+        args = (rows, b, H, G, dim, vdim, qw, kw, 1e-6, inv_freq, positions, seq, dtype)
+        live = [0, 1, 2]        # (the twin takes no missing page: the second sequence's tokens only there)
+        got = ops.softcap_prepare(*args, table, *mine, values_transposed=transposed)
+        want = twin.softcap_prepare(rows[live], b, H, G, dim, vdim, qw, kw, 1e-6, inv_freq, positions[live], seq[live], dtype, table,
+                                    *other, values_transposed=transposed)
+        _close(got[live], want, _tol(dtype))
+        for x, y in zip(mine, other):
+            _close(x, y, _tol(dtype))
+        _close(ops.softcap_prepare(*args), twin.softcap_prepare(*args), _tol(dtype))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("W,off", [(4, 0), (260, 0), (4100, 0), (260, 1), (6, 0)])
+def test_embed_streams_rows(dtype, W, off):
+    table = _rand(_gen(W), 3 * W + off, dtype=dtype)[off:].view(3, W)
+    ids = torch.tensor([2, -1, 0, 3], dtype=torch.int32, device=DEV)      # (outside the table: zeros)
+    got = ops.embed_streams(ids, table, 3)
+    for t, row in enumerate((table[2].float(), torch.zeros(W, device=DEV), table[0].float(), torch.zeros(W, device=DEV))):
+        assert all(bool(torch.equal(got[t, s], row)) for s in range(3))
