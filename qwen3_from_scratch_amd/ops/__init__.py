@@ -91,11 +91,15 @@ class OperandError(ValueError):
     """An operand has a shape, dtype or placement the kernel does not take."""
 
 
+_void_p = ctypes.c_void_p
+
+
 def _ptr(t):
-    return ctypes.c_void_p(0 if t is None else t.data_ptr())
+    return None if t is None else _void_p(t.data_ptr())
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)   # the handle without a Stream object around it
+_raw_device = getattr(torch._C, "_cuda_getDevice", None)             # the index without a look at the initialisation
 
 
 def _stream():
@@ -103,7 +107,7 @@ def _stream():
     hundreds of times in a step that is not a graph replay, so the short way is taken where this
     PyTorch has it (a fifth of such a step's host time otherwise)."""
     if _raw_stream is not None:
-        return ctypes.c_void_p(_raw_stream(torch.cuda.current_device()))
+        return _void_p(_raw_stream(_raw_device() if _raw_device is not None else torch.cuda.current_device()))
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
@@ -116,8 +120,10 @@ def _dev(*tensors):
     for t in tensors:
         if t is None:
             continue
-        _need(t.is_cuda, "operands must be on the GPU; there is no host implementation")
-        _need(t.is_contiguous(), "operands must be contiguous")
+        if not t.is_cuda:
+            raise OperandError("operands must be on the GPU; there is no host implementation")
+        if not t.is_contiguous():
+            raise OperandError("operands must be contiguous")
 
 
 def _check(status, what):
@@ -340,20 +346,25 @@ def rmsnorm(x, weight, eps, out_dtype, delta=None, rows=None, write_back=True, o
     once to `out_dtype`. All arithmetic is float32.
     """
     _dev(x, weight, delta, rows, out)
-    _need(x.dim() == 2 and x.dtype == torch.float32, "x must be float32 (T, H)")
+    if not (x.dim() == 2 and x.dtype == torch.float32):
+        raise OperandError("x must be float32 (T, H)")
     T, H = x.shape
-    _need(weight.shape == (H,) and weight.dtype in _DT, "weight must be (H,) bfloat16 or float32")
-    _need(out_dtype in _DT, "out_dtype must be bfloat16 or float32")
+    if not (weight.shape == (H,) and weight.dtype in _DT):
+        raise OperandError("weight must be (H,) bfloat16 or float32")
+    if not (out_dtype in _DT):
+        raise OperandError("out_dtype must be bfloat16 or float32")
     if delta is not None:
-        _need(delta.shape == (T, H) and delta.dtype == out_dtype,
-              "delta must be (T, H) of the activation dtype")
+        if not (delta.shape == (T, H) and delta.dtype == out_dtype):
+            raise OperandError("delta must be (T, H) of the activation dtype")
     n_out = T
     if rows is not None:
-        _need(rows.dtype == torch.int32 and rows.dim() == 1, "rows must be int32 (R,)")
+        if not (rows.dtype == torch.int32 and rows.dim() == 1):
+            raise OperandError("rows must be int32 (R,)")
         n_out = rows.shape[0]
     if out is None:
         out = torch.empty((n_out, H), dtype=out_dtype, device=x.device)
-    _need(out.shape == (n_out, H) and out.dtype == out_dtype, "out must be (rows, H) of out_dtype")
+    if not (out.shape == (n_out, H) and out.dtype == out_dtype):
+        raise OperandError("out must be (rows, H) of out_dtype")
     if n_out:
         _check(library("norm").q3_rmsnorm(
             _ptr(x), _ptr(delta), _ptr(weight), _ptr(rows), _ptr(out), n_out, T, H,
@@ -1481,38 +1492,46 @@ def qk_norm_rope_store(qkv, num_q_heads, num_kv_heads, head_dim, positions, seq_
     if (cu_seqlens_q is None) != (kv_lens is None):
         raise OperandError("cu_seqlens_q and kv_lens are given together or not at all")
     if kv_lens is not None:
-        _need(kv_lens.dtype == torch.int32 and cu_seqlens_q.dtype == torch.int32
-              and cu_seqlens_q.shape == (kv_lens.shape[0] + 1,) and max_q_len > 0,
-              "cu_seqlens_q int32 (B+1,), kv_lens int32 (B,), max_q_len > 0")
+        if not (kv_lens.dtype == torch.int32 and cu_seqlens_q.dtype == torch.int32
+                and cu_seqlens_q.shape == (kv_lens.shape[0] + 1,) and max_q_len > 0):
+            raise OperandError("cu_seqlens_q int32 (B+1,), kv_lens int32 (B,), max_q_len > 0")
     Hq, Hkv, D = num_q_heads, num_kv_heads, head_dim
-    _need(qkv.dim() == 2 and qkv.shape[1] == (Hq + 2 * Hkv) * D and qkv.dtype in _DT,
-          "qkv must be (T, (Hq + 2 Hkv) D) bfloat16 or float32")
+    if not (qkv.dim() == 2 and qkv.shape[1] == (Hq + 2 * Hkv) * D and qkv.dtype in _DT):
+        raise OperandError("qkv must be (T, (Hq + 2 Hkv) D) bfloat16 or float32")
     T = qkv.shape[0]
-    _need(1 <= D <= 512, "head_dim must be in 1..512")
+    if not (1 <= D <= 512):
+        raise OperandError("head_dim must be in 1..512")
     for t in (positions, seq_index):
-        _need(t.dtype == torch.int32 and t.shape == (T,), "positions and seq_index must be int32 (T,)")
+        if not (t.dtype == torch.int32 and t.shape == (T,)):
+            raise OperandError("positions and seq_index must be int32 (T,)")
     w_dtype = 0
     if (q_weight is None) != (k_weight is None):
         raise OperandError("q_weight and k_weight are given together or not at all")
     if q_weight is not None:
-        _need(q_weight.shape == (D,) and k_weight.shape == (D,) and q_weight.dtype in _DT
-              and k_weight.dtype == q_weight.dtype, "norm weights must be (D,), same dtype")
+        if not (q_weight.shape == (D,) and k_weight.shape == (D,) and q_weight.dtype in _DT
+                and k_weight.dtype == q_weight.dtype):
+            raise OperandError("norm weights must be (D,), same dtype")
         w_dtype = _DT[q_weight.dtype]
     rotary_dim, max_pos = 0, 0
     if table is not None:
-        _need(table.dim() == 2 and table.dtype == torch.float32, "table must be float32 (P, R)")
+        if not (table.dim() == 2 and table.dtype == torch.float32):
+            raise OperandError("table must be float32 (P, R)")
         max_pos, rotary_dim = table.shape
-        _need(rotary_dim % 2 == 0 and rotary_dim <= D, "rotary dim must be even and at most D")
-        _need(max_kv_len <= max_pos, "the step reaches position %d, the rotation table ends at %d"
-              % (max_kv_len - 1, max_pos - 1))
+        if not (rotary_dim % 2 == 0 and rotary_dim <= D):
+            raise OperandError("rotary dim must be even and at most D")
+        if not (max_kv_len <= max_pos):
+            raise OperandError("the step reaches position %d, the rotation table ends at %d"
+                               % (max_kv_len - 1, max_pos - 1))
     page, stride = 0, 0
     if k_cache is not None:
-        _need(v_cache is not None and block_table is not None, "a cache needs k, v and a block table")
-        _need(k_cache.dim() == 4 and k_cache.shape[1] == Hkv and k_cache.shape[3] == D
-              and v_cache.shape == (k_cache.shape[0], Hkv, D, k_cache.shape[2])
-              and k_cache.dtype == qkv.dtype and v_cache.dtype == qkv.dtype,
-              "caches must be keys (pages, Hkv, page, D) and values (pages, Hkv, D, page) of the activation dtype")
-        _need(block_table.dim() == 2 and block_table.dtype == torch.int32, "block_table must be int32 (B, W)")
+        if not (v_cache is not None and block_table is not None):
+            raise OperandError("a cache needs k, v and a block table")
+        if not (k_cache.dim() == 4 and k_cache.shape[1] == Hkv and k_cache.shape[3] == D
+                and v_cache.shape == (k_cache.shape[0], Hkv, D, k_cache.shape[2])
+                and k_cache.dtype == qkv.dtype and v_cache.dtype == qkv.dtype):
+            raise OperandError("caches must be keys (pages, Hkv, page, D) and values (pages, Hkv, D, page) of the activation dtype")
+        if not (block_table.dim() == 2 and block_table.dtype == torch.int32):
+            raise OperandError("block_table must be int32 (B, W)")
         page, stride = k_cache.shape[2], block_table.shape[1]
     if T:
         _check(library("rotary").q3_qk_norm_rope_store(
@@ -1561,71 +1580,86 @@ def paged_attention(q, num_q_heads, k_cache, v_cache, block_table, cu_seqlens_q,
     _dev(k_cache, v_cache, block_table, cu_seqlens_q, kv_lens, out, sink)
     if sink is not None:
         _f32(sink, (num_q_heads,), "sink")
-    _need(q.is_cuda and q.dim() == 3 and q.stride(2) == 1 and q.stride(1) == q.shape[2],
-          "q must be (T, Hq, D) with contiguous heads")
+    if not (q.is_cuda and q.dim() == 3 and q.stride(2) == 1 and q.stride(1) == q.shape[2]):
+        raise OperandError("q must be (T, Hq, D) with contiguous heads")
     T, Hq, D = q.shape
-    _need(Hq == num_q_heads, "q's head count differs from num_q_heads")
-    _need(q.dtype in _DT and k_cache.dtype == q.dtype and v_cache.dtype == q.dtype,
-          "q and the caches must share bfloat16 or float32")
-    _need(k_cache.dim() == 4 and k_cache.shape[3] == D, "the key cache must be (pages, Hkv, page, D)")
+    if not (Hq == num_q_heads):
+        raise OperandError("q's head count differs from num_q_heads")
+    if not (q.dtype in _DT and k_cache.dtype == q.dtype and v_cache.dtype == q.dtype):
+        raise OperandError("q and the caches must share bfloat16 or float32")
+    if not (k_cache.dim() == 4 and k_cache.shape[3] == D):
+        raise OperandError("the key cache must be (pages, Hkv, page, D)")
     Hkv, page = k_cache.shape[1], k_cache.shape[2]
     vdim = v_cache.shape[2] if span is not None and v_cache.dim() == 4 else D       # in that build alone they may differ
-    _need(v_cache.shape == (k_cache.shape[0], Hkv, vdim, page), "the value cache must be (pages, Hkv, D, page)")
-    _need(Hq % Hkv == 0, "query heads must be a multiple of key heads")
-    _need(D % 16 == 0 and 16 <= D <= 256, "head_dim must be a multiple of 16 in 16..256, found %d" % D)
+    if not (v_cache.shape == (k_cache.shape[0], Hkv, vdim, page)):
+        raise OperandError("the value cache must be (pages, Hkv, D, page)")
+    if not (Hq % Hkv == 0):
+        raise OperandError("query heads must be a multiple of key heads")
+    if not (D % 16 == 0 and 16 <= D <= 256):
+        raise OperandError("head_dim must be a multiple of 16 in 16..256, found %d" % D)
     B = kv_lens.shape[0]
-    _need(cu_seqlens_q.dtype == torch.int32 and cu_seqlens_q.shape == (B + 1,), "cu_seqlens_q must be int32 (B+1,)")
-    _need(kv_lens.dtype == torch.int32, "kv_lens must be int32 (B,)")
-    _need(block_table.dim() == 2 and block_table.dtype == torch.int32 and block_table.shape[0] >= B,
-          "block_table must be int32 (B, W)")
-    _need(block_table.shape[1] * page >= max_kv_len, "block_table is narrower than the longest sequence")
-    _need(1 <= min_q_len <= max_q_len, "need 1 <= min_q_len <= max_q_len")
+    if not (cu_seqlens_q.dtype == torch.int32 and cu_seqlens_q.shape == (B + 1,)):
+        raise OperandError("cu_seqlens_q must be int32 (B+1,)")
+    if not (kv_lens.dtype == torch.int32):
+        raise OperandError("kv_lens must be int32 (B,)")
+    if not (block_table.dim() == 2 and block_table.dtype == torch.int32 and block_table.shape[0] >= B):
+        raise OperandError("block_table must be int32 (B, W)")
+    if not (block_table.shape[1] * page >= max_kv_len):
+        raise OperandError("block_table is narrower than the longest sequence")
+    if not (1 <= min_q_len <= max_q_len):
+        raise OperandError("need 1 <= min_q_len <= max_q_len")
     if out is None:
         out = torch.empty((T, Hq * vdim), dtype=q.dtype, device=q.device)
-    _need(out.shape == (T, Hq * vdim) and out.dtype == q.dtype, "out must be (T, Hq D)")
+    if not (out.shape == (T, Hq * vdim) and out.dtype == q.dtype):
+        raise OperandError("out must be (T, Hq D)")
     if T and B:
-        kinds = [kind for kind, on in (("capped", softcap > 0), ("pooled", runs is not None),
-                                       ("sigmoid", sigmoid_bias is not None), ("span", span is not None)) if on]
-        _need(len(kinds) <= 1, "capped scores, runs, sigmoid weights and spans exclude each other")
+        kinds = []
+        if softcap > 0 or runs is not None or sigmoid_bias is not None or span is not None:
+            kinds = [kind for kind, on in (("capped", softcap > 0), ("pooled", runs is not None),
+                                           ("sigmoid", sigmoid_bias is not None), ("span", span is not None)) if on]
+        if not (len(kinds) <= 1):
+            raise OperandError("capped scores, runs, sigmoid weights and spans exclude each other")
         lib = library("_".join(["attention"] + kinds))
         if kinds:
-            _need(lib.q3_paged_attention_fast_path(Hq, Hkv, D, page, _DT[q.dtype]) and q.stride(0) % 8 == 0,
-                  "capped scores, runs and sigmoid weights need bfloat16, a head size of 64 or 128 and pages of a power "
-                  "of two from 16; spans the sizes of span_sizes")
+            if not (lib.q3_paged_attention_fast_path(Hq, Hkv, D, page, _DT[q.dtype]) and q.stride(0) % 8 == 0):
+                raise OperandError("capped scores, runs and sigmoid weights need bfloat16, a head size of 64 or 128 and pages of a power "
+                                   "of two from 16; spans the sizes of span_sizes")
         if softcap > 0:
             lib.q3_set_score_cap.restype = None
             lib.q3_set_score_cap(ctypes.c_float(softcap))
         visible = int(max_kv_len)                      # keys that a row may see, for how they are shared out
         longest = visible if max_kv_len_of_many is None else int(max_kv_len_of_many)
         if runs is not None:
-            _need(window > 0 and runs[2].shape[0] >= B and max_kv_len // runs[3] <= runs[2].shape[1] * page,
-                  "runs stand behind a window, with a block table that covers them")
+            if not (window > 0 and runs[2].shape[0] >= B and max_kv_len // runs[3] <= runs[2].shape[1] * page):
+                raise OperandError("runs stand behind a window, with a block table that covers them")
             k_ptr, v_ptr, t_ptr, width, pool = _runs_args(runs, Hkv, page, D, D, q.dtype)
             lib.q3_set_runs.restype = None
             lib.q3_set_runs(k_ptr, v_ptr, t_ptr, width, runs[0].shape[0], pool)
             visible = min(visible, window + visible // pool)
             longest = min(longest, window + longest // pool)
         if sigmoid_bias is not None:
-            _need(sink is None and window == 0, "sigmoid weights take no sink and no window")
+            if not (sink is None and window == 0):
+                raise OperandError("sigmoid weights take no sink and no window")
             _f32(sigmoid_bias, (Hq,), "sigmoid_bias")
             lib.q3_set_sigmoid_bias.restype = None
             lib.q3_set_sigmoid_bias(_ptr(sigmoid_bias))
         if span is not None:
             chunk, keep = int(span[0]), int(span[1])
-            _need(span_sizes(Hq, Hkv, D, vdim, page, q.dtype) and chunk >= 0 and keep >= 0 and not (chunk and window),
-                  "a span is a chunk or a window, and first keys, of sizes that span_sizes takes")
+            if not (span_sizes(Hq, Hkv, D, vdim, page, q.dtype) and chunk >= 0 and keep >= 0 and not (chunk and window)):
+                raise OperandError("a span is a chunk or a window, and first keys, of sizes that span_sizes takes")
             lib.q3_set_span.restype = None
             lib.q3_set_span(chunk, keep, vdim)
             if chunk or window:
                 visible = min(visible, (chunk or window) + keep)
                 longest = min(longest, (chunk or window) + keep)
-        _need(gate is None or runs is not None or sigmoid_bias is not None or span is not None,
-              "a gate comes with runs, sigmoid weights or spans only")
+        if not (gate is None or runs is not None or sigmoid_bias is not None or span is not None):
+            raise OperandError("a gate comes with runs, sigmoid weights or spans only")
         if runs is not None or sigmoid_bias is not None or span is not None:
             gate_stride = 0
             if gate is not None:
                 gate_stride = _rows_view(gate, "gate")
-                _need(gate.shape in ((T, Hq), (T, Hq * vdim)) and gate.dtype == torch.float32, "gate must be float32 (T, Hq) or (T, Hq D)")
+                if not (gate.shape in ((T, Hq), (T, Hq * vdim)) and gate.dtype == torch.float32):
+                    raise OperandError("gate must be float32 (T, Hq) or (T, Hq D)")
             lib.q3_set_gate.restype = None
             lib.q3_set_gate(_ptr(gate), ctypes.c_long(gate_stride), 1 if gate is not None and gate.shape[1] != Hq else 0)
         splits, workspace, prompt_splits, prompt_workspace = 1, None, 1, None
@@ -1712,27 +1746,38 @@ def decode_attention(qkv, num_q_heads, num_kv_heads, head_dim, k_cache, v_cache,
     _dev(qkv, k_cache, v_cache, block_table, cu_seqlens_q, kv_lens, q_weight, k_weight, table)
     Hq, Hkv, D = num_q_heads, num_kv_heads, head_dim
     B = kv_lens.shape[0]
-    _need(qkv.dtype == torch.bfloat16 and qkv.shape == (B, (Hq + 2 * Hkv) * D), "qkv must be bfloat16 (B, (Hq + 2 Hkv) D)")
-    _need(k_cache.dtype == torch.bfloat16 and v_cache.dtype == torch.bfloat16 and k_cache.dim() == 4
-          and k_cache.shape[1] == Hkv and k_cache.shape[3] == D, "key cache must be bfloat16 (pages, Hkv, page, D)")
+    if not (qkv.dtype == torch.bfloat16 and qkv.shape == (B, (Hq + 2 * Hkv) * D)):
+        raise OperandError("qkv must be bfloat16 (B, (Hq + 2 Hkv) D)")
+    if not (k_cache.dtype == torch.bfloat16 and v_cache.dtype == torch.bfloat16 and k_cache.dim() == 4
+            and k_cache.shape[1] == Hkv and k_cache.shape[3] == D):
+        raise OperandError("key cache must be bfloat16 (pages, Hkv, page, D)")
     page = k_cache.shape[2]
-    _need(v_cache.shape == (k_cache.shape[0], Hkv, D, page), "value cache must be (pages, Hkv, D, page)")
-    _need(block_table.dtype == torch.int32 and block_table.dim() == 2 and block_table.shape[0] >= B, "block table int32 (B, blocks)")
-    _need(cu_seqlens_q.dtype == torch.int32 and cu_seqlens_q.shape == (B + 1,), "cu_seqlens_q int32 (B + 1,)")
-    _need(kv_lens.dtype == torch.int32, "kv_lens int32 (B,)")
-    _need((q_weight is None) == (k_weight is None), "q and k norm weights come together")
+    if not (v_cache.shape == (k_cache.shape[0], Hkv, D, page)):
+        raise OperandError("value cache must be (pages, Hkv, D, page)")
+    if not (block_table.dtype == torch.int32 and block_table.dim() == 2 and block_table.shape[0] >= B):
+        raise OperandError("block table int32 (B, blocks)")
+    if not (cu_seqlens_q.dtype == torch.int32 and cu_seqlens_q.shape == (B + 1,)):
+        raise OperandError("cu_seqlens_q int32 (B + 1,)")
+    if not (kv_lens.dtype == torch.int32):
+        raise OperandError("kv_lens int32 (B,)")
+    if not ((q_weight is None) == (k_weight is None)):
+        raise OperandError("q and k norm weights come together")
     w_dtype = 0
     if q_weight is not None:
-        _need(q_weight.shape == (D,) and k_weight.shape == (D,) and q_weight.dtype == k_weight.dtype
-              and q_weight.dtype in _DT, "norm weights (D,) of one dtype")
+        if not (q_weight.shape == (D,) and k_weight.shape == (D,) and q_weight.dtype == k_weight.dtype
+                and q_weight.dtype in _DT):
+            raise OperandError("norm weights (D,) of one dtype")
         w_dtype = _DT[q_weight.dtype]
     rotary_dim = max_pos = 0
     if table is not None:
-        _need(table.dtype == torch.float32 and table.dim() == 2, "rotation table float32 (positions, rotary_dim)")
+        if not (table.dtype == torch.float32 and table.dim() == 2):
+            raise OperandError("rotation table float32 (positions, rotary_dim)")
         max_pos, rotary_dim = table.shape
-        _need(max_kv_len <= max_pos, "the step reaches position %d, the rotation table ends at %d"
-              % (max_kv_len - 1, max_pos - 1))
-    _need(decode_attention_takes(Hq, Hkv, D, page, qkv.dtype, rotary_dim), "sizes the decoding kernel does not take")
+        if not (max_kv_len <= max_pos):
+            raise OperandError("the step reaches position %d, the rotation table ends at %d"
+                               % (max_kv_len - 1, max_pos - 1))
+    if not (decode_attention_takes(Hq, Hkv, D, page, qkv.dtype, rotary_dim)):
+        raise OperandError("sizes the decoding kernel does not take")
     out = torch.empty((B, Hq * D), dtype=qkv.dtype, device=qkv.device)
     if B:
         lib = library("attention")
@@ -1791,16 +1836,17 @@ def _tiled_ok(tiled, weight, M):
     if tiled is None or not 1 <= M <= few_rows_limit(weight):
         return False
     N, K = weight.shape
-    _need(tiled.is_cuda and tiled.dtype == torch.bfloat16 and tiled.is_contiguous()
-          and tiled.numel() == (-(-N // 16) * 16) * K and K % 32 == 0,
-          "the tiled copy does not belong to this weight")
+    if not (tiled.is_cuda and tiled.dtype == torch.bfloat16 and tiled.is_contiguous()
+            and tiled.numel() == (-(-N // 16) * 16) * K and K % 32 == 0):
+        raise OperandError("the tiled copy does not belong to this weight")
     return True
 
 
 def _check_sums(sums, M):
     _dev(sums)
-    _need(sums.dtype == torch.float32 and sums.dim() == 2 and sums.shape[1] == sums_stride(M) and sums.shape[0] > 0
-          and sums.is_contiguous(), "row sums must be float32 (P, M rounded up to 16)")
+    if not (sums.dtype == torch.float32 and sums.dim() == 2 and sums.shape[1] == sums_stride(M) and sums.shape[0] > 0
+            and sums.is_contiguous()):
+        raise OperandError("row sums must be float32 (P, M rounded up to 16)")
 
 
 def _row_sums_args(unscaled, M, K):
@@ -1841,8 +1887,10 @@ def _tiles_scaled(x, weight, out, unscaled, swiglu, what):
     sums, eps, width = unscaled
     M, K = x.shape
     _check_sums(sums, M)
-    _need(width == K, "the rows' width must be the product's inner size")
-    _need(x.is_contiguous() and out.is_contiguous(), "operands must be contiguous")
+    if not (width == K):
+        raise OperandError("the rows' width must be the product's inner size")
+    if not (x.is_contiguous() and out.is_contiguous()):
+        raise OperandError("operands must be contiguous")
     _check(_matmul().q3_tiles_scaled(
         _ptr(x), _ptr(weight), _ptr(out), M, weight.shape[0], K, _DT[out.dtype], 1 if swiglu else 0, _ptr(sums),
         sums.shape[0], sums.shape[1], ctypes.c_float(eps), int(width), _stream()), what)
@@ -1902,16 +1950,21 @@ def linear(x, weight, out_dtype=None, out=None, tiled=None, unscaled=None):
     more rows is the vendor library's product or the tiled kernel's.
     """
     _dev(x, weight, out)
-    _need(x.dim() == 2 and weight.dim() == 2 and x.shape[1] == weight.shape[1], "x (M, K) and weight (N, K)")
-    _need(x.dtype in _DT and weight.dtype == x.dtype, "x and weight must share bfloat16 or float32")
+    if not (x.dim() == 2 and weight.dim() == 2 and x.shape[1] == weight.shape[1]):
+        raise OperandError("x (M, K) and weight (N, K)")
+    if not (x.dtype in _DT and weight.dtype == x.dtype):
+        raise OperandError("x and weight must share bfloat16 or float32")
     M, K = x.shape
     N = weight.shape[0]
     out_dtype = out_dtype or x.dtype
-    _need(out_dtype in _DT, "out dtype must be bfloat16 or float32")
-    _need(not (x.dtype == torch.float32 and out_dtype != torch.float32), "float32 inputs give float32 output")
+    if not (out_dtype in _DT):
+        raise OperandError("out dtype must be bfloat16 or float32")
+    if not (not (x.dtype == torch.float32 and out_dtype != torch.float32)):
+        raise OperandError("float32 inputs give float32 output")
     if out is None:
         out = torch.empty((M, N), dtype=out_dtype, device=x.device)
-    _need(out.shape == (M, N) and out.dtype == out_dtype, "out must be (M, N) of out_dtype")
+    if not (out.shape == (M, N) and out.dtype == out_dtype):
+        raise OperandError("out must be (M, N) of out_dtype")
     if M and x.dtype == torch.bfloat16 and _tiled_ok(tiled, weight, M):
         sums, sums_rows, eps, width, stride = _row_sums_args(unscaled, M, K)
         _check(library("gemm").q3_linear_tiled(
@@ -1923,14 +1976,16 @@ def linear(x, weight, out_dtype=None, out=None, tiled=None, unscaled=None):
         return out
     if unscaled is not None and x.dtype == torch.bfloat16 and fused_rows_take(weight, M):
         return _tiles_scaled(x, weight, out, unscaled, False, "linear")
-    _need(unscaled is None, "unscaled rows need bfloat16 and few rows with a tiled weight (few_rows_limit), or 17 to "
-          "128 rows (640 of a small weight, fused_rows_most) with an inner size that is a multiple of 64")
+    if not (unscaled is None):
+        raise OperandError("unscaled rows need bfloat16 and few rows with a tiled weight (few_rows_limit), or 17 to "
+                           "128 rows (640 of a small weight, fused_rows_most) with an inner size that is a multiple of 64")
     if M and x.dtype == torch.bfloat16 and not library("gemm").q3_linear_is_skinny(M, N, K, 1):
         # bfloat16 products with many rows go to the vendor library (hipBLASLt), as the
         # reference's engine uses its vendor library for them, or to the hand-written tiled
         # kernel, as a table of sizes and a rule of thumb say; accumulation is float32.
         # Few rows take the weight-streaming kernel below.
-        _need(x.is_contiguous() and weight.is_contiguous() and out.is_contiguous(), "operands must be contiguous")
+        if not (x.is_contiguous() and weight.is_contiguous() and out.is_contiguous()):
+            raise OperandError("operands must be contiguous")
         status = _matmul().q3_matmul(_ptr(x), _ptr(weight), _ptr(out), M, N, K, _DT[out_dtype], _stream())
         if status == _UNSUPPORTED:
             # a size neither hipBLASLt nor the tiled kernel has a kernel for (an odd inner size,
@@ -1973,19 +2028,22 @@ def linear_swiglu(x, weight, tiled=None, unscaled=None, kind="silu"):
     bfloat16 rows the activation is the product kernel's epilogue (silu in every kernel for up to 128 rows, the
     tanh form of gelu in the few-row and the weight-streaming kernel, the exact gelu nowhere); otherwise
     it is the product followed by `gated_act`, with the same bits. `unscaled`: as for `linear`."""
-    _need(kind in GATE_KINDS, "kind is one of %s" % ", ".join(sorted(GATE_KINDS)))
+    if not (kind in GATE_KINDS):
+        raise OperandError("kind is one of %s" % ", ".join(sorted(GATE_KINDS)))
     if kind == "gelu_erf":
         return gated_act(linear(x, weight, tiled=tiled, unscaled=unscaled), kind)
     _dev(x, weight)
-    _need(x.dim() == 2 and weight.dim() == 2 and x.shape[1] == weight.shape[1] and weight.shape[0] % 2 == 0,
-          "x (M, K) and weight (2I, K)")
-    _need(x.dtype in _DT and weight.dtype == x.dtype, "x and weight must share bfloat16 or float32")
+    if not (x.dim() == 2 and weight.dim() == 2 and x.shape[1] == weight.shape[1] and weight.shape[0] % 2 == 0):
+        raise OperandError("x (M, K) and weight (2I, K)")
+    if not (x.dtype in _DT and weight.dtype == x.dtype):
+        raise OperandError("x and weight must share bfloat16 or float32")
     M, K = x.shape
     N = weight.shape[0]
     if x.dtype == torch.bfloat16 and tiled is not None and STREAM_ROWS_LEAST <= M <= FEW_ROWS and N % 4 == 0:
         # a whole gate/up product of 9 to 16 rows: the streaming kernel, where it takes the size
         if unscaled is not None:
-            _need(unscaled[0].dim() == 2 and unscaled[0].shape[1] == sums_stride(M), "row sums (P, M rounded up to 16)")
+            if not (unscaled[0].dim() == 2 and unscaled[0].shape[1] == sums_stride(M)):
+                raise OperandError("row sums (P, M rounded up to 16)")
         out = torch.empty((M, N // 2), dtype=x.dtype, device=x.device)
         if _stream_product(x, weight, tiled, out, True, unscaled, "linear_swiglu", kind):
             return out
@@ -2006,8 +2064,9 @@ def linear_swiglu(x, weight, tiled=None, unscaled=None, kind="silu"):
     if unscaled is not None and x.dtype == torch.bfloat16 and fused_rows_take(weight, M):
         out = torch.empty((M, N // 2), dtype=x.dtype, device=x.device)
         return _tiles_scaled(x, weight, out, unscaled, True, "linear_swiglu")
-    _need(unscaled is None, "unscaled rows need bfloat16 and few rows with a tiled weight (few_rows_limit), or 17 to "
-          "128 rows (640 of a small weight, fused_rows_most) with an inner size that is a multiple of 64")
+    if not (unscaled is None):
+        raise OperandError("unscaled rows need bfloat16 and few rows with a tiled weight (few_rows_limit), or 17 to "
+                           "128 rows (640 of a small weight, fused_rows_most) with an inner size that is a multiple of 64")
     if M and library("gemm").q3_linear_is_skinny(M, N, K, _DT[x.dtype]):
         out = torch.empty((M, N // 2), dtype=x.dtype, device=x.device)
         _check(library("gemm").q3_linear_swiglu(_ptr(x), _ptr(weight), _ptr(out), M, N, K, _DT[x.dtype], _stream()),
@@ -2034,16 +2093,19 @@ def linear_residual_norm(x, weight, tiled, residual, norm_weight):
     nothing was done, for a size at which the plain product (`linear`) followed by the norm's own
     kernel is the faster way."""
     _dev(x, weight, tiled, residual, norm_weight)
-    _need(x.dim() == 2 and weight.dim() == 2 and x.shape[1] == weight.shape[1], "x (M, K) and weight (N, K)")
+    if not (x.dim() == 2 and weight.dim() == 2 and x.shape[1] == weight.shape[1]):
+        raise OperandError("x (M, K) and weight (N, K)")
     M, K = x.shape
     N = weight.shape[0]
-    _need(residual.shape == (M, N) and residual.dtype == torch.float32 and residual.is_contiguous(),
-          "residual must be float32 (M, N)")
-    _need(norm_weight.shape == (N,) and norm_weight.dtype in _DT and norm_weight.is_contiguous(), "norm weight (N,)")
+    if not (residual.shape == (M, N) and residual.dtype == torch.float32 and residual.is_contiguous()):
+        raise OperandError("residual must be float32 (M, N)")
+    if not (norm_weight.shape == (N,) and norm_weight.dtype in _DT and norm_weight.is_contiguous()):
+        raise OperandError("norm weight (N,)")
     values = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
     few = x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and N % 16 == 0 and _tiled_ok(tiled, weight, M)
     if not few and x.dtype == torch.bfloat16 and fused_rows_take(weight, M):
-        _need(x.is_contiguous(), "x must be contiguous")
+        if not (x.is_contiguous()):
+            raise OperandError("x must be contiguous")
         lib = _matmul()
         sums = torch.empty((lib.q3_tiles_residual_chunks(N), sums_stride(M)), dtype=torch.float32, device=x.device)
         status = lib.q3_tiles_residual(
@@ -2053,8 +2115,9 @@ def linear_residual_norm(x, weight, tiled, residual, norm_weight):
             return None
         _check(status, "linear_residual_norm")
         return values, sums
-    _need(few, "bfloat16, a tiled weight with a width that is a multiple of 16 and no more rows than few_rows_limit, "
-          "or 17 to 128 rows (640 of a small weight, fused_rows_most) with an inner size that is a multiple of 64")
+    if not (few):
+        raise OperandError("bfloat16, a tiled weight with a width that is a multiple of 16 and no more rows than few_rows_limit, "
+                           "or 17 to 128 rows (640 of a small weight, fused_rows_most) with an inner size that is a multiple of 64")
     sums = torch.empty((N // 16, sums_stride(M)), dtype=torch.float32, device=x.device)
     _check(library("gemm").q3_linear_tiled(
         _ptr(x), _ptr(tiled), _ptr(values), M, N, K, 1, 2, None, 0, ctypes.c_float(0.0), 0,
