@@ -1574,7 +1574,8 @@ def paged_attention(q, num_q_heads, k_cache, v_cache, block_table, cu_seqlens_q,
     over several blocks; `max_kv_len` stands in).
 
     bfloat16 with head size 64 or 128 and a page size that is a power of two from 16
-    runs on the matrix cores; everything else (float32, other head sizes in
+    runs on the matrix cores, and so do float32 heads of 16, 32, 64 and 128 over pages in steps
+    of 16 with at most 16 query heads a key head (in float32); everything else (other head sizes in
     steps of 16 up to 256, other page sizes) takes the general kernel.
     """
     _dev(k_cache, v_cache, block_table, cu_seqlens_q, kv_lens, out, sink)
@@ -2002,7 +2003,8 @@ def linear(x, weight, out_dtype=None, out=None, tiled=None, unscaled=None):
 def linear_plain(x, weight, out):
     """out = x @ weight^T by plain multiply-adds with float32 sums, for any size: what serves a
     bfloat16 product with more than 16 rows that neither the vendor library nor the tiled
-    kernel takes, and every float32 product."""
+    kernel takes, and every float32 product (from 17 rows on by the matrix cores' float32
+    instruction where the rows can be read sixteen bytes at a time, with the same bits)."""
     _dev(x, weight, out)
     _need(x.dim() == 2 and weight.dim() == 2 and x.shape[1] == weight.shape[1] and x.dtype in _DT
           and weight.dtype == x.dtype, "x (M, K) and weight (N, K) of one dtype")
