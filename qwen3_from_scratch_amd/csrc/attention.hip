@@ -587,7 +587,8 @@ __device__ __forceinline__ TilePages tile_pages(const int* __restrict__ bt_row, 
 // kb is key 8 (m / 4) + 4 kb + m % 4. The values of those keys are then one 16-byte load per 16 columns. A half
 // that is not there points at the cache's first page, so that no load waits behind a branch (with the loads
 // guarded one by one, the compiler waited for each before it asked for the next: 4,000 of the 17,000 cycles a
-// block took for one request over 1,100 keys), and `there` says whose loads count.
+// block took for one request over 1,100 keys), and `there` says whose loads count. A first page there is, also with
+// `num_pages` 0: whoever launches a kernel that comes here sees to it.
 struct TileAddr {
   const bf16_t* k;   // the lane's key row of product 0, from element 8 g on; product 1's is four keys on
   const bf16_t* v;   // the lane's first value row, from key 8 g on; its others are 16 rows apart
@@ -2165,6 +2166,7 @@ extern "C" int q3_paged_attention(const void* q, int q_stride, void* out, const 
     if (prompt_splits < 1 || prompt_splits > 4 || (prompt_splits > 1 && prompt_workspace == nullptr))
       return Q3_ERR_BAD_ARGUMENT;
     (void)max_kv_len;
+    if (!k_cache || !v_cache) return Q3_ERR_BAD_ARGUMENT;    // (tiles without a page read the first one: TileAddr)
     float* ws_acc = workspace;
 #ifdef Q3_SPAN
     const int DV = g_span_value_dim;
@@ -2245,6 +2247,7 @@ extern "C" int q3_decode_attention(const void* qkv, void* out, void* k_cache, vo
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv || page <= 0) return Q3_ERR_BAD_ARGUMENT;
   if (B > 65535) return Q3_ERR_UNSUPPORTED;
   if (!q3_decode_attention_takes(Hq, Hkv, D, page, Q3_BF16, table ? rotary_dim : 0)) return Q3_ERR_UNSUPPORTED;
+  if (!k_cache || !v_cache) return Q3_ERR_BAD_ARGUMENT;      // (tiles without a page read the first one: TileAddr)
   if ((q_weight == nullptr) != (k_weight == nullptr)) return Q3_ERR_BAD_ARGUMENT;
   if (q_weight && w_dtype != Q3_F32 && w_dtype != Q3_BF16) return Q3_ERR_BAD_ARGUMENT;
   if (splits < 1 || splits > MAX_SPLITS || (splits > 1 && workspace == nullptr)) return Q3_ERR_BAD_ARGUMENT;

@@ -1545,6 +1545,14 @@ def qk_norm_rope_store(qkv, num_q_heads, num_kv_heads, head_dim, positions, seq_
     return qkv
 
 
+def _with_a_page(k_cache, v_cache):
+    """The caches, or a page of each in the place of caches without any. The decoding kernels' loads wait behind no branch:
+    where a tile has no page they read the cache's first, which has to be memory, and count it as zeros."""
+    if k_cache.shape[0]:
+        return k_cache, v_cache
+    return k_cache.new_empty((1,) + k_cache.shape[1:]), v_cache.new_empty((1,) + v_cache.shape[1:])
+
+
 def paged_attention(q, num_q_heads, k_cache, v_cache, block_table, cu_seqlens_q, kv_lens,
                     max_q_len, max_kv_len, scale, window=0, out=None, min_q_len=1, max_kv_len_of_many=None, softcap=0.0,
                     sink=None, runs=None, sigmoid_bias=None, gate=None, span=None):
@@ -1676,8 +1684,10 @@ def paged_attention(q, num_q_heads, k_cache, v_cache, block_table, cu_seqlens_q,
                 if prompt_splits > 1:
                     prompt_workspace = torch.empty((T * Hq * prompt_splits * (vdim + 2),), dtype=torch.float32,
                                                    device=q.device)
+        pages = k_cache.shape[0]
+        k_cache, v_cache = _with_a_page(k_cache, v_cache)
         _check(lib.q3_paged_attention(
-            _ptr(q), q.stride(0), _ptr(out), _ptr(k_cache), _ptr(v_cache), k_cache.shape[0],
+            _ptr(q), q.stride(0), _ptr(out), _ptr(k_cache), _ptr(v_cache), pages,
             _ptr(block_table), block_table.shape[1], _ptr(cu_seqlens_q), _ptr(kv_lens),
             B, T, Hq, Hkv, D, page, ctypes.c_float(scale), int(window), int(max_q_len), int(min_q_len),
             int(max_kv_len), _DT[q.dtype], splits, _ptr(workspace), prompt_splits, _ptr(prompt_workspace), _ptr(sink),
@@ -1787,11 +1797,13 @@ def decode_attention(qkv, num_q_heads, num_kv_heads, head_dim, k_cache, v_cache,
             lib.q3_paged_attention_workspace.restype = ctypes.c_long
             workspace = torch.empty((lib.q3_paged_attention_workspace(B, Hkv, D, splits),), dtype=torch.float32,
                                     device=qkv.device)
+        pages = k_cache.shape[0]
+        k_cache, v_cache = _with_a_page(k_cache, v_cache)
         _check(lib.q3_decode_attention(
-            _ptr(qkv), _ptr(out), _ptr(k_cache), _ptr(v_cache), k_cache.shape[0], _ptr(block_table),
+            _ptr(qkv), _ptr(out), _ptr(k_cache), _ptr(v_cache), pages, _ptr(block_table),
             block_table.shape[1], _ptr(cu_seqlens_q), _ptr(kv_lens), B, Hq, Hkv, D, page, ctypes.c_float(scale),
             int(window), splits, _ptr(workspace), _ptr(q_weight), _ptr(k_weight), w_dtype, ctypes.c_float(eps),
-            _ptr(table), int(rotary_dim), int(max_pos), 1 if store else 0, int(max_kv_len), _stream()),
+            _ptr(table), int(rotary_dim), int(max_pos), 1 if store and pages else 0, int(max_kv_len), _stream()),
             "decode_attention")
     return out
 
