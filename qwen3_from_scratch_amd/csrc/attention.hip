@@ -240,12 +240,12 @@ __global__ __launch_bounds__(512) void attn_f32_mma_kernel(
       sc[i] = seen ? s4[i] * scale : -INFINITY;
     }
     const float m_new = fmaxf(m_run, quad_rows_max(fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]))));
-    float alpha = 1.f, p[4] = {0.f, 0.f, 0.f, 0.f};
-    if (m_new > -INFINITY) {
-      alpha = expf(m_run - m_new);
+    // (no number among the scores yet: hidden keys count exp(-inf) = 0, and a NaN, which no maximum keeps, stays one)
+    const float m_use = m_new > -INFINITY ? m_new : 0.f;
+    const float alpha = expf(m_run - m_use);
+    float p[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) p[i] = expf(sc[i] - m_new);
-    }
+    for (int i = 0; i < 4; ++i) p[i] = expf(sc[i] - m_use);
     l_run = l_run * alpha + ((p[0] + p[1]) + (p[2] + p[3]));
     m_run = m_new;
 #pragma unroll

@@ -92,3 +92,15 @@ def test_attention_float32(Hq, Hkv, D, page, window, with_sink):
         one = (q[first + i:first + i + 1], kc, vc, bt[4:5], torch.tensor([0, 1], dtype=torch.int32).cuda(),
                torch.tensor([150 - 37 + i + 1], dtype=torch.int32).cuda())
         assert torch.equal(_attention(ops, one, Hq, scale, window=window, sink=sink)[0], got[first + i])
+
+
+@pytest.mark.parametrize("L,at", [(1, 0), (16, 15), (17, 16), (33, 32), (200, 100), (129, 128)])
+def test_attention_float32_keeps_a_nan(L, at):
+    """A key of NaN is seen in the result, also where it is the only key of its tile and no wavefront has another; a row
+    before it does not look."""
+    ops = _ops()
+    q, kc, vc, bt, cu, kvl = _paged_case(torch.float32, 1, 4, 2, 64, 16, [min(2, L)], [L], 73)
+    kc[int(bt[0, at // 16]), :, at % 16] = float("nan")
+    got = _attention(ops, (q, kc, vc, bt, cu, kvl), 4, 0.125)
+    assert bool(got[-1].isnan().all())
+    assert L == 1 or bool(got[0].isnan().all()) == (at < L - 1)
