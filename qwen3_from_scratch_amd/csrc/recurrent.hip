@@ -754,15 +754,18 @@ struct StateColumns {
     }
   }
   // S = decay S + key push, and what the rows of the wavefront give of sum_n S[n] query[n] into part[wave]; `keys` and
-  // `queries` hold zeros past the rows that exist.
-  __device__ void step(float decay, const float* keys, const float* queries, const float (&push)[4], int group, float (*part)[64]) {
+  // `queries` hold zeros past the `rows` that exist, whose state stays zero whatever `push` is (zero times infinity is NaN).
+  // (more than 8 EACH rows exist where EACH is above its least: the first half of a thread's rows always do)
+  __device__ void step(float decay, const float* keys, const float* queries, const float (&push)[4], int rows, int group,
+                       float (*part)[64]) {
     float acc[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int k = 0; k < EACH; ++k) {
       const float key = keys[group + 16 * k], query = queries[group + 16 * k];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        S[k][e] = decay * S[k][e] + key * push[e];
+        const float grown = decay * S[k][e] + key * push[e];
+        S[k][e] = (EACH > 2 && k < EACH / 2) || group + 16 * k < rows ? grown : 0.f;
         acc[e] += S[k][e] * query;
       }
     }
@@ -817,7 +820,7 @@ __global__ void __launch_bounds__(256) mamba2_scan_kernel(
       rb = row[at_b], rc = row[at_b + G * N], ro = row[h * P + (own < P ? own : 0)], rd = dt[(size_t)(t + 1) * dt_stride + h];
       rx.template load<false>(row + h * P, column, P);
     }
-    at.step(decay, sB, sC, push, group, part);
+    at.step(decay, sB, sC, push, N, group, part);
     __syncthreads();
     if (tid < 64 && own < P)
       y[((size_t)t * H + h) * P + own] = ((part[0][tid] + part[1][tid]) + (part[2][tid] + part[3][tid])) + skip * x_own;
@@ -880,7 +883,7 @@ __global__ void __launch_bounds__(256) retention_scan_kernel(
       position = positions[t + 1];
       rv.template load<false>(rows + (size_t)(t + 1) * width + 2 * hd + h * vdim, column, vdim);
     }
-    at.step(decay, sk, sq, push, group, part);
+    at.step(decay, sk, sq, push, dim, group, part);
     __syncthreads();
     if (tid < 64 && own < vdim)
       raw[(size_t)t * hv + h * vdim + own] = (part[0][tid] + part[1][tid]) + (part[2][tid] + part[3][tid]);

@@ -93,6 +93,22 @@ def test_state_walked_row_by_row(dtype, rows, width, off, lengths):
     _close(a, b, 3e-5)
 
 
+@pytest.mark.parametrize("rows", [1, 16, 20, 32, 48, 66, 130])
+def test_state_walked_with_an_infinite_input(rows):
+    """An infinity in one column stays there, and one: rows that fill a state up to 16 EACH make no NaN of it."""
+    H, P = 2, 8
+    xbc, zero = torch.ones(2, H * P + 2 * rows, device=DEV), torch.zeros(H, device=DEV)
+    xbc[0, 3] = float("inf")
+    cu, _, slots = _step([2], [0])
+    a, b = torch.zeros(1, H * rows * P, device=DEV), torch.zeros(1, H * rows * P, device=DEV)
+    args = (xbc, torch.zeros(2, H, device=DEV), zero, zero, zero + 1)
+    got = ops.mamba2_scan(*args, a, slots, cu, H, P, rows, 1, max_q_len=2)
+    want = twin.mamba2_scan(*args, b, slots, cu, H, P, rows, 1)
+    assert bool(want[:, 3].isinf().all()) and torch.equal(got.isinf(), want.isinf()) and not bool(got.isnan().any())
+    torch.testing.assert_close(got[want.isfinite()], want[want.isfinite()], rtol=1e-5, atol=0)
+    assert torch.equal(a.isinf(), b.isinf())
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("C,taps,lengths", [(8, 4, [256]), (520, 4, [1, 2, 255]), (512, 4, [263, 1]), (520, 8, [259]), (1024, 1, [256])])
 def test_causal_conv_tiles(dtype, C, taps, lengths):
