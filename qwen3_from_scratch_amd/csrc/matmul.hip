@@ -257,10 +257,11 @@ Choice plain_by_rule(int M, int N, int K) {
 // 14.4 / 13.5, of 1,024 x 4,096 in eight shares 13.3 / 13.8 / 16.5; 400 rows of the last, in four, 17.4 / 15.7 / 16.7; 400
 // of 8,192 x 1,024 (448 tiles) 16.4 / 20.6 / 15.5 / 15.5; 532 of it (320 tiles of 128 x 128) 23.3 / 29.4 / 20.9 / 17.4.
 Choice fused_by_rule(int kind, int M, int N, int K) {
-  (void)kind;
   Choice c;
   if (g_kernels == KERNELS_LIBRARY) return c;
   if (M > 128) {
+    // (a residual's product always goes through partial products; where not even one share's fit, it is declined)
+    if (kind == KIND_RESIDUAL && (size_t)M * N * sizeof(float) > PARTIALS_BYTES) return c;
     const long small = (long)((M + 63) / 64) * ((N + 127) / 128), large = (long)((M + 127) / 128) * ((N + 127) / 128);
     if (small > 256 && large > 256 && g_kernels == KERNELS_BOTH) return c;
     c.own = small > 256 ? 1 : 5;

@@ -24,6 +24,19 @@ def test_rows_and_weights_that_take_part():
     assert [ops.fused_rows_take(w, 129) for w in (large, tiny)] == [False, False]
 
 
+def test_a_stream_too_wide_for_the_partial_products():
+    """640 rows of 65,536 columns: the plain product and the norm's own kernel, whichever kernels are asked for."""
+    ops = _ops()
+    x, w = (torch.ones(n, 64, dtype=torch.bfloat16, device="cuda") for n in (640, 65536))
+    residual = torch.zeros(640, 65536, device="cuda")
+    for which in ("own", "both"):
+        ops.matmul_kernels(which)
+        try:
+            assert ops.linear_residual_norm(x, w, None, residual, torch.ones(65536, device="cuda")) is None
+        finally:
+            ops.matmul_kernels("both")
+
+
 @pytest.mark.parametrize("inner", [4096, 8192])       # 8,192: the gate and up product is too large, its neighbours are not
 def test_prompts_whole_and_in_portions(inner):
     from qwen3_from_scratch_amd.config import ModelConfig
