@@ -1706,9 +1706,11 @@ def span_sizes(heads, kv_heads, dim, vdim, page, dtype):
 
 
 def _splits(B, Hkv, max_kv_len):
-    """Into how many blocks a sequence's keys are split when a step has few rows per sequence. Measured with
-    8 key heads of 128, keys and values from memory, contexts all alike and spread over a quarter to the whole of
-    the longest, in microseconds with the merge:
+    """Into how many blocks a sequence's keys are split when a step has few rows per sequence. `max_kv_len` bounds the
+    longest sequence: it is its length, or, in a captured step, a power of two up to twice that, so a line below is drawn
+    where the parts pay for the lengths behind it, alike or not. Measured with 8 key heads of 128 without a window, keys and
+    values from memory, contexts all alike / spread over a quarter to the whole of the longest, in microseconds with the
+    merge (other head sizes, and the builds for capped scores, runs, sigmoid weights and spans, go by the same rule):
 
     - up to 256 keys a block has two tiles a wavefront and the merge costs more than a split gains (1 to 24
       requests 9 to 12 whole, 11 to 18 in parts); up to 512 only where few blocks run (one request 11.2 and
@@ -1717,23 +1719,28 @@ def _splits(B, Hkv, max_kv_len):
       requests over 2,000 keys 22.5 in four parts, 23.2 in eight, 27.1 in two; two over 4,000 15.6 in sixteen, 18.8 in
       24; twelve over 2,000 29.7 in two, 35.3 in three; twenty over 1,000 24.5 whole, 27.3 in three; one over
       8,000 15.5 in 32 and 17.3 in sixteen, over 1,000 11.4 in either;
-    - where that leaves a sequence whole, long contexts are as a rule uneven ones and the longest would be waited
-      for: 20 requests over 1,000 to 4,000 keys 61.6 whole, 54.4 in three (all over 4,000: 71.7 and 72.2), 24
-      66.7 and 63.2; over 2,000 to 8,000 115.6 whole, 89.0 in six, 122 and 108;
-    - with 8,192 keys or more a block's work dwarfs its start and what counts is that the blocks come in even rounds:
-      at least eight parts up to 384 (sequence, key head) pairs and four beyond (33 sequences over 8,200 keys: 257
-      whole, 199 in eight parts; 48: 295 whole, 274 in four; over 32,000 keys 955 and 713, 1,110 and 1,018);
-    - 257 to 320 pairs, a little more than a block each: 36 requests over 2,000 keys 79.5 whole, 72.9 in three (over
-      1,000 44.3 and 44.6); from 48 requests on one part is the fastest there."""
+    - that leaves 129 to 256 (sequence, key head) pairs whole, and the longest of uneven contexts is waited for. Up to 160
+      pairs three parts, two rounds of blocks, cost even ones next to nothing from 2,560 keys on: 20 requests over 2,560
+      47.2 / 41.1 whole, 50.5 / 38.7 in three, over 4,000 69.2 / 61.0 and 70.1 / 53.2, over 6,000 95.1 / 85.4 and 95.1 /
+      72.1 (over 1,500 31.4 / 27.1 and 33.7 / 27.4). More pairs stay whole: three parts of 24 requests come to a little
+      more than two rounds (over 2,060 44.5 / 37.9 whole, 54.0 / 38.5 in three, 49.6 / 39.9 in four; over 4,000 79.3 / 66.4,
+      91.8 / 62.4 and 82.9 / 64.1);
+    - 257 to 320 pairs, a little more than a block each, in three parts from 1,536 keys on: 36 requests over 1,540 61.3 /
+      42.3 whole, 57.8 / 41.5 in three, over 2,000 78.5 / 51.5 and 71.2 / 49.6 (over 1,030 44.4 / 31.3 and 45.1 / 34.1);
+      from 48 requests on one part is the fastest there;
+    - from 7,168 keys on a block's work dwarfs its start and what counts is that the blocks come in even rounds: at least
+      eight parts below 384 pairs and four from there on. 12 requests over 7,200 in two 74.2 / 61.7, in eight 75.4 / 55.4; 20 in
+      three 112 / 82, in eight 114 / 79; 24 whole 127 / 107, in eight 134 / 94; 36 in three 204 / 135, in eight 195 / 139; 48
+      whole 260 / 186, in four 252 / 175 (in eight 258 / 183); over 32,000 33 whole 955, in eight 713, 48 whole 1,110, in four 1,018."""
     pairs = B * Hkv
     if max_kv_len <= 256:
         return 1
     if max_kv_len <= 512:
         return max_kv_len // 64 if pairs <= 32 else 1
     splits = max(1, min(max_kv_len // 64, 256 // pairs, 32 if max_kv_len >= 4096 else 16))
-    if max_kv_len >= 8192 and pairs < 512:
-        splits = max(splits, 8 if pairs <= 384 else 4)
-    elif (max_kv_len >= 4096 and 128 < pairs <= 192) or (max_kv_len >= 2048 and 256 < pairs <= 320):
+    if max_kv_len >= 7168 and pairs < 512:
+        splits = max(splits, 8 if pairs < 384 else 4)
+    elif (max_kv_len >= 2560 and 128 < pairs <= 160) or (max_kv_len >= 1536 and 256 < pairs <= 320):
         splits = 3
     return splits
 
