@@ -84,7 +84,7 @@ __all__ = [
 
 _DT = {torch.float32: 0, torch.bfloat16: 1}
 _UNSUPPORTED = 10002          # a launcher's refusal of a size it has no kernel for
-_DECLINED = 1                 # the fused product of 17 to 128 rows did nothing: the plain product is faster here
+_DECLINED = 1                 # the kernel asked for did nothing: another way is faster for the size (or the only one)
 
 
 class OperandError(ValueError):
@@ -215,7 +215,7 @@ def matmul_plan(M, N, K, out_dtype=torch.bfloat16):
 
 
 def matmul_fused_plan(kind, M, N, K):
-    """What serves a product of 17 to 128 rows that carries a norm (`kind` "scaled",
+    """What serves a product that carries a norm (`fused_rows_take`; `kind` "scaled",
     "scaled_swiglu" or "residual"): (tile shape or -1 for the library's product with the norm's
     work behind it, shares of K); None with the tuner on for a size it has not met."""
     info = (ctypes.c_int * 2)()

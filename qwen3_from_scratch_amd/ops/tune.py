@@ -7,7 +7,8 @@
 For each row count and each of the layer's products (q/k/v, output, gate/up, down) the
 tuner times the vendor library's candidates and the hand-written kernel's tile shapes on
 random operands, with cold caches, and the fastest is written down as a table entry; row
-counts from 17 to 128 also get entries for the products that carry a norm. The output is
+counts at which a product may carry a norm (from 17 to 128, or 640 for a small weight:
+`ops.fused_rows_take`) also get entries for that. The output is
 the file `matmul_table.json` beside this module reads (`--merge FILE` adds to an existing
 table, newer entries replacing older ones for the same size). Nothing in the engine runs
 this: the table is data, made beforehand, so that every process chooses the same kernels.
@@ -65,7 +66,7 @@ def tune_layer(hidden, heads, kv_heads, head_dim, intermediate, rows_list, seed=
                     rows = ops.matmul_rows_key("plain", M)
                     entries[("plain", rows, N, K, out_name)] = _entry(
                         "plain", rows, N, K, out_name, dict(own=p[4], splits=p[5], library=p[6], us=p[3]))
-                if name != "head" and 16 < M <= ops.FUSED_ROWS_MOST and ops.fused_rows_take(w, M):
+                if name != "head" and ops.fused_rows_take(w, M):
                     residual = torch.zeros((M, N), dtype=torch.float32, device=device)
                     if name in ("o", "down") and N == hidden:
                         ops.linear_residual_norm(x, w, None, residual, norm_weight)

@@ -3,7 +3,7 @@
 import pytest
 import torch
 
-from test_kernels_gpu import _ops, test_linear_residual_norm_and_unscaled_rows_beyond_sixteen as _fused_products
+from test_kernels_gpu import _forget_choices, _ops, _rand, rules_alone, test_linear_residual_norm_and_unscaled_rows_beyond_sixteen as _fused_products
 
 pytestmark = pytest.mark.gpu
 
@@ -22,6 +22,38 @@ def test_rows_and_weights_that_take_part():
     small, large, tiny = (torch.empty(n, 1024, dtype=torch.bfloat16, device="cuda") for n in (8192, 10240, 512))
     assert [ops.fused_rows_take(small, m) for m in (16, 17, 128, 129, 640, 641)] == [False, True, True, True, True, False]
     assert [ops.fused_rows_take(w, 129) for w in (large, tiny)] == [False, False]
+
+
+def test_the_tuner_and_the_table_reach_640_rows(rules_alone):
+    """Rows beyond 128 of small weights get entries of their own, those beyond 640 and those of a smaller weight do not; a
+    size follows its entry, another keeps the rule."""
+    from qwen3_from_scratch_amd.ops import tune
+
+    ops = rules_alone
+    ops.matmul_candidates(1)
+    try:
+        entries = tune.tune_layer(1088, 16, 8, 64, 2048, [256, 648])
+    finally:
+        ops.matmul_candidates(16)
+    sizes = {kind: {(e["rows"], e["N"], e["K"]) for e in entries if e["kind"] == kind} for kind in ops._KINDS}
+    assert sizes["scaled"] == {(256, 2048, 1088)} and sizes["scaled_swiglu"] == {(256, 4096, 1088)}
+    assert sizes["residual"] == {(256, 1088, 1024), (256, 1088, 2048)}
+    assert (648 + 31) // 32 * 32 in {rows for rows, _, _ in sizes["plain"]}
+
+    M, N, K = 256, 2048, 1088
+    x, w, sums = _rand((M, K), torch.bfloat16, 81), _rand((N, K), torch.bfloat16, 82, scale=0.05), torch.ones(2, M, device="cuda")
+    want = (x.double() @ w.double().T) * (2.0 / K + 1e-6) ** -0.5
+    _forget_choices(ops)
+    beyond = ops.matmul_fused_plan("scaled", M + 8, N, K)
+    for choice in ((1, 2), (0, 1), (-1, 1)):
+        entry = {"kind": "scaled", "rows": ops.matmul_rows_key("scaled", M), "N": N, "K": K}
+        entry.update(dict(library=0) if choice[0] < 0 else dict(own=choice[0], splits=choice[1]))
+        ops.matmul_table([entry], clear=True)
+        _forget_choices(ops)
+        got = ops.linear(x, w, unscaled=(sums, 1e-6, K))
+        assert ops.matmul_fused_plan("scaled", M, N, K) == choice
+        torch.testing.assert_close(got.double(), want, rtol=1.6e-2, atol=1e-2)
+        assert ops.matmul_fused_plan("scaled", M + 8, N, K) == beyond
 
 
 def test_a_stream_too_wide_for_the_partial_products():

@@ -60,4 +60,5 @@ def test_the_shipped_table_is_well_formed():
         step = 8 if (e["kind"] != "plain" or e["rows"] <= 64) else 32
         assert e["rows"] > 16 and e["rows"] % step == 0, key
         if e["kind"] != "plain":
-            assert e["rows"] <= ops.FUSED_ROWS_MOST
+            small = ops.SMALL_WEIGHT_LEAST <= 2 * e["N"] * e["K"] <= ops.SMALL_WEIGHT_BYTES       # as ops.fused_rows_most
+            assert e["rows"] <= (ops.FUSED_ROWS_SMALL if small else ops.FUSED_ROWS_MOST)
