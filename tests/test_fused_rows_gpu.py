@@ -70,16 +70,21 @@ def test_a_stream_too_wide_for_the_partial_products():
 
 
 @pytest.mark.parametrize("inner", [4096, 8192])       # 8,192: the gate and up product is too large, its neighbours are not
-def test_prompts_whole_and_in_portions(inner):
+def test_prompts_whole_and_in_portions(inner, tmp_path):
+    import plain_qwen3
+    from helpers import off_by
     from qwen3_from_scratch_amd.config import ModelConfig
-    from qwen3_from_scratch_amd.engine import ModelRunner, StepEntry, random_model
+    from qwen3_from_scratch_amd.engine import StepEntry, load_runner
+    from qwen3_from_scratch_amd.weights import write_random_model
 
     config = ModelConfig.from_dict(dict(
         architectures=["Qwen3ForCausalLM"], vocab_size=2048, hidden_size=1024, hidden_act="silu", num_hidden_layers=3,
         max_position_embeddings=2048, num_attention_heads=16, num_key_value_heads=8, head_dim=128,
         intermediate_size=inner, rms_norm_eps=1e-6, rope_theta=1e6, tie_word_embeddings=False))
-    runner = ModelRunner(random_model(config, device="cuda:0", seed=3, std=0.02), 16, 100, 2)
+    folder = write_random_model(str(tmp_path / "model"), config, seed=3)
+    runner = load_runner(folder, dtype="bfloat16", device="cuda:0", page_size=16, max_tokens=1600, max_requests=2)
     tokens = torch.randint(0, 2048, (641,), generator=torch.Generator().manual_seed(4)).tolist()
+    plain = plain_qwen3.logits_of_sequence(*plain_qwen3.read_model_folder(folder), tokens).cuda()
 
     def logits(cuts):
         at = 0
@@ -95,3 +100,7 @@ def test_prompts_whole_and_in_portions(inner):
         portions = logits([100] * (M // 100) + [M % 100 or 100][:1] * bool(M % 100))
         # two bfloat16 ways through three layers: a few roundings of 2^-9 each
         assert float((whole - portions).norm() / portions.norm()) < 2e-2, M
+        # and neither farther from a plain float32 pass than that
+        for got in (whole, portions):
+            assert off_by(got[0], plain[M - 1], "bfloat16") <= 1.0, M
+            assert float((got[0] - plain[M - 1]).norm() / plain[M - 1].norm()) < 2e-2, M
