@@ -164,7 +164,8 @@ __global__ void hyper_norm_kernel(float* __restrict__ x, const TA* __restrict__ 
 // rows, STREAMS streams): the streams, what enters them, the tables and the norm's weight are all asked for at once and
 // u stays in registers. Few rows are bound by latency, where the kernel above waits for a table, a column of u and a
 // weight in turn: 8 rows of four streams of 2,048 take 4.9 us, there 9.0. Many are bound by memory: 2,048 such rows
-// (84 MB read, 76 written) 28 us, 5.7 TB/s, there 31. Other numbers of streams, widths and addresses stay with it.
+// (76 MB read and 76 written in bfloat16) 28 us, 5.4 TB/s, there 31. Other numbers of streams, widths and addresses stay
+// with it (one stream was not tried).
 template <typename TA, int STREAMS>
 __global__ void __launch_bounds__(1024) hyper_norm_row_kernel(float* __restrict__ x, const TA* __restrict__ delta,
                                                               const float* __restrict__ mix, const float* __restrict__ write,

@@ -13,8 +13,8 @@
 //      data made beforehand by the tuner below, keyed by (kind of product, rows
 //      rounded up, N, K, output type);
 //   2. a rule of thumb: the library's first candidate for a plain product; for
-//      the products of 17 to 128 rows that carry a norm the 64 x 128 tiles with
-//      K shared out until the chip is full, unless those tiles fit the chip badly.
+//      the products that carry a norm (17 to 128 rows, 640 of a small weight) 64 x 128
+//      tiles with K shared out until the chip is full, unless those tiles fit the chip badly.
 // The library's list is asked for the exact size every time, so a kernel is
 // never run on a size the library has not offered it for.
 //
@@ -247,15 +247,17 @@ Choice plain_by_rule(int M, int N, int K) {
   return Choice();   // the library's first candidate
 }
 
-// The products of 17 to 128 rows that carry a norm: 64 x 128 tiles in five stages (with K shared out they need
+// The products that carry a norm. 17 to 128 rows: 64 x 128 tiles in five stages (with K shared out they need
 // the fewest shares to fill the chip), unless the tiles come to a little more than a whole number of rounds over
 // the 256 CUs and leave most of them idle in the last one: then the library's product with the norm's work in a
 // kernel behind it (for KIND_RESIDUAL: declined, the caller's plain product and the norm's own kernel).
-// 129 to 640 rows (small weights): 64 x 128 tiles while they fit the chip in one round, in three stages (four blocks a
-// CU; five where more than 256 rows share K out), then 128 x 128, then the library. The products alone, us, three
-// stages / five / 128 x 128 / library: 201 rows of 4,096 x 1,024 10.5 / 11.1 / 14.0 / 12.0, of 8,192 x 1,024 11.1 / 11.7 /
-// 14.4 / 13.5, of 1,024 x 4,096 in eight shares 13.3 / 13.8 / 16.5; 400 rows of the last, in four, 17.4 / 15.7 / 16.7; 400
-// of 8,192 x 1,024 (448 tiles) 16.4 / 20.6 / 15.5 / 15.5; 532 of it (320 tiles of 128 x 128) 23.3 / 29.4 / 20.9 / 17.4.
+// 129 to 640 rows (small weights): 64 x 128 tiles while there is at most one a CU (up to 256), in three stages, two
+// blocks of which share a CU where K is shared out (in five, one block a CU, where more than 256 rows share K out),
+// then 128 x 128, one block a CU, while that is one round, then the library. The products alone, us, three stages / five /
+// 128 x 128 / library: 201 rows of 4,096 x 1,024 10.5 / 11.1 / 14.0 / 12.0, of 8,192 x 1,024 11.1 / 11.7 / 14.4 / 13.5, of
+// 1,024 x 4,096 in eight shares 13.3 / 13.8 / 16.5; 400 rows of the last, in four, 17.4 / 15.7 / 16.7; 400 of 8,192 x 1,024
+// (448 tiles of 64 x 128, less than two a CU) 16.4 / 20.6 / 15.5 / 15.5; 532 of it (320 tiles of 128 x 128) 23.3 / 29.4 /
+// 20.9 / 17.4.
 Choice fused_by_rule(int kind, int M, int N, int K) {
   Choice c;
   if (g_kernels == KERNELS_LIBRARY) return c;
@@ -845,7 +847,7 @@ extern "C" int q3_matmul_plan(int M, int N, int K, int out_dtype, float* info) {
   return 1;
 }
 
-// What serves a product of 17 to 128 rows that carries a norm (`kind` 1, 2 or 3 as in the table) under the
+// What serves a product of more than 16 rows that carries a norm (`kind` 1, 2 or 3 as in the table) under the
 // current settings: info[0] the tile shape or -1 (the library's product with the norm's work behind it, or
 // declined), info[1] the shares of K. With the tuner on: what it found, and 0 is returned for a size it has
 // not met.

@@ -115,8 +115,9 @@ struct Eight<float> {
 };
 
 // A thread's tile is Q3_CONV_TILE rows. TAPS 4: that many, and a thread takes its channels' taps straight from memory; 0:
-// up to Q3_TAPS_MOST, through shared memory. Bound by memory and the taps' passage: 2,048 rows of 4,352 bfloat16 channels and 4 taps (36 MB) 22 us, 37 with an input's wait before
-// each next one and taps that 32 lanes read from one bank of shared memory.
+// up to Q3_TAPS_MOST, through shared memory. Bound by memory and the taps' passage: 2,048 rows of 4,352 bfloat16 channels
+// and 4 taps (36 MB) 22 us, 37 with an input's wait before each next one and taps that 32 lanes read from one bank of
+// shared memory (as they still are for other numbers of taps).
 #define Q3_CONV_TILE 8
 template <typename TI, typename TO, int TAPS>
 __global__ void __launch_bounds__(64) causal_conv_wide_kernel(const TI* __restrict__ x, long x_stride, const float* __restrict__ in_bias,

@@ -351,7 +351,7 @@ def rmsnorm(x, weight, eps, out_dtype, delta=None, rows=None, write_back=True, o
     T, H = x.shape
     if not (weight.shape == (H,) and weight.dtype in _DT):
         raise OperandError("weight must be (H,) bfloat16 or float32")
-    if not (out_dtype in _DT):
+    if out_dtype not in _DT:
         raise OperandError("out_dtype must be bfloat16 or float32")
     if delta is not None:
         if not (delta.shape == (T, H) and delta.dtype == out_dtype):
@@ -1592,7 +1592,7 @@ def paged_attention(q, num_q_heads, k_cache, v_cache, block_table, cu_seqlens_q,
     if not (q.is_cuda and q.dim() == 3 and q.stride(2) == 1 and q.stride(1) == q.shape[2]):
         raise OperandError("q must be (T, Hq, D) with contiguous heads")
     T, Hq, D = q.shape
-    if not (Hq == num_q_heads):
+    if Hq != num_q_heads:
         raise OperandError("q's head count differs from num_q_heads")
     if not (q.dtype in _DT and k_cache.dtype == q.dtype and v_cache.dtype == q.dtype):
         raise OperandError("q and the caches must share bfloat16 or float32")
@@ -1778,7 +1778,7 @@ def decode_attention(qkv, num_q_heads, num_kv_heads, head_dim, k_cache, v_cache,
         raise OperandError("cu_seqlens_q int32 (B + 1,)")
     if not (kv_lens.dtype == torch.int32):
         raise OperandError("kv_lens int32 (B,)")
-    if not ((q_weight is None) == (k_weight is None)):
+    if (q_weight is None) != (k_weight is None):
         raise OperandError("q and k norm weights come together")
     w_dtype = 0
     if q_weight is not None:
@@ -1794,7 +1794,7 @@ def decode_attention(qkv, num_q_heads, num_kv_heads, head_dim, k_cache, v_cache,
         if not (max_kv_len <= max_pos):
             raise OperandError("the step reaches position %d, the rotation table ends at %d"
                                % (max_kv_len - 1, max_pos - 1))
-    if not (decode_attention_takes(Hq, Hkv, D, page, qkv.dtype, rotary_dim)):
+    if not decode_attention_takes(Hq, Hkv, D, page, qkv.dtype, rotary_dim):
         raise OperandError("sizes the decoding kernel does not take")
     out = torch.empty((B, Hq * D), dtype=qkv.dtype, device=qkv.device)
     if B:
@@ -1907,7 +1907,7 @@ def _tiles_scaled(x, weight, out, unscaled, swiglu, what):
     sums, eps, width = unscaled
     M, K = x.shape
     _check_sums(sums, M)
-    if not (width == K):
+    if width != K:
         raise OperandError("the rows' width must be the product's inner size")
     if not (x.is_contiguous() and out.is_contiguous()):
         raise OperandError("operands must be contiguous")
@@ -1977,9 +1977,9 @@ def linear(x, weight, out_dtype=None, out=None, tiled=None, unscaled=None):
     M, K = x.shape
     N = weight.shape[0]
     out_dtype = out_dtype or x.dtype
-    if not (out_dtype in _DT):
+    if out_dtype not in _DT:
         raise OperandError("out dtype must be bfloat16 or float32")
-    if not (not (x.dtype == torch.float32 and out_dtype != torch.float32)):
+    if x.dtype == torch.float32 and out_dtype != torch.float32:
         raise OperandError("float32 inputs give float32 output")
     if out is None:
         out = torch.empty((M, N), dtype=out_dtype, device=x.device)
@@ -1996,7 +1996,7 @@ def linear(x, weight, out_dtype=None, out=None, tiled=None, unscaled=None):
         return out
     if unscaled is not None and x.dtype == torch.bfloat16 and fused_rows_take(weight, M):
         return _tiles_scaled(x, weight, out, unscaled, False, "linear")
-    if not (unscaled is None):
+    if unscaled is not None:
         raise OperandError("unscaled rows need bfloat16 and few rows with a tiled weight (few_rows_limit), or 17 to "
                            "128 rows (640 of a small weight, fused_rows_most) with an inner size that is a multiple of 64")
     if M and x.dtype == torch.bfloat16 and not library("gemm").q3_linear_is_skinny(M, N, K, 1):
@@ -2046,10 +2046,10 @@ _FEW_ROW_EPILOGUES = {"silu": 1, "gelu_tanh": 3}      # the few-row kernel's cod
 def linear_swiglu(x, weight, tiled=None, unscaled=None, kind="silu"):
     """act(gate) * up of x @ weight^T for a weight whose rows interleave gate and up (row 2i gate's, row
     2i + 1 up's): (M, K) x (2I, K) -> (M, I); `kind` names the activation (`GATE_KINDS`). With few
-    bfloat16 rows the activation is the product kernel's epilogue (silu in every kernel for up to 128 rows, the
-    tanh form of gelu in the few-row and the weight-streaming kernel, the exact gelu nowhere); otherwise
-    it is the product followed by `gated_act`, with the same bits. `unscaled`: as for `linear`."""
-    if not (kind in GATE_KINDS):
+    bfloat16 rows, and with as many as may come unscaled (`fused_rows_most`), the activation is the product kernel's
+    epilogue (silu in every kernel, the tanh form of gelu in the few-row and the weight-streaming kernel, the exact gelu
+    nowhere); otherwise it is the product followed by `gated_act`, with the same bits. `unscaled`: as for `linear`."""
+    if kind not in GATE_KINDS:
         raise OperandError("kind is one of %s" % ", ".join(sorted(GATE_KINDS)))
     if kind == "gelu_erf":
         return gated_act(linear(x, weight, tiled=tiled, unscaled=unscaled), kind)
@@ -2085,7 +2085,7 @@ def linear_swiglu(x, weight, tiled=None, unscaled=None, kind="silu"):
     if unscaled is not None and x.dtype == torch.bfloat16 and fused_rows_take(weight, M):
         out = torch.empty((M, N // 2), dtype=x.dtype, device=x.device)
         return _tiles_scaled(x, weight, out, unscaled, True, "linear_swiglu")
-    if not (unscaled is None):
+    if unscaled is not None:
         raise OperandError("unscaled rows need bfloat16 and few rows with a tiled weight (few_rows_limit), or 17 to "
                            "128 rows (640 of a small weight, fused_rows_most) with an inner size that is a multiple of 64")
     if M and library("gemm").q3_linear_is_skinny(M, N, K, _DT[x.dtype]):
@@ -2125,7 +2125,7 @@ def linear_residual_norm(x, weight, tiled, residual, norm_weight):
     values = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
     few = x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and N % 16 == 0 and _tiled_ok(tiled, weight, M)
     if not few and x.dtype == torch.bfloat16 and fused_rows_take(weight, M):
-        if not (x.is_contiguous()):
+        if not x.is_contiguous():
             raise OperandError("x must be contiguous")
         lib = _matmul()
         sums = torch.empty((lib.q3_tiles_residual_chunks(N), sums_stride(M)), dtype=torch.float32, device=x.device)
@@ -2136,7 +2136,7 @@ def linear_residual_norm(x, weight, tiled, residual, norm_weight):
             return None
         _check(status, "linear_residual_norm")
         return values, sums
-    if not (few):
+    if not few:
         raise OperandError("bfloat16, a tiled weight with a width that is a multiple of 16 and no more rows than few_rows_limit, "
                            "or 17 to 128 rows (640 of a small weight, fused_rows_most) with an inner size that is a multiple of 64")
     sums = torch.empty((N // 16, sums_stride(M)), dtype=torch.float32, device=x.device)
