@@ -1724,7 +1724,8 @@ def _splits(B, Hkv, max_kv_len):
       47.2 / 41.1 whole, 50.5 / 38.7 in three, over 4,000 69.2 / 61.0 and 70.1 / 53.2, over 6,000 95.1 / 85.4 and 95.1 /
       72.1 (over 1,500 31.4 / 27.1 and 33.7 / 27.4). More pairs stay whole: three parts of 24 requests come to a little
       more than two rounds (over 2,060 44.5 / 37.9 whole, 54.0 / 38.5 in three, 49.6 / 39.9 in four; over 4,000 79.3 / 66.4,
-      91.8 / 62.4 and 82.9 / 64.1);
+      91.8 / 62.4 and 82.9 / 64.1). A captured step of 17 to 24 requests has 24 rows: over 2,049 to 4,096 keys those take 4 %
+      more whole than in the best of one to eight parts, on average, 3 % in three, 14 % in two;
     - 257 to 320 pairs, a little more than a block each, in three parts from 1,536 keys on: 36 requests over 1,540 61.3 /
       42.3 whole, 57.8 / 41.5 in three, over 2,000 78.5 / 51.5 and 71.2 / 49.6 (over 1,030 44.4 / 31.3 and 45.1 / 34.1);
       from 48 requests on one part is the fastest there;
