@@ -1891,7 +1891,9 @@ def fused_rows_most(weight):
     library's products with the norms as kernels of their own are faster), or 640 for a weight of 2 to 18 MB. There the
     norm's kernel, the activation's and a product's second one cost more than the products' difference: a prompt of the
     0.6B shape in one step, 3.49 ms at 136 to 256 rows and 3.71 at 512 with the kernels apart, 2.80 to 2.83 and 2.91 so;
-    level at 640 (3.71, 3.58), 3.91 against 3.94 at 768. The 8B shape (33 to 201 MB) 6.93 apart and 8.34 so at 136."""
+    level at 640 (3.71, 3.58), 3.91 against 3.94 at 768. The 8B shape (33 to 201 MB) 6.93 apart and 8.34 so at 136. (The
+    parts that read through a norm say whether they take so many rows: `unscaled_rows_most`, which the attention and the
+    feed-forward of that shape have; the others, where it was not measured, take 128.)"""
     size = weight.numel() * weight.element_size()
     return FUSED_ROWS_SMALL if SMALL_WEIGHT_LEAST <= size <= SMALL_WEIGHT_BYTES else FUSED_ROWS_MOST
 
