@@ -111,6 +111,8 @@ def _stream():
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
+# The operations that every step of the Qwen3 decoder makes check their operands in place and form a message only where it is
+# needed: some three thousand calls of this function were 12 % of a small model's prompt step. The others call it.
 def _need(cond, message):
     if not cond:
         raise OperandError(message)
