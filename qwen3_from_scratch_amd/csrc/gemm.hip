@@ -1,6 +1,7 @@
 // out = x @ weight^T with float32 accumulation: x (M, K), weight (N, K), out (M, N).
 #include "common.h"
 #include "gates.h"
+#include "gemm_parts.h"
 
 // ---------------------------------------------------------------------------
 // Plain fused multiply-adds for any size: float32 products whose inner size is no multiple of 4 (or whose
@@ -766,6 +767,15 @@ extern "C" int q3_linear(const void* x, const void* weight, void* out, int M, in
   }
   return out_dtype == Q3_F32 ? launch_skinny<float, EPI_PLAIN>(x, weight, out, M, N, K, stream)
                              : launch_skinny<bf16_t, EPI_PLAIN>(x, weight, out, M, N, K, stream);
+}
+
+// float32 x (M, K) with a weight (N, K) whose numbers bfloat16 holds exactly, all of them finite, given in
+// bfloat16 (gemm_parts.h): out (M, N) float32, or with `silu` (rows interleave gate and up, N even) out (M, N / 2) =
+// silu(gate) * up. K a multiple of 64, operands at multiples of 16 bytes.
+extern "C" int q3_linear_narrow(const void* x, const void* weight, void* out, int M, int N, int K, int silu, hipStream_t stream) {
+  if (!x || !weight || !out || !parts::takes(M, N, K) || (silu && N % 2)) return Q3_ERR_BAD_ARGUMENT;
+  if (((size_t)x | (size_t)weight | (size_t)out) & 15) return Q3_ERR_BAD_ARGUMENT;
+  return silu ? parts::launch<true>(x, weight, out, M, N, K, stream) : parts::launch<false>(x, weight, out, M, N, K, stream);
 }
 
 // out (M, N / 2) = silu(gate) * up where x @ weight^T interleaves gate and up columns

@@ -77,6 +77,7 @@ __all__ = [
     "matmul_plan",
     "stream_plan",
     "tile_weight",
+    "narrow_weight",
     "sample",
     "measured_read_rate",
     "measured_matrix_rate",
@@ -1833,6 +1834,30 @@ def tile_weight(weight):
     return tiles.contiguous().view(-1)
 
 
+def narrow_weight(weight):
+    """A bfloat16 copy of a float32 matrix (N, K) on the GPU whose numbers bfloat16 holds exactly, as those of a bfloat16
+    checkpoint are: `linear` takes it as `narrow`. None for any other matrix, and where an infinity, a NaN or an inner
+    size that is no multiple of 64 leaves the product to the float32 kernels."""
+    if weight.dtype != torch.float32 or weight.dim() != 2 or not weight.is_cuda or weight.shape[1] % 64 or not weight.numel():
+        return None
+    copy = weight.to(torch.bfloat16)
+    rows = max(1, (64 << 20) // weight.shape[1])          # some at a time: a difference takes a float32 copy
+    for at in range(0, weight.shape[0], rows):
+        if bool((weight[at:at + rows] - copy[at:at + rows]).any()):   # (an infinity's or a NaN's difference is a NaN)
+            return None
+    return copy
+
+
+def _narrow_ok(narrow, x, weight):
+    """Whether the product goes by the bfloat16 copy of its float32 weight."""
+    if narrow is None or x.dtype != torch.float32 or not x.shape[0]:
+        return False
+    if not (narrow.is_cuda and narrow.dtype == torch.bfloat16 and narrow.shape == weight.shape and narrow.is_contiguous()
+            and weight.shape[1] % 64 == 0):
+        raise OperandError("the bfloat16 copy does not belong to this weight")
+    return x.data_ptr() % 16 == 0 and narrow.data_ptr() % 16 == 0
+
+
 FEW_ROWS = 16                   # the few-row kernel's rows: one matrix instruction's worth of x
 SMALL_WEIGHT_BYTES = 18 << 20   # up to this size the few-row kernel serves 32 rows, up to half of it 64
 
@@ -1963,11 +1988,14 @@ def _stream_product(x, weight, tiled, out, swiglu, unscaled, what, kind="silu"):
     return True
 
 
-def linear(x, weight, out_dtype=None, out=None, tiled=None, unscaled=None):
+def linear(x, weight, out_dtype=None, out=None, tiled=None, unscaled=None, narrow=None):
     """out = x @ weight^T with float32 accumulation. x (M, K), weight (N, K).
     `tiled` is `tile_weight(weight)`, if the caller keeps one: few rows are then served from it.
     `unscaled` (see `linear_residual_norm`) says that x's rows still lack their 1 / rms factor;
     the product's rows receive it. Only the few-row kernel on a tiled weight does this.
+
+    `narrow` is `narrow_weight(weight)`, if the caller keeps one: float32 rows are then multiplied
+    with it, in float32 precision all the same.
 
     float32 operands take a float32 kernel with no reduced-precision mode;
     bfloat16 operands with at most 16 rows (32 or 64 with the tiled copy of a small
@@ -1990,6 +2018,9 @@ def linear(x, weight, out_dtype=None, out=None, tiled=None, unscaled=None):
         out = torch.empty((M, N), dtype=out_dtype, device=x.device)
     if not (out.shape == (M, N) and out.dtype == out_dtype):
         raise OperandError("out must be (M, N) of out_dtype")
+    if unscaled is None and _narrow_ok(narrow, x, weight) and out.data_ptr() % 16 == 0:
+        _check(library("gemm").q3_linear_narrow(_ptr(x), _ptr(narrow), _ptr(out), M, N, K, 0, _stream()), "linear")
+        return out
     if M and x.dtype == torch.bfloat16 and _tiled_ok(tiled, weight, M):
         sums, sums_rows, eps, width, stride = _row_sums_args(unscaled, M, K)
         _check(library("gemm").q3_linear_tiled(
@@ -2048,16 +2079,17 @@ def linear_plain(x, weight, out):
 _FEW_ROW_EPILOGUES = {"silu": 1, "gelu_tanh": 3}      # the few-row kernel's codes of its gated epilogues
 
 
-def linear_swiglu(x, weight, tiled=None, unscaled=None, kind="silu"):
+def linear_swiglu(x, weight, tiled=None, unscaled=None, kind="silu", narrow=None):
     """act(gate) * up of x @ weight^T for a weight whose rows interleave gate and up (row 2i gate's, row
     2i + 1 up's): (M, K) x (2I, K) -> (M, I); `kind` names the activation (`GATE_KINDS`). With few
     bfloat16 rows, and with as many as may come unscaled (`fused_rows_most`), the activation is the product kernel's
     epilogue (silu in every kernel, the tanh form of gelu in the few-row and the weight-streaming kernel, the exact gelu
-    nowhere); otherwise it is the product followed by `gated_act`, with the same bits. `unscaled`: as for `linear`."""
+    nowhere); otherwise it is the product followed by `gated_act`, with the same bits. `unscaled` and `narrow`: as for
+    `linear` (silu is the epilogue of the products with a bfloat16 copy too)."""
     if kind not in GATE_KINDS:
         raise OperandError("kind is one of %s" % ", ".join(sorted(GATE_KINDS)))
     if kind == "gelu_erf":
-        return gated_act(linear(x, weight, tiled=tiled, unscaled=unscaled), kind)
+        return gated_act(linear(x, weight, tiled=tiled, unscaled=unscaled, narrow=narrow), kind)
     _dev(x, weight)
     if not (x.dim() == 2 and weight.dim() == 2 and x.shape[1] == weight.shape[1] and weight.shape[0] % 2 == 0):
         raise OperandError("x (M, K) and weight (2I, K)")
@@ -2086,7 +2118,11 @@ def linear_swiglu(x, weight, tiled=None, unscaled=None, kind="silu"):
         if _stream_product(x, weight, tiled, out, True, unscaled, "linear_swiglu", kind):
             return out
     if kind != "silu":
-        return gated_act(linear(x, weight, tiled=tiled, unscaled=unscaled), kind)
+        return gated_act(linear(x, weight, tiled=tiled, unscaled=unscaled, narrow=narrow), kind)
+    if unscaled is None and _narrow_ok(narrow, x, weight):
+        out = torch.empty((M, N // 2), dtype=x.dtype, device=x.device)
+        _check(library("gemm").q3_linear_narrow(_ptr(x), _ptr(narrow), _ptr(out), M, N, K, 1, _stream()), "linear_swiglu")
+        return out
     if unscaled is not None and x.dtype == torch.bfloat16 and fused_rows_take(weight, M):
         out = torch.empty((M, N // 2), dtype=x.dtype, device=x.device)
         return _tiles_scaled(x, weight, out, unscaled, True, "linear_swiglu")

@@ -20,7 +20,8 @@ class Precision:
     """Compute dtypes of one engine instance. Activations, matrices and the
     cache share `act`; the residual stream and logits are float32. `tiled`:
     keep a second, tile-ordered copy of every bfloat16 matrix for the few-row
-    product kernel (decoding); it costs the matrices' memory once more."""
+    product kernel (decoding); it costs the matrices' memory once more. And a bfloat16
+    copy of every float32 matrix that bfloat16 holds exactly, for half its memory more."""
 
     act: torch.dtype
     tiled: bool = True

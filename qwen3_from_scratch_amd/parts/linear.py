@@ -1,5 +1,5 @@
-"""A weight matrix as the parts hold it: row-major, and for bfloat16 a second copy
-in the order the few-row product kernel streams it."""
+"""A weight matrix as the parts hold it: row-major, and a second copy for its kernels: of bfloat16 in the
+order the few-row product kernel streams it, of float32 in bfloat16 where that loses nothing."""
 
 import torch
 
@@ -25,11 +25,14 @@ class LinearWeight:
     rows (the vendor library's) and for float32; when the precision asks for
     it, a tile-ordered bfloat16 copy serves steps with few rows (16, or 32 or 64
     for a small weight), where every weight is read once and the order in memory
-    decides the bandwidth. The copy doubles the weight's memory."""
+    decides the bandwidth. The copy doubles the weight's memory. A float32 weight that
+    bfloat16 holds exactly has a bfloat16 copy instead, half its memory more: the products
+    then read half as much and run on the bfloat16 matrix cores, in float32 precision."""
 
     def __init__(self, weight, precision):
         self.weight = weight
         self.tiled = ops.tile_weight(weight) if precision.tiled else None
+        self.narrow = ops.narrow_weight(weight) if precision.tiled else None
         if weight.is_cuda and weight.dtype == torch.bfloat16:
             ops.matmul_init()          # the many-row products' buffers: now, not inside a step
 
@@ -37,12 +40,16 @@ class LinearWeight:
         """x @ W^T; x may be UnscaledRows (see `fuses`)."""
         if isinstance(x, UnscaledRows):
             return ops.linear(x.values, self.weight, out_dtype=out_dtype, tiled=self.tiled, unscaled=x.scale_args())
+        if self.narrow is not None:
+            return ops.linear(x, self.weight, out_dtype=out_dtype, narrow=self.narrow)
         return ops.linear(x, self.weight, out_dtype=out_dtype, tiled=self.tiled)
 
     def forward_swiglu(self, x, kind="silu"):
         """act(gate) * up of x @ W^T for a W whose rows interleave gate and up; `kind` names the activation."""
         if isinstance(x, UnscaledRows):
             return ops.linear_swiglu(x.values, self.weight, tiled=self.tiled, unscaled=x.scale_args(), kind=kind)
+        if self.narrow is not None:
+            return ops.linear_swiglu(x, self.weight, kind=kind, narrow=self.narrow)
         return ops.linear_swiglu(x, self.weight, tiled=self.tiled, kind=kind)
 
     @property
