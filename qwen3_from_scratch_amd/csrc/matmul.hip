@@ -13,7 +13,8 @@
 //      data made beforehand by the tuner below, keyed by (kind of product, rows
 //      rounded up, N, K, output type);
 //   2. a rule of thumb: the library's first candidate for a plain product; for
-//      the products that carry a norm (17 to 128 rows, 640 of a small weight) 64 x 128
+//      the products that carry a norm (17 to 128 rows, 640 of a small weight) the kernel that shares K out
+//      inside a block (gemm_groups.h) for a small weight, else 64 x 128
 //      tiles with K shared out until the chip is full, unless those tiles fit the chip badly.
 // The library's list is asked for the exact size every time, so a kernel is
 // never run on a size the library has not offered it for.
@@ -37,6 +38,7 @@
 #include "common.h"
 #include "gemm_tiles.h"
 #include "gemm_stream.h"
+#include "gemm_groups.h"
 
 #include <hipblaslt/hipblaslt.h>
 
@@ -55,9 +57,12 @@ constexpr size_t EVICT_BYTES = 512u << 20;     // twice the 256 MB last-level ca
 constexpr size_t PARTIALS_BYTES = 128u << 20;  // float32 partial products of the hand-written kernel's K shares
 constexpr size_t STAGING_BYTES = 64u << 20;
 constexpr int FUSED_ROWS_LIMIT = 640;         // rows of a product that carries a norm (128 but for small weights)
+constexpr size_t GROUPS_MOST_WEIGHT_BYTES = 18u << 20;
 constexpr int EVICT_BLOCKS = 2048, EVICT_THREADS = 256;
 constexpr int MAX_CANDIDATES = 64;
 constexpr int LIBRARY = -1;                    // a Choice's `own` when the library serves the size
+constexpr int GROUPS_FIRST = 16;               // a Choice's `own` from here on: gemm_groups.h's shapes (no table entry)
+static_assert(GROUPS_FIRST >= tiles::NUM_CONFIGS, "one numbering");
 
 // Reads the whole buffer; the store never happens (the buffer holds zeros) but keeps the loads alive.
 __global__ void evict_kernel(float4* buffer, size_t count) {
@@ -247,7 +252,12 @@ Choice plain_by_rule(int M, int N, int K) {
   return Choice();   // the library's first candidate
 }
 
-// The products that carry a norm. 17 to 128 rows: 64 x 128 tiles in five stages (with K shared out they need
+// The products that carry a norm. A weight of up to 18 MB, or a product of more than 96 rows in 128 x 128 tiles: the kernel of
+// gemm_groups.h where it covers the product in one round. (A larger weight's few rows are bound by its passage, which many small tiles with
+// their own rows of x beside it slow down: 24 and 64 rows of 6,144 x 4,096 16.6 and 20.8 us there, 15.9 and 17.8 in 64 x 128
+// tiles; 64 of 4,096 x 12,288 34.8 and 28.2. 128 rows of 24,576 x 4,096 with SwiGLU, 192 tiles of 128 x 128, 58.8 and 74.3, the
+// library's with a kernel behind it; up to 96 rows the weight-streaming kernel has it.)
+// 17 to 128 rows: 64 x 128 tiles in five stages (with K shared out they need
 // the fewest shares to fill the chip), unless the tiles come to a little more than a whole number of rounds over
 // the 256 CUs and leave most of them idle in the last one: then the library's product with the norm's work in a
 // kernel behind it (for KIND_RESIDUAL: declined, the caller's plain product and the norm's own kernel).
@@ -261,6 +271,14 @@ Choice plain_by_rule(int M, int N, int K) {
 Choice fused_by_rule(int kind, int M, int N, int K) {
   Choice c;
   if (g_kernels == KERNELS_LIBRARY) return c;
+  if (g_kernels == KERNELS_BOTH) {
+    const int shape = groups::shape_for(M, N, K);
+    const bool small = (size_t)N * K * 2 <= GROUPS_MOST_WEIGHT_BYTES;
+    if (shape >= 0 && (small || (kind != KIND_RESIDUAL && M > 96 && shape == groups::NUM_SHAPES - 1))) {
+      c.own = GROUPS_FIRST + shape;
+      return c;
+    }
+  }
   if (M > 128) {
     // (a residual's product always goes through partial products; where not even one share's fit, it is declined)
     if (kind == KIND_RESIDUAL && (size_t)M * N * sizeof(float) > PARTIALS_BYTES) return c;
@@ -582,6 +600,12 @@ extern "C" int q3_tiles_scaled(const void* x, const void* w, void* out, int M, i
   scale.eps = eps;
   scale.inv_width = 1.f / (float)width;
   auto launch = [&](int config, int splits) {
+    if (config >= GROUPS_FIRST) {
+      const int shape = config - GROUPS_FIRST;
+      if (swiglu) return groups::launch<bf16_t, groups::EPI_SWIGLU>(shape, x, w, out, M, N, K, stream, scale);
+      if (out_dtype == Q3_F32) return groups::launch<float, groups::EPI_PLAIN>(shape, x, w, out, M, N, K, stream, scale);
+      return groups::launch<bf16_t, groups::EPI_PLAIN>(shape, x, w, out, M, N, K, stream, scale);
+    }
     if (swiglu)
       return tiles::launch<bf16_t, tiles::EPI_SWIGLU>(config, x, w, out, M, N, K, stream, splits, d.partials, scale);
     if (out_dtype == Q3_F32)
@@ -622,15 +646,34 @@ extern "C" int q3_tiles_scaled(const void* x, const void* w, void* out, int M, i
   return launch(c.own, c.splits);
 }
 
+// Whether q3_tiles_scaled would serve a size by the kernel that shares K out inside a block, with the few-row kernel's bits:
+// a row's results do not depend on how many rows are beside it where the few-row kernel takes them (its callers' rule).
+extern "C" int q3_groups_as_few(int M, int N, int K) {
+  std::lock_guard<std::mutex> hold(g_lock);
+  if (g_mode != MODE_RULE || M > FUSED_ROWS_LIMIT) return 0;
+  const int own = choice_for(KIND_SCALED, M, N, K, Q3_BF16).own;
+  return own >= GROUPS_FIRST && groups::shares_of_few_rows(own - GROUPS_FIRST, N, K);
+}
+
 // q3_tiles_residual: residual (M, N) float32 += bfloat16(x @ w^T) in place; values (M, N) bfloat16 =
-// residual * norm_weight; sums (ceil(N / 1024), sums_stride) float32 = the rows' sums of squares of the new
-// residual over chunks of 1,024 columns (row m in column m): what q3_tiles_scaled takes for the next product. Returns Q3_DECLINED, and has done
-// nothing, where the plain product followed by the norm's own kernel is the way for this size.
-extern "C" int q3_tiles_residual_chunks(int N) { return (N + tiles::CHUNK_COLUMNS - 1) / tiles::CHUNK_COLUMNS; }
+// residual * norm_weight; sums (q3_tiles_residual_chunks(M, N, K), sums_stride) float32 = the rows' sums of squares of the new
+// residual over so many chunks of columns (row m in column m): what q3_tiles_scaled takes for the next product. `chunks` is the number
+// that `sums` has room for. Returns Q3_DECLINED, and has done
+// nothing, where the plain product followed by the norm's own kernel is the way for this size, or where the settings have changed
+// since the chunks were asked for and these are too few.
+static int chunks_of(int columns, int N) { return (N + columns - 1) / columns; }
+static int residual_chunks(const Choice& c, int N) {
+  return chunks_of(c.own >= GROUPS_FIRST ? groups::SHAPES[c.own - GROUPS_FIRST][1] : tiles::CHUNK_COLUMNS, N);
+}
+extern "C" int q3_tiles_residual_chunks(int M, int N, int K) {
+  std::lock_guard<std::mutex> hold(g_lock);
+  if (g_mode == MODE_TUNE) return chunks_of(tiles::CHUNK_COLUMNS, N);   // the tuner times the tiled kernel's shapes
+  return residual_chunks(choice_for(KIND_RESIDUAL, M, N, K, Q3_BF16), N);
+}
 
 extern "C" int q3_tiles_residual(const void* x, const void* w, int M, int N, int K, float* residual,
                                  const void* norm_weight, int norm_weight_dtype, void* values, float* sums,
-                                 int sums_stride, void* stream_) {
+                                 int chunks, int sums_stride, void* stream_) {
   if (!x || !w || !residual || !norm_weight || !values || !sums || sums_stride < M) return Q3_ERR_BAD_ARGUMENT;
   if (M < 1 || M > FUSED_ROWS_LIMIT || N % 4 || !tiles::takes(M, N, K)) return Q3_ERR_BAD_ARGUMENT;
   if (norm_weight_dtype != Q3_BF16 && norm_weight_dtype != Q3_F32) return Q3_ERR_BAD_ARGUMENT;
@@ -653,13 +696,22 @@ extern "C" int q3_tiles_residual(const void* x, const void* w, int M, int N, int
       },
       [&]() { return product(d, x, w, values, M, N, K, Q3_BF16, stream); }, c);
   if (status) return status;
-  if (c.own == LIBRARY) return Q3_DECLINED;
+  if (c.own == LIBRARY || chunks != residual_chunks(c, N)) return Q3_DECLINED;
+  if (c.own >= GROUPS_FIRST) {
+    groups::Residual res;
+    res.stream = residual;
+    res.norm_weight = norm_weight;
+    res.norm_weight_f32 = norm_weight_dtype == Q3_F32;
+    res.sums = sums;
+    res.sums_stride = sums_stride;
+    return groups::launch<bf16_t, groups::EPI_RESIDUAL>(c.own - GROUPS_FIRST, x, w, values, M, N, K, stream, tiles::RowScale(), res);
+  }
   if ((size_t)c.splits * M * N * sizeof(float) > PARTIALS_BYTES) return Q3_ERR_UNSUPPORTED;   // also a single share
   int used = 1;
   status = tiles::launch<bf16_t, tiles::EPI_PLAIN>(c.own, x, w, values, M, N, K, stream, c.splits, d.partials,
                                                    tiles::RowScale(), true, &used);
   if (status) return status;
-  const dim3 grid(q3_tiles_residual_chunks(N), M);
+  const dim3 grid(chunks, M);
   if (norm_weight_dtype == Q3_F32)
     hipLaunchKernelGGL(tiles::tiles_residual_kernel<float>, grid, dim3(256), 0, stream, d.partials, used, residual,
                        (const float*)norm_weight, (bf16_t*)values, sums, sums_stride, M, N);
@@ -848,7 +900,7 @@ extern "C" int q3_matmul_plan(int M, int N, int K, int out_dtype, float* info) {
 }
 
 // What serves a product of more than 16 rows that carries a norm (`kind` 1, 2 or 3 as in the table) under the
-// current settings: info[0] the tile shape or -1 (the library's product with the norm's work behind it, or
+// current settings: info[0] the tile shape, from 16 on those of the kernel that shares K out inside a block, or -1 (the library's product with the norm's work behind it, or
 // declined), info[1] the shares of K. With the tuner on: what it found, and 0 is returned for a size it has
 // not met.
 extern "C" int q3_matmul_fused_plan(int kind, int M, int N, int K, int* info) {

@@ -219,7 +219,7 @@ def matmul_plan(M, N, K, out_dtype=torch.bfloat16):
 
 def matmul_fused_plan(kind, M, N, K):
     """What serves a product that carries a norm (`fused_rows_take`; `kind` "scaled",
-    "scaled_swiglu" or "residual"): (tile shape or -1 for the library's product with the norm's
+    "scaled_swiglu" or "residual"): (tile shape, from 16 on those of the kernel that shares K out inside a block, or -1 for the library's product with the norm's
     work behind it, shares of K); None with the tuner on for a size it has not met."""
     info = (ctypes.c_int * 2)()
     if not _matmul().q3_matmul_fused_plan(_KINDS[kind], int(M), int(N), int(K), info):
@@ -1880,6 +1880,19 @@ def sums_stride(M):
     return -(-M // 16) * 16
 
 
+GROUPS_LEAST_COLUMNS = 4096
+
+
+def _groups_before_few(weight, M, unscaled):
+    """Whether rows that still lack their norm go by the kernel that shares K out inside a block although the few-row kernel
+    takes as many: 17 rows and more of a small weight of 4,096 columns or more, where both add alike (an inner size of 1,024, say),
+    so that a row's bits do not change with the number of rows. There the few-row kernel, a block per 16
+    columns and 16 rows, needs two rounds of blocks: 24, 32 and 64 rows of 4,096 x 1,024 6.4, 6.7 and 10.3 us, of 8,192 x 1,024
+    10.7, 11.4 and 18.5, the other kernel 5.4, 5.6, 6.1 and 6.9, 7.0, 8.3; 24 rows of 1,024 x 2,048 6.2 and 6.8."""
+    return (unscaled is not None and M > FEW_ROWS and weight.shape[0] >= GROUPS_LEAST_COLUMNS and fused_rows_take(weight, M)
+            and _matmul().q3_groups_as_few(M, weight.shape[0], weight.shape[1]))
+
+
 def _tiled_ok(tiled, weight, M):
     if tiled is None or not 1 <= M <= few_rows_limit(weight):
         return False
@@ -2021,7 +2034,7 @@ def linear(x, weight, out_dtype=None, out=None, tiled=None, unscaled=None, narro
     if unscaled is None and _narrow_ok(narrow, x, weight) and out.data_ptr() % 16 == 0:
         _check(library("gemm").q3_linear_narrow(_ptr(x), _ptr(narrow), _ptr(out), M, N, K, 0, _stream()), "linear")
         return out
-    if M and x.dtype == torch.bfloat16 and _tiled_ok(tiled, weight, M):
+    if M and x.dtype == torch.bfloat16 and _tiled_ok(tiled, weight, M) and not _groups_before_few(weight, M, unscaled):
         sums, sums_rows, eps, width, stride = _row_sums_args(unscaled, M, K)
         _check(library("gemm").q3_linear_tiled(
             _ptr(x), _ptr(tiled), _ptr(out), M, N, K, _DT[out_dtype], 0, sums, sums_rows, eps, width,
@@ -2105,7 +2118,7 @@ def linear_swiglu(x, weight, tiled=None, unscaled=None, kind="silu", narrow=None
         out = torch.empty((M, N // 2), dtype=x.dtype, device=x.device)
         if _stream_product(x, weight, tiled, out, True, unscaled, "linear_swiglu", kind):
             return out
-    if M and x.dtype == torch.bfloat16 and _tiled_ok(tiled, weight, M):
+    if M and x.dtype == torch.bfloat16 and _tiled_ok(tiled, weight, M) and not (kind == "silu" and _groups_before_few(weight, M, unscaled)):
         out = torch.empty((M, N // 2), dtype=x.dtype, device=x.device)
         sums, sums_rows, eps, width, stride = _row_sums_args(unscaled, M, K)
         _check(library("gemm").q3_linear_tiled(
@@ -2150,7 +2163,8 @@ def linear_residual_norm(x, weight, tiled, residual, norm_weight):
 
     Up to `few_rows_limit(weight)` rows, with the weight's tiled copy and N a multiple of 16, it
     is the few-row kernel's epilogue (P = N / 16, partial sums of 16 columns). With more rows, up
-    to 128 or 640 (`fused_rows_take`; `tiled` is not used), the tiled kernel's partial products are added
+    to 128 or 640 (`fused_rows_take`; `tiled` is not used), it is the epilogue of the kernel that shares K out inside
+    a block (a small weight; P = N over its tiles' columns, 16 to 128), or the tiled kernel's partial products are added
     by a second kernel that does the same (P = ceil(N / 1024)). There the result is None, and
     nothing was done, for a size at which the plain product (`linear`) followed by the norm's own
     kernel is the faster way."""
@@ -2169,10 +2183,10 @@ def linear_residual_norm(x, weight, tiled, residual, norm_weight):
         if not x.is_contiguous():
             raise OperandError("x must be contiguous")
         lib = _matmul()
-        sums = torch.empty((lib.q3_tiles_residual_chunks(N), sums_stride(M)), dtype=torch.float32, device=x.device)
+        sums = torch.empty((lib.q3_tiles_residual_chunks(M, N, K), sums_stride(M)), dtype=torch.float32, device=x.device)
         status = lib.q3_tiles_residual(
             _ptr(x), _ptr(weight), M, N, K, _ptr(residual), _ptr(norm_weight), _DT[norm_weight.dtype], _ptr(values),
-            _ptr(sums), sums.shape[1], _stream())
+            _ptr(sums), sums.shape[0], sums.shape[1], _stream())
         if status == _DECLINED:
             return None
         _check(status, "linear_residual_norm")

@@ -1,0 +1,71 @@
+"""Products that carry a norm by the kernel that shares K out inside a block, at the edges of its tiles."""
+
+import pytest
+import torch
+
+from test_kernels_gpu import _ops, _rand
+
+pytestmark = pytest.mark.gpu
+
+
+# every shape of the dispatch (by its number), at rows and columns that end inside a tile, and inner sizes that leave
+# groups without a stage, with a short share and with an uneven one
+@pytest.mark.parametrize("M,N,K,shape", [(17, 4096, 64, 0), (17, 1028, 8640, 0), (33, 4084, 192, 1), (64, 4096, 1024, 1), (100, 4092, 1344, 2),
+                                         (65, 8188, 1024, 3), (201, 8188, 320, 4), (257, 8180, 1088, 5), (640, 4100, 2176, 5),
+                                         (128, 32764, 1088, 5)])
+def test_products_that_carry_a_norm(M, N, K, shape):
+    ops = _ops()
+    assert ops.matmul_fused_plan("scaled", M, N, K) == (16 + shape, 1)
+    x, w = _rand((M, K), torch.bfloat16, 91), _rand((N, K), torch.bfloat16, 92, scale=0.05)
+    sums = (0.5 + torch.rand((37, ops.sums_stride(M)), generator=torch.Generator().manual_seed(93))).cuda() * K / 37
+    eps = 1e-5
+    factor = torch.rsqrt(sums[:, :M].double().sum(dim=0) / K + eps)[:, None]
+    exact = (x.double() @ w.double().T) * factor
+    # K products of bfloat16 numbers summed in float32, K roundings of 2^-24 of the sum of the magnitudes at most, and the
+    # factor's few
+    bound = (K + 64) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T) * factor
+    got = ops.linear(x, w, out_dtype=torch.float32, unscaled=(sums, eps, K))
+    assert bool(((got.double() - exact).abs() <= bound).all())
+    assert torch.equal(ops.linear(x, w, unscaled=(sums, eps, K)), got.bfloat16())
+    assert torch.equal(ops.linear_swiglu(x, w, unscaled=(sums, eps, K)), ops.swiglu(got.bfloat16()))
+
+
+@pytest.mark.parametrize("norm_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K,columns", [(65, 1024, 2048, 16), (129, 1012, 4096, 32), (400, 1024, 1088, 32), (640, 1016, 3200, 64),
+                                           (300, 4100, 320, 128)])
+def test_residual_addition_and_the_next_norm(M, N, K, columns, norm_dtype):
+    ops = _ops()
+    x, w = _rand((M, K), torch.bfloat16, 94), _rand((N, K), torch.bfloat16, 95, scale=0.05)
+    nw = (1.0 + _rand((N,), torch.float32, 96, scale=0.2)).to(norm_dtype)
+    residual = _rand((M, N), torch.float32, 97, scale=2.0)
+    exact = x.double() @ w.double().T
+    stream = residual.clone()
+    values, sums = ops.linear_residual_norm(x, w, None, stream, nw)
+    assert sums.shape == (-(-N // columns), ops.sums_stride(M))
+    # the product rounded to bfloat16 once, from a float32 sum that is off by what its additions round
+    delta = (stream - residual).double()
+    bound = 2.0 ** -8 * exact.abs() + (K + 64) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T) + 2.0 ** -23 * stream.double().abs()
+    assert bool(((delta - exact).abs() <= bound).all())
+    assert torch.equal(values, (stream * nw.float()).bfloat16())
+    torch.testing.assert_close(sums[:, :M].double().sum(dim=0), (stream.double() ** 2).sum(dim=1), rtol=1e-5, atol=1e-6)
+    again = residual.clone()
+    v2, s2 = ops.linear_residual_norm(x, w, None, again, nw)
+    assert torch.equal(again, stream) and torch.equal(v2, values) and torch.equal(s2[:, :M], sums[:, :M])
+
+
+def test_rows_that_two_kernels_take():
+    """17 to 64 rows of a small weight: from 4,096 columns on not the few-row kernel, with its bits."""
+    ops = _ops()
+    for N, M in ((4096, 17), (4096, 64), (8192, 32), (1024, 64)):
+        torch.manual_seed(100)
+        x, w = _rand((M, 1024), torch.bfloat16, 98), _rand((N, 1024), torch.bfloat16, 99, scale=0.05)
+        tiled, sums = ops.tile_weight(w), torch.rand((64, ops.sums_stride(M)), device="cuda") * 32.0
+        got = ops.linear(x, w, out_dtype=torch.float32, tiled=tiled, unscaled=(sums, 1e-5, 1024))
+        by_tiles = ops.linear(x, w, out_dtype=torch.float32, unscaled=(sums, 1e-5, 1024))
+        assert bool(ops._groups_before_few(w, M, (sums, 1e-5, 1024))) == (N >= 4096)
+        assert not ops._groups_before_few(w, 16, (sums, 1e-5, 1024)) and not ops._groups_before_few(w, M, None)
+        torch.testing.assert_close(got, by_tiles, rtol=1e-4, atol=1e-4)
+        first = ops.linear(x[:16].contiguous(), w, out_dtype=torch.float32, tiled=tiled, unscaled=(sums[:, :16].contiguous(), 1e-5, 1024))
+        assert torch.equal(first, got[:16])
+    w = _rand((4096, 2048), torch.bfloat16, 99)          # eight shares of K there, four here
+    assert not ops._groups_before_few(w, 32, (sums, 1e-5, 2048))
