@@ -78,6 +78,19 @@ class CacheStorage:
         """`block_tables`: per paged group the step's int32 (B, W) device tensor."""
         self._block_tables = block_tables
 
+    def pages_of(self, planes, names):
+        """([per plane its tensors of these names], the block table) for planes of one group of pages that has them, as `view`
+        gives them one by one; (None, None) for planes of several groups."""
+        groups = {self.manager.group_of_plane[plane] for plane in planes}
+        if len(groups) != 1 or min(groups) < 0:
+            return None, None
+        g = groups.pop()
+        held = self.manager.groups[g].planes
+        if not all(name in self.paged[g] for name in names):
+            return None, None
+        tensors = [self.paged[g][name].unbind(0) for name in names]
+        return [tuple(t[held.index(plane)] for t in tensors) for plane in planes], self._block_tables[g]
+
     def view(self, plane, writes=True):
         m = self.manager
         view = LayerCacheView(writes=writes)

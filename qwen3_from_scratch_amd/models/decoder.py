@@ -6,6 +6,7 @@ import torch
 
 from ..parts.base import build_part
 from ..weights.checkpoint import check_tensors
+from .layer_run import layer_runs
 
 
 class _Layer:
@@ -55,6 +56,7 @@ class DecoderModel:
         self.head = build_part(spec.head, spec.head_prefix, precision, device)
         # each run-order entry that owns a cache gets a plane; readers point at the owner's
         self.observer = None      # called with (run-order entry, stream, what it still lacks) behind every layer
+        self.runs = {}            # step -> the stretch of layers that may run as one native call with it (set by load)
         self.plane_of_step = []
         self.plane_needs = []
         for i, step in enumerate(spec.order):
@@ -127,6 +129,7 @@ class DecoderModel:
         with torch.no_grad():
             for part in self.parts():
                 part.load(fetch)
+        self.runs = layer_runs(self)
         return self
 
     @torch.no_grad()
@@ -139,7 +142,16 @@ class DecoderModel:
         start = x.clone() if getattr(self.pass_vectors, "wants_start", False) else None
         pending = None
         order = self.spec.order
+        behind = 0                           # the first step that is not done yet
         for i, step in enumerate(order):
+            if i < behind:
+                continue
+            if i in self.runs and self.observer is None:
+                done = self.runs[i].forward(i, x, pending, batch, cache)
+                if done is not None:
+                    x, pending = done
+                    behind = self.runs[i].end
+                    continue
             view = cache.view(self.plane_of_step[i], writes=step.reads_cache_of is None)
             # the norm at the next block's entry, if that block can take over its division
             entry = getattr(self.layers[order[i + 1].layer].block, "entry_norm", None) if i + 1 < len(order) else None

@@ -1,0 +1,54 @@
+"""Stretches of equal layers that a step may run as one native call."""
+
+from ..ops.layers import DecoderLayers
+from ..parts.base import UnscaledRows
+
+
+class LayerRun:
+    """The steps `begin` .. `end - 1` of a model's run order, whose layers `ops.layers.DecoderLayers` takes: layers of one shape,
+    each with a cache plane of its own to write, each followed by one whose entry norm its last product prepares."""
+
+    def __init__(self, begin, end, native, position, planes, exit_norm):
+        self.begin, self.end = begin, end
+        self.native, self.position, self.planes, self.exit_norm = native, position, planes, exit_norm
+
+    def forward(self, first, x, pending, batch, cache):
+        """The layers from step `first` on, as their blocks would run them: (stream, what it still lacks), or None, with nothing
+        done, for a step that is another kernel's: one that does not come as UnscaledRows, of single tokens alone
+        (attention with its own preparation), or of rows that a product does not take in the form that carries its norm."""
+        if not isinstance(pending, UnscaledRows) or batch.max_q_len == 1 or not self.native.rows_fit(x.shape[0]):
+            return None
+        caches, block_table = cache.pages_of(self.planes[first - self.begin:], ("keys", "values"))
+        if caches is None:
+            return None
+        table = self.position.rotation_table() if self.position is not None else None
+        done = self.native.run(first - self.begin, self.end - first, x, pending.values, pending.sums, caches, block_table,
+                               batch.positions, batch.seq_index, batch.cu_seqlens_q, batch.kv_lens, batch.max_q_len,
+                               batch.min_q_len, batch.max_kv_len, getattr(batch, "max_kv_len_portions", None), table)
+        if done is None:
+            return None
+        return x, UnscaledRows(done[0], done[1], self.exit_norm.eps, self.exit_norm.size)
+
+
+def layer_runs(model):
+    """{step of the run order: the LayerRun it belongs to} for every step that belongs to one."""
+    order, found, runs = model.spec.order, [], {}
+    for i, step in enumerate(order):
+        block, entry = model.layers[step.layer].block, None
+        if step.enters is None and step.reads_cache_of is None and i + 1 < len(order) and order[i + 1].enters is None:
+            after = getattr(model.layers[order[i + 1].layer].block, "entry_norm", None)
+            entry = after() if after else None
+        found.append(block.native_layer(entry) if entry is not None and hasattr(block, "native_layer") else None)
+    at = 0
+    while at < len(order):
+        end = at
+        while end < len(order) and found[at] and found[end] and found[end][1:] == found[at][1:]:
+            end += 1
+        if end > at:
+            native = DecoderLayers.of([f[0] for f in found[at:end]], **found[at][1])
+            if native is not None:
+                exit_norm = model.layers[order[end].layer].block.entry_norm()
+                run = LayerRun(at, end, native, found[at][2], [model.plane_of_step[i] for i in range(at, end)], exit_norm)
+                runs.update((i, run) for i in range(at, end))
+        at = max(end, at + 1)
+    return runs

@@ -31,7 +31,7 @@ FLAGS = [
     "-Wno-unused-command-line-argument",
 ]
 MODULES = ("elementwise", "norm", "rotary", "attention", "attention_capped", "attention_pooled", "attention_sigmoid", "attention_span", "latent", "moe",
-           "hyper", "recurrent", "mlstm", "delta", "softcap", "gemm", "matmul", "sampling", "probes")
+           "hyper", "recurrent", "mlstm", "delta", "softcap", "gemm", "matmul", "sampling", "probes", "layers")
 # what a module links besides the HIP runtime
 LINKS = {"matmul": ["-lhipblaslt"]}
 

@@ -1,0 +1,161 @@
+"""A stretch of equal decoder layers as one native call (csrc/layers.hip): what the layers' parts would do operation by
+operation, for steps whose time is the host's."""
+
+import ctypes
+
+import torch
+
+from . import (_DT, _check, _matmul, _splits, _stream, few_rows_limit, fused_rows_most, library, matmul_fused_plan, sums_stride,
+               FUSED_ROWS_SMALL, OperandError)
+
+_P, _I, _F = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
+
+
+class _Layer(ctypes.Structure):
+    _fields_ = [(n, _P) for n in ("qkv", "out", "gate_up", "down", "q_norm", "k_norm", "middle_norm", "next_norm", "keys", "values")
+                ] + [("entry_eps", _F), ("middle_eps", _F)]
+
+
+class _Step(ctypes.Structure):
+    _fields_ = ([(n, _P) for n in ("scaled", "residual", "prepare", "attention", "stream")]
+                + [(n, _I) for n in ("rows", "width", "heads", "kv_heads", "dim", "inner", "norm_dtype", "qk_dtype")]
+                + [("qk_eps", _F), ("scale", _F), ("window", _I), ("table", _P), ("rotary_dim", _I), ("max_pos", _I)]
+                + [(n, _P) for n in ("positions", "seq_index", "block_table", "cu_q", "kv_lens")]
+                + [(n, _I) for n in ("table_width", "sequences", "page", "num_pages", "max_q_len", "min_q_len", "max_kv_len",
+                                     "splits", "prompt_splits")]
+                + [(n, _P) for n in ("workspace", "prompt_workspace", "residual_rows", "entry_values", "entry_sums")]
+                + [(n, _I) for n in ("entry_chunks", "sums_stride", "middle_chunks", "exit_chunks")]
+                + [(n, _P) for n in ("qkv_rows", "attended", "hidden", "norm_rows", "middle_sums", "exit_sums")])
+
+
+_OPERATIONS = ("the product of queries, keys and values", "qk_norm_rope_store", "paged_attention", "the attention's output product",
+               "the gated product", "the product back into the stream")
+
+
+def _matrix(t, shape):
+    return (t is not None and t.is_cuda and t.dtype == torch.bfloat16 and t.shape == shape and t.is_contiguous()
+            and fused_rows_most(t) == FUSED_ROWS_SMALL and shape[1] % 64 == 0 and shape[0] % 4 == 0)
+
+
+def _vector(t, size, dtype):
+    return t is not None and t.is_cuda and t.shape == (size,) and t.dtype == dtype and t.is_contiguous()
+
+
+class DecoderLayers:
+    """Layers of one shape: `layers`, per layer a dict of its tensors (`qkv`, `out`, `gate_up` with its rows interleaved, `down`;
+    `q_norm`, `k_norm` or None; `middle_norm`, `next_norm`) and `entry_eps`, `middle_eps`; and the sizes they share. The
+    tensors are looked at here, once; `None` from `of` if they are not what the native call takes."""
+
+    def __init__(self, layers, heads, kv_heads, dim, width, inner, qk_eps, scale, window):
+        self.layers = layers
+        self.heads, self.kv_heads, self.dim, self.width, self.inner = heads, kv_heads, dim, width, inner
+        self.qk_eps, self.scale, self.window = float(qk_eps), float(scale), int(window)
+        self.norm_dtype = layers[0]["middle_norm"].dtype
+        self.qk_dtype = layers[0]["q_norm"].dtype if layers[0]["q_norm"] is not None else torch.float32
+        self.least_rows = 1 + max(few_rows_limit(l[n]) for l in layers for n in ("qkv", "out", "gate_up", "down"))
+
+    @classmethod
+    def of(cls, layers, heads, kv_heads, dim, width, inner, qk_eps, scale, window):
+        norm_dtype = getattr(layers[0]["middle_norm"], "dtype", None)
+        for l in layers:
+            if not (_matrix(l["qkv"], ((heads + 2 * kv_heads) * dim, width)) and _matrix(l["out"], (width, heads * dim))
+                    and _matrix(l["gate_up"], (2 * inner, width)) and _matrix(l["down"], (width, inner))
+                    and norm_dtype in _DT and _vector(l["middle_norm"], width, norm_dtype) and _vector(l["next_norm"], width, norm_dtype)):
+                return None
+            if (l["q_norm"] is None) != (l["k_norm"] is None) or (l["q_norm"] is None) != (layers[0]["q_norm"] is None):
+                return None
+            if l["q_norm"] is not None and not (l["q_norm"].dtype in _DT and _vector(l["q_norm"], dim, layers[0]["q_norm"].dtype)
+                                                and _vector(l["k_norm"], dim, layers[0]["q_norm"].dtype)):
+                return None
+        return cls(layers, heads, kv_heads, dim, width, inner, qk_eps, scale, window)
+
+    def rows_fit(self, rows):
+        """Whether a step of so many rows is one whose four products all carry their norms by kernels that take row-major weights."""
+        if not self.least_rows <= rows <= FUSED_ROWS_SMALL:
+            return False
+        plans = [matmul_fused_plan("residual", rows, self.width, k) for k in (self.heads * self.dim, self.inner)]
+        return all(plan is not None and plan[0] >= 0 for plan in plans)
+
+    def run(self, first, count, stream, values, sums, caches, block_table, positions, seq_index, cu_seqlens_q, kv_lens, max_q_len,
+            min_q_len, max_kv_len, max_kv_len_of_many, table):
+        """Layers `first` .. `first + count - 1` over the residual `stream` (T, width) float32, in place, from rows
+        (`values`, `sums`: see `linear_residual_norm`) that lack the first one's entry norm. `caches`: per layer (keys, values), as
+        `paged_attention` takes them, all of one shape. Returns the rows that lack the norm behind the last layer, as (values,
+        sums); None, and nothing is done, where the attention is not one for the matrix cores."""
+        if not (0 <= first and 0 < count <= len(self.layers) - first and len(caches) == count and caches[0][0].dim() == 4):
+            raise OperandError("a cache for each of the layers, keys (pages, Hkv, page, D)")
+        T = values.shape[0]
+        H, G, D, page = self.heads, self.kv_heads, self.dim, caches[0][0].shape[2]
+        B = kv_lens.shape[0]
+        stride = sums_stride(T)
+        if not (stream.is_cuda and stream.shape == (T, self.width) and stream.dtype == torch.float32 and stream.is_contiguous()
+                and values.shape == (T, self.width) and values.dtype == torch.bfloat16 and values.is_cuda and values.is_contiguous()
+                and sums.is_cuda and sums.dim() == 2 and sums.shape[1] == stride and sums.dtype == torch.float32 and sums.is_contiguous()):
+            raise OperandError("a float32 stream, bfloat16 rows and float32 sums of squares, contiguous")
+        for t, shape in ((positions, (T,)), (seq_index, (T,)), (cu_seqlens_q, (B + 1,)), (kv_lens, (B,))):
+            if not (t.is_cuda and t.dtype == torch.int32 and t.shape == shape and t.is_contiguous()):
+                raise OperandError("positions and seq_index int32 (T,), cu_seqlens_q int32 (B+1,), kv_lens int32 (B,)")
+        if not (block_table.is_cuda and block_table.dim() == 2 and block_table.dtype == torch.int32 and block_table.shape[0] >= B
+                and block_table.is_contiguous() and block_table.shape[1] * page >= max_kv_len and 1 <= min_q_len <= max_q_len):
+            raise OperandError("block_table must be int32 (B, W) and hold the longest sequence")
+        pages = caches[0][0].shape[0]
+        for keys, held in caches:
+            if not (keys.is_cuda and keys.dtype == torch.bfloat16 and keys.shape == (pages, G, page, D) and keys.is_contiguous()
+                    and held.is_cuda and held.dtype == torch.bfloat16 and held.shape == (pages, G, D, page) and held.is_contiguous()
+                    and pages > 0):
+                raise OperandError("caches must be keys (pages, Hkv, page, D) and values (pages, Hkv, D, page) in bfloat16")
+        rotary_dim, max_pos = 0, 0
+        if table is not None:
+            if not (table.is_cuda and table.dim() == 2 and table.dtype == torch.float32 and table.is_contiguous()
+                    and table.shape[1] % 2 == 0 and table.shape[1] <= D and max_kv_len <= table.shape[0]):
+                raise OperandError("table must be float32 (P, R) and hold the step's last position")
+            max_pos, rotary_dim = table.shape
+        matmul, rotary, attention = _matmul(), library("rotary"), library("attention")
+        if not attention.q3_paged_attention_fast_path(H, G, D, page, 1):
+            return None
+
+        def empty(*shape, dtype=torch.bfloat16):
+            return torch.empty(shape, dtype=dtype, device=values.device)
+
+        splits, workspace, prompt_splits, prompt_workspace = 1, None, 1, None
+        if min_q_len * (H // G) <= 16:
+            splits = _splits(B, G, int(max_kv_len))
+            if splits > 1:
+                attention.q3_paged_attention_workspace.restype = ctypes.c_long
+                workspace = empty(attention.q3_paged_attention_workspace(B, G, D, splits), dtype=torch.float32)
+        if max_q_len * (H // G) > 16:
+            longest = int(max_kv_len if max_kv_len_of_many is None else max_kv_len_of_many)
+            prompt_splits = attention.q3_paged_attention_prompt_splits(T, H, G, longest)
+            if prompt_splits > 1:
+                prompt_workspace = empty(T * H * prompt_splits * (D + 2), dtype=torch.float32)
+        out = empty(T, self.width)
+        middle = empty(matmul.q3_tiles_residual_chunks(T, self.width, H * D), stride, dtype=torch.float32)
+        exit_ = empty(matmul.q3_tiles_residual_chunks(T, self.width, self.inner), stride, dtype=torch.float32)
+        qkv, attended, hidden = empty(T, (H + 2 * G) * D), empty(T, H * D), empty(T, self.inner)
+
+        def at(t):
+            return None if t is None else t.data_ptr()
+
+        step = _Step(
+            scaled=ctypes.cast(matmul.q3_tiles_scaled, _P), residual=ctypes.cast(matmul.q3_tiles_residual, _P),
+            prepare=ctypes.cast(rotary.q3_qk_norm_rope_store, _P), attention=ctypes.cast(attention.q3_paged_attention, _P),
+            stream=_stream(), rows=T, width=self.width, heads=H, kv_heads=G, dim=D, inner=self.inner,
+            norm_dtype=_DT[self.norm_dtype], qk_dtype=_DT[self.qk_dtype], qk_eps=self.qk_eps, scale=self.scale, window=self.window,
+            table=at(table), rotary_dim=rotary_dim, max_pos=max_pos, positions=at(positions), seq_index=at(seq_index),
+            block_table=at(block_table), cu_q=at(cu_seqlens_q), kv_lens=at(kv_lens), table_width=block_table.shape[1], sequences=B,
+            page=page, num_pages=pages, max_q_len=int(max_q_len), min_q_len=int(min_q_len), max_kv_len=int(max_kv_len),
+            splits=splits, prompt_splits=prompt_splits, workspace=at(workspace), prompt_workspace=at(prompt_workspace),
+            residual_rows=at(stream), entry_values=at(values), entry_sums=at(sums), entry_chunks=sums.shape[0], sums_stride=stride,
+            middle_chunks=middle.shape[0], exit_chunks=exit_.shape[0], qkv_rows=at(qkv), attended=at(attended), hidden=at(hidden),
+            norm_rows=at(out), middle_sums=at(middle), exit_sums=at(exit_))
+        layers = (_Layer * count)()
+        for native, l, (keys, held) in zip(layers, self.layers[first:first + count], caches):
+            native.qkv, native.out, native.gate_up, native.down = at(l["qkv"]), at(l["out"]), at(l["gate_up"]), at(l["down"])
+            native.q_norm, native.k_norm = at(l["q_norm"]), at(l["k_norm"])
+            native.middle_norm, native.next_norm = at(l["middle_norm"]), at(l["next_norm"])
+            native.keys, native.values = keys.data_ptr(), held.data_ptr()
+            native.entry_eps, native.middle_eps = l["entry_eps"], l["middle_eps"]
+        failed = ctypes.c_int(0)
+        _check(library("layers").q3_decoder_layers(layers, count, ctypes.byref(step), ctypes.byref(failed)),
+               _OPERATIONS[failed.value])
+        return out, exit_

@@ -97,6 +97,14 @@ class PagedAttention(Part):
     def unscaled_rows_most(self):
         return self.qkv.fused_rows_most
 
+    def native_half(self):
+        """What a native stretch of layers (`ops.layers.DecoderLayers`) needs of this part, or None."""
+        if type(self) is not PagedAttention or self.qkv is None:
+            return None
+        return (dict(qkv=self.qkv.weight, out=self.out.weight, q_norm=self.q_weight, k_norm=self.k_weight),
+                dict(heads=self.num_heads, kv_heads=self.num_kv_heads, dim=self.head_dim, width=self.hidden_size,
+                     qk_eps=self.qk_norm_eps, scale=self.scale, window=self.window))
+
     def forward(self, x, batch, cache, sink=None):
         Hq, Hkv, D = self.num_heads, self.num_kv_heads, self.head_dim
         qkv = self.qkv.forward(x)

@@ -4,6 +4,7 @@ from ..config.registry import register_part
 import torch
 
 from .base import BiasedRows, HyperAddend, Part, TensorShape, UnscaledRows
+from .norm import RMSNorm
 
 
 def _says(part, what):
@@ -49,6 +50,24 @@ class PreNormBlock(Part):
         """The norm a preceding block may fuse into its last product (see
         NormSink), or None if this block's mixer wants finished rows."""
         return self.mixer_norm if _says(self.mixer, "takes_unscaled") and hasattr(self.mixer_norm, "sink_for") else None
+
+    def native_layer(self, next_norm):
+        """(a layer's tensors, the sizes that equal layers share, the position part) for `ops.layers.DecoderLayers`, or None
+        for a layer of other parts, or of parts that do not go from UnscaledRows to UnscaledRows."""
+        parts = (self.mixer, self.feed_forward)
+        norms = (self.mixer_norm, self.feed_forward_norm, next_norm)
+        if type(self) is not PreNormBlock or not all(hasattr(part, "native_half") for part in parts):
+            return None
+        if not all(type(norm) is RMSNorm and norm.weight is not None for norm in norms):
+            return None
+        if not all(_says(part, "takes_unscaled") and _says(part, "feeds_sink") and part.precision.tiled for part in parts):
+            return None
+        halves = [part.native_half() for part in parts]
+        if None in halves:
+            return None
+        (mixing, sizes), (feeding, more) = halves
+        return (dict(mixing, **feeding, middle_norm=norms[1].weight, next_norm=norms[2].weight, entry_eps=norms[0].eps,
+                     middle_eps=norms[1].eps), dict(sizes, **more), self.mixer.position)
 
     def forward(self, x, pending, batch, cache, next_norm=None):
         """`pending`: None, the addend the stream still lacks, or UnscaledRows

@@ -57,6 +57,12 @@ class SwiGLU(Part):
     def unscaled_rows_most(self):
         return self.gate_up.fused_rows_most
 
+    def native_half(self):
+        """What a native stretch of layers (`ops.layers.DecoderLayers`) needs of this part, or None."""
+        if type(self) is not SwiGLU or self.activation != "silu" or self.gate_up is None:
+            return None
+        return dict(gate_up=self.gate_up.weight, down=self.down.weight), dict(inner=self.intermediate_size)
+
     def forward(self, x, batch=None, sink=None):
         h = self.gate_up.forward_swiglu(x, self.activation)
         return self.down.forward(h) if sink is None else self.down.forward_into(h, sink)

@@ -1,0 +1,88 @@
+"""Stretches of layers that run as one native call against the same layers run part by part."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _model(layers=5, qk_norm="Qwen3ForCausalLM", dtype="bfloat16", tiled=True):
+    from qwen3_from_scratch_amd.config import ModelConfig
+    from qwen3_from_scratch_amd.engine import random_model
+
+    config = ModelConfig.from_dict(dict(
+        architectures=[qk_norm], vocab_size=512, hidden_size=1024, hidden_act="silu", num_hidden_layers=layers,
+        max_position_embeddings=8192, num_attention_heads=16, num_key_value_heads=8, head_dim=128,
+        intermediate_size=2048, rms_norm_eps=1e-6, rope_theta=1e6, tie_word_embeddings=False))
+    return random_model(config, dtype=dtype, device="cuda:0", seed=5)
+
+
+def _steps(seed, *steps):
+    from qwen3_from_scratch_amd.engine import StepEntry
+
+    g = torch.Generator().manual_seed(seed)
+    return [[StepEntry(rid, torch.randint(0, 512, (n,), generator=g).tolist(), [n - 1]) for rid, n in step] for step in steps]
+
+
+def _logits(model, steps, calls=None):
+    from qwen3_from_scratch_amd.engine import ModelRunner
+
+    runner = ModelRunner(model, 16, 700, max_requests=8)
+    out = []
+    for entries in steps:
+        if calls is not None:
+            calls.append(0)
+        out.append(runner.step(entries).clone())
+    return out
+
+
+# prompts alone (of 65 and of 640 rows too), a portion beside requests that decode, with prefixes long enough that keys are
+# shared out (decoding ones and a portion), and a step of too many rows, which is not the native call's
+STEPS = ((("a", 65),), (("b", 200), ("a", 1)), (("c", 640),), (("a", 3000),), (("a", 300), ("b", 1), ("c", 1)), (("d", 641),),
+         (("a", 1), ("b", 2), ("c", 70)))
+
+
+def test_the_same_bits(monkeypatch):
+    from qwen3_from_scratch_amd.ops.layers import DecoderLayers
+
+    model = _model()
+    assert sorted(model.runs) == [0, 1, 2, 3] and len(set(map(id, model.runs.values()))) == 1
+    steps = _steps(6, *STEPS)
+    took = []
+    run = DecoderLayers.run
+
+    def counted(self, first, count, *args):
+        done = run(self, first, count, *args)
+        took[-1] = (first, count)
+        assert done is not None
+        return done
+
+    monkeypatch.setattr(DecoderLayers, "run", counted)
+    got = _logits(model, steps, took)
+    # the first layer reads a norm's finished rows: the stretch begins behind it
+    assert took == [(1, 3), (1, 3), (1, 3), 0, (1, 3), 0, (1, 3)]
+    model.observer = lambda *args: None
+    want = _logits(model, steps, took)
+    assert took[7:] == [0] * 7
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+
+
+def test_layers_that_are_not_taken():
+    from qwen3_from_scratch_amd import ops
+
+    assert not _model(dtype="float32", layers=3).runs
+    model = _model(layers=3)
+    native = model.runs[0].native
+    assert [native.rows_fit(rows) for rows in (64, 65, 640, 641)] == [False, True, True, False]
+    try:
+        ops.matmul_kernels("library")                  # the residual's product is declined then
+        assert not native.rows_fit(200)
+    finally:
+        ops.matmul_kernels("both")
+    layer = dict(native.layers[0], down=native.layers[0]["down"][:, :-64])
+    sizes = dict(heads=16, kv_heads=8, dim=128, width=1024, inner=2048, qk_eps=1e-6, scale=1.0, window=0)
+    assert type(native).of([native.layers[0]], **sizes) is not None and type(native).of([layer], **sizes) is None
+    with pytest.raises(ops.OperandError):
+        rows = torch.zeros(70, 1024, device="cuda")
+        native.run(0, 1, rows, rows, rows, [(rows, rows)], rows, rows, rows, rows, rows, 70, 70, 70, None, None)
