@@ -404,6 +404,7 @@ static thread_local OutGate g_gate{};
 extern "C" void q3_set_gate(const float* gate, long stride, int wide) { g_gate = OutGate{gate, stride, wide}; }
 #define Q3_GATE_PARAM , OutGate gate
 #define Q3_GATE_ARG , g_gate
+#define Q3_GATE_PASS , gate
 // the factor of column d of head `head` (of D) of row `row`
 __device__ __forceinline__ float open_gate(const OutGate& g, int row, int head, int D, int d) {
   if (g.gate == nullptr) return 1.f;
@@ -414,12 +415,14 @@ __device__ __forceinline__ float open_gate(const OutGate& g, int row, int head, 
 #else
 #define Q3_GATE_PARAM
 #define Q3_GATE_ARG
+#define Q3_GATE_PASS
 #define Q3_OPEN(row, head, D, d)
 #endif
 
 #ifdef Q3_SIGMOID
 #define Q3_BIAS_PARAM , const float* __restrict__ score_bias
 #define Q3_BIAS_ARG , g_score_bias
+#define Q3_BIAS_PASS , score_bias
 static thread_local const float* g_score_bias = nullptr;
 extern "C" void q3_set_sigmoid_bias(const float* bias) { g_score_bias = bias; }
 // sigmoid of an argument that is given times log2(e); minus infinity gives nothing
@@ -427,6 +430,7 @@ __device__ __forceinline__ float sigmoid_log2(float x) { return __builtin_amdgcn
 #else
 #define Q3_BIAS_PARAM
 #define Q3_BIAS_ARG
+#define Q3_BIAS_PASS
 #endif
 
 // A build with Q3_POOLED (attention_pooled.hip) sees, beside the window's tokens, one key and value per
@@ -444,6 +448,7 @@ struct RunSource {
 };
 #define Q3_RUNS_PARAM , RunSource runs
 #define Q3_RUNS_ARG , g_runs
+#define Q3_RUNS_PASS , runs
 static thread_local RunSource g_runs{};
 extern "C" void q3_set_runs(const void* k, const void* v, const int* table, int stride, int num_pages, int pool) {
   g_runs = RunSource{(const bf16_t*)k, (const bf16_t*)v, table, stride, num_pages, pool};
@@ -456,6 +461,7 @@ __device__ __forceinline__ int runs_seen(int pos, int window, int pool) {
 #else
 #define Q3_RUNS_PARAM
 #define Q3_RUNS_ARG
+#define Q3_RUNS_PASS
 #endif
 
 // Which keys before its own position a row sees. Ordinarily `window` says it: all of them (0) or fewer than
@@ -904,15 +910,23 @@ __device__ __forceinline__ void store_new_value(const Half8 (&raw)[2], int c, bf
 
 // (left alone the compiler takes more registers than leave room for two wavefronts a SIMD)
 #define Q3_DECODE_WAVES __attribute__((amdgpu_waves_per_eu(2)))
-template <int D, bool PREP, typename W, bool AHEAD, int DV = D>
-__global__ __launch_bounds__(256) Q3_DECODE_WAVES void attn_decode_kernel(
-    const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, const bf16_t* __restrict__ k_cache,
+constexpr int DECODE_WAVES = 4;
+template <int D, bool PREP, int DV>
+struct DecodeShared {
+  float k[PREP ? D : 1], v[PREP ? D : 1];
+  float m[DECODE_WAVES + 1][16], l[DECODE_WAVES][16];
+  __attribute__((aligned(16))) float acc[DECODE_WAVES][16][DV + 4];
+};
+
+// A block's work: split `split` of sequence `b`'s keys for key head `g_kv`.
+template <int D, bool PREP, typename W, bool AHEAD, int DV>
+__device__ __forceinline__ void decode_block(
+    DecodeShared<D, PREP, DV>& shared, const int split, const int g_kv, const int b, const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, const bf16_t* __restrict__ k_cache,
     const bf16_t* __restrict__ v_cache, int num_pages, const int* __restrict__ block_table, int bt_stride,
     const int* __restrict__ cu_q, const int* __restrict__ kv_lens, int Hq, int Hkv, int page, score_scale_t scale_log2,
     span_t window, int splits, float* __restrict__ ws_acc, float* __restrict__ ws_ml, DecodePrep prep,
     const float* __restrict__ sink Q3_BIAS_PARAM Q3_RUNS_PARAM Q3_GATE_PARAM) {
-  constexpr int WAVES = 4;
-  const int b = blockIdx.z, g_kv = blockIdx.y, split = blockIdx.x;
+  constexpr int WAVES = DECODE_WAVES;
   const int G = Hq / Hkv;
   // a step of single tokens (PREP): sequence b's token is row b, and nothing is read to know it
   const int q0 = PREP ? b : cu_q[b];
@@ -963,7 +977,7 @@ __global__ __launch_bounds__(256) Q3_DECODE_WAVES void attn_decode_kernel(
   if (PREP && kv_len < 1) {
     // not a step of single tokens (the host sends no such row): the row's output is zero, and
     // the merge finds an empty share in this block's place, not whatever the workspace held
-    for (int i = threadIdx.x; i < rows * D; i += blockDim.x) {
+    for (int i = threadIdx.x; i < rows * D; i += 64 * WAVES) {
       const int r = i / D, d = i - r * D;
       if (splits == 1) {
         out[(size_t)(q0 + r / G) * Hq * D + (size_t)(g_kv * G + r % G) * D + d] = float_to_bf16(0.f);
@@ -1055,7 +1069,7 @@ __global__ __launch_bounds__(256) Q3_DECODE_WAVES void attn_decode_kernel(
   if constexpr (VALUES_AHEAD) load_values(even, page);
   __builtin_amdgcn_sched_barrier(0);     // the loads above are on their way before anything waits for them
 
-  __shared__ float sh_k[PREP ? D : 1], sh_v[PREP ? D : 1];
+  auto &sh_k = shared.k, &sh_v = shared.v;
   if (col >= rows) {
 #pragma unroll
     for (int i = 0; i < D / 32; ++i) qreg[0][i].u = make_uint4(0, 0, 0, 0);
@@ -1137,8 +1151,9 @@ __global__ __launch_bounds__(256) Q3_DECODE_WAVES void attn_decode_kernel(
 
   // the merge of the wavefronts, and of the new key as one more contribution of one key:
   // its score is its maximum, its sum is one, its accumulator is the value itself
-  __shared__ float sh_m[WAVES + 1][16], sh_l[WAVES][16];
-  __shared__ __attribute__((aligned(16))) float sh_acc[4][16][DV + 4];
+  auto& sh_m = shared.m;
+  auto& sh_l = shared.l;
+  auto& sh_acc = shared.acc;
   if (grp == 0) {
     sh_m[wave][col] = m_run[0];
     sh_l[wave][col] = l;
@@ -1194,6 +1209,19 @@ __global__ __launch_bounds__(256) Q3_DECODE_WAVES void attn_decode_kernel(
       if (d == 0) *reinterpret_cast<float2*>(ws_ml + slot * 2) = make_float2(mr, lr);
     }
   }
+}
+
+template <int D, bool PREP, typename W, bool AHEAD, int DV = D>
+__global__ __launch_bounds__(64 * DECODE_WAVES) Q3_DECODE_WAVES void attn_decode_kernel(
+    const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, const bf16_t* __restrict__ k_cache,
+    const bf16_t* __restrict__ v_cache, int num_pages, const int* __restrict__ block_table, int bt_stride,
+    const int* __restrict__ cu_q, const int* __restrict__ kv_lens, int Hq, int Hkv, int page, score_scale_t scale_log2,
+    span_t window, int splits, float* __restrict__ ws_acc, float* __restrict__ ws_ml, DecodePrep prep,
+    const float* __restrict__ sink Q3_BIAS_PARAM Q3_RUNS_PARAM Q3_GATE_PARAM) {
+  __shared__ DecodeShared<D, PREP, DV> shared;
+  decode_block<D, PREP, W, AHEAD, DV>(shared, blockIdx.x, blockIdx.y, blockIdx.z, q, q_stride, out, k_cache, v_cache, num_pages,
+                                      block_table, bt_stride, cu_q, kv_lens, Hq, Hkv, page, scale_log2, window, splits, ws_acc,
+                                      ws_ml, prep, sink Q3_BIAS_PASS Q3_RUNS_PASS Q3_GATE_PASS);
 }
 
 // Merge the splits' partial results: grid (Hkv, B), 256 threads; splits <= 64.
@@ -1436,22 +1464,29 @@ __device__ __forceinline__ void softmax_tile(const f32x4_t (&s)[KB4], bool full,
 #endif
 }
 
-template <int D, int TILE, int STAGES, int DV = D>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_prefill_kernel(
-    const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, const bf16_t* __restrict__ k_cache,
+template <int D, int TILE, int STAGES, int DV>
+struct PrefillShared {
+  __attribute__((aligned(16))) unsigned char stages[STAGES * PrefillSmem<D, TILE, DV>::STAGE];
+  long long kaddr[PREFILL_PAGES], vaddr[PREFILL_PAGES];
+  int pages[PREFILL_PAGES];
+};
+
+// A block's work: row tile and keys' share `y` of sequence `b`'s rows for key head `g_kv`.
+template <int D, int TILE, int STAGES, int DV>
+__device__ __forceinline__ void prefill_block(
+    PrefillShared<D, TILE, STAGES, DV>& shared, const int g_kv, const int y, const int b, const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, const bf16_t* __restrict__ k_cache,
     const bf16_t* __restrict__ v_cache, int num_pages, const int* __restrict__ block_table, int bt_stride,
     const int* __restrict__ cu_q, const int* __restrict__ kv_lens, int Hq, int Hkv, int page, score_scale_t scale_log2,
     span_t window, int tokens_per_block, int key_splits, float* __restrict__ part_acc, float* __restrict__ part_ml,
     const float* __restrict__ sink Q3_BIAS_PARAM Q3_RUNS_PARAM Q3_GATE_PARAM) {
   typedef PrefillSmem<D, TILE, DV> SM;
   constexpr int KB4 = TILE / 16;  // 16-key blocks per tile
-  __shared__ __attribute__((aligned(16))) unsigned char smem[STAGES * SM::STAGE];
-  __shared__ int sh_pages[PREFILL_PAGES];  // the block-table entries of the tiles in hand
+  auto& smem = shared.stages;
+  auto& sh_pages = shared.pages;   // the block-table entries of the tiles in hand
   // and the address at which each entry's (page, this key head) begins in either cache: worked out
   // once per entry, so that a tile's load finds its address with one read of this table and one
   // addition of a number the thread keeps for the whole kernel
-  __shared__ long long sh_kaddr[PREFILL_PAGES], sh_vaddr[PREFILL_PAGES];
-  const int b = blockIdx.z, g_kv = blockIdx.x;
+  auto &sh_kaddr = shared.kaddr, &sh_vaddr = shared.vaddr;
   const int G = Hq / Hkv;
   const int q0 = cu_q[b];
   const int q_len = cu_q[b + 1] - q0;
@@ -1459,7 +1494,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int n_tiles = (q_len + tokens_per_block - 1) / tokens_per_block;
   // with `key_splits` > 1 a row tile's keys are shared out over that many blocks, whose
   // unnormalised results attn_prefill_merge_kernel joins
-  const int split = (int)blockIdx.y % key_splits, tile_index = (int)blockIdx.y / key_splits;
+  const int split = y % key_splits, tile_index = y / key_splits;
   if (tile_index >= n_tiles) return;
   // the first half of a head's blocks takes the row tiles from the sequence's end downwards (the
   // long ones start first), the second half from its start upwards: block i and block
@@ -1960,6 +1995,85 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
 }
 
+template <int D, int TILE, int STAGES, int DV = D>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_prefill_kernel(
+    const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, const bf16_t* __restrict__ k_cache,
+    const bf16_t* __restrict__ v_cache, int num_pages, const int* __restrict__ block_table, int bt_stride,
+    const int* __restrict__ cu_q, const int* __restrict__ kv_lens, int Hq, int Hkv, int page, score_scale_t scale_log2,
+    span_t window, int tokens_per_block, int key_splits, float* __restrict__ part_acc, float* __restrict__ part_ml,
+    const float* __restrict__ sink Q3_BIAS_PARAM Q3_RUNS_PARAM Q3_GATE_PARAM) {
+  __shared__ PrefillShared<D, TILE, STAGES, DV> shared;
+  prefill_block<D, TILE, STAGES, DV>(shared, blockIdx.x, blockIdx.y, blockIdx.z, q, q_stride, out, k_cache, v_cache, num_pages,
+                                     block_table, bt_stride, cu_q, kv_lens, Hq, Hkv, page, scale_log2, window, tokens_per_block,
+                                     key_splits, part_acc, part_ml, sink Q3_BIAS_PASS Q3_RUNS_PASS Q3_GATE_PASS);
+}
+
+#if !defined(Q3_POOLED) && !defined(Q3_SIGMOID) && !defined(Q3_SPAN)
+// Row tile number `n` among those of all sequences of many rows, in their order: its sequence, and its number there in `n`; -1
+// behind the last. All lanes of a wavefront together.
+__device__ __forceinline__ int sequence_of_tile(int& n, const int* __restrict__ cu_q, int sequences, int G, int tokens_per_block) {
+  const int lane = threadIdx.x & 63;
+  for (int first = 0; first < sequences; first += 64) {
+    const int b = first + lane, rows = b < sequences ? cu_q[b + 1] - cu_q[b] : 0;
+    const int tiles = rows * G > 16 ? (rows + tokens_per_block - 1) / tokens_per_block : 0;
+    int upto = tiles;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int below = __shfl_up(upto, off, 64);
+      if (lane >= off) upto += below;
+    }
+    const unsigned long long past = __ballot(upto > n);
+    if (past) {
+      const int at = __ffsll((long long)past) - 1;
+      n -= __shfl(upto - tiles, at, 64);
+      return first + at;
+    }
+    n -= __shfl(upto, 63, 64);
+  }
+  return -1;
+}
+
+// Both kinds of sequences of a step without a window in one launch: `prompt_blocks` blocks for the prompts (Hkv per key share
+// and row tile, of as many row tiles as the sequences can come to; the last find none), the others for the decoding ones (splits x Hkv x
+// sequences). The decoding ones wait for memory and the prompts' for the matrix cores and the vector unit; a block of either
+// takes half a CU's registers and shared memory, so they run side by side. The kind that comes first (both in multiples of
+// eight blocks, so that a key head's blocks stay on its chiplet) is the prompts', whose chains are longer, where it leaves half of the
+// room, else the decoding one. 23 requests over 150 to 3,000 keys beside a prompt's rows, 32 heads in groups of four, microseconds:
+// one kernel after the other / in one launch, prompts first / decoding first: 512 rows over 512 keys 68 / 48 / 49, over 1,024 80 /
+// 51 / 58, 276 over 1,300 86 / 54 / 65, 512 over 3,584 (512 blocks of them) 109 / 104 / 84; 5 requests beside the first 38 / 27 / 31.
+template <int D, int TILE, int STAGES>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_mixed_kernel(
+    const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, const bf16_t* __restrict__ k_cache,
+    const bf16_t* __restrict__ v_cache, int num_pages, const int* __restrict__ block_table, int bt_stride,
+    const int* __restrict__ cu_q, const int* __restrict__ kv_lens, int sequences, int Hq, int Hkv, int page,
+    score_scale_t scale_log2, int prompts_first, int first_blocks, int tokens_per_block, int key_splits, float* __restrict__ part_acc,
+    float* __restrict__ part_ml, int splits, float* __restrict__ ws_acc, float* __restrict__ ws_ml,
+    const float* __restrict__ sink) {
+  __shared__ union {
+    DecodeShared<D, false, D> decode;
+    PrefillShared<D, TILE, STAGES, D> prompt;
+  } shared;
+  const bool first = (int)blockIdx.x < first_blocks;
+  const int id = first ? (int)blockIdx.x : (int)blockIdx.x - first_blocks;
+  if (first == (prompts_first != 0)) {
+    const int share = id / Hkv;
+    int tile = share / key_splits;
+    const int b = __builtin_amdgcn_readfirstlane(sequence_of_tile(tile, cu_q, sequences, Hq / Hkv, tokens_per_block));
+    if (b < 0) return;
+    tile = __builtin_amdgcn_readfirstlane(tile);
+    prefill_block<D, TILE, STAGES, D>(shared.prompt, id % Hkv, tile * key_splits + share % key_splits, b, q, q_stride, out,
+                                      k_cache, v_cache, num_pages, block_table, bt_stride, cu_q, kv_lens, Hq, Hkv, page,
+                                      scale_log2, 0, tokens_per_block, key_splits, part_acc, part_ml, sink);
+  } else {
+    const int pair = id / splits;
+    if (pair >= Hkv * sequences) return;
+    decode_block<D, false, float, true, D>(shared.decode, id % splits, pair % Hkv, pair / Hkv, q, q_stride, out, k_cache, v_cache,
+                                           num_pages, block_table, bt_stride, cu_q, kv_lens, Hq, Hkv, page, scale_log2, 0,
+                                           splits, ws_acc, ws_ml, DecodePrep{}, sink);
+  }
+}
+#endif
+
 // Joins the key splits of attn_prefill_kernel: grid (max_q_len, B), 256 threads; a block takes
 // one token of a sequence, a thread four neighbouring output elements of one (token, head)
 // row at a time. Sequences of few rows are the decoding kernel's.
@@ -2049,7 +2163,27 @@ static int launch_fast(const void* q, int q_stride, void* out, const void* k_cac
 #ifdef Q3_SIGMOID
   if (window != 0 || g_score_bias == nullptr || sink != nullptr) return Q3_ERR_BAD_ARGUMENT;
 #endif
-  if (min_q_len * G <= 16) {
+  const bool few = min_q_len * G <= 16, many = max_q_len * G > 16;
+  const int tokens_per_block = many ? prompt_tokens_per_block(total_tokens, G, Hkv, key_splits) : 1;
+  const int tiles = (max_q_len + tokens_per_block - 1) / tokens_per_block;
+  if (many && tiles * key_splits > 65535) return Q3_ERR_UNSUPPORTED;
+  float* part_acc = prompt_ws;
+  float* part_ml = prompt_ws ? prompt_ws + (size_t)total_tokens * Hq * key_splits * DV : nullptr;
+  bool together = false;
+#if !defined(Q3_POOLED) && !defined(Q3_SIGMOID) && !defined(Q3_SPAN)
+  // row tiles of the sequences of many rows: one each beyond whole ones, and as many sequences as there are rows for
+  const long row_tiles = total_tokens / tokens_per_block + min(B, total_tokens / (16 / G + 1));
+  const long prompt_blocks = (row_tiles * key_splits * Hkv + 7) / 8 * 8, decode_blocks = ((long)splits * Hkv * B + 7) / 8 * 8;
+  const bool prompts_first = (long)((total_tokens + tokens_per_block - 1) / tokens_per_block) * key_splits * Hkv <= 256;
+  together = few && many && window == 0 && (prompt_blocks + decode_blocks) * 256 < (1L << 32);
+  if (together)
+    hipLaunchKernelGGL((attn_mixed_kernel<D, TILE, PF_STAGES>), dim3((unsigned)(prompt_blocks + decode_blocks)), dim3(256), 0,
+                       stream, (const bf16_t*)q, q_stride, (bf16_t*)out, (const bf16_t*)k_cache, (const bf16_t*)v_cache,
+                       num_pages, block_table, bt_stride, cu_q, kv_lens, B, Hq, Hkv, page, scale_log2, prompts_first ? 1 : 0,
+                       (int)(prompts_first ? prompt_blocks : decode_blocks), tokens_per_block, key_splits, part_acc, part_ml,
+                       splits, ws_acc, ws_ml, sink);
+#endif
+  if (few && !together) {
 #if !defined(Q3_POOLED) && !defined(Q3_SPAN)
     if (window == 0)
       hipLaunchKernelGGL((attn_decode_kernel<D, false, float, true>), dim3(splits, Hkv, B), dim3(256), 0, stream,
@@ -2062,24 +2196,18 @@ static int launch_fast(const void* q, int q_stride, void* out, const void* k_cac
                          (const bf16_t*)q, q_stride, (bf16_t*)out, (const bf16_t*)k_cache, (const bf16_t*)v_cache,
                          num_pages, block_table, bt_stride, cu_q, kv_lens, Hq, Hkv, page, scale_log2, span, splits,
                          ws_acc, ws_ml, DecodePrep{}, sink Q3_BIAS_ARG Q3_RUNS_ARG Q3_GATE_ARG);
-    if (splits > 1)
-      hipLaunchKernelGGL(attn_decode_reduce_kernel<DV>, dim3(Hkv, B), dim3(256), 0, stream, (bf16_t*)out, cu_q, Hq,
-                         Hkv, splits, ws_acc, ws_ml, sink Q3_GATE_ARG);
   }
-  if (max_q_len * G > 16) {
-    const int tokens_per_block = prompt_tokens_per_block(total_tokens, G, Hkv, key_splits);
-    const int tiles = (max_q_len + tokens_per_block - 1) / tokens_per_block;
-    if (tiles * key_splits > 65535) return Q3_ERR_UNSUPPORTED;
-    float* part_acc = prompt_ws;
-    float* part_ml = prompt_ws ? prompt_ws + (size_t)total_tokens * Hq * key_splits * DV : nullptr;
+  if (few && splits > 1)
+    hipLaunchKernelGGL(attn_decode_reduce_kernel<DV>, dim3(Hkv, B), dim3(256), 0, stream, (bf16_t*)out, cu_q, Hq,
+                       Hkv, splits, ws_acc, ws_ml, sink Q3_GATE_ARG);
+  if (many && !together)
     hipLaunchKernelGGL((attn_prefill_kernel<D, TILE, PF_STAGES, DV>), dim3(Hkv, tiles * key_splits, B), dim3(256), 0,
                        stream, (const bf16_t*)q, q_stride, (bf16_t*)out, (const bf16_t*)k_cache,
                        (const bf16_t*)v_cache, num_pages, block_table, bt_stride, cu_q, kv_lens, Hq, Hkv, page,
                        scale_log2, span, tokens_per_block, key_splits, part_acc, part_ml, sink Q3_BIAS_ARG Q3_RUNS_ARG Q3_GATE_ARG);
-    if (key_splits > 1)
-      hipLaunchKernelGGL(attn_prefill_merge_kernel<DV>, dim3(max_q_len, B), dim3(256), 0, stream,
-                         (bf16_t*)out, cu_q, Hq, Hkv, key_splits, part_acc, part_ml, sink Q3_GATE_ARG);
-  }
+  if (many && key_splits > 1)
+    hipLaunchKernelGGL(attn_prefill_merge_kernel<DV>, dim3(max_q_len, B), dim3(256), 0, stream,
+                       (bf16_t*)out, cu_q, Hq, Hkv, key_splits, part_acc, part_ml, sink Q3_GATE_ARG);
   return q3_launch_status();
 }
 
