@@ -918,19 +918,21 @@ struct DecodeShared {
   __attribute__((aligned(16))) float acc[DECODE_WAVES][16][DV + 4];
 };
 
-// A block's work: split `split` of sequence `b`'s keys for key head `g_kv`.
-template <int D, bool PREP, typename W, bool AHEAD, int DV>
+// A block's work: split `split` of sequence `b`'s keys for key head `g_kv`. With CHUNK the rows are `tokens` tokens of the sequence, from
+// its number `first_token` of this step on (at most 16 rows), which see the keys up to the last of them.
+template <int D, bool PREP, typename W, bool AHEAD, int DV, bool CHUNK = false>
 __device__ __forceinline__ void decode_block(
     DecodeShared<D, PREP, DV>& shared, const int split, const int g_kv, const int b, const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, const bf16_t* __restrict__ k_cache,
     const bf16_t* __restrict__ v_cache, int num_pages, const int* __restrict__ block_table, int bt_stride,
     const int* __restrict__ cu_q, const int* __restrict__ kv_lens, int Hq, int Hkv, int page, score_scale_t scale_log2,
     span_t window, int splits, float* __restrict__ ws_acc, float* __restrict__ ws_ml, DecodePrep prep,
-    const float* __restrict__ sink Q3_BIAS_PARAM Q3_RUNS_PARAM Q3_GATE_PARAM) {
+    const float* __restrict__ sink Q3_BIAS_PARAM Q3_RUNS_PARAM Q3_GATE_PARAM, const int first_token = 0, const int tokens = 0) {
   constexpr int WAVES = DECODE_WAVES;
   const int G = Hq / Hkv;
   // a step of single tokens (PREP): sequence b's token is row b, and nothing is read to know it
-  const int q0 = PREP ? b : cu_q[b];
-  const int q_len = PREP ? 1 : cu_q[b + 1] - q0;
+  const int q_begin = PREP ? b : cu_q[b], q_all = PREP ? 1 : cu_q[b + 1] - q_begin;
+  const int q0 = CHUNK ? q_begin + first_token : q_begin;
+  const int q_len = CHUNK ? min(tokens, q_all - first_token) : q_all;
   if (q_len <= 0 || q_len * G > 16) return;  // the other kernel's sequence
   const int* bt_row = block_table + (size_t)b * bt_stride;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -938,7 +940,7 @@ __device__ __forceinline__ void decode_block(
   const int rows = q_len * G;
   // Without a window (AHEAD: the host launches this form then) a wavefront's tiles are first, first + step, ...
   // of the whole sequence, known before its length is: the table entries are asked for beside the length.
-  const int kv_len = kv_lens[b];
+  const int kv_len = CHUNK ? kv_lens[b] - (q_all - first_token - q_len) : kv_lens[b];
   const int ahead_first = split * WAVES + wave, ahead_step = WAVES * splits;
   TilePages p_first{}, p_second{};
   if constexpr (AHEAD) {
@@ -2009,13 +2011,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 }
 
 #if !defined(Q3_POOLED) && !defined(Q3_SIGMOID) && !defined(Q3_SPAN)
-// Row tile number `n` among those of all sequences of many rows, in their order: its sequence, and its number there in `n`; -1
-// behind the last. All lanes of a wavefront together.
+// Row tile number `n` among those of all sequences (MANY: of those of many rows alone), in their order: its sequence, and its
+// number there in `n`; -1 behind the last. All lanes of a wavefront together.
+template <bool MANY>
 __device__ __forceinline__ int sequence_of_tile(int& n, const int* __restrict__ cu_q, int sequences, int G, int tokens_per_block) {
   const int lane = threadIdx.x & 63;
   for (int first = 0; first < sequences; first += 64) {
     const int b = first + lane, rows = b < sequences ? cu_q[b + 1] - cu_q[b] : 0;
-    const int tiles = rows * G > 16 ? (rows + tokens_per_block - 1) / tokens_per_block : 0;
+    const int tiles = !MANY || rows * G > 16 ? (rows + tokens_per_block - 1) / tokens_per_block : 0;
     int upto = tiles;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
@@ -2031,6 +2034,31 @@ __device__ __forceinline__ int sequence_of_tile(int& n, const int* __restrict__ 
     n -= __shfl(upto, 63, 64);
   }
   return -1;
+}
+
+// A step of few rows in all: 16 of them a block, whatever sequence they are of, as the decoding kernel treats its 16. The prompt
+// kernel's 32 to 128 rows a block walk tiles of 64 keys one after the other through shared memory; here four wavefronts share the keys in
+// tiles of 32, straight from the L2, which every block asks for them anew: the way as long as a CU has two such blocks at most
+// (SHORT_BLOCKS, a little less for the tiles that do not come). Microseconds, prompt kernel / this, 16 and 32 heads over 8 of 128: three
+// prompts of 33, 67 and 101 tokens 10.9 / 7.0 and 11.0 / 9.6; one of 200 11.6 / 8.1 and 13.2 / 10.4; 64 rows over 512 keys 17.7 / 10.4
+// and 17.8 / 10.4; 32 over 1,000 30 / 15; 400 over 400 (400 and 800 blocks) 17.6 / 13.2 and 18.1 / 20.9; four prompts of 128
+// (512 and 1,024) 9.7 / 10.3 and 10.2 / 18.4.
+#define SHORT_BLOCKS 448
+template <int D>
+__global__ __launch_bounds__(64 * DECODE_WAVES) Q3_DECODE_WAVES void attn_short_kernel(
+    const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, const bf16_t* __restrict__ k_cache,
+    const bf16_t* __restrict__ v_cache, int num_pages, const int* __restrict__ block_table, int bt_stride,
+    const int* __restrict__ cu_q, const int* __restrict__ kv_lens, int sequences, int Hq, int Hkv, int page,
+    score_scale_t scale_log2, const float* __restrict__ sink) {
+  __shared__ DecodeShared<D, false, D> shared;
+  const int G = Hq / Hkv, tokens = 16 / G;
+  int tile = blockIdx.y;
+  const int b = __builtin_amdgcn_readfirstlane(sequence_of_tile<false>(tile, cu_q, sequences, G, tokens));
+  if (b < 0) return;
+  tile = __builtin_amdgcn_readfirstlane(tile);
+  decode_block<D, false, float, true, D, true>(shared, 0, blockIdx.x, b, q, q_stride, out, k_cache, v_cache, num_pages,
+                                               block_table, bt_stride, cu_q, kv_lens, Hq, Hkv, page, scale_log2, 0, 1, nullptr,
+                                               nullptr, DecodePrep{}, sink, tile * tokens, tokens);
 }
 
 // Both kinds of sequences of a step without a window in one launch: `prompt_blocks` blocks for the prompts (Hkv per key share
@@ -2058,7 +2086,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   if (first == (prompts_first != 0)) {
     const int share = id / Hkv;
     int tile = share / key_splits;
-    const int b = __builtin_amdgcn_readfirstlane(sequence_of_tile(tile, cu_q, sequences, Hq / Hkv, tokens_per_block));
+    const int b = __builtin_amdgcn_readfirstlane(sequence_of_tile<true>(tile, cu_q, sequences, Hq / Hkv, tokens_per_block));
     if (b < 0) return;
     tile = __builtin_amdgcn_readfirstlane(tile);
     prefill_block<D, TILE, STAGES, D>(shared.prompt, id % Hkv, tile * key_splits + share % key_splits, b, q, q_stride, out,
@@ -2169,6 +2197,16 @@ static int launch_fast(const void* q, int q_stride, void* out, const void* k_cac
   if (many && tiles * key_splits > 65535) return Q3_ERR_UNSUPPORTED;
   float* part_acc = prompt_ws;
   float* part_ml = prompt_ws ? prompt_ws + (size_t)total_tokens * Hq * key_splits * DV : nullptr;
+#if !defined(Q3_POOLED) && !defined(Q3_SIGMOID) && !defined(Q3_SPAN)
+  const int chunk_tokens = 16 / G;
+  const long short_tiles = max(0, total_tokens - B) / chunk_tokens + B;   // (the most that so many tokens of so many sequences come to)
+  if (many && window == 0 && splits == 1 && key_splits == 1 && short_tiles * Hkv <= SHORT_BLOCKS) {
+    hipLaunchKernelGGL(attn_short_kernel<D>, dim3(Hkv, (unsigned)short_tiles), dim3(256), 0, stream, (const bf16_t*)q, q_stride,
+                       (bf16_t*)out, (const bf16_t*)k_cache, (const bf16_t*)v_cache, num_pages, block_table, bt_stride, cu_q,
+                       kv_lens, B, Hq, Hkv, page, scale_log2, sink);
+    return q3_launch_status();
+  }
+#endif
   bool together = false;
 #if !defined(Q3_POOLED) && !defined(Q3_SIGMOID) && !defined(Q3_SPAN)
   // row tiles of the sequences of many rows: one each beyond whole ones, and as many sequences as there are rows for

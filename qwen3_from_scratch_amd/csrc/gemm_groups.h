@@ -59,7 +59,7 @@ struct Shape {
   static constexpr int SMEM_BYTES = AREA + ROW_NUMBERS * BM * 4;
   static constexpr int RESIDENT = SMEM_BYTES <= 80 * 1024 && ALL <= 1024 ? 2 : 1;
   static_assert(BM * 8 % THREADS == 0 && BN * 8 % THREADS == 0, "whole turns");
-  static_assert(ALL % BM == 0 && ALL <= 1024, "threads");
+  static_assert(ALL % BM == 0 && ALL <= 1024 && THREADS % 128 == 0, "threads (16 rows a turn or more: the places of the copies)");
   static_assert(STAGES >= 2 && STAGES <= 5 && (STAGES - 2) * LOADS < 64, "the wait counts");
 };
 
