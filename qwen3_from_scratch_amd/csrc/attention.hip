@@ -2254,7 +2254,7 @@ template <int D, typename W>
 static int launch_decode_prep(const void* qkv, void* out, const void* k_cache, const void* v_cache, int num_pages,
                               const int* block_table, int bt_stride, const int* cu_q, const int* kv_lens, int B,
                               int Hq, int Hkv, int page, float scale, int window, int splits, float* ws_acc,
-                              float* ws_ml, const DecodePrep& prep, hipStream_t stream) {
+                              float* ws_ml, const DecodePrep& prep, bool merge, hipStream_t stream) {
   const score_scale_t scale_log2 = make_score_scale(scale);
   if (window == 0)
     hipLaunchKernelGGL((attn_decode_kernel<D, true, W, true>), dim3(splits, Hkv, B), dim3(256), 0, stream,
@@ -2266,7 +2266,7 @@ static int launch_decode_prep(const void* qkv, void* out, const void* k_cache, c
                        (const bf16_t*)qkv, (Hq + 2 * Hkv) * D, (bf16_t*)out, (const bf16_t*)k_cache,
                        (const bf16_t*)v_cache, num_pages, block_table, bt_stride, cu_q, kv_lens, Hq, Hkv, page,
                        scale_log2, window, splits, ws_acc, ws_ml, prep, (const float*)nullptr);
-  if (splits > 1)
+  if (splits > 1 && merge)
     hipLaunchKernelGGL(attn_decode_reduce_kernel<D>, dim3(Hkv, B), dim3(256), 0, stream, (bf16_t*)out,
                        (const int*)nullptr, Hq, Hkv, splits, ws_acc, ws_ml, (const float*)nullptr);
   return q3_launch_status();
@@ -2402,13 +2402,14 @@ extern "C" int q3_decode_attention_takes(int Hq, int Hkv, int D, int page, int d
 // key and value written to the caches at position kv_lens[b] - 1 (if `store`), and attention
 // over the cache, in one kernel and, with more than one split, the merge of its partial
 // results (workspace as for q3_paged_attention). out (B, Hq D) bfloat16. `max_kv_len`: a bound
-// on kv_lens that the host knows; a step that would pass the rotation table's end is refused.
+// on kv_lens that the host knows; a step that would pass the rotation table's end is refused. Without `merge` the splits' partial
+// results are left in the workspace for a product that reads them so (q3_linear_of_splits), and `out` is not written.
 extern "C" int q3_decode_attention(const void* qkv, void* out, void* k_cache, void* v_cache, int num_pages,
                                    const int* block_table, int bt_stride, const int* cu_q, const int* kv_lens,
                                    int B, int Hq, int Hkv, int D, int page, float scale, int window, int splits,
                                    float* workspace, const void* q_weight, const void* k_weight, int w_dtype,
                                    float eps, const float* table, int rotary_dim, int max_pos, int store,
-                                   int max_kv_len, hipStream_t stream) {
+                                   int max_kv_len, int merge, hipStream_t stream) {
   if (table && max_kv_len > max_pos) return Q3_ERR_BAD_ARGUMENT;
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv || page <= 0) return Q3_ERR_BAD_ARGUMENT;
   if (B > 65535) return Q3_ERR_UNSUPPORTED;
@@ -2429,7 +2430,7 @@ extern "C" int q3_decode_attention(const void* qkv, void* out, void* k_cache, vo
   prep.v_cache = store ? (bf16_t*)v_cache : nullptr;
 #define Q3_DECODE_PREP(DD, WW)                                                                                    \
   return launch_decode_prep<DD, WW>(qkv, out, k_cache, v_cache, num_pages, block_table, bt_stride, cu_q, kv_lens, \
-                                    B, Hq, Hkv, page, scale, window, splits, ws_acc, ws_ml, prep, stream)
+                                    B, Hq, Hkv, page, scale, window, splits, ws_acc, ws_ml, prep, merge != 0, stream)
   if (D == 64) {
     if (w_dtype == Q3_F32) Q3_DECODE_PREP(64, float);
     Q3_DECODE_PREP(64, bf16_t);

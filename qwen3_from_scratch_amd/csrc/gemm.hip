@@ -292,6 +292,41 @@ struct SkinnyFusion {
   int sums_stride;   // floats between two partial sums of a row, in row_sums and in sums_out: 16 or more, in steps of 4
 };
 
+// The residual of four outputs and the next norm's weights of their columns, and the addition: see EPI_RESIDUAL. Returns
+// the new residual's sum of squares.
+__device__ inline void load_residual(const SkinnyFusion& fu, size_t at, int n, float4& res, float4& nw) {
+  res = *reinterpret_cast<const float4*>(fu.residual + at);
+  if (fu.norm_weight_f32) {
+    nw = *reinterpret_cast<const float4*>(static_cast<const float*>(fu.norm_weight) + n);
+  } else {
+    union {
+      uint2 u;
+      bf16_t e[4];
+    } pk;
+    pk.u = *reinterpret_cast<const uint2*>(static_cast<const bf16_t*>(fu.norm_weight) + n);
+    nw = make_float4(bf16_to_float(pk.e[0]), bf16_to_float(pk.e[1]), bf16_to_float(pk.e[2]), bf16_to_float(pk.e[3]));
+  }
+}
+__device__ inline float add_to_residual(const SkinnyFusion& fu, size_t at, const f32x4_t& acc, const float4& res,
+                                        const float4& nw, bf16_t* values) {
+  const float xn[4] = {res.x + bf16_to_float(float_to_bf16(acc[0])), res.y + bf16_to_float(float_to_bf16(acc[1])),
+                       res.z + bf16_to_float(float_to_bf16(acc[2])), res.w + bf16_to_float(float_to_bf16(acc[3]))};
+  *reinterpret_cast<float4*>(fu.residual + at) = make_float4(xn[0], xn[1], xn[2], xn[3]);
+  const float wn[4] = {nw.x, nw.y, nw.z, nw.w};
+  union {
+    uint2 u;
+    bf16_t e[4];
+  } pk;
+  float ss = 0.f;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    ss += xn[j] * xn[j];
+    pk.e[j] = float_to_bf16(xn[j] * wn[j]);
+  }
+  *reinterpret_cast<uint2*>(values + at) = pk.u;
+  return ss;
+}
+
 #ifndef SKINNY_PAIR_SLABS
 #define SKINNY_PAIR_SLABS 384   // from this many slabs on, and with more than eight rows of x, two slabs share a block
 #endif
@@ -347,19 +382,7 @@ __global__ __launch_bounds__(1024) void gemm_skinny_kernel(const bf16_t* __restr
   const int n = n0 + 4 * grp;
   float4 res = make_float4(0.f, 0.f, 0.f, 0.f), nw = res;
   const bool owner = EPI == EPI_RESIDUAL && ksplit == 0 && col < M && n + 3 < N;
-  if (EPI == EPI_RESIDUAL && owner) {
-    res = *reinterpret_cast<const float4*>(fu.residual + (size_t)col * N + n);
-    if (fu.norm_weight_f32) {
-      nw = *reinterpret_cast<const float4*>(static_cast<const float*>(fu.norm_weight) + n);
-    } else {
-      union {
-        uint2 u;
-        bf16_t e[4];
-      } pk;
-      pk.u = *reinterpret_cast<const uint2*>(static_cast<const bf16_t*>(fu.norm_weight) + n);
-      nw = make_float4(bf16_to_float(pk.e[0]), bf16_to_float(pk.e[1]), bf16_to_float(pk.e[2]), bf16_to_float(pk.e[3]));
-    }
-  }
+  if (EPI == EPI_RESIDUAL && owner) load_residual(fu, (size_t)col * N + n, n, res, nw);
 
   const bool row_ok = TILED ? n0 < N : n0 + col < N;
   const bool x_ok = col < M;
@@ -420,23 +443,7 @@ __global__ __launch_bounds__(1024) void gemm_skinny_kernel(const bf16_t* __restr
   }
   if constexpr (EPI == EPI_RESIDUAL) {
     // N is a multiple of 16 here: a slab is whole or absent
-    float ss = 0.f;
-    if (owner) {
-      const float xn[4] = {res.x + bf16_to_float(float_to_bf16(acc[0])), res.y + bf16_to_float(float_to_bf16(acc[1])),
-                           res.z + bf16_to_float(float_to_bf16(acc[2])), res.w + bf16_to_float(float_to_bf16(acc[3]))};
-      *reinterpret_cast<float4*>(fu.residual + (size_t)col * N + n) = make_float4(xn[0], xn[1], xn[2], xn[3]);
-      const float wn[4] = {nw.x, nw.y, nw.z, nw.w};
-      union {
-        uint2 u;
-        bf16_t e[4];
-      } pk;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        ss += xn[j] * xn[j];
-        pk.e[j] = float_to_bf16(xn[j] * wn[j]);
-      }
-      *reinterpret_cast<uint2*>(reinterpret_cast<bf16_t*>(out) + (size_t)col * N + n) = pk.u;
-    }
+    float ss = owner ? add_to_residual(fu, (size_t)col * N + n, acc, res, nw, reinterpret_cast<bf16_t*>(out)) : 0.f;
     ss += __shfl_xor(ss, 16, 64);
     ss += __shfl_xor(ss, 32, 64);
     if constexpr (GROUPS) {
@@ -477,6 +484,138 @@ __global__ __launch_bounds__(1024) void gemm_skinny_kernel(const bf16_t* __restr
     for (int j = 0; j < 4; ++j)
       if (n + j < N) o[j] = from_float<OUT>(acc[j]);
   }
+}
+
+// The product with the residual addition, its rows the results of decoding attention whose keys several blocks shared out: the
+// merge of their partial results (attn_decode_reduce_kernel) in the product's first lines, in the place of a launch of its own, which is
+// a chain of latencies beside which the weights could be on their way already. A wavefront forms the rows of x of its own
+// share of K, 256 numbers at a time (four a lane; the partial results of one split after the other, each weighted by its
+// maximum), leaves them in shared memory and reads its operands there: no other wavefront is waited for. All that its
+// first numbers need is asked for at once, the partial results first, then the weights of two turns; later partial results
+// while the ones before them are added. Every block reads all partial results, out of the L2, so only short ones come here
+// (SPLITS_MOST_BYTES). Attention and product of one layer, keys and weights from memory, microseconds, with a merge launched between
+// / so: a request of 16 heads of 128 over 1,100 keys (16 parts) and a product of 1,024 15.2 / 13.5, over 3,000 16.8 / 15.2.
+#define MERGE_SPLITS 16
+#define MERGE_BATCH 8
+struct SplitResults {
+  const float *acc, *ml;   // (rows, key heads, splits, 16, D) and pairs (maximum, sum): q3_decode_attention's workspace
+  int splits, heads, kv_heads;
+};
+
+template <int D>
+__global__ __launch_bounds__(512) void gemm_skinny_splits_kernel(SplitResults parts, const bf16_t* __restrict__ w,
+                                                                 bf16_t* __restrict__ out, int M, int N, int K, int k_per_wave,
+                                                                 SkinnyFusion fu) {
+  extern __shared__ float red[];  // [waves][64][4], then the wavefronts' rows of x
+  constexpr int LANES = D / 4;    // of a head
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = blockDim.x >> 6;
+  const int col = lane & 15, grp = lane >> 4;
+  const int slab = blockIdx.x, n = slab * 16 + 4 * grp;
+  const int k_begin = wave * k_per_wave, k_end = min(K, k_begin + k_per_wave);
+  const int stride = k_per_wave + 8;   // of a row of x in shared memory: sixteen bytes more spread the rows over the banks
+  bf16_t* xs = reinterpret_cast<bf16_t*>(red + nwaves * 256) + (size_t)wave * M * stride;
+  const int G = parts.heads / parts.kv_heads, S = parts.splits;
+  const bool owner = wave == 0 && col < M;
+  float4 res = make_float4(0.f, 0.f, 0.f, 0.f), nw = res;
+
+  // a row's 256 numbers are formed in steps of MERGE_BATCH splits (past the last: that one again, of weight zero)
+  const int steps = (S + MERGE_BATCH - 1) / MERGE_BATCH, items = (k_end - k_begin) / 256 * M * steps;
+  struct Part {
+    float2 ml;
+    float4 v[MERGE_BATCH];
+  };
+  auto load = [&](int i, Part& p) {
+    const int row = i / steps, first = (i - row * steps) * MERGE_BATCH, run = row / M, m = row - run * M;
+    const int head = (k_begin + run * 256) / D + lane / LANES, r = head % G, s = lane % LANES;
+    const size_t base = ((size_t)m * parts.kv_heads + head / G) * S;
+    const float* acc = parts.acc + (base * 16 + r) * D + 4 * s;
+    p.ml = *reinterpret_cast<const float2*>(parts.ml + ((base + min(s, S - 1)) * 16 + r) * 2);
+#pragma unroll
+    for (int k = 0; k < MERGE_BATCH; ++k) p.v[k] = *reinterpret_cast<const float4*>(acc + (size_t)min(first + k, S - 1) * 16 * D);
+  };
+  float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+  auto merge = [&](int i, const Part& p) {
+    const int row = i / steps, step = i - row * steps, run = row / M, m = row - run * M;
+    float top = p.ml.x;
+#pragma unroll
+    for (int off = LANES / 2; off > 0; off >>= 1) top = fmaxf(top, __shfl_xor(top, off, 64));
+    const float weight = p.ml.x > -INFINITY && lane % LANES < S ? exp2f(p.ml.x - top) : 0.f;
+#pragma unroll
+    for (int k = 0; k < MERGE_BATCH; ++k) {
+      const float of = __shfl(weight, (lane & ~(LANES - 1)) + step * MERGE_BATCH + k, 64);
+      sum.x = fmaf(of, p.v[k].x, sum.x); sum.y = fmaf(of, p.v[k].y, sum.y);
+      sum.z = fmaf(of, p.v[k].z, sum.z); sum.w = fmaf(of, p.v[k].w, sum.w);
+    }
+    if (step < steps - 1) return;
+    float total = weight * p.ml.y;
+#pragma unroll
+    for (int off = LANES / 2; off > 0; off >>= 1) total += __shfl_xor(total, off, 64);
+    const float inv = total > 0.f ? 1.f / total : 0.f;    // (no key at all: zeros, as the merge gives)
+    union {
+      uint2 u;
+      bf16_t e[4];
+    } pk;
+    pk.e[0] = float_to_bf16(sum.x * inv); pk.e[1] = float_to_bf16(sum.y * inv);
+    pk.e[2] = float_to_bf16(sum.z * inv); pk.e[3] = float_to_bf16(sum.w * inv);
+    *reinterpret_cast<uint2*>(xs + (size_t)m * stride + run * 256 + 4 * lane) = pk.u;
+    sum = make_float4(0.f, 0.f, 0.f, 0.f);
+  };
+  const bf16_t* wp = w + (size_t)slab * (K / 32) * 512 + lane * 8;
+  auto load_weights = [&](Pack16 (&a)[SKINNY_U], int k) {
+#pragma unroll
+    for (int u = 0; u < SKINNY_U; ++u) a[u].u = *reinterpret_cast<const uint4*>(wp + (size_t)((k + 32 * u) / 32) * 512);
+  };
+  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+  if (items > 0) {
+    Part p0, p1;
+    Pack16 a0[SKINNY_U], a1[SKINNY_U];
+    load(0, p0);
+    if (items > 1) load(1, p1);
+    load_weights(a0, k_begin);
+    if (k_begin + 32 * SKINNY_U < k_end) load_weights(a1, k_begin + 32 * SKINNY_U);
+    if (owner) load_residual(fu, (size_t)col * N + n, n, res, nw);
+    __builtin_amdgcn_sched_barrier(0);
+    for (int i = 0; i < items; i += 2) {
+      merge(i, p0);
+      if (i + 2 < items) load(i + 2, p0);
+      if (i + 1 < items) {
+        merge(i + 1, p1);
+        if (i + 3 < items) load(i + 3, p1);
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    auto multiply = [&](const Pack16 (&a)[SKINNY_U], int k) {
+#pragma unroll
+      for (int u = 0; u < SKINNY_U; ++u) {
+        Pack16 b;
+        b.u = col < M ? *reinterpret_cast<const uint4*>(xs + (size_t)col * stride + (k - k_begin) + 32 * u + 8 * grp)
+                      : make_uint4(0, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u].v, b.v, acc, 0, 0, 0);
+      }
+    };
+    constexpr int TURN = 32 * SKINNY_U;
+    for (int k = k_begin; k < k_end; k += 2 * TURN) {
+      multiply(a0, k);
+      if (k + 2 * TURN < k_end) load_weights(a0, k + 2 * TURN);
+      if (k + TURN < k_end) {
+        multiply(a1, k + TURN);
+        if (k + 3 * TURN < k_end) load_weights(a1, k + 3 * TURN);
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) red[(wave * 64 + lane) * 4 + j] = acc[j];
+  __syncthreads();
+  if (wave != 0) return;
+  for (int s = 1; s < nwaves; ++s)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[j] += red[(s * 64 + lane) * 4 + j];
+  float ss = owner ? add_to_residual(fu, (size_t)col * N + n, acc, res, nw, out) : 0.f;
+  ss += __shfl_xor(ss, 16, 64);
+  ss += __shfl_xor(ss, 32, 64);
+  if (grp == 0) fu.sums_out[slab * 16 + col] = ss;
 }
 
 // Two slabs per block from the tile-ordered copy: a wavefront's rows of x (the second operand)
@@ -710,6 +849,56 @@ __global__ __launch_bounds__(256) void gemm_f32_few_rows_kernel(const float* __r
       const float total = wave_sum(acc[j][m]);
       if (lane == 0 && m < M && n0 + j < N) out[(size_t)m * N + n0 + j] = total;
     }
+}
+
+// The product with the residual addition (q3_linear_tiled's epilogue 2) of rows that decoding attention has left in `splits` partial
+// results each: `workspace` as q3_decode_attention leaves it, `heads` query heads over `kv_heads` of `dim` (64 or 128). K = heads dim, a
+// multiple of 256; N of 16; M <= 16; at most 16 splits. q3_linear_of_splits_most: into how many splits attention that would be cut into `splits`
+// is best cut for it, or 0 where the sizes are not its or the partial results so many that reading them in every block costs more
+// than the merge's launch: attention and product, microseconds, merged before / inside, 128 KB of partial results 15.2 / 13.5 (K = 2,048, 1 row),
+// 16.2 / 14.6 (2 rows of 8 parts), 22.9 / 22.1 (K = 4,096, 8 parts); 192 KB 15.4 / 15.6 and 22.3 / 23.2; 256 KB 15.3 / 15.8 and 21.3 / 22.5.
+// Thirty-two parts (from 4,096 keys on) become sixteen: a request over 4,200 keys 18.7 merged before, 17.3 so, over 6,000 19.7 and 18.6, over
+// 8,100 20.6 and 20.7, over 30,000 35.7 and 38.4 (the caller's line is at 8,192).
+#define SPLITS_MOST_BYTES (128 << 10)
+extern "C" int q3_linear_of_splits_most(int M, int N, int heads, int kv_heads, int dim, int splits) {
+  const int K = heads * dim;
+  if (splits > MERGE_SPLITS) splits = MERGE_SPLITS;
+  const bool takes = M >= 1 && M <= 16 && N > 0 && N % 16 == 0 && kv_heads > 0 && heads > 0 && heads % kv_heads == 0 &&
+                     heads / kv_heads <= 16 && (dim == 64 || dim == 128) && K % 256 == 0 && K <= 8 * 1024 && splits >= 2 &&
+                     (long)M * K * splits * 4 <= SPLITS_MOST_BYTES;
+  return takes ? splits : 0;
+}
+
+extern "C" int q3_linear_of_splits(const float* workspace, int splits, int heads, int kv_heads, int dim, const void* weight_tiled,
+                                   void* out, int M, int N, float* residual, const void* norm_weight, int norm_w_dtype,
+                                   float* sums_out, hipStream_t stream) {
+  if (!workspace || !weight_tiled || !out || !residual || !norm_weight || !sums_out ||
+      (norm_w_dtype != Q3_F32 && norm_w_dtype != Q3_BF16) ||
+      q3_linear_of_splits_most(M, N, heads, kv_heads, dim, splits) != splits)
+    return Q3_ERR_BAD_ARGUMENT;
+  const int K = heads * dim;
+  SkinnyFusion fu{};
+  fu.residual = residual;
+  fu.norm_weight = norm_weight;
+  fu.norm_weight_f32 = norm_w_dtype == Q3_F32;
+  fu.sums_out = sums_out;
+  SplitResults parts{workspace, workspace + (size_t)M * kv_heads * splits * 16 * dim, splits, heads, kv_heads};
+  const int waves = min(8, K / 256), k_per_wave = (K / 256 + waves - 1) / waves * 256;
+  const size_t smem = (size_t)waves * (1024 + (size_t)M * (k_per_wave + 8) * 2);
+  auto kernel = dim == 64 ? gemm_skinny_splits_kernel<64> : gemm_skinny_splits_kernel<128>;
+  if (smem > 65536) {
+    static std::atomic<bool> raised[2][16];   // the dynamic shared-memory limit, once per device
+    int device = 0;
+    if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 16) return Q3_ERR_BAD_ARGUMENT;
+    if (!raised[dim == 128][device]) {
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+      if (e != hipSuccess) return (int)e;
+      raised[dim == 128][device] = true;
+    }
+  }
+  hipLaunchKernelGGL(kernel, dim3(N / 16), dim3(64 * waves), smem, stream, parts, (const bf16_t*)weight_tiled, (bf16_t*)out, M,
+                     N, K, k_per_wave, fu);
+  return q3_launch_status();
 }
 
 // Whether the weight-streaming kernel takes this product.

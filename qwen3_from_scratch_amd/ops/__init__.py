@@ -13,6 +13,7 @@ statistics and logits are float32 in both modes.
 import ctypes
 import json
 import os
+from typing import NamedTuple
 
 import torch
 
@@ -1759,12 +1760,14 @@ def decode_attention_takes(num_q_heads, num_kv_heads, head_dim, page_size, dtype
 
 def decode_attention(qkv, num_q_heads, num_kv_heads, head_dim, k_cache, v_cache, block_table, cu_seqlens_q,
                      kv_lens, max_kv_len, scale, window=0, q_weight=None, k_weight=None, eps=0.0, table=None,
-                     store=True):
+                     store=True, residual_width=0):
     """`qk_norm_rope_store` and `paged_attention` of a step in which every sequence brings one
     token, in one kernel: qkv (B, (Hq + 2 Hkv) D) bfloat16 holds the raw projections of
     sequence b's token in row b; the new key and value go to position kv_lens[b] - 1 of the
     caches (unless `store` is false: a layer that reads another layer's cache) and the
-    attention output (B, Hq D) is returned. qkv is left as it was."""
+    attention output (B, Hq D) is returned. qkv is left as it was. With `residual_width` the
+    output is for `linear_residual_norm` with a weight of so many rows, and where that takes it unmerged,
+    the parts that several blocks made of a sequence are returned (SplitRows)."""
     _dev(qkv, k_cache, v_cache, block_table, cu_seqlens_q, kv_lens, q_weight, k_weight, table)
     Hq, Hkv, D = num_q_heads, num_kv_heads, head_dim
     B = kv_lens.shape[0]
@@ -1800,10 +1803,15 @@ def decode_attention(qkv, num_q_heads, num_kv_heads, head_dim, k_cache, v_cache,
                                % (max_kv_len - 1, max_pos - 1))
     if not decode_attention_takes(Hq, Hkv, D, page, qkv.dtype, rotary_dim):
         raise OperandError("sizes the decoding kernel does not take")
-    out = torch.empty((B, Hq * D), dtype=qkv.dtype, device=qkv.device)
+    splits, merge, out = _splits(B, Hkv, max_kv_len) if B else 1, True, None
+    if residual_width and splits > 1 and max_kv_len <= 8192:
+        # (sixteen parts at most come unmerged; over more keys thirty-two and their merge are faster)
+        most = library("gemm").q3_linear_of_splits_most(B, residual_width, Hq, Hkv, D, splits)
+        splits, merge = most or splits, not most
+    if merge:
+        out = torch.empty((B, Hq * D), dtype=qkv.dtype, device=qkv.device)
     if B:
-        lib = library("attention")
-        splits, workspace = _splits(B, Hkv, max_kv_len), None
+        lib, workspace = library("attention"), None
         if splits > 1:
             lib.q3_paged_attention_workspace.restype = ctypes.c_long
             workspace = torch.empty((lib.q3_paged_attention_workspace(B, Hkv, D, splits),), dtype=torch.float32,
@@ -1814,9 +1822,20 @@ def decode_attention(qkv, num_q_heads, num_kv_heads, head_dim, k_cache, v_cache,
             _ptr(qkv), _ptr(out), _ptr(k_cache), _ptr(v_cache), pages, _ptr(block_table),
             block_table.shape[1], _ptr(cu_seqlens_q), _ptr(kv_lens), B, Hq, Hkv, D, page, ctypes.c_float(scale),
             int(window), splits, _ptr(workspace), _ptr(q_weight), _ptr(k_weight), w_dtype, ctypes.c_float(eps),
-            _ptr(table), int(rotary_dim), int(max_pos), 1 if store and pages else 0, int(max_kv_len), _stream()),
-            "decode_attention")
-    return out
+            _ptr(table), int(rotary_dim), int(max_pos), 1 if store and pages else 0, int(max_kv_len), 1 if merge else 0,
+            _stream()), "decode_attention")
+    return out if merge else SplitRows(workspace, splits, B, Hq, Hkv, D)
+
+
+class SplitRows(NamedTuple):
+    """Rows (B, Hq D) of decoding attention as the blocks left them that shared out their keys: see `decode_attention`."""
+
+    workspace: torch.Tensor
+    splits: int
+    rows: int
+    heads: int
+    kv_heads: int
+    dim: int
 
 
 def tile_weight(weight):
@@ -2167,7 +2186,11 @@ def linear_residual_norm(x, weight, tiled, residual, norm_weight):
     a block (a small weight; P = N over its tiles' columns, 16 to 128), or the tiled kernel's partial products are added
     by a second kernel that does the same (P = ceil(N / 1024)). There the result is None, and
     nothing was done, for a size at which the plain product (`linear`) followed by the norm's own
-    kernel is the faster way."""
+    kernel is the faster way.
+
+    x may be SplitRows, with the weight's tiled copy."""
+    if isinstance(x, SplitRows):
+        return _split_rows_residual_norm(x, weight, tiled, residual, norm_weight)
     _dev(x, weight, tiled, residual, norm_weight)
     if not (x.dim() == 2 and weight.dim() == 2 and x.shape[1] == weight.shape[1]):
         raise OperandError("x (M, K) and weight (N, K)")
@@ -2199,6 +2222,23 @@ def linear_residual_norm(x, weight, tiled, residual, norm_weight):
         _ptr(x), _ptr(tiled), _ptr(values), M, N, K, 1, 2, None, 0, ctypes.c_float(0.0), 0,
         _ptr(residual), _ptr(norm_weight), _DT[norm_weight.dtype], _ptr(sums), sums.shape[1], _stream()),
         "linear_residual_norm")
+    return values, sums
+
+
+def _split_rows_residual_norm(x, weight, tiled, residual, norm_weight):
+    _dev(x.workspace, weight, tiled, residual, norm_weight)
+    M, N = x.rows, weight.shape[0]
+    if not (weight.dim() == 2 and weight.shape[1] == x.heads * x.dim and _tiled_ok(tiled, weight, M)):
+        raise OperandError("a tiled weight (N, Hq D)")
+    if not (residual.shape == (M, N) and residual.dtype == torch.float32 and residual.is_contiguous()):
+        raise OperandError("residual must be float32 (M, N)")
+    if not (norm_weight.shape == (N,) and norm_weight.dtype in _DT and norm_weight.is_contiguous()):
+        raise OperandError("norm weight (N,)")
+    values = torch.empty((M, N), dtype=torch.bfloat16, device=weight.device)
+    sums = torch.empty((N // 16, 16), dtype=torch.float32, device=weight.device)
+    _check(library("gemm").q3_linear_of_splits(
+        _ptr(x.workspace), x.splits, x.heads, x.kv_heads, x.dim, _ptr(tiled), _ptr(values), M, N, _ptr(residual),
+        _ptr(norm_weight), _DT[norm_weight.dtype], _ptr(sums), _stream()), "linear_residual_norm")
     return values, sums
 
 

@@ -116,7 +116,8 @@ class PagedAttention(Part):
             o = ops.decode_attention(
                 qkv, Hq, Hkv, D, keys, values, cache.block_table, batch.cu_seqlens_q, batch.kv_lens,
                 batch.max_kv_len, self.scale, window=self.window, q_weight=self.q_weight, k_weight=self.k_weight,
-                eps=self.qk_norm_eps, table=table, store=cache.writes)
+                eps=self.qk_norm_eps, table=table, store=cache.writes,
+                residual_width=self.hidden_size if sink is not None and self.out.tiled is not None else 0)
             return self.out.forward(o) if sink is None else self.out.forward_into(o, sink)
         ops.qk_norm_rope_store(
             qkv, Hq, Hkv, D, batch.positions, batch.seq_index,

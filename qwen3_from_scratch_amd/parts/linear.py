@@ -68,7 +68,11 @@ class LinearWeight:
 
     def forward_into(self, x, sink):
         """x @ W^T added into the sink's residual and prepared for its norm, as
-        UnscaledRows; or, where the kernels do not take the case, returned."""
+        UnscaledRows; or, where the kernels do not take the case, returned. SplitRows
+        (see `ops.decode_attention`) are added in any case."""
+        if isinstance(x, ops.SplitRows):
+            return UnscaledRows(*ops.linear_residual_norm(x, self.weight, self.tiled, sink.residual, sink.weight),
+                                sink.eps, sink.width)
         rows = x.shape[0]
         if self.tiled is None or not (self.weight.shape[0] % 16 == 0 if rows <= ops.few_rows_limit(self.weight)
                                       else ops.fused_rows_take(self.weight, rows)):
