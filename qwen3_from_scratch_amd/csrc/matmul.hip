@@ -39,6 +39,7 @@
 #include "gemm_tiles.h"
 #include "gemm_stream.h"
 #include "gemm_groups.h"
+#include "gemm_rounds.h"
 
 #include <hipblaslt/hipblaslt.h>
 
@@ -60,9 +61,11 @@ constexpr int FUSED_ROWS_LIMIT = 640;         // rows of a product that carries 
 constexpr size_t GROUPS_MOST_WEIGHT_BYTES = 18u << 20;
 constexpr int EVICT_BLOCKS = 2048, EVICT_THREADS = 256;
 constexpr int MAX_CANDIDATES = 64;
+constexpr int MISALIGNED = 256;                // in a plan's key: operands that are not at multiples of 16 bytes
 constexpr int LIBRARY = -1;                    // a Choice's `own` when the library serves the size
 constexpr int GROUPS_FIRST = 16;               // a Choice's `own` from here on: gemm_groups.h's shapes (no table entry)
-static_assert(GROUPS_FIRST >= tiles::NUM_CONFIGS, "one numbering");
+constexpr int ROUNDS_FIRST = 32;               // and from here on: gemm_rounds.h's, plus the tile's height (no table entry)
+static_assert(GROUPS_FIRST >= tiles::NUM_CONFIGS && ROUNDS_FIRST >= GROUPS_FIRST + groups::NUM_SHAPES, "one numbering");
 
 // Reads the whole buffer; the store never happens (the buffer holds zeros) but keeps the loads alive.
 __global__ void evict_kernel(float4* buffer, size_t count) {
@@ -105,7 +108,7 @@ struct Device {
   float* partials = nullptr;
   float* staging = nullptr;   // a float32 product on its way to the kernel that divides its rows (q3_tiles_scaled)
   hipEvent_t begin = nullptr, end = nullptr;
-  std::map<std::tuple<int, int, int, int>, Plan> plans;   // by the exact size
+  std::map<std::tuple<int, int, int, int>, Plan> plans;   // by the exact size and the output type (plus MISALIGNED)
   std::map<Key, Choice> noted;                            // what the tuner found, by rounded rows
 };
 
@@ -212,6 +215,7 @@ int candidates_of(Device& d, const Plan& p, int want, std::vector<hipblasLtMatmu
 
 int run_own(Device& d, int config, int splits, const void* x, const void* w, void* out, int M, int N, int K,
             int out_dtype, hipStream_t stream) {
+  if (config >= ROUNDS_FIRST) return rounds::launch(config - ROUNDS_FIRST, x, w, out, M, N, K, stream);
   if (splits > 1 && (size_t)splits * M * N * sizeof(float) > PARTIALS_BYTES) return Q3_ERR_UNSUPPORTED;
   return out_dtype == Q3_F32
              ? tiles::launch<float, tiles::EPI_PLAIN>(config, x, w, out, M, N, K, stream, splits, d.partials)
@@ -304,9 +308,16 @@ Choice fused_by_rule(int kind, int M, int N, int K) {
   return c;
 }
 
-// What the table or the rule says for a size.
-Choice choice_for(int kind, int M, int N, int K, int out_dtype) {
+// What the table or the rule says for a size. A plain product that gemm_rounds.h covers in one round is its, whatever the table has
+// for the rows around it (the library's kernels); `aligned`: its operands lie at multiples of sixteen bytes, as its copies need.
+Choice choice_for(int kind, int M, int N, int K, int out_dtype, bool aligned = true) {
   if (g_kernels == KERNELS_BOTH) {
+    const int height = kind == KIND_PLAIN && out_dtype == Q3_BF16 && aligned ? rounds::height_for(M, N, K) : 0;
+    if (height) {
+      Choice c;
+      c.own = ROUNDS_FIRST + height;
+      return c;
+    }
     auto entry = g_table.find(Key(kind, rows_key(kind, M), N, K, out_dtype));
     if (entry != g_table.end()) {
       Choice c = entry->second;
@@ -459,7 +470,8 @@ int settle(Device& d, Plan& p, Choice c, int M, int N, int K) {
 int product(Device& d, const void* x, const void* w, void* out, int M, int N, int K, int out_dtype, hipStream_t stream) {
   int status = ready_device(d, stream);
   if (status) return status;
-  Plan& p = d.plans[std::make_tuple(M, N, K, out_dtype)];
+  const bool aligned = (((size_t)x | (size_t)w | (size_t)out) & 15) == 0;
+  Plan& p = d.plans[std::make_tuple(M, N, K, aligned ? out_dtype : out_dtype + MISALIGNED)];
   if (!p.desc) {
     status = describe(p, M, N, K, out_dtype);
     if (status) {
@@ -487,7 +499,7 @@ int product(Device& d, const void* x, const void* w, void* out, int M, int N, in
     }
   }
   if (!p.ready) {
-    status = settle(d, p, choice_for(KIND_PLAIN, M, N, K, out_dtype), M, N, K);
+    status = settle(d, p, choice_for(KIND_PLAIN, M, N, K, out_dtype, aligned), M, N, K);
     if (status) {
       forget(p);
       return status;

@@ -210,7 +210,8 @@ def matmul_kernels(which):
 def matmul_plan(M, N, K, out_dtype=torch.bfloat16):
     """What serves a plain product of this size on the current device, or None if it has not
     been met: (candidates timed (1 without the tuner), index chosen, microseconds of the first
-    candidate, of the chosen one, the hand-written kernel's tile shape if that serves it, else
+    candidate, of the chosen one, the hand-written kernel's tile shape if that serves it (from 32 on
+    the tile's height in units of 16 rows, of the kernel that covers a product in one round), else
     -1, over how many blocks it shares K out, the library's candidate number)."""
     info = (ctypes.c_float * 7)()
     if not _matmul().q3_matmul_plan(int(M), int(N), int(K), _DT[out_dtype], info):
