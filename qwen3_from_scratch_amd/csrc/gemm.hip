@@ -518,7 +518,8 @@ __global__ __launch_bounds__(512) void gemm_skinny_splits_kernel(SplitResults pa
   const bool owner = wave == 0 && col < M;
   float4 res = make_float4(0.f, 0.f, 0.f, 0.f), nw = res;
 
-  // a row's 256 numbers are formed in steps of MERGE_BATCH splits (past the last: that one again, of weight zero)
+  // a row's 256 numbers are formed in steps of MERGE_BATCH splits (past the last that one is read again, so that no load waits
+  // behind a branch, and not added: an infinity times a weight of zero would be a NaN)
   const int steps = (S + MERGE_BATCH - 1) / MERGE_BATCH, items = (k_end - k_begin) / 256 * M * steps;
   struct Part {
     float2 ml;
@@ -540,11 +541,18 @@ __global__ __launch_bounds__(512) void gemm_skinny_splits_kernel(SplitResults pa
 #pragma unroll
     for (int off = LANES / 2; off > 0; off >>= 1) top = fmaxf(top, __shfl_xor(top, off, 64));
     const float weight = p.ml.x > -INFINITY && lane % LANES < S ? exp2f(p.ml.x - top) : 0.f;
-#pragma unroll
-    for (int k = 0; k < MERGE_BATCH; ++k) {
+    auto add = [&](int k) {
       const float of = __shfl(weight, (lane & ~(LANES - 1)) + step * MERGE_BATCH + k, 64);
       sum.x = fmaf(of, p.v[k].x, sum.x); sum.y = fmaf(of, p.v[k].y, sum.y);
       sum.z = fmaf(of, p.v[k].z, sum.z); sum.w = fmaf(of, p.v[k].w, sum.w);
+    };
+    if ((step + 1) * MERGE_BATCH <= S) {
+#pragma unroll
+      for (int k = 0; k < MERGE_BATCH; ++k) add(k);
+    } else {
+#pragma unroll
+      for (int k = 0; k < MERGE_BATCH - 1; ++k)
+        if (step * MERGE_BATCH + k < S) add(k);
     }
     if (step < steps - 1) return;
     float total = weight * p.ml.y;

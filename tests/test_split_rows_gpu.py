@@ -65,3 +65,23 @@ def test_partial_results_too_many_to_read_in_every_block_are_merged_first(Hq, kv
     args = (Hq, Hkv, D, kc, vc, bt, cu, kvl, max(kv_lens), D ** -0.5)
     got = ops.decode_attention(qkv, *args, residual_width=4096)
     assert torch.equal(got, ops.decode_attention(qkv, *args))
+
+
+def test_an_infinite_value_stays_one():
+    """An infinity among the values of the last of ten parts, which are merged in steps of eight: as merged beforehand."""
+    ops = _ops()
+    B, Hq, Hkv, D, N, keys = 12, 2, 2, 128, 64, 2000
+    _, kc, vc, bt, cu, kvl = _paged_case(torch.bfloat16, B, Hq, Hkv, D, 16, [1] * B, [keys] * B, 28)
+    qkv, weight = _rand((B, (Hq + 2 * Hkv) * D), torch.bfloat16, 29), _rand((N, Hq * D), torch.bfloat16, 30, scale=0.05)
+    args = (Hq, Hkv, D, kc, vc, bt, cu, kvl, keys, D ** -0.5)
+    splits = ops.decode_attention(qkv, *args, residual_width=N).splits
+    assert splits == 10
+    key = 32 * 4 * (splits - 1)                # a wavefront's tiles of 32 keys: every (4 splits)-th, from this one on
+    vc[int(bt[3, key // 16]), 1, 5, key % 16] = float("inf")
+    norm, results = torch.ones(N, device="cuda"), []
+    for width in (N, 0):
+        rows, residual = ops.decode_attention(qkv, *args, residual_width=width), torch.zeros(B, N, device="cuda")
+        ops.linear_residual_norm(rows, weight, ops.tile_weight(weight), residual, norm)
+        results.append(residual)
+    assert bool(results[1][3].isinf().all()) and bool(results[1].isfinite()[torch.arange(B) != 3].all())
+    assert torch.equal(results[0][3], results[1][3]) and bool(results[0].isfinite()[torch.arange(B) != 3].all())
