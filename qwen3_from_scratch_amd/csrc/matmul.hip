@@ -14,7 +14,7 @@
 //      rounded up, N, K, output type);
 //   2. a rule of thumb: the library's first candidate for a plain product; for
 //      the products that carry a norm (17 to 128 rows, 640 of a small weight) the kernel that shares K out
-//      inside a block (gemm_groups.h) for a small weight, else 64 x 128
+//      inside a block (gemm_groups.hip) for a small weight, else 64 x 128
 //      tiles with K shared out until the chip is full, unless those tiles fit the chip badly.
 // The library's list is asked for the exact size every time, so a kernel is
 // never run on a size the library has not offered it for.
@@ -63,8 +63,8 @@ constexpr int EVICT_BLOCKS = 2048, EVICT_THREADS = 256;
 constexpr int MAX_CANDIDATES = 64;
 constexpr int MISALIGNED = 256;                // in a plan's key: operands that are not at multiples of 16 bytes
 constexpr int LIBRARY = -1;                    // a Choice's `own` when the library serves the size
-constexpr int GROUPS_FIRST = 16;               // a Choice's `own` from here on: gemm_groups.h's shapes (no table entry)
-constexpr int ROUNDS_FIRST = 32;               // and from here on: gemm_rounds.h's, plus the tile's height (no table entry)
+constexpr int GROUPS_FIRST = 16;               // a Choice's `own` from here on: gemm_groups.hip's shapes (no table entry)
+constexpr int ROUNDS_FIRST = 32;               // and from here on: gemm_rounds.hip's, plus the tile's height (no table entry)
 static_assert(GROUPS_FIRST >= tiles::NUM_CONFIGS && ROUNDS_FIRST >= GROUPS_FIRST + groups::NUM_SHAPES, "one numbering");
 
 // Reads the whole buffer; the store never happens (the buffer holds zeros) but keeps the loads alive.
@@ -257,7 +257,7 @@ Choice plain_by_rule(int M, int N, int K) {
 }
 
 // The products that carry a norm. A weight of up to 18 MB, or a product of more than 96 rows in 128 x 128 tiles: the kernel of
-// gemm_groups.h where it covers the product in one round. (A larger weight's few rows are bound by its passage, which many small tiles with
+// gemm_groups.hip where it covers the product in one round. (A larger weight's few rows are bound by its passage, which many small tiles with
 // their own rows of x beside it slow down: 24 and 64 rows of 6,144 x 4,096 16.6 and 20.8 us there, 15.9 and 17.8 in 64 x 128
 // tiles; 64 of 4,096 x 12,288 34.8 and 28.2. 128 rows of 24,576 x 4,096 with SwiGLU, 192 tiles of 128 x 128, 58.8 and 74.3, the
 // library's with a kernel behind it; up to 96 rows the weight-streaming kernel has it.)
@@ -308,7 +308,7 @@ Choice fused_by_rule(int kind, int M, int N, int K) {
   return c;
 }
 
-// What the table or the rule says for a size. A plain product that gemm_rounds.h covers in one round is its, whatever the table has
+// What the table or the rule says for a size. A plain product that gemm_rounds.hip covers in one round is its, whatever the table has
 // for the rows around it (the library's kernels); `aligned`: its operands lie at multiples of sixteen bytes, as its copies need.
 Choice choice_for(int kind, int M, int N, int K, int out_dtype, bool aligned = true) {
   if (g_kernels == KERNELS_BOTH) {
@@ -612,12 +612,8 @@ extern "C" int q3_tiles_scaled(const void* x, const void* w, void* out, int M, i
   scale.eps = eps;
   scale.inv_width = 1.f / (float)width;
   auto launch = [&](int config, int splits) {
-    if (config >= GROUPS_FIRST) {
-      const int shape = config - GROUPS_FIRST;
-      if (swiglu) return groups::launch<bf16_t, groups::EPI_SWIGLU>(shape, x, w, out, M, N, K, stream, scale);
-      if (out_dtype == Q3_F32) return groups::launch<float, groups::EPI_PLAIN>(shape, x, w, out, M, N, K, stream, scale);
-      return groups::launch<bf16_t, groups::EPI_PLAIN>(shape, x, w, out, M, N, K, stream, scale);
-    }
+    if (config >= GROUPS_FIRST)
+      return groups::scaled(config - GROUPS_FIRST, swiglu, out_dtype, x, w, out, M, N, K, stream, scale);
     if (swiglu)
       return tiles::launch<bf16_t, tiles::EPI_SWIGLU>(config, x, w, out, M, N, K, stream, splits, d.partials, scale);
     if (out_dtype == Q3_F32)
@@ -716,7 +712,7 @@ extern "C" int q3_tiles_residual(const void* x, const void* w, int M, int N, int
     res.norm_weight_f32 = norm_weight_dtype == Q3_F32;
     res.sums = sums;
     res.sums_stride = sums_stride;
-    return groups::launch<bf16_t, groups::EPI_RESIDUAL>(c.own - GROUPS_FIRST, x, w, values, M, N, K, stream, tiles::RowScale(), res);
+    return groups::residual(c.own - GROUPS_FIRST, x, w, values, M, N, K, stream, res);
   }
   if ((size_t)c.splits * M * N * sizeof(float) > PARTIALS_BYTES) return Q3_ERR_UNSUPPORTED;   // also a single share
   int used = 1;

@@ -32,6 +32,11 @@ FLAGS = [
 ]
 MODULES = ("elementwise", "norm", "rotary", "attention", "attention_capped", "attention_pooled", "attention_sigmoid", "attention_span", "latent", "moe",
            "hyper", "recurrent", "mlstm", "delta", "softcap", "gemm", "matmul", "sampling", "probes", "layers")
+# A module's further sources, compiled on their own: their kernels are code objects of their own in its library. Where a kernel's
+# code lies decides how long a launch of it takes to get going: with the kernels of these two between those of matmul.hip, the
+# tiled and the weight-streaming product of a step of 64 requests took 0.1 to 0.9 us longer each, with the same instructions
+# (a step of the 8B shape 7,656 us before they were added, 7,770 with them in one code object, 7,659 so).
+FURTHER = {"matmul": ["gemm_groups.hip", "gemm_rounds.hip"]}
 # what a module links besides the HIP runtime
 LINKS = {"matmul": ["-lhipblaslt"]}
 
@@ -55,9 +60,9 @@ def _hipcc():
 
 
 def _sources(module):
-    """The module's .hip file and the headers of this folder that it includes, directly or
+    """The module's .hip files and the headers of this folder that they include, directly or
     through another header."""
-    found, todo = [], [module + ".hip"]
+    found, todo = [], [module + ".hip"] + FURTHER.get(module, [])
     while todo:
         name = todo.pop()
         if name in found or not os.path.isfile(os.path.join(CSRC, name)):
@@ -116,7 +121,7 @@ def compile_module(module, force=False):
             continue
         so = os.path.join(lib_dir, module + ".so")
         tmp = so + ".tmp%d" % os.getpid()
-        cmd = [hipcc] + FLAGS + ["-I", CSRC, source, "-o", tmp]
+        cmd = [hipcc] + FLAGS + ["-I", CSRC, source] + [os.path.join(CSRC, name) for name in FURTHER.get(module, [])] + ["-o", tmp]
         if module in LINKS:
             rocm_lib = os.path.join(os.path.dirname(os.path.dirname(os.path.realpath(hipcc))), "lib")
             cmd += ["-L" + rocm_lib] + LINKS[module]

@@ -3,6 +3,7 @@ finds is stubbed; the entry format, the merge with an existing table and the shi
 well-formedness are checked."""
 
 import json
+import os
 
 from qwen3_from_scratch_amd import ops
 from qwen3_from_scratch_amd.ops import tune
@@ -42,6 +43,18 @@ def test_merge_keeps_old_sizes_and_replaces_the_ones_tuned_again(tmp_path, monke
     assert by_key[("plain", 2048, 4096, 4096, "bfloat16")]["library"] == 1              # kept
     assert by_key[("plain", 64, 4096, 4096, "float32")]["library"] == 7                 # another output type: kept
     assert by_key[("residual", 24, 4096, 12288, "bfloat16")]["splits"] == 8             # new
+
+
+def test_every_source_of_a_library_counts_when_it_may_be_stale():
+    """Also those that are compiled on their own, and what they include."""
+    from qwen3_from_scratch_amd.ops import build
+
+    sources = build._sources("matmul")
+    assert set(build.FURTHER["matmul"]) | {"matmul.hip", "gemm_groups.h", "gemm_tiles.h", "gates.h", "common.h"} <= set(sources)
+    for name in build.FURTHER["matmul"]:
+        header = name.replace(".hip", ".h")
+        with open(os.path.join(build.CSRC, header), encoding="utf-8") as fh:
+            assert "__global__" not in fh.read(), header          # its kernels are in no other code object
 
 
 def test_the_shipped_table_is_well_formed():
