@@ -4,7 +4,7 @@ interfaces, never by architecture."""
 
 import torch
 
-from ..parts.base import build_part
+from ..parts.base import UnscaledRows, build_part
 from ..weights.checkpoint import check_tensors
 from .layer_run import layer_runs
 
@@ -143,15 +143,18 @@ class DecoderModel:
         pending = None
         order = self.spec.order
         behind = 0                           # the first step that is not done yet
+        declined = None                      # the stretch of layers that left this pass to their parts: not asked again
         for i, step in enumerate(order):
             if i < behind:
                 continue
-            if i in self.runs and self.observer is None:
-                done = self.runs[i].forward(i, x, pending, batch, cache)
+            run = self.runs.get(i) if self.observer is None else None
+            if run is not None and run is not declined and isinstance(pending, UnscaledRows):
+                done = run.forward(i, x, pending, batch, cache)
                 if done is not None:
                     x, pending = done
-                    behind = self.runs[i].end
+                    behind = run.end
                     continue
+                declined = run
             view = cache.view(self.plane_of_step[i], writes=step.reads_cache_of is None)
             # the norm at the next block's entry, if that block can take over its division
             entry = getattr(self.layers[order[i + 1].layer].block, "entry_norm", None) if i + 1 < len(order) else None

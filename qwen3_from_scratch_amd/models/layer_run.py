@@ -13,10 +13,10 @@ class LayerRun:
         self.native, self.position, self.planes, self.exit_norm = native, position, planes, exit_norm
 
     def forward(self, first, x, pending, batch, cache):
-        """The layers from step `first` on, as their blocks would run them: (stream, what it still lacks), or None, with nothing
-        done, for a step that is another kernel's: one that does not come as UnscaledRows, of single tokens alone
-        (attention with its own preparation), or of rows that a product does not take in the form that carries its norm."""
-        if not isinstance(pending, UnscaledRows) or batch.max_q_len == 1 or not self.native.rows_fit(x.shape[0]):
+        """The layers from step `first` on, from UnscaledRows, as their blocks would run them: (stream, what it still lacks), or
+        None, with nothing done, for a step that is another kernel's: of single tokens alone (attention with its own preparation),
+        of rows that a product does not take in the form that carries its norm, or over pages that the matrix cores do not take."""
+        if batch.max_q_len == 1 or not self.native.rows_fit(x.shape[0]) or not hasattr(cache, "pages_of"):
             return None
         caches, block_table = cache.pages_of(self.planes[first - self.begin:], ("keys", "values"))
         if caches is None:

@@ -67,6 +67,8 @@ class DecoderLayers:
             if l["q_norm"] is not None and not (l["q_norm"].dtype in _DT and _vector(l["q_norm"], dim, layers[0]["q_norm"].dtype)
                                                 and _vector(l["k_norm"], dim, layers[0]["q_norm"].dtype)):
                 return None
+        if not library("attention").q3_paged_attention_fast_path(heads, kv_heads, dim, 16, _DT[torch.bfloat16]):
+            return None                               # (a head size whose attention is another kernel's at any page)
         return cls(layers, heads, kv_heads, dim, width, inner, qk_eps, scale, window)
 
     def rows_fit(self, rows):
@@ -86,6 +88,9 @@ class DecoderLayers:
             raise OperandError("a cache for each of the layers, keys (pages, Hkv, page, D)")
         T = values.shape[0]
         H, G, D, page = self.heads, self.kv_heads, self.dim, caches[0][0].shape[2]
+        attention = library("attention")
+        if not attention.q3_paged_attention_fast_path(H, G, D, page, _DT[torch.bfloat16]):
+            return None
         B = kv_lens.shape[0]
         stride = sums_stride(T)
         if not (stream.is_cuda and stream.shape == (T, self.width) and stream.dtype == torch.float32 and stream.is_contiguous()
@@ -110,9 +115,7 @@ class DecoderLayers:
                     and table.shape[1] % 2 == 0 and table.shape[1] <= D and max_kv_len <= table.shape[0]):
                 raise OperandError("table must be float32 (P, R) and hold the step's last position")
             max_pos, rotary_dim = table.shape
-        matmul, rotary, attention = _matmul(), library("rotary"), library("attention")
-        if not attention.q3_paged_attention_fast_path(H, G, D, page, 1):
-            return None
+        matmul, rotary = _matmul(), library("rotary")
 
         def empty(*shape, dtype=torch.bfloat16):
             return torch.empty(shape, dtype=dtype, device=values.device)

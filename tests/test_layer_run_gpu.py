@@ -6,13 +6,13 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-def _model(layers=5, qk_norm="Qwen3ForCausalLM", dtype="bfloat16", tiled=True):
+def _model(layers=5, dtype="bfloat16", head_dim=128):
     from qwen3_from_scratch_amd.config import ModelConfig
     from qwen3_from_scratch_amd.engine import random_model
 
     config = ModelConfig.from_dict(dict(
-        architectures=[qk_norm], vocab_size=512, hidden_size=1024, hidden_act="silu", num_hidden_layers=layers,
-        max_position_embeddings=8192, num_attention_heads=16, num_key_value_heads=8, head_dim=128,
+        architectures=["Qwen3ForCausalLM"], vocab_size=512, hidden_size=1024, hidden_act="silu", num_hidden_layers=layers,
+        max_position_embeddings=8192, num_attention_heads=16, num_key_value_heads=8, head_dim=head_dim,
         intermediate_size=2048, rms_norm_eps=1e-6, rope_theta=1e6, tie_word_embeddings=False))
     return random_model(config, dtype=dtype, device="cuda:0", seed=5)
 
@@ -24,10 +24,10 @@ def _steps(seed, *steps):
     return [[StepEntry(rid, torch.randint(0, 512, (n,), generator=g).tolist(), [n - 1]) for rid, n in step] for step in steps]
 
 
-def _logits(model, steps, calls=None):
+def _logits(model, steps, calls=None, page=16):
     from qwen3_from_scratch_amd.engine import ModelRunner
 
-    runner = ModelRunner(model, 16, 700, max_requests=8)
+    runner = ModelRunner(model, page, 700, max_requests=8)
     out = []
     for entries in steps:
         if calls is not None:
@@ -86,3 +86,33 @@ def test_layers_that_are_not_taken():
     with pytest.raises(ops.OperandError):
         rows = torch.zeros(70, 1024, device="cuda")
         native.run(0, 1, rows, rows, rows, [(rows, rows)], rows, rows, rows, rows, rows, 70, 70, 70, None, None)
+
+
+def test_layers_that_the_matrix_cores_do_not_attend_for(monkeypatch):
+    """A head size that they take at no page leaves no stretch; a page that they do not take is found out once a step."""
+    from qwen3_from_scratch_amd.ops.layers import DecoderLayers
+
+    assert not _model(layers=3, head_dim=96).runs
+    model, asked, run = _model(), [], DecoderLayers.run
+    monkeypatch.setattr(DecoderLayers, "run", lambda self, *args: asked.append(run(self, *args)) or asked[-1])
+    steps = _steps(7, (("a", 200),), (("b", 90), ("a", 1)))
+    got = _logits(model, steps, page=24)
+    assert asked == [None, None]
+    model.observer = lambda *args: None
+    for a, b in zip(got, _logits(model, steps, page=24)):
+        assert torch.equal(a, b)
+
+
+def test_a_cache_that_gives_views_alone():
+    """What a model asks of a cache is `view`."""
+    model = _model()
+    steps = _steps(8, (("a", 200),))
+    want = _logits(model, steps)
+    forward = model.forward
+
+    class Views:
+        def __init__(self, cache):
+            self.view = cache.view
+
+    model.forward = lambda batch, cache: forward(batch, Views(cache))
+    assert torch.equal(_logits(model, steps)[0], want[0])
