@@ -57,7 +57,7 @@ struct Q3LayerStep {
   float *middle_sums, *exit_sums;
 };
 
-// The first refusal or error ends it; `*failed` then says in which of a layer's six operations.
+// The first refusal, decline or error ends it; `*failed` then says where: six times the layer, plus which of its operations.
 int q3_decoder_layers(const Q3Layer* layers, int n, const Q3LayerStep* step, int* failed) {
   if (!layers || n < 1 || !step || !failed || !step->scaled || !step->residual || !step->prepare || !step->attention)
     return Q3_ERR_BAD_ARGUMENT;
@@ -69,31 +69,31 @@ int q3_decoder_layers(const Q3Layer* layers, int n, const Q3LayerStep* step, int
     const float* sums = i ? s.exit_sums : s.entry_sums;
     int status = s.scaled(rows, l.qkv, s.qkv_rows, s.rows, joined, s.width, Q3_BF16, 0, sums, i ? s.exit_chunks : s.entry_chunks,
                           s.sums_stride, l.entry_eps, s.width, s.stream);
-    *failed = 0;
+    *failed = 6 * i;
     if (status) return status;
     status = s.prepare(s.qkv_rows, l.q_norm, l.k_norm, s.qk_dtype, s.qk_eps, s.table, s.rotary_dim, s.max_pos, s.positions,
                        s.seq_index, s.block_table, s.table_width, s.sequences, l.keys, l.values, s.page, s.num_pages, s.rows,
                        s.heads, s.kv_heads, s.dim, Q3_BF16, s.cu_q, s.kv_lens, s.sequences, s.max_q_len, s.max_kv_len,
                        (hipStream_t)s.stream);
-    *failed = 1;
+    *failed = 6 * i + 1;
     if (status) return status;
     status = s.attention(s.qkv_rows, joined, s.attended, l.keys, l.values, s.num_pages, s.block_table, s.table_width, s.cu_q,
                          s.kv_lens, s.sequences, s.rows, s.heads, s.kv_heads, s.dim, s.page, s.scale, s.window, s.max_q_len,
                          s.min_q_len, s.max_kv_len, Q3_BF16, s.splits, s.workspace, s.prompt_splits, s.prompt_workspace,
                          nullptr, (hipStream_t)s.stream);
-    *failed = 2;
+    *failed = 6 * i + 2;
     if (status) return status;
     status = s.residual(s.attended, l.out, s.rows, s.width, attended, s.residual_rows, l.middle_norm, s.norm_dtype, s.norm_rows,
                         s.middle_sums, s.middle_chunks, s.sums_stride, s.stream);
-    *failed = 3;
+    *failed = 6 * i + 3;
     if (status) return status;
     status = s.scaled(s.norm_rows, l.gate_up, s.hidden, s.rows, 2 * s.inner, s.width, Q3_BF16, 1, s.middle_sums, s.middle_chunks,
                       s.sums_stride, l.middle_eps, s.width, s.stream);
-    *failed = 4;
+    *failed = 6 * i + 4;
     if (status) return status;
     status = s.residual(s.hidden, l.down, s.rows, s.width, s.inner, s.residual_rows, l.next_norm, s.norm_dtype, s.norm_rows,
                         s.exit_sums, s.exit_chunks, s.sums_stride, s.stream);
-    *failed = 5;
+    *failed = 6 * i + 5;
     if (status) return status;
   }
   return 0;

@@ -151,8 +151,7 @@ class DecoderModel:
             if run is not None and run is not declined and isinstance(pending, UnscaledRows):
                 done = run.forward(i, x, pending, batch, cache)
                 if done is not None:
-                    x, pending = done
-                    behind = run.end
+                    x, pending, behind = done
                     continue
                 declined = run
             view = cache.view(self.plane_of_step[i], writes=step.reads_cache_of is None)

@@ -1,6 +1,6 @@
 """Stretches of equal layers that a step may run as one native call."""
 
-from ..ops.layers import DecoderLayers
+from ..ops.layers import Declined, DecoderLayers
 from ..parts.base import UnscaledRows
 
 
@@ -8,14 +8,15 @@ class LayerRun:
     """The steps `begin` .. `end - 1` of a model's run order, whose layers `ops.layers.DecoderLayers` takes: layers of one shape,
     each with a cache plane of its own to write, each followed by one whose entry norm its last product prepares."""
 
-    def __init__(self, begin, end, native, position, planes, exit_norm):
+    def __init__(self, begin, end, native, position, planes, blocks, exit_norm):
         self.begin, self.end = begin, end
-        self.native, self.position, self.planes, self.exit_norm = native, position, planes, exit_norm
+        self.native, self.position, self.planes, self.blocks, self.exit_norm = native, position, planes, blocks, exit_norm
 
     def forward(self, first, x, pending, batch, cache):
-        """The layers from step `first` on, from UnscaledRows, as their blocks would run them: (stream, what it still lacks), or
-        None, with nothing done, for a step that is another kernel's: of single tokens alone (attention with its own preparation),
-        of rows that a product does not take in the form that carries its norm, or over pages that the matrix cores do not take."""
+        """The layers from step `first` on, from UnscaledRows, as their blocks would run them: (stream, what it still lacks, the
+        first step that is not done yet), or None, with nothing done, for a step that is another kernel's: of single tokens alone
+        (attention with its own preparation), of rows that a product does not take in the form that carries its norm, or over
+        pages that the matrix cores do not take."""
         if batch.max_q_len == 1 or not self.native.rows_fit(x.shape[0]) or not hasattr(cache, "pages_of"):
             return None
         caches, block_table = cache.pages_of(self.planes[first - self.begin:], ("keys", "values"))
@@ -27,7 +28,14 @@ class LayerRun:
                                batch.min_q_len, batch.max_kv_len, getattr(batch, "max_kv_len_portions", None), table)
         if done is None:
             return None
-        return x, UnscaledRows(done[0], done[1], self.exit_norm.eps, self.exit_norm.size)
+        if isinstance(done, Declined):
+            step = first + done.layer
+            block = self.blocks[step - self.begin]
+            if not done.of_attention:
+                return x, block.feed_forward.down.forward(done.rows), step + 1
+            h = block.feed_forward_norm.forward(x, delta=block.mixer.out.forward(done.rows))
+            return x, block.feed_forward.forward(h, batch), step + 1
+        return x, UnscaledRows(done[0], done[1], self.exit_norm.eps, self.exit_norm.size), self.end
 
 
 def layer_runs(model):
@@ -48,7 +56,8 @@ def layer_runs(model):
             native = DecoderLayers.of([f[0] for f in found[at:end]], **found[at][1])
             if native is not None:
                 exit_norm = model.layers[order[end].layer].block.entry_norm()
-                run = LayerRun(at, end, native, found[at][2], [model.plane_of_step[i] for i in range(at, end)], exit_norm)
+                run = LayerRun(at, end, native, found[at][2], [model.plane_of_step[i] for i in range(at, end)],
+                               [model.layers[order[i].layer].block for i in range(at, end)], exit_norm)
                 runs.update((i, run) for i in range(at, end))
         at = max(end, at + 1)
     return runs

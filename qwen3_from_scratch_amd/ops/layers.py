@@ -2,10 +2,11 @@
 operation, for steps whose time is the host's."""
 
 import ctypes
+from typing import NamedTuple
 
 import torch
 
-from . import (_DT, _check, _matmul, _splits, _stream, few_rows_limit, fused_rows_most, library, matmul_fused_plan, sums_stride,
+from . import (_DECLINED, _DT, _check, _matmul, _splits, _stream, few_rows_limit, fused_rows_most, library, matmul_fused_plan, sums_stride,
                FUSED_ROWS_SMALL, OperandError)
 
 _P, _I, _F = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
@@ -30,6 +31,16 @@ class _Step(ctypes.Structure):
 
 _OPERATIONS = ("the product of queries, keys and values", "qk_norm_rope_store", "paged_attention", "the attention's output product",
                "the gated product", "the product back into the stream")
+_ATTENTION_OUT, _DOWN = 3, 5        # the two that add into the stream
+
+
+class Declined(NamedTuple):
+    """Where a stretch ended early: `layer` (from the first one run) whose product into the stream was left to the plain product and
+    the norm's own kernel, the attention's output product (`of_attention`) or the feed-forward's, and the rows that lack it."""
+
+    layer: int
+    of_attention: bool
+    rows: torch.Tensor
 
 
 def _matrix(t, shape):
@@ -83,7 +94,8 @@ class DecoderLayers:
         """Layers `first` .. `first + count - 1` over the residual `stream` (T, width) float32, in place, from rows
         (`values`, `sums`: see `linear_residual_norm`) that lack the first one's entry norm. `caches`: per layer (keys, values), as
         `paged_attention` takes them, all of one shape. Returns the rows that lack the norm behind the last layer, as (values,
-        sums); None, and nothing is done, where the attention is not one for the matrix cores."""
+        sums); None, and nothing is done, where the attention is not one for the matrix cores; Declined where a product into the
+        stream is not one of those that carry a norm after all (`rows_fit` was asked, and another thread has changed which kernels serve)."""
         if not (0 <= first and 0 < count <= len(self.layers) - first and len(caches) == count and caches[0][0].dim() == 4):
             raise OperandError("a cache for each of the layers, keys (pages, Hkv, page, D)")
         T = values.shape[0]
@@ -159,6 +171,9 @@ class DecoderLayers:
             native.keys, native.values = keys.data_ptr(), held.data_ptr()
             native.entry_eps, native.middle_eps = l["entry_eps"], l["middle_eps"]
         failed = ctypes.c_int(0)
-        _check(library("layers").q3_decoder_layers(layers, count, ctypes.byref(step), ctypes.byref(failed)),
-               _OPERATIONS[failed.value])
+        status = library("layers").q3_decoder_layers(layers, count, ctypes.byref(step), ctypes.byref(failed))
+        layer, operation = divmod(failed.value, len(_OPERATIONS))
+        if status == _DECLINED and operation in (_ATTENTION_OUT, _DOWN):
+            return Declined(layer, operation == _ATTENTION_OUT, attended if operation == _ATTENTION_OUT else hidden)
+        _check(status, _OPERATIONS[operation])
         return out, exit_

@@ -6,14 +6,14 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-def _model(layers=5, dtype="bfloat16", head_dim=128):
+def _model(layers=5, dtype="bfloat16", head_dim=128, inner=2048):
     from qwen3_from_scratch_amd.config import ModelConfig
     from qwen3_from_scratch_amd.engine import random_model
 
     config = ModelConfig.from_dict(dict(
         architectures=["Qwen3ForCausalLM"], vocab_size=512, hidden_size=1024, hidden_act="silu", num_hidden_layers=layers,
         max_position_embeddings=8192, num_attention_heads=16, num_key_value_heads=8, head_dim=head_dim,
-        intermediate_size=2048, rms_norm_eps=1e-6, rope_theta=1e6, tie_word_embeddings=False))
+        intermediate_size=inner, rms_norm_eps=1e-6, rope_theta=1e6, tie_word_embeddings=False))
     return random_model(config, dtype=dtype, device="cuda:0", seed=5)
 
 
@@ -116,3 +116,29 @@ def test_a_cache_that_gives_views_alone():
 
     model.forward = lambda batch, cache: forward(batch, Views(cache))
     assert torch.equal(_logits(model, steps)[0], want[0])
+
+
+@pytest.mark.parametrize("inner", [True, False])
+def test_a_product_that_declines_after_all(monkeypatch, inner):
+    """The product into the stream is declined when the settings change between the question and the step (here: by a
+    number of partial sums that is not the kernel's): its layer is finished by its parts, as it would have been without the stretch."""
+    from qwen3_from_scratch_amd.ops import layers
+
+    steps = _steps(9, (("a", 200),), (("b", 90), ("a", 1)))
+    lib, asked, run = layers._matmul(), [], layers.DecoderLayers.run
+
+    class Other:
+        q3_tiles_scaled, q3_tiles_residual = lib.q3_tiles_scaled, lib.q3_tiles_residual
+
+        @staticmethod
+        def q3_tiles_residual_chunks(M, N, K):
+            return lib.q3_tiles_residual_chunks(M, N, K) + (2048 == K if not inner else 4096 == K)
+
+    model = _model(inner=4096)                   # (the attention's output product has 2,048 numbers a row)
+    monkeypatch.setattr(layers, "_matmul", lambda: Other)
+    monkeypatch.setattr(layers.DecoderLayers, "run", lambda self, *args: asked.append(run(self, *args)) or asked[-1])
+    got = _logits(model, steps)
+    assert len(asked) == 4 and all(isinstance(d, layers.Declined) and d.layer == 0 and d.of_attention != inner for d in asked)
+    model.observer = lambda *args: None
+    for a, b in zip(got, _logits(model, steps)):
+        assert float((a - b).norm() / b.norm()) < 0.02       # another rounding of one product in bfloat16 a layer
