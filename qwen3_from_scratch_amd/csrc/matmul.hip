@@ -654,12 +654,12 @@ extern "C" int q3_tiles_scaled(const void* x, const void* w, void* out, int M, i
   return launch(c.own, c.splits);
 }
 
-// Whether q3_tiles_scaled would serve a size by the kernel that shares K out inside a block, with the few-row kernel's bits:
-// a row's results do not depend on how many rows are beside it where the few-row kernel takes them (its callers' rule).
-extern "C" int q3_groups_as_few(int M, int N, int K) {
+// Whether q3_tiles_scaled (`epilogue`: its own) would serve a size by the kernel that shares K out inside a block, with the few-row
+// kernel's bits: a row's results do not depend on how many rows are beside it where the few-row kernel takes them (its callers' rule).
+extern "C" int q3_groups_as_few(int M, int N, int K, int epilogue) {
   std::lock_guard<std::mutex> hold(g_lock);
   if (g_mode != MODE_RULE || M > FUSED_ROWS_LIMIT) return 0;
-  const int own = choice_for(KIND_SCALED, M, N, K, Q3_BF16).own;
+  const int own = choice_for(epilogue == tiles::EPI_SWIGLU ? KIND_SCALED_SWIGLU : KIND_SCALED, M, N, K, Q3_BF16).own;
   return own >= GROUPS_FIRST && groups::shares_of_few_rows(own - GROUPS_FIRST, N, K);
 }
 

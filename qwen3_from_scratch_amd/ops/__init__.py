@@ -1903,14 +1903,14 @@ def sums_stride(M):
 GROUPS_LEAST_COLUMNS = 4096
 
 
-def _groups_before_few(weight, M, unscaled):
+def _groups_before_few(weight, M, unscaled, swiglu=False):
     """Whether rows that still lack their norm go by the kernel that shares K out inside a block although the few-row kernel
     takes as many: 17 rows and more of a small weight of 4,096 columns or more, where both add alike (an inner size of 1,024, say),
     so that a row's bits do not change with the number of rows. There the few-row kernel, a block per 16
     columns and 16 rows, needs two rounds of blocks: 24, 32 and 64 rows of 4,096 x 1,024 6.4, 6.7 and 10.3 us, of 8,192 x 1,024
     10.7, 11.4 and 18.5, the other kernel 5.4, 5.6, 6.1 and 6.9, 7.0, 8.3; 24 rows of 1,024 x 2,048 6.2 and 6.8."""
     return (unscaled is not None and M > FEW_ROWS and weight.shape[0] >= GROUPS_LEAST_COLUMNS and fused_rows_take(weight, M)
-            and _matmul().q3_groups_as_few(M, weight.shape[0], weight.shape[1]))
+            and _matmul().q3_groups_as_few(M, weight.shape[0], weight.shape[1], 1 if swiglu else 0))
 
 
 def _tiled_ok(tiled, weight, M):
@@ -2138,7 +2138,7 @@ def linear_swiglu(x, weight, tiled=None, unscaled=None, kind="silu", narrow=None
         out = torch.empty((M, N // 2), dtype=x.dtype, device=x.device)
         if _stream_product(x, weight, tiled, out, True, unscaled, "linear_swiglu", kind):
             return out
-    if M and x.dtype == torch.bfloat16 and _tiled_ok(tiled, weight, M) and not (kind == "silu" and _groups_before_few(weight, M, unscaled)):
+    if M and x.dtype == torch.bfloat16 and _tiled_ok(tiled, weight, M) and not (kind == "silu" and _groups_before_few(weight, M, unscaled, True)):
         out = torch.empty((M, N // 2), dtype=x.dtype, device=x.device)
         sums, sums_rows, eps, width, stride = _row_sums_args(unscaled, M, K)
         _check(library("gemm").q3_linear_tiled(

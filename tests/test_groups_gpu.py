@@ -3,7 +3,7 @@
 import pytest
 import torch
 
-from test_kernels_gpu import _ops, _rand
+from test_kernels_gpu import _forget_choices, _ops, _rand, rules_alone
 
 pytestmark = pytest.mark.gpu
 
@@ -69,3 +69,21 @@ def test_rows_that_two_kernels_take():
         assert torch.equal(first, got[:16])
     w = _rand((4096, 2048), torch.bfloat16, 99)          # eight shares of K there, four here
     assert not ops._groups_before_few(w, 32, (sums, 1e-5, 2048))
+
+
+@pytest.mark.parametrize("kind,other", [("scaled_swiglu", "scaled"), ("scaled", "scaled_swiglu")])
+def test_a_table_entry_for_one_of_the_two_epilogues(rules_alone, kind, other):
+    """A size that the table sends to the tiles, with the activation or without: the few-row kernel keeps its rows there, and
+    either way a row's bits are those it has among sixteen."""
+    ops, (M, N, K) = rules_alone, (32, 4096, 1024)
+    ops.matmul_table([{"kind": kind, "rows": M, "N": N, "K": K, "own": 1, "splits": 8}], clear=True)
+    _forget_choices(ops)
+    x, w = _rand((M, K), torch.bfloat16, 98), _rand((N, K), torch.bfloat16, 99, scale=0.05)
+    tiled, sums = ops.tile_weight(w), torch.rand((64, M), generator=torch.Generator().manual_seed(97)).cuda() * 32.0
+    products = {"scaled": lambda x, sums: ops.linear(x, w, out_dtype=torch.float32, tiled=tiled, unscaled=(sums, 1e-5, K)),
+                "scaled_swiglu": lambda x, sums: ops.linear_swiglu(x, w, tiled=tiled, unscaled=(sums, 1e-5, K))}
+    unscaled = (sums, 1e-5, K)
+    assert not ops._groups_before_few(w, M, unscaled, kind == "scaled_swiglu")
+    assert ops._groups_before_few(w, M, unscaled, other == "scaled_swiglu")
+    for product in products.values():
+        assert torch.equal(product(x, sums)[:16], product(x[:16].contiguous(), sums[:, :16].contiguous()))
