@@ -9,7 +9,7 @@
 // reproducible. The decision is, in this order,
 //   1. an entry of the table that the caller loaded (q3_matmul_table_add): a
 //      place in the library's ranked list of candidates for the size, or a tile
-//      shape of the hand-written kernel with a number of shares of K; the table is
+//      shape of a hand-written kernel with a number of shares of K; the table is
 //      data made beforehand by the tuner below, keyed by (kind of product, rows
 //      rounded up, N, K, output type);
 //   2. a rule of thumb: the library's first candidate for a plain product; for
@@ -21,9 +21,9 @@
 //
 // The tuner (q3_matmul_set_mode(1), off unless asked for) is what the table is
 // made with: a size first met outside a graph capture has its candidates timed
-// on the caller's own operands, the library's leading ones and the tile shapes
+// on the caller's own operands, the library's leading ones, the tile shapes
 // that fit the rows, each also with K shared out where its tiles alone would not
-// fill the chip, and the fastest is kept for the life of the process
+// fill the chip, and the tile of gemm_groups.hip or gemm_rounds.hip where they take the size, and the fastest is kept for the life of the process
 // (q3_matmul_plan and q3_matmul_fused_plan tell what it was). In the model every
 // weight is read once a step, with gigabytes of other traffic in between, so a
 // candidate is timed with cold caches: a kernel that reads a buffer larger than
@@ -63,8 +63,8 @@ constexpr int EVICT_BLOCKS = 2048, EVICT_THREADS = 256;
 constexpr int MAX_CANDIDATES = 64;
 constexpr int MISALIGNED = 256;                // in a plan's key: operands that are not at multiples of 16 bytes
 constexpr int LIBRARY = -1;                    // a Choice's `own` when the library serves the size
-constexpr int GROUPS_FIRST = 16;               // a Choice's `own` from here on: gemm_groups.hip's shapes (no table entry)
-constexpr int ROUNDS_FIRST = 32;               // and from here on: gemm_rounds.hip's, plus the tile's height (no table entry)
+constexpr int GROUPS_FIRST = 16;               // a Choice's `own` from here on: gemm_groups.hip's shapes
+constexpr int ROUNDS_FIRST = 32;               // and from here on: gemm_rounds.hip's, plus the tile's height
 static_assert(GROUPS_FIRST >= tiles::NUM_CONFIGS && ROUNDS_FIRST >= GROUPS_FIRST + groups::NUM_SHAPES, "one numbering");
 
 // Reads the whole buffer; the store never happens (the buffer holds zeros) but keeps the loads alive.
@@ -77,8 +77,9 @@ __global__ void evict_kernel(float4* buffer, size_t count) {
   if (sum == 12345.f) buffer[0].x = sum;
 }
 
-// The kinds of product a choice is made for.
-enum { KIND_PLAIN = 0, KIND_SCALED = 1, KIND_SCALED_SWIGLU = 2, KIND_RESIDUAL = 3 };
+// The kinds of product a choice is made for. (KIND_ROUND: a plain product of a size that gemm_rounds.hip takes. What was found for the
+// other sizes that share its rows says nothing about it.)
+enum { KIND_PLAIN = 0, KIND_SCALED = 1, KIND_SCALED_SWIGLU = 2, KIND_RESIDUAL = 3, KIND_ROUND = 4, KINDS = 5 };
 
 // Who serves a size: the library's candidate number `library` (own == LIBRARY), or the hand-written kernel's
 // tile shape `own` with K shared out over `splits` blocks per tile.
@@ -99,7 +100,7 @@ struct Plan {
   float first_us = 0.f, best_us = 0.f;
 };
 
-typedef std::tuple<int, int, int, int, int> Key;   // kind (+ 4 * which kernels, for the tuner's notes), rows, N, K, output type
+typedef std::tuple<int, int, int, int, int> Key;   // kind (+ KINDS * which kernels, for the tuner's notes), rows, N, K, output type
 
 struct Device {
   hipblasLtHandle_t handle = nullptr;
@@ -125,7 +126,7 @@ int g_mode = MODE_RULE;
 // prompt's portion plus however many requests decode): up to 64 rows, and the products that carry a norm at
 // any count, in steps of 8; plain products beyond 64 rows in steps of 32.
 int rows_key(int kind, int M) {
-  if (kind != KIND_PLAIN || M <= 64) return (M + 7) / 8 * 8;
+  if ((kind != KIND_PLAIN && kind != KIND_ROUND) || M <= 64) return (M + 7) / 8 * 8;
   return (M + 31) / 32 * 32;
 }
 
@@ -308,25 +309,39 @@ Choice fused_by_rule(int kind, int M, int N, int K) {
   return c;
 }
 
-// What the table or the rule says for a size. A plain product that gemm_rounds.hip covers in one round is its, whatever the table has
-// for the rows around it (the library's kernels); `aligned`: its operands lie at multiples of sixteen bytes, as its copies need.
+// The height of gemm_rounds.hip's tile for a plain product, 0 where it is not its; `aligned`: the operands lie at multiples of sixteen
+// bytes, as its copies need.
+int round_height(int kind, int M, int N, int K, int out_dtype, bool aligned) {
+  if (kind != KIND_PLAIN || g_kernels != KERNELS_BOTH || out_dtype != Q3_BF16 || !aligned) return 0;
+  return rounds::height_for(M, N, K);
+}
+
+// A choice made for this size or for another that shares its entry, as it is for this one.
+Choice for_size(Choice c, int height) {
+  if (c.own >= ROUNDS_FIRST) c.own = ROUNDS_FIRST + height;
+  return c;
+}
+
+// What the table or the rule says for a size.
 Choice choice_for(int kind, int M, int N, int K, int out_dtype, bool aligned = true) {
+  const int height = round_height(kind, M, N, K, out_dtype, aligned);
   if (g_kernels == KERNELS_BOTH) {
-    const int height = kind == KIND_PLAIN && out_dtype == Q3_BF16 && aligned ? rounds::height_for(M, N, K) : 0;
-    if (height) {
-      Choice c;
-      c.own = ROUNDS_FIRST + height;
-      return c;
-    }
-    auto entry = g_table.find(Key(kind, rows_key(kind, M), N, K, out_dtype));
+    const int filed = height ? (int)KIND_ROUND : kind;
+    auto entry = g_table.find(Key(filed, rows_key(filed, M), N, K, out_dtype));
     if (entry != g_table.end()) {
-      Choice c = entry->second;
-      const bool fits = c.own == LIBRARY ||
+      const Choice c = for_size(entry->second, height);
+      const bool fits = c.own == LIBRARY || c.own >= ROUNDS_FIRST ||
+                        (tiles::takes(M, N, K) && c.own >= GROUPS_FIRST && N % 4 == 0) ||
                         (tiles::takes(M, N, K) && c.own < tiles::NUM_CONFIGS && c.splits >= 1 && c.splits <= K / tiles::BK &&
                          c.splits <= 64 && (c.splits == 1 || N % 4 == 0) &&
                          (size_t)c.splits * ((M + 7) / 8 * 8) * N * sizeof(float) <= PARTIALS_BYTES);
       if (fits) return c;
     }
+  }
+  if (height) {
+    Choice c;
+    c.own = ROUNDS_FIRST + height;
+    return c;
   }
   return kind == KIND_PLAIN ? plain_by_rule(M, N, K) : fused_by_rule(kind, M, N, K);
 }
@@ -337,7 +352,7 @@ Choice choice_for(int kind, int M, int N, int K, int out_dtype, bool aligned = t
 // and 32B models there). Each enters a second time with K shared out where its tiles alone would not fill the
 // chip.
 constexpr int OWN_FEW_ROWS[] = {1, 5}, OWN_SOME_ROWS[] = {0, 1, 2}, OWN_MANY_ROWS[] = {0, 2, 4};
-constexpr int MAX_OWN = 6;
+constexpr int MAX_OWN = 7;
 inline const int* own_shapes(int M, int& count) {
   if (M <= 256) {
     count = 2;
@@ -364,7 +379,7 @@ float time_runs(Device& d, hipStream_t stream, int reps, Launch launch) {
 }
 
 // Times the candidates for the plan's size on the caller's operands and leaves the fastest in the plan.
-int tune_plain(Device& d, Plan& p, const void* x, const void* w, void* out, int M, int N, int K, int out_dtype,
+int tune_plain(Device& d, Plan& p, const void* x, const void* w, void* out, int M, int N, int K, int out_dtype, int height,
                hipStream_t stream) {
   const int set = set_up_tuner(d, stream);
   if (set) return set;
@@ -376,8 +391,12 @@ int tune_plain(Device& d, Plan& p, const void* x, const void* w, void* out, int 
     if (status && !(status == Q3_ERR_UNSUPPORTED && own_takes)) return status;
     got = (int)found.size();
   }
-  // candidates from `got` on are the hand-written kernel's: (tile shape, shares of K)
+  // candidates from `got` on are the hand-written kernels': (tile shape, shares of K)
   int own_config[MAX_OWN], own_splits[MAX_OWN], owns = 0;
+  if (height) {
+    own_config[owns] = ROUNDS_FIRST + height;
+    own_splits[owns++] = 1;
+  }
   if (own_takes) {
     int count = 0;
     const int* shapes = own_shapes(M, count);
@@ -471,6 +490,7 @@ int product(Device& d, const void* x, const void* w, void* out, int M, int N, in
   int status = ready_device(d, stream);
   if (status) return status;
   const bool aligned = (((size_t)x | (size_t)w | (size_t)out) & 15) == 0;
+  const int height = round_height(KIND_PLAIN, M, N, K, out_dtype, aligned);
   Plan& p = d.plans[std::make_tuple(M, N, K, aligned ? out_dtype : out_dtype + MISALIGNED)];
   if (!p.desc) {
     status = describe(p, M, N, K, out_dtype);
@@ -483,13 +503,14 @@ int product(Device& d, const void* x, const void* w, void* out, int M, int N, in
     const bool in_capture = capturing(stream, status);
     if (status) return status;
     if (!in_capture) {
-      const Key near(KIND_PLAIN + 4 * g_kernels, rows_key(KIND_PLAIN, M), N, K, out_dtype);
+      const int kind = height ? KIND_ROUND : KIND_PLAIN;
+      const Key near(kind + KINDS * g_kernels, rows_key(kind, M), N, K, out_dtype);
       auto noted = d.noted.find(near);
       if (noted != d.noted.end()) {   // a neighbour's choice, asked of the library anew for this size
-        status = settle(d, p, noted->second, M, N, K);
+        status = settle(d, p, for_size(noted->second, height), M, N, K);
         if (status == 0) p.timed = true;
       } else {
-        status = tune_plain(d, p, x, w, out, M, N, K, out_dtype, stream);
+        status = tune_plain(d, p, x, w, out, M, N, K, out_dtype, height, stream);
         if (status == 0) d.noted[near] = p.choice;
       }
       if (status) {
@@ -509,7 +530,7 @@ int product(Device& d, const void* x, const void* w, void* out, int M, int N, in
 }
 
 // Tile shape and shares of K for a product of some tens of rows that carries a norm, or LIBRARY: `other()`
-// then does the same work around the library's product. `launch(config, splits)` runs the tiled kernel
+// then does the same work around the library's product. `launch(config, splits)` runs the hand-written kernel
 // without side effects and returns its status. By the table or the rule; with the tuner on, timed once per
 // size with cold caches outside a graph capture.
 template <typename Launch, typename Other>
@@ -518,7 +539,7 @@ int choose_fused(Device& d, int kind, int M, int N, int K, hipStream_t stream, L
     c = choice_for(kind, M, N, K, Q3_BF16);
     return 0;
   }
-  const Key key(kind + 4 * g_kernels, rows_key(kind, M), N, K, Q3_BF16);
+  const Key key(kind + KINDS * g_kernels, rows_key(kind, M), N, K, Q3_BF16);
   auto known = d.noted.find(key);
   if (known != d.noted.end()) {
     c = known->second;
@@ -534,7 +555,12 @@ int choose_fused(Device& d, int kind, int M, int N, int K, hipStream_t stream, L
   // 64 x 128 tiles also with five stages: with K shared out they need fewer shares to fill the chip (q/k/v at
   // 64 rows 17.7 us in 5 shares against 21.9 in 8). The 64 x 256 tiles lose here too (gate/up 67 us against 51).
   constexpr int FUSED_SHAPES[] = {1, 5, 8};
-  int configs[6], shares[6], n = 0;
+  int configs[7], shares[7], n = 0;
+  const int groups_shape = g_kernels == KERNELS_BOTH ? groups::shape_for(M, N, K) : -1;
+  if (groups_shape >= 0) {
+    configs[n] = GROUPS_FIRST + groups_shape;
+    shares[n++] = 1;
+  }
   for (int shape : FUSED_SHAPES) {
     const int fill = tiles::splits_that_fill(shape, M, N, K);   // the same for all rows that share the choice
     if (fill > 1 && (size_t)fill * ((M + 7) / 8 * 8) * N * sizeof(float) <= PARTIALS_BYTES) {
@@ -673,10 +699,28 @@ static int chunks_of(int columns, int N) { return (N + columns - 1) / columns; }
 static int residual_chunks(const Choice& c, int N) {
   return chunks_of(c.own >= GROUPS_FIRST ? groups::SHAPES[c.own - GROUPS_FIRST][1] : tiles::CHUNK_COLUMNS, N);
 }
+static int add_into(const float* partials, int shares, float* residual, const void* norm_weight, int norm_weight_dtype, void* values,
+                    float* sums, int sums_stride, int M, int N, hipStream_t stream) {
+  const dim3 grid(chunks_of(tiles::CHUNK_COLUMNS, N), M);
+  if (norm_weight_dtype == Q3_F32)
+    hipLaunchKernelGGL(tiles::tiles_residual_kernel<float>, grid, dim3(256), 0, stream, partials, shares, residual,
+                       (const float*)norm_weight, (bf16_t*)values, sums, sums_stride, M, N);
+  else
+    hipLaunchKernelGGL(tiles::tiles_residual_kernel<bf16_t>, grid, dim3(256), 0, stream, partials, shares, residual,
+                       (const bf16_t*)norm_weight, (bf16_t*)values, sums, sums_stride, M, N);
+  return q3_launch_status();
+}
 extern "C" int q3_tiles_residual_chunks(int M, int N, int K) {
   std::lock_guard<std::mutex> hold(g_lock);
-  if (g_mode == MODE_TUNE) return chunks_of(tiles::CHUNK_COLUMNS, N);   // the tuner times the tiled kernel's shapes
-  return residual_chunks(choice_for(KIND_RESIDUAL, M, N, K, Q3_BF16), N);
+  if (g_mode != MODE_TUNE) return residual_chunks(choice_for(KIND_RESIDUAL, M, N, K, Q3_BF16), N);
+  // what the tuner has found, or before it has the rule's (declined once where its contest then ends otherwise)
+  int device = 0;
+  if (hipGetDevice(&device) == hipSuccess) {
+    const auto& noted = g_devices[device].noted;
+    auto known = noted.find(Key(KIND_RESIDUAL + KINDS * g_kernels, rows_key(KIND_RESIDUAL, M), N, K, Q3_BF16));
+    if (known != noted.end()) return residual_chunks(known->second, N);
+  }
+  return residual_chunks(fused_by_rule(KIND_RESIDUAL, M, N, K), N);
 }
 
 extern "C" int q3_tiles_residual(const void* x, const void* w, int M, int N, int K, float* residual,
@@ -693,16 +737,28 @@ extern "C" int q3_tiles_residual(const void* x, const void* w, int M, int N, int
   int status = ready_device(d, stream);
   if (status) return status;
   Choice c;
-  // the tuner times the products alone (the tiled kernel's partial products; the other product into `values`,
-  // which the real run overwrites): each way has one small kernel more, and the residual is not touched
+  // the tuner times the products into `values`, which the real run overwrites, and leaves the residual alone: for the small kernel
+  // behind the tiled kernel's partial products, and for the norm's own behind the library's product, the former is run over the
+  // staging buffer (where that and `sums` are large enough)
+  auto second = [&](int shares) {
+    if ((size_t)M * N * sizeof(float) > STAGING_BYTES || chunks < chunks_of(tiles::CHUNK_COLUMNS, N)) return 0;
+    return add_into(d.partials, shares, d.staging, norm_weight, norm_weight_dtype, values, sums, sums_stride, M, N, stream);
+  };
   status = choose_fused(
       d, KIND_RESIDUAL, M, N, K, stream,
       [&](int config, int splits) {
+        if (config >= GROUPS_FIRST)
+          return groups::scaled(config - GROUPS_FIRST, false, Q3_BF16, x, w, values, M, N, K, stream, tiles::RowScale());
         if ((size_t)splits * M * N * sizeof(float) > PARTIALS_BYTES) return Q3_ERR_UNSUPPORTED;
-        return tiles::launch<bf16_t, tiles::EPI_PLAIN>(config, x, w, values, M, N, K, stream, splits, d.partials,
-                                                       tiles::RowScale(), true);
+        const int launched = tiles::launch<bf16_t, tiles::EPI_PLAIN>(config, x, w, values, M, N, K, stream, splits, d.partials,
+                                                                     tiles::RowScale(), true);
+        return launched ? launched : second(splits);
       },
-      [&]() { return product(d, x, w, values, M, N, K, Q3_BF16, stream); }, c);
+      [&]() {
+        const int run = product(d, x, w, values, M, N, K, Q3_BF16, stream);
+        return run ? run : second(1);
+      },
+      c);
   if (status) return status;
   if (c.own == LIBRARY || chunks != residual_chunks(c, N)) return Q3_DECLINED;
   if (c.own >= GROUPS_FIRST) {
@@ -719,14 +775,7 @@ extern "C" int q3_tiles_residual(const void* x, const void* w, int M, int N, int
   status = tiles::launch<bf16_t, tiles::EPI_PLAIN>(c.own, x, w, values, M, N, K, stream, c.splits, d.partials,
                                                    tiles::RowScale(), true, &used);
   if (status) return status;
-  const dim3 grid(chunks, M);
-  if (norm_weight_dtype == Q3_F32)
-    hipLaunchKernelGGL(tiles::tiles_residual_kernel<float>, grid, dim3(256), 0, stream, d.partials, used, residual,
-                       (const float*)norm_weight, (bf16_t*)values, sums, sums_stride, M, N);
-  else
-    hipLaunchKernelGGL(tiles::tiles_residual_kernel<bf16_t>, grid, dim3(256), 0, stream, d.partials, used, residual,
-                       (const bf16_t*)norm_weight, (bf16_t*)values, sums, sums_stride, M, N);
-  return q3_launch_status();
+  return add_into(d.partials, used, residual, norm_weight, norm_weight_dtype, values, sums, sums_stride, M, N, stream);
 }
 
 // A product of 17 to 96 rows (and a gate/up product of 9 to 16) by the weight-streaming kernel of gemm_stream.h, from the tile-ordered copy `wt` of
@@ -860,14 +909,24 @@ extern "C" int q3_matmul_set_kernels(int mode) {
 }
 
 // The table: `kind` 0 a plain product, 1 a product whose rows still lack their norm's division, 2 the same with
-// the SwiGLU activation, 3 a product that is added into the residual stream; `rows` as q3_matmul_rows_key
-// rounds them; `own` >= 0: the hand-written kernel's tile shape with `splits` shares of K; own < 0: the
-// library's candidate number `library` (for kind 3: the caller's plain product and separate norm).
+// the SwiGLU activation, 3 a product that is added into the residual stream, 4 a plain product of a size that gemm_rounds.hip takes
+// (q3_matmul_plain_kind); `rows` as q3_matmul_rows_key rounds them; `own` >= 0: the tiled kernel's tile shape with `splits` shares of
+// K, or as q3_matmul_plan and q3_matmul_fused_plan give it, from 16 on (kinds 1 to 3) gemm_groups.hip's, from 32 on (kind 4)
+// gemm_rounds.hip's; own < 0: the library's candidate number `library` (for kind 3: the caller's plain product and separate norm).
 extern "C" int q3_matmul_rows_key(int kind, int M) { return rows_key(kind, M); }
 
+// Under which kind a plain product of this size is filed, its operands at multiples of sixteen bytes.
+extern "C" int q3_matmul_plain_kind(int M, int N, int K, int out_dtype) {
+  std::lock_guard<std::mutex> hold(g_lock);
+  return round_height(KIND_PLAIN, M, N, K, out_dtype, true) ? KIND_ROUND : KIND_PLAIN;
+}
+
 extern "C" int q3_matmul_table_add(int kind, int rows, int N, int K, int out_dtype, int library, int own, int splits) {
-  if (kind < KIND_PLAIN || kind > KIND_RESIDUAL || rows < 1 || N < 1 || K < 1) return Q3_ERR_BAD_ARGUMENT;
-  if (library < 0 || library >= MAX_CANDIDATES || own >= tiles::NUM_CONFIGS || splits < 1 || splits > 64)
+  if (kind < KIND_PLAIN || kind >= KINDS || rows < 1 || N < 1 || K < 1) return Q3_ERR_BAD_ARGUMENT;
+  const bool of_groups = own >= GROUPS_FIRST && own < GROUPS_FIRST + groups::NUM_SHAPES && kind != KIND_PLAIN && kind != KIND_ROUND;
+  const bool of_rounds = own >= ROUNDS_FIRST + rounds::LEAST && own <= ROUNDS_FIRST + rounds::MOST && kind == KIND_ROUND;
+  if (library < 0 || library >= MAX_CANDIDATES || splits < 1 || splits > ((of_groups || of_rounds) ? 1 : 64) ||
+      !(own < tiles::NUM_CONFIGS || of_groups || of_rounds))
     return Q3_ERR_BAD_ARGUMENT;
   std::lock_guard<std::mutex> hold(g_lock);
   Choice c;
@@ -920,7 +979,7 @@ extern "C" int q3_matmul_fused_plan(int kind, int M, int N, int K, int* info) {
     if (hipGetDevice(&device) != hipSuccess) return 0;
     auto d = g_devices.find(device);
     if (d == g_devices.end()) return 0;
-    auto known = d->second.noted.find(Key(kind + 4 * g_kernels, rows_key(kind, M), N, K, Q3_BF16));
+    auto known = d->second.noted.find(Key(kind + KINDS * g_kernels, rows_key(kind, M), N, K, Q3_BF16));
     if (known == d->second.noted.end()) return 0;
     c = known->second;
   } else {

@@ -71,6 +71,7 @@ __all__ = [
     "matmul_table",
     "matmul_tuner",
     "matmul_rows_key",
+    "matmul_plain_kind",
     "matmul_fused_plan",
     "gemm_tiles",
     "gemm_tiles_configs",
@@ -137,7 +138,7 @@ def _check(status, what):
         raise RuntimeError("%s failed: HIP error %d" % (what, status))
 
 
-_KINDS = {"plain": 0, "scaled": 1, "scaled_swiglu": 2, "residual": 3}
+_KINDS = {"plain": 0, "scaled": 1, "scaled_swiglu": 2, "residual": 3, "plain_round": 4}
 TABLE_FILE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "matmul_table.json")
 _table_loaded = False
 
@@ -169,9 +170,10 @@ def matmul_init():
 
 
 def matmul_table(entries, clear=False):
-    """Load kernel choices: each entry {"kind": "plain" | "scaled" | "scaled_swiglu" | "residual",
+    """Load kernel choices: each entry {"kind": "plain" | "plain_round" | "scaled" | "scaled_swiglu" | "residual",
     "rows": rounded rows (`matmul_rows_key`), "N", "K", "out": "bfloat16" | "float32",
-    "library": the library's candidate number, or "own": tile shape and "splits": shares of K}.
+    "library": the library's candidate number, or "own": tile shape (as `matmul_plan` and
+    `matmul_fused_plan` number them) and "splits": shares of K}. Plain products are filed as `matmul_plain_kind` says.
     Sizes without an entry follow the rules of thumb. Sizes already met keep their kernel."""
     lib = _matmul()                      # the package's own table first, if it is not in yet
     if clear:
@@ -182,6 +184,13 @@ def matmul_table(entries, clear=False):
 def matmul_rows_key(kind, M):
     """The rows a table entry for `M` rows is filed under (sizes within a step of rows share one)."""
     return int(library("matmul").q3_matmul_rows_key(_KINDS[kind], int(M)))
+
+
+def matmul_plain_kind(M, N, K, out_dtype=torch.bfloat16):
+    """The kind a plain product's table entry is filed under: "plain_round" for a size that the kernel takes that covers a
+    product in one round of blocks, else "plain"."""
+    kind = library("matmul").q3_matmul_plain_kind(int(M), int(N), int(K), _DT[out_dtype])
+    return next(name for name, number in _KINDS.items() if number == kind)
 
 
 def matmul_tuner(on):

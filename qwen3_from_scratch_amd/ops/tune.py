@@ -5,7 +5,7 @@
         --rows 24,32,48,64,96,128,256,512,576,1024,2048 > table.json
 
 For each row count and each of the layer's products (q/k/v, output, gate/up, down) the
-tuner times the vendor library's candidates and the hand-written kernel's tile shapes on
+tuner times the vendor library's candidates and the hand-written kernels' tile shapes on
 random operands, with cold caches, and the fastest is written down as a table entry; row
 counts at which a product may carry a norm (from 17 to 128, or 640 for a small weight:
 `ops.fused_rows_take`) also get entries for that. The output is
@@ -63,9 +63,10 @@ def tune_layer(hidden, heads, kv_heads, head_dim, intermediate, rows_list, seed=
                 ops.linear(x, w, out_dtype=out_dtype)
                 p = ops.matmul_plan(M, N, K, out_dtype)
                 if p is not None:
-                    rows = ops.matmul_rows_key("plain", M)
-                    entries[("plain", rows, N, K, out_name)] = _entry(
-                        "plain", rows, N, K, out_name, dict(own=p[4], splits=p[5], library=p[6], us=p[3]))
+                    kind = ops.matmul_plain_kind(M, N, K, out_dtype)
+                    rows = ops.matmul_rows_key(kind, M)
+                    entries[(kind, rows, N, K, out_name)] = _entry(
+                        kind, rows, N, K, out_name, dict(own=p[4], splits=p[5], library=p[6], us=p[3]))
                 if name != "head" and ops.fused_rows_take(w, M):
                     residual = torch.zeros((M, N), dtype=torch.float32, device=device)
                     if name in ("o", "down") and N == hidden:

@@ -87,3 +87,43 @@ def test_a_table_entry_for_one_of_the_two_epilogues(rules_alone, kind, other):
     assert ops._groups_before_few(w, M, unscaled, other == "scaled_swiglu")
     for product in products.values():
         assert torch.equal(product(x, sums)[:16], product(x[:16].contiguous(), sums[:, :16].contiguous()))
+
+
+def test_the_tuner_finds_these_kernels_and_a_table_names_them(rules_alone):
+    """Where they are the fastest by far the contest ends with them, what it found goes into a table, and a table that says
+    otherwise is followed, plain products of one round of tiles among them."""
+    from qwen3_from_scratch_amd.ops import tune
+
+    ops = rules_alone
+    ops.matmul_candidates(1)
+    try:
+        small, large = tune.tune_layer(1024, 16, 8, 128, 4096, [201]), tune.tune_layer(4096, 32, 8, 128, 1024, [535])
+    finally:
+        ops.matmul_candidates(16)
+    found = {(e["kind"], e["N"], e["K"]): e for e in small + large}
+    carrying = [("scaled", 4096, 1024), ("scaled_swiglu", 8192, 1024), ("residual", 1024, 2048), ("residual", 1024, 4096)]
+    rules = [ops.matmul_fused_plan(kind, 201, N, K) for kind, N, K in carrying]
+    assert [(found[c].get("own"), found[c].get("splits")) for c in carrying] == rules and all(own >= 16 for own, _ in rules)
+    assert found["plain_round", 4096, 4096]["own"] == 32 + 9 and ("plain", 4096, 4096) not in found
+
+    x, w = _rand((535, 4096), torch.bfloat16, 31), _rand((4096, 4096), torch.bfloat16, 32, scale=0.05)
+    want = x.double() @ w.double().T
+    others = [dict(e, **other) for e, other in ((found["scaled", 4096, 1024], dict(own=18)),
+                                               (dict(found["plain_round", 4096, 4096], library=0), dict(own=-1)))]
+    for table, scaled, plain in ((list(found.values()), rules[0][0], 32 + 9), (others, 18, -1)):
+        ops.matmul_table(table, clear=True)
+        _forget_choices(ops)
+        assert ops.matmul_fused_plan("scaled", 201, 4096, 1024) == (scaled, 1)
+        torch.testing.assert_close(ops.linear(x, w).double(), want, rtol=1.6e-2, atol=5e-2)
+        assert ops.matmul_plan(535, 4096, 4096)[4] == plain
+    # neighbours of the same step of rows take the height that is theirs; a plain entry does not speak for them
+    size = {"rows": 352, "N": 5120, "K": 5120}
+    ops.matmul_table([dict(size, kind="plain_round", own=32 + 7), dict(size, kind="plain", library=0)], clear=True)
+    _forget_choices(ops)
+    w = _rand((5120, 5120), torch.bfloat16, 33, scale=0.05)
+    for M, height in ((330, 7), (340, 8)):
+        ops.linear(_rand((M, 5120), torch.bfloat16, 34), w)
+        assert ops.matmul_plan(M, 5120, 5120)[4] == 32 + height
+    for entry in (dict(own=22), dict(own=18, splits=2), dict(own=42)):
+        with pytest.raises(RuntimeError):
+            ops.matmul_table([dict({"kind": "scaled", "rows": 208, "N": 4096, "K": 1024}, **entry)])
