@@ -19,6 +19,7 @@ struct Residual {
 // The tiles on offer, each twice the one before: rows, columns. K in four up to 64 x 32, in two up to 64 x 128.
 constexpr int NUM_SHAPES = 6;
 constexpr int SHAPES[NUM_SHAPES][2] = {{32, 16}, {32, 32}, {64, 32}, {64, 64}, {64, 128}, {128, 128}};
+inline bool in_four(int shape) { return shape <= 2; }
 
 // The smallest tile that covers the product in one round of the 256 CUs, a block a CU; -1 if none does. (As each is twice
 // the one before, more than half of the CUs have a block where it is not the smallest.) Two rounds of a smaller tile lose: 336 rows of 4,096 x 1,024
@@ -34,7 +35,7 @@ inline int shape_for(int M, int N, int K) {
 // Whether a product's sums over k are the few-row kernel's to the bit: with K in four, its shares of K are these (see
 // launch_skinny in gemm.hip: up to eight wavefronts with 128 k or more each, in steps of 256).
 inline bool shares_of_few_rows(int shape, int N, int K) {
-  if (shape > 2 || (N + 15) / 16 < 256) return false;
+  if (!in_four(shape) || (N + 15) / 16 < 256) return false;
   int kw = 1;
   while (kw < 8 && K / (kw * 2) >= 128) kw *= 2;
   return ((K + kw - 1) / kw + 255) / 256 * 256 == (K / tiles::BK + 3) / 4 * tiles::BK;

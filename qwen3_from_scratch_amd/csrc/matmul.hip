@@ -257,11 +257,7 @@ Choice plain_by_rule(int M, int N, int K) {
   return Choice();   // the library's first candidate
 }
 
-// The products that carry a norm. A weight of up to 18 MB, or a product of more than 96 rows in 128 x 128 tiles: the kernel of
-// gemm_groups.hip where it covers the product in one round. (A larger weight's few rows are bound by its passage, which many small tiles with
-// their own rows of x beside it slow down: 24 and 64 rows of 6,144 x 4,096 16.6 and 20.8 us there, 15.9 and 17.8 in 64 x 128
-// tiles; 64 of 4,096 x 12,288 34.8 and 28.2. 128 rows of 24,576 x 4,096 with SwiGLU, 192 tiles of 128 x 128, 58.8 and 74.3, the
-// library's with a kernel behind it; up to 96 rows the weight-streaming kernel has it.)
+// The tiled kernel's shape and shares of K for a product that carries a norm, or the library.
 // 17 to 128 rows: 64 x 128 tiles in five stages (with K shared out they need
 // the fewest shares to fill the chip), unless the tiles come to a little more than a whole number of rounds over
 // the 256 CUs and leave most of them idle in the last one: then the library's product with the norm's work in a
@@ -269,21 +265,9 @@ Choice plain_by_rule(int M, int N, int K) {
 // 129 to 640 rows (small weights): 64 x 128 tiles while there is at most one a CU (up to 256), in three stages, two
 // blocks of which share a CU where K is shared out (in five, one block a CU, where more than 256 rows share K out),
 // then 128 x 128, one block a CU, while that is one round, then the library. The products alone, us, three stages / five /
-// 128 x 128 / library: 201 rows of 4,096 x 1,024 10.5 / 11.1 / 14.0 / 12.0, of 8,192 x 1,024 11.1 / 11.7 / 14.4 / 13.5, of
-// 1,024 x 4,096 in eight shares 13.3 / 13.8 / 16.5; 400 rows of the last, in four, 17.4 / 15.7 / 16.7; 400 of 8,192 x 1,024
-// (448 tiles of 64 x 128, less than two a CU) 16.4 / 20.6 / 15.5 / 15.5; 532 of it (320 tiles of 128 x 128) 23.3 / 29.4 /
-// 20.9 / 17.4.
-Choice fused_by_rule(int kind, int M, int N, int K) {
+// 128 x 128: 201 rows of 1,024 x 4,096 in eight shares 13.3 / 13.8 / 16.5; 400 rows of it, in four, 17.4 / 15.7 / 16.7.
+Choice tiled_by_rule(int kind, int M, int N, int K) {
   Choice c;
-  if (g_kernels == KERNELS_LIBRARY) return c;
-  if (g_kernels == KERNELS_BOTH) {
-    const int shape = groups::shape_for(M, N, K);
-    const bool small = (size_t)N * K * 2 <= GROUPS_MOST_WEIGHT_BYTES;
-    if (shape >= 0 && (small || (kind != KIND_RESIDUAL && M > 96 && shape == groups::NUM_SHAPES - 1))) {
-      c.own = GROUPS_FIRST + shape;
-      return c;
-    }
-  }
   if (M > 128) {
     // (a residual's product always goes through partial products; where not even one share's fit, it is declined)
     if (kind == KIND_RESIDUAL && (size_t)M * N * sizeof(float) > PARTIALS_BYTES) return c;
@@ -307,6 +291,42 @@ Choice fused_by_rule(int kind, int M, int N, int K) {
     if (tiles_n < rounds * 256 * 7 / 10) return Choice();
   }
   return c;
+}
+
+// The products that carry a norm: the kernel of gemm_groups.hip (`shape`: the tile that covers the product in one round) or what
+// tiled_by_rule says (`c`).
+//
+// A weight of up to 18 MB goes by groups up to an inner size of 5,120, 4,096 where a block has K in fewer than four. Beyond, its one
+// pass over K costs more than the second kernel of shares over blocks, by as much as its tile is far from the 64 x 128 of those: a
+// block brings 64 k of its rows through for every stage, the other's 192 rows for a stage of its share, and 3,800 rows' worth of time
+// goes to the second kernel. Microseconds, c / groups: 640 rows of 512 x 16,384 29.5 / 48.0, 320 of 1,024 x 8,192 20.4 / 26.1, 64 of it
+// 14.8 / 16.1, 320 of 1,024 x 5,120 16.2 / 19.3, of 2,048 x 4,608 20.7 / 22.9 (these by c); 100 of 1,792 x 5,120 21.8 / 13.2, 160 of
+// 1,536 x 5,120 19.2 / 15.1, 400 of 896 x 4,864 23.1 / 14.5. (Of 412 sizes up to 16,384 k two lose, 5 and 3 %.) Up to 32 rows, which the
+// few-row kernel has wherever there is a tiled copy, are not asked: 17 of 1,536 x 5,120 11.3 / 11.1, of 1,024 x 8,192 11.9 / 14.3.
+//
+// A larger weight's few rows are bound by its passage, which many small tiles with their own rows of x beside it slow down: 24 and 64
+// rows of 6,144 x 4,096 16.6 and 20.8 us there, 15.9 and 17.8 in 64 x 128 tiles; 64 of 4,096 x 12,288 34.8 and 28.2. From 97 rows
+// on (up to 96 the weight-streaming kernel has them) one round of 128 x 128 tiles wins where it leaves few CUs idle, 180 tiles or more, or
+// the inner size is short: 128 rows with SwiGLU of 23,552 x 4,096, 5,120 and 8,192 76.7 / 56.9, 97.5 / 69.9 and 135.8 / 105.4, of
+// 16,512, 18,432 and 20,480 x 2,048 32.6 / 28.7, 34.2 / 29.5 and 32.5 / 30.6; but of 22,528 (176 tiles) x 4,096, 5,120
+// and 8,192 53.4 / 55.6, 61.1 / 68.3 and 98.6 / 105.9, of 18,432 x 2,560 36.1 / 38.8.
+Choice fused_by_rule(int kind, int M, int N, int K) {
+  if (g_kernels == KERNELS_LIBRARY) return Choice();
+  const Choice c = tiled_by_rule(kind, M, N, K);
+  const int shape = g_kernels == KERNELS_BOTH ? groups::shape_for(M, N, K) : -1;
+  if (shape < 0) return c;
+  const int rows = groups::SHAPES[shape][0], columns = groups::SHAPES[shape][1];
+  bool wins;
+  if ((size_t)N * K * 2 <= GROUPS_MOST_WEIGHT_BYTES) {
+    wins = M <= 32 || (K < 5120 && (K <= 4096 || groups::in_four(shape)));
+    if (!wins && c.own >= 0) wins = K / tiles::BK * (rows + columns) <= (K / tiles::BK + c.splits - 1) / c.splits * 192 + 3800;
+  } else {
+    wins = kind != KIND_RESIDUAL && M > 96 && shape == groups::NUM_SHAPES - 1 && (K <= 2048 || (N + columns - 1) / columns >= 180);
+  }
+  if (!wins) return c;
+  Choice by_groups;
+  by_groups.own = GROUPS_FIRST + shape;
+  return by_groups;
 }
 
 // The height of gemm_rounds.hip's tile for a plain product, 0 where it is not its; `aligned`: the operands lie at multiples of sixteen

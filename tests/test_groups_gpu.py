@@ -127,3 +127,26 @@ def test_the_tuner_finds_these_kernels_and_a_table_names_them(rules_alone):
     for entry in (dict(own=22), dict(own=18, splits=2), dict(own=42)):
         with pytest.raises(RuntimeError):
             ops.matmul_table([dict({"kind": "scaled", "rows": 208, "N": 4096, "K": 1024}, **entry)])
+
+
+# long inner sizes of small weights, large weights that leave many CUs idle, and their neighbours on the other side of either line
+@pytest.mark.parametrize("kind,M,N,K,own", [
+    ("residual", 320, 1024, 8192, 8), ("residual", 320, 1024, 4864, 18), ("scaled", 640, 512, 16384, 8), ("scaled", 64, 1024, 8192, 8),
+    ("scaled", 100, 1792, 5120, 17), ("scaled", 200, 768, 8192, 5), ("residual", 320, 2048, 4608, 8), ("residual", 320, 2048, 4096, 19), ("residual", 400, 896, 4864, 18),
+    ("scaled_swiglu", 128, 22528, 4096, -1), ("scaled_swiglu", 128, 23552, 4096, 21), ("scaled", 128, 18432, 5120, -1),
+    ("scaled", 97, 18432, 2048, 21), ("scaled", 97, 18432, 2112, -1), ("residual", 128, 24576, 4096, 8)])
+def test_where_another_kernel_is_the_faster_one(rules_alone, kind, M, N, K, own):
+    ops = rules_alone
+    assert ops.matmul_fused_plan(kind, M, N, K)[0] == own
+    x, w = _rand((M, K), torch.bfloat16, 91), _rand((N, K), torch.bfloat16, 92, scale=0.05)
+    exact = x.double() @ w.double().T
+    if kind == "residual":
+        stream = torch.zeros(M, N, device="cuda")
+        assert ops.linear_residual_norm(x, w, None, stream, torch.ones(N, device="cuda")) is not None
+        got = stream
+    else:
+        sums = torch.full((1, ops.sums_stride(M)), float(K), device="cuda")
+        got = ops.linear(x, w, unscaled=(sums, 0.0, K)) if kind == "scaled" else ops.linear_swiglu(x, w, unscaled=(sums, 0.0, K))
+        if kind == "scaled_swiglu":
+            exact = torch.nn.functional.silu(exact[:, ::2]) * exact[:, 1::2]
+    torch.testing.assert_close(got.double(), exact, rtol=1.6e-2, atol=0.1)
