@@ -863,7 +863,7 @@ __global__ __launch_bounds__(256) void gemm_f32_few_rows_kernel(const float* __r
 // results each: `workspace` as q3_decode_attention leaves it, `heads` query heads over `kv_heads` of `dim` (64 or 128). K = heads dim, a
 // multiple of 256; N of 16; M <= 16; at most 16 splits. q3_linear_of_splits_most: into how many splits attention that would be cut into `splits`
 // is best cut for it, or 0 where the sizes are not its or the partial results so many that reading them in every block costs more
-// than the merge's launch: attention and product, microseconds, merged before / inside, 128 KB of partial results 15.2 / 13.5 (K = 2,048, 1 row),
+// than the merge's launch (few rows of few numbers may still be merged faster beforehand, which the caller decides): attention and product, microseconds, merged before / inside, 128 KB of partial results 15.2 / 13.5 (K = 2,048, 1 row),
 // 16.2 / 14.6 (2 rows of 8 parts), 22.9 / 22.1 (K = 4,096, 8 parts); 192 KB 15.4 / 15.6 and 22.3 / 23.2; 256 KB 15.3 / 15.8 and 21.3 / 22.5.
 // Thirty-two parts (from 4,096 keys on) become sixteen: a request over 4,200 keys 18.7 merged before, 17.3 so, over 6,000 19.7 and 18.6, over
 // 8,100 20.6 and 20.7, over 30,000 35.7 and 38.4 (the caller's line is at 8,192).

@@ -31,6 +31,7 @@ __all__ = [
     "paged_attention",
     "decode_attention",
     "decode_attention_takes",
+    "split_rows_pay",
     "swiglu",
     "gated_act",
     "layernorm_addend",
@@ -1758,6 +1759,18 @@ def _splits(B, Hkv, max_kv_len):
     elif (max_kv_len >= 2560 and 128 < pairs <= 160) or (max_kv_len >= 1536 and 256 < pairs <= 320):
         splits = 3
     return splits
+
+
+def split_rows_pay(rows, num_q_heads, num_kv_heads, head_dim, max_kv_len):
+    """Whether a decoding step's attention is best left unmerged for the product that reads it (`decode_attention` with
+    `residual_width`): a wavefront of that product forms its rows 256 numbers at a time, eight parts a step, one step after the other, and the
+    merge's launch is as long as three. Attention and product, microseconds, merged before / inside: one step (8 heads of
+    128 over 300 keys, one request) 14.5 / 11.5, two (16 heads, 1,100 keys) 15.2 / 13.5, three (8 heads, three requests over 300) 16.0 /
+    15.1; four 16.7 / 17.5 (16 heads, four over 300) and 33.3 / 38.3 (64 heads, one), but two requests of sixteen parts level or
+    up to a tenth faster; six 16.3 / 18.9, eight 16.3 / 21.4, sixteen 15.8 / 28.9."""
+    parts, pieces = min(_splits(rows, num_kv_heads, max_kv_len), 16), -(-num_q_heads * head_dim // 256)
+    runs, turns = -(-pieces // min(8, max(1, pieces))), -(-parts // 8)
+    return parts > 1 and (runs * rows * turns <= 3 or (rows, turns, runs) == (2, 2, 1))
 
 
 def decode_attention_takes(num_q_heads, num_kv_heads, head_dim, page_size, dtype, rotary_dim=0):

@@ -113,11 +113,13 @@ class PagedAttention(Part):
         if batch.max_q_len == 1 and qkv.shape[0] == batch.kv_lens.shape[0] and ops.decode_attention_takes(
                 Hq, Hkv, D, keys.shape[2], qkv.dtype, 0 if table is None else table.shape[1]):
             # every sequence brings one token: preparation, cache write and attention are one kernel
+            unmerged = (sink is not None and self.out.tiled is not None
+                        and ops.split_rows_pay(qkv.shape[0], Hq, Hkv, D, batch.max_kv_len))
             o = ops.decode_attention(
                 qkv, Hq, Hkv, D, keys, values, cache.block_table, batch.cu_seqlens_q, batch.kv_lens,
                 batch.max_kv_len, self.scale, window=self.window, q_weight=self.q_weight, k_weight=self.k_weight,
                 eps=self.qk_norm_eps, table=table, store=cache.writes,
-                residual_width=self.hidden_size if sink is not None and self.out.tiled is not None else 0)
+                residual_width=self.hidden_size if unmerged else 0)
             return self.out.forward(o) if sink is None else self.out.forward_into(o, sink)
         ops.qk_norm_rope_store(
             qkv, Hq, Hkv, D, batch.positions, batch.seq_index,

@@ -24,3 +24,12 @@ def test_splits_stay_in_range(keys):
     (48, 7200, 4), (48, 32000, 4), (64, 8192, 1)])
 def test_splits_that_were_faster(requests, keys, parts):
     assert ops._splits(requests, 8, keys) == parts
+
+
+@pytest.mark.parametrize("rows,heads,kv_heads,dim,keys,pays", [
+    (1, 16, 8, 128, 1100, True), (1, 16, 8, 128, 5000, True), (1, 32, 8, 128, 300, True), (2, 16, 8, 128, 450, True),
+    (3, 8, 1, 128, 300, True), (2, 8, 1, 128, 1100, True), (2, 4, 4, 64, 3000, True), (4, 16, 8, 128, 300, False),
+    (2, 32, 8, 128, 300, False), (1, 64, 8, 128, 300, False), (3, 4, 4, 64, 700, False), (6, 16, 16, 64, 700, False),
+    (8, 8, 1, 128, 300, False), (16, 4, 4, 64, 1800, False), (1, 16, 8, 128, 200, False), (40, 16, 8, 128, 1000, False)])
+def test_attention_that_is_best_merged_inside_the_product(rows, heads, kv_heads, dim, keys, pays):
+    assert ops.split_rows_pay(rows, heads, kv_heads, dim, keys) == pays
