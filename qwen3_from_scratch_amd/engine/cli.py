@@ -48,7 +48,7 @@ def main(argv=None):
                    metavar="BOOL", help="requests take over cached blocks of a prefix they share (default true)")
     p.add_argument("--tiled_weights", type=lambda v: str(v).lower() in ("1", "true", "yes", "on"), default=None,
                    metavar="BOOL", help="keep the second, tile-ordered copy of the matrices (default true: faster "
-                                        "decoding, twice the memory)")
+                                        "decoding, twice the memory; in float32 a bfloat16 copy, half the memory more)")
     p.add_argument("--log_interval", type=int, default=0)
     p.add_argument("--write_random", metavar="DIR", help="write a random-weights model folder and exit")
     p.add_argument("--from_config", metavar="JSON", help="config.json for --write_random")

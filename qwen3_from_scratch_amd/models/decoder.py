@@ -5,6 +5,7 @@ interfaces, never by architecture."""
 import torch
 
 from ..parts.base import UnscaledRows, build_part
+from ..parts.linear import copy_float32_matrices
 from ..weights.checkpoint import check_tensors
 from .layer_run import layer_runs
 
@@ -129,6 +130,7 @@ class DecoderModel:
         with torch.no_grad():
             for part in self.parts():
                 part.load(fetch)
+            copy_float32_matrices(self.parts())
         self.runs = layer_runs(self)
         return self
 

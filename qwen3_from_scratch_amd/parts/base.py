@@ -21,7 +21,8 @@ class Precision:
     cache share `act`; the residual stream and logits are float32. `tiled`:
     keep a second, tile-ordered copy of every bfloat16 matrix for the few-row
     product kernel (decoding); it costs the matrices' memory once more. And a bfloat16
-    copy of every float32 matrix that bfloat16 holds exactly, for half its memory more."""
+    copy of the float32 matrices that bfloat16 holds exactly, for half their memory more, as
+    far as a quarter of what is free behind the loading holds them."""
 
     act: torch.dtype
     tiled: bool = True

@@ -4,7 +4,41 @@ order the few-row product kernel streams it, of float32 in bfloat16 where that l
 import torch
 
 from .. import ops
-from .base import UnscaledRows
+from .base import Part, UnscaledRows
+
+COPIES_MOST = 4                 # float32 matrices' bfloat16 copies take a quarter at most of the memory that is free
+
+
+def free_memory(device):
+    """Bytes of the device that nobody holds, what PyTorch keeps for later among them."""
+    return (torch.cuda.mem_get_info(device)[0] + torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device))
+
+
+def _matrices(held, seen):
+    """Every LinearWeight that a part, or a list of parts, holds, once each, in their order."""
+    if id(held) in seen:
+        return
+    seen.add(id(held))
+    if isinstance(held, LinearWeight):
+        yield held
+    elif isinstance(held, (Part, list, tuple, dict)):
+        inner = vars(held).values() if isinstance(held, Part) else held.values() if isinstance(held, dict) else held
+        for value in inner:
+            yield from _matrices(value, seen)
+
+
+def copy_float32_matrices(parts):
+    """Give the float32 matrices of `parts`, one after the other, the bfloat16 copies that `LinearWeight` multiplies with, once
+    all are loaded: so that whatever fits without them fits with them, and most of what is left stays the cache's."""
+    matrices = [m for m in _matrices(list(parts), set()) if m.wants_copy]
+    if not matrices:
+        return
+    room = free_memory(matrices[0].weight.device) // COPIES_MOST
+    for m in matrices:
+        size = 2 * m.weight.numel()
+        if size <= room:
+            m.narrow = ops.narrow_weight(m.weight)
+            room -= size if m.narrow is not None else 0
 
 
 def joined_rows(matrices, multiple=16):
@@ -26,13 +60,14 @@ class LinearWeight:
     it, a tile-ordered bfloat16 copy serves steps with few rows (16, or 32 or 64
     for a small weight), where every weight is read once and the order in memory
     decides the bandwidth. The copy doubles the weight's memory. A float32 weight that
-    bfloat16 holds exactly has a bfloat16 copy instead, half its memory more: the products
+    bfloat16 holds exactly may have a bfloat16 copy instead (`copy_float32_matrices`), half its memory more: the products
     then read half as much and run on the bfloat16 matrix cores, in float32 precision."""
 
     def __init__(self, weight, precision):
         self.weight = weight
         self.tiled = ops.tile_weight(weight) if precision.tiled else None
-        self.narrow = ops.narrow_weight(weight) if precision.tiled else None
+        self.narrow = None
+        self.wants_copy = precision.tiled and weight.is_cuda and weight.dtype == torch.float32
         if weight.is_cuda and weight.dtype == torch.bfloat16:
             ops.matmul_init()          # the many-row products' buffers: now, not inside a step
 

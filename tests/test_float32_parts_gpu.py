@@ -77,3 +77,30 @@ def test_what_has_a_copy():
     assert ops.narrow_weight(w[:, :96].contiguous()) is None
     with pytest.raises(ValueError):
         ops.linear(_rand((3, 128), torch.float32, 87), w, narrow=ops.narrow_weight(w[:39]))
+
+
+def test_copies_leave_room(monkeypatch):
+    """A model's copies are made when everything is loaded and end where a quarter of what is free is theirs; the products of the
+    matrices that have none are the float32 kernels', and no model has to have them."""
+    from qwen3_from_scratch_amd.config import ModelConfig
+    from qwen3_from_scratch_amd.engine import ModelRunner, StepEntry, random_model
+    from qwen3_from_scratch_amd.parts import linear
+
+    config = ModelConfig.from_dict(dict(
+        architectures=["Qwen3ForCausalLM"], vocab_size=512, hidden_size=256, hidden_act="silu", num_hidden_layers=2,
+        max_position_embeddings=512, num_attention_heads=4, num_key_value_heads=2, head_dim=64, intermediate_size=512,
+        rms_norm_eps=1e-6, rope_theta=1e6, tie_word_embeddings=False))
+    first = 2 * (512 * 256 + 256 * 256)              # bytes of the copies of the first layer's attention
+    held, logits = [], []
+    for free, tiled in ((1 << 40, True), (4 * first, True), (0, True), (1 << 40, False)):
+        asked = []
+        monkeypatch.setattr(linear, "free_memory", lambda device: asked.append(torch.cuda.memory_allocated()) or free)
+        model = random_model(config, dtype="float32", device="cuda:0", seed=5, tiled_weights=tiled)
+        matrices = [m for m in linear._matrices(list(model.parts()), set())]
+        held.append([m.narrow is not None for m in matrices])
+        assert len(asked) == tiled and all(at >= sum(4 * m.weight.numel() for m in matrices) for at in asked)
+        logits.append(ModelRunner(model, 16, 32, max_requests=2).step([StepEntry("a", list(range(40)), [39])]).clone())
+    assert held == [[True] * 9, [True] * 2 + [False] * 7, [False] * 9, [False] * 9]
+    for other in logits[1:]:
+        torch.testing.assert_close(other, logits[0], rtol=1e-4, atol=1e-5)
+    assert torch.equal(logits[2], logits[3])
