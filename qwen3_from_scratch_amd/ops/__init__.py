@@ -1930,7 +1930,8 @@ def _groups_before_few(weight, M, unscaled, swiglu=False):
     takes as many: 17 rows and more of a small weight of 4,096 columns or more, where both add alike (an inner size of 1,024, say),
     so that a row's bits do not change with the number of rows. There the few-row kernel, a block per 16
     columns and 16 rows, needs two rounds of blocks: 24, 32 and 64 rows of 4,096 x 1,024 6.4, 6.7 and 10.3 us, of 8,192 x 1,024
-    10.7, 11.4 and 18.5, the other kernel 5.4, 5.6, 6.1 and 6.9, 7.0, 8.3; 24 rows of 1,024 x 2,048 6.2 and 6.8."""
+    10.7, 11.4 and 18.5, the other kernel 5.4, 5.6, 6.1 and 6.9, 7.0, 8.3; 24 rows of 1,024 x 2,048 6.2 and 6.8. (Its copies to
+    shared memory need rows at multiples of 16 bytes, the few-row kernel's loads do not: its callers look.)"""
     return (unscaled is not None and M > FEW_ROWS and weight.shape[0] >= GROUPS_LEAST_COLUMNS and fused_rows_take(weight, M)
             and _matmul().q3_groups_as_few(M, weight.shape[0], weight.shape[1], 1 if swiglu else 0))
 
@@ -2076,7 +2077,8 @@ def linear(x, weight, out_dtype=None, out=None, tiled=None, unscaled=None, narro
     if unscaled is None and _narrow_ok(narrow, x, weight) and out.data_ptr() % 16 == 0:
         _check(library("gemm").q3_linear_narrow(_ptr(x), _ptr(narrow), _ptr(out), M, N, K, 0, _stream()), "linear")
         return out
-    if M and x.dtype == torch.bfloat16 and _tiled_ok(tiled, weight, M) and not _groups_before_few(weight, M, unscaled):
+    if M and x.dtype == torch.bfloat16 and _tiled_ok(tiled, weight, M) and not (
+            _groups_before_few(weight, M, unscaled) and x.data_ptr() % 16 == 0):
         sums, sums_rows, eps, width, stride = _row_sums_args(unscaled, M, K)
         _check(library("gemm").q3_linear_tiled(
             _ptr(x), _ptr(tiled), _ptr(out), M, N, K, _DT[out_dtype], 0, sums, sums_rows, eps, width,
@@ -2160,7 +2162,8 @@ def linear_swiglu(x, weight, tiled=None, unscaled=None, kind="silu", narrow=None
         out = torch.empty((M, N // 2), dtype=x.dtype, device=x.device)
         if _stream_product(x, weight, tiled, out, True, unscaled, "linear_swiglu", kind):
             return out
-    if M and x.dtype == torch.bfloat16 and _tiled_ok(tiled, weight, M) and not (kind == "silu" and _groups_before_few(weight, M, unscaled, True)):
+    if M and x.dtype == torch.bfloat16 and _tiled_ok(tiled, weight, M) and not (
+            kind == "silu" and _groups_before_few(weight, M, unscaled, True) and x.data_ptr() % 16 == 0):
         out = torch.empty((M, N // 2), dtype=x.dtype, device=x.device)
         sums, sums_rows, eps, width, stride = _row_sums_args(unscaled, M, K)
         _check(library("gemm").q3_linear_tiled(

@@ -150,3 +150,22 @@ def test_where_another_kernel_is_the_faster_one(rules_alone, kind, M, N, K, own)
         if kind == "scaled_swiglu":
             exact = torch.nn.functional.silu(exact[:, ::2]) * exact[:, 1::2]
     torch.testing.assert_close(got.double(), exact, rtol=1.6e-2, atol=0.1)
+
+
+def test_rows_off_sixteen_bytes_stay_the_few_row_kernels(monkeypatch):
+    """32 rows that begin eight bytes off a multiple of sixteen: not a kernel's that copies them sixteen bytes at a time, the same bits."""
+    ops = _ops()
+    M, N, K = 32, 4096, 1024
+    x, w = _rand((M, K), torch.bfloat16, 98), _rand((N, K), torch.bfloat16, 99, scale=0.05)
+    tiled, sums = ops.tile_weight(w), torch.rand((64, M), generator=torch.Generator().manual_seed(97)).cuda() * 32.0
+    more = dict(tiled=tiled, unscaled=(sums, 1e-5, K))
+    flat = torch.empty(M * K + 4, dtype=torch.bfloat16, device="cuda")
+    flat[4:] = x.view(-1)
+    off, want, gated = flat[4:].view(M, K), ops.linear(x, w, **more), ops.linear_swiglu(x, w, **more)
+    assert off.data_ptr() % 16 == 8
+
+    def copies(*args):
+        raise AssertionError("rows off sixteen bytes")
+
+    monkeypatch.setattr(ops, "_tiles_scaled", copies)
+    assert torch.equal(ops.linear(off, w, **more), want) and torch.equal(ops.linear_swiglu(off, w, **more), gated)
