@@ -6,15 +6,21 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-def _model(layers=5, dtype="bfloat16", head_dim=128, inner=2048):
+def _model(layers=5, dtype="bfloat16", head_dim=128, inner=2048, tiled=True, **mixer):
     from qwen3_from_scratch_amd.config import ModelConfig
-    from qwen3_from_scratch_amd.engine import random_model
+    from qwen3_from_scratch_amd.models.decoder import build_model
+    from qwen3_from_scratch_amd.parts.base import Precision
+    from qwen3_from_scratch_amd.weights import RandomWeights
 
     config = ModelConfig.from_dict(dict(
         architectures=["Qwen3ForCausalLM"], vocab_size=512, hidden_size=1024, hidden_act="silu", num_hidden_layers=layers,
         max_position_embeddings=8192, num_attention_heads=16, num_key_value_heads=8, head_dim=head_dim,
         intermediate_size=inner, rms_norm_eps=1e-6, rope_theta=1e6, tie_word_embeddings=False))
-    return random_model(config, dtype=dtype, device="cuda:0", seed=5)
+    components = {"mixer": {"name": "attention", "kwargs": mixer}} if mixer else None
+    model = build_model(config, Precision.named(dtype, tiled=tiled), "cuda:0", components=components)
+    model.load(RandomWeights(model.tensors(), seed=5, std=0.02, norm_jitter=0.1, generate_on="cuda:0"))
+    model.config = config
+    return model
 
 
 def _steps(seed, *steps):
@@ -142,3 +148,20 @@ def test_a_product_that_declines_after_all(monkeypatch, inner):
     model.observer = lambda *args: None
     for a, b in zip(got, _logits(model, steps)):
         assert float((a - b).norm() / b.norm()) < 0.02       # another rounding of one product in bfloat16 a layer
+
+
+@pytest.mark.parametrize("mixer", [dict(qk_norm=False), dict(window=90), dict(qk_norm=False, window=33, scale=0.1)])
+def test_the_same_bits_without_norms_of_the_heads_and_behind_a_window(mixer):
+    model = _model(**mixer)
+    assert sorted(model.runs) == [0, 1, 2, 3]
+    native = model.runs[0].native
+    assert native.window == mixer.get("window", 0) and (native.layers[0]["q_norm"] is None) == (mixer.get("qk_norm") is False)
+    steps = _steps(10, (("a", 65),), (("b", 200), ("a", 1)), (("a", 300), ("b", 1)))
+    got = _logits(model, steps)
+    model.observer = lambda *args: None
+    for a, b in zip(got, _logits(model, steps)):
+        assert torch.equal(a, b)
+
+
+def test_matrices_held_once_leave_no_stretch():
+    assert not _model(layers=3, tiled=False).runs

@@ -3,7 +3,6 @@
 import pytest
 import torch
 
-import torch_ops
 from test_kernels_gpu import _ops, _paged_case
 
 pytestmark = pytest.mark.gpu
@@ -28,27 +27,48 @@ def _lens(name):
     }[name]
 
 
+def _exact(q, kc, vc, bt, cu, kvl, scale, sink, cap):
+    """The attention in float64, and of every result the sum of the magnitudes that it adds."""
+    Hq, Hkv, page = q.shape[1], kc.shape[1], kc.shape[2]
+    result, size = [], []
+    for b, L in enumerate(kvl.tolist()):
+        rows = q[int(cu[b]):int(cu[b + 1])].double()
+        n, pages = rows.shape[0], bt[b, :-(-L // page)].long()
+        k = kc[pages].double().permute(1, 0, 2, 3).flatten(1, 2)[:, :L].repeat_interleave(Hq // Hkv, dim=0)
+        v = vc[pages].double().permute(1, 0, 3, 2).flatten(1, 2)[:, :L].repeat_interleave(Hq // Hkv, dim=0)
+        s = torch.matmul(rows.transpose(0, 1), k.transpose(1, 2).contiguous()) * scale
+        s = cap * torch.tanh(s / cap) if cap else s
+        s = s.masked_fill(torch.arange(L, device="cuda") > torch.arange(L - n, L, device="cuda")[:, None], float("-inf"))
+        if sink is not None:
+            s = torch.cat((s, sink.double()[:, None, None].expand(Hq, n, 1)), dim=2)
+        w = torch.softmax(s, dim=2)[:, :, :L]
+        result.append(torch.matmul(w, v).transpose(0, 1).flatten(1))
+        size.append(torch.matmul(w, v.abs()).transpose(0, 1).flatten(1))
+    return torch.cat(result), torch.cat(size)
+
+
+def _bound(got, size):
+    """A bfloat16 result (eight significant bits: half a unit is 2^-8 of a number at most) is off by its own rounding and by that of
+    the probabilities in the second product, 2^-8 of the sum of the magnitudes it adds; the rest, float32, is far below."""
+    return 2.0 ** -8 * (size + got.double().abs()) * 1.05 + 1e-5
+
+
 @pytest.mark.parametrize("Hq,Hkv,D,page", [(8, 2, 128, 16), (16, 8, 128, 16), (3, 3, 64, 32), (16, 1, 64, 16)])
 @pytest.mark.parametrize("name", ["among", "many", "shared", "filled", "few", "short"])
 @pytest.mark.parametrize("with_sink", [False, True])
-def test_few_and_many_rows_in_one_launch(name, Hq, Hkv, D, page, with_sink):
+@pytest.mark.parametrize("cap", [0.0, 12.0])             # (capped scores: a build of their own)
+def test_few_and_many_rows_in_one_launch(name, Hq, Hkv, D, page, with_sink, cap):
     ops = _ops()
     lens = _lens(name)
     q_lens, kv_lens = [q for q, _ in lens], [k for _, k in lens]
     q, kc, vc, bt, cu, kvl = _paged_case(torch.bfloat16, len(lens), Hq, Hkv, D, page, q_lens, kv_lens, 32)
     sink = torch.randn(Hq, generator=torch.Generator().manual_seed(33)).cuda() if with_sink else None
     got = ops.paged_attention(q, Hq, kc, vc, bt, cu, kvl, max(q_lens), max(kv_lens), D ** -0.5, min_q_len=1,
-                              max_kv_len_of_many=max(k for q, k in lens if q > 1), sink=sink)
+                              max_kv_len_of_many=max(k for q, k in lens if q > 1), sink=sink, softcap=cap)
     assert bool(got.isfinite().all())
-    # A bfloat16 result (eight significant bits: half a unit is 2^-8 of a number at most) is off by its own rounding and by that of
-    # the probabilities in the second product, 2^-8 of the sum of the magnitudes it adds (a sink only makes the probabilities
-    # smaller); the rest, float32, is far below.
-    args = (bt, cu, kvl, max(q_lens), max(kv_lens), D ** -0.5)
-    magnitude = torch_ops.paged_attention(q.float(), Hq, kc.float(), vc.float().abs(), *args).float()
-    bound = 2.0 ** -8 * (magnitude + got.float().abs()) * 1.05 + 1e-5
-    if sink is None:
-        want = torch_ops.paged_attention(q.float(), Hq, kc.float(), vc.float(), *args).float()
-        assert bool(((got.float() - want).abs() <= bound).all())
+    want, size = _exact(q, kc, vc, bt, cu, kvl, D ** -0.5, sink, cap)
+    bound = _bound(got, size)
+    assert bool(((got.double() - want).abs() <= bound).all())
     # each kind by itself, in kernels of its own
     G = Hq // Hkv
     for kind in (lambda n: 0 < n * G <= 16, lambda n: n * G > 16):
@@ -58,5 +78,19 @@ def test_few_and_many_rows_in_one_launch(name, Hq, Hkv, D, page, with_sink):
         alone = ops.paged_attention(q[rows].contiguous(), Hq, kc, vc, bt[at].contiguous(),
                                     torch.tensor([0] + counts).cumsum(0).int().cuda(), kvl[at].contiguous(), max(counts),
                                     max(kv_lens), D ** -0.5, min_q_len=min(counts),
-                                    max_kv_len_of_many=max(k for q, k in lens if q > 1), sink=sink)
-        assert bool(((got[rows].float() - alone.float()).abs() <= 2 * bound[rows]).all())
+                                    max_kv_len_of_many=max(k for q, k in lens if q > 1), sink=sink, softcap=cap)
+        assert bool(((got[rows].double() - alone.double()).abs() <= 2 * bound[rows]).all())
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,page", [(8, 2, 128, 16), (16, 8, 128, 16), (3, 3, 64, 32), (16, 1, 64, 16)])
+@pytest.mark.parametrize("lens", [[(17, 1984)], [(40, 1900), (17, 17), (20, 1000)], [(33, 1970), (21, 1500)]])
+@pytest.mark.parametrize("cap", [0.0, 12.0])
+def test_few_rows_over_many_keys(Hq, Hkv, D, page, lens, cap):
+    """Blocks of sixteen rows over as many keys as no block of them shares with another."""
+    ops = _ops()
+    q_lens, kv_lens = [q for q, _ in lens], [k for _, k in lens]
+    assert ops.library("attention").q3_paged_attention_prompt_splits(sum(q_lens), Hq, Hkv, max(kv_lens)) == 1
+    q, kc, vc, bt, cu, kvl = _paged_case(torch.bfloat16, len(lens), Hq, Hkv, D, page, q_lens, kv_lens, 34)
+    got = ops.paged_attention(q, Hq, kc, vc, bt, cu, kvl, max(q_lens), max(kv_lens), D ** -0.5, min_q_len=min(q_lens), softcap=cap)
+    want, size = _exact(q, kc, vc, bt, cu, kvl, D ** -0.5, None, cap)
+    assert bool(((got.double() - want).abs() <= _bound(got, size)).all())
