@@ -7,7 +7,8 @@
 // More rows (gemm_parts_kernel) run on the bfloat16 matrix cores. A float32 number is exactly the sum of three bfloat16
 // numbers, its significand's upper, middle and lower eight bits: the parts are cut off, not rounded, so nothing overflows,
 // and the product of a part and a weight is exact in float32. Three matrix instructions (v_mfma_f32_16x16x32_bf16, 2.5
-// PFLOP/s) do the work of eight of v_mfma_f32_16x16x4_f32 (157 TFLOP/s) at a sixteenth of the cost each, and only the additions round:
+// PFLOP/s) do the work of eight of v_mfma_f32_16x16x4_f32 (157 TFLOP/s) at half the cost each, 16 / 3 times less matrix time in
+// all, and only the additions round:
 // against 64 bits the results are off by 1.0e-7 to 1.9e-7 (2-norm, 1,024 to 4,096 k) where a chain of multiply-adds is off
 // by 5.7e-7 to 1.2e-6.
 //
@@ -369,9 +370,11 @@ int launch(const void* x, const void* w, void* out, int M, int N, int K, hipStre
   // K shared out 30; 336 rows of 4,096, 192 tiles: 22 and 24; 201 rows of 4,096, 128 tiles: 22 and 16). Below, K shared out
   // inside the block, one block a CU: the smallest tiles that still are one round of the 256 CUs (1,024 x 4,096:
   // 100 rows, 256 tiles of 32 x 16: 18.2 us, in 32 x 32 19.7; 201 rows, 224 tiles of 32 x 32: 20.4, in 32 x 64 24.2; 336 rows, 352 tiles
-  // of 32 x 32: 38, in 32 x 64 25).
+  // of 32 x 32: 38, in 32 x 64 25). An inner size that leaves groups without a stage has nothing to share out where it takes
+  // two rounds (600 rows of 2,048 x 64 and x 128 9.1 and 9.2 in 32 x 64, 5.7 and 7.0 in 64 x 128; 300 of 4,096 x 192 10.5 and 8.5).
   const long m32 = (M + 31) / 32;
-  if ((long)((M + 63) / 64) * ((N + 127) / 128) >= 192) return launch_shape<SILU, 4, 1, 1, 8, 1, 2>(x, w, out, M, N, K, stream);
+  const bool few_stages = K < 4 * BK && m32 * ((N + 63) / 64) > 256;
+  if (few_stages || (long)((M + 63) / 64) * ((N + 127) / 128) >= 192) return launch_shape<SILU, 4, 1, 1, 8, 1, 2>(x, w, out, M, N, K, stream);
   if (m32 * ((N + 15) / 16) <= 256) return launch_shape<SILU, 2, 1, 1, 1, 4, 4>(x, w, out, M, N, K, stream);
   if (m32 * ((N + 31) / 32) <= 256) return launch_shape<SILU, 2, 1, 1, 2, 4, 3>(x, w, out, M, N, K, stream);
   return launch_shape<SILU, 2, 1, 1, 4, 4, 2>(x, w, out, M, N, K, stream);

@@ -16,9 +16,11 @@ def _weight(N, K, seed, scale=0.1):
 
 
 # the few-row kernel (each of its row counts), every tile of the dispatch (32 x 16, 32 x 32, 32 x 64, 64 x 128), rows and
-# columns that end inside a tile, inner sizes of one stage (three shares of K empty), of five (a share empty, one short) and of many
+# columns that end inside a tile, inner sizes of one stage (three shares of K empty), of five (a share empty, one short) and of many; of one and of
+# three where K is not shared out
 @pytest.mark.parametrize("M,N,K", [(1, 1, 64), (4, 21, 512), (7, 130, 576), (16, 999, 1024), (17, 2, 64), (33, 1030, 320),
-                                   (100, 1026, 192), (65, 2050, 1088), (130, 4094, 320), (257, 6146, 64), (1030, 3010, 448)])
+                                   (100, 1026, 192), (65, 2050, 1088), (130, 4094, 320), (257, 6146, 64), (1030, 3010, 448),
+                                   (600, 2050, 64), (301, 4094, 192)])
 def test_products_from_the_copy(M, N, K):
     ops = _ops()
     x, w = _rand((M, K), torch.float32, 81), _weight(N, K, 82)
