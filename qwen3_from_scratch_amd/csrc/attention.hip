@@ -2041,7 +2041,8 @@ __device__ __forceinline__ int sequence_of_tile(int& n, const int* __restrict__ 
 // tiles of 32, straight from the L2, which every block asks for them anew: the way as long as a CU has two such blocks at most
 // (SHORT_BLOCKS, a little less for the tiles that do not come). Microseconds, prompt kernel / this, 16 and 32 heads over 8 of 128: three
 // prompts of 33, 67 and 101 tokens 10.9 / 7.0 and 11.0 / 9.6; one of 200 11.6 / 8.1 and 13.2 / 10.4; 64 rows over 512 keys 17.7 / 10.4
-// and 17.8 / 10.4; 32 over 1,000 30 / 15; 400 over 400 (400 and 800 blocks) 17.6 / 13.2 and 18.1 / 20.9; four prompts of 128
+// and 17.8 / 10.4; 32 over 1,000 30 / 15, over 1,900 51 / 23 (from 1,985 keys on the prompt kernel shares them out); 440 and 220 over
+// 1,900 (440 blocks each) 52 / 40; 400 over 400 (400 and 800 blocks) 17.6 / 13.2 and 18.1 / 20.9; four prompts of 128
 // (512 and 1,024) 9.7 / 10.3 and 10.2 / 18.4.
 #define SHORT_BLOCKS 448
 template <int D>

@@ -11,7 +11,11 @@ constexpr int BN = 64, BK = 128;   // columns of a tile, k of a stage
 constexpr int LEAST = 5, MOST = 9;
 
 // The height (in units of 16 rows) of the least tile that covers the product in one round of 256 blocks, if that leaves
-// little undone: at least 82 % of what 256 such tiles hold (256 rows of 4,096 x 4,096, 80 %, 22.2 us and the library 20.0), 0 otherwise. Up to
+// little undone: at least 82 % of what 256 such tiles hold, 0 otherwise. From there on none of 59 products timed on both sides (3,072 to
+// 16,384 columns, 1,024 to 5,120 k) is slower than the library's or the shared-out tiles by more than 1 %: 276 rows of 5,120 x 5,120 (90 %)
+// 31.8 there and 32.2 here, 250 of 8,192 x 4,096 (98 %) 31.5 and 31.7, 268 of 4,096 x 4,096 (84 %) 25.3 and 21.1. Below they part:
+// 256 and 230 rows of 4,096 x 4,096 (80 and 72 %) 20.9 and 21.8, 21.9 and 23.4; 215 of 6,144 x 4,096 (72 %) 26.5 and 28.3; but
+// 512 of 2,048 x 4,096 (80 %) 28.5 and 21.6. Up to
 // 640 rows and 5,120 k: of longer sums tiles that share K out over blocks bring less through the caches (535 rows of 4,096 x 12,288 80.5 us, 78.4 so).
 inline int height_for(int M, int N, int K) {
   if (M <= 128 || M > 640 || N < BN || K % BK || K < 1024 || K > 5120 || (size_t)N * K * 2 < (16u << 20)) return 0;

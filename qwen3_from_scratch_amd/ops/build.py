@@ -34,8 +34,9 @@ MODULES = ("elementwise", "norm", "rotary", "attention", "attention_capped", "at
            "hyper", "recurrent", "mlstm", "delta", "softcap", "gemm", "matmul", "sampling", "probes", "layers")
 # A module's further sources, compiled on their own: their kernels are code objects of their own in its library. Where a kernel's
 # code lies decides how long a launch of it takes to get going: with the kernels of these two between those of matmul.hip, the
-# tiled and the weight-streaming product of a step of 64 requests took 0.1 to 0.9 us longer each, with the same instructions
-# (a step of the 8B shape 7,656 us before they were added, 7,770 with them in one code object, 7,659 so).
+# tiled and the weight-streaming product of a step of 64 requests of the 8B shape took 11.7 and 39.9 us with the instructions
+# that had taken 10.9 and 39.1, and take 11.1 and 39.4 so. (As many misses in the instruction cache, but longer ones: 7,440 requests
+# of a weight-streaming launch met one under way, 4,420 before and so.)
 FURTHER = {"matmul": ["gemm_groups.hip", "gemm_rounds.hip"]}
 # what a module links besides the HIP runtime
 LINKS = {"matmul": ["-lhipblaslt"]}
