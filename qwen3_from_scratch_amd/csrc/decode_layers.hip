@@ -1,0 +1,1013 @@
+// All decoder layers of a step of single tokens in one launch: pre-norm layers of softmax attention with grouped heads of 128 and a
+// gated unit, bfloat16, up to 16 rows. What gemm.hip's few-row products and attention.hip's decoding attention do layer by layer.
+//
+// A kernel that waits for its predecessor costs 2 us inside a graph if it does nothing and 4 to 4.5 if it loads, reduces and stores a
+// row, and a step of the 0.6B shape was 145 of them: 1,011 us where its bytes take 240. Here a block per compute unit stays for all
+// layers and blocks exchange rows through memory past the chiplets' own caches. What is exchanged says itself that it is there: the
+// exchange is filled with words of ones (ABSENT) beforehand, a block stores its results and nobody anything else, and a reader asks for
+// what it needs until no word of ones is among it. So a product's rows reach the next one in a store's way to memory and a load's
+// back, some 1.2 us, where flags behind the data took 3.8 and a barrier of all blocks alone 2.6 (256 blocks, 2,048 numbers a
+// block). The weights of a product's first steps are asked for while the last one's results are on their way, so memory is not idle
+// meanwhile.
+//
+// What it measured (us a step in a graph, the layers' kernels one by one / this): the 0.6B shape, one request over 1,100 keys
+// 1,013 / 809, over 30,000 1,545 / 1,366, eight over 2,000 1,415 / 1,155, sixteen 1,910 / 1,686; the 8B shape, one over 2,060 3,407 / 3,026,
+// eight 3,954 / 3,510, eight over 8,000 5,057 / 4,636, sixteen over 300 3,849 / 3,754, over 2,060 4,836 / 4,520. None of 28 sizes between
+// was slower; more than 16 rows have no registers here.
+//
+// What bounds it: one request of the small shape the chain of five or six exchanges a layer, 26 us, of which the way through memory is
+// some 7 and the rest the few hundred instructions of each wavefront between them; the large shape its weights (5.0 of the 5.8 TB/s that
+// a plain read reaches, the whole step through) and the attention's part, where no weights move.
+// What did not help: the block split into wavefronts that multiply and wavefronts that look, prepare and store, with the weights in a
+// ring in shared memory (0.6B 905: more handovers a product), asking for the sums of squares together with the rows (lines that many blocks
+// write and all ask for again and again are slow to change: 915), copies of what all read (nothing), the first keys asked for ahead of
+// the [q | k | v] product's end (937: a second copy of the product, 61 KB of code beyond what the instruction caches keep).
+#include "common.h"
+#include "attention_tiles.h"
+#include "gates.h"
+
+namespace {
+
+typedef __attribute__((ext_vector_type(4))) unsigned u32x4_t;
+typedef __attribute__((ext_vector_type(2))) unsigned u32x2_t;
+
+constexpr int WAVES = 8;                      // of a block
+constexpr int THREADS = 64 * WAVES;
+constexpr int HEAD = 128;                     // the head size
+constexpr int MOST_SLABS = 8;                 // slabs of 16 weight rows that a block multiplies between two barriers
+constexpr int RESULTS = 64;                   // of them times rows, at most
+constexpr int CHUNKS = 16;                    // kilobytes of weights that a wavefront has on their way
+constexpr unsigned ABSENT = 0xffffffffu;      // a word of the exchange that nobody has written yet
+constexpr unsigned CLOSED = 0x80000000u;
+constexpr int THROUGH = 16;                   // cache policy of what blocks exchange: past the chiplets' own caches (sc1)
+constexpr int MOST_SPLITS = 32;
+constexpr int MOST_ROWS = 16;
+constexpr int MOST_LAYERS = 128;
+
+// One layer as the host gives it and as the launch's table holds it.
+struct Layer {
+  const void* w[4];            // tile-ordered: [q | k | v], the attention's output, gate and up interleaved, down
+  const void *q_norm, *k_norm, *entry_norm, *middle_norm;
+  void *keys, *values;
+  float entry_eps, middle_eps;
+};
+constexpr int LAYERS_A_LAUNCH = 32;           // as many as the preparing kernel's arguments hold
+struct LayerPack {
+  Layer layer[LAYERS_A_LAUNCH];
+};
+
+struct Args {
+  const Layer* layers;
+  unsigned* control;
+  char* exchange;
+  float* residual;
+  const float* table;
+  const int *block_table, *kv_lens;
+  long per_layer;              // bytes of exchange
+  int at_part, at_att, at_mid, at_mid_sums, at_hid, at_out, at_out_sums;
+  int count, rows, width, heads, kv_heads, inner, norm_f32, max_pos, table_width, page, num_pages, splits, patience, limit;
+  float qk_eps, scale_log2;
+};
+
+struct AttentionShared {
+  float k[HEAD], v[HEAD];                     // the token's own, as the caches hold them
+  __attribute__((aligned(16))) bf16_t q[16][HEAD + 8];
+  float m[WAVES + 1][16], l[WAVES][16];
+  __attribute__((aligned(16))) float acc[WAVES][16][HEAD + 4];
+};
+struct Shared {
+  // the wavefronts' shares of K of a product: [slab][wavefront][four columns of sixteen][row], 16 bytes each; twice, in turn
+  __attribute__((aligned(16))) char red[2][RESULTS * WAVES * 4 * 16];
+  AttentionShared attention;
+  __attribute__((aligned(16))) uint64_t layers[MOST_LAYERS * sizeof(Layer) / 8];
+  float scale[16];
+  int rank, blocks;
+};
+
+// Sixteen bytes, or eight, of memory through a pointer out of the launch's table (an access through a plain pointer is one to
+// either kind of memory, which waits for whatever is on its way in both).
+typedef const __attribute__((address_space(1))) u32x4_t* memory16;
+typedef const __attribute__((address_space(1))) u32x2_t* memory8;
+__device__ __forceinline__ uint4 load16(const void* p) {
+  const u32x4_t v = *(memory16)p;
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ float4 load_four(const float* p) {
+  const u32x4_t v = *(memory16)p;
+  return make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
+}
+__device__ __forceinline__ void store16(void* p, const u32x4_t& v) { *(__attribute__((address_space(1))) u32x4_t*)p = v; }
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, long bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
+}
+__device__ __forceinline__ u32x4_t peek16(__amdgpu_buffer_rsrc_t r, int at) { return __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, THROUGH); }
+__device__ __forceinline__ bool there(const u32x4_t& v) { return v.x != ABSENT && v.y != ABSENT && v.z != ABSENT && v.w != ABSENT; }
+// A word of results that happens to be the mark (not a number, either way) becomes another one.
+__device__ __forceinline__ unsigned marked(unsigned w, unsigned instead) { return w == ABSENT ? instead : w; }
+__device__ __forceinline__ void put8(__amdgpu_buffer_rsrc_t r, int at, uint2 v) {
+  const u32x2_t p = {marked(v.x, 0x7fc07fc0u), marked(v.y, 0x7fc07fc0u)};
+  __builtin_amdgcn_raw_buffer_store_b64(p, r, at, 0, THROUGH);
+}
+__device__ __forceinline__ void put4(__amdgpu_buffer_rsrc_t r, int at, unsigned v, unsigned instead) {
+  __builtin_amdgcn_raw_buffer_store_b32(marked(v, instead), r, at, 0, THROUGH);
+}
+__device__ __forceinline__ void compiler_fence() { asm volatile("" ::: "memory"); }
+
+// Until shared memory holds what the block's wavefronts have written (and nothing about memory)
+__device__ __forceinline__ void meet() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// ---- which slabs of 16 weight rows a block multiplies ----
+
+struct Product {
+  int first, count, steps;     // slabs first, first + blocks, ...; k in steps of 32
+};
+// The four products of a layer: [q | k | v], the attention's output, gate and up, down. The two that add into the stream go to the same
+// blocks, which are others than those of the attention's first items.
+struct Shares {
+  int rank, shifted, qkv, stream, gate_up;             // of a block: the first slabs, how many
+  int width_steps, heads_steps, inner_steps;
+  __device__ __forceinline__ Product of(int which) const {
+    // (the members' values first: a choice between the members themselves is one between addresses, and the struct then lies in memory)
+    const int into = stream, at = shifted, first = rank, first_count = qkv, third = gate_up, s0 = width_steps, s1 = heads_steps, s3 = inner_steps;
+    return Product{which & 1 ? at : first, which & 1 ? into : which == 0 ? first_count : third, which == 1 ? s1 : which == 3 ? s3 : s0};
+  }
+};
+__device__ __forceinline__ Shares shares_of(const Args& a, int rank, int blocks) {
+  Shares s;
+  s.rank = rank;
+  s.shifted = rank >= blocks / 2 ? rank - blocks / 2 : rank + blocks - blocks / 2;
+  auto count = [&](int slabs, int first) { return first < slabs ? (slabs - first + blocks - 1) / blocks : 0; };
+  s.qkv = count((a.heads + 2 * a.kv_heads) * HEAD / 16, rank);
+  s.stream = count(a.width / 16, s.shifted);
+  s.gate_up = count(2 * a.inner / 16, rank);
+  s.width_steps = a.width / 32;
+  s.heads_steps = a.heads * HEAD / 32;
+  s.inner_steps = a.inner / 32;
+  return s;
+}
+
+typedef const __attribute__((address_space(4))) int* entries_ptr;
+typedef const __attribute__((address_space(1))) char* memory;
+constexpr int LAYER_WORDS = sizeof(Layer) / 8;
+enum { Q_NORM = 4, K_NORM, ENTRY_NORM, MIDDLE_NORM, KEYS, VALUES, EPS };    // words of an entry behind its four matrices
+
+template <typename QKW>
+struct Block {
+  Shared& sh;
+  const Args& a;
+  const int rank, blocks;
+  int wave, lane, tid;
+  Shares shares;
+  int most;                    // looks at the exchange before a wait is given up
+  int alive;
+  unsigned rows_inverse;
+  int turn;                    // of the two halves of shared memory's results
+  int held;                    // the product whose first weights are on their way: four times its layer, and which
+  Pack16 w[CHUNKS];            // they
+
+  // (as a number of its own: what is computed from it is not kept in registers over the whole launch)
+  __device__ __forceinline__ static int anew(int v) {
+    asm volatile("" : "+v"(v));
+    return v;
+  }
+  // Between two looks at the exchange: whether to look again. Every wait ends: after so many looks nothing is waited for any more.
+  __device__ __forceinline__ bool again(int n) {
+    if (n >= most) alive = 0;
+    alive = __builtin_amdgcn_readfirstlane(alive);
+    return alive != 0;
+  }
+
+  // ---- products ----
+
+  // A wavefront's steps are every eighth, one at least; they are taken sixteen at a time, or where K has no more, eight of two slabs and four of
+  // four. Steps behind the last one are that one again, times zero.
+  __device__ __forceinline__ int own_steps(int steps) const { return (steps - wave + WAVES - 1) / WAVES; }
+  __device__ __forceinline__ static int together(int steps) { return steps > 8 * WAVES ? 16 : steps > 4 * WAVES ? 8 : 4; }
+  // A pointer, or the two norms' eps, out of a layer's entry
+  __device__ __forceinline__ uint64_t entry(int layer, int word) const {
+    const uint64_t v = sh.layers[layer * LAYER_WORDS + word];
+    return (uint64_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32 | (unsigned)__builtin_amdgcn_readfirstlane((int)v);
+  }
+  __device__ __forceinline__ memory weights_of(const Product& p, int layer, int which, int slab) const {
+    return (memory)entry(layer, which) + ((long)((p.first + slab * blocks) * p.steps + wave) << 10);
+  }
+  // What the registers of weights hold is of no use any more (a load that is left out would otherwise keep it where registers are scarce)
+  __device__ __forceinline__ void forget() {
+    Pack16 nothing[CHUNKS];
+#pragma unroll
+    for (int j = 0; j < CHUNKS; ++j) {
+      asm volatile("" : "=v"(nothing[j].u.x), "=v"(nothing[j].u.y), "=v"(nothing[j].u.z), "=v"(nothing[j].u.w));
+      w[j] = nothing[j];
+    }
+  }
+  // The first weights of product `which`, or the first one behind it that this block has part in, asked for as early as their registers are free
+  __device__ __forceinline__ void look_ahead(int layer, int which) {
+    forget();
+    Product p;
+    for (;; ++which) {
+      if (which == 4) which = 0, ++layer;
+      if (layer >= a.count) return;
+      p = shares.of(which);
+      if (p.count) break;
+    }
+    held = 4 * layer + which;
+    begin(p, layer, which, 0);
+  }
+  __device__ __forceinline__ void begin(const Product& p, int layer, int which, int done) {
+    // kilobyte j: sixteen steps of a slab, eight of two or four of four, of which there are `own`
+    const int take = together(p.steps), own = own_steps(p.steps), kilobytes = take * min(CHUNKS / take, p.count - done);
+    const memory at = weights_of(p, layer, which, done);
+    const long stride = (long)blocks * p.steps << 10;
+    const unsigned off = lane * 16;
+#pragma unroll
+    for (int quarter = 0; quarter < 4; ++quarter)
+      if (quarter == 0 || kilobytes > 4 * quarter) {
+        const int slab = take == 16 ? 0 : take == 8 ? quarter >> 1 : quarter, step = take == 16 ? 4 * quarter : take == 8 ? 4 * (quarter & 1) : 0;
+        const memory from = at + slab * stride;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const u32x4_t v = *(memory16)(from + (long)min(step + j, own - 1) * (WAVES << 10) + off);
+          w[4 * quarter + j].u = make_uint4(v.x, v.y, v.z, v.w);
+        }
+      }
+  }
+
+  // Sixteen steps of rows, `left` of which there are, from the wavefront's step `i` on: lane (row, eight k of 32)
+  __device__ __forceinline__ void look(Pack16 (&x)[CHUNKS], __amdgpu_buffer_rsrc_t ex, int src, int K, int i, int left) const {
+    const int lane = anew(this->lane), col = lane & 15, grp = lane >> 4;
+    const int at = (col * K + (wave + i * WAVES) * 32 + 8 * grp) * 2;
+#pragma unroll
+    for (int j = 0; j < CHUNKS; ++j) x[j].u = make_uint4(0, 0, 0, 0);
+#pragma unroll
+    for (int quarter = 0; quarter < 4; ++quarter)
+      if (left > 4 * quarter) {
+        if (col < a.rows) {
+#pragma unroll
+          for (int j = 4 * quarter; j < 4 * quarter + 4; ++j) {
+            const u32x4_t v = peek16(ex, src + at + min(j, left - 1) * (WAVES * 64));
+            x[j].u = make_uint4(v.x, v.y, v.z, v.w);
+          }
+        }
+        if (left < 4 * quarter + 4) {
+#pragma unroll
+          for (int j = 4 * quarter + 1; j < 4 * quarter + 4; ++j)
+            if (j >= left) x[j].u = make_uint4(0, 0, 0, 0);
+        }
+      }
+  }
+  __device__ __forceinline__ static bool all_there(const Pack16 (&x)[CHUNKS]) {
+    unsigned least = 0;                                  // (the mark is the largest word)
+#pragma unroll
+    for (int j = 0; j < CHUNKS; ++j) least = max(max(least, max(x[j].u.x, x[j].u.y)), max(x[j].u.z, x[j].u.w));
+    return __all(least != ABSENT);
+  }
+  // Four of a norm's weights as they lie in memory, and as numbers
+  __device__ __forceinline__ u32x4_t raw_norm(const void* n, int at) const {
+    if (a.norm_f32) return *(memory16)(static_cast<const float*>(n) + at);
+    const u32x2_t v = *(memory8)(static_cast<const bf16_t*>(n) + at);
+    return u32x4_t{v.x, v.y, 0, 0};
+  }
+  __device__ __forceinline__ float4 norm_of(const u32x4_t& v) const {
+    if (a.norm_f32) return make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
+    return make_float4(__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xffff0000u));
+  }
+
+  // A slab's sums of this wavefront's steps into shared memory
+  __device__ __forceinline__ void leave(const f32x4_t& acc, int slab) {
+    const int col = lane & 15, grp = lane >> 4;
+    if (col < a.rows) *reinterpret_cast<f32x4_t*>(sh.red[turn] + (unsigned)(((slab * WAVES + wave) * 4 + grp) * a.rows + col) * 16) = acc;
+  }
+
+  // What a product multiplies with: K numbers a row at `src` of the exchange, their squares' partial sums at `sums`
+  struct Rows {
+    __amdgpu_buffer_rsrc_t ex;
+    int src, sums, K;            // (sums 0: no scales)
+    float eps;
+  };
+  // The look at the exchange is the wait: a word without the mark is there.
+  __device__ __forceinline__ void fetch(Pack16 (&x)[CHUNKS], const Rows& r, int i, int left) {
+    left = __builtin_amdgcn_readfirstlane(left);
+    if (i == 0 && a.rows >= 4)   // one look at one place first: so many rows asked for again and again hold up those that write them
+      for (int n = 0;; ++n) {
+        compiler_fence();
+        const u32x4_t v = peek16(r.ex, r.src + (wave + (min(left, 16) - 1) * WAVES) * 64);
+        if (__builtin_amdgcn_readfirstlane((int)there(v)) || !again(n)) break;
+      }
+    for (int n = 0;; ++n) {
+      compiler_fence();
+      look(x, r.ex, r.src, r.K, i, left);
+      if (all_there(x) || !again(n)) break;
+    }
+  }
+
+  // `slabs` slabs from `done` on, whose first group's weights have been asked for
+  __device__ __forceinline__ void multiply(const Rows& r, const Product& p, int layer, int which, int done, int slabs) {
+    const int own = own_steps(p.steps), take = together(p.steps), together = CHUNKS / take;
+    const long stride = (long)blocks * p.steps << 10;
+    memory slab = weights_of(p, layer, which, done);
+    if (own > 16) {            // every slab in sections, whose rows are asked for with each
+#pragma unroll 1
+      for (int s = 0; s < slabs; ++s, slab += stride) {
+        f32x4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll 1
+        for (int i = 0; i < own; i += 16) {
+          Pack16 x[CHUNKS];
+          fetch(x, r, i, own - i);
+          const bool ends = i + 16 >= own;
+          if (!ends || s + 1 < slabs)
+            sixteen(acc, x, ends ? slab + stride : slab + (long)(i + 16) * (WAVES << 10), ends ? own : own - i - 16);
+          else
+#pragma unroll
+            for (int j = 0; j < CHUNKS; ++j) acc[j & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j].v, x[j].v, acc[j & 1], 0, 0, 0);
+        }
+        leave(acc[0] + acc[1], s);
+      }
+      return;
+    }
+    Pack16 x[CHUNKS];
+    fetch(x, r, 0, own);
+    if (take == 16) {
+#pragma unroll 1
+      for (int s = 0; s < slabs; ++s, slab += stride) {
+        f32x4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+        if (s + 1 < slabs)
+          sixteen(acc, x, slab + stride, own);
+        else
+#pragma unroll
+          for (int j = 0; j < CHUNKS; ++j) acc[j & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j].v, x[j].v, acc[j & 1], 0, 0, 0);
+        leave(acc[0] + acc[1], s);
+      }
+      return;
+    }
+#pragma unroll 1
+    for (int s = 0; s < slabs; s += together) {
+      f32x4_t acc[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) acc[q] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      if (take == 8) {
+#pragma unroll
+        for (int j = 0; j < CHUNKS; ++j) acc[j >> 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j].v, x[j & 7].v, acc[j >> 2], 0, 0, 0);
+        acc[0] += acc[1];
+        acc[1] = acc[2] + acc[3];
+      } else {
+#pragma unroll
+        for (int j = 0; j < CHUNKS; ++j) acc[j >> 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j].v, x[j & 3].v, acc[j >> 2], 0, 0, 0);
+      }
+      if (s + together < slabs) begin(p, layer, which, done + s + together);
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (q < together && s + q < slabs) leave(acc[q], s + q);
+    }
+  }
+  // Sixteen steps of a slab, and in the place of each kilobyte the next group's, `left` of which there are
+  __device__ __forceinline__ void sixteen(f32x4_t (&acc)[2], const Pack16 (&x)[CHUNKS], memory next, int left) {
+    const unsigned off = lane * 16;
+#pragma unroll
+    for (int j = 0; j < CHUNKS; ++j) {
+      acc[j & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j].v, x[j].v, acc[j & 1], 0, 0, 0);
+      const u32x4_t v = *(memory16)(next + (long)min(j, left - 1) * (WAVES << 10) + off);
+      w[j].u = make_uint4(v.x, v.y, v.z, v.w);
+    }
+  }
+
+  // The rows' scales from the partial sums of squares, [row][slab]
+  __device__ __forceinline__ void scales(const Rows& r) {
+    const int slabs = a.width / 16;
+    for (int row = wave; row < a.rows; row += WAVES) {
+      float s = 0.f;
+      for (int k = lane * 4; k < ((slabs + 255) & ~255); k += 256) {
+        u32x4_t v = {0, 0, 0, 0};
+        for (int n = 0;; ++n) {
+          compiler_fence();
+          if (k < slabs) v = peek16(r.ex, r.sums + (row * slabs + k) * 4);
+          if (__all(there(v)) || !again(n)) break;
+        }
+        s += (__uint_as_float(v.x) + __uint_as_float(v.y)) + (__uint_as_float(v.z) + __uint_as_float(v.w));
+      }
+      s = wave_sum(s);
+      if (lane == 0) sh.scale[row] = rsqrtf(s * (1.f / (float)a.width) + r.eps);
+    }
+  }
+
+  // The wavefronts' shares of K of one pass, added in a fixed order, and what follows the product. `res`, `raw`: the stream and the
+  // norm's weights at the lane's first four results.
+  __device__ __forceinline__ int over_rows(int n) const { return (unsigned)n * rows_inverse >> 20; }    // n / a.rows, n below 4,096
+  struct Follow {
+    float4 res;
+    u32x4_t raw;
+  };
+  __device__ __forceinline__ Follow follow(const Product& p, int done, int slabs, const void* norm) const {
+    const int tid = anew(this->tid), q = tid >> 2, s = over_rows(q), row = q - s * a.rows, n = (p.first + (done + s) * blocks) * 16 + 4 * (tid & 3);
+    Follow f;
+    f.res = make_float4(0.f, 0.f, 0.f, 0.f);
+    f.raw = u32x4_t{0, 0, 0, 0};
+    if (s < slabs) {
+      f.res = load_four(a.residual + (size_t)row * a.width + n);
+      if (norm) f.raw = raw_norm(norm, n);
+    }
+    return f;
+  }
+  __device__ __forceinline__ void finish(__amdgpu_buffer_rsrc_t ex, int which, const Product& p, int done, int slabs, const void* norm, Follow f) {
+    const bool stream = which & 1;
+    const int tid = anew(this->tid), entries = slabs * 4 * a.rows, grp = tid & 3;
+    const int width = which == 0 ? (a.heads + 2 * a.kv_heads) * HEAD : which == 2 ? a.inner : a.width;
+    const int dst = which == 0 ? 0 : which == 1 ? a.at_mid : which == 2 ? a.at_hid : a.at_out;
+    for (int idx = tid; idx < entries; idx += THREADS) {
+      const int q = idx >> 2, s = over_rows(q), row = q - s * a.rows, slab = p.first + (done + s) * blocks, n = slab * 16 + 4 * grp;
+      const char* part = sh.red[turn] + (unsigned)((s * WAVES * 4 + grp) * a.rows + row) * 16;
+      f32x4_t acc = *reinterpret_cast<const f32x4_t*>(part);
+#pragma unroll
+      for (int v = 1; v < WAVES; ++v) acc += *reinterpret_cast<const f32x4_t*>(part + (unsigned)(v * 4 * a.rows) * 16);
+      union {
+        uint2 u;
+        __bf16 e[4];
+      } pk;
+      if (stream) {
+        if (idx != tid) {
+          f.res = load_four(a.residual + (size_t)row * a.width + n);
+          if (norm) f.raw = raw_norm(norm, n);
+        }
+        const float x[4] = {f.res.x + (float)(__bf16)acc[0], f.res.y + (float)(__bf16)acc[1], f.res.z + (float)(__bf16)acc[2],
+                            f.res.w + (float)(__bf16)acc[3]};
+        if (norm) {
+          const float4 nw = norm_of(f.raw);
+          const float w4[4] = {nw.x, nw.y, nw.z, nw.w};
+          float ss = 0.f;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            ss += x[e] * x[e];
+            pk.e[e] = (__bf16)(x[e] * w4[e]);
+          }
+          put8(ex, dst + (row * width + n) * 2, pk.u);
+          ss += __shfl_xor(ss, 1, 64);
+          ss += __shfl_xor(ss, 2, 64);
+          const int sums = which == 1 ? a.at_mid_sums : a.at_out_sums;
+          if (grp == 0) put4(ex, sums + (row * (width / 16) + slab) * 4, __float_as_uint(ss), 0x7fc00000u);
+        }
+        store16(a.residual + (size_t)row * a.width + n,
+                u32x4_t{__float_as_uint(x[0]), __float_as_uint(x[1]), __float_as_uint(x[2]), __float_as_uint(x[3])});
+      } else {
+        acc *= sh.scale[row];
+        if (which == 2) {
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            const float g = (float)(__bf16)acc[2 * e], u = (float)(__bf16)acc[2 * e + 1];
+            pk.e[e] = (__bf16)(gate_value<0>(g) * u);
+          }
+          put4(ex, dst + (row * width + n / 2) * 2, pk.u.x, 0x7fc07fc0u);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) pk.e[e] = (__bf16)acc[e];
+          put8(ex, dst + (row * width + n) * 2, pk.u);
+        }
+      }
+    }
+  }
+
+  __device__ __forceinline__ void product_of(const Rows& r, __amdgpu_buffer_rsrc_t ex, int layer, int which, const Product& p, const void* norm) {
+    const int pass = min(MOST_SLABS, RESULTS / a.rows);
+#pragma unroll 1
+    for (int done = 0; done < p.count; done += pass) {
+      const int slabs = min(pass, p.count - done);
+      if (done || held != 4 * layer + which) begin(p, layer, which, done);
+      Follow f;
+      if (which & 1) f = follow(p, done, slabs, norm);
+      multiply(r, p, layer, which, done, slabs);
+      if (done == 0 && !(which & 1)) scales(r);
+      if (done + slabs >= p.count && which != 0) look_ahead(layer, which + 1);
+      meet();
+      finish(ex, which, p, done, slabs, norm, f);
+      turn ^= 1;
+    }
+  }
+
+  // ---- attention ----
+
+  // A piece of the attention: a split of a sequence's keys for one key head, and what all layers have of it in common.
+  struct Item {
+    int split, g_kv, b, kv_len;
+    TilePages first, second;     // of this wavefront's first two tiles
+  };
+  __device__ __forceinline__ TilePages pages_of(int b, int tile) const {
+    const entries_ptr row = (entries_ptr)(uintptr_t)(a.block_table + (size_t)b * a.table_width);
+    TilePages p;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int entry = (tile * FAST_TILE + 16 * h) / a.page;
+      p.pg[h] = entry < a.table_width ? row[entry] : -1;
+    }
+    return p;
+  }
+  __device__ __forceinline__ Item item_of(int n) const {
+    Item it;
+    const int pair = n / a.splits;
+    it.split = n - pair * a.splits;
+    it.b = pair / a.kv_heads;
+    it.g_kv = pair - it.b * a.kv_heads;
+    it.kv_len = ((entries_ptr)(uintptr_t)a.kv_lens)[it.b];
+    const int first = it.split * WAVES + wave;
+    it.first = pages_of(it.b, first);
+    it.second = pages_of(it.b, first + WAVES * a.splits);
+    return it;
+  }
+
+  // What attention.hip's decoding block does, from and to the exchange. The heads' norms and rotations are shared out: a wavefront
+  // prepares one query row, the next ones the token's key and value. A wavefront asks for its next tile's keys when this one's have been
+  // multiplied, and for the values likewise.
+  __device__ __forceinline__ void attend(__amdgpu_buffer_rsrc_t ex, int layer, const Item& it) {
+    constexpr int D = HEAD;
+    AttentionShared& s = sh.attention;
+    const bf16_t *keys = (const bf16_t*)entry(layer, KEYS), *values = (const bf16_t*)entry(layer, VALUES);
+    const char *q_norm = (const char*)entry(layer, Q_NORM), *k_norm = (const char*)entry(layer, K_NORM);
+    const int split = it.split, g_kv = it.g_kv, b = it.b;
+    const int lane = anew(this->lane), col = lane & 15, grp = lane >> 4;
+    const int G = a.heads / a.kv_heads, joined = (a.heads + 2 * a.kv_heads) * D;
+    const int first = split * WAVES + wave, step = WAVES * a.splits;
+    const bool brings_new = split == a.splits - 1;
+    const int pos = it.kv_len - 1;                    // the token's own position; the cache is read up to the one before
+    const bool turned = a.table != nullptr && pos >= 0 && pos < a.max_pos;
+    const int kv_seen = max(pos, 0), row_pos = col < G ? pos - 1 : -1;
+    const int last = (kv_seen + FAST_TILE - 1) / FAST_TILE;
+    auto addr_of = [&](const TilePages& p, int t) {
+      return tile_addr(p, keys, values, a.num_pages, a.kv_heads, g_kv, a.page, D, D, t * FAST_TILE);
+    };
+    TileRegs<D, D> r;
+    auto ask_keys = [&](const TileAddr& to) {
+      r.at = to;
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int j = 0; j < D / 32; ++j) r.k[kb][j].u = load16(to.k + 4 * D * kb + 32 * j);
+    };
+    auto ask_values = [&]() {
+#pragma unroll
+      for (int nb = 0; nb < D / 16; ++nb) r.v[nb].u = load16(r.at.v + (size_t)(16 * nb) * a.page);
+    };
+    TilePages next = it.second;
+    if (first < last) {
+      ask_keys(addr_of(it.first, first));
+      ask_values();
+    }
+    // the token's rows: lane n has elements 2 n and 2 n + 1, its pair's other half is lane n ^ 32
+    for (int row = wave; row < G + (brings_new ? 2 : 0); row += WAVES) {
+      const int head = row < G ? g_kv * G + row : a.heads + (row == G ? 0 : a.kv_heads) + g_kv;
+      const bool prepared = row <= G;                 // (values are taken as they are)
+      float2 norm = make_float2(1.f, 1.f), cs = make_float2(1.f, 1.f), sn = make_float2(0.f, 0.f);
+      if (prepared && q_norm != nullptr) {
+        const char* weights = row < G ? q_norm : k_norm;
+        if constexpr (sizeof(QKW) == 4) {
+          const u32x2_t v = *(memory8)(weights + 8 * lane);
+          norm = make_float2(__uint_as_float(v.x), __uint_as_float(v.y));
+        } else {
+          const unsigned v = *(const __attribute__((address_space(1))) unsigned*)(weights + 4 * lane);
+          norm = make_float2(__uint_as_float(v << 16), __uint_as_float(v & 0xffff0000u));
+        }
+      }
+      if (prepared && turned) {
+        const float* at = a.table + (size_t)pos * D + 2 * (lane & 31);
+        const u32x2_t c = *(memory8)at, n = *(memory8)(at + D / 2);
+        cs = make_float2(__uint_as_float(c.x), __uint_as_float(c.y));
+        sn = make_float2(__uint_as_float(n.x), __uint_as_float(n.y));
+      }
+      unsigned v;
+      for (int n = 0;; ++n) {
+        compiler_fence();
+        v = __builtin_amdgcn_raw_buffer_load_b32(ex, (b * joined + head * D) * 2 + lane * 4, 0, THROUGH);
+        if (__all(v != ABSENT) || !again(n)) break;
+      }
+      float x0 = __uint_as_float(v << 16), x1 = __uint_as_float(v & 0xffff0000u);
+      if (prepared && q_norm != nullptr) {
+        const float scale = head_norm_scale(wave_sum(__fmaf_rn(x0, x0, __fmul_rn(x1, x1))), D, a.qk_eps);
+        x0 = __fmul_rn(__fmul_rn(x0, scale), norm.x);
+        x1 = __fmul_rn(__fmul_rn(x1, scale), norm.y);
+      }
+      if (prepared && turned) {
+        const float y0 = __shfl_xor(x0, 32, 64), y1 = __shfl_xor(x1, 32, 64);
+        const float sign = lane < 32 ? -1.f : 1.f;
+        x0 = __fmaf_rn(x0, cs.x, __fmul_rn(sign * y0, sn.x));
+        x1 = __fmaf_rn(x1, cs.y, __fmul_rn(sign * y1, sn.y));
+      }
+      union {
+        unsigned u;
+        __bf16 e[2];
+      } pk;
+      pk.e[0] = (__bf16)x0;
+      pk.e[1] = (__bf16)x1;
+      if (row < G)
+        *reinterpret_cast<unsigned*>(&s.q[row][2 * lane]) = pk.u;
+      else
+        *reinterpret_cast<float2*>((row == G ? s.k : s.v) + 2 * lane) = make_float2((float)pk.e[0], (float)pk.e[1]);
+    }
+    meet();
+    Pack16 q[D / 32];
+#pragma unroll
+    for (int j = 0; j < D / 32; ++j) {
+      q[j].u = make_uint4(0, 0, 0, 0);
+      if (col < G) q[j].u = *reinterpret_cast<const uint4*>(&s.q[col][32 * j + 8 * grp]);
+    }
+    if (brings_new) {                                 // the new key's scores: the rows shared out once more
+      for (int row = wave; row < G; row += WAVES) {
+        const bf16_t* mine = &s.q[row][2 * lane];
+        const float dot = wave_sum(fmaf(bf16_to_float(mine[0]), s.k[2 * lane], bf16_to_float(mine[1]) * s.k[2 * lane + 1]));
+        if (lane == 0) s.m[WAVES][row] = pos >= 0 ? dot * a.scale_log2 : -INFINITY;
+      }
+    } else if (wave == 0 && lane < 16) {
+      s.m[WAVES][lane] = -INFINITY;
+    }
+    f32x4_t acc[D / 16];
+#pragma unroll
+    for (int nb = 0; nb < D / 16; ++nb) acc[nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    float m_run = -INFINITY, l_run = 0.f;
+    for (int t = first; t < last; t += step) {
+      const bool more = t + step < last;
+      const int have = r.at.there, key0 = t * FAST_TILE;
+      if (have != 3 && !((have >> (col >> 3)) & 1)) {          // a half without a page counts as zeros
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+          for (int j = 0; j < D / 32; ++j) r.k[kb][j].u = make_uint4(0, 0, 0, 0);
+      }
+      f32x4_t sc[2];
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) {
+        sc[kb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < D / 32; ++j) sc[kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(r.k[kb][j].v, q[j].v, sc[kb], 0, 0, 0);
+      }
+      if (more) {
+        ask_keys(addr_of(next, t + step));
+        next = pages_of(b, t + 2 * step);
+      }
+      const Pack16 p = softmax_step<D / 16>(sc, false, key0, grp, row_pos, 0, a.scale_log2, m_run, l_run, acc);
+      if (have != 3 && !((have >> (grp >> 1)) & 1)) {
+#pragma unroll
+        for (int nb = 0; nb < D / 16; ++nb) r.v[nb].u = make_uint4(0, 0, 0, 0);
+      }
+      if (key0 + FAST_TILE > kv_seen) {  // slots past the sequence's end hold anything: zero them, 0 * NaN is NaN
+#pragma unroll
+        for (int nb = 0; nb < D / 16; ++nb)
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            if (key0 + 8 * grp + e >= kv_seen) r.v[nb].e[e] = (__bf16)0.f;
+      }
+#pragma unroll
+      for (int nb = 0; nb < D / 16; ++nb) acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(r.v[nb].v, p.v, acc[nb], 0, 0, 0);
+      if (more) ask_values();
+    }
+    float l_all = l_run;
+    l_all += __shfl_xor(l_all, 16, 64);
+    l_all += __shfl_xor(l_all, 32, 64);
+    if (grp == 0) {
+      s.m[wave][col] = m_run;
+      s.l[wave][col] = l_all;
+    }
+    if (col < G) {
+#pragma unroll
+      for (int nb = 0; nb < D / 16; ++nb) *reinterpret_cast<f32x4_t*>(&s.acc[wave][col][16 * nb + 4 * grp]) = acc[nb];
+    }
+    meet();
+    const int tid = anew(this->tid);
+    for (int idx = tid; idx < G * (D / 4); idx += THREADS) {
+      const int row = idx / (D / 4), d = idx % (D / 4) * 4;
+      float m[WAVES + 1], mr = -INFINITY, lr = 0.f;
+#pragma unroll
+      for (int v = 0; v <= WAVES; ++v) mr = fmaxf(mr, m[v] = s.m[v][row]);
+      f32x4_t o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int v = 0; v < WAVES; ++v) {
+        const float weight = m[v] > -INFINITY ? fast_exp2(m[v] - mr) : 0.f;
+        lr += s.l[v][row] * weight;
+        o += *reinterpret_cast<const f32x4_t*>(&s.acc[v][row][d]) * weight;
+      }
+      if (m[WAVES] > -INFINITY) {
+        const float weight = fast_exp2(m[WAVES] - mr);
+        lr += weight;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] += s.v[d + e] * weight;
+      }
+      if (a.splits == 1) {
+        const float inv = lr > 0.f ? 1.f / lr : lr;      // (a row that sees nothing, a sequence without a length, is zero)
+        union {
+          uint2 u;
+          __bf16 e[4];
+        } pk;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) pk.e[e] = (__bf16)(o[e] * inv);
+        put8(ex, a.at_att + ((b * a.heads + g_kv * G + row) * D + d) * 2, pk.u);
+      } else {
+        const int slot = ((b * a.kv_heads + g_kv) * a.splits + split) * G + row;
+        u32x4_t p;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) p[e] = marked(__float_as_uint(o[e]), 0x7fc00000u);
+        __builtin_amdgcn_raw_buffer_store_b128(p, ex, a.at_part + (slot * D + d) * 4, 0, THROUGH);
+        if (d == 0) {
+          const u32x2_t ml = {marked(__float_as_uint(mr), 0x7fc00000u), marked(__float_as_uint(lr), 0x7fc00000u)};
+          __builtin_amdgcn_raw_buffer_store_b64(ml, ex, a.at_part + (a.rows * a.heads * a.splits * D + slot * 2) * 4, 0, THROUGH);
+        }
+      }
+    }
+    if (brings_new && pos >= 0 && tid >= THREADS - 2 * HEAD) {       // the token's key and value into the caches, for later steps
+      const int d = tid & (HEAD - 1), blk = pos / a.page, at = pos % a.page;
+      const int pg = blk < a.table_width ? ((entries_ptr)(uintptr_t)(a.block_table + (size_t)b * a.table_width))[blk] : -1;
+      if (pg >= 0 && pg < a.num_pages) {
+        const size_t head = (size_t)pg * a.kv_heads + g_kv;
+        const bool value = tid >= THREADS - HEAD;
+        auto dst = (__attribute__((address_space(1))) uint16_t*)(value ? values : keys) + head * D * a.page;
+        dst[value ? (size_t)d * a.page + at : (size_t)at * D + d] = float_to_bf16(value ? s.v[d] : s.k[d]).bits;
+      }
+    }
+    meet();      // (whoever writes here next)
+  }
+
+  // The splits of sequence `b` and key head `g_kv`, joined
+  __device__ __forceinline__ void merge(__amdgpu_buffer_rsrc_t ex, int g_kv, int b) {
+    constexpr int D = HEAD, N = 8;
+    const int tid = anew(this->tid), G = a.heads / a.kv_heads, all = a.rows * a.heads * a.splits * D;
+    for (int idx = tid; idx < ((G * (D / 4) + 63) & ~63); idx += THREADS) {
+      const int r = min(idx / (D / 4), G - 1), d = idx % (D / 4) * 4;
+      float m = -INFINITY, sum = 0.f;
+      f32x4_t o = {0.f, 0.f, 0.f, 0.f};
+      for (int s0 = 0; s0 < a.splits; s0 += N) {
+        u32x4_t p[N];
+        u32x2_t ml[N];
+        for (int n = 0;; ++n) {
+          compiler_fence();
+          bool ok = true;
+#pragma unroll
+          for (int s = 0; s < N; ++s) {
+            const int slot = ((b * a.kv_heads + g_kv) * a.splits + min(s0 + s, a.splits - 1)) * G + r;
+            p[s] = peek16(ex, a.at_part + (slot * D + d) * 4);
+            ml[s] = __builtin_amdgcn_raw_buffer_load_b64(ex, a.at_part + (all + slot * 2) * 4, 0, THROUGH);
+          }
+#pragma unroll
+          for (int s = 0; s < N; ++s) ok = ok && there(p[s]) && ml[s].x != ABSENT && ml[s].y != ABSENT;
+          if (__all(ok) || !again(n)) break;
+        }
+        float m_all = m;
+#pragma unroll
+        for (int s = 0; s < N; ++s)
+          if (s0 + s < a.splits) m_all = fmaxf(m_all, __uint_as_float(ml[s].x));
+        const float kept = m > -INFINITY ? fast_exp2(m - m_all) : 0.f;
+        sum *= kept;
+        o *= kept;
+#pragma unroll
+        for (int s = 0; s < N; ++s)
+          if (s0 + s < a.splits && __uint_as_float(ml[s].x) > -INFINITY) {
+            const float weight = fast_exp2(__uint_as_float(ml[s].x) - m_all);
+            sum += __uint_as_float(ml[s].y) * weight;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] += __uint_as_float(p[s][e]) * weight;
+          }
+        m = m_all;
+      }
+      const float inv = sum > 0.f ? 1.f / sum : sum;
+      union {
+        uint2 u;
+        __bf16 e[4];
+      } pk;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) pk.e[e] = (__bf16)(o[e] * inv);
+      if (idx < G * (D / 4)) put8(ex, a.at_att + ((b * a.heads + g_kv * G + r) * D + d) * 2, pk.u);
+    }
+  }
+
+  __device__ __forceinline__ void layers() {
+    const int items = a.rows * a.kv_heads * a.splits;
+    const Item mine = item_of(min(rank, items - 1));
+    look_ahead(0, 0);
+#pragma unroll 1
+    for (int n = 0; n < a.count; ++n) {
+      const auto ex = buffer_of(a.exchange + n * a.per_layer, a.per_layer);
+      const bool last = n == a.count - 1;
+#pragma unroll 1
+      for (int which = 0; which < 4; ++which) {
+        // (new numbers to the compiler: it would otherwise work out every product's addresses ahead of all of them, and has no registers for those)
+        asm volatile("" : "+v"(lane), "+v"(tid));
+        if (which == 1) {
+#pragma unroll 1
+          for (int n_item = rank; n_item < items; n_item += blocks) {
+            Item it = mine;
+            if (n_item != rank) it = item_of(n_item);
+            attend(ex, n, it);
+          }
+          if (a.splits > 1)      // (its loads would come behind the next weights')
+#pragma unroll 1
+            for (int pair = rank >= blocks / 4 ? rank - blocks / 4 : rank + blocks - blocks / 4; pair < a.rows * a.kv_heads; pair += blocks)
+              merge(ex, pair % a.kv_heads, pair / a.kv_heads);
+          look_ahead(n, 1);
+        }
+        const Product p = shares.of(which);
+        if (p.count == 0) continue;
+        Rows r;
+        r.ex = which == 0 ? buffer_of(a.exchange + (n - 1) * a.per_layer, a.per_layer) : ex;
+        r.src = which == 0 ? a.at_out : which == 1 ? a.at_att : which == 2 ? a.at_mid : a.at_hid;
+        r.sums = which == 0 ? a.at_out_sums : which == 2 ? a.at_mid_sums : 0;
+        r.K = p.steps * 32;
+        r.eps = __uint_as_float(which == 0 ? (unsigned)entry(n, EPS) : (unsigned)(entry(n, EPS) >> 32));
+        const void* norm = which == 1 ? (const void*)entry(n, MIDDLE_NORM) : which == 3 && !last ? (const void*)entry(n + 1, ENTRY_NORM) : nullptr;
+        product_of(r, ex, n, which, p, norm);
+      }
+    }
+    if (!alive) {              // a wait that did not end: no number of the result stands
+      const Product p = shares.of(3);
+      for (int done = 0; done < p.count; ++done)
+        for (int idx = tid; idx < 16 * a.rows; idx += THREADS)
+          a.residual[(size_t)(idx >> 4) * a.width + (p.first + done * blocks) * 16 + (idx & 15)] = __uint_as_float(0x7fc00000u);
+    }
+  }
+};
+
+// The blocks that are here when the launch begins share its work; one that only finds room later has none. Nothing is assumed
+// about how many run at once, so two such launches on two streams, or a kernel that keeps some of the processors, cannot wait
+// for each other without end. control[0]: how many have come, and CLOSED; control[1]: how many there are, if not all came in time.
+__device__ __forceinline__ void gather(const Args& a, int& rank, int& blocks) {
+  unsigned* came = a.control;
+  const unsigned ticket = __hip_atomic_fetch_add(came, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  rank = blocks = 0;
+  if (ticket & CLOSED) return;
+  for (int n = 0;; ++n) {
+    unsigned now = __hip_atomic_load(came, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (now == gridDim.x) {
+      rank = blockIdx.x;
+      blocks = gridDim.x;
+      return;
+    }
+    if (!(now & CLOSED) && n >= a.patience) {
+      const unsigned seen = now;
+      if (__hip_atomic_compare_exchange_strong(came, &now, seen | CLOSED, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        __hip_atomic_store(came + 1, seen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      continue;
+    }
+    if (now & CLOSED) {
+      const unsigned closed_at = __hip_atomic_load(came + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (closed_at) {
+        rank = ticket;
+        blocks = closed_at;
+        return;
+      }
+      if (n >= a.patience + a.limit) return;
+    }
+    __builtin_amdgcn_s_sleep(2);
+  }
+}
+
+template <typename QKW>
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void decode_layers_kernel(Args a) {
+  __shared__ Shared sh;
+  if (threadIdx.x == 0) gather(a, sh.rank, sh.blocks);
+  __syncthreads();
+  const int rank = __builtin_amdgcn_readfirstlane(sh.rank), blocks = __builtin_amdgcn_readfirstlane(sh.blocks);
+  if (blocks == 0) return;
+  for (int i = threadIdx.x; i < a.count * LAYER_WORDS; i += THREADS) sh.layers[i] = reinterpret_cast<const uint64_t*>(a.layers)[i];
+  __syncthreads();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  Block<QKW> b{sh, a, rank, blocks, wave, (int)threadIdx.x & 63, (int)threadIdx.x, shares_of(a, rank, blocks), a.limit, 1, (1u << 20) / a.rows + 1, 0, -1};
+  b.layers();
+}
+
+// The launch's table, its control words, an exchange without a word in it, and before its first layer's part the stream's rows as a
+// last product would leave them there.
+struct Entry {
+  const float* residual;
+  const void* norm;
+  int rows, width, norm_f32;
+  char *out, *sums;
+};
+__global__ __launch_bounds__(256) void decode_layers_begin_kernel(LayerPack pack, int first, int count, Layer* layers, unsigned* control, uint4* exchange,
+                                                                  long pieces, Entry entry) {
+  if (blockIdx.x == 0) {
+    const unsigned* from = reinterpret_cast<const unsigned*>(&pack);
+    unsigned* to = reinterpret_cast<unsigned*>(layers + first);
+    for (int i = threadIdx.x; i < count * (int)(sizeof(Layer) / 4); i += 256) to[i] = from[i];
+    if (threadIdx.x < 2) control[threadIdx.x] = 0;
+  }
+  const long each = (long)gridDim.x * 256, me = (long)blockIdx.x * 256 + threadIdx.x;
+  for (long i = me; i < pieces; i += each) exchange[i] = make_uint4(ABSENT, ABSENT, ABSENT, ABSENT);
+  for (long i = me; i < (long)entry.rows * entry.width / 4; i += each) {       // (sixteen columns are four neighbouring lanes')
+    const float4 x = reinterpret_cast<const float4*>(entry.residual)[i];
+    const int n = (int)(i * 4 % entry.width);
+    float4 w;
+    if (entry.norm_f32) {
+      w = *reinterpret_cast<const float4*>(static_cast<const float*>(entry.norm) + n);
+    } else {
+      const uint2 v = *reinterpret_cast<const uint2*>(static_cast<const bf16_t*>(entry.norm) + n);
+      w = make_float4(__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xffff0000u));
+    }
+    union {
+      uint2 u;
+      __bf16 e[4];
+    } pk;
+    pk.e[0] = (__bf16)(x.x * w.x), pk.e[1] = (__bf16)(x.y * w.y), pk.e[2] = (__bf16)(x.z * w.z), pk.e[3] = (__bf16)(x.w * w.w);
+    reinterpret_cast<uint2*>(entry.out)[i] = make_uint2(marked(pk.u.x, 0x7fc07fc0u), marked(pk.u.y, 0x7fc07fc0u));
+    float ss = x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w;
+    ss += __shfl_xor(ss, 1, 64);
+    ss += __shfl_xor(ss, 2, 64);
+    if ((i & 3) == 0) reinterpret_cast<unsigned*>(entry.sums)[i / 4] = marked(__float_as_uint(ss), 0x7fc00000u);
+  }
+}
+
+inline long up(long n) { return (n + 255) & ~255l; }
+
+struct Layout {
+  long part, att, mid, mid_sums, hid, out, out_sums, size;
+};
+inline Layout layout_of(long rows, long width, long heads, long kv_heads, long inner, long splits) {
+  Layout l;
+  l.part = up(rows * (heads + 2 * kv_heads) * HEAD * 2);
+  l.att = l.part + (splits > 1 ? up(rows * heads * splits * (HEAD + 2) * 4) : 0);
+  l.mid = l.att + up(rows * heads * HEAD * 2);
+  l.mid_sums = l.mid + up(rows * width * 2);
+  l.hid = l.mid_sums + up(rows * (width / 16) * 4);
+  l.out = l.hid + up(rows * inner * 2);
+  l.out_sums = l.out + up(rows * width * 2);
+  l.size = l.out_sums + up(rows * (width / 16) * 4);
+  return l;
+}
+
+// (every wavefront of a block has a step of 32 of each product's K at least: the smallest K is 256, from two heads on)
+inline bool sizes_fit(int rows, int width, int heads, int kv_heads, int dim, int inner) {
+  return rows >= 1 && rows <= MOST_ROWS && dim == HEAD && heads >= 1 && kv_heads >= 1 && heads % kv_heads == 0 && heads / kv_heads <= 16 &&
+         width >= 32 * WAVES && width % 128 == 0 && inner >= 32 * WAVES && inner % 128 == 0 && heads * HEAD >= 32 * WAVES &&
+         width <= (1 << 16) && inner <= (1 << 18) && heads <= 512;
+}
+
+}  // namespace
+
+extern "C" {
+
+// Bytes of workspace for a step of `rows` single tokens over `count` layers: the layers' table, the control words, the exchange;
+// 0 for sizes that are not taken.
+long q3_decode_layers_workspace(int count, int rows, int width, int heads, int kv_heads, int dim, int inner, int splits) {
+  if (count < 1 || count > MOST_LAYERS || !sizes_fit(rows, width, heads, kv_heads, dim, inner) || splits < 1 || splits > MOST_SPLITS) return 0;
+  const Layout l = layout_of(rows, width, heads, kv_heads, inner, splits);
+  if (l.size > (1l << 30)) return 0;
+  return up((long)count * sizeof(Layer)) + 256 + (count + 1) * l.size;
+}
+
+// Row b is the one token of sequence b, at position kv_lens[b] - 1, whose key and value are written to the caches; `residual` (rows,
+// width) float32 is the stream, which the layers add to in place. `blocks`: of the launch (0: one per processor); `patience`, `limit`: looks
+// before the launch goes on with the blocks it has, and before a wait gives up.
+int q3_decode_layers(const Layer* layers, int count, float* residual, int rows, int width, int heads, int kv_heads, int dim, int inner,
+                     int norm_dtype, int qk_dtype, float qk_eps, float scale, const float* table, int rotary_dim, int max_pos,
+                     const int* block_table, int table_width, const int* kv_lens, int max_kv_len, int page, int num_pages, int splits,
+                     void* workspace, int blocks, int patience, int limit, hipStream_t stream) {
+  if (!layers || !residual || !block_table || !kv_lens || !workspace || count < 1 || count > MOST_LAYERS || page < 16 || (page & (page - 1)) || num_pages < 1)
+    return Q3_ERR_BAD_ARGUMENT;
+  if (!sizes_fit(rows, width, heads, kv_heads, dim, inner) || splits < 1 || splits > MOST_SPLITS || (table && rotary_dim != dim))
+    return Q3_ERR_UNSUPPORTED;
+  if ((table && max_kv_len > max_pos) || (long)table_width * page < max_kv_len || max_kv_len < 1 || patience < 1 || limit < 1 || blocks < 0)
+    return Q3_ERR_BAD_ARGUMENT;
+  if ((norm_dtype != Q3_F32 && norm_dtype != Q3_BF16) || (qk_dtype != Q3_F32 && qk_dtype != Q3_BF16)) return Q3_ERR_BAD_ARGUMENT;
+  for (int i = 0; i < count; ++i) {
+    const Layer& l = layers[i];
+    if (!l.w[0] || !l.w[1] || !l.w[2] || !l.w[3] || !l.entry_norm || !l.middle_norm || !l.keys || !l.values ||
+        (l.q_norm == nullptr) != (l.k_norm == nullptr))
+      return Q3_ERR_BAD_ARGUMENT;
+  }
+  if (blocks == 0) {
+    int device = 0;
+    hipError_t status = hipGetDevice(&device);
+    if (status == hipSuccess) status = hipDeviceGetAttribute(&blocks, hipDeviceAttributeMultiprocessorCount, device);
+    if (status != hipSuccess) return (int)status;
+  }
+  const Layout l = layout_of(rows, width, heads, kv_heads, inner, splits);
+  if (l.size > (1l << 30)) return Q3_ERR_UNSUPPORTED;
+  Layer* held = (Layer*)workspace;
+  unsigned* control = (unsigned*)((char*)workspace + up((long)count * sizeof(Layer)));
+  char *entry_part = (char*)control + 256, *exchange = entry_part + l.size;
+  const long pieces = count * l.size / 16;
+  const Entry entry{residual, layers[0].entry_norm, rows, width, norm_dtype == Q3_F32, entry_part + l.out, entry_part + l.out_sums};
+  for (int first = 0; first < count; first += LAYERS_A_LAUNCH) {
+    const int n = count - first < LAYERS_A_LAUNCH ? count - first : LAYERS_A_LAUNCH;
+    LayerPack pack{};
+    for (int i = 0; i < n; ++i) pack.layer[i] = layers[first + i];
+    const long share = first == 0 ? pieces : 0;
+    const long wanted = (share + 2047) / 2048;
+    hipLaunchKernelGGL(decode_layers_begin_kernel, dim3((unsigned)(wanted < 1 ? 1 : wanted > 1024 ? 1024 : wanted)), dim3(256), 0, stream, pack, first, n,
+                       held, control, (uint4*)exchange, share, first == 0 ? entry : Entry{});
+  }
+  Args a{};
+  a.layers = held;
+  a.control = control;
+  a.exchange = exchange;
+  a.residual = residual;
+  a.table = table;
+  a.block_table = block_table;
+  a.kv_lens = kv_lens;
+  a.per_layer = l.size;
+  a.at_part = (int)l.part, a.at_att = (int)l.att, a.at_mid = (int)l.mid, a.at_mid_sums = (int)l.mid_sums, a.at_hid = (int)l.hid;
+  a.at_out = (int)l.out, a.at_out_sums = (int)l.out_sums;
+  a.count = count, a.rows = rows, a.width = width, a.heads = heads, a.kv_heads = kv_heads, a.inner = inner;
+  a.norm_f32 = norm_dtype == Q3_F32;
+  a.max_pos = max_pos, a.table_width = table_width, a.page = page, a.num_pages = num_pages, a.splits = splits;
+  a.patience = patience, a.limit = limit;
+  a.qk_eps = qk_eps;
+  a.scale_log2 = make_score_scale(scale);
+  if (qk_dtype == Q3_F32)
+    hipLaunchKernelGGL(decode_layers_kernel<float>, dim3(blocks), dim3(THREADS), 0, stream, a);
+  else
+    hipLaunchKernelGGL(decode_layers_kernel<bf16_t>, dim3(blocks), dim3(THREADS), 0, stream, a);
+  return q3_launch_status();
+}
+
+}  // extern "C"

@@ -7,7 +7,7 @@ import torch
 from ..parts.base import UnscaledRows, build_part
 from ..parts.linear import copy_float32_matrices
 from ..weights.checkpoint import check_tensors
-from .layer_run import layer_runs
+from .layer_run import decode_run, layer_runs
 
 
 class _Layer:
@@ -58,6 +58,7 @@ class DecoderModel:
         # each run-order entry that owns a cache gets a plane; readers point at the owner's
         self.observer = None      # called with (run-order entry, stream, what it still lacks) behind every layer
         self.runs = {}            # step -> the stretch of layers that may run as one native call with it (set by load)
+        self.decode_run = None    # all layers in one launch, for steps of single tokens (set by load)
         self.plane_of_step = []
         self.plane_needs = []
         for i, step in enumerate(spec.order):
@@ -132,6 +133,7 @@ class DecoderModel:
                 part.load(fetch)
             copy_float32_matrices(self.parts())
         self.runs = layer_runs(self)
+        self.decode_run = decode_run(self)
         return self
 
     @torch.no_grad()
@@ -145,6 +147,8 @@ class DecoderModel:
         pending = None
         order = self.spec.order
         behind = 0                           # the first step that is not done yet
+        if self.decode_run is not None and self.observer is None and self.decode_run.forward(x, batch, cache):
+            behind = len(order)
         declined = None                      # the stretch of layers that left this pass to their parts: not asked again
         for i, step in enumerate(order):
             if i < behind:

@@ -177,3 +177,115 @@ class DecoderLayers:
             return Declined(layer, operation == _ATTENTION_OUT, attended if operation == _ATTENTION_OUT else hidden)
         _check(status, _OPERATIONS[operation])
         return out, exit_
+
+
+DECODE_ROWS_MOST = 16          # rows of a step of single tokens that `DecodeLayers` takes
+
+
+class _DecodeLayer(ctypes.Structure):
+    _fields_ = [(n, _P) for n in ("qkv", "out", "gate_up", "down", "q_norm", "k_norm", "entry_norm", "middle_norm", "keys", "values")
+                ] + [("entry_eps", _F), ("middle_eps", _F)]
+
+
+class DecodeLayers:
+    """All layers of one shape for steps of single tokens, in one launch (csrc/decode_layers.hip): `layers` as `DecoderLayers` has
+    them, and their tile-ordered matrices (`qkv_tiles`, `out_tiles`, `gate_up_tiles`, `down_tiles`) and `entry_norm`. The tensors
+    are looked at here, once; `None` from `of` if they are not what the launch takes."""
+
+    def __init__(self, layers, heads, kv_heads, dim, width, inner, qk_eps, scale):
+        self.layers = layers
+        self.heads, self.kv_heads, self.dim, self.width, self.inner = heads, kv_heads, dim, width, inner
+        self.qk_eps, self.scale = float(qk_eps), float(scale)
+        self.norm_dtype = layers[0]["middle_norm"].dtype
+        self.qk_dtype = layers[0]["q_norm"].dtype if layers[0]["q_norm"] is not None else torch.float32
+        lib = library("decode_layers")
+        lib.q3_decode_layers_workspace.restype = ctypes.c_long
+        self._workspace = lib.q3_decode_layers_workspace
+
+    @classmethod
+    def of(cls, layers, heads, kv_heads, dim, width, inner, qk_eps, scale, window):
+        norm_dtype = getattr(layers[0]["middle_norm"], "dtype", None)
+        if window or norm_dtype not in _DT:
+            return None
+        for l in layers:
+            for name, shape in (("qkv", ((heads + 2 * kv_heads) * dim, width)), ("out", (width, heads * dim)),
+                                ("gate_up", (2 * inner, width)), ("down", (width, inner))):
+                if not (l[name] is not None and l[name].shape == shape and shape[0] % 16 == 0
+                        and _vector(l[name + "_tiles"], shape[0] * shape[1], torch.bfloat16)):
+                    return None
+            if not (_vector(l["entry_norm"], width, norm_dtype) and _vector(l["middle_norm"], width, norm_dtype)):
+                return None
+            if (l["q_norm"] is None) != (l["k_norm"] is None) or (l["q_norm"] is None) != (layers[0]["q_norm"] is None):
+                return None
+            if l["q_norm"] is not None and not (l["q_norm"].dtype in _DT and _vector(l["q_norm"], dim, layers[0]["q_norm"].dtype)
+                                                and _vector(l["k_norm"], dim, layers[0]["q_norm"].dtype)):
+                return None
+            if any(l[n].data_ptr() % 16 for n in ("entry_norm", "middle_norm", "q_norm", "k_norm") if l[n] is not None):
+                return None
+        found = cls(layers, heads, kv_heads, dim, width, inner, qk_eps, scale)
+        return found if found._workspace(1, 1, width, heads, kv_heads, dim, inner, 1) > 0 else None
+
+    def splits(self, rows, max_kv_len):
+        """Into how many blocks a sequence's keys are shared out: as many as leave each wavefront a tile of 32 keys, while there is a
+        block for each share."""
+        tiles = -(-int(max_kv_len) // 32)
+        return max(1, min(256 // (rows * self.kv_heads), -(-tiles // 8), 32))
+
+    def run(self, stream, caches, block_table, kv_lens, max_kv_len, table, blocks=0, patience=64):
+        """The layers over the residual `stream` (T, width) float32, in place: row b is sequence b's one token, at position
+        kv_lens[b] - 1 of its caches (per layer keys and values as `decode_attention` takes them). Whether that was done: not for a step
+        or pages that the launch does not take. `blocks`, `patience`: of how many blocks (0: one per compute unit), and how often they
+        look for each other before those that are there go on by themselves."""
+        if not (stream.dim() == 2 and caches and caches[0][0].dim() == 4):
+            raise OperandError("a stream (T, width), keys (pages, Hkv, page, D)")
+        T = stream.shape[0]
+        H, G, D, page = self.heads, self.kv_heads, self.dim, caches[0][0].shape[2]
+        if not 1 <= T <= DECODE_ROWS_MOST or page < 16 or page & (page - 1) or (table is not None and table.shape[1] != D):
+            return False
+        count = len(self.layers)
+        if len(caches) != count:
+            raise OperandError("a cache for each of the layers")
+        if not (stream.is_cuda and stream.shape == (T, self.width) and stream.dtype == torch.float32 and stream.is_contiguous()):
+            raise OperandError("a float32 stream (T, width), contiguous")
+        if not (kv_lens.is_cuda and kv_lens.dtype == torch.int32 and kv_lens.shape == (T,) and kv_lens.is_contiguous()):
+            raise OperandError("kv_lens int32, one per row")
+        if not (block_table.is_cuda and block_table.dim() == 2 and block_table.dtype == torch.int32 and block_table.shape[0] >= T
+                and block_table.is_contiguous() and block_table.shape[1] * page >= max_kv_len):
+            raise OperandError("block_table must be int32 (B, W) and hold the longest sequence")
+        pages = caches[0][0].shape[0]
+        for keys, held in caches:
+            if not (keys.is_cuda and keys.dtype == torch.bfloat16 and keys.shape == (pages, G, page, D) and keys.is_contiguous()
+                    and held.is_cuda and held.dtype == torch.bfloat16 and held.shape == (pages, G, D, page) and held.is_contiguous()
+                    and pages > 0):
+                raise OperandError("caches must be keys (pages, Hkv, page, D) and values (pages, Hkv, D, page) in bfloat16")
+        max_pos = 0
+        if table is not None:
+            if not (table.is_cuda and table.dim() == 2 and table.dtype == torch.float32 and table.is_contiguous()
+                    and max_kv_len <= table.shape[0]):
+                raise OperandError("table must be float32 (P, D) and hold the step's last position")
+            max_pos = table.shape[0]
+        if any(t.data_ptr() % 16 for t in (stream, *(table,) * (table is not None), *(t for pair in caches for t in pair))):
+            return False
+        splits = self.splits(T, max_kv_len)
+        size = self._workspace(count, T, self.width, H, G, D, self.inner, splits)
+        if size <= 0:
+            return False
+        workspace = torch.empty(size, dtype=torch.uint8, device=stream.device)
+        layers = (_DecodeLayer * count)()
+
+        def at(t):
+            return None if t is None else t.data_ptr()
+
+        for native, l, (keys, held) in zip(layers, self.layers, caches):
+            for name in ("qkv", "out", "gate_up", "down"):
+                setattr(native, name, at(l[name + "_tiles"]))
+            for name in ("q_norm", "k_norm", "entry_norm", "middle_norm"):
+                setattr(native, name, at(l[name]))
+            native.keys, native.values = keys.data_ptr(), held.data_ptr()
+            native.entry_eps, native.middle_eps = l["entry_eps"], l["middle_eps"]
+        _check(library("decode_layers").q3_decode_layers(
+            layers, count, _P(at(stream)), T, self.width, H, G, D, self.inner, _DT[self.norm_dtype], _DT[self.qk_dtype],
+            _F(self.qk_eps), _F(self.scale), _P(at(table)), D if table is not None else 0, max_pos, _P(at(block_table)),
+            block_table.shape[1], _P(at(kv_lens)), int(max_kv_len), page, pages, splits, _P(at(workspace)), int(blocks), int(patience),
+            1 << 18, _stream()), "the layers of a step of single tokens")
+        return True

@@ -101,7 +101,8 @@ class PagedAttention(Part):
         """What a native stretch of layers (`ops.layers.DecoderLayers`) needs of this part, or None."""
         if type(self) is not PagedAttention or self.qkv is None:
             return None
-        return (dict(qkv=self.qkv.weight, out=self.out.weight, q_norm=self.q_weight, k_norm=self.k_weight),
+        return (dict(qkv=self.qkv.weight, out=self.out.weight, qkv_tiles=self.qkv.tiled, out_tiles=self.out.tiled, q_norm=self.q_weight,
+                     k_norm=self.k_weight),
                 dict(heads=self.num_heads, kv_heads=self.num_kv_heads, dim=self.head_dim, width=self.hidden_size,
                      qk_eps=self.qk_norm_eps, scale=self.scale, window=self.window))
 

@@ -51,11 +51,12 @@ class PreNormBlock(Part):
         NormSink), or None if this block's mixer wants finished rows."""
         return self.mixer_norm if _says(self.mixer, "takes_unscaled") and hasattr(self.mixer_norm, "sink_for") else None
 
-    def native_layer(self, next_norm):
+    def native_layer(self, next_norm=None):
         """(a layer's tensors, the sizes that equal layers share, the position part) for `ops.layers.DecoderLayers`, or None
-        for a layer of other parts, or of parts that do not go from UnscaledRows to UnscaledRows."""
+        for a layer of other parts, or of parts that do not go from UnscaledRows to UnscaledRows; without the norm that follows, for
+        `ops.layers.DecodeLayers`."""
         parts = (self.mixer, self.feed_forward)
-        norms = (self.mixer_norm, self.feed_forward_norm, next_norm)
+        norms = (self.mixer_norm, self.feed_forward_norm) + ((next_norm,) if next_norm is not None else ())
         if type(self) is not PreNormBlock or not all(hasattr(part, "native_half") for part in parts):
             return None
         if not all(type(norm) is RMSNorm and norm.weight is not None for norm in norms):
@@ -66,8 +67,9 @@ class PreNormBlock(Part):
         if None in halves:
             return None
         (mixing, sizes), (feeding, more) = halves
-        return (dict(mixing, **feeding, middle_norm=norms[1].weight, next_norm=norms[2].weight, entry_eps=norms[0].eps,
-                     middle_eps=norms[1].eps), dict(sizes, **more), self.mixer.position)
+        return (dict(mixing, **feeding, entry_norm=norms[0].weight, middle_norm=norms[1].weight,
+                     next_norm=None if next_norm is None else next_norm.weight, entry_eps=norms[0].eps, middle_eps=norms[1].eps),
+                dict(sizes, **more), self.mixer.position)
 
     def forward(self, x, pending, batch, cache, next_norm=None):
         """`pending`: None, the addend the stream still lacks, or UnscaledRows

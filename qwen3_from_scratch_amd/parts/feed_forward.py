@@ -61,7 +61,8 @@ class SwiGLU(Part):
         """What a native stretch of layers (`ops.layers.DecoderLayers`) needs of this part, or None."""
         if type(self) is not SwiGLU or self.activation != "silu" or self.gate_up is None:
             return None
-        return dict(gate_up=self.gate_up.weight, down=self.down.weight), dict(inner=self.intermediate_size)
+        return (dict(gate_up=self.gate_up.weight, down=self.down.weight, gate_up_tiles=self.gate_up.tiled, down_tiles=self.down.tiled),
+                dict(inner=self.intermediate_size))
 
     def forward(self, x, batch=None, sink=None):
         h = self.gate_up.forward_swiglu(x, self.activation)
