@@ -11,13 +11,16 @@
 // meanwhile.
 //
 // What it measured (us a step in a graph, the layers' kernels one by one / this): the 0.6B shape, one request over 1,100 keys
-// 1,013 / 809, over 30,000 1,545 / 1,366, eight over 2,000 1,415 / 1,155, sixteen 1,910 / 1,686; the 8B shape, one over 2,060 3,407 / 3,026,
-// eight 3,954 / 3,510, eight over 8,000 5,057 / 4,636, sixteen over 300 3,849 / 3,754, over 2,060 4,836 / 4,520. None of 28 sizes between
-// was slower; more than 16 rows have no registers here.
+// 1,013 / 701; the 8B shape, one over 2,060 3,407 / 2,820, eight 3,954 / 3,440. The first form of this kernel (805, 3,012, 3,561) was faster
+// than the kernels at each of 28 sizes from 1 to 16 rows and 100 to 30,000 keys; more than 16 rows have no registers here.
 //
-// What bounds it: one request of the small shape the chain of five or six exchanges a layer, 26 us, of which the way through memory is
-// some 7 and the rest the few hundred instructions of each wavefront between them; the large shape its weights (5.0 of the 5.8 TB/s that
-// a plain read reaches, the whole step through) and the attention's part, where no weights move.
+// What bounds it: one request of the small shape the chain of five or six exchanges a layer; a look that fails costs a second one behind
+// the first, a store holds up the wavefront's next look (they come back in order), and a wavefront alone on its SIMD takes 4 to 5 cycles
+// an instruction, 20 for a number that goes from a vector's lane into scalar arithmetic. So what is between two exchanges is kept short:
+// offsets that are constants of an instruction, steps of K in one stretch, bounds by the descriptors (500 instructions a product less:
+// 801 -> 779), the next weights asked for behind the results (779 -> 749; 8B 2,990 -> 2,860) and behind all wavefronts' results, with
+// the shares of K read together (749 -> 701; 2,860 -> 2,820). The large shape is bound by its weights (5.4 of the 5.8 TB/s that a
+// plain read reaches, the whole step through) and the attention's part, where few weights move.
 // What did not help: the block split into wavefronts that multiply and wavefronts that look, prepare and store, with the weights in a
 // ring in shared memory (0.6B 905: more handovers a product), asking for the sums of squares together with the rows (lines that many blocks
 // write and all ask for again and again are slow to change: 915), copies of what all read (nothing), the first keys asked for ahead of
@@ -43,6 +46,7 @@ constexpr int THROUGH = 16;                   // cache policy of what blocks exc
 constexpr int MOST_SPLITS = 32;
 constexpr int MOST_ROWS = 16;
 constexpr int MOST_LAYERS = 128;
+constexpr int NOWHERE = 1 << 30;              // an offset behind the end of every buffer: reads of it are zero
 
 // One layer as the host gives it and as the launch's table holds it.
 struct Layer {
@@ -65,7 +69,7 @@ struct Args {
   const int *block_table, *kv_lens;
   long per_layer;              // bytes of exchange
   int at_part, at_att, at_mid, at_mid_sums, at_hid, at_out, at_out_sums;
-  int count, rows, width, heads, kv_heads, inner, norm_f32, max_pos, table_width, page, num_pages, splits, patience, limit;
+  int count, rows, width, heads, kv_heads, group, inner, norm_f32, max_pos, table_width, page, page_bits, num_pages, splits, patience, limit;
   float qk_eps, scale_log2;
 };
 
@@ -80,6 +84,7 @@ struct Shared {
   __attribute__((aligned(16))) char red[2][RESULTS * WAVES * 4 * 16];
   AttentionShared attention;
   __attribute__((aligned(16))) uint64_t layers[MOST_LAYERS * sizeof(Layer) / 8];
+  uint64_t first_at[THREADS][2];              // where a thread's first keys and values of the block's first item lie in each layer's caches
   float scale[16];
   int rank, blocks;
 };
@@ -100,7 +105,7 @@ __device__ __forceinline__ void store16(void* p, const u32x4_t& v) { *(__attribu
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, long bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
 }
-__device__ __forceinline__ u32x4_t peek16(__amdgpu_buffer_rsrc_t r, int at) { return __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, THROUGH); }
+__device__ __forceinline__ u32x4_t peek16(__amdgpu_buffer_rsrc_t r, int at, int base = 0) { return __builtin_amdgcn_raw_buffer_load_b128(r, at, base, THROUGH); }
 __device__ __forceinline__ bool there(const u32x4_t& v) { return v.x != ABSENT && v.y != ABSENT && v.z != ABSENT && v.w != ABSENT; }
 // A word of results that happens to be the mark (not a number, either way) becomes another one.
 __device__ __forceinline__ unsigned marked(unsigned w, unsigned instead) { return w == ABSENT ? instead : w; }
@@ -116,38 +121,37 @@ __device__ __forceinline__ void compiler_fence() { asm volatile("" ::: "memory")
 // Until shared memory holds what the block's wavefronts have written (and nothing about memory)
 __device__ __forceinline__ void meet() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// ---- which slabs of 16 weight rows a block multiplies ----
+// ---- which slabs of 16 weight rows a block multiplies, and which steps of 32 of K a wavefront ----
 
-struct Product {
-  int first, count, steps;     // slabs first, first + blocks, ...; k in steps of 32
-};
-// The four products of a layer: [q | k | v], the attention's output, gate and up, down. The two that add into the stream go to the same
-// blocks, which are others than those of the attention's first items.
-struct Shares {
-  int rank, shifted, qkv, stream, gate_up;             // of a block: the first slabs, how many
-  int width_steps, heads_steps, inner_steps;
-  __device__ __forceinline__ Product of(int which) const {
-    // (the members' values first: a choice between the members themselves is one between addresses, and the struct then lies in memory)
-    const int into = stream, at = shifted, first = rank, first_count = qkv, third = gate_up, s0 = width_steps, s1 = heads_steps, s3 = inner_steps;
-    return Product{which & 1 ? at : first, which & 1 ? into : which == 0 ? first_count : third, which == 1 ? s1 : which == 3 ? s3 : s0};
+// What a wavefront knows of a product, each number in a lane of one register (lane 16 product + number): numbers that are computed
+// where they are needed, over and over, are what the compiler moves ahead of loops, 500 instructions a product on the way from one
+// exchange to the next. A block has the slabs SLAB, SLAB + blocks, ..; the two products that add into the stream go to
+// blocks others than those of the attention's first items.
+enum { OWN, FIRST_STEP, START, STRIDE, COUNT, SLAB, SRC, SUMS, DST, DST_SUMS, ROW_BYTES, OUT_WIDTH };
+__device__ __forceinline__ int numbers_of(const Args& a, int rank, int blocks, int wave, int lane) {
+  const int which = lane >> 4, qkv = (a.heads + 2 * a.kv_heads) * HEAD;
+  const int K = which == 1 ? a.heads * HEAD : which == 3 ? a.inner : a.width, steps = K / 32;
+  const int slabs = (which == 0 ? qkv : which == 2 ? 2 * a.inner : a.width) / 16;
+  const int slab = !(which & 1) ? rank : rank >= blocks / 2 ? rank - blocks / 2 : rank + blocks - blocks / 2;
+  const int each = steps / WAVES, more = steps % WAVES, first = wave * each + min(wave, more);
+  switch (lane & 15) {
+    case OWN: return each + (wave < more ? 1 : 0);
+    case FIRST_STEP: return first;
+    case START: return slab * steps + first;                  // in kilobytes of the tile-ordered matrix
+    case STRIDE: return blocks * steps;
+    case COUNT: return slab < slabs ? (slabs - slab + blocks - 1) / blocks : 0;
+    case SLAB: return slab;
+    case SRC: return which == 0 ? a.at_out : which == 1 ? a.at_att : which == 2 ? a.at_mid : a.at_hid;
+    case SUMS: return which == 0 ? a.at_out_sums : a.at_mid_sums;
+    case DST: return which == 0 ? 0 : which == 1 ? a.at_mid : which == 2 ? a.at_hid : a.at_out;
+    case DST_SUMS: return which == 1 ? a.at_mid_sums : a.at_out_sums;
+    case ROW_BYTES: return 2 * K;
+    case OUT_WIDTH: return which == 0 ? qkv : which == 2 ? a.inner : a.width;
   }
-};
-__device__ __forceinline__ Shares shares_of(const Args& a, int rank, int blocks) {
-  Shares s;
-  s.rank = rank;
-  s.shifted = rank >= blocks / 2 ? rank - blocks / 2 : rank + blocks - blocks / 2;
-  auto count = [&](int slabs, int first) { return first < slabs ? (slabs - first + blocks - 1) / blocks : 0; };
-  s.qkv = count((a.heads + 2 * a.kv_heads) * HEAD / 16, rank);
-  s.stream = count(a.width / 16, s.shifted);
-  s.gate_up = count(2 * a.inner / 16, rank);
-  s.width_steps = a.width / 32;
-  s.heads_steps = a.heads * HEAD / 32;
-  s.inner_steps = a.inner / 32;
-  return s;
+  return 0;
 }
 
 typedef const __attribute__((address_space(4))) int* entries_ptr;
-typedef const __attribute__((address_space(1))) char* memory;
 constexpr int LAYER_WORDS = sizeof(Layer) / 8;
 enum { Q_NORM = 4, K_NORM, ENTRY_NORM, MIDDLE_NORM, KEYS, VALUES, EPS };    // words of an entry behind its four matrices
 
@@ -157,7 +161,8 @@ struct Block {
   const Args& a;
   const int rank, blocks;
   int wave, lane, tid;
-  Shares shares;
+  int numbers;                 // of the products
+  int pass;                    // slabs between two barriers
   int most;                    // looks at the exchange before a wait is given up
   int alive;
   unsigned rows_inverse;
@@ -179,17 +184,12 @@ struct Block {
 
   // ---- products ----
 
-  // A wavefront's steps are every eighth, one at least; they are taken sixteen at a time, or where K has no more, eight of two slabs and four of
-  // four. Steps behind the last one are that one again, times zero.
-  __device__ __forceinline__ int own_steps(int steps) const { return (steps - wave + WAVES - 1) / WAVES; }
-  __device__ __forceinline__ static int together(int steps) { return steps > 8 * WAVES ? 16 : steps > 4 * WAVES ? 8 : 4; }
+  __device__ __forceinline__ int number(int which, int k) const { return __builtin_amdgcn_readlane(numbers, 16 * which + k); }
   // A pointer, or the two norms' eps, out of a layer's entry
-  __device__ __forceinline__ uint64_t entry(int layer, int word) const {
-    const uint64_t v = sh.layers[layer * LAYER_WORDS + word];
+  __device__ __forceinline__ uint64_t entry(int layer, int which) const { return word(layer * LAYER_WORDS + which); }
+  __device__ __forceinline__ uint64_t word(int at) const {
+    const uint64_t v = sh.layers[at];
     return (uint64_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32 | (unsigned)__builtin_amdgcn_readfirstlane((int)v);
-  }
-  __device__ __forceinline__ memory weights_of(const Product& p, int layer, int which, int slab) const {
-    return (memory)entry(layer, which) + ((long)((p.first + slab * blocks) * p.steps + wave) << 10);
   }
   // What the registers of weights hold is of no use any more (a load that is left out would otherwise keep it where registers are scarce)
   __device__ __forceinline__ void forget() {
@@ -200,76 +200,108 @@ struct Block {
       w[j] = nothing[j];
     }
   }
+  // The wavefront's steps of a slab; what is behind them reads as zeros
+  __device__ __forceinline__ static __amdgpu_buffer_rsrc_t slab_of(uint64_t matrix, int kilobytes, int own) {
+    return buffer_of((const char*)matrix + ((uint64_t)(unsigned)kilobytes << 10), own << 10);
+  }
+  __device__ __forceinline__ void load(Pack16& to, __amdgpu_buffer_rsrc_t r, int at) const {
+    const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, 0);
+    to.u = make_uint4(v.x, v.y, v.z, v.w);
+  }
+  // Sixteen kilobytes of `left` slabs: as many steps of one, or where K has no more for a wavefront, eight of two or four of four
+  template <int N>
+  __device__ __forceinline__ void ask(uint64_t matrix, int at, int stride, int left, int own) {
+    const int off = lane * 16;
+#pragma unroll
+    for (int s = 0; s < CHUNKS / N; ++s)
+      if (s == 0 || s < left) {
+        const auto r = slab_of(matrix, at + s * stride, own);
+#pragma unroll
+        for (int j = 0; j < N; ++j) load(w[s * N + j], r, off + 1024 * j);
+      }
+  }
+  __device__ __forceinline__ void begin(int layer, int which, int done) {
+    const uint64_t matrix = entry(layer, which);
+    const int own = number(which, OWN), stride = number(which, STRIDE), left = number(which, COUNT) - done, at = number(which, START) + done * stride;
+    if (own > 8)
+      ask<16>(matrix, at, stride, left, own);
+    else if (own > 4)
+      ask<8>(matrix, at, stride, left, own);
+    else
+      ask<4>(matrix, at, stride, left, own);
+  }
   // The first weights of product `which`, or the first one behind it that this block has part in, asked for as early as their registers are free
   __device__ __forceinline__ void look_ahead(int layer, int which) {
-    forget();
-    Product p;
     for (;; ++which) {
       if (which == 4) which = 0, ++layer;
       if (layer >= a.count) return;
-      p = shares.of(which);
-      if (p.count) break;
+      if (number(which, COUNT)) break;
     }
     held = 4 * layer + which;
-    begin(p, layer, which, 0);
-  }
-  __device__ __forceinline__ void begin(const Product& p, int layer, int which, int done) {
-    // kilobyte j: sixteen steps of a slab, eight of two or four of four, of which there are `own`
-    const int take = together(p.steps), own = own_steps(p.steps), kilobytes = take * min(CHUNKS / take, p.count - done);
-    const memory at = weights_of(p, layer, which, done);
-    const long stride = (long)blocks * p.steps << 10;
-    const unsigned off = lane * 16;
-#pragma unroll
-    for (int quarter = 0; quarter < 4; ++quarter)
-      if (quarter == 0 || kilobytes > 4 * quarter) {
-        const int slab = take == 16 ? 0 : take == 8 ? quarter >> 1 : quarter, step = take == 16 ? 4 * quarter : take == 8 ? 4 * (quarter & 1) : 0;
-        const memory from = at + slab * stride;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const u32x4_t v = *(memory16)(from + (long)min(step + j, own - 1) * (WAVES << 10) + off);
-          w[4 * quarter + j].u = make_uint4(v.x, v.y, v.z, v.w);
-        }
-      }
+    begin(layer, which, 0);
   }
 
-  // Sixteen steps of rows, `left` of which there are, from the wavefront's step `i` on: lane (row, eight k of 32)
-  __device__ __forceinline__ void look(Pack16 (&x)[CHUNKS], __amdgpu_buffer_rsrc_t ex, int src, int K, int i, int left) const {
-    const int lane = anew(this->lane), col = lane & 15, grp = lane >> 4;
-    const int at = (col * K + (wave + i * WAVES) * 32 + 8 * grp) * 2;
+  // What a product multiplies with: K numbers a row at `src` of the exchange, their squares' partial sums at `sums`
+  struct Rows {
+    __amdgpu_buffer_rsrc_t ex;
+    int src, sums, at;           // (at: the lane's first eight numbers, row lane % 16 and eight k of 32; nowhere for a row that is none)
+    float eps;
+  };
+  // N steps of rows, `left` of which there are, from `at` on
+  template <int N>
+  __device__ __forceinline__ static void look(Pack16 (&x)[CHUNKS], const Rows& r, int at, int left) {
 #pragma unroll
-    for (int j = 0; j < CHUNKS; ++j) x[j].u = make_uint4(0, 0, 0, 0);
+    for (int quarter = 0; quarter < N / 4; ++quarter) {
+      if (N < 16 || quarter == 0 || left > 4 * quarter) {
 #pragma unroll
-    for (int quarter = 0; quarter < 4; ++quarter)
-      if (left > 4 * quarter) {
-        if (col < a.rows) {
-#pragma unroll
-          for (int j = 4 * quarter; j < 4 * quarter + 4; ++j) {
-            const u32x4_t v = peek16(ex, src + at + min(j, left - 1) * (WAVES * 64));
-            x[j].u = make_uint4(v.x, v.y, v.z, v.w);
-          }
+        for (int j = 4 * quarter; j < 4 * quarter + 4; ++j) {
+          const u32x4_t v = peek16(r.ex, at + 64 * j, r.src);
+          x[j].u = make_uint4(v.x, v.y, v.z, v.w);
         }
-        if (left < 4 * quarter + 4) {
+      } else {
 #pragma unroll
-          for (int j = 4 * quarter + 1; j < 4 * quarter + 4; ++j)
-            if (j >= left) x[j].u = make_uint4(0, 0, 0, 0);
-        }
+        for (int j = 4 * quarter; j < 4 * quarter + 4; ++j) x[j].u = make_uint4(0, 0, 0, 0);
       }
+    }
+    if (left < N && (left == 0 || left & 3)) {
+#pragma unroll
+      for (int j = 0; j < N; ++j)
+        if (j >= left) x[j].u = make_uint4(0, 0, 0, 0);
+    }
   }
+  template <int N>
   __device__ __forceinline__ static bool all_there(const Pack16 (&x)[CHUNKS]) {
     unsigned least = 0;                                  // (the mark is the largest word)
 #pragma unroll
-    for (int j = 0; j < CHUNKS; ++j) least = max(max(least, max(x[j].u.x, x[j].u.y)), max(x[j].u.z, x[j].u.w));
+    for (int j = 0; j < N; ++j) least = max(max(least, max(x[j].u.x, x[j].u.y)), max(x[j].u.z, x[j].u.w));
     return __all(least != ABSENT);
   }
-  // Four of a norm's weights as they lie in memory, and as numbers
-  __device__ __forceinline__ u32x4_t raw_norm(const void* n, int at) const {
-    if (a.norm_f32) return *(memory16)(static_cast<const float*>(n) + at);
-    const u32x2_t v = *(memory8)(static_cast<const bf16_t*>(n) + at);
-    return u32x4_t{v.x, v.y, 0, 0};
+  // The look at the exchange is the wait: a word without the mark is there.
+  template <int N>
+  __device__ __forceinline__ void fetch(Pack16 (&x)[CHUNKS], const Rows& r, int i, int left) {
+    const int at = r.at + 64 * i;
+    if (i == 0 && a.rows >= 4 && left > 0) {   // one look at one place first: so many rows asked for again and again hold up those that write them
+      const int place = __builtin_amdgcn_readfirstlane(at) + 64 * (min(left, N) - 1);
+      for (int n = 0;; ++n) {
+        compiler_fence();
+        const u32x4_t v = peek16(r.ex, place, r.src);
+        if (__builtin_amdgcn_readfirstlane((int)there(v)) || !again(n)) break;
+      }
+    }
+    for (int n = 0;; ++n) {
+      compiler_fence();
+      look<N>(x, r, at, left);
+      if (all_there<N>(x) || !again(n)) break;
+    }
   }
-  __device__ __forceinline__ float4 norm_of(const u32x4_t& v) const {
+  // Four of a norm's weights among the sixteen bytes around them, and as numbers
+  __device__ __forceinline__ u32x4_t raw_norm(const void* n, int at) const {
+    return *(memory16)(static_cast<const char*>(n) + (a.norm_f32 ? 4 * at : 2 * (at & ~7)));
+  }
+  __device__ __forceinline__ float4 norm_of(const u32x4_t& v, int at) const {
     if (a.norm_f32) return make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
-    return make_float4(__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xffff0000u));
+    const unsigned x = at & 4 ? v.z : v.x, y = at & 4 ? v.w : v.y;
+    return make_float4(__uint_as_float(x << 16), __uint_as_float(x & 0xffff0000u), __uint_as_float(y << 16), __uint_as_float(y & 0xffff0000u));
   }
 
   // A slab's sums of this wavefront's steps into shared memory
@@ -278,109 +310,98 @@ struct Block {
     if (col < a.rows) *reinterpret_cast<f32x4_t*>(sh.red[turn] + (unsigned)(((slab * WAVES + wave) * 4 + grp) * a.rows + col) * 16) = acc;
   }
 
-  // What a product multiplies with: K numbers a row at `src` of the exchange, their squares' partial sums at `sums`
-  struct Rows {
-    __amdgpu_buffer_rsrc_t ex;
-    int src, sums, K;            // (sums 0: no scales)
-    float eps;
-  };
-  // The look at the exchange is the wait: a word without the mark is there.
-  __device__ __forceinline__ void fetch(Pack16 (&x)[CHUNKS], const Rows& r, int i, int left) {
-    left = __builtin_amdgcn_readfirstlane(left);
-    if (i == 0 && a.rows >= 4)   // one look at one place first: so many rows asked for again and again hold up those that write them
-      for (int n = 0;; ++n) {
-        compiler_fence();
-        const u32x4_t v = peek16(r.ex, r.src + (wave + (min(left, 16) - 1) * WAVES) * 64);
-        if (__builtin_amdgcn_readfirstlane((int)there(v)) || !again(n)) break;
+  // `slabs` slabs from `done` on, whose first group's weights have been asked for. With `scaled`, the first look at the rows' sums is
+  // asked for between the rows and the multiplications.
+  __device__ __forceinline__ u32x4_t multiply(const Rows& r, int layer, int which, int done, int slabs, bool scaled) {
+    const uint64_t matrix = entry(layer, which);
+    const int own = number(which, OWN), stride = number(which, STRIDE), off = lane * 16;
+    int at = number(which, START) + done * stride;
+    u32x4_t sums = {0, 0, 0, 0};
+    Pack16 x[CHUNKS];
+    if (own > 8) {
+      const bool sections = own > 16;                    // (whose rows are asked for with every slab)
+      if (!sections) {
+        fetch<16>(x, r, 0, own);
+        if (scaled) sums = first_sums(r);
       }
-    for (int n = 0;; ++n) {
-      compiler_fence();
-      look(x, r.ex, r.src, r.K, i, left);
-      if (all_there(x) || !again(n)) break;
-    }
-  }
-
-  // `slabs` slabs from `done` on, whose first group's weights have been asked for
-  __device__ __forceinline__ void multiply(const Rows& r, const Product& p, int layer, int which, int done, int slabs) {
-    const int own = own_steps(p.steps), take = together(p.steps), together = CHUNKS / take;
-    const long stride = (long)blocks * p.steps << 10;
-    memory slab = weights_of(p, layer, which, done);
-    if (own > 16) {            // every slab in sections, whose rows are asked for with each
 #pragma unroll 1
-      for (int s = 0; s < slabs; ++s, slab += stride) {
+      for (int s = 0; s < slabs; ++s, at += stride) {
+        const auto here = slab_of(matrix, at, own), after = slab_of(matrix, at + stride, own);
         f32x4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll 1
         for (int i = 0; i < own; i += 16) {
-          Pack16 x[CHUNKS];
-          fetch(x, r, i, own - i);
+          if (sections) {
+            fetch<16>(x, r, i, own - i);
+            if (scaled && i == 0 && s == 0) sums = first_sums(r);
+          }
           const bool ends = i + 16 >= own;
-          if (!ends || s + 1 < slabs)
-            sixteen(acc, x, ends ? slab + stride : slab + (long)(i + 16) * (WAVES << 10), ends ? own : own - i - 16);
-          else
+          if (!ends || s + 1 < slabs) {
+            const auto next = ends ? after : here;
+            const int from = ends ? off : off + ((i + 16) << 10);
+#pragma unroll
+            for (int j = 0; j < CHUNKS; ++j) {
+              acc[j & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j].v, x[j].v, acc[j & 1], 0, 0, 0);
+              load(w[j], next, from + 1024 * j);
+            }
+          } else {
 #pragma unroll
             for (int j = 0; j < CHUNKS; ++j) acc[j & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j].v, x[j].v, acc[j & 1], 0, 0, 0);
+          }
         }
         leave(acc[0] + acc[1], s);
       }
-      return;
-    }
-    Pack16 x[CHUNKS];
-    fetch(x, r, 0, own);
-    if (take == 16) {
+    } else if (own > 4) {
+      fetch<8>(x, r, 0, own);
+      if (scaled) sums = first_sums(r);
 #pragma unroll 1
-      for (int s = 0; s < slabs; ++s, slab += stride) {
-        f32x4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-        if (s + 1 < slabs)
-          sixteen(acc, x, slab + stride, own);
-        else
+      for (int s = 0; s < slabs; s += 2) {
+        f32x4_t acc[4];
 #pragma unroll
-          for (int j = 0; j < CHUNKS; ++j) acc[j & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j].v, x[j].v, acc[j & 1], 0, 0, 0);
-        leave(acc[0] + acc[1], s);
-      }
-      return;
-    }
-#pragma unroll 1
-    for (int s = 0; s < slabs; s += together) {
-      f32x4_t acc[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) acc[q] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-      if (take == 8) {
+        for (int q = 0; q < 4; ++q) acc[q] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int j = 0; j < CHUNKS; ++j) acc[j >> 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j].v, x[j & 7].v, acc[j >> 2], 0, 0, 0);
-        acc[0] += acc[1];
-        acc[1] = acc[2] + acc[3];
-      } else {
+        if (s + 2 < slabs) ask<8>(matrix, at += 2 * stride, stride, slabs - s - 2, own);
+        leave(acc[0] + acc[1], s);
+        if (s + 1 < slabs) leave(acc[2] + acc[3], s + 1);
+      }
+    } else {
+      fetch<4>(x, r, 0, own);
+      if (scaled) sums = first_sums(r);
+#pragma unroll 1
+      for (int s = 0; s < slabs; s += 4) {
+        f32x4_t acc[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc[q] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int j = 0; j < CHUNKS; ++j) acc[j >> 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j].v, x[j & 3].v, acc[j >> 2], 0, 0, 0);
+        if (s + 4 < slabs) ask<4>(matrix, at += 4 * stride, stride, slabs - s - 4, own);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (s + q < slabs) leave(acc[q], s + q);
       }
-      if (s + together < slabs) begin(p, layer, which, done + s + together);
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        if (q < together && s + q < slabs) leave(acc[q], s + q);
     }
-  }
-  // Sixteen steps of a slab, and in the place of each kilobyte the next group's, `left` of which there are
-  __device__ __forceinline__ void sixteen(f32x4_t (&acc)[2], const Pack16 (&x)[CHUNKS], memory next, int left) {
-    const unsigned off = lane * 16;
-#pragma unroll
-    for (int j = 0; j < CHUNKS; ++j) {
-      acc[j & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j].v, x[j].v, acc[j & 1], 0, 0, 0);
-      const u32x4_t v = *(memory16)(next + (long)min(j, left - 1) * (WAVES << 10) + off);
-      w[j].u = make_uint4(v.x, v.y, v.z, v.w);
-    }
+    return sums;
   }
 
-  // The rows' scales from the partial sums of squares, [row][slab]
-  __device__ __forceinline__ void scales(const Rows& r) {
+  // The rows' scales from the partial sums of squares, [row][slab]; `v`: the first of them, as they were when the rows had come
+  __device__ __forceinline__ u32x4_t first_sums(const Rows& r) const {
+    const int lane = anew(this->lane), slabs = a.width / 16;
+    return peek16(r.ex, wave < a.rows && lane * 4 < slabs ? (wave * slabs + lane * 4) * 4 : NOWHERE, r.sums);
+  }
+  __device__ __forceinline__ void scales(const Rows& r, u32x4_t v) {
     const int slabs = a.width / 16;
+    bool asked = true;
+#pragma unroll 1
     for (int row = wave; row < a.rows; row += WAVES) {
       float s = 0.f;
-      for (int k = lane * 4; k < ((slabs + 255) & ~255); k += 256) {
-        u32x4_t v = {0, 0, 0, 0};
+#pragma unroll 1
+      for (int k = lane * 4; __builtin_amdgcn_readfirstlane(k) < slabs; k += 256) {
+        const int at = k < slabs ? (row * slabs + k) * 4 : NOWHERE;
         for (int n = 0;; ++n) {
-          compiler_fence();
-          if (k < slabs) v = peek16(r.ex, r.sums + (row * slabs + k) * 4);
+          if (!asked) v = peek16(r.ex, at, r.sums);
+          asked = false;
           if (__all(there(v)) || !again(n)) break;
+          compiler_fence();
         }
         s += (__uint_as_float(v.x) + __uint_as_float(v.y)) + (__uint_as_float(v.z) + __uint_as_float(v.w));
       }
@@ -396,8 +417,8 @@ struct Block {
     float4 res;
     u32x4_t raw;
   };
-  __device__ __forceinline__ Follow follow(const Product& p, int done, int slabs, const void* norm) const {
-    const int tid = anew(this->tid), q = tid >> 2, s = over_rows(q), row = q - s * a.rows, n = (p.first + (done + s) * blocks) * 16 + 4 * (tid & 3);
+  __device__ __forceinline__ Follow follow(int which, int done, int slabs, const void* norm) const {
+    const int tid = anew(this->tid), q = tid >> 2, s = over_rows(q), row = q - s * a.rows, n = (number(which, SLAB) + (done + s) * blocks) * 16 + 4 * (tid & 3);
     Follow f;
     f.res = make_float4(0.f, 0.f, 0.f, 0.f);
     f.raw = u32x4_t{0, 0, 0, 0};
@@ -407,30 +428,30 @@ struct Block {
     }
     return f;
   }
-  __device__ __forceinline__ void finish(__amdgpu_buffer_rsrc_t ex, int which, const Product& p, int done, int slabs, const void* norm, Follow f) {
+  __device__ __forceinline__ void finish(__amdgpu_buffer_rsrc_t ex, int which, int done, int slabs, const void* norm, Follow f) {
     const bool stream = which & 1;
     const int tid = anew(this->tid), entries = slabs * 4 * a.rows, grp = tid & 3;
-    const int width = which == 0 ? (a.heads + 2 * a.kv_heads) * HEAD : which == 2 ? a.inner : a.width;
-    const int dst = which == 0 ? 0 : which == 1 ? a.at_mid : which == 2 ? a.at_hid : a.at_out;
-    for (int idx = tid; idx < entries; idx += THREADS) {
-      const int q = idx >> 2, s = over_rows(q), row = q - s * a.rows, slab = p.first + (done + s) * blocks, n = slab * 16 + 4 * grp;
+    const int width = number(which, OUT_WIDTH), dst = number(which, DST), first = number(which, SLAB) + done * blocks;
+    if (tid < entries) {         // (a thread has one at most)
+      const int q = tid >> 2, s = over_rows(q), row = q - s * a.rows, slab = first + s * blocks, n = slab * 16 + 4 * grp;
       const char* part = sh.red[turn] + (unsigned)((s * WAVES * 4 + grp) * a.rows + row) * 16;
-      f32x4_t acc = *reinterpret_cast<const f32x4_t*>(part);
+      f32x4_t share[WAVES];
 #pragma unroll
-      for (int v = 1; v < WAVES; ++v) acc += *reinterpret_cast<const f32x4_t*>(part + (unsigned)(v * 4 * a.rows) * 16);
+      for (int v = 0; v < WAVES; ++v) share[v] = *reinterpret_cast<const f32x4_t*>(part + (unsigned)(v * 4 * a.rows) * 16);
+#pragma unroll
+      for (int v = 0; v < WAVES; ++v) asm volatile("" : "+v"(share[v]));       // (all of them asked for, then added)
+      f32x4_t acc = share[0];
+#pragma unroll
+      for (int v = 1; v < WAVES; ++v) acc += share[v];
       union {
         uint2 u;
         __bf16 e[4];
       } pk;
       if (stream) {
-        if (idx != tid) {
-          f.res = load_four(a.residual + (size_t)row * a.width + n);
-          if (norm) f.raw = raw_norm(norm, n);
-        }
         const float x[4] = {f.res.x + (float)(__bf16)acc[0], f.res.y + (float)(__bf16)acc[1], f.res.z + (float)(__bf16)acc[2],
                             f.res.w + (float)(__bf16)acc[3]};
         if (norm) {
-          const float4 nw = norm_of(f.raw);
+          const float4 nw = norm_of(f.raw, n);
           const float w4[4] = {nw.x, nw.y, nw.z, nw.w};
           float ss = 0.f;
 #pragma unroll
@@ -441,8 +462,7 @@ struct Block {
           put8(ex, dst + (row * width + n) * 2, pk.u);
           ss += __shfl_xor(ss, 1, 64);
           ss += __shfl_xor(ss, 2, 64);
-          const int sums = which == 1 ? a.at_mid_sums : a.at_out_sums;
-          if (grp == 0) put4(ex, sums + (row * (width / 16) + slab) * 4, __float_as_uint(ss), 0x7fc00000u);
+          if (grp == 0) put4(ex, number(which, DST_SUMS) + (row * (width / 16) + slab) * 4, __float_as_uint(ss), 0x7fc00000u);
         }
         store16(a.residual + (size_t)row * a.width + n,
                 u32x4_t{__float_as_uint(x[0]), __float_as_uint(x[1]), __float_as_uint(x[2]), __float_as_uint(x[3])});
@@ -464,19 +484,21 @@ struct Block {
     }
   }
 
-  __device__ __forceinline__ void product_of(const Rows& r, __amdgpu_buffer_rsrc_t ex, int layer, int which, const Product& p, const void* norm) {
-    const int pass = min(MOST_SLABS, RESULTS / a.rows);
+  __device__ __forceinline__ void product_of(const Rows& r, __amdgpu_buffer_rsrc_t ex, int layer, int which, int count, const void* norm) {
 #pragma unroll 1
-    for (int done = 0; done < p.count; done += pass) {
-      const int slabs = min(pass, p.count - done);
-      if (done || held != 4 * layer + which) begin(p, layer, which, done);
+    for (int done = 0; done < count; done += pass) {
+      const int slabs = min(pass, count - done);
+      if (done || held != 4 * layer + which) begin(layer, which, done);
       Follow f;
-      if (which & 1) f = follow(p, done, slabs, norm);
-      multiply(r, p, layer, which, done, slabs);
-      if (done == 0 && !(which & 1)) scales(r);
-      if (done + slabs >= p.count && which != 0) look_ahead(layer, which + 1);
+      if (which & 1) f = follow(which, done, slabs, norm);
+      const bool scaled = done == 0 && !(which & 1);
+      const u32x4_t sums = multiply(r, layer, which, done, slabs, scaled);
+      if (scaled) scales(r, sums);
+      forget();
       meet();
-      finish(ex, which, p, done, slabs, norm, f);
+      finish(ex, which, done, slabs, norm, f);
+      meet();                    // (the results on their way ahead of the other wavefronts' loads: 8B shape, one request, 3 us a product otherwise)
+      if (done + slabs >= count && which != 0) look_ahead(layer, which + 1);
       turn ^= 1;
     }
   }
@@ -485,15 +507,16 @@ struct Block {
 
   // A piece of the attention: a split of a sequence's keys for one key head, and what all layers have of it in common.
   struct Item {
-    int split, g_kv, b, kv_len;
-    TilePages first, second;     // of this wavefront's first two tiles
+    int split, g_kv, b, kv_len, there;
+    TilePages second;            // of this wavefront's second tile
+    uint64_t keys, values;       // where the lane's parts of its first one lie
   };
   __device__ __forceinline__ TilePages pages_of(int b, int tile) const {
     const entries_ptr row = (entries_ptr)(uintptr_t)(a.block_table + (size_t)b * a.table_width);
     TilePages p;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const int entry = (tile * FAST_TILE + 16 * h) / a.page;
+      const int entry = (tile * FAST_TILE + 16 * h) >> a.page_bits;
       p.pg[h] = entry < a.table_width ? row[entry] : -1;
     }
     return p;
@@ -506,7 +529,10 @@ struct Block {
     it.g_kv = pair - it.b * a.kv_heads;
     it.kv_len = ((entries_ptr)(uintptr_t)a.kv_lens)[it.b];
     const int first = it.split * WAVES + wave;
-    it.first = pages_of(it.b, first);
+    const TileAddr t = tile_addr(pages_of(it.b, first), nullptr, nullptr, a.num_pages, a.kv_heads, it.g_kv, a.page, HEAD, HEAD, first * FAST_TILE);
+    it.there = t.there;
+    it.keys = (uint64_t)t.k;
+    it.values = (uint64_t)t.v;
     it.second = pages_of(it.b, first + WAVES * a.splits);
     return it;
   }
@@ -521,7 +547,7 @@ struct Block {
     const char *q_norm = (const char*)entry(layer, Q_NORM), *k_norm = (const char*)entry(layer, K_NORM);
     const int split = it.split, g_kv = it.g_kv, b = it.b;
     const int lane = anew(this->lane), col = lane & 15, grp = lane >> 4;
-    const int G = a.heads / a.kv_heads, joined = (a.heads + 2 * a.kv_heads) * D;
+    const int G = a.group, joined = (a.heads + 2 * a.kv_heads) * D;
     const int first = split * WAVES + wave, step = WAVES * a.splits;
     const bool brings_new = split == a.splits - 1;
     const int pos = it.kv_len - 1;                    // the token's own position; the cache is read up to the one before
@@ -545,22 +571,23 @@ struct Block {
     };
     TilePages next = it.second;
     if (first < last) {
-      ask_keys(addr_of(it.first, first));
+      ask_keys(TileAddr{(const bf16_t*)((uint64_t)keys + it.keys), (const bf16_t*)((uint64_t)values + it.values), it.there});
       ask_values();
     }
     // the token's rows: lane n has elements 2 n and 2 n + 1, its pair's other half is lane n ^ 32
     for (int row = wave; row < G + (brings_new ? 2 : 0); row += WAVES) {
       const int head = row < G ? g_kv * G + row : a.heads + (row == G ? 0 : a.kv_heads) + g_kv;
       const bool prepared = row <= G;                 // (values are taken as they are)
-      float2 norm = make_float2(1.f, 1.f), cs = make_float2(1.f, 1.f), sn = make_float2(0.f, 0.f);
+      unsigned norm[2] = {0, 0};                      // as they lie in memory
+      float2 cs = make_float2(1.f, 1.f), sn = make_float2(0.f, 0.f);
       if (prepared && q_norm != nullptr) {
         const char* weights = row < G ? q_norm : k_norm;
         if constexpr (sizeof(QKW) == 4) {
           const u32x2_t v = *(memory8)(weights + 8 * lane);
-          norm = make_float2(__uint_as_float(v.x), __uint_as_float(v.y));
+          norm[0] = v.x;
+          norm[1] = v.y;
         } else {
-          const unsigned v = *(const __attribute__((address_space(1))) unsigned*)(weights + 4 * lane);
-          norm = make_float2(__uint_as_float(v << 16), __uint_as_float(v & 0xffff0000u));
+          norm[0] = *(const __attribute__((address_space(1))) unsigned*)(weights + 4 * lane);
         }
       }
       if (prepared && turned) {
@@ -578,8 +605,8 @@ struct Block {
       float x0 = __uint_as_float(v << 16), x1 = __uint_as_float(v & 0xffff0000u);
       if (prepared && q_norm != nullptr) {
         const float scale = head_norm_scale(wave_sum(__fmaf_rn(x0, x0, __fmul_rn(x1, x1))), D, a.qk_eps);
-        x0 = __fmul_rn(__fmul_rn(x0, scale), norm.x);
-        x1 = __fmul_rn(__fmul_rn(x1, scale), norm.y);
+        x0 = __fmul_rn(__fmul_rn(x0, scale), __uint_as_float(sizeof(QKW) == 4 ? norm[0] : norm[0] << 16));
+        x1 = __fmul_rn(__fmul_rn(x1, scale), __uint_as_float(sizeof(QKW) == 4 ? norm[1] : norm[0] & 0xffff0000u));
       }
       if (prepared && turned) {
         const float y0 = __shfl_xor(x0, 32, 64), y1 = __shfl_xor(x1, 32, 64);
@@ -707,7 +734,7 @@ struct Block {
       }
     }
     if (brings_new && pos >= 0 && tid >= THREADS - 2 * HEAD) {       // the token's key and value into the caches, for later steps
-      const int d = tid & (HEAD - 1), blk = pos / a.page, at = pos % a.page;
+      const int d = tid & (HEAD - 1), blk = pos >> a.page_bits, at = pos & (a.page - 1);
       const int pg = blk < a.table_width ? ((entries_ptr)(uintptr_t)(a.block_table + (size_t)b * a.table_width))[blk] : -1;
       if (pg >= 0 && pg < a.num_pages) {
         const size_t head = (size_t)pg * a.kv_heads + g_kv;
@@ -722,7 +749,7 @@ struct Block {
   // The splits of sequence `b` and key head `g_kv`, joined
   __device__ __forceinline__ void merge(__amdgpu_buffer_rsrc_t ex, int g_kv, int b) {
     constexpr int D = HEAD, N = 8;
-    const int tid = anew(this->tid), G = a.heads / a.kv_heads, all = a.rows * a.heads * a.splits * D;
+    const int tid = anew(this->tid), G = a.group, all = a.rows * a.heads * a.splits * D;
     for (int idx = tid; idx < ((G * (D / 4) + 63) & ~63); idx += THREADS) {
       const int r = min(idx / (D / 4), G - 1), d = idx % (D / 4) * 4;
       float m = -INFINITY, sum = 0.f;
@@ -772,13 +799,15 @@ struct Block {
   }
 
   __device__ __forceinline__ void layers() {
-    const int items = a.rows * a.kv_heads * a.splits;
-    const Item mine = item_of(min(rank, items - 1));
+    const int items = a.rows * a.kv_heads * a.splits, pairs = a.rows * a.kv_heads;
+    Item mine = item_of(min(rank, items - 1));
+    sh.first_at[tid][0] = mine.keys;
+    sh.first_at[tid][1] = mine.values;
+    const int my_pair = rank >= blocks / 4 ? rank - blocks / 4 : rank + blocks - blocks / 4, my_b = my_pair / a.kv_heads, my_g = my_pair - my_b * a.kv_heads;
     look_ahead(0, 0);
 #pragma unroll 1
     for (int n = 0; n < a.count; ++n) {
       const auto ex = buffer_of(a.exchange + n * a.per_layer, a.per_layer);
-      const bool last = n == a.count - 1;
 #pragma unroll 1
       for (int which = 0; which < 4; ++which) {
         // (new numbers to the compiler: it would otherwise work out every product's addresses ahead of all of them, and has no registers for those)
@@ -787,32 +816,40 @@ struct Block {
 #pragma unroll 1
           for (int n_item = rank; n_item < items; n_item += blocks) {
             Item it = mine;
+            it.keys = sh.first_at[tid][0];
+            it.values = sh.first_at[tid][1];
             if (n_item != rank) it = item_of(n_item);
             attend(ex, n, it);
           }
           if (a.splits > 1)      // (its loads would come behind the next weights')
 #pragma unroll 1
-            for (int pair = rank >= blocks / 4 ? rank - blocks / 4 : rank + blocks - blocks / 4; pair < a.rows * a.kv_heads; pair += blocks)
-              merge(ex, pair % a.kv_heads, pair / a.kv_heads);
+            for (int pair = my_pair; pair < pairs; pair += blocks) {
+              const bool first = pair == my_pair;
+              const int b = first ? my_b : pair / a.kv_heads, g = first ? my_g : pair - pair / a.kv_heads * a.kv_heads;
+              merge(ex, g, b);
+            }
           look_ahead(n, 1);
         }
-        const Product p = shares.of(which);
-        if (p.count == 0) continue;
+        const int count = number(which, COUNT);
+        if (count == 0) continue;
+        const int col = lane & 15;
         Rows r;
         r.ex = which == 0 ? buffer_of(a.exchange + (n - 1) * a.per_layer, a.per_layer) : ex;
-        r.src = which == 0 ? a.at_out : which == 1 ? a.at_att : which == 2 ? a.at_mid : a.at_hid;
-        r.sums = which == 0 ? a.at_out_sums : which == 2 ? a.at_mid_sums : 0;
-        r.K = p.steps * 32;
-        r.eps = __uint_as_float(which == 0 ? (unsigned)entry(n, EPS) : (unsigned)(entry(n, EPS) >> 32));
-        const void* norm = which == 1 ? (const void*)entry(n, MIDDLE_NORM) : which == 3 && !last ? (const void*)entry(n + 1, ENTRY_NORM) : nullptr;
-        product_of(r, ex, n, which, p, norm);
+        r.src = number(which, SRC);
+        r.sums = number(which, SUMS);
+        r.at = col < a.rows ? col * number(which, ROW_BYTES) + 64 * number(which, FIRST_STEP) + 16 * (lane >> 4) : NOWHERE;
+        const uint64_t eps = entry(n, EPS);
+        r.eps = __uint_as_float((unsigned)(which == 0 ? eps : eps >> 32));
+        // (the last layer's down product prepares no rows: its norm is the one behind the layers, of another kernel)
+        const int at = which == 1 ? n * LAYER_WORDS + MIDDLE_NORM : which == 3 && n + 1 < a.count ? (n + 1) * LAYER_WORDS + ENTRY_NORM : -1;
+        const void* norm = at >= 0 ? (const void*)word(at) : nullptr;
+        product_of(r, ex, n, which, count, norm);
       }
     }
     if (!alive) {              // a wait that did not end: no number of the result stands
-      const Product p = shares.of(3);
-      for (int done = 0; done < p.count; ++done)
+      for (int done = 0; done < number(3, COUNT); ++done)
         for (int idx = tid; idx < 16 * a.rows; idx += THREADS)
-          a.residual[(size_t)(idx >> 4) * a.width + (p.first + done * blocks) * 16 + (idx & 15)] = __uint_as_float(0x7fc00000u);
+          a.residual[(size_t)(idx >> 4) * a.width + (number(3, SLAB) + done * blocks) * 16 + (idx & 15)] = __uint_as_float(0x7fc00000u);
     }
   }
 };
@@ -861,7 +898,8 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
   for (int i = threadIdx.x; i < a.count * LAYER_WORDS; i += THREADS) sh.layers[i] = reinterpret_cast<const uint64_t*>(a.layers)[i];
   __syncthreads();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  Block<QKW> b{sh, a, rank, blocks, wave, (int)threadIdx.x & 63, (int)threadIdx.x, shares_of(a, rank, blocks), a.limit, 1, (1u << 20) / a.rows + 1, 0, -1};
+  Block<QKW> b{sh, a, rank, blocks, wave, (int)threadIdx.x & 63, (int)threadIdx.x, numbers_of(a, rank, blocks, wave, threadIdx.x & 63),
+                  min(MOST_SLABS, RESULTS / a.rows), a.limit, 1, (1u << 20) / a.rows + 1, 0, -1};
   b.layers();
 }
 
@@ -997,9 +1035,9 @@ int q3_decode_layers(const Layer* layers, int count, float* residual, int rows, 
   a.per_layer = l.size;
   a.at_part = (int)l.part, a.at_att = (int)l.att, a.at_mid = (int)l.mid, a.at_mid_sums = (int)l.mid_sums, a.at_hid = (int)l.hid;
   a.at_out = (int)l.out, a.at_out_sums = (int)l.out_sums;
-  a.count = count, a.rows = rows, a.width = width, a.heads = heads, a.kv_heads = kv_heads, a.inner = inner;
+  a.count = count, a.rows = rows, a.width = width, a.heads = heads, a.kv_heads = kv_heads, a.group = heads / kv_heads, a.inner = inner;
   a.norm_f32 = norm_dtype == Q3_F32;
-  a.max_pos = max_pos, a.table_width = table_width, a.page = page, a.num_pages = num_pages, a.splits = splits;
+  a.max_pos = max_pos, a.table_width = table_width, a.page = page, a.page_bits = __builtin_ctz(page), a.num_pages = num_pages, a.splits = splits;
   a.patience = patience, a.limit = limit;
   a.qk_eps = qk_eps;
   a.scale_log2 = make_score_scale(scale);
