@@ -10,20 +10,22 @@
 // block). The weights of a product's first steps are asked for while the last one's results are on their way, so memory is not idle
 // meanwhile.
 //
-// What it measured (us a step in a graph, the layers' kernels one by one / this): the 0.6B shape, one request over 1,100 keys
-// 1,013 / 701; the 8B shape, one over 2,060 3,407 / 2,820, eight 3,954 / 3,440. The first form of this kernel (805, 3,012, 3,561) was faster
-// than the kernels at each of 28 sizes from 1 to 16 rows and 100 to 30,000 keys; more than 16 rows have no registers here.
+// What it measured (us a step in a graph, the layers' kernels one by one / this): the 0.6B shape, one request over 100 keys 971 / 533,
+// over 1,100 1,013 / 576, over 8,000 1,140 / 773, four 1,141 / 674, eight over 2,000 1,415 / 941, sixteen 1,910 / 1,369; the 8B shape, one over
+// 2,060 3,407 / 2,760, eight 3,954 / 3,460. The first form of this kernel (809, 3,026, 3,510) was faster than the kernels at each of 28 sizes
+// from 1 to 16 rows and 100 to 30,000 keys; more than 16 rows have no registers here.
 //
 // What bounds it: one request of the small shape the chain of five or six exchanges a layer; a look that fails costs a second one behind
 // the first, a store holds up the wavefront's next look (they come back in order), and a wavefront alone on its SIMD takes 4 to 5 cycles
 // an instruction, 20 for a number that goes from a vector's lane into scalar arithmetic. So what is between two exchanges is kept short:
 // offsets that are constants of an instruction, steps of K in one stretch, bounds by the descriptors (500 instructions a product less:
 // 801 -> 779), the next weights asked for behind the results (779 -> 749; 8B 2,990 -> 2,860) and behind all wavefronts' results, with
-// the shares of K read together (749 -> 701; 2,860 -> 2,820). The large shape is bound by its weights (5.4 of the 5.8 TB/s that a
-// plain read reaches, the whole step through) and the attention's part, where few weights move.
+// the shares of K read together (749 -> 701; 2,860 -> 2,820), blocks of their own for the products into the stream of a small model (701 -> 597),
+// weights in registers that nothing copies (585 -> 576; 2,820 -> 2,760). The large shape is bound by its weights (5.5 of the
+// 5.8 TB/s that a plain read reaches, the whole step through) and the attention's part, where few weights move.
 // What did not help: the block split into wavefronts that multiply and wavefronts that look, prepare and store, with the weights in a
 // ring in shared memory (0.6B 905: more handovers a product), asking for the sums of squares together with the rows (lines that many blocks
-// write and all ask for again and again are slow to change: 915), copies of what all read (nothing), the first keys asked for ahead of
+// write and all ask for again and again are slow to change: 915; in the rows' own lines, 80 bytes for 32 numbers, 600 for 576), copies of what all read (nothing), the first keys asked for ahead of
 // the [q | k | v] product's end (937: a second copy of the product, 61 KB of code beyond what the instruction caches keep).
 #include "common.h"
 #include "attention_tiles.h"
@@ -118,6 +120,12 @@ __device__ __forceinline__ void put4(__amdgpu_buffer_rsrc_t r, int at, unsigned 
 }
 __device__ __forceinline__ void compiler_fence() { asm volatile("" ::: "memory"); }
 
+// Lane ^ N's value, N 1 or 2
+template <int N>
+__device__ __forceinline__ float quad_xor(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), N == 1 ? 0xb1 : 0x4e, 0xf, 0xf, true));
+}
+
 // Until shared memory holds what the block's wavefronts have written (and nothing about memory)
 __device__ __forceinline__ void meet() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
@@ -125,22 +133,49 @@ __device__ __forceinline__ void meet() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts
 
 // What a wavefront knows of a product, each number in a lane of one register (lane 16 product + number): numbers that are computed
 // where they are needed, over and over, are what the compiler moves ahead of loops, 500 instructions a product on the way from one
-// exchange to the next. A block has the slabs SLAB, SLAB + blocks, ..; the two products that add into the stream go to
-// blocks others than those of the attention's first items.
-enum { OWN, FIRST_STEP, START, STRIDE, COUNT, SLAB, SRC, SUMS, DST, DST_SUMS, ROW_BYTES, OUT_WIDTH };
+// exchange to the next. A block has COUNT slabs, SLAB and every STEP-th behind it: neighbours where products have blocks for themselves
+// (whose results lie in the same lines; the 0.6B shape 596 -> 585 us), else one beside the other blocks' (all blocks then read
+// one stretch of memory; the 8B shape 2,841 -> 2,819).
+enum { OWN, FIRST_STEP, START, STRIDE, COUNT, SLAB, STEP, SRC, SUMS, DST, DST_SUMS, ROW_BYTES, OUT_WIDTH };
+// Who does what. Where a quarter of the blocks has a slab for each of the two products that add into the stream, those have the
+// last quarter for themselves, and the other two products the rest: of two products that follow one another each finds its block
+// waiting, its weights there and nothing of its own on the way to memory.
+struct Roles {
+  int apart;                   // how many blocks the products into the stream have for themselves, or none
+  __device__ __forceinline__ Roles(const Args& a, int blocks) : apart(4 * (a.width / 16) <= blocks ? a.width / 16 : 0) {}
+  // a block's place among those that share product `which` out, and how many they are; its first item of the attention and its first pair of
+  // row and key head whose splits it joins
+  __device__ __forceinline__ int place(int which, int rank, int blocks) const {
+    if (apart) return which & 1 ? rank - (blocks - apart) : rank;
+    return !(which & 1) ? rank : rank >= blocks / 2 ? rank - blocks / 2 : rank + blocks - blocks / 2;
+  }
+  __device__ __forceinline__ int places(int which, int blocks) const { return !apart ? blocks : which & 1 ? apart : blocks - apart; }
+  // the first pieces of attention are the stream's blocks', whose keys come while the first product is multiplied
+  __device__ __forceinline__ int item(int rank, int blocks) const {
+    return !apart ? rank : rank >= blocks - apart ? rank - (blocks - apart) : rank + apart;
+  }
+  __device__ __forceinline__ int pair(int rank, int blocks) const {
+    const int all = blocks - apart, middle = apart ? all / 2 : blocks / 4;
+    return rank >= all ? 1 << 24 : rank >= middle ? rank - middle : rank + all - middle;
+  }
+};
 __device__ __forceinline__ int numbers_of(const Args& a, int rank, int blocks, int wave, int lane) {
   const int which = lane >> 4, qkv = (a.heads + 2 * a.kv_heads) * HEAD;
   const int K = which == 1 ? a.heads * HEAD : which == 3 ? a.inner : a.width, steps = K / 32;
   const int slabs = (which == 0 ? qkv : which == 2 ? 2 * a.inner : a.width) / 16;
-  const int slab = !(which & 1) ? rank : rank >= blocks / 2 ? rank - blocks / 2 : rank + blocks - blocks / 2;
+  const Roles roles(a, blocks);
+  const int place = roles.place(which, rank, blocks), places = roles.places(which, blocks);
+  const int share = slabs / places, extra = slabs % places, count = place >= 0 && place < places ? share + (place < extra ? 1 : 0) : 0;
+  const int slab = roles.apart ? place * share + min(place, extra) : place, step = roles.apart ? 1 : places;
   const int each = steps / WAVES, more = steps % WAVES, first = wave * each + min(wave, more);
   switch (lane & 15) {
     case OWN: return each + (wave < more ? 1 : 0);
     case FIRST_STEP: return first;
     case START: return slab * steps + first;                  // in kilobytes of the tile-ordered matrix
-    case STRIDE: return blocks * steps;
-    case COUNT: return slab < slabs ? (slabs - slab + blocks - 1) / blocks : 0;
+    case STRIDE: return step * steps;
+    case COUNT: return count;
     case SLAB: return slab;
+    case STEP: return step;
     case SRC: return which == 0 ? a.at_out : which == 1 ? a.at_att : which == 2 ? a.at_mid : a.at_hid;
     case SUMS: return which == 0 ? a.at_out_sums : a.at_mid_sums;
     case DST: return which == 0 ? 0 : which == 1 ? a.at_mid : which == 2 ? a.at_hid : a.at_out;
@@ -168,7 +203,7 @@ struct Block {
   unsigned rows_inverse;
   int turn;                    // of the two halves of shared memory's results
   int held;                    // the product whose first weights are on their way: four times its layer, and which
-  Pack16 w[CHUNKS];            // they
+  u32x4_t w[CHUNKS];           // they
 
   // (as a number of its own: what is computed from it is not kept in registers over the whole launch)
   __device__ __forceinline__ static int anew(int v) {
@@ -193,42 +228,39 @@ struct Block {
   }
   // What the registers of weights hold is of no use any more (a load that is left out would otherwise keep it where registers are scarce)
   __device__ __forceinline__ void forget() {
-    Pack16 nothing[CHUNKS];
+    u32x4_t nothing;
 #pragma unroll
     for (int j = 0; j < CHUNKS; ++j) {
-      asm volatile("" : "=v"(nothing[j].u.x), "=v"(nothing[j].u.y), "=v"(nothing[j].u.z), "=v"(nothing[j].u.w));
-      w[j] = nothing[j];
+      asm volatile("" : "=v"(nothing));
+      w[j] = nothing;
     }
   }
   // The wavefront's steps of a slab; what is behind them reads as zeros
   __device__ __forceinline__ static __amdgpu_buffer_rsrc_t slab_of(uint64_t matrix, int kilobytes, int own) {
     return buffer_of((const char*)matrix + ((uint64_t)(unsigned)kilobytes << 10), own << 10);
   }
-  __device__ __forceinline__ void load(Pack16& to, __amdgpu_buffer_rsrc_t r, int at) const {
-    const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, 0);
-    to.u = make_uint4(v.x, v.y, v.z, v.w);
+  __device__ __forceinline__ static u32x4_t load(__amdgpu_buffer_rsrc_t r, int at) { return __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, 0); }
+  __device__ __forceinline__ static f32x4_t dot(const u32x4_t& w, const u32x4_t& x, const f32x4_t& acc) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, w), __builtin_bit_cast(bf16x8_t, x), acc, 0, 0, 0);
   }
-  // Sixteen kilobytes of `left` slabs: as many steps of one, or where K has no more for a wavefront, eight of two or four of four
-  template <int N>
+  // Sixteen kilobytes of `left` slabs: as many steps of one, or where K has no more for a wavefront, eight of two or four of four. (One
+  // sequence for all three: registers that several may have loaded are copied behind each, and so waited for.)
   __device__ __forceinline__ void ask(uint64_t matrix, int at, int stride, int left, int own) {
-    const int off = lane * 16;
+    const int off = anew(lane) * 16, bits = own > 8 ? 2 : own > 4 ? 1 : 0;
 #pragma unroll
-    for (int s = 0; s < CHUNKS / N; ++s)
-      if (s == 0 || s < left) {
+    for (int quarter = 0; quarter < 4; ++quarter) {
+      const int s = quarter >> bits;
+      if (quarter == 0 || s < left) {
         const auto r = slab_of(matrix, at + s * stride, own);
+        const int from = off + ((quarter - (s << bits)) << 12);
 #pragma unroll
-        for (int j = 0; j < N; ++j) load(w[s * N + j], r, off + 1024 * j);
+        for (int j = 0; j < 4; ++j) w[4 * quarter + j] = load(r, from + 1024 * j);
       }
+    }
   }
   __device__ __forceinline__ void begin(int layer, int which, int done) {
-    const uint64_t matrix = entry(layer, which);
-    const int own = number(which, OWN), stride = number(which, STRIDE), left = number(which, COUNT) - done, at = number(which, START) + done * stride;
-    if (own > 8)
-      ask<16>(matrix, at, stride, left, own);
-    else if (own > 4)
-      ask<8>(matrix, at, stride, left, own);
-    else
-      ask<4>(matrix, at, stride, left, own);
+    const int stride = number(which, STRIDE);
+    ask(entry(layer, which), number(which, START) + done * stride, stride, number(which, COUNT) - done, number(which, OWN));
   }
   // The first weights of product `which`, or the first one behind it that this block has part in, asked for as early as their registers are free
   __device__ __forceinline__ void look_ahead(int layer, int which) {
@@ -249,36 +281,29 @@ struct Block {
   };
   // N steps of rows, `left` of which there are, from `at` on
   template <int N>
-  __device__ __forceinline__ static void look(Pack16 (&x)[CHUNKS], const Rows& r, int at, int left) {
+  __device__ __forceinline__ static void look(u32x4_t (&x)[CHUNKS], const Rows& r, int at, int left) {
 #pragma unroll
     for (int quarter = 0; quarter < N / 4; ++quarter) {
-      if (N < 16 || quarter == 0 || left > 4 * quarter) {
+      const int from = N < 16 || quarter == 0 || left > 4 * quarter ? at : NOWHERE;
 #pragma unroll
-        for (int j = 4 * quarter; j < 4 * quarter + 4; ++j) {
-          const u32x4_t v = peek16(r.ex, at + 64 * j, r.src);
-          x[j].u = make_uint4(v.x, v.y, v.z, v.w);
-        }
-      } else {
-#pragma unroll
-        for (int j = 4 * quarter; j < 4 * quarter + 4; ++j) x[j].u = make_uint4(0, 0, 0, 0);
-      }
+      for (int j = 4 * quarter; j < 4 * quarter + 4; ++j) x[j] = peek16(r.ex, from + 64 * j, r.src);
     }
     if (left < N && (left == 0 || left & 3)) {
 #pragma unroll
       for (int j = 0; j < N; ++j)
-        if (j >= left) x[j].u = make_uint4(0, 0, 0, 0);
+        if (j >= left) x[j] = u32x4_t{0, 0, 0, 0};
     }
   }
   template <int N>
-  __device__ __forceinline__ static bool all_there(const Pack16 (&x)[CHUNKS]) {
+  __device__ __forceinline__ static bool all_there(const u32x4_t (&x)[CHUNKS]) {
     unsigned least = 0;                                  // (the mark is the largest word)
 #pragma unroll
-    for (int j = 0; j < N; ++j) least = max(max(least, max(x[j].u.x, x[j].u.y)), max(x[j].u.z, x[j].u.w));
+    for (int j = 0; j < N; ++j) least = max(max(least, max(x[j].x, x[j].y)), max(x[j].z, x[j].w));
     return __all(least != ABSENT);
   }
   // The look at the exchange is the wait: a word without the mark is there.
   template <int N>
-  __device__ __forceinline__ void fetch(Pack16 (&x)[CHUNKS], const Rows& r, int i, int left) {
+  __device__ __forceinline__ void fetch(u32x4_t (&x)[CHUNKS], const Rows& r, int i, int left) {
     const int at = r.at + 64 * i;
     if (i == 0 && a.rows >= 4 && left > 0) {   // one look at one place first: so many rows asked for again and again hold up those that write them
       const int place = __builtin_amdgcn_readfirstlane(at) + 64 * (min(left, N) - 1);
@@ -290,7 +315,7 @@ struct Block {
     }
     for (int n = 0;; ++n) {
       compiler_fence();
-      look<N>(x, r, at, left);
+      look<N>(x, r, anew(at), left);
       if (all_there<N>(x) || !again(n)) break;
     }
   }
@@ -317,7 +342,7 @@ struct Block {
     const int own = number(which, OWN), stride = number(which, STRIDE), off = lane * 16;
     int at = number(which, START) + done * stride;
     u32x4_t sums = {0, 0, 0, 0};
-    Pack16 x[CHUNKS];
+    u32x4_t x[CHUNKS];
     if (own > 8) {
       const bool sections = own > 16;                    // (whose rows are asked for with every slab)
       if (!sections) {
@@ -337,15 +362,15 @@ struct Block {
           const bool ends = i + 16 >= own;
           if (!ends || s + 1 < slabs) {
             const auto next = ends ? after : here;
-            const int from = ends ? off : off + ((i + 16) << 10);
+            const int from = anew(ends ? off : off + ((i + 16) << 10));
 #pragma unroll
             for (int j = 0; j < CHUNKS; ++j) {
-              acc[j & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j].v, x[j].v, acc[j & 1], 0, 0, 0);
-              load(w[j], next, from + 1024 * j);
+              acc[j & 1] = dot(w[j], x[j], acc[j & 1]);
+              w[j] = load(next, from + 1024 * j);
             }
           } else {
 #pragma unroll
-            for (int j = 0; j < CHUNKS; ++j) acc[j & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j].v, x[j].v, acc[j & 1], 0, 0, 0);
+            for (int j = 0; j < CHUNKS; ++j) acc[j & 1] = dot(w[j], x[j], acc[j & 1]);
           }
         }
         leave(acc[0] + acc[1], s);
@@ -359,8 +384,8 @@ struct Block {
 #pragma unroll
         for (int q = 0; q < 4; ++q) acc[q] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int j = 0; j < CHUNKS; ++j) acc[j >> 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j].v, x[j & 7].v, acc[j >> 2], 0, 0, 0);
-        if (s + 2 < slabs) ask<8>(matrix, at += 2 * stride, stride, slabs - s - 2, own);
+        for (int j = 0; j < CHUNKS; ++j) acc[j >> 2] = dot(w[j], x[j & 7], acc[j >> 2]);
+        if (s + 2 < slabs) ask(matrix, at += 2 * stride, stride, slabs - s - 2, own);
         leave(acc[0] + acc[1], s);
         if (s + 1 < slabs) leave(acc[2] + acc[3], s + 1);
       }
@@ -373,8 +398,8 @@ struct Block {
 #pragma unroll
         for (int q = 0; q < 4; ++q) acc[q] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int j = 0; j < CHUNKS; ++j) acc[j >> 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j].v, x[j & 3].v, acc[j >> 2], 0, 0, 0);
-        if (s + 4 < slabs) ask<4>(matrix, at += 4 * stride, stride, slabs - s - 4, own);
+        for (int j = 0; j < CHUNKS; ++j) acc[j >> 2] = dot(w[j], x[j & 3], acc[j >> 2]);
+        if (s + 4 < slabs) ask(matrix, at += 4 * stride, stride, slabs - s - 4, own);
 #pragma unroll
         for (int q = 0; q < 4; ++q)
           if (s + q < slabs) leave(acc[q], s + q);
@@ -418,7 +443,7 @@ struct Block {
     u32x4_t raw;
   };
   __device__ __forceinline__ Follow follow(int which, int done, int slabs, const void* norm) const {
-    const int tid = anew(this->tid), q = tid >> 2, s = over_rows(q), row = q - s * a.rows, n = (number(which, SLAB) + (done + s) * blocks) * 16 + 4 * (tid & 3);
+    const int tid = anew(this->tid), q = tid >> 2, s = over_rows(q), row = q - s * a.rows, n = (number(which, SLAB) + (done + s) * number(which, STEP)) * 16 + 4 * (tid & 3);
     Follow f;
     f.res = make_float4(0.f, 0.f, 0.f, 0.f);
     f.raw = u32x4_t{0, 0, 0, 0};
@@ -431,9 +456,9 @@ struct Block {
   __device__ __forceinline__ void finish(__amdgpu_buffer_rsrc_t ex, int which, int done, int slabs, const void* norm, Follow f) {
     const bool stream = which & 1;
     const int tid = anew(this->tid), entries = slabs * 4 * a.rows, grp = tid & 3;
-    const int width = number(which, OUT_WIDTH), dst = number(which, DST), first = number(which, SLAB) + done * blocks;
+    const int width = number(which, OUT_WIDTH), dst = number(which, DST), step = number(which, STEP), first = number(which, SLAB) + done * step;
     if (tid < entries) {         // (a thread has one at most)
-      const int q = tid >> 2, s = over_rows(q), row = q - s * a.rows, slab = first + s * blocks, n = slab * 16 + 4 * grp;
+      const int q = tid >> 2, s = over_rows(q), row = q - s * a.rows, slab = first + s * step, n = slab * 16 + 4 * grp;
       const char* part = sh.red[turn] + (unsigned)((s * WAVES * 4 + grp) * a.rows + row) * 16;
       f32x4_t share[WAVES];
 #pragma unroll
@@ -460,8 +485,8 @@ struct Block {
             pk.e[e] = (__bf16)(x[e] * w4[e]);
           }
           put8(ex, dst + (row * width + n) * 2, pk.u);
-          ss += __shfl_xor(ss, 1, 64);
-          ss += __shfl_xor(ss, 2, 64);
+          ss += quad_xor<1>(ss);
+          ss += quad_xor<2>(ss);
           if (grp == 0) put4(ex, number(which, DST_SUMS) + (row * (width / 16) + slab) * 4, __float_as_uint(ss), 0x7fc00000u);
         }
         store16(a.residual + (size_t)row * a.width + n,
@@ -521,6 +546,25 @@ struct Block {
     }
     return p;
   }
+  // attention_tiles.h's tile_addr (with the lane as a number of its own: what follows from it is not kept over the launch)
+  __device__ __forceinline__ TileAddr addr_of(const TilePages& p, const bf16_t* keys, const bf16_t* values, int g_kv, int tile) const {
+    const int lane = anew(this->lane), col = lane & 15, grp = lane >> 4;
+    long kh[2], vh[2];
+    TileAddr t;
+    t.there = 0;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const bool there = p.pg[h] >= 0 && p.pg[h] < a.num_pages;
+      const long head = (long)(there ? p.pg[h] : 0) * a.kv_heads + g_kv;
+      const int slot = (tile * FAST_TILE + 16 * h) & (a.page - 1);
+      kh[h] = (head * a.page + slot) * HEAD;
+      vh[h] = head * HEAD * a.page + slot;
+      t.there |= there ? 1 << h : 0;
+    }
+    t.k = keys + (col >> 3 ? kh[1] : kh[0]) + (unsigned)((8 * ((col >> 2) & 1) + (col & 3)) * HEAD + 8 * grp);
+    t.v = values + (grp >> 1 ? vh[1] : vh[0]) + (unsigned)(col * a.page + 8 * (grp & 1));
+    return t;
+  }
   __device__ __forceinline__ Item item_of(int n) const {
     Item it;
     const int pair = n / a.splits;
@@ -529,7 +573,7 @@ struct Block {
     it.g_kv = pair - it.b * a.kv_heads;
     it.kv_len = ((entries_ptr)(uintptr_t)a.kv_lens)[it.b];
     const int first = it.split * WAVES + wave;
-    const TileAddr t = tile_addr(pages_of(it.b, first), nullptr, nullptr, a.num_pages, a.kv_heads, it.g_kv, a.page, HEAD, HEAD, first * FAST_TILE);
+    const TileAddr t = addr_of(pages_of(it.b, first), nullptr, nullptr, it.g_kv, first);
     it.there = t.there;
     it.keys = (uint64_t)t.k;
     it.values = (uint64_t)t.v;
@@ -554,9 +598,6 @@ struct Block {
     const bool turned = a.table != nullptr && pos >= 0 && pos < a.max_pos;
     const int kv_seen = max(pos, 0), row_pos = col < G ? pos - 1 : -1;
     const int last = (kv_seen + FAST_TILE - 1) / FAST_TILE;
-    auto addr_of = [&](const TilePages& p, int t) {
-      return tile_addr(p, keys, values, a.num_pages, a.kv_heads, g_kv, a.page, D, D, t * FAST_TILE);
-    };
     TileRegs<D, D> r;
     auto ask_keys = [&](const TileAddr& to) {
       r.at = to;
@@ -662,7 +703,7 @@ struct Block {
         for (int j = 0; j < D / 32; ++j) sc[kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(r.k[kb][j].v, q[j].v, sc[kb], 0, 0, 0);
       }
       if (more) {
-        ask_keys(addr_of(next, t + step));
+        ask_keys(addr_of(next, keys, values, g_kv, t + step));
         next = pages_of(b, t + 2 * step);
       }
       const Pack16 p = softmax_step<D / 16>(sc, false, key0, grp, row_pos, 0, a.scale_log2, m_run, l_run, acc);
@@ -800,10 +841,12 @@ struct Block {
 
   __device__ __forceinline__ void layers() {
     const int items = a.rows * a.kv_heads * a.splits, pairs = a.rows * a.kv_heads;
-    Item mine = item_of(min(rank, items - 1));
+    const Roles roles(a, blocks);
+    const int my_item = roles.item(rank, blocks), my_pair = roles.pair(rank, blocks), pair_step = blocks - roles.apart;
+    Item mine = item_of(min(my_item, items - 1));
     sh.first_at[tid][0] = mine.keys;
     sh.first_at[tid][1] = mine.values;
-    const int my_pair = rank >= blocks / 4 ? rank - blocks / 4 : rank + blocks - blocks / 4, my_b = my_pair / a.kv_heads, my_g = my_pair - my_b * a.kv_heads;
+    const int my_b = my_pair / a.kv_heads, my_g = my_pair - my_b * a.kv_heads;
     look_ahead(0, 0);
 #pragma unroll 1
     for (int n = 0; n < a.count; ++n) {
@@ -814,16 +857,16 @@ struct Block {
         asm volatile("" : "+v"(lane), "+v"(tid));
         if (which == 1) {
 #pragma unroll 1
-          for (int n_item = rank; n_item < items; n_item += blocks) {
+          for (int n_item = my_item; n_item < items; n_item += blocks) {
             Item it = mine;
             it.keys = sh.first_at[tid][0];
             it.values = sh.first_at[tid][1];
-            if (n_item != rank) it = item_of(n_item);
+            if (n_item != my_item) it = item_of(n_item);
             attend(ex, n, it);
           }
           if (a.splits > 1)      // (its loads would come behind the next weights')
 #pragma unroll 1
-            for (int pair = my_pair; pair < pairs; pair += blocks) {
+            for (int pair = my_pair; pair < pairs; pair += pair_step) {
               const bool first = pair == my_pair;
               const int b = first ? my_b : pair / a.kv_heads, g = first ? my_g : pair - pair / a.kv_heads * a.kv_heads;
               merge(ex, g, b);
@@ -849,7 +892,7 @@ struct Block {
     if (!alive) {              // a wait that did not end: no number of the result stands
       for (int done = 0; done < number(3, COUNT); ++done)
         for (int idx = tid; idx < 16 * a.rows; idx += THREADS)
-          a.residual[(size_t)(idx >> 4) * a.width + (number(3, SLAB) + done * blocks) * 16 + (idx & 15)] = __uint_as_float(0x7fc00000u);
+          a.residual[(size_t)(idx >> 4) * a.width + (number(3, SLAB) + done * number(3, STEP)) * 16 + (idx & 15)] = __uint_as_float(0x7fc00000u);
     }
   }
 };
