@@ -41,12 +41,12 @@ constexpr int THREADS = 64 * WAVES;
 constexpr int HEAD = 128;                     // the head size
 constexpr int MOST_SLABS = 8;                 // slabs of 16 weight rows that a block multiplies between two barriers
 constexpr int RESULTS = 64;                   // of them times rows, at most
-constexpr int CHUNKS = 16;                    // kilobytes of weights that a wavefront has on their way
+constexpr int CHUNKS = 16;                    // steps of K, times groups of sixteen rows, that a wavefront has in registers
 constexpr unsigned ABSENT = 0xffffffffu;      // a word of the exchange that nobody has written yet
 constexpr unsigned CLOSED = 0x80000000u;
 constexpr int THROUGH = 16;                   // cache policy of what blocks exchange: past the chiplets' own caches (sc1)
 constexpr int MOST_SPLITS = 32;
-constexpr int MOST_ROWS = 16;
+constexpr int MOST_ROWS = 32;                 // in two groups of sixteen
 constexpr int MOST_LAYERS = 128;
 constexpr int NOWHERE = 1 << 30;              // an offset behind the end of every buffer: reads of it are zero
 
@@ -87,7 +87,7 @@ struct Shared {
   AttentionShared attention;
   __attribute__((aligned(16))) uint64_t layers[MOST_LAYERS * sizeof(Layer) / 8];
   uint64_t first_at[THREADS][2];              // where a thread's first keys and values of the block's first item lie in each layer's caches
-  float scale[16];
+  float scale[MOST_ROWS];
   int rank, blocks;
 };
 
@@ -190,7 +190,7 @@ typedef const __attribute__((address_space(4))) int* entries_ptr;
 constexpr int LAYER_WORDS = sizeof(Layer) / 8;
 enum { Q_NORM = 4, K_NORM, ENTRY_NORM, MIDDLE_NORM, KEYS, VALUES, EPS };    // words of an entry behind its four matrices
 
-template <typename QKW>
+template <typename QKW, int GROUPS>
 struct Block {
   Shared& sh;
   const Args& a;
@@ -203,7 +203,8 @@ struct Block {
   unsigned rows_inverse;
   int turn;                    // of the two halves of shared memory's results
   int held;                    // the product whose first weights are on their way: four times its layer, and which
-  u32x4_t w[CHUNKS];           // they
+  static constexpr int STEPS = CHUNKS / GROUPS;          // kilobytes of weights that a wavefront has on their way
+  u32x4_t w[STEPS];            // they
 
   // (as a number of its own: what is computed from it is not kept in registers over the whole launch)
   __device__ __forceinline__ static int anew(int v) {
@@ -230,7 +231,7 @@ struct Block {
   __device__ __forceinline__ void forget() {
     u32x4_t nothing;
 #pragma unroll
-    for (int j = 0; j < CHUNKS; ++j) {
+    for (int j = 0; j < STEPS; ++j) {
       asm volatile("" : "=v"(nothing));
       w[j] = nothing;
     }
@@ -243,12 +244,12 @@ struct Block {
   __device__ __forceinline__ static f32x4_t dot(const u32x4_t& w, const u32x4_t& x, const f32x4_t& acc) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, w), __builtin_bit_cast(bf16x8_t, x), acc, 0, 0, 0);
   }
-  // Sixteen kilobytes of `left` slabs: as many steps of one, or where K has no more for a wavefront, eight of two or four of four. (One
-  // sequence for all three: registers that several may have loaded are copied behind each, and so waited for.)
+  // STEPS kilobytes of `left` slabs: as many steps of one, or where K has no more for a wavefront, eight of two or four of four. (One
+  // sequence for all: registers that several may have loaded are copied behind each, and so waited for.)
   __device__ __forceinline__ void ask(uint64_t matrix, int at, int stride, int left, int own) {
-    const int off = anew(lane) * 16, bits = own > 8 ? 2 : own > 4 ? 1 : 0;
+    const int off = anew(lane) * 16, bits = own <= 4 ? 0 : STEPS == 8 || own <= 8 ? 1 : 2;
 #pragma unroll
-    for (int quarter = 0; quarter < 4; ++quarter) {
+    for (int quarter = 0; quarter < STEPS / 4; ++quarter) {
       const int s = quarter >> bits;
       if (quarter == 0 || s < left) {
         const auto r = slab_of(matrix, at + s * stride, own);
@@ -276,37 +277,41 @@ struct Block {
   // What a product multiplies with: K numbers a row at `src` of the exchange, their squares' partial sums at `sums`
   struct Rows {
     __amdgpu_buffer_rsrc_t ex;
-    int src, sums, at;           // (at: the lane's first eight numbers, row lane % 16 and eight k of 32; nowhere for a row that is none)
+    int src, sums;
+    int at[GROUPS];              // the lane's first eight numbers, row lane % 16 (and 16 behind it) and eight k of 32; nowhere for a row that is none
     float eps;
   };
-  // N steps of rows, `left` of which there are, from `at` on
+  // N steps of rows, `left` of which there are, from step `i` on; of a second group behind those of the first
   template <int N>
-  __device__ __forceinline__ static void look(u32x4_t (&x)[CHUNKS], const Rows& r, int at, int left) {
+  __device__ __forceinline__ static void look(u32x4_t (&x)[CHUNKS], const Rows& r, int i, int left) {
 #pragma unroll
-    for (int quarter = 0; quarter < N / 4; ++quarter) {
-      const int from = N < 16 || quarter == 0 || left > 4 * quarter ? at : NOWHERE;
+    for (int g = 0; g < GROUPS; ++g) {
+      const int at = anew(r.at[g] + 64 * i);
 #pragma unroll
-      for (int j = 4 * quarter; j < 4 * quarter + 4; ++j) x[j] = peek16(r.ex, from + 64 * j, r.src);
-    }
-    if (left < N && (left == 0 || left & 3)) {
+      for (int quarter = 0; quarter < N / 4; ++quarter) {
+        const int from = N < STEPS || quarter == 0 || left > 4 * quarter ? at : NOWHERE;
 #pragma unroll
-      for (int j = 0; j < N; ++j)
-        if (j >= left) x[j] = u32x4_t{0, 0, 0, 0};
+        for (int j = 4 * quarter; j < 4 * quarter + 4; ++j) x[N * g + j] = peek16(r.ex, from + 64 * j, r.src);
+      }
+      if (left < N && (left == 0 || left & 3)) {
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+          if (j >= left) x[N * g + j] = u32x4_t{0, 0, 0, 0};
+      }
     }
   }
   template <int N>
   __device__ __forceinline__ static bool all_there(const u32x4_t (&x)[CHUNKS]) {
     unsigned least = 0;                                  // (the mark is the largest word)
 #pragma unroll
-    for (int j = 0; j < N; ++j) least = max(max(least, max(x[j].x, x[j].y)), max(x[j].z, x[j].w));
+    for (int j = 0; j < N * GROUPS; ++j) least = max(max(least, max(x[j].x, x[j].y)), max(x[j].z, x[j].w));
     return __all(least != ABSENT);
   }
   // The look at the exchange is the wait: a word without the mark is there.
   template <int N>
   __device__ __forceinline__ void fetch(u32x4_t (&x)[CHUNKS], const Rows& r, int i, int left) {
-    const int at = r.at + 64 * i;
     if (i == 0 && a.rows >= 4 && left > 0) {   // one look at one place first: so many rows asked for again and again hold up those that write them
-      const int place = __builtin_amdgcn_readfirstlane(at) + 64 * (min(left, N) - 1);
+      const int place = __builtin_amdgcn_readfirstlane(r.at[0]) + 64 * (min(left, N) - 1);
       for (int n = 0;; ++n) {
         compiler_fence();
         const u32x4_t v = peek16(r.ex, place, r.src);
@@ -315,7 +320,7 @@ struct Block {
     }
     for (int n = 0;; ++n) {
       compiler_fence();
-      look<N>(x, r, anew(at), left);
+      look<N>(x, r, i, left);
       if (all_there<N>(x) || !again(n)) break;
     }
   }
@@ -330,52 +335,61 @@ struct Block {
   }
 
   // A slab's sums of this wavefront's steps into shared memory
-  __device__ __forceinline__ void leave(const f32x4_t& acc, int slab) {
-    const int col = lane & 15, grp = lane >> 4;
+  __device__ __forceinline__ void leave(const f32x4_t& acc, int slab, int group) {
+    const int col = (lane & 15) + 16 * group, grp = lane >> 4;
     if (col < a.rows) *reinterpret_cast<f32x4_t*>(sh.red[turn] + (unsigned)(((slab * WAVES + wave) * 4 + grp) * a.rows + col) * 16) = acc;
   }
 
   // `slabs` slabs from `done` on, whose first group's weights have been asked for. With `scaled`, the first look at the rows' sums is
   // asked for between the rows and the multiplications.
-  __device__ __forceinline__ u32x4_t multiply(const Rows& r, int layer, int which, int done, int slabs, bool scaled) {
+  struct Sums {
+    u32x4_t v[2 * GROUPS];       // of every eighth row, from the wavefront's number on
+  };
+  __device__ __forceinline__ Sums multiply(const Rows& r, int layer, int which, int done, int slabs, bool scaled) {
     const uint64_t matrix = entry(layer, which);
     const int own = number(which, OWN), stride = number(which, STRIDE), off = lane * 16;
     int at = number(which, START) + done * stride;
-    u32x4_t sums = {0, 0, 0, 0};
+    Sums sums;
     u32x4_t x[CHUNKS];
-    if (own > 8) {
-      const bool sections = own > 16;                    // (whose rows are asked for with every slab)
+    if (own > STEPS / 2) {
+      const bool sections = own > STEPS;                 // (whose rows are asked for with every slab)
       if (!sections) {
-        fetch<16>(x, r, 0, own);
+        fetch<STEPS>(x, r, 0, own);
         if (scaled) sums = first_sums(r);
       }
 #pragma unroll 1
       for (int s = 0; s < slabs; ++s, at += stride) {
         const auto here = slab_of(matrix, at, own), after = slab_of(matrix, at + stride, own);
-        f32x4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+        f32x4_t acc[2][GROUPS];
+#pragma unroll
+        for (int g = 0; g < GROUPS; ++g) acc[0][g] = acc[1][g] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
-        for (int i = 0; i < own; i += 16) {
+        for (int i = 0; i < own; i += STEPS) {
           if (sections) {
-            fetch<16>(x, r, i, own - i);
+            fetch<STEPS>(x, r, i, own - i);
             if (scaled && i == 0 && s == 0) sums = first_sums(r);
           }
-          const bool ends = i + 16 >= own;
+          const bool ends = i + STEPS >= own;
           if (!ends || s + 1 < slabs) {
             const auto next = ends ? after : here;
-            const int from = anew(ends ? off : off + ((i + 16) << 10));
+            const int from = anew(ends ? off : off + ((i + STEPS) << 10));
 #pragma unroll
-            for (int j = 0; j < CHUNKS; ++j) {
-              acc[j & 1] = dot(w[j], x[j], acc[j & 1]);
+            for (int j = 0; j < STEPS; ++j) {
+#pragma unroll
+              for (int g = 0; g < GROUPS; ++g) acc[j & 1][g] = dot(w[j], x[STEPS * g + j], acc[j & 1][g]);
               w[j] = load(next, from + 1024 * j);
             }
           } else {
 #pragma unroll
-            for (int j = 0; j < CHUNKS; ++j) acc[j & 1] = dot(w[j], x[j], acc[j & 1]);
+            for (int j = 0; j < STEPS; ++j)
+#pragma unroll
+              for (int g = 0; g < GROUPS; ++g) acc[j & 1][g] = dot(w[j], x[STEPS * g + j], acc[j & 1][g]);
           }
         }
-        leave(acc[0] + acc[1], s);
+#pragma unroll
+        for (int g = 0; g < GROUPS; ++g) leave(acc[0][g] + acc[1][g], s, g);
       }
-    } else if (own > 4) {
+    } else if (STEPS > 8 && own > 4) {
       fetch<8>(x, r, 0, own);
       if (scaled) sums = first_sums(r);
 #pragma unroll 1
@@ -384,40 +398,56 @@ struct Block {
 #pragma unroll
         for (int q = 0; q < 4; ++q) acc[q] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int j = 0; j < CHUNKS; ++j) acc[j >> 2] = dot(w[j], x[j & 7], acc[j >> 2]);
+        for (int j = 0; j < STEPS; ++j) acc[j >> 2] = dot(w[j], x[j & 7], acc[j >> 2]);
         if (s + 2 < slabs) ask(matrix, at += 2 * stride, stride, slabs - s - 2, own);
-        leave(acc[0] + acc[1], s);
-        if (s + 1 < slabs) leave(acc[2] + acc[3], s + 1);
+        leave(acc[0] + acc[1], s, 0);
+        if (s + 1 < slabs) leave(acc[2] + acc[3], s + 1, 0);
       }
     } else {
+      constexpr int EACH = STEPS / 4;
       fetch<4>(x, r, 0, own);
       if (scaled) sums = first_sums(r);
 #pragma unroll 1
-      for (int s = 0; s < slabs; s += 4) {
-        f32x4_t acc[4];
+      for (int s = 0; s < slabs; s += EACH) {
+        f32x4_t acc[EACH][GROUPS];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) acc[q] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        for (int q = 0; q < EACH; ++q)
 #pragma unroll
-        for (int j = 0; j < CHUNKS; ++j) acc[j >> 2] = dot(w[j], x[j & 3], acc[j >> 2]);
-        if (s + 4 < slabs) ask(matrix, at += 4 * stride, stride, slabs - s - 4, own);
+          for (int g = 0; g < GROUPS; ++g) acc[q][g] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-          if (s + q < slabs) leave(acc[q], s + q);
+        for (int j = 0; j < STEPS; ++j)
+#pragma unroll
+          for (int g = 0; g < GROUPS; ++g) acc[j >> 2][g] = dot(w[j], x[4 * g + (j & 3)], acc[j >> 2][g]);
+        if (s + EACH < slabs) ask(matrix, at += EACH * stride, stride, slabs - s - EACH, own);
+#pragma unroll
+        for (int q = 0; q < EACH; ++q)
+#pragma unroll
+          for (int g = 0; g < GROUPS; ++g)
+            if (s + q < slabs) leave(acc[q][g], s + q, g);
       }
     }
     return sums;
   }
 
-  // The rows' scales from the partial sums of squares, [row][slab]; `v`: the first of them, as they were when the rows had come
-  __device__ __forceinline__ u32x4_t first_sums(const Rows& r) const {
+  // The rows' scales from the partial sums of squares, [row][slab]; `first`: the first of them, as they were when the rows had come
+  __device__ __forceinline__ Sums first_sums(const Rows& r) const {
     const int lane = anew(this->lane), slabs = a.width / 16;
-    return peek16(r.ex, wave < a.rows && lane * 4 < slabs ? (wave * slabs + lane * 4) * 4 : NOWHERE, r.sums);
+    Sums first;
+#pragma unroll
+    for (int i = 0; i < 2 * GROUPS; ++i) {
+      const int row = wave + WAVES * i;
+      first.v[i] = peek16(r.ex, row < a.rows && lane * 4 < slabs ? (row * slabs + lane * 4) * 4 : NOWHERE, r.sums);
+    }
+    return first;
   }
-  __device__ __forceinline__ void scales(const Rows& r, u32x4_t v) {
+  __device__ __forceinline__ void scales(const Rows& r, Sums first) {
     const int slabs = a.width / 16;
-    bool asked = true;
-#pragma unroll 1
-    for (int row = wave; row < a.rows; row += WAVES) {
+#pragma unroll
+    for (int i = 0; i < 2 * GROUPS; ++i) {
+      const int row = wave + WAVES * i;
+      if (row >= a.rows) break;
+      u32x4_t v = first.v[i];
+      bool asked = true;
       float s = 0.f;
 #pragma unroll 1
       for (int k = lane * 4; __builtin_amdgcn_readfirstlane(k) < slabs; k += 256) {
@@ -517,7 +547,7 @@ struct Block {
       Follow f;
       if (which & 1) f = follow(which, done, slabs, norm);
       const bool scaled = done == 0 && !(which & 1);
-      const u32x4_t sums = multiply(r, layer, which, done, slabs, scaled);
+      const Sums sums = multiply(r, layer, which, done, slabs, scaled);
       if (scaled) scales(r, sums);
       forget();
       meet();
@@ -880,7 +910,9 @@ struct Block {
         r.ex = which == 0 ? buffer_of(a.exchange + (n - 1) * a.per_layer, a.per_layer) : ex;
         r.src = number(which, SRC);
         r.sums = number(which, SUMS);
-        r.at = col < a.rows ? col * number(which, ROW_BYTES) + 64 * number(which, FIRST_STEP) + 16 * (lane >> 4) : NOWHERE;
+#pragma unroll
+        for (int g = 0; g < GROUPS; ++g)
+          r.at[g] = col + 16 * g < a.rows ? (col + 16 * g) * number(which, ROW_BYTES) + 64 * number(which, FIRST_STEP) + 16 * (lane >> 4) : NOWHERE;
         const uint64_t eps = entry(n, EPS);
         r.eps = __uint_as_float((unsigned)(which == 0 ? eps : eps >> 32));
         // (the last layer's down product prepares no rows: its norm is the one behind the layers, of another kernel)
@@ -931,7 +963,7 @@ __device__ __forceinline__ void gather(const Args& a, int& rank, int& blocks) {
   }
 }
 
-template <typename QKW>
+template <typename QKW, int GROUPS>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void decode_layers_kernel(Args a) {
   __shared__ Shared sh;
   if (threadIdx.x == 0) gather(a, sh.rank, sh.blocks);
@@ -941,7 +973,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
   for (int i = threadIdx.x; i < a.count * LAYER_WORDS; i += THREADS) sh.layers[i] = reinterpret_cast<const uint64_t*>(a.layers)[i];
   __syncthreads();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  Block<QKW> b{sh, a, rank, blocks, wave, (int)threadIdx.x & 63, (int)threadIdx.x, numbers_of(a, rank, blocks, wave, threadIdx.x & 63),
+  Block<QKW, GROUPS> b{sh, a, rank, blocks, wave, (int)threadIdx.x & 63, (int)threadIdx.x, numbers_of(a, rank, blocks, wave, threadIdx.x & 63),
                   min(MOST_SLABS, RESULTS / a.rows), a.limit, 1, (1u << 20) / a.rows + 1, 0, -1};
   b.layers();
 }
@@ -1007,7 +1039,7 @@ inline Layout layout_of(long rows, long width, long heads, long kv_heads, long i
 
 // (every wavefront of a block has a step of 32 of each product's K at least: the smallest K is 256, from two heads on)
 inline bool sizes_fit(int rows, int width, int heads, int kv_heads, int dim, int inner) {
-  return rows >= 1 && rows <= MOST_ROWS && dim == HEAD && heads >= 1 && kv_heads >= 1 && heads % kv_heads == 0 && heads / kv_heads <= 16 &&
+  return rows >= 1 && rows <= (width <= 1024 ? MOST_ROWS : 16) && dim == HEAD && heads >= 1 && kv_heads >= 1 && heads % kv_heads == 0 && heads / kv_heads <= 16 &&
          width >= 32 * WAVES && width % 128 == 0 && inner >= 32 * WAVES && inner % 128 == 0 && heads * HEAD >= 32 * WAVES &&
          width <= (1 << 16) && inner <= (1 << 18) && heads <= 512;
 }
@@ -1084,10 +1116,9 @@ int q3_decode_layers(const Layer* layers, int count, float* residual, int rows, 
   a.patience = patience, a.limit = limit;
   a.qk_eps = qk_eps;
   a.scale_log2 = make_score_scale(scale);
-  if (qk_dtype == Q3_F32)
-    hipLaunchKernelGGL(decode_layers_kernel<float>, dim3(blocks), dim3(THREADS), 0, stream, a);
-  else
-    hipLaunchKernelGGL(decode_layers_kernel<bf16_t>, dim3(blocks), dim3(THREADS), 0, stream, a);
+  void (*kernel)(Args) = qk_dtype == Q3_F32 ? (rows > 16 ? decode_layers_kernel<float, 2> : decode_layers_kernel<float, 1>)
+                                            : (rows > 16 ? decode_layers_kernel<bf16_t, 2> : decode_layers_kernel<bf16_t, 1>);
+  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(THREADS), 0, stream, a);
   return q3_launch_status();
 }
 

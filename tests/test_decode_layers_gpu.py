@@ -45,7 +45,8 @@ def _logits(model, lengths, steps, graphs=False, page=16, launch=True):
     (1, 1, {}, 16), (1, 32, {}, 16), (1, 700, dict(intermediate_size=3072), 16), (2, 2100, dict(hidden_size=640, intermediate_size=1408), 16),
     (3, 65, dict(num_attention_heads=8, num_key_value_heads=1), 32), (4, 300, dict(num_attention_heads=4, num_key_value_heads=4), 16),
     (5, 97, dict(hidden_size=2560, intermediate_size=9728), 16), (8, 513, {}, 16), (9, 40, dict(hidden_size=256, intermediate_size=384, num_attention_heads=2, num_key_value_heads=1), 16),
-    (16, 260, dict(intermediate_size=5120), 16)])
+    (16, 260, dict(intermediate_size=5120), 16), (17, 90, {}, 16), (24, 400, dict(intermediate_size=3072), 16),
+    (32, 35, dict(hidden_size=384, num_attention_heads=6, num_key_value_heads=2, intermediate_size=640), 16)])
 def test_against_the_parts(rows, longest, sizes, page):
     model = _model(**sizes)
     assert model.decode_run is not None
@@ -55,7 +56,7 @@ def test_against_the_parts(rows, longest, sizes, page):
     # both round every product and row to bfloat16 (each some 0.008 off exact numbers over these layers), at sums in other orders
     assert (got - want).norm() <= 0.02 * want.norm()
     assert not torch.equal(got, want)                    # (it was another kernel)
-    if rows in (1, 2, 3, 8, 16):                         # (sizes that graphs are captured for: no row fills up)
+    if rows in (1, 2, 3, 8, 16, 24):                        # (sizes that graphs are captured for: no row fills up)
         replayed = _logits(model, lengths, 3, page=page, graphs=True, launch=True)
         assert (replayed - want).norm() <= 0.02 * want.norm()
 
@@ -78,10 +79,12 @@ def test_what_is_not_taken():
 
     model = _model()
     native = model.decode_run.native
-    rows = torch.zeros(17, 1024, device="cuda")
+    rows = torch.zeros(33, 1024, device="cuda")
     caches = [(torch.zeros(4, 8, 16, 128, dtype=torch.bfloat16, device="cuda"), torch.zeros(4, 8, 128, 16, dtype=torch.bfloat16, device="cuda"))] * 3
-    table, lens = torch.zeros(17, 4, dtype=torch.int32, device="cuda"), torch.ones(17, dtype=torch.int32, device="cuda")
+    table, lens = torch.zeros(33, 4, dtype=torch.int32, device="cuda"), torch.ones(33, dtype=torch.int32, device="cuda")
     assert not native.run(rows, caches, table, lens, 1, None)                # more rows than there are registers for
+    wide = _model(hidden_size=1152).decode_run.native
+    assert not wide.run(torch.zeros(17, 1152, device="cuda"), caches, table, lens[:17], 1, None)      # or than it is the faster way for
     with pytest.raises(ops.OperandError):
         native.run(rows[:4], caches[:2], table, lens[:4], 1, None)
     with pytest.raises(ops.OperandError):
