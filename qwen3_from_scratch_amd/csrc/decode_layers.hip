@@ -1,5 +1,5 @@
 // All decoder layers of a step of single tokens in one launch: pre-norm layers of softmax attention with grouped heads of 128 and a
-// gated unit, bfloat16, up to 16 rows. What gemm.hip's few-row products and attention.hip's decoding attention do layer by layer.
+// gated unit, bfloat16, up to 16 rows, or 32 of a small model. What gemm.hip's few-row products and attention.hip's decoding attention do layer by layer.
 //
 // A kernel that waits for its predecessor costs 2 us inside a graph if it does nothing and 4 to 4.5 if it loads, reduces and stores a
 // row, and a step of the 0.6B shape was 145 of them: 1,011 us where its bytes take 240. Here a block per compute unit stays for all
@@ -11,9 +11,10 @@
 // meanwhile.
 //
 // What it measured (us a step in a graph, the layers' kernels one by one / this): the 0.6B shape, one request over 100 keys 971 / 533,
-// over 1,100 1,013 / 576, over 8,000 1,140 / 773, four 1,141 / 674, eight over 2,000 1,415 / 941, sixteen 1,910 / 1,369; the 8B shape, one over
-// 2,060 3,407 / 2,760, eight 3,954 / 3,460. The first form of this kernel (809, 3,026, 3,510) was faster than the kernels at each of 28 sizes
-// from 1 to 16 rows and 100 to 30,000 keys; more than 16 rows have no registers here.
+// over 1,100 1,013 / 575, over 8,000 1,140 / 773, four 1,141 / 668, eight over 2,000 1,415 / 927, sixteen 1,910 / 1,356, 20 over 770
+// 1,413 / 1,173, 24 over 2,000 2,003 / 1,725, 32 2,377 / 2,174; the 8B shape, one over 2,060 3,407 / 2,770, eight 3,954 / 3,310, sixteen
+// 4,836 / 4,150. The first form of this kernel (0.6B, one request 805; 8B 3,012) was faster than the kernels at each of 28 sizes from 1 to 16 rows and
+// 100 to 30,000 keys.
 //
 // What bounds it: one request of the small shape the chain of five or six exchanges a layer; a look that fails costs a second one behind
 // the first, a store holds up the wavefront's next look (they come back in order), and a wavefront alone on its SIMD takes 4 to 5 cycles
@@ -40,7 +41,7 @@ constexpr int WAVES = 8;                      // of a block
 constexpr int THREADS = 64 * WAVES;
 constexpr int HEAD = 128;                     // the head size
 constexpr int MOST_SLABS = 8;                 // slabs of 16 weight rows that a block multiplies between two barriers
-constexpr int RESULTS = 64;                   // of them times rows, at most
+constexpr int RESULTS = 128;                  // of them times rows, at most
 constexpr int CHUNKS = 16;                    // steps of K, times groups of sixteen rows, that a wavefront has in registers
 constexpr unsigned ABSENT = 0xffffffffu;      // a word of the exchange that nobody has written yet
 constexpr unsigned CLOSED = 0x80000000u;
@@ -82,8 +83,8 @@ struct AttentionShared {
   __attribute__((aligned(16))) float acc[WAVES][16][HEAD + 4];
 };
 struct Shared {
-  // the wavefronts' shares of K of a product: [slab][wavefront][four columns of sixteen][row], 16 bytes each; twice, in turn
-  __attribute__((aligned(16))) char red[2][RESULTS * WAVES * 4 * 16];
+  // the wavefronts' shares of K of a product: [slab][wavefront][four columns of sixteen][row], 16 bytes each
+  __attribute__((aligned(16))) char red[RESULTS * WAVES * 4 * 16];
   AttentionShared attention;
   __attribute__((aligned(16))) uint64_t layers[MOST_LAYERS * sizeof(Layer) / 8];
   uint64_t first_at[THREADS][2];              // where a thread's first keys and values of the block's first item lie in each layer's caches
@@ -190,7 +191,7 @@ typedef const __attribute__((address_space(4))) int* entries_ptr;
 constexpr int LAYER_WORDS = sizeof(Layer) / 8;
 enum { Q_NORM = 4, K_NORM, ENTRY_NORM, MIDDLE_NORM, KEYS, VALUES, EPS };    // words of an entry behind its four matrices
 
-template <typename QKW, int GROUPS>
+template <typename QKW, int GROUPS, bool MANY>
 struct Block {
   Shared& sh;
   const Args& a;
@@ -201,7 +202,6 @@ struct Block {
   int most;                    // looks at the exchange before a wait is given up
   int alive;
   unsigned rows_inverse;
-  int turn;                    // of the two halves of shared memory's results
   int held;                    // the product whose first weights are on their way: four times its layer, and which
   static constexpr int STEPS = CHUNKS / GROUPS;          // kilobytes of weights that a wavefront has on their way
   u32x4_t w[STEPS];            // they
@@ -305,9 +305,10 @@ struct Block {
     unsigned least = 0;                                  // (the mark is the largest word)
 #pragma unroll
     for (int j = 0; j < N * GROUPS; ++j) least = max(max(least, max(x[j].x, x[j].y)), max(x[j].z, x[j].w));
-    return __all(least != ABSENT);
+    return least != ABSENT;
   }
-  // The look at the exchange is the wait: a word without the mark is there.
+  // The look at the exchange is the wait: a word without the mark is there. With many rows, a lane that has all of its numbers asks no
+  // more (24 rows of the 0.6B shape 1,146 -> 1,122 us, sixteen 849 -> 837; one row 574 -> 582, and so not with few).
   template <int N>
   __device__ __forceinline__ void fetch(u32x4_t (&x)[CHUNKS], const Rows& r, int i, int left) {
     if (i == 0 && a.rows >= 4 && left > 0) {   // one look at one place first: so many rows asked for again and again hold up those that write them
@@ -318,10 +319,14 @@ struct Block {
         if (__builtin_amdgcn_readfirstlane((int)there(v)) || !again(n)) break;
       }
     }
+    bool have = false;
     for (int n = 0;; ++n) {
       compiler_fence();
-      look<N>(x, r, i, left);
-      if (all_there<N>(x) || !again(n)) break;
+      if (!MANY || !have) {
+        look<N>(x, r, i, left);
+        have = all_there<N>(x);
+      }
+      if (__all(have) || !again(n)) break;
     }
   }
   // Four of a norm's weights among the sixteen bytes around them, and as numbers
@@ -337,7 +342,7 @@ struct Block {
   // A slab's sums of this wavefront's steps into shared memory
   __device__ __forceinline__ void leave(const f32x4_t& acc, int slab, int group) {
     const int col = (lane & 15) + 16 * group, grp = lane >> 4;
-    if (col < a.rows) *reinterpret_cast<f32x4_t*>(sh.red[turn] + (unsigned)(((slab * WAVES + wave) * 4 + grp) * a.rows + col) * 16) = acc;
+    if (col < a.rows) *reinterpret_cast<f32x4_t*>(sh.red + (unsigned)(((slab * WAVES + wave) * 4 + grp) * a.rows + col) * 16) = acc;
   }
 
   // `slabs` slabs from `done` on, whose first group's weights have been asked for. With `scaled`, the first look at the rows' sums is
@@ -489,7 +494,7 @@ struct Block {
     const int width = number(which, OUT_WIDTH), dst = number(which, DST), step = number(which, STEP), first = number(which, SLAB) + done * step;
     if (tid < entries) {         // (a thread has one at most)
       const int q = tid >> 2, s = over_rows(q), row = q - s * a.rows, slab = first + s * step, n = slab * 16 + 4 * grp;
-      const char* part = sh.red[turn] + (unsigned)((s * WAVES * 4 + grp) * a.rows + row) * 16;
+      const char* part = sh.red + (unsigned)((s * WAVES * 4 + grp) * a.rows + row) * 16;
       f32x4_t share[WAVES];
 #pragma unroll
       for (int v = 0; v < WAVES; ++v) share[v] = *reinterpret_cast<const f32x4_t*>(part + (unsigned)(v * 4 * a.rows) * 16);
@@ -554,7 +559,6 @@ struct Block {
       finish(ex, which, done, slabs, norm, f);
       meet();                    // (the results on their way ahead of the other wavefronts' loads: 8B shape, one request, 3 us a product otherwise)
       if (done + slabs >= count && which != 0) look_ahead(layer, which + 1);
-      turn ^= 1;
     }
   }
 
@@ -963,7 +967,7 @@ __device__ __forceinline__ void gather(const Args& a, int& rank, int& blocks) {
   }
 }
 
-template <typename QKW, int GROUPS>
+template <typename QKW, int GROUPS, bool MANY>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void decode_layers_kernel(Args a) {
   __shared__ Shared sh;
   if (threadIdx.x == 0) gather(a, sh.rank, sh.blocks);
@@ -973,8 +977,8 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
   for (int i = threadIdx.x; i < a.count * LAYER_WORDS; i += THREADS) sh.layers[i] = reinterpret_cast<const uint64_t*>(a.layers)[i];
   __syncthreads();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  Block<QKW, GROUPS> b{sh, a, rank, blocks, wave, (int)threadIdx.x & 63, (int)threadIdx.x, numbers_of(a, rank, blocks, wave, threadIdx.x & 63),
-                  min(MOST_SLABS, RESULTS / a.rows), a.limit, 1, (1u << 20) / a.rows + 1, 0, -1};
+  Block<QKW, GROUPS, MANY> b{sh, a, rank, blocks, wave, (int)threadIdx.x & 63, (int)threadIdx.x, numbers_of(a, rank, blocks, wave, threadIdx.x & 63),
+                  min(MOST_SLABS, RESULTS / a.rows), a.limit, 1, (1u << 20) / a.rows + 1, -1};
   b.layers();
 }
 
@@ -1116,8 +1120,11 @@ int q3_decode_layers(const Layer* layers, int count, float* residual, int rows, 
   a.patience = patience, a.limit = limit;
   a.qk_eps = qk_eps;
   a.scale_log2 = make_score_scale(scale);
-  void (*kernel)(Args) = qk_dtype == Q3_F32 ? (rows > 16 ? decode_layers_kernel<float, 2> : decode_layers_kernel<float, 1>)
-                                            : (rows > 16 ? decode_layers_kernel<bf16_t, 2> : decode_layers_kernel<bf16_t, 1>);
+  void (*kernel)(Args);
+  if (qk_dtype == Q3_F32)
+    kernel = rows > 16 ? decode_layers_kernel<float, 2, true> : rows >= 8 ? decode_layers_kernel<float, 1, true> : decode_layers_kernel<float, 1, false>;
+  else
+    kernel = rows > 16 ? decode_layers_kernel<bf16_t, 2, true> : rows >= 8 ? decode_layers_kernel<bf16_t, 1, true> : decode_layers_kernel<bf16_t, 1, false>;
   hipLaunchKernelGGL(kernel, dim3(blocks), dim3(THREADS), 0, stream, a);
   return q3_launch_status();
 }
