@@ -127,6 +127,28 @@ __device__ __forceinline__ float quad_xor(float v) {
   return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), N == 1 ? 0xb1 : 0x4e, 0xf, 0xf, true));
 }
 
+// The lanes' sum, with wave_sum's bits: the same pairs are added in the same order, by the vector unit alone (a shuffle is a way
+// through shared memory, six of them 0.3 us on the way from one exchange to the next)
+template <int N>
+__device__ __forceinline__ float plus_rotated(float v) {      // rows of sixteen lanes; v repeats itself every 2 N of them
+  return v + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x120 + N, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float lanes_sum(float v) {
+  unsigned u = __float_as_uint(v);
+  const auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  u = __float_as_uint(v);
+  const auto b = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  v = __uint_as_float(b[0]) + __uint_as_float(b[1]);
+  return plus_rotated<1>(plus_rotated<2>(plus_rotated<4>(plus_rotated<8>(v))));
+}
+// Lane ^ 32's value
+__device__ __forceinline__ float other_half(float v, int lane) {
+  const unsigned u = __float_as_uint(v);
+  const auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return __uint_as_float(lane < 32 ? a[1] : a[0]);
+}
+
 // Until shared memory holds what the block's wavefronts have written (and nothing about memory)
 __device__ __forceinline__ void meet() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
@@ -465,7 +487,7 @@ struct Block {
         }
         s += (__uint_as_float(v.x) + __uint_as_float(v.y)) + (__uint_as_float(v.z) + __uint_as_float(v.w));
       }
-      s = wave_sum(s);
+      s = lanes_sum(s);
       if (lane == 0) sh.scale[row] = rsqrtf(s * (1.f / (float)a.width) + r.eps);
     }
   }
@@ -679,12 +701,12 @@ struct Block {
       }
       float x0 = __uint_as_float(v << 16), x1 = __uint_as_float(v & 0xffff0000u);
       if (prepared && q_norm != nullptr) {
-        const float scale = head_norm_scale(wave_sum(__fmaf_rn(x0, x0, __fmul_rn(x1, x1))), D, a.qk_eps);
+        const float scale = head_norm_scale(lanes_sum(__fmaf_rn(x0, x0, __fmul_rn(x1, x1))), D, a.qk_eps);
         x0 = __fmul_rn(__fmul_rn(x0, scale), __uint_as_float(sizeof(QKW) == 4 ? norm[0] : norm[0] << 16));
         x1 = __fmul_rn(__fmul_rn(x1, scale), __uint_as_float(sizeof(QKW) == 4 ? norm[1] : norm[0] & 0xffff0000u));
       }
       if (prepared && turned) {
-        const float y0 = __shfl_xor(x0, 32, 64), y1 = __shfl_xor(x1, 32, 64);
+        const float y0 = other_half(x0, lane), y1 = other_half(x1, lane);
         const float sign = lane < 32 ? -1.f : 1.f;
         x0 = __fmaf_rn(x0, cs.x, __fmul_rn(sign * y0, sn.x));
         x1 = __fmaf_rn(x1, cs.y, __fmul_rn(sign * y1, sn.y));
@@ -710,7 +732,7 @@ struct Block {
     if (brings_new) {                                 // the new key's scores: the rows shared out once more
       for (int row = wave; row < G; row += WAVES) {
         const bf16_t* mine = &s.q[row][2 * lane];
-        const float dot = wave_sum(fmaf(bf16_to_float(mine[0]), s.k[2 * lane], bf16_to_float(mine[1]) * s.k[2 * lane + 1]));
+        const float dot = lanes_sum(fmaf(bf16_to_float(mine[0]), s.k[2 * lane], bf16_to_float(mine[1]) * s.k[2 * lane + 1]));
         if (lane == 0) s.m[WAVES][row] = pos >= 0 ? dot * a.scale_log2 : -INFINITY;
       }
     } else if (wave == 0 && lane < 16) {
@@ -756,9 +778,7 @@ struct Block {
       for (int nb = 0; nb < D / 16; ++nb) acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(r.v[nb].v, p.v, acc[nb], 0, 0, 0);
       if (more) ask_values();
     }
-    float l_all = l_run;
-    l_all += __shfl_xor(l_all, 16, 64);
-    l_all += __shfl_xor(l_all, 32, 64);
+    const float l_all = quad_rows_sum(l_run);
     if (grp == 0) {
       s.m[wave][col] = m_run;
       s.l[wave][col] = l_all;
