@@ -127,21 +127,6 @@ __device__ __forceinline__ float quad_xor(float v) {
   return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), N == 1 ? 0xb1 : 0x4e, 0xf, 0xf, true));
 }
 
-// The lanes' sum, with wave_sum's bits: the same pairs are added in the same order, by the vector unit alone (a shuffle is a way
-// through shared memory, six of them 0.3 us on the way from one exchange to the next)
-template <int N>
-__device__ __forceinline__ float plus_rotated(float v) {      // rows of sixteen lanes; v repeats itself every 2 N of them
-  return v + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x120 + N, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float lanes_sum(float v) {
-  unsigned u = __float_as_uint(v);
-  const auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-  u = __float_as_uint(v);
-  const auto b = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  v = __uint_as_float(b[0]) + __uint_as_float(b[1]);
-  return plus_rotated<1>(plus_rotated<2>(plus_rotated<4>(plus_rotated<8>(v))));
-}
 // Lane ^ 32's value
 __device__ __forceinline__ float other_half(float v, int lane) {
   const unsigned u = __float_as_uint(v);
@@ -487,7 +472,7 @@ struct Block {
         }
         s += (__uint_as_float(v.x) + __uint_as_float(v.y)) + (__uint_as_float(v.z) + __uint_as_float(v.w));
       }
-      s = lanes_sum(s);
+      s = wave_sum(s);
       if (lane == 0) sh.scale[row] = rsqrtf(s * (1.f / (float)a.width) + r.eps);
     }
   }
@@ -701,7 +686,7 @@ struct Block {
       }
       float x0 = __uint_as_float(v << 16), x1 = __uint_as_float(v & 0xffff0000u);
       if (prepared && q_norm != nullptr) {
-        const float scale = head_norm_scale(lanes_sum(__fmaf_rn(x0, x0, __fmul_rn(x1, x1))), D, a.qk_eps);
+        const float scale = head_norm_scale(wave_sum(__fmaf_rn(x0, x0, __fmul_rn(x1, x1))), D, a.qk_eps);
         x0 = __fmul_rn(__fmul_rn(x0, scale), __uint_as_float(sizeof(QKW) == 4 ? norm[0] : norm[0] << 16));
         x1 = __fmul_rn(__fmul_rn(x1, scale), __uint_as_float(sizeof(QKW) == 4 ? norm[1] : norm[0] & 0xffff0000u));
       }
@@ -732,7 +717,7 @@ struct Block {
     if (brings_new) {                                 // the new key's scores: the rows shared out once more
       for (int row = wave; row < G; row += WAVES) {
         const bf16_t* mine = &s.q[row][2 * lane];
-        const float dot = lanes_sum(fmaf(bf16_to_float(mine[0]), s.k[2 * lane], bf16_to_float(mine[1]) * s.k[2 * lane + 1]));
+        const float dot = wave_sum(fmaf(bf16_to_float(mine[0]), s.k[2 * lane], bf16_to_float(mine[1]) * s.k[2 * lane + 1]));
         if (lane == 0) s.m[WAVES][row] = pos >= 0 ? dot * a.scale_log2 : -INFINITY;
       }
     } else if (wave == 0 && lane < 16) {
