@@ -10,11 +10,11 @@
 // block). The weights of a product's first steps are asked for while the last one's results are on their way, so memory is not idle
 // meanwhile.
 //
-// What it measured (us a step in a graph, the layers' kernels one by one / this): the 0.6B shape, one request over 100 keys 971 / 533,
-// over 1,100 1,013 / 575, over 8,000 1,140 / 773, four 1,141 / 668, eight over 2,000 1,415 / 927, sixteen 1,910 / 1,356, 20 over 770
-// 1,413 / 1,173, 24 over 2,000 2,003 / 1,725, 32 2,377 / 2,174; the 8B shape, one over 2,060 3,407 / 2,770, eight 3,954 / 3,310, sixteen
-// 4,836 / 4,150. The first form of this kernel (0.6B, one request 805; 8B 3,012) was faster than the kernels at each of 28 sizes from 1 to 16 rows and
-// 100 to 30,000 keys.
+// What it measured (us a step in a graph, the layers' kernels one by one / this): the 0.6B shape, one request over 100 keys 968 / 504,
+// over 1,100 1,012 / 561, over 8,000 1,142 / 751, over 30,000 1,530 / 1,132, four over 1,100 1,136 / 654, eight over 2,000 1,402 / 913,
+// sixteen 1,892 / 1,337, 20 over 770 1,404 / 1,139, 32 over 2,000 2,375 / 2,131; the 8B shape, one over 2,060 3,375 / 2,756, eight
+// 3,926 / 3,293, sixteen 4,796 / 4,115, eight over 8,000 5,020 / 4,383. The first form of this kernel (0.6B, one request 805; 8B 3,012) was
+// faster than the kernels at each of 28 sizes from 1 to 16 rows and 100 to 30,000 keys.
 //
 // What bounds it: one request of the small shape the chain of five or six exchanges a layer; a look that fails costs a second one behind
 // the first, a store holds up the wavefront's next look (they come back in order), and a wavefront alone on its SIMD takes 4 to 5 cycles
@@ -22,7 +22,7 @@
 // offsets that are constants of an instruction, steps of K in one stretch, bounds by the descriptors (500 instructions a product less:
 // 801 -> 779), the next weights asked for behind the results (779 -> 749; 8B 2,990 -> 2,860) and behind all wavefronts' results, with
 // the shares of K read together (749 -> 701; 2,860 -> 2,820), blocks of their own for the products into the stream of a small model (701 -> 597),
-// weights in registers that nothing copies (585 -> 576; 2,820 -> 2,760). The large shape is bound by its weights (5.5 of the
+// weights in registers that nothing copies (585 -> 576; 2,820 -> 2,760), lane sums in the vector unit (575 -> 563). The large shape is bound by its weights (5.5 of the
 // 5.8 TB/s that a plain read reaches, the whole step through) and the attention's part, where few weights move.
 // What did not help: the block split into wavefronts that multiply and wavefronts that look, prepare and store, with the weights in a
 // ring in shared memory (0.6B 905: more handovers a product), asking for the sums of squares together with the rows (lines that many blocks
@@ -58,7 +58,7 @@ struct Layer {
   void *keys, *values;
   float entry_eps, middle_eps;
 };
-constexpr int LAYERS_A_LAUNCH = 32;           // as many as the preparing kernel's arguments hold
+constexpr int LAYERS_A_LAUNCH = 40;           // as many as the preparing kernel's arguments hold
 struct LayerPack {
   Layer layer[LAYERS_A_LAUNCH];
 };
@@ -1046,7 +1046,9 @@ inline Layout layout_of(long rows, long width, long heads, long kv_heads, long i
   return l;
 }
 
-// (every wavefront of a block has a step of 32 of each product's K at least: the smallest K is 256, from two heads on)
+// Every wavefront of a block has a step of 32 of each product's K at least: the smallest K is 256, from two heads on. More than sixteen
+// rows of a wide model do not stay in registers from slab to slab and are asked for with each: 24 rows of the 8B shape over 2,060 keys
+// 5,964 us, 5,024 kernel by kernel, 20 over 1,000 5,229 and 4,327; of the 0.6B shape 17 over 100 947 and 1,149, 32 over 2,000 2,127 and 2,377.
 inline bool sizes_fit(int rows, int width, int heads, int kv_heads, int dim, int inner) {
   return rows >= 1 && rows <= (width <= 1024 ? MOST_ROWS : 16) && dim == HEAD && heads >= 1 && kv_heads >= 1 && heads % kv_heads == 0 && heads / kv_heads <= 16 &&
          width >= 32 * WAVES && width % 128 == 0 && inner >= 32 * WAVES && inner % 128 == 0 && heads * HEAD >= 32 * WAVES &&
