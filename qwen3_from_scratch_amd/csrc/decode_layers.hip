@@ -46,7 +46,10 @@ constexpr int CHUNKS = 16;                    // steps of K, times groups of six
 constexpr unsigned ABSENT = 0xffffffffu;      // a word of the exchange that nobody has written yet
 constexpr unsigned CLOSED = 0x80000000u;
 constexpr int THROUGH = 16;                   // cache policy of what blocks exchange: past the chiplets' own caches (sc1)
-constexpr int MOST_SPLITS = 32;
+constexpr int MOST_PARTS = 32;                // of a sequence's keys
+constexpr int ITEMS_MOST = 512;               // pieces of attention, where sequences are in parts
+constexpr int ROUND = 256;                    // of them that run side by side (not the launch's blocks: their number changes no bit)
+constexpr int PIECE = 3;                      // steps of a wavefront's walk over tiles that the start of a piece is counted as
 constexpr int MOST_ROWS = 32;                 // in two groups of sixteen
 constexpr int MOST_LAYERS = 128;
 constexpr int NOWHERE = 1 << 30;              // an offset behind the end of every buffer: reads of it are zero
@@ -63,19 +66,31 @@ struct LayerPack {
   Layer layer[LAYERS_A_LAUNCH];
 };
 
+struct ShareArgs {
+  const int* kv_lens;
+  int rows, kv_heads, parts_most, items_most;
+};
 struct Args {
   const Layer* layers;
   unsigned* control;
   char* exchange;
   float* residual;
   const float* table;
-  const int *block_table, *kv_lens;
+  const int* block_table;
   long per_layer;              // bytes of exchange
   int at_part, at_att, at_mid, at_mid_sums, at_hid, at_out, at_out_sums;
-  int count, rows, width, heads, kv_heads, group, inner, norm_f32, max_pos, table_width, page, page_bits, num_pages, splits, patience, limit;
+  int at_ml;
+  ShareArgs shares;
+  int count, rows, width, heads, kv_heads, group, inner, norm_f32, max_pos, table_width, page, page_bits, num_pages, patience, limit;
   float qk_eps, scale_log2;
 };
 
+// The step's attention as pieces: a sequence's keys for one key head, in `parts` parts. Sequence b's are FIRST and those behind it,
+// the parts of a key head side by side; those of sequences in many parts come first, and a block takes every so many-th.
+struct Shares {
+  int first[MOST_ROWS], parts[MOST_ROWS], kv_len[MOST_ROWS], tiles[MOST_ROWS];
+  int items, in_parts;
+};
 struct AttentionShared {
   float k[HEAD], v[HEAD];                     // the token's own, as the caches hold them
   __attribute__((aligned(16))) bf16_t q[16][HEAD + 8];
@@ -90,6 +105,7 @@ struct Shared {
   uint64_t first_at[THREADS][2];              // where a thread's first keys and values of the block's first item lie in each layer's caches
   float scale[MOST_ROWS];
   int rank, blocks;
+  Shares shares;
 };
 
 // Sixteen bytes, or eight, of memory through a pointer out of the launch's table (an access through a plain pointer is one to
@@ -152,7 +168,7 @@ struct Roles {
   int apart;                   // how many blocks the products into the stream have for themselves, or none
   __device__ __forceinline__ Roles(const Args& a, int blocks) : apart(4 * (a.width / 16) <= blocks ? a.width / 16 : 0) {}
   // a block's place among those that share product `which` out, and how many they are; its first item of the attention and its first pair of
-  // row and key head whose splits it joins
+  // row and key head whose parts it joins
   __device__ __forceinline__ int place(int which, int rank, int blocks) const {
     if (apart) return which & 1 ? rank - (blocks - apart) : rank;
     return !(which & 1) ? rank : rank >= blocks / 2 ? rank - blocks / 2 : rank + blocks - blocks / 2;
@@ -192,6 +208,45 @@ __device__ __forceinline__ int numbers_of(const Args& a, int rank, int blocks, i
     case OUT_WIDTH: return which == 0 ? qkv : which == 2 ? a.inner : a.width;
   }
   return 0;
+}
+
+// How the keys are shared out (one wavefront; every block comes to the same). A sequence gets as many parts as its tiles ask for where the
+// longest one has `s`, and s is the number for which the rounds of pieces cost least: per round a piece's start (PIECE steps of a wavefront's walk) and
+// the longest piece's steps, and half a step for every eight parts that have to be joined. It is their lengths that count, not the bound that a
+// captured step has for them, and not their number alone: 24 requests of the 0.6B shape of which one holds 30,000 keys and the others 500 took 9,700 us a
+// step with a part a sequence (2,738 kernel by kernel), and take 1,782; one of 8,000 3,153 (1,906), 1,279; sixteen with one of 8,000 1,898 (1,803), 1,012;
+// of the 8B shape eight with one of 30,000 5,768 (5,079), 3,737, sixteen 8,964 (5,645), 4,241. With a PIECE of 2 sixteen over 2,000 take 1,318 us
+// and not 1,286, with 6 the first of these 2,052.
+__device__ __forceinline__ int parts_of(int tiles, float per_tile, int s) { return min(max((int)ceilf((float)tiles * per_tile), 1), s); }
+__device__ __forceinline__ void share_out(const ShareArgs& a, Shares& sh, int lane) {
+  const bool row = lane < a.rows;
+  const int kv_len = row ? max(a.kv_lens[lane], 0) : 0, tiles = (max(kv_len - 1, 0) + FAST_TILE - 1) / FAST_TILE;
+  if (row) sh.tiles[lane] = tiles, sh.kv_len[lane] = kv_len;
+  const int longest = (int)wave_max((float)tiles);
+  int s = 1;
+  if (a.parts_most > 1 && longest > WAVES) {
+    const int tried = lane + 1;                     // (a lane tries a number)
+    const float per_tile = (float)tried / (float)longest;
+    int items = 0;
+    for (int r = 0; r < a.rows; ++r) items += parts_of(sh.tiles[r], per_tile, tried);
+    items *= a.kv_heads;
+    const int steps = (longest + WAVES * tried - 1) / (WAVES * tried), rounds = (items + ROUND - 1) / ROUND;
+    const int cost = 2 * rounds * (PIECE + steps) + (tried > 1 ? (tried + 7) / 8 : 0);
+    const bool fits = tried == 1 || (tried <= a.parts_most && items <= a.items_most && WAVES * (tried - 1) < longest);
+    int best = fits ? cost * 64 + 63 - tried : 0x7fffffff;          // (of equal ones the most parts: 8B shape, four over 2,060 keys 2,896 us, in five 2,961)
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) best = min(best, __shfl_xor(best, off, 64));
+    s = 63 - (best & 63);
+  }
+  const int parts = row ? parts_of(tiles, (float)s / (float)max(longest, 1), s) : 0;
+  int first = 0, all = 0;
+  for (int r = 0; r < a.rows; ++r) {
+    const int others = __shfl(parts, r, 64);
+    if (others > parts || (others == parts && r < lane)) first += others;
+    all += others;
+  }
+  if (row) sh.first[lane] = first * a.kv_heads, sh.parts[lane] = parts;
+  if (lane == 0) sh.items = all * a.kv_heads, sh.in_parts = s > 1;
 }
 
 typedef const __attribute__((address_space(4))) int* entries_ptr;
@@ -573,9 +628,9 @@ struct Block {
 
   // ---- attention ----
 
-  // A piece of the attention: a split of a sequence's keys for one key head, and what all layers have of it in common.
+  // A piece of the attention, and what all layers have of it in common.
   struct Item {
-    int split, g_kv, b, kv_len, there;
+    int n, part, parts, g_kv, b, kv_len, there;
     TilePages second;            // of this wavefront's second tile
     uint64_t keys, values;       // where the lane's parts of its first one lie
   };
@@ -610,17 +665,20 @@ struct Block {
   }
   __device__ __forceinline__ Item item_of(int n) const {
     Item it;
-    const int pair = n / a.splits;
-    it.split = n - pair * a.splits;
-    it.b = pair / a.kv_heads;
-    it.g_kv = pair - it.b * a.kv_heads;
-    it.kv_len = ((entries_ptr)(uintptr_t)a.kv_lens)[it.b];
-    const int first = it.split * WAVES + wave;
+    const int row = min(lane, a.rows - 1), from = sh.shares.first[row], parts = sh.shares.parts[row], kv_len = sh.shares.kv_len[row];
+    it.b = __builtin_ctzll(__builtin_amdgcn_ballot_w64(n >= from && n < from + parts * a.kv_heads));
+    it.n = n;
+    it.parts = __builtin_amdgcn_readlane(parts, it.b);
+    it.kv_len = __builtin_amdgcn_readlane(kv_len, it.b);
+    const int within = n - __builtin_amdgcn_readlane(from, it.b);
+    it.g_kv = within / it.parts;
+    it.part = within - it.g_kv * it.parts;
+    const int first = it.part * WAVES + wave;
     const TileAddr t = addr_of(pages_of(it.b, first), nullptr, nullptr, it.g_kv, first);
     it.there = t.there;
     it.keys = (uint64_t)t.k;
     it.values = (uint64_t)t.v;
-    it.second = pages_of(it.b, first + WAVES * a.splits);
+    it.second = pages_of(it.b, first + WAVES * it.parts);
     return it;
   }
 
@@ -632,11 +690,11 @@ struct Block {
     AttentionShared& s = sh.attention;
     const bf16_t *keys = (const bf16_t*)entry(layer, KEYS), *values = (const bf16_t*)entry(layer, VALUES);
     const char *q_norm = (const char*)entry(layer, Q_NORM), *k_norm = (const char*)entry(layer, K_NORM);
-    const int split = it.split, g_kv = it.g_kv, b = it.b;
+    const int g_kv = it.g_kv, b = it.b;
     const int lane = anew(this->lane), col = lane & 15, grp = lane >> 4;
     const int G = a.group, joined = (a.heads + 2 * a.kv_heads) * D;
-    const int first = split * WAVES + wave, step = WAVES * a.splits;
-    const bool brings_new = split == a.splits - 1;
+    const int first = it.part * WAVES + wave, step = WAVES * it.parts;
+    const bool brings_new = it.part == it.parts - 1;
     const int pos = it.kv_len - 1;                    // the token's own position; the cache is read up to the one before
     const bool turned = a.table != nullptr && pos >= 0 && pos < a.max_pos;
     const int kv_seen = max(pos, 0), row_pos = col < G ? pos - 1 : -1;
@@ -794,7 +852,7 @@ struct Block {
 #pragma unroll
         for (int e = 0; e < 4; ++e) o[e] += s.v[d + e] * weight;
       }
-      if (a.splits == 1) {
+      if (it.parts == 1) {
         const float inv = lr > 0.f ? 1.f / lr : lr;      // (a row that sees nothing, a sequence without a length, is zero)
         union {
           uint2 u;
@@ -804,14 +862,14 @@ struct Block {
         for (int e = 0; e < 4; ++e) pk.e[e] = (__bf16)(o[e] * inv);
         put8(ex, a.at_att + ((b * a.heads + g_kv * G + row) * D + d) * 2, pk.u);
       } else {
-        const int slot = ((b * a.kv_heads + g_kv) * a.splits + split) * G + row;
+        const int slot = it.n * G + row;
         u32x4_t p;
 #pragma unroll
         for (int e = 0; e < 4; ++e) p[e] = marked(__float_as_uint(o[e]), 0x7fc00000u);
         __builtin_amdgcn_raw_buffer_store_b128(p, ex, a.at_part + (slot * D + d) * 4, 0, THROUGH);
         if (d == 0) {
           const u32x2_t ml = {marked(__float_as_uint(mr), 0x7fc00000u), marked(__float_as_uint(lr), 0x7fc00000u)};
-          __builtin_amdgcn_raw_buffer_store_b64(ml, ex, a.at_part + (a.rows * a.heads * a.splits * D + slot * 2) * 4, 0, THROUGH);
+          __builtin_amdgcn_raw_buffer_store_b64(ml, ex, a.at_ml + slot * 8, 0, THROUGH);
         }
       }
     }
@@ -828,15 +886,15 @@ struct Block {
     meet();      // (whoever writes here next)
   }
 
-  // The splits of sequence `b` and key head `g_kv`, joined
-  __device__ __forceinline__ void merge(__amdgpu_buffer_rsrc_t ex, int g_kv, int b) {
+  // The parts of sequence `b` and key head `g_kv`, pieces `first` to `first` + `parts` - 1, joined
+  __device__ __forceinline__ void merge(__amdgpu_buffer_rsrc_t ex, int g_kv, int b, int first, int parts) {
     constexpr int D = HEAD, N = 8;
-    const int tid = anew(this->tid), G = a.group, all = a.rows * a.heads * a.splits * D;
+    const int tid = anew(this->tid), G = a.group;
     for (int idx = tid; idx < ((G * (D / 4) + 63) & ~63); idx += THREADS) {
       const int r = min(idx / (D / 4), G - 1), d = idx % (D / 4) * 4;
       float m = -INFINITY, sum = 0.f;
       f32x4_t o = {0.f, 0.f, 0.f, 0.f};
-      for (int s0 = 0; s0 < a.splits; s0 += N) {
+      for (int s0 = 0; s0 < parts; s0 += N) {
         u32x4_t p[N];
         u32x2_t ml[N];
         for (int n = 0;; ++n) {
@@ -844,9 +902,9 @@ struct Block {
           bool ok = true;
 #pragma unroll
           for (int s = 0; s < N; ++s) {
-            const int slot = ((b * a.kv_heads + g_kv) * a.splits + min(s0 + s, a.splits - 1)) * G + r;
+            const int slot = (first + min(s0 + s, parts - 1)) * G + r;
             p[s] = peek16(ex, a.at_part + (slot * D + d) * 4);
-            ml[s] = __builtin_amdgcn_raw_buffer_load_b64(ex, a.at_part + (all + slot * 2) * 4, 0, THROUGH);
+            ml[s] = __builtin_amdgcn_raw_buffer_load_b64(ex, a.at_ml + slot * 8, 0, THROUGH);
           }
 #pragma unroll
           for (int s = 0; s < N; ++s) ok = ok && there(p[s]) && ml[s].x != ABSENT && ml[s].y != ABSENT;
@@ -855,13 +913,13 @@ struct Block {
         float m_all = m;
 #pragma unroll
         for (int s = 0; s < N; ++s)
-          if (s0 + s < a.splits) m_all = fmaxf(m_all, __uint_as_float(ml[s].x));
+          if (s0 + s < parts) m_all = fmaxf(m_all, __uint_as_float(ml[s].x));
         const float kept = m > -INFINITY ? fast_exp2(m - m_all) : 0.f;
         sum *= kept;
         o *= kept;
 #pragma unroll
         for (int s = 0; s < N; ++s)
-          if (s0 + s < a.splits && __uint_as_float(ml[s].x) > -INFINITY) {
+          if (s0 + s < parts && __uint_as_float(ml[s].x) > -INFINITY) {
             const float weight = fast_exp2(__uint_as_float(ml[s].x) - m_all);
             sum += __uint_as_float(ml[s].y) * weight;
 #pragma unroll
@@ -881,13 +939,25 @@ struct Block {
   }
 
   __device__ __forceinline__ void layers() {
-    const int items = a.rows * a.kv_heads * a.splits, pairs = a.rows * a.kv_heads;
+    const int items = __builtin_amdgcn_readfirstlane(sh.shares.items), pairs = a.rows * a.kv_heads;
     const Roles roles(a, blocks);
     const int my_item = roles.item(rank, blocks), my_pair = roles.pair(rank, blocks), pair_step = blocks - roles.apart;
     Item mine = item_of(min(my_item, items - 1));
     sh.first_at[tid][0] = mine.keys;
     sh.first_at[tid][1] = mine.values;
-    const int my_b = my_pair / a.kv_heads, my_g = my_pair - my_b * a.kv_heads;
+    struct Pair {
+      int b, g, first, parts;
+    };
+    auto pair_of = [&](int n) {
+      Pair p;
+      p.b = n / a.kv_heads;
+      p.g = n - p.b * a.kv_heads;
+      const int row = min(p.b, a.rows - 1);
+      p.parts = __builtin_amdgcn_readfirstlane(sh.shares.parts[row]);
+      p.first = __builtin_amdgcn_readfirstlane(sh.shares.first[row]) + p.g * p.parts;
+      return p;
+    };
+    const Pair my = pair_of(my_pair);
     look_ahead(0, 0);
 #pragma unroll 1
     for (int n = 0; n < a.count; ++n) {
@@ -905,12 +975,11 @@ struct Block {
             if (n_item != my_item) it = item_of(n_item);
             attend(ex, n, it);
           }
-          if (a.splits > 1)      // (its loads would come behind the next weights')
+          if (a.shares.parts_most > 1)  // (its loads would come behind the next weights')
 #pragma unroll 1
             for (int pair = my_pair; pair < pairs; pair += pair_step) {
-              const bool first = pair == my_pair;
-              const int b = first ? my_b : pair / a.kv_heads, g = first ? my_g : pair - pair / a.kv_heads * a.kv_heads;
-              merge(ex, g, b);
+              const Pair p = pair == my_pair ? my : pair_of(pair);
+              if (p.parts > 1) merge(ex, p.g, p.b, p.first, p.parts);
             }
           look_ahead(n, 1);
         }
@@ -978,6 +1047,7 @@ template <typename QKW, int GROUPS, bool MANY>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void decode_layers_kernel(Args a) {
   __shared__ Shared sh;
   if (threadIdx.x == 0) gather(a, sh.rank, sh.blocks);
+  if (threadIdx.x >> 6 == 1) share_out(a.shares, sh.shares, threadIdx.x & 63);
   __syncthreads();
   const int rank = __builtin_amdgcn_readfirstlane(sh.rank), blocks = __builtin_amdgcn_readfirstlane(sh.blocks);
   if (blocks == 0) return;
@@ -989,24 +1059,52 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
   b.layers();
 }
 
-// The launch's table, its control words, an exchange without a word in it, and before its first layer's part the stream's rows as a
-// last product would leave them there.
+// The launch's table, its control words, an exchange without a word in it (a row of blocks fills a layer's), and before its first
+// layer's part the stream's rows as a last product would leave them there. What parts of sequences there are room for but none of, stays
+// as it is (24 rows of the 0.6B shape over 770 keys: 15 MB, 1,184 us a step and 1,169 without); where there are few a layer, asking how many
+// there are takes longer.
 struct Entry {
   const float* residual;
   const void* norm;
   int rows, width, norm_f32;
   char *out, *sums;
 };
-__global__ __launch_bounds__(256) void decode_layers_begin_kernel(LayerPack pack, int first, int count, Layer* layers, unsigned* control, uint4* exchange,
-                                                                  long pieces, Entry entry) {
-  if (blockIdx.x == 0) {
+struct Blank {
+  char* exchange;
+  long per_layer;
+  int at_part, at_ml, at_att, group;
+  ShareArgs shares;
+};
+constexpr int ITEMS_BLANKED = 256;
+__device__ __forceinline__ void blank(char* from, long bytes) {
+  const long each = (long)gridDim.x * 256;
+  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < bytes / 16; i += each)
+    reinterpret_cast<uint4*>(from)[i] = make_uint4(ABSENT, ABSENT, ABSENT, ABSENT);
+}
+__global__ __launch_bounds__(256) void decode_layers_begin_kernel(LayerPack pack, int first, int count, Layer* layers, unsigned* control, Blank to_blank,
+                                                                  Entry entry) {
+  if (blockIdx.x == 0 && blockIdx.y == 0) {
     const unsigned* from = reinterpret_cast<const unsigned*>(&pack);
     unsigned* to = reinterpret_cast<unsigned*>(layers + first);
     for (int i = threadIdx.x; i < count * (int)(sizeof(Layer) / 4); i += 256) to[i] = from[i];
     if (threadIdx.x < 2) control[threadIdx.x] = 0;
   }
-  const long each = (long)gridDim.x * 256, me = (long)blockIdx.x * 256 + threadIdx.x;
-  for (long i = me; i < pieces; i += each) exchange[i] = make_uint4(ABSENT, ABSENT, ABSENT, ABSENT);
+  if (to_blank.exchange) {
+    char* mine = to_blank.exchange + blockIdx.y * to_blank.per_layer;
+    if (to_blank.shares.items_most <= ITEMS_BLANKED) {
+      blank(mine, to_blank.per_layer);
+    } else {
+      __shared__ Shares shares;
+      if (threadIdx.x < 64) share_out(to_blank.shares, shares, threadIdx.x);
+      blank(mine, to_blank.at_part);
+      blank(mine + to_blank.at_att, to_blank.per_layer - to_blank.at_att);
+      __syncthreads();
+      const long rows = shares.in_parts ? (long)shares.items * to_blank.group : 0;
+      blank(mine + to_blank.at_part, rows * HEAD * 4);
+      blank(mine + to_blank.at_ml, (rows * 8 + 15) & ~15l);
+    }
+  }
+  const long each = (long)gridDim.x * gridDim.y * 256, me = ((long)blockIdx.y * gridDim.x + blockIdx.x) * 256 + threadIdx.x;
   for (long i = me; i < (long)entry.rows * entry.width / 4; i += each) {       // (sixteen columns are four neighbouring lanes')
     const float4 x = reinterpret_cast<const float4*>(entry.residual)[i];
     const int n = (int)(i * 4 % entry.width);
@@ -1030,15 +1128,23 @@ __global__ __launch_bounds__(256) void decode_layers_begin_kernel(LayerPack pack
   }
 }
 
+__global__ void decode_layers_shares_kernel(ShareArgs args, int* out) {
+  __shared__ Shares shares;
+  share_out(args, shares, threadIdx.x);
+  __syncthreads();
+  if ((int)threadIdx.x < args.rows) out[2 * threadIdx.x] = shares.first[threadIdx.x], out[2 * threadIdx.x + 1] = shares.parts[threadIdx.x];
+}
+
 inline long up(long n) { return (n + 255) & ~255l; }
 
 struct Layout {
-  long part, att, mid, mid_sums, hid, out, out_sums, size;
+  long part, ml, att, mid, mid_sums, hid, out, out_sums, size;
 };
-inline Layout layout_of(long rows, long width, long heads, long kv_heads, long inner, long splits) {
+inline Layout layout_of(long rows, long width, long heads, long kv_heads, long inner, long items) {
   Layout l;
   l.part = up(rows * (heads + 2 * kv_heads) * HEAD * 2);
-  l.att = l.part + (splits > 1 ? up(rows * heads * splits * (HEAD + 2) * 4) : 0);
+  l.ml = l.part + items * (heads / kv_heads) * HEAD * 4;
+  l.att = l.ml + up(items * (heads / kv_heads) * 8);
   l.mid = l.att + up(rows * heads * HEAD * 2);
   l.mid_sums = l.mid + up(rows * width * 2);
   l.hid = l.mid_sums + up(rows * (width / 16) * 4);
@@ -1046,6 +1152,13 @@ inline Layout layout_of(long rows, long width, long heads, long kv_heads, long i
   l.out_sums = l.out + up(rows * width * 2);
   l.size = l.out_sums + up(rows * (width / 16) * 4);
   return l;
+}
+
+// Into how many parts a sequence may go, up to `parts`, and how many pieces that are in parts there may be
+inline int parts_taken(long pairs, int parts) { return pairs < ITEMS_MOST ? parts : 1; }
+inline long items_taken(long pairs, int parts) {
+  if (parts_taken(pairs, parts) == 1) return 0;
+  return pairs * parts < ITEMS_MOST ? pairs * parts : ITEMS_MOST;
 }
 
 // Every wavefront of a block has a step of 32 of each product's K at least: the smallest K is 256, from two heads on. More than sixteen
@@ -1063,23 +1176,32 @@ extern "C" {
 
 // Bytes of workspace for a step of `rows` single tokens over `count` layers: the layers' table, the control words, the exchange;
 // 0 for sizes that are not taken.
-long q3_decode_layers_workspace(int count, int rows, int width, int heads, int kv_heads, int dim, int inner, int splits) {
-  if (count < 1 || count > MOST_LAYERS || !sizes_fit(rows, width, heads, kv_heads, dim, inner) || splits < 1 || splits > MOST_SPLITS) return 0;
-  const Layout l = layout_of(rows, width, heads, kv_heads, inner, splits);
+long q3_decode_layers_workspace(int count, int rows, int width, int heads, int kv_heads, int dim, int inner, int parts) {
+  if (count < 1 || count > MOST_LAYERS || !sizes_fit(rows, width, heads, kv_heads, dim, inner) || parts < 1 || parts > MOST_PARTS) return 0;
+  const Layout l = layout_of(rows, width, heads, kv_heads, inner, items_taken((long)rows * kv_heads, parts));
   if (l.size > (1l << 30)) return 0;
   return up((long)count * sizeof(Layer)) + 256 + (count + 1) * l.size;
 }
 
+// How a step of `rows` sequences shares out their keys: per row its first piece and its parts, `out` (rows, 2).
+int q3_decode_layers_shares(const int* kv_lens, int rows, int kv_heads, int parts, int* out, hipStream_t stream) {
+  if (!kv_lens || !out || rows < 1 || rows > MOST_ROWS || kv_heads < 1 || kv_heads > 512 || parts < 1 || parts > MOST_PARTS) return Q3_ERR_BAD_ARGUMENT;
+  const long pairs = (long)rows * kv_heads;
+  const ShareArgs shares{kv_lens, rows, kv_heads, parts_taken(pairs, parts), (int)items_taken(pairs, parts)};
+  hipLaunchKernelGGL(decode_layers_shares_kernel, dim3(1), dim3(64), 0, stream, shares, out);
+  return q3_launch_status();
+}
+
 // Row b is the one token of sequence b, at position kv_lens[b] - 1, whose key and value are written to the caches; `residual` (rows,
-// width) float32 is the stream, which the layers add to in place. `blocks`: of the launch (0: one per processor); `patience`, `limit`: looks
+// width) float32 is the stream, which the layers add to in place. `parts`: of a sequence's keys, at most. `blocks`: of the launch (0: one per processor); `patience`, `limit`: looks
 // before the launch goes on with the blocks it has, and before a wait gives up.
 int q3_decode_layers(const Layer* layers, int count, float* residual, int rows, int width, int heads, int kv_heads, int dim, int inner,
                      int norm_dtype, int qk_dtype, float qk_eps, float scale, const float* table, int rotary_dim, int max_pos,
-                     const int* block_table, int table_width, const int* kv_lens, int max_kv_len, int page, int num_pages, int splits,
+                     const int* block_table, int table_width, const int* kv_lens, int max_kv_len, int page, int num_pages, int parts,
                      void* workspace, int blocks, int patience, int limit, hipStream_t stream) {
   if (!layers || !residual || !block_table || !kv_lens || !workspace || count < 1 || count > MOST_LAYERS || page < 16 || (page & (page - 1)) || num_pages < 1)
     return Q3_ERR_BAD_ARGUMENT;
-  if (!sizes_fit(rows, width, heads, kv_heads, dim, inner) || splits < 1 || splits > MOST_SPLITS || (table && rotary_dim != dim))
+  if (!sizes_fit(rows, width, heads, kv_heads, dim, inner) || parts < 1 || parts > MOST_PARTS || (table && rotary_dim != dim))
     return Q3_ERR_UNSUPPORTED;
   if ((table && max_kv_len > max_pos) || (long)table_width * page < max_kv_len || max_kv_len < 1 || patience < 1 || limit < 1 || blocks < 0)
     return Q3_ERR_BAD_ARGUMENT;
@@ -1096,21 +1218,24 @@ int q3_decode_layers(const Layer* layers, int count, float* residual, int rows, 
     if (status == hipSuccess) status = hipDeviceGetAttribute(&blocks, hipDeviceAttributeMultiprocessorCount, device);
     if (status != hipSuccess) return (int)status;
   }
-  const Layout l = layout_of(rows, width, heads, kv_heads, inner, splits);
+  const long items = items_taken((long)rows * kv_heads, parts);
+  const Layout l = layout_of(rows, width, heads, kv_heads, inner, items);
   if (l.size > (1l << 30)) return Q3_ERR_UNSUPPORTED;
   Layer* held = (Layer*)workspace;
   unsigned* control = (unsigned*)((char*)workspace + up((long)count * sizeof(Layer)));
   char *entry_part = (char*)control + 256, *exchange = entry_part + l.size;
-  const long pieces = count * l.size / 16;
+  const ShareArgs shares{kv_lens, rows, kv_heads, parts_taken((long)rows * kv_heads, parts), (int)items};
+  const Blank to_blank{exchange, l.size, (int)l.part, (int)l.ml, (int)l.att, heads / kv_heads, shares};
   const Entry entry{residual, layers[0].entry_norm, rows, width, norm_dtype == Q3_F32, entry_part + l.out, entry_part + l.out_sums};
   for (int first = 0; first < count; first += LAYERS_A_LAUNCH) {
     const int n = count - first < LAYERS_A_LAUNCH ? count - first : LAYERS_A_LAUNCH;
     LayerPack pack{};
     for (int i = 0; i < n; ++i) pack.layer[i] = layers[first + i];
-    const long share = first == 0 ? pieces : 0;
-    const long wanted = (share + 2047) / 2048;
-    hipLaunchKernelGGL(decode_layers_begin_kernel, dim3((unsigned)(wanted < 1 ? 1 : wanted > 1024 ? 1024 : wanted)), dim3(256), 0, stream, pack, first, n,
-                       held, control, (uint4*)exchange, share, first == 0 ? entry : Entry{});
+    // (eight pieces of sixteen bytes a thread)
+    const long wanted = (l.size + 16 * 2048 - 1) / (16 * 2048);
+    const dim3 grid = first == 0 ? dim3((unsigned)(wanted > 32 ? 32 : wanted), (unsigned)count) : dim3(1);
+    hipLaunchKernelGGL(decode_layers_begin_kernel, grid, dim3(256), 0, stream, pack, first, n, held, control, first == 0 ? to_blank : Blank{},
+                       first == 0 ? entry : Entry{});
   }
   Args a{};
   a.layers = held;
@@ -1119,13 +1244,13 @@ int q3_decode_layers(const Layer* layers, int count, float* residual, int rows, 
   a.residual = residual;
   a.table = table;
   a.block_table = block_table;
-  a.kv_lens = kv_lens;
   a.per_layer = l.size;
-  a.at_part = (int)l.part, a.at_att = (int)l.att, a.at_mid = (int)l.mid, a.at_mid_sums = (int)l.mid_sums, a.at_hid = (int)l.hid;
+  a.at_part = (int)l.part, a.at_ml = (int)l.ml, a.shares = shares;
+  a.at_att = (int)l.att, a.at_mid = (int)l.mid, a.at_mid_sums = (int)l.mid_sums, a.at_hid = (int)l.hid;
   a.at_out = (int)l.out, a.at_out_sums = (int)l.out_sums;
   a.count = count, a.rows = rows, a.width = width, a.heads = heads, a.kv_heads = kv_heads, a.group = heads / kv_heads, a.inner = inner;
   a.norm_f32 = norm_dtype == Q3_F32;
-  a.max_pos = max_pos, a.table_width = table_width, a.page = page, a.page_bits = __builtin_ctz(page), a.num_pages = num_pages, a.splits = splits;
+  a.max_pos = max_pos, a.table_width = table_width, a.page = page, a.page_bits = __builtin_ctz(page), a.num_pages = num_pages;
   a.patience = patience, a.limit = limit;
   a.qk_eps = qk_eps;
   a.scale_log2 = make_score_scale(scale);

@@ -225,11 +225,21 @@ class DecodeLayers:
         found = cls(layers, heads, kv_heads, dim, width, inner, qk_eps, scale)
         return found if found._workspace(1, 1, width, heads, kv_heads, dim, inner, 1) > 0 else None
 
-    def splits(self, rows, max_kv_len):
-        """Into how many blocks a sequence's keys are shared out: as many as leave each wavefront a tile of 32 keys, while there is a
-        block for each share."""
-        tiles = -(-int(max_kv_len) // 32)
-        return max(1, min(256 // (rows * self.kv_heads), -(-tiles // 8), 32))
+    def parts(self, max_kv_len):
+        """Into how many parts, at most, a sequence's keys are shared out over blocks: as many as leave each wavefront a tile of 32 keys.
+        How many it is, the launch finds from the lengths themselves."""
+        return max(1, min(-(-int(max_kv_len) // 256), 32))
+
+    def shares(self, kv_lens, max_kv_len):
+        """How a step over these lengths (int32, on the GPU) shares out their keys: int32 (rows, 2), a row's first piece and its parts."""
+        rows = kv_lens.shape[0]
+        if not (kv_lens.is_cuda and kv_lens.dtype == torch.int32 and kv_lens.dim() == 1 and kv_lens.is_contiguous()
+                and 1 <= rows <= DECODE_ROWS_MOST):
+            raise OperandError("kv_lens int32, of 1 to %d rows" % DECODE_ROWS_MOST)
+        out = torch.empty((rows, 2), dtype=torch.int32, device=kv_lens.device)
+        _check(library("decode_layers").q3_decode_layers_shares(
+            _P(kv_lens.data_ptr()), rows, self.kv_heads, self.parts(max_kv_len), _P(out.data_ptr()), _stream()), "the shares of a step's keys")
+        return out
 
     def run(self, stream, caches, block_table, kv_lens, max_kv_len, table, blocks=0, patience=64):
         """The layers over the residual `stream` (T, width) float32, in place: row b is sequence b's one token, at position
@@ -266,8 +276,8 @@ class DecodeLayers:
             max_pos = table.shape[0]
         if any(t.data_ptr() % 16 for t in (stream, *(table,) * (table is not None), *(t for pair in caches for t in pair))):
             return False
-        splits = self.splits(T, max_kv_len)
-        size = self._workspace(count, T, self.width, H, G, D, self.inner, splits)
+        parts = self.parts(max_kv_len)
+        size = self._workspace(count, T, self.width, H, G, D, self.inner, parts)
         if size <= 0:
             return False
         workspace = torch.empty(size, dtype=torch.uint8, device=stream.device)
@@ -286,6 +296,6 @@ class DecodeLayers:
         _check(library("decode_layers").q3_decode_layers(
             layers, count, _P(at(stream)), T, self.width, H, G, D, self.inner, _DT[self.norm_dtype], _DT[self.qk_dtype],
             _F(self.qk_eps), _F(self.scale), _P(at(table)), D if table is not None else 0, max_pos, _P(at(block_table)),
-            block_table.shape[1], _P(at(kv_lens)), int(max_kv_len), page, pages, splits, _P(at(workspace)), int(blocks), int(patience),
+            block_table.shape[1], _P(at(kv_lens)), int(max_kv_len), page, pages, parts, _P(at(workspace)), int(blocks), int(patience),
             1 << 18, _stream()), "the layers of a step of single tokens")
         return True

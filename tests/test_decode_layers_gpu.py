@@ -96,3 +96,88 @@ def test_what_is_not_taken():
     sizes = dict(heads=16, kv_heads=8, dim=128, width=1024, inner=2048, qk_eps=1e-6, scale=1.0)
     assert type(native).of([native.layers[0]], window=0, **sizes) is not None
     assert type(native).of([native.layers[0]], window=8, **sizes) is None and type(native).of([layer], window=0, **sizes) is None
+
+
+def _layer(heads, kv_heads, inner=256):
+    """A layer whose product into the stream passes the attention on as it is and whose other weights are zeros: every key weighs the same."""
+    from qwen3_from_scratch_amd import ops
+    from qwen3_from_scratch_amd.ops.layers import DecodeLayers
+
+    width = heads * 128
+    layer = dict(q_norm=None, k_norm=None, entry_norm=torch.ones(width, device="cuda"), middle_norm=torch.ones(width, device="cuda"),
+                 entry_eps=1e-6, middle_eps=1e-6)
+    for name, shape in (("qkv", ((heads + 2 * kv_heads) * 128, width)), ("out", None), ("gate_up", (2 * inner, width)), ("down", (width, inner))):
+        layer[name] = (torch.eye(width, device="cuda") if shape is None else torch.zeros(shape, device="cuda")).to(torch.bfloat16)
+        layer[name + "_tiles"] = ops.tile_weight(layer[name])
+    native = DecodeLayers.of([layer], heads, kv_heads, 128, width, inner, 1e-6, 128 ** -0.5, 0)
+    assert native is not None
+    return native
+
+
+def _marked_caches(lengths, kv_heads, page, absent=()):
+    """Caches where the keys of tile t (of 32) have a one in place t % 128 of their value and zeros elsewhere, in pages in no order, those of the table entries
+    `absent` (row, entry) missing; what lies behind a sequence's end is not a number. And what every row's attention over them is."""
+    g = torch.Generator().manual_seed(7)
+    entries = [-(-n // page) for n in lengths]
+    order = torch.randperm(sum(entries), generator=g).tolist()
+    keys = torch.full((len(order), kv_heads, page, 128), float("nan"), dtype=torch.bfloat16)
+    values = torch.full((len(order), kv_heads, 128, page), float("nan"), dtype=torch.bfloat16)
+    table = torch.full((len(lengths), max(entries)), -1, dtype=torch.int32)
+    want = torch.zeros(len(lengths), 128, dtype=torch.float64)
+    for b, n in enumerate(lengths):
+        for e in range(entries[b]):
+            at = order.pop()
+            held = min(n - 1 - e * page, page)            # (the last token comes with the step)
+            if held > 0:
+                keys[at, :, :held] = 0
+                values[at, :, :, :held] = 0
+                for slot in range(held):
+                    values[at, :, (e * page + slot) // 32 % 128, slot] = 1
+            if (b, e) in absent:
+                continue
+            table[b, e] = at
+            for slot in range(max(held, 0)):
+                want[b, (e * page + slot) // 32 % 128] += 1 / n
+    return keys.cuda(), values.cuda(), table.cuda(), want
+
+
+# contexts all alike and one long one among short ones: whole, in as many parts as there are blocks, in two rounds of pieces; rows that bring
+# their first token; many key heads and one
+UNEVEN = [([1], 8, 8), ([2050], 8, 8), ([1, 4100], 8, 2), ([3000, 31, 33, 64, 1], 8, 1), ([9000] + [40] * 5, 8, 8), ([600] * 8, 16, 16),
+          ([50, 700, 5] * 4 + [6000], 16, 16), ([500] * 15 + [8000], 8, 8), ([30 + i for i in range(23)] + [9000], 8, 8), ([257] * 32, 8, 8),
+          ([9000] * 2 + [300] * 30, 8, 4), ([2100 - 130 * i for i in range(16)], 32, 32)]
+
+
+@pytest.mark.parametrize("lengths,heads,kv_heads", UNEVEN)
+def test_every_key_counts_once(lengths, heads, kv_heads):
+    native = _layer(heads, kv_heads)
+    keys, values, table, want = _marked_caches(lengths, kv_heads, 16)
+    lens = torch.tensor(lengths, dtype=torch.int32, device="cuda")
+    stream = torch.zeros(len(lengths), heads * 128, device="cuda")
+    assert native.run(stream, [(keys, values)], table, lens, max(lengths), None)
+    got = stream.view(len(lengths), heads, 128).double().cpu()
+    # ones and whole sums are exact, the quotient is rounded to bfloat16; a key more or less is 1 / 32 of a place that one tile has
+    assert ((got - want[:, None]).abs() <= 2 ** -8 * want[:, None] + 1e-30).all()
+    for b, n in enumerate(lengths):                          # the token's own key and value: zeros, where nothing was
+        at, slot = int(table[b, (n - 1) // 16]), (n - 1) % 16
+        assert not keys[at, :, slot].any() and not values[at, :, :, slot].any()
+
+
+def test_uneven_keys_go_over_many_blocks():
+    """A long sequence among short ones is in as many parts at least as attention of its own kernel would cut it into, pieces are numbered one
+    behind the other, and where there are several a sequence, no more of them than the exchange has room for."""
+    from qwen3_from_scratch_amd import ops
+
+    native = _layer(8, 8)
+    for rows in (1, 6, 8, 12, 16, 24, 32):
+        for long in (2000, 8000, 30000):
+            lens = torch.full((rows,), 500, dtype=torch.int32, device="cuda")
+            lens[rows // 2] = long
+            shares = native.shares(lens, long).cpu()
+            assert shares[rows // 2, 1] >= (ops._splits(rows, 8, long) if long > 2000 else 1)
+            order = shares[:, 0].argsort()
+            assert shares[order[0], 0] == 0 and (shares[order][1:, 0] == (shares[order][:-1, 0] + 8 * shares[order][:-1, 1])).all()
+            items = 8 * int(shares[:, 1].sum())
+            assert items <= 512 and (shares[:, 1] <= 32).all()
+            alike = native.shares(torch.full_like(lens, long), long).cpu()
+            assert (alike[:, 1] == alike[0, 1]).all() and (alike[0, 1] == 1 or 8 * rows * int(alike[0, 1]) <= 512)
