@@ -1,5 +1,5 @@
 // All decoder layers of a step of single tokens in one launch: pre-norm layers of softmax attention with grouped heads of 128 and a
-// gated unit, bfloat16, up to 16 rows, or 32 of a small model. What gemm.hip's few-row products and attention.hip's decoding attention do layer by layer.
+// gated unit, bfloat16, up to 16 rows, 32 of a small model, or 3 to 8 of a wide one. What gemm.hip's few-row products and attention.hip's decoding attention do layer by layer.
 //
 // A kernel that waits for its predecessor costs 2 us inside a graph if it does nothing and 4 to 4.5 if it loads, reduces and stores a
 // row, and a step of the 0.6B shape was 145 of them: 1,011 us where its bytes take 240. Here a block per compute unit stays for all
@@ -1161,13 +1161,28 @@ inline long items_taken(long pairs, int parts) {
   return pairs * parts < ITEMS_MOST ? pairs * parts : ITEMS_MOST;
 }
 
-// Every wavefront of a block has a step of 32 of each product's K at least: the smallest K is 256, from two heads on. More than sixteen
-// rows of a wide model do not stay in registers from slab to slab and are asked for with each: 24 rows of the 8B shape over 2,060 keys
-// 5,964 us, 5,024 kernel by kernel, 20 over 1,000 5,229 and 4,327; of the 0.6B shape 17 over 100 947 and 1,149, 32 over 2,000 2,127 and 2,377.
+// Up to how many rows this launch is the faster way (what is slower it does not take). Rows of more than 4,096 numbers, of two groups of
+// sixteen more than 2,048, do not stay in registers from slab to slab and are asked for with each, rows / 16 of what its weights
+// are; a width of that size is where a block has many slabs. The kernels one by one / this, us a step:
+// - two groups, up to a width of 1,024: the 0.6B shape 17 rows over 100 keys 1,149 / 947, 32 over 2,000 2,377 / 2,127; an inner size of 8,192
+//   (16 layers) 17 over 100 785 / 743, 24 over 1,000 1,014 / 957, 32 over 300 899 / 928; 16,384 17 over 300 1,043 / 1,186, 32 1,103 / 1,382;
+//   the 8B shape 20 over 1,000 4,327 / 5,229;
+// - one group, up to 4,096: 12 shapes from 512 to 4,096 wide, inner sizes to 18,944, 1 to 16 rows over 300 to 8,000 keys, all the faster
+//   here, by 10 (the 8B shape, sixteen over 8,000) to 80 percent;
+// - wider ones by how evenly the blocks have the slabs of the products into the stream. A last round half full or more: 6,144
+//   (8 layers), one row 1,392 / 1,220, 8 1,541 / 1,501, 16 1,860 / 1,945; 8,192 (6 layers), one 1,954 / 1,783, 8 2,101 / 2,026, 16 2,373 / 2,441.
+//   Less than that: 5,120 with an inner size of 17,408 (12 layers), 3 rows 2,007 / 1,987, 4 1,988 / 1,995, 5 2,105 / 2,164, 16 2,584 / 2,766; with
+//   25,600 (10 layers) 3 rows 2,297 / 2,230, 5 2,395 / 2,411, 16 2,951 / 3,120; 4,608, 3 rows 1,052 / 1,028, 6 1,089 / 1,118.
+inline int rows_most(int width, int heads, int inner) {
+  if (width > 4096) return width / 16 % 256 == 0 || width / 16 % 256 >= 128 ? 8 : 3;
+  const int longest = inner > heads * HEAD ? inner : heads * HEAD;
+  return width > 1024 || longest > 8192 ? 16 : longest > 4096 ? 24 : MOST_ROWS;
+}
+// Every wavefront of a block has a step of 32 of each product's K at least: the smallest K is 256, from two heads on.
 inline bool sizes_fit(int rows, int width, int heads, int kv_heads, int dim, int inner) {
-  return rows >= 1 && rows <= (width <= 1024 ? MOST_ROWS : 16) && dim == HEAD && heads >= 1 && kv_heads >= 1 && heads % kv_heads == 0 && heads / kv_heads <= 16 &&
+  return rows >= 1 && dim == HEAD && heads >= 1 && kv_heads >= 1 && heads % kv_heads == 0 && heads / kv_heads <= 16 &&
          width >= 32 * WAVES && width % 128 == 0 && inner >= 32 * WAVES && inner % 128 == 0 && heads * HEAD >= 32 * WAVES &&
-         width <= (1 << 16) && inner <= (1 << 18) && heads <= 512;
+         width <= (1 << 16) && inner <= (1 << 18) && heads <= 512 && rows <= rows_most(width, heads, inner);
 }
 
 }  // namespace

@@ -71,7 +71,7 @@ class DecodeRun:
 
     def forward(self, x, batch, cache):
         """The layers over the stream x, in place, if the step is one of single tokens that the launch takes; whether it was.
-        (What it takes it is the faster way for at every size measured: csrc/decode_layers.hip.)"""
+        (It takes the rows, widths and inner sizes for which it was measured to be the faster way: csrc/decode_layers.hip, `rows_most`.)"""
         if batch.max_q_len != 1 or not 1 <= x.shape[0] <= DECODE_ROWS_MOST or batch.kv_lens.shape[0] != x.shape[0]:
             return False
         if not hasattr(cache, "pages_of"):

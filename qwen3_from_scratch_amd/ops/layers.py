@@ -179,7 +179,7 @@ class DecoderLayers:
         return out, exit_
 
 
-DECODE_ROWS_MOST = 32          # rows of a step of single tokens that `DecodeLayers` takes (of wider models than 1,024: 16)
+DECODE_ROWS_MOST = 32          # rows of a step of single tokens that `DecodeLayers` takes (of wider models than 1,024: 16, and of very wide ones fewer)
 
 
 class _DecodeLayer(ctypes.Structure):
@@ -255,6 +255,10 @@ class DecodeLayers:
         count = len(self.layers)
         if len(caches) != count:
             raise OperandError("a cache for each of the layers")
+        parts = self.parts(max_kv_len)
+        size = self._workspace(count, T, self.width, H, G, D, self.inner, parts)
+        if size <= 0:
+            return False
         if not (stream.is_cuda and stream.shape == (T, self.width) and stream.dtype == torch.float32 and stream.is_contiguous()):
             raise OperandError("a float32 stream (T, width), contiguous")
         if not (kv_lens.is_cuda and kv_lens.dtype == torch.int32 and kv_lens.shape == (T,) and kv_lens.is_contiguous()):
@@ -275,10 +279,6 @@ class DecodeLayers:
                 raise OperandError("table must be float32 (P, D) and hold the step's last position")
             max_pos = table.shape[0]
         if any(t.data_ptr() % 16 for t in (stream, *(table,) * (table is not None), *(t for pair in caches for t in pair))):
-            return False
-        parts = self.parts(max_kv_len)
-        size = self._workspace(count, T, self.width, H, G, D, self.inner, parts)
-        if size <= 0:
             return False
         workspace = torch.empty(size, dtype=torch.uint8, device=stream.device)
         layers = (_DecodeLayer * count)()

@@ -1,5 +1,7 @@
 """All layers of a step of single tokens in one launch against the same layers run part by part."""
 
+import ctypes
+
 import pytest
 import torch
 
@@ -181,3 +183,15 @@ def test_uneven_keys_go_over_many_blocks():
             assert items <= 512 and (shares[:, 1] <= 32).all()
             alike = native.shares(torch.full_like(lens, long), long).cpu()
             assert (alike[:, 1] == alike[0, 1]).all() and (alike[0, 1] == 1 or 8 * rows * int(alike[0, 1]) <= 512)
+
+
+@pytest.mark.parametrize("width,heads,inner,rows", [(1024, 16, 4096, 32), (1024, 16, 8192, 24), (1024, 33, 4096, 24), (1024, 16, 8320, 16), (1152, 9, 3072, 16),
+                                                    (4096, 32, 25600, 16), (4608, 36, 14336, 3), (5120, 40, 17408, 3), (5120, 64, 25600, 3),
+                                                    (6144, 48, 16384, 8), (8192, 64, 28672, 8)])
+def test_rows_that_other_kernels_are_faster_for(width, heads, inner, rows):
+    from qwen3_from_scratch_amd.ops import library
+
+    lib = library("decode_layers")
+    lib.q3_decode_layers_workspace.restype = ctypes.c_long
+    taken = [n for n in range(1, 40) if lib.q3_decode_layers_workspace(4, n, width, heads, heads, 128, inner, 2) > 0]
+    assert taken == list(range(1, rows + 1))
