@@ -45,6 +45,7 @@ constexpr int RESULTS = 128;                  // of them times rows, at most
 constexpr int CHUNKS = 16;                    // steps of K, times groups of sixteen rows, that a wavefront has in registers
 constexpr unsigned ABSENT = 0xffffffffu;      // a word of the exchange that nobody has written yet
 constexpr unsigned CLOSED = 0x80000000u;
+enum { CAME, CLOSED_AT, GAVE_UP, CONTROL_WORDS };
 constexpr int THROUGH = 16;                   // cache policy of what blocks exchange: past the chiplets' own caches (sc1)
 constexpr int MOST_PARTS = 32;                // of a sequence's keys
 constexpr int ITEMS_MOST = 512;               // pieces of attention, where sequences are in parts
@@ -52,6 +53,7 @@ constexpr int ROUND = 256;                    // of them that run side by side (
 constexpr int PIECE = 3;                      // steps of a wavefront's walk over tiles that the start of a piece is counted as
 constexpr int MOST_ROWS = 32;                 // in two groups of sixteen
 constexpr int MOST_LAYERS = 128;
+constexpr int CLOSING = 1 << 18;               // looks for how many blocks there are, once their number is closed
 constexpr int NOWHERE = 1 << 30;              // an offset behind the end of every buffer: reads of it are zero
 
 // One layer as the host gives it and as the launch's table holds it.
@@ -104,7 +106,7 @@ struct Shared {
   __attribute__((aligned(16))) uint64_t layers[MOST_LAYERS * sizeof(Layer) / 8];
   uint64_t first_at[THREADS][2];              // where a thread's first keys and values of the block's first item lie in each layer's caches
   float scale[MOST_ROWS];
-  int rank, blocks;
+  int rank, blocks, gave_up;
   Shares shares;
 };
 
@@ -253,6 +255,13 @@ typedef const __attribute__((address_space(4))) int* entries_ptr;
 constexpr int LAYER_WORDS = sizeof(Layer) / 8;
 enum { Q_NORM = 4, K_NORM, ENTRY_NORM, MIDDLE_NORM, KEYS, VALUES, EPS };    // words of an entry behind its four matrices
 
+// A wait has been given up: nobody's result stands (`Block::layers`, at its end).
+__device__ __forceinline__ void gave_up(const Args& a) {
+  __hip_atomic_store(a.control + GAVE_UP, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __builtin_amdgcn_s_waitcnt(0);
+  compiler_fence();
+}
+
 template <typename QKW, int GROUPS, bool MANY>
 struct Block {
   Shared& sh;
@@ -273,9 +282,14 @@ struct Block {
     asm volatile("" : "+v"(v));
     return v;
   }
-  // Between two looks at the exchange: whether to look again. Every wait ends: after so many looks nothing is waited for any more.
+  // Between two looks at the exchange: whether to look again. Every wait ends: after so many looks this wavefront waits for nothing
+  // any more. That is in the control words before anything that it passes on afterwards (and in shared memory, for its own block's token).
   __device__ __forceinline__ bool again(int n) {
-    if (n >= most) alive = 0;
+    if (n >= most) {
+      alive = 0;
+      gave_up(a);
+      sh.gave_up = 1;
+    }
     alive = __builtin_amdgcn_readfirstlane(alive);
     return alive != 0;
   }
@@ -873,7 +887,7 @@ struct Block {
         }
       }
     }
-    if (brings_new && pos >= 0 && tid >= THREADS - 2 * HEAD) {       // the token's key and value into the caches, for later steps
+    if (brings_new && pos >= 0 && tid >= THREADS - 2 * HEAD && !sh.gave_up) {       // the token's key and value into the caches, for later steps
       const int d = tid & (HEAD - 1), blk = pos >> a.page_bits, at = pos & (a.page - 1);
       const int pg = blk < a.table_width ? ((entries_ptr)(uintptr_t)(a.block_table + (size_t)b * a.table_width))[blk] : -1;
       if (pg >= 0 && pg < a.num_pages) {
@@ -1001,19 +1015,25 @@ struct Block {
         product_of(r, ex, n, which, count, norm);
       }
     }
-    if (!alive) {              // a wait that did not end: no number of the result stands
-      for (int done = 0; done < number(3, COUNT); ++done)
-        for (int idx = tid; idx < 16 * a.rows; idx += THREADS)
-          a.residual[(size_t)(idx >> 4) * a.width + (number(3, SLAB) + done * number(3, STEP)) * 16 + (idx & 15)] = __uint_as_float(0x7fc00000u);
+    // A wait that was given up, in whatever block: no number of the result stands. Every block with a part in the last product has multiplied with
+    // numbers that come, over however many blocks, from each of those that had work before it, and these say that they gave up
+    // before they pass anything on. (A thread stores what `finish` had it store.)
+    const int count = number(3, COUNT);
+    if (count && __hip_atomic_load(a.control + GAVE_UP, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+      const unsigned nan = 0x7fc00000u;
+      for (int done = 0; done < count; done += pass) {
+        const int q = tid >> 2, s = over_rows(q), row = q - s * a.rows, n = (number(3, SLAB) + (done + s) * number(3, STEP)) * 16 + 4 * (tid & 3);
+        if (s < min(pass, count - done)) store16(a.residual + (size_t)row * a.width + n, u32x4_t{nan, nan, nan, nan});
+      }
     }
   }
 };
 
 // The blocks that are here when the launch begins share its work; one that only finds room later has none. Nothing is assumed
 // about how many run at once, so two such launches on two streams, or a kernel that keeps some of the processors, cannot wait
-// for each other without end. control[0]: how many have come, and CLOSED; control[1]: how many there are, if not all came in time.
+// for each other without end. CAME: how many have come, and CLOSED; CLOSED_AT: how many there are, if not all came in time.
 __device__ __forceinline__ void gather(const Args& a, int& rank, int& blocks) {
-  unsigned* came = a.control;
+  unsigned* came = a.control + CAME;
   const unsigned ticket = __hip_atomic_fetch_add(came, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   rank = blocks = 0;
   if (ticket & CLOSED) return;
@@ -1027,17 +1047,20 @@ __device__ __forceinline__ void gather(const Args& a, int& rank, int& blocks) {
     if (!(now & CLOSED) && n >= a.patience) {
       const unsigned seen = now;
       if (__hip_atomic_compare_exchange_strong(came, &now, seen | CLOSED, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-        __hip_atomic_store(came + 1, seen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(a.control + CLOSED_AT, seen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       continue;
     }
     if (now & CLOSED) {
-      const unsigned closed_at = __hip_atomic_load(came + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const unsigned closed_at = __hip_atomic_load(a.control + CLOSED_AT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (closed_at) {
         rank = ticket;
         blocks = closed_at;
         return;
       }
-      if (n >= a.patience + a.limit) return;
+      if (n >= a.patience + CLOSING) {
+        gave_up(a);
+        return;
+      }
     }
     __builtin_amdgcn_s_sleep(2);
   }
@@ -1046,7 +1069,10 @@ __device__ __forceinline__ void gather(const Args& a, int& rank, int& blocks) {
 template <typename QKW, int GROUPS, bool MANY>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void decode_layers_kernel(Args a) {
   __shared__ Shared sh;
-  if (threadIdx.x == 0) gather(a, sh.rank, sh.blocks);
+  if (threadIdx.x == 0) {
+    sh.gave_up = 0;
+    gather(a, sh.rank, sh.blocks);
+  }
   if (threadIdx.x >> 6 == 1) share_out(a.shares, sh.shares, threadIdx.x & 63);
   __syncthreads();
   const int rank = __builtin_amdgcn_readfirstlane(sh.rank), blocks = __builtin_amdgcn_readfirstlane(sh.blocks);
@@ -1087,7 +1113,7 @@ __global__ __launch_bounds__(256) void decode_layers_begin_kernel(LayerPack pack
     const unsigned* from = reinterpret_cast<const unsigned*>(&pack);
     unsigned* to = reinterpret_cast<unsigned*>(layers + first);
     for (int i = threadIdx.x; i < count * (int)(sizeof(Layer) / 4); i += 256) to[i] = from[i];
-    if (threadIdx.x < 2) control[threadIdx.x] = 0;
+    if (threadIdx.x < CONTROL_WORDS) control[threadIdx.x] = 0;
   }
   if (to_blank.exchange) {
     char* mine = to_blank.exchange + blockIdx.y * to_blank.per_layer;
@@ -1209,7 +1235,7 @@ int q3_decode_layers_shares(const int* kv_lens, int rows, int kv_heads, int part
 
 // Row b is the one token of sequence b, at position kv_lens[b] - 1, whose key and value are written to the caches; `residual` (rows,
 // width) float32 is the stream, which the layers add to in place. `parts`: of a sequence's keys, at most. `blocks`: of the launch (0: one per processor); `patience`, `limit`: looks
-// before the launch goes on with the blocks it has, and before a wait gives up.
+// before the launch goes on with the blocks it has, and before a wait gives up (the stream is then not numbers, all of it).
 int q3_decode_layers(const Layer* layers, int count, float* residual, int rows, int width, int heads, int kv_heads, int dim, int inner,
                      int norm_dtype, int qk_dtype, float qk_eps, float scale, const float* table, int rotary_dim, int max_pos,
                      const int* block_table, int table_width, const int* kv_lens, int max_kv_len, int page, int num_pages, int parts,

@@ -241,11 +241,12 @@ class DecodeLayers:
             _P(kv_lens.data_ptr()), rows, self.kv_heads, self.parts(max_kv_len), _P(out.data_ptr()), _stream()), "the shares of a step's keys")
         return out
 
-    def run(self, stream, caches, block_table, kv_lens, max_kv_len, table, blocks=0, patience=64):
+    def run(self, stream, caches, block_table, kv_lens, max_kv_len, table, blocks=0, patience=64, limit=1 << 18):
         """The layers over the residual `stream` (T, width) float32, in place: row b is sequence b's one token, at position
         kv_lens[b] - 1 of its caches (per layer keys and values as `decode_attention` takes them). Whether that was done: not for a step
         or pages that the launch does not take. `blocks`, `patience`: of how many blocks (0: one per compute unit), and how often they
-        look for each other before those that are there go on by themselves."""
+        look for each other before those that are there go on by themselves. `limit`: how often a block looks for another's results before it
+        gives up; the stream is then not numbers, all of it (a look takes a microsecond: it is there so that every launch ends)."""
         if not (stream.dim() == 2 and caches and caches[0][0].dim() == 4):
             raise OperandError("a stream (T, width), keys (pages, Hkv, page, D)")
         T = stream.shape[0]
@@ -297,5 +298,5 @@ class DecodeLayers:
             layers, count, _P(at(stream)), T, self.width, H, G, D, self.inner, _DT[self.norm_dtype], _DT[self.qk_dtype],
             _F(self.qk_eps), _F(self.scale), _P(at(table)), D if table is not None else 0, max_pos, _P(at(block_table)),
             block_table.shape[1], _P(at(kv_lens)), int(max_kv_len), page, pages, parts, _P(at(workspace)), int(blocks), int(patience),
-            1 << 18, _stream()), "the layers of a step of single tokens")
+            int(limit), _stream()), "the layers of a step of single tokens")
         return True

@@ -195,3 +195,28 @@ def test_rows_that_other_kernels_are_faster_for(width, heads, inner, rows):
     lib.q3_decode_layers_workspace.restype = ctypes.c_long
     taken = [n for n in range(1, 40) if lib.q3_decode_layers_workspace(4, n, width, heads, heads, 128, inner, 2) > 0]
     assert taken == list(range(1, rows + 1))
+
+
+def test_a_wait_that_is_given_up_leaves_no_numbers():
+    """One look more than none at what other blocks pass on, which is too few for most: the stream is not numbers from end to end, whichever blocks
+    and wavefronts gave up, and the launch ends."""
+    for sizes, rows in (({}, 1), ({}, 3), ({}, 24), (dict(hidden_size=2560, intermediate_size=4096), 1), (dict(hidden_size=2560, intermediate_size=4096), 16)):
+        model = _model(**sizes)
+        native, width = model.decode_run.native, sizes.get("hidden_size", 1024)
+        lengths = [500 - 7 * i for i in range(rows)]
+        keys, values, table, _ = _marked_caches(lengths, 8, 16)
+        caches = [(keys.clone(), values.clone()) for _ in native.layers]
+        lens = torch.tensor(lengths, dtype=torch.int32, device="cuda")
+        g = torch.Generator(device="cuda").manual_seed(2)
+        first = torch.randn(rows, width, generator=g, device="cuda")
+        rotation = model.position.rotation_table()
+
+        def result(**named):
+            stream = first.clone()
+            assert native.run(stream, caches, table, lens, max(lengths), rotation, **named)
+            return stream
+
+        want = result()
+        assert torch.isfinite(want).all()
+        assert torch.isnan(result(limit=1)).all()
+        assert torch.equal(result(), want)
