@@ -155,7 +155,7 @@ class _DecodeGraph:
     def _capture(self, runner, batch, block_tables):
         runner.storage.bind(block_tables)
         # once eagerly on a side stream (libraries build and tune at first use), then capture
-        side = torch.cuda.Stream(device=runner.device)
+        side = runner.side_stream()
         side.wait_stream(torch.cuda.current_stream(runner.device))
         with torch.cuda.stream(side):
             # mixers with a recurrent state would otherwise take this step's tokens twice
@@ -166,7 +166,7 @@ class _DecodeGraph:
         torch.cuda.synchronize(runner.device)
         graph = torch.cuda.CUDAGraph()
         with collector_paused():
-            with torch.cuda.graph(graph):
+            with torch.cuda.graph(graph, pool=runner.graph_pool):
                 self.logits = runner.model.forward(batch, runner.storage)
         self.graph = graph
 
@@ -202,6 +202,16 @@ class ModelRunner:
         self.use_graphs = bool(use_graphs) and self.device.type == "cuda" and model.graph_safe()
         self._graphs = {}
         self.max_graphs = 32
+        # The graphs are replayed one at a time, so what one needs between its first kernel and its last they all may have in the same
+        # memory (the exchange of `ops.layers.DecodeLayers` alone is 77 MB for sixteen rows of the 8B shape); each keeps its logits.
+        self.graph_pool = torch.cuda.graph_pool_handle() if self.use_graphs else None
+        self._side = None
+
+    def side_stream(self):
+        """Where a step runs once before it is captured: one stream for all, whose memory the next such step finds again."""
+        if self._side is None:
+            self._side = torch.cuda.Stream(device=self.device)
+        return self._side
 
     def step(self, entries, device_tokens=None):
         """entries: list of StepEntry. Returns logits (R, V) float32 on the

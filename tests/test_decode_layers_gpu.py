@@ -220,3 +220,35 @@ def test_a_wait_that_is_given_up_leaves_no_numbers():
         assert torch.isfinite(want).all()
         assert torch.isnan(result(limit=1)).all()
         assert torch.equal(result(), want)
+
+
+def test_graphs_share_what_they_need_between_kernels():
+    """Captured for one size after another, the launches' exchanges lie in the same memory, and each graph goes on giving what the parts give,
+    whichever ran in between."""
+    from qwen3_from_scratch_amd.engine import ModelRunner, StepEntry
+
+    model = _model(layers=64)
+    runs, sizes, steps = model.decode_run, (24, 16, 12, 8, 6, 4), 3
+    g = torch.Generator().manual_seed(3)
+    ids = [torch.randint(0, 512, (300 + steps * len(sizes),), generator=g).tolist() for _ in range(sizes[0])]
+    taken, logits = [], {}
+    for launch in (True, False):
+        model.decode_run = runs if launch else None
+        runner = ModelRunner(model, 16, 24 * 24, max_requests=24, use_graphs=launch)
+        at = [200 + 3 * i for i in range(24)]
+        for i, n in enumerate(at):
+            runner.step([StepEntry(i, ids[i][:n], [])])
+        out = []
+        for _ in range(steps):
+            for rows in sizes:
+                out.append(runner.step([StepEntry(i, [ids[i][at[i]]], [0]) for i in range(rows)]).clone())
+                at = [n + (i < rows) for i, n in enumerate(at)]
+                if launch and len(taken) < len(sizes):
+                    torch.cuda.synchronize()
+                    taken.append(torch.cuda.memory_reserved())
+        logits[launch] = out
+    model.decode_run = runs
+    for got, want in zip(logits[True], logits[False]):
+        assert (got - want).norm() <= 0.04 * want.norm()
+    own = [runs.native._workspace(64, rows, 1024, 16, 8, 128, 2048, 1) for rows in sizes[1:]]
+    assert taken[-1] - taken[0] < sum(own) // 4, (taken, own)
