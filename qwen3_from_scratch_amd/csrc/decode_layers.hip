@@ -658,7 +658,8 @@ struct Block {
     }
     return p;
   }
-  // attention_tiles.h's tile_addr (with the lane as a number of its own: what follows from it is not kept over the launch)
+  // attention_tiles.h's tile_addr over again, with the lane as a number of its own: what follows from it is not kept over the launch. (As an
+  // argument of that function the lane changes the registers of all of attention.hip's kernels.)
   __device__ __forceinline__ TileAddr addr_of(const TilePages& p, const bf16_t* keys, const bf16_t* values, int g_kv, int tile) const {
     const int lane = anew(this->lane), col = lane & 15, grp = lane >> 4;
     long kh[2], vh[2];
@@ -730,7 +731,9 @@ struct Block {
       ask_keys(TileAddr{(const bf16_t*)((uint64_t)keys + it.keys), (const bf16_t*)((uint64_t)values + it.values), it.there});
       ask_values();
     }
-    // the token's rows: lane n has elements 2 n and 2 n + 1, its pair's other half is lane n ^ 32
+    // the token's rows: lane n has elements 2 n and 2 n + 1, its pair's other half is lane n ^ 32. qk_prepare.h's steps, each product and sum rounded where
+    // it is there, but the squares summed over all 64 lanes at once and not in eights: a key may differ in its last bit from the one
+    // that another kernel makes of the same row (and does anyway by the row itself, a product whose K is added up in another order).
     for (int row = wave; row < G + (brings_new ? 2 : 0); row += WAVES) {
       const int head = row < G ? g_kv * G + row : a.heads + (row == G ? 0 : a.kv_heads) + g_kv;
       const bool prepared = row <= G;                 // (values are taken as they are)

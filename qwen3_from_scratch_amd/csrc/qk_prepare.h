@@ -2,7 +2,8 @@
 // rotation of the pairs (d, d + D / 2), in pieces of eight pairs. Two kernels share it: the
 // one that prepares a whole step's heads, and the decoding attention kernel, which prepares
 // its own rows. Every product and sum is written with the rounding it is meant to have, so
-// that both give the same bits whatever the compiler would contract elsewhere.
+// that both give the same bits whatever the compiler would contract elsewhere. (decode_layers.hip has a form of its own, a row a
+// wavefront, with the squares in another order: eight lanes a row are a longer way from one exchange to the next.)
 #pragma once
 
 #include "common.h"
