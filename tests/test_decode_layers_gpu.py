@@ -8,7 +8,9 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-def _model(layers=3, **sizes):
+def _model(layers=3, dtype="bfloat16", scales=None, sharp=1.0, turned=True, components=None, **sizes):
+    """`scales`: the type of the norms' weights; `sharp`: a factor on the queries' norm weights, so that a row looks at few keys; `turned`:
+    whether queries and keys are."""
     from qwen3_from_scratch_amd.config import ModelConfig
     from qwen3_from_scratch_amd.models.decoder import build_model
     from qwen3_from_scratch_amd.parts.base import Precision
@@ -18,8 +20,17 @@ def _model(layers=3, **sizes):
     config = ModelConfig.from_dict(dict(
         dict(shape, **sizes), architectures=["Qwen3ForCausalLM"], vocab_size=512, hidden_act="silu", num_hidden_layers=layers,
         max_position_embeddings=8192, rms_norm_eps=1e-6, rope_theta=1e6, tie_word_embeddings=False))
-    model = build_model(config, Precision.named("bfloat16"), "cuda:0")
-    model.load(RandomWeights(model.tensors(), seed=5, std=0.02, norm_jitter=0.1, generate_on="cuda:0"))
+    class Source(RandomWeights):
+        def get(self, name, device):
+            t = super().get(name, device)
+            if "q_norm" in name:
+                t = t * sharp
+            return t.float() * (1 + 2 ** -12) if scales == torch.float32 and "norm" in name else t
+
+    model = build_model(config, Precision.named(dtype), "cuda:0", components=components)
+    for step in model.spec.order if not turned else ():
+        model.layers[step.layer].block.mixer.attach_position(None)
+    model.load(Source(model.tensors(), seed=5, std=0.02, norm_jitter=0.1, generate_on="cuda:0"))
     return model
 
 
@@ -252,3 +263,113 @@ def test_graphs_share_what_they_need_between_kernels():
         assert (got - want).norm() <= 0.04 * want.norm()
     own = [runs.native._workspace(64, rows, 1024, 16, 8, 128, 2048, 1) for rows in sizes[1:]]
     assert taken[-1] - taken[0] < sum(own) // 4, (taken, own)
+
+
+NO_QK_NORM = {"mixer": {"name": "attention", "kwargs": dict(qk_norm=False)}}
+
+
+# float32 weights of the norms, heads without norms, without a rotation, more layers than the launch's table takes at a time, by rows that take other
+# instantiations; contexts far apart
+@pytest.mark.parametrize("lengths,named", [
+    ([300], dict(scales=torch.float32)), ([90, 5] * 5, dict(scales=torch.float32)), ([40 + i for i in range(20)], dict(scales=torch.float32)),
+    ([300, 20], dict(components=NO_QK_NORM)), ([77] * 12, dict(components=NO_QK_NORM)), ([64] * 18, dict(components=NO_QK_NORM)),
+    ([300, 20], dict(turned=False)), ([33, 600] * 9, dict(turned=False, scales=torch.float32)),
+    ([70], dict(layers=43, hidden_size=256, num_attention_heads=2, num_key_value_heads=1, intermediate_size=256)),
+    ([6000] + [40, 300, 5] * 3, {}), ([4, 2500] + [90] * 20, {})])
+def test_other_layers_against_the_parts(lengths, named):
+    model = _model(**named)
+    assert model.decode_run is not None
+    want = _logits(model, lengths, 2, launch=False)
+    got = _logits(model, lengths, 2)
+    # as in `test_against_the_parts`, whose three layers are off by 0.008 each side; rounding adds up with the root of the depth
+    bound = 0.02 * max(1.0, (named.get("layers", 3) / 3) ** 0.5)
+    assert (got - want).norm() <= bound * want.norm() and not torch.equal(got, want)
+
+
+@pytest.mark.parametrize("lengths", [[700], [2100, 40], [90, 400, 33, 260] * 2, [1000 - 60 * i for i in range(14)], [35 * i + 5 for i in range(24)]])
+def test_as_near_to_float32_as_the_parts(lengths):
+    """Queries that look at few keys, row by row: the launch is as far from the same layers in float32 as the parts are. A tile of keys left out or
+    counted twice shows in the rows that look at it."""
+    exact = _logits(_model(dtype="float32", sharp=4.0), lengths, 2)
+    model = _model(sharp=4.0)
+    away = [(_logits(model, lengths, 2, launch=launch) - exact).norm(dim=-1) / exact.norm(dim=-1) for launch in (False, True)]
+    assert away[1].max() <= 2 * away[0].max(), away
+    assert away[1].pow(2).mean().sqrt() <= 1.25 * away[0].pow(2).mean().sqrt(), away
+
+
+@pytest.mark.parametrize("rows", [5, 9, 17, 25])
+def test_rows_that_fill_a_captured_step_up(rows):
+    """Captured for the next larger size, with rows that stand for nobody: the requests' logits are those of a step without them."""
+    model = _model()
+    lengths = [50 + 11 * i for i in range(rows)]
+    eager, replayed = _logits(model, lengths, 3), _logits(model, lengths, 3, graphs=True)
+    want = _logits(model, lengths, 3, launch=False)
+    assert (replayed - want).norm() <= 0.02 * want.norm()
+    # (the same kernel, or another one of two groups of rows or of how rows are asked for: sums in the same order)
+    assert torch.equal(eager, replayed)
+
+
+@pytest.mark.parametrize("page", [16, 32])
+def test_table_entries_without_a_page(page):
+    """Keys of a page that is not there count as zeros with values of zeros: first, last old and inner ones, whole tiles and halves."""
+    lengths, heads, kv_heads = [600, 97, 40], 8, 4
+    absent = {(0, 0), (0, 7), (0, 8), (0, 600 // page - 1), (1, 1), (2, 0)}
+    native = _layer(heads, kv_heads)
+    keys, values, table, want = _marked_caches(lengths, kv_heads, page, absent)
+    lens = torch.tensor(lengths, dtype=torch.int32, device="cuda")
+    stream = torch.zeros(3, heads * 128, device="cuda")
+    assert native.run(stream, [(keys, values)], table, lens, max(lengths), None)
+    got = stream.view(3, heads, 128).double().cpu()
+    assert ((got - want[:, None]).abs() <= 2 ** -8 * want[:, None] + 1e-30).all()
+
+
+@pytest.mark.parametrize("lengths", [[40, 70, 33], [900, 500, 1200]])
+@pytest.mark.parametrize("which,bad", [("keys", float("inf")), ("keys", float("nan")), ("values", float("inf")), ("values", float("nan"))])
+def test_what_is_no_number_in_the_caches(lengths, which, bad):
+    """One number of the middle request's keys or values that is none: its logits are none, as the parts have it, and the others' are unharmed."""
+    from qwen3_from_scratch_amd.engine import ModelRunner, StepEntry
+
+    model = _model()
+    run, logits = model.decode_run, {}
+    for launch in (True, False):
+        for harmed in (False, True):
+            model.decode_run = run if launch else None
+            runner = ModelRunner(model, 16, 400, max_requests=3, use_graphs=False)
+            for i, n in enumerate(lengths):
+                runner.step([StepEntry(i, [(7 * j + i) % 512 for j in range(n)], [])])
+            if harmed:
+                at = runner.manager.block_table(1, 0)[1]
+                runner.storage.paged[0][which][1][at, 3].view(-1)[200] = bad
+            logits[launch, harmed] = runner.step([StepEntry(i, [9], [0]) for i in range(3)]).clone()
+    model.decode_run = run
+    for launch in (True, False):
+        assert not torch.isfinite(logits[launch, True][1]).any(), launch
+        assert torch.equal(logits[launch, True][[0, 2]], logits[launch, False][[0, 2]]), launch
+
+
+def test_two_launches_on_two_streams():
+    """Both in flight at once, each on whatever processors it finds: each gives what it gives alone."""
+    model = _model()
+    native, rotation, g = model.decode_run.native, model.position.rotation_table(), torch.Generator(device="cuda").manual_seed(4)
+    steps = []
+    for lengths in ([700, 90, 300], [400 + 9 * i for i in range(20)]):
+        keys, values, table, _ = _marked_caches(lengths, 8, 16)
+        steps.append((torch.randn(len(lengths), 1024, generator=g, device="cuda"), [(keys.clone(), values.clone()) for _ in native.layers], table,
+                      torch.tensor(lengths, dtype=torch.int32, device="cuda"), max(lengths)))
+
+    def launch(first, caches, table, lens, longest):
+        stream = first.clone()
+        assert native.run(stream, caches, table, lens, longest, rotation)
+        return stream
+
+    want = [launch(*step) for step in steps]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    got = []
+    for turn in range(10):
+        for on, step in zip(streams, steps):
+            with torch.cuda.stream(on):
+                got.append(launch(*step))
+    torch.cuda.synchronize()
+    for i, stream in enumerate(got):
+        assert torch.equal(stream, want[i % 2]), i
