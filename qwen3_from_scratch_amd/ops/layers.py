@@ -253,6 +253,8 @@ class DecodeLayers:
         H, G, D, page = self.heads, self.kv_heads, self.dim, caches[0][0].shape[2]
         if not 1 <= T <= DECODE_ROWS_MOST or page < 16 or page & (page - 1) or (table is not None and table.shape[1] != D):
             return False
+        if max_kv_len < 1 or not caches[0][0].shape[0]:          # (`decode_attention` has steps over nothing, and caches without a page)
+            return False
         count = len(self.layers)
         if len(caches) != count:
             raise OperandError("a cache for each of the layers")

@@ -373,3 +373,20 @@ def test_two_launches_on_two_streams():
     torch.cuda.synchronize()
     for i, stream in enumerate(got):
         assert torch.equal(stream, want[i % 2]), i
+
+
+def test_steps_over_nothing_are_left_to_the_parts():
+    """Caches without a page, and sequences without a length: refused by neither."""
+    from types import SimpleNamespace
+
+    model = _model(layers=1)
+    native, rotation = model.decode_run.native, model.position.rotation_table()
+    stream, lens, table = torch.ones(2, 1024, device="cuda"), torch.ones(2, dtype=torch.int32, device="cuda"), torch.zeros(2, 4, dtype=torch.int32, device="cuda")
+    for pages, longest in ((0, 1), (3, 0)):
+        caches = [(torch.zeros(pages, 8, 16, 128, dtype=torch.bfloat16, device="cuda"), torch.zeros(pages, 8, 128, 16, dtype=torch.bfloat16, device="cuda"))]
+        assert not native.run(stream, caches, table, lens * longest, longest, rotation)
+        view = SimpleNamespace(paged=dict(keys=caches[0][0], values=caches[0][1]), block_table=table, writes=True)
+        cache = SimpleNamespace(pages_of=lambda planes, names: (caches, table), view=lambda plane, writes=True: view)
+        batch = SimpleNamespace(token_ids=torch.zeros(2, dtype=torch.int32, device="cuda"), max_q_len=1, min_q_len=1, kv_lens=lens * longest, max_kv_len=longest,
+                                cu_seqlens_q=torch.arange(3, dtype=torch.int32, device="cuda"), logits_rows=None)
+        assert torch.isfinite(model.forward(batch, cache)).all()
