@@ -90,7 +90,8 @@ struct Args {
 // The step's attention as pieces: a sequence's keys for one key head, in `parts` parts. Sequence b's are FIRST and those behind it,
 // the parts of a key head side by side; those of sequences in many parts come first, and a block takes every so many-th.
 struct Shares {
-  int first[MOST_ROWS], parts[MOST_ROWS], kv_len[MOST_ROWS], tiles[MOST_ROWS];
+  __attribute__((aligned(16))) float tiles[MOST_ROWS];
+  int first[MOST_ROWS], parts[MOST_ROWS], kv_len[MOST_ROWS];
   int items, in_parts;
 };
 struct AttentionShared {
@@ -219,36 +220,41 @@ __device__ __forceinline__ int numbers_of(const Args& a, int rank, int blocks, i
 // step with a part a sequence (2,738 kernel by kernel), and take 1,782; one of 8,000 3,153 (1,906), 1,279; sixteen with one of 8,000 1,898 (1,803), 1,012;
 // of the 8B shape eight with one of 30,000 5,768 (5,079), 3,737, sixteen 8,964 (5,645), 4,241. With a PIECE of 2 sixteen over 2,000 take 1,318 us
 // and not 1,286, with 6 the first of these 2,052.
-__device__ __forceinline__ int parts_of(int tiles, float per_tile, int s) { return min(max((int)ceilf((float)tiles * per_tile), 1), s); }
+// (Straight code, and sums and maxima in the vector unit: it runs beside the gathering of the blocks, which takes 2.6 us.)
+__device__ __forceinline__ float parts_of(float tiles, float per_tile, float s) { return fminf(fmaxf(ceilf(tiles * per_tile), 1.f), s); }
 __device__ __forceinline__ void share_out(const ShareArgs& a, Shares& sh, int lane) {
   const bool row = lane < a.rows;
-  const int kv_len = row ? max(a.kv_lens[lane], 0) : 0, tiles = (max(kv_len - 1, 0) + FAST_TILE - 1) / FAST_TILE;
-  if (row) sh.tiles[lane] = tiles, sh.kv_len[lane] = kv_len;
-  const int longest = (int)wave_max((float)tiles);
-  int s = 1;
+  const int kv_len = row ? max(a.kv_lens[lane], 0) : 0;
+  const float tiles = (float)((max(kv_len - 1, 0) + FAST_TILE - 1) / FAST_TILE);
+  if (lane < MOST_ROWS) sh.tiles[lane] = tiles, sh.kv_len[lane] = kv_len;
+  const float longest = wave_max(tiles);
+  float s = 1.f;
   if (a.parts_most > 1 && longest > WAVES) {
-    const int tried = lane + 1;                     // (a lane tries a number)
-    const float per_tile = (float)tried / (float)longest;
-    int items = 0;
-    for (int r = 0; r < a.rows; ++r) items += parts_of(sh.tiles[r], per_tile, tried);
-    items *= a.kv_heads;
-    const int steps = (longest + WAVES * tried - 1) / (WAVES * tried), rounds = (items + ROUND - 1) / ROUND;
-    const int cost = 2 * rounds * (PIECE + steps) + (tried > 1 ? (tried + 7) / 8 : 0);
-    const bool fits = tried == 1 || (tried <= a.parts_most && items <= a.items_most && WAVES * (tried - 1) < longest);
-    int best = fits ? cost * 64 + 63 - tried : 0x7fffffff;          // (of equal ones the most parts: 8B shape, four over 2,060 keys 2,896 us, in five 2,961)
+    const float tried = (float)(lane + 1), per_tile = tried / longest;            // (a lane tries a number)
+    float items = (float)(a.rows - MOST_ROWS);     // (rows that are none count as a part here)
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) best = min(best, __shfl_xor(best, off, 64));
-    s = 63 - (best & 63);
+    for (int r = 0; r < MOST_ROWS; r += 4) {
+      const float4 t = *reinterpret_cast<const float4*>(&sh.tiles[r]);
+      items += (parts_of(t.x, per_tile, tried) + parts_of(t.y, per_tile, tried)) + (parts_of(t.z, per_tile, tried) + parts_of(t.w, per_tile, tried));
+    }
+    items *= (float)a.kv_heads;
+    const float steps = ceilf(longest / (WAVES * tried)), rounds = ceilf(items * (1.f / ROUND));
+    const float cost = fminf(2.f * rounds * (PIECE + steps) + (lane > 0 ? (float)((lane + 8) / 8) : 0.f), 131071.f);
+    const bool fits = lane == 0 || (lane < a.parts_most && items <= (float)a.items_most && (float)(WAVES * lane) < longest);
+    // (of equal ones the most parts: 8B shape, four over 2,060 keys 2,896 us, in five parts 2,961)
+    const int best = (int)-wave_max(fits ? -(cost * 64.f + (float)(63 - lane)) : -INFINITY);
+    s = (float)(64 - (best & 63));
   }
-  const int parts = row ? parts_of(tiles, (float)s / (float)max(longest, 1), s) : 0;
+  const int parts = row ? (int)parts_of(tiles, s / fmaxf(longest, 1.f), s) : 0, key = parts * 64 + 63 - lane;
   int first = 0, all = 0;
-  for (int r = 0; r < a.rows; ++r) {
-    const int others = __shfl(parts, r, 64);
-    if (others > parts || (others == parts && r < lane)) first += others;
-    all += others;
+#pragma unroll
+  for (int r = 0; r < MOST_ROWS; ++r) {
+    const int other = __builtin_amdgcn_readlane(key, r);
+    first += other > key ? other >> 6 : 0;
+    all += other >> 6;
   }
-  if (row) sh.first[lane] = first * a.kv_heads, sh.parts[lane] = parts;
-  if (lane == 0) sh.items = all * a.kv_heads, sh.in_parts = s > 1;
+  if (lane < MOST_ROWS) sh.first[lane] = first * a.kv_heads, sh.parts[lane] = parts;
+  if (lane == 0) sh.items = all * a.kv_heads, sh.in_parts = s > 1.f;
 }
 
 typedef const __attribute__((address_space(4))) int* entries_ptr;
@@ -792,7 +798,7 @@ struct Block {
       if (col < G) q[j].u = *reinterpret_cast<const uint4*>(&s.q[col][32 * j + 8 * grp]);
     }
     if (brings_new) {                                 // the new key's scores: the rows shared out once more
-      for (int row = wave; row < G; row += WAVES) {
+      for (int row = WAVES - 1 - wave; row < G; row += WAVES) {      // (by wavefronts that may have no tile: the first ones have)
         const bf16_t* mine = &s.q[row][2 * lane];
         const float dot = wave_sum(fmaf(bf16_to_float(mine[0]), s.k[2 * lane], bf16_to_float(mine[1]) * s.k[2 * lane + 1]));
         if (lane == 0) s.m[WAVES][row] = pos >= 0 ? dot * a.scale_log2 : -INFINITY;
