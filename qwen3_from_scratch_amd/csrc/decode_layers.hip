@@ -291,7 +291,7 @@ struct Block {
   // Between two looks at the exchange: whether to look again. Every wait ends: after so many looks this wavefront waits for nothing
   // any more. That is in the control words before anything that it passes on afterwards (and in shared memory, for its own block's token).
   __device__ __forceinline__ bool again(int n) {
-    if (n >= most) {
+    if (__builtin_expect(n >= most, 0)) {
       alive = 0;
       gave_up(a);
       sh.gave_up = 1;
@@ -791,6 +791,7 @@ struct Block {
         *reinterpret_cast<float2*>((row == G ? s.k : s.v) + 2 * lane) = make_float2((float)pk.e[0], (float)pk.e[1]);
     }
     meet();
+    const int failed = sh.gave_up;                    // (the token's rows may not have come)
     Pack16 q[D / 32];
 #pragma unroll
     for (int j = 0; j < D / 32; ++j) {
@@ -896,7 +897,7 @@ struct Block {
         }
       }
     }
-    if (brings_new && pos >= 0 && tid >= THREADS - 2 * HEAD && !sh.gave_up) {       // the token's key and value into the caches, for later steps
+    if (brings_new && pos >= 0 && tid >= THREADS - 2 * HEAD && !failed) {       // the token's key and value into the caches, for later steps
       const int d = tid & (HEAD - 1), blk = pos >> a.page_bits, at = pos & (a.page - 1);
       const int pg = blk < a.table_width ? ((entries_ptr)(uintptr_t)(a.block_table + (size_t)b * a.table_width))[blk] : -1;
       if (pg >= 0 && pg < a.num_pages) {
