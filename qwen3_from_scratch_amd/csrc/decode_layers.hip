@@ -10,11 +10,11 @@
 // block). The weights of a product's first steps are asked for while the last one's results are on their way, so memory is not idle
 // meanwhile.
 //
-// What it measured (us a step in a graph, the layers' kernels one by one / this): the 0.6B shape, one request over 100 keys 968 / 504,
-// over 1,100 1,012 / 561, over 8,000 1,142 / 751, over 30,000 1,530 / 1,132, four over 1,100 1,136 / 654, eight over 2,000 1,402 / 913,
-// sixteen 1,892 / 1,337, 20 over 770 1,404 / 1,139, 32 over 2,000 2,375 / 2,131; the 8B shape, one over 2,060 3,375 / 2,756, eight
-// 3,926 / 3,293, sixteen 4,796 / 4,115, eight over 8,000 5,020 / 4,383. The first form of this kernel (0.6B, one request 805; 8B 3,012) was
-// faster than the kernels at each of 28 sizes from 1 to 16 rows and 100 to 30,000 keys.
+// What it measured (us a step in a graph, the layers' kernels one by one / this): the 0.6B shape, one request over 100 keys 978 / 506,
+// over 1,100 1,014 / 563, over 8,000 1,149 / 753, over 30,000 1,540 / 1,139, four over 1,100 1,134 / 646, eight over 2,000 1,407 / 915,
+// sixteen 1,886 / 1,341, 20 over 770 1,412 / 1,150, 32 over 2,000 2,414 / 2,147; the 8B shape, one over 2,060 3,383 / 2,768, eight
+// 3,926 / 3,331, sixteen 4,818 / 4,171, eight over 8,000 5,043 / 4,423. Faster at each of 39 sizes of these two from 1 to 32 rows (16) and 100 to
+// 30,000 keys, all contexts alike, by 3 percent (32 over 8,000) to 93; uneven ones: `share_out`; other shapes: `rows_most`.
 //
 // What bounds it: one request of the small shape the chain of five or six exchanges a layer; a look that fails costs a second one behind
 // the first, a store holds up the wavefront's next look (they come back in order), and a wavefront alone on its SIMD takes 4 to 5 cycles
