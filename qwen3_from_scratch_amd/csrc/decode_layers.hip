@@ -1027,7 +1027,8 @@ struct Block {
     }
     // A wait that was given up, in whatever block: no number of the result stands. Every block with a part in the last product has multiplied with
     // numbers that come, over however many blocks, from each of those that had work before it, and these say that they gave up
-    // before they pass anything on. (A thread stores what `finish` had it store.)
+    // before they pass anything on. One that gives up in the last product itself may be too late for the others: its own columns of every row are
+    // no numbers, and so the norm behind the layers and all logits. (A thread stores what `finish` had it store.)
     const int count = number(3, COUNT);
     if (count && __hip_atomic_load(a.control + GAVE_UP, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
       const unsigned nan = 0x7fc00000u;
@@ -1245,7 +1246,8 @@ int q3_decode_layers_shares(const int* kv_lens, int rows, int kv_heads, int part
 
 // Row b is the one token of sequence b, at position kv_lens[b] - 1, whose key and value are written to the caches; `residual` (rows,
 // width) float32 is the stream, which the layers add to in place. `parts`: of a sequence's keys, at most. `blocks`: of the launch (0: one per processor); `patience`, `limit`: looks
-// before the launch goes on with the blocks it has, and before a wait gives up (the stream is then not numbers, all of it).
+// before the launch goes on with the blocks it has, and before a wait gives up (the stream is then not numbers, all of it, or some columns of
+// every row: `Block::layers`, at its end).
 int q3_decode_layers(const Layer* layers, int count, float* residual, int rows, int width, int heads, int kv_heads, int dim, int inner,
                      int norm_dtype, int qk_dtype, float qk_eps, float scale, const float* table, int rotary_dim, int max_pos,
                      const int* block_table, int table_width, const int* kv_lens, int max_kv_len, int page, int num_pages, int parts,

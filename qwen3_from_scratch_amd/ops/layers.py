@@ -246,7 +246,8 @@ class DecodeLayers:
         kv_lens[b] - 1 of its caches (per layer keys and values as `decode_attention` takes them). Whether that was done: not for a step
         or pages that the launch does not take. `blocks`, `patience`: of how many blocks (0: one per compute unit), and how often they
         look for each other before those that are there go on by themselves. `limit`: how often a block looks for another's results before it
-        gives up; the stream is then not numbers, all of it (a look takes a microsecond: it is there so that every launch ends)."""
+        gives up; the stream is then not numbers, all of it, or where that was in the last product, that block's columns of every row (a look takes a
+        microsecond: it is there so that every launch ends)."""
         if not (stream.dim() == 2 and caches and caches[0][0].dim() == 4):
             raise OperandError("a stream (T, width), keys (pages, Hkv, page, D)")
         T = stream.shape[0]
