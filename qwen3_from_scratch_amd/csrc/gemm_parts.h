@@ -19,17 +19,22 @@
 // beside it. With G = 4 each share is a group's of the block's wavefronts: a tile's K is shared out inside the block, which
 // keeps a CU's four SIMDs busy where there are few tiles.
 //
-// What bounds it is the splitting (six vector instructions a number of x and wavefront that reads it, four cycles each)
-// beside the matrix instructions (sixteen), hence wavefronts above each other rather than side by side, so that each splits
-// other rows; in the shapes of few tiles, the chain of stages. Weights from memory, microseconds, float32 matrix instruction
-// on float32 weights / this: 336 rows of 4,096 x 1,024, 8,192 x 1,024, 1,024 x 2,048 and 1,024 x 4,096 37 / 22, 67 / 31,
-// 28 / 13, 53 / 25; 17 rows 12 / 7, 13 / 8, 20 / 10, 37 / 17; 2,048 rows 154 / 67, 304 / 138, 82 / 40, 156 / 74.
+// What bounds it: three pipes that a wavefront keeps busy one after the other, per 16 rows x 128 columns x 32 k 384 cycles of matrix
+// instructions, some 210 of splitting (six vector instructions a number of x and wavefront that reads it) and, for a block's four
+// wavefronts together, 450 of shared memory; with everything but the operands' reads taken out a stage still takes half its time. Hence
+// wavefronts above each other rather than side by side, so that each splits other rows. What a split leaves out (no number, an infinity,
+// bits below bfloat16's smallest) is collected and looked at once at the end, where the block then walks its K again with every
+// split looked at: two branches a split, with the waits that the compiler puts before them, cost a tenth to a sixth of the time. Weights
+// from memory, microseconds, a float32 weight by the float32 matrix instruction / branches at each split / this: 336 rows of 4,096 x 1,024,
+// 8,192 x 1,024, 1,024 x 2,048 and 1,024 x 4,096 37 / 22 / 18.5, 67 / 29 / 27, 28 / 13 / 12, 53 / 24 / 22; 17 rows 12 / 6.7 / 6.2, 13 / 8.7 / 8.1, 20 /
+// 9.5 / 8.5, 37 / 17 / 14.5; 2,048 rows 154 / 67 / 61, 304 / 124 / 119, 82 / 40 / 34, 156 / 72 / 65.
 #pragma once
 
 #include "common.h"
 #include "gates.h"
 
 #include <atomic>
+#include <type_traits>
 
 namespace parts {
 
@@ -83,6 +88,21 @@ __device__ inline bool split8(float (&v)[8], Frag (&part)[3]) {
   if (!__any(left & 0xffffu)) return false;
   drop_upper(v);
   return true;
+}
+
+// The same without a branch: what split8 would have to look at joins `left` (the bits below the lower part's eight: the lower
+// sixteen of the word) and `most` (the largest magnitude, no number if one was none).
+__device__ inline void split8_plain(float (&v)[8], Frag (&part)[3], unsigned& left, float& most) {
+#pragma unroll
+  for (int e = 0; e < 8; e += 2)
+    most = __builtin_elementwise_maximum(most, __builtin_elementwise_maximum(__builtin_fabsf(v[e]), __builtin_fabsf(v[e + 1])));
+  part[0].u = upper_halves8(v);
+  drop_upper(v);
+  part[1].u = upper_halves8(v);
+  drop_upper(v);
+  part[2].u = upper_halves8(v);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) left |= __float_as_uint(v[e]);
 }
 
 // Outputs n .. n + 3 of row m; with SILU the columns are (gate, up) pairs and out is (M, N / 2) = silu(gate) * up.
@@ -182,11 +202,10 @@ __global__ __launch_bounds__(64 * WM * WN * G, (Shape<WM, WN, MI, NJ, G, STAGES>
 
   const f32x4_t zeros = {0.f, 0.f, 0.f, 0.f};
   f32x4_t upper[MI][NJ], lower[MI][NJ], total[MI][NJ];
-#pragma unroll
-  for (int i = 0; i < MI; ++i)
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) upper[i][j] = lower[i][j] = total[i][j] = zeros;
-  auto multiply = [&](int place) {
+  // what the exact sum of three parts leaves out: whether a number of x is none or infinite, or has bits below bfloat16's smallest
+  unsigned left = 0;
+  float most = 0.f;
+  auto multiply = [&](int place, auto careful) {
     const unsigned char* at = mine + place * S::STAGE_BYTES;
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
@@ -203,7 +222,9 @@ __global__ __launch_bounds__(64 * WM * WN * G, (Shape<WM, WN, MI, NJ, G, STAGES>
         const float4 a = *reinterpret_cast<const float4*>(row + 16 * (piece ^ col));
         const float4 b = *reinterpret_cast<const float4*>(row + 16 * ((piece + 1) ^ col));
         float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-        if (split8(v, xf[i])) {   // (sixteen bits below 2^-133: two parts more, 2^64 times as large)
+        if constexpr (!decltype(careful)::value) {
+          split8_plain(v, xf[i], left, most);
+        } else if (split8(v, xf[i])) {   // (sixteen bits below 2^-133: two parts more, 2^64 times as large)
 #pragma unroll
           for (int e = 0; e < 8; ++e) v[e] *= 18446744073709551616.f;
           Frag low[2];
@@ -234,25 +255,45 @@ __global__ __launch_bounds__(64 * WM * WN * G, (Shape<WM, WN, MI, NJ, G, STAGES>
   const int all = K / BK, share_stages = (all + 3) / 4;
   const int first = group * share_stages;   // G 4: this group's share
   const int stages = G == 1 ? all : max(0, min(share_stages, all - first)), walked = G == 1 ? all : share_stages;
+  auto walk = [&](auto careful) {
 #pragma unroll
-  for (int ahead = 0; ahead < STAGES - 1; ++ahead)
-    if (ahead < stages) copy_stage(first + ahead, ahead);
-  int to_join = share_stages;
-  for (int st = 0; st < walked; ++st) {
-    wait_for_stage(min(st + STAGES - 2, stages - 1) - st);
-    __syncthreads();
-    if (st + STAGES - 1 < stages) copy_stage(first + st + STAGES - 1, (st + STAGES - 1) % STAGES);
-    if (G == 1 || st < stages) multiply(st % STAGES);
-    if (G == 1 && (--to_join == 0 || st == walked - 1)) {
-      to_join = share_stages;
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
-      for (int i = 0; i < MI; ++i)
+      for (int j = 0; j < NJ; ++j) upper[i][j] = lower[i][j] = total[i][j] = zeros;
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-          total[i][j] += upper[i][j] + lower[i][j];
-          upper[i][j] = lower[i][j] = zeros;
-        }
+    for (int ahead = 0; ahead < STAGES - 1; ++ahead)
+      if (ahead < stages) copy_stage(first + ahead, ahead);
+    int to_join = share_stages;
+    for (int st = 0; st < walked; ++st) {
+      wait_for_stage(min(st + STAGES - 2, stages - 1) - st);
+      __syncthreads();
+      if (st + STAGES - 1 < stages) copy_stage(first + st + STAGES - 1, (st + STAGES - 1) % STAGES);
+      if (G == 1 || st < stages) multiply(st % STAGES, careful);
+      if (G == 1 && (--to_join == 0 || st == walked - 1)) {
+        to_join = share_stages;
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) {
+            total[i][j] += upper[i][j] + lower[i][j];
+            upper[i][j] = lower[i][j] = zeros;
+          }
+      }
     }
+  };
+  walk(std::false_type());
+  // rare, and the whole block's (a word a wavefront in the stages' place, where every copy has landed and been read)
+  unsigned* odd = reinterpret_cast<unsigned*>(smem);
+  const bool seen = __any((left & 0xffffu) != 0 || !(most < __builtin_inff()));
+  __syncthreads();
+  if (lane == 0) odd[threadIdx.x >> 6] = seen;
+  __syncthreads();
+  unsigned again = 0;
+#pragma unroll
+  for (int v = 0; v < WM * WN * G; ++v) again |= odd[v];
+  if (__builtin_amdgcn_readfirstlane(again)) {
+    __syncthreads();
+    walk(std::true_type());
   }
   auto put = [&](int m, int n, const float4& v) { store_quad<SILU>(out, m, n, M, N, v); };
   if constexpr (G == 1) {
@@ -366,8 +407,8 @@ int launch(const void* x, const void* w, void* out, int M, int N, int K, hipStre
       hipLaunchKernelGGL((few_rows_kernel<16, SILU>), grid, dim3(256), 0, stream, (const float*)x, (const bf16_t*)w, (float*)out, M, N, K);
     return q3_launch_status();
   }
-  // 64 x 128 tiles, two blocks a CU, from 192 of them on (201 rows of 8,192 x 1,024, 256 tiles: 23 us, in 32 x 64 with
-  // K shared out 30; 336 rows of 4,096, 192 tiles: 22 and 24; 201 rows of 4,096, 128 tiles: 22 and 16). Below, K shared out
+  // 64 x 128 tiles, two blocks a CU, from 192 of them on (201 rows of 8,192 x 1,024, 256 tiles: 19 us, in 32 x 64 with
+  // K shared out 30; 336 rows of 4,096, 192 tiles: 18 and 20; 201 rows of 4,096, 128 tiles: 18 and 15). Below, K shared out
   // inside the block, one block a CU: the smallest tiles that still are one round of the 256 CUs (1,024 x 4,096:
   // 100 rows, 256 tiles of 32 x 16: 18.2 us, in 32 x 32 19.7; 201 rows, 224 tiles of 32 x 32: 20.4, in 32 x 64 24.2; 336 rows, 352 tiles
   // of 32 x 32: 38, in 32 x 64 25). An inner size that leaves groups without a stage has nothing to share out where it takes
