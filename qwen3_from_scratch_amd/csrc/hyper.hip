@@ -224,6 +224,83 @@ __global__ void __launch_bounds__(1024) hyper_norm_row_kernel(float* __restrict_
   store_quad(out + (size_t)r * W + j, v);
 }
 
+// The streams as what they are sums of: every stream is a weighted sum of the embedding's rows and of the sublayers' results so
+// far, with weights that the model's tables fix, and so is what a sublayer or the last norm reads of them. While these sources
+// take less memory than the streams (see HyperConnectionBlock.plan) nothing is kept but them:
+//   u = c[0] float(table[ids[t]]) + sum_j c[1 + j] values[j][t],   out = the layer norm of u as above.
+// SOURCES of them, four columns a thread and the whole row in a block, everything asked for at once. An id outside the table
+// counts as a row of zeros.
+//
+// Bound by memory for many rows and by latency for few. 2,048 rows of 2,048, bfloat16, four streams: the update and read of the streams
+// moves 151 MB (21 to 28 us a sublayer, and 18 for the streams' beginning), this 8.4 MB a source and 8.4 out: two sources 8.7 us, four 9.8,
+// seven 12.5. 8 rows 3.7 to 4.6, where the update and read take 4.7 and the streams' beginning 5.5.
+#define Q3_SOURCES_MOST 16
+struct Sources {
+  const void* at[Q3_SOURCES_MOST];      // the table, then the results
+  float c[Q3_SOURCES_MOST];
+};
+template <typename TA, int SOURCES>
+__global__ void __launch_bounds__(1024) read_sources_kernel(Sources from, const int* __restrict__ ids, int V,
+                                                            const float* __restrict__ weight, const int* __restrict__ rows,
+                                                            TA* __restrict__ out, int W, float eps) {
+  __shared__ float scratch[17];
+  const int r = blockIdx.x;
+  const size_t src = rows ? (size_t)rows[r] : (size_t)r;
+  const bool live = 4 * threadIdx.x < (unsigned)W;
+  const int j = live ? 4 * threadIdx.x : 0;      // a thread past the end reads column 0 and adds nothing
+  float got[SOURCES][4];
+#pragma unroll
+  for (int k = 1; k < SOURCES; ++k) load_quad((const TA*)from.at[k] + src * W + j, got[k]);
+  const float4 w4 = *reinterpret_cast<const float4*>(weight + j);
+  const int id = ids[src];
+  const bool ok = id >= 0 && id < V;
+  load_quad((const TA*)from.at[0] + (size_t)(ok ? id : 0) * W + j, got[0]);
+  float u[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    u[e] = ok ? from.c[0] * got[0][e] : 0.f;
+#pragma unroll
+    for (int k = 1; k < SOURCES; ++k) u[e] += from.c[k] * got[k][e];
+  }
+  const float mean = block_sum(live ? (u[0] + u[1]) + (u[2] + u[3]) : 0.f, scratch) / (float)W;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) u[e] -= mean;
+  const float inv =
+      rsqrtf(block_sum(live ? (u[0] * u[0] + u[1] * u[1]) + (u[2] * u[2] + u[3] * u[3]) : 0.f, scratch) / (float)W + eps);
+  if (!live) return;
+  const float v[4] = {u[0] * inv * w4.x, u[1] * inv * w4.y, u[2] * inv * w4.z, u[3] * inv * w4.w};
+  store_quad(out + (size_t)r * W + j, v);
+}
+
+// The streams themselves from their sources, for the sublayers behind the one from which on they are the smaller: grid (T), four columns a
+// thread; `c` (streams, sources) float32.
+template <typename TA>
+__global__ void streams_from_sources_kernel(Sources from, int sources, const float* __restrict__ c, const int* __restrict__ ids,
+                                            int V, float* __restrict__ x, int S, int W) {
+  const size_t t = blockIdx.x;
+  const int id = ids[t];
+  const bool ok = id >= 0 && id < V;
+  for (int j = 4 * threadIdx.x; j < W; j += 4 * blockDim.x) {
+    float sum[Q3_STREAMS_MOST][4];
+#pragma unroll
+    for (int s = 0; s < Q3_STREAMS_MOST; ++s) sum[s][0] = sum[s][1] = sum[s][2] = sum[s][3] = 0.f;
+    for (int k = 0; k < sources; ++k) {
+      float got[4];
+      load_quad((const TA*)from.at[k] + (k ? t : (size_t)(ok ? id : 0)) * W + j, got);
+      if (k == 0 && !ok) continue;
+#pragma unroll
+      for (int s = 0; s < Q3_STREAMS_MOST; ++s) {
+        const float by = s < S ? c[s * sources + k] : 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum[s][e] += by * got[e];
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < Q3_STREAMS_MOST; ++s)
+      if (s < S) store_quad(x + (t * S + s) * W + j, sum[s]);
+  }
+}
+
 // One block per (token, part): v = y * silu(gate); out = v * rsqrt(mean(v^2) + eps) * weight over
 // the part's `size` numbers. y float32 (T, inner); gate rows `gate_stride` apart.
 template <typename TA>
@@ -325,6 +402,51 @@ extern "C" int q3_hyper_norm(float* x, const void* delta, const float* mix, cons
                       hipLaunchKernelGGL((hyper_norm_kernel<TA, 1>), dim3(n_out), dim3(threads_for(W)),
                                          (size_t)W * sizeof(float), stream, x, (const TA*)delta, mix, write, read, weight,
                                          rows, (TA*)out, S, W, eps, write_back));
+  return q3_launch_status();
+}
+
+extern "C" int q3_sources_most() { return Q3_SOURCES_MOST; }
+
+// `at` (sources) and `c` (sources) are the host's. W a multiple of four up to 4,096, sixteen-byte rows.
+template <typename TA, int SOURCES = Q3_SOURCES_MOST>
+static void launch_read_sources(int sources, const Sources& from, const int* ids, int V, const float* weight, const int* rows,
+                                void* out, int n_out, int W, float eps, hipStream_t stream) {
+  if (sources == SOURCES) {
+    hipLaunchKernelGGL((read_sources_kernel<TA, SOURCES>), dim3(n_out), dim3((W / 4 + 63) / 64 * 64), 0, stream, from, ids, V,
+                       weight, rows, (TA*)out, W, eps);
+  } else if constexpr (SOURCES > 1) {
+    launch_read_sources<TA, SOURCES - 1>(sources, from, ids, V, weight, rows, out, n_out, W, eps, stream);
+  }
+}
+static int take_sources(Sources* from, const void* const* at, const float* c, int sources, int W) {
+  if (sources < 1 || sources > Q3_SOURCES_MOST || W <= 0 || W % 4 || W > 4096 || !at) return Q3_ERR_BAD_ARGUMENT;
+  for (int k = 0; k < sources; ++k) {
+    if (!at[k] || ((size_t)at[k] & 15)) return Q3_ERR_BAD_ARGUMENT;
+    from->at[k] = at[k];
+    from->c[k] = c ? c[k] : 0.f;
+  }
+  return 0;
+}
+extern "C" int q3_read_sources(const void* const* at, const float* c, int sources, const int* ids, int V, const float* weight,
+                               const int* rows, void* out, int n_out, int W, float eps, int act_dtype, hipStream_t stream) {
+  Sources from{};
+  if (n_out <= 0 || V <= 0 || !ids || !weight || !out || !c || (((size_t)weight | (size_t)out) & 15)) return Q3_ERR_BAD_ARGUMENT;
+  const int wrong = take_sources(&from, at, c, sources, W);
+  if (wrong) return wrong;
+  Q3_DISPATCH_DTYPE(act_dtype, TA, launch_read_sources<TA>(sources, from, ids, V, weight, rows, out, n_out, W, eps, stream));
+  return q3_launch_status();
+}
+// `c` (S, sources) is the device's.
+extern "C" int q3_streams_from_sources(const void* const* at, const float* c, int sources, const int* ids, int V, float* x, int T,
+                                       int S, int W, int act_dtype, hipStream_t stream) {
+  Sources from{};
+  if (T <= 0 || V <= 0 || S <= 0 || S > Q3_STREAMS_MOST || !ids || !c || !x || ((size_t)x & 15)) return Q3_ERR_BAD_ARGUMENT;
+  const int wrong = take_sources(&from, at, nullptr, sources, W);
+  if (wrong) return wrong;
+  const int threads = W >= 2048 ? 256 : 128;
+  Q3_DISPATCH_DTYPE(act_dtype, TA,
+                    hipLaunchKernelGGL(streams_from_sources_kernel<TA>, dim3(T), dim3(threads), 0, stream, from, sources, c, ids, V,
+                                       x, S, W));
   return q3_launch_status();
 }
 

@@ -8,6 +8,7 @@ from ..parts.base import UnscaledRows, build_part
 from ..parts.linear import copy_float32_matrices
 from ..weights.checkpoint import check_tensors
 from .layer_run import decode_run, layer_runs
+from .stream_sources import stream_plan
 
 
 class _Layer:
@@ -59,6 +60,7 @@ class DecoderModel:
         self.observer = None      # called with (run-order entry, stream, what it still lacks) behind every layer
         self.runs = {}            # step -> the stretch of layers that may run as one native call with it (set by load)
         self.decode_run = None    # all layers in one launch, for steps of single tokens (set by load)
+        self.stream_plan = None   # how a residual in several streams is kept as the sums that they are (set by load)
         self.plane_of_step = []
         self.plane_needs = []
         for i, step in enumerate(spec.order):
@@ -134,14 +136,17 @@ class DecoderModel:
             copy_float32_matrices(self.parts())
         self.runs = layer_runs(self)
         self.decode_run = decode_run(self)
+        self.stream_plan = stream_plan(self)
         return self
 
     @torch.no_grad()
     def forward(self, batch, cache):
         """Logits (R, V) float32 at batch.logits_rows, from batch.token_ids and
         what `cache` holds. `cache.view(plane, writes)` gives a mixer its view."""
-        x = self.embedding.forward(batch.token_ids)
-        x = self.position.on_embeddings(x, batch)
+        if self.stream_plan is not None and self.observer is None and batch.token_ids.shape[0]:
+            x = self.stream_plan.start(batch.token_ids, self.embedding.weight)
+        else:
+            x = self.position.on_embeddings(self.embedding.forward(batch.token_ids), batch)
         # a model whose passes begin with the embedding's output once more keeps a copy: the stream moves on in place
         start = x.clone() if getattr(self.pass_vectors, "wants_start", False) else None
         pending = None

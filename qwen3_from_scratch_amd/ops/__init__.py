@@ -47,6 +47,8 @@ __all__ = [
     "moe_gated_experts",
     "embed_streams",
     "hyper_norm",
+    "read_sources",
+    "streams_from_sources",
     "causal_conv",
     "mamba2_scan",
     "gated_rmsnorm",
@@ -913,6 +915,56 @@ def hyper_norm(x, weight, eps, out_dtype, read=None, delta=None, mix=None, write
             _ptr(x), _ptr(delta), _ptr(mix), _ptr(write), _ptr(read), _ptr(weight), _ptr(rows), _ptr(out), n_out, S, W,
             ctypes.c_float(eps), _DT[out_dtype], 1 if (write_back and rows is None and delta is not None) else 0,
             _stream()), "hyper_norm")
+    return out
+
+
+SOURCES_MOST = 16     # that `read_sources` takes
+
+
+def _sources(ids, table, values):
+    _need(ids.dtype == torch.int32 and ids.dim() == 1 and table.dim() == 2 and table.dtype in _DT,
+          "ids int32 (T,), table (V, W) bfloat16 or float32")
+    _dev(ids, table, *values)
+    T, W = ids.shape[0], table.shape[1]
+    _need(1 + len(values) <= SOURCES_MOST and W % 4 == 0 and W <= 4096, "up to %d sources, rows of a multiple of 4 up to 4,096 numbers" % SOURCES_MOST)
+    for v in values:
+        _need(v.shape == (T, W) and v.dtype == table.dtype, "a source is (T, W) of the table's dtype")
+    return (ctypes.c_void_p * (1 + len(values)))(table.data_ptr(), *(v.data_ptr() for v in values))
+
+
+def read_sources(ids, table, values, coefficients, weight, eps, rows=None):
+    """Layer norm of a weighted sum of an embedding's rows and of further rows, float32 until the result is rounded:
+    u = coefficients[0] table[ids] + sum_j coefficients[1 + j] values[j], out = (u - mean(u)) rsqrt(mean((u - mean(u))^2) + eps)
+    weight, for all rows or for `rows` of them. `values` (T, W) each of the table's dtype; `coefficients` numbers of the host."""
+    at = _sources(ids, table, values)
+    T, (V, W) = ids.shape[0], table.shape
+    _need(len(coefficients) == len(at), "one coefficient per source")
+    _f32(weight, (W,), "weight")
+    n_out = T
+    if rows is not None:
+        _dev(rows)
+        _need(rows.dtype == torch.int32 and rows.dim() == 1, "rows must be int32 (R,)")
+        n_out = rows.shape[0]
+    out = torch.empty((n_out, W), dtype=table.dtype, device=table.device)
+    if n_out:
+        _check(library("hyper").q3_read_sources(
+            at, (ctypes.c_float * len(at))(*coefficients), len(at), _ptr(ids), V, _ptr(weight), _ptr(rows), _ptr(out), n_out, W,
+            ctypes.c_float(eps), _DT[table.dtype], _stream()), "read_sources")
+    return out
+
+
+def streams_from_sources(ids, table, values, coefficients):
+    """x[t, s] = coefficients[s, 0] table[ids[t]] + sum_j coefficients[s, 1 + j] values[j][t], float32 (T, S, W); `coefficients`
+    float32 (S, sources) on the GPU."""
+    at = _sources(ids, table, values)
+    T, (V, W) = ids.shape[0], table.shape
+    S = coefficients.shape[0]
+    _f32(coefficients, (S, len(at)), "coefficients")
+    _need(1 <= S <= 8, "1 to 8 streams")
+    out = torch.empty((T, S, W), dtype=torch.float32, device=table.device)
+    if T:
+        _check(library("hyper").q3_streams_from_sources(at, _ptr(coefficients), len(at), _ptr(ids), V, _ptr(out), T, S, W,
+                                                        _DT[table.dtype], _stream()), "streams_from_sources")
     return out
 
 

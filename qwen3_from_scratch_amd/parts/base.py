@@ -12,6 +12,7 @@ from dataclasses import dataclass, field
 
 import torch
 
+from .. import ops
 from ..config.registry import lookup_part
 
 
@@ -198,11 +199,20 @@ class HyperAddend:
     x_t <- sum_s mix[s, t] x_s + write[t] * y, with `mix` (streams, streams) indexed [from, to] and
     `write` (streams,), both float32 (a multiplier of the residual is part of `write`). A norm that
     takes it as `delta` does this in float32 in the kernel that also reads the streams for the
-    next sublayer."""
+    next sublayer. Where the streams are kept as the sums that they are, y may come as several results, of which
+    `scales` says by how much each counts."""
 
-    values: torch.Tensor
+    values: object
     mix: torch.Tensor
     write: torch.Tensor
+    scales: tuple = (1.0,)
+
+    def joined(self):
+        """y in one tensor."""
+        if not isinstance(self.values, tuple):
+            return self.values
+        (a, b), (alpha, beta) = self.values, self.scales
+        return ops.scaled_sum(a, alpha, b, beta)
 
 
 def build_part(spec, prefix, precision, device):

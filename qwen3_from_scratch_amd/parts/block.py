@@ -187,10 +187,19 @@ class HyperConnectionBlock(Part):
                 mix = torch.ones((1, 1), dtype=torch.float32, device=self.device)
             self.tables[q] = (read, write, mix)
 
+    def numbers(self):
+        """Per sublayer its tables as the host's numbers, and the scales of the results that it gives where the streams are
+        kept as the sums that they are."""
+        for q in self._sublayers():
+            yield tuple(t.double().tolist() for t in self.tables[q]), getattr(self.mixer, "scales", (1.0,)) if q == 1 else (1.0,)
+
     def forward(self, x, pending, batch, cache, next_norm=None):
         read, write, mix = self.tables[1]
-        y = self.mixer.forward(self.mixer_norm.forward(x, delta=pending, read=read), batch, cache)
-        pending = HyperAddend(y, mix, write)
+        h = self.mixer_norm.forward(x, delta=pending, read=read)
+        if isinstance(x, torch.Tensor) or not hasattr(self.mixer, "scales"):
+            pending = HyperAddend(self.mixer.forward(h, batch, cache), mix, write)
+        else:
+            pending = HyperAddend(self.mixer.forward_sides(h, batch, cache), mix, write, self.mixer.scales)
         if self.feed_forward is not None:
             read, write, mix = self.tables[2]
             y = self.feed_forward.forward(self.feed_forward_norm.forward(x, delta=pending, read=read), batch)

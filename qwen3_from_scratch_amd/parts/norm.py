@@ -102,7 +102,7 @@ class StreamReader(Part):
 class LayerNorm(Part):
     """y = (u - mean(u)) * rsqrt(var(u) + eps) * weight, var the mean of the squared deviations,
     a weight and no bias. u is read from a float32 residual that is held in one or several
-    streams, (T, width) or (T, streams, width): u = sum_s read[s] x_s (`read` None: the plain sum,
+    streams, (T, width) or (T, streams, width), or as the sources whose sums the streams are (`StreamSources`): u = sum_s read[s] x_s (`read` None: the plain sum,
     which is also what the model's last norm wants). A `HyperAddend` given as `delta` first enters
     all streams at once (x_t <- sum_s mix[s, t] x_s + write[t] y), a plain tensor is added to the
     only stream; all of it float32 in one kernel, the result rounded once."""
@@ -122,6 +122,8 @@ class LayerNorm(Part):
         self.weight = fetch(self._name(self.leaf), torch.float32)
 
     def forward(self, x, delta=None, rows=None, read=None):
+        if not isinstance(x, torch.Tensor):      # streams that are kept as the sums they are
+            return x.read(self, delta, read, rows)
         streams = x if x.dim() == 3 else x.unsqueeze(1)
         mix = write = values = None
         if isinstance(delta, HyperAddend):

@@ -74,8 +74,14 @@ class ParallelMixers(Part):
             view.state = cache.state[:, first:last]
         return view
 
+    @property
+    def scales(self):
+        return tuple(scale for _, _, scale in self.sides)
+
+    def forward_sides(self, x, batch, cache):
+        """Both sides' results, for a reader that adds them up with `scales` itself."""
+        return tuple(side.forward(x, batch, self._view(name, cache)) for name, side, _ in self.sides)
+
     def forward(self, x, batch, cache):
-        (ln, left, ls), (rn, right, rs) = self.sides
-        a = left.forward(x, batch, self._view(ln, cache))
-        b = right.forward(x, batch, self._view(rn, cache))
-        return ops.scaled_sum(a, ls, b, rs)
+        (a, b), (alpha, beta) = self.forward_sides(x, batch, cache), self.scales
+        return ops.scaled_sum(a, alpha, b, beta)
