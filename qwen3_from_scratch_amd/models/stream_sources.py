@@ -88,16 +88,24 @@ def stream_plan(model):
         reads.append([sum(w * x for w, x in zip(weights, c)) for c in each])
         until += 1
 
+    # every table's numbers in one copy to the host
+    tables = [t for block in blocks for q, _ in block.sublayer_scales() for t in block.tables[q]]
+    flat, numbers = torch.cat([t.reshape(-1) for t in tables]).tolist(), {}
+    for i, block in enumerate(blocks):
+        for q, _ in block.sublayer_scales():
+            read, write, mix = flat[:streams], flat[streams:2 * streams], flat[2 * streams:2 * streams + streams * streams]
+            numbers[i, q] = read, write, [mix[s * streams:(s + 1) * streams] for s in range(streams)]
+            flat = flat[2 * streams + streams * streams:]
     for step in order:
-        for (read, write, mix), scales in blocks[step.layer].numbers():
+        for q, scales in blocks[step.layer].sublayer_scales():
+            read, write, mix = numbers[step.layer, q]
             take(read)
             each = [[sum(c[s] * mix[s][t] for s in range(streams)) for t in range(streams)] for c in each]
             each += [[w * scale for w in write] for scale in scales]
             if at_streams is not None:
                 break
     take([1.0] * streams)
-    numbers = [x for row in reads + (at_streams or []) for x in row]
-    if until == 0 or not all(math.isfinite(x) and abs(x) < 2.0 ** 127 for x in numbers):
+    if until == 0 or not all(math.isfinite(x) and abs(x) < 2.0 ** 127 for row in reads + (at_streams or []) for x in row):
         return None
     if at_streams is not None:
         at_streams = torch.tensor(at_streams, dtype=torch.float32, device=model.device)

@@ -187,11 +187,9 @@ class HyperConnectionBlock(Part):
                 mix = torch.ones((1, 1), dtype=torch.float32, device=self.device)
             self.tables[q] = (read, write, mix)
 
-    def numbers(self):
-        """Per sublayer its tables as the host's numbers, and the scales of the results that it gives where the streams are
-        kept as the sums that they are."""
-        for q in self._sublayers():
-            yield tuple(t.double().tolist() for t in self.tables[q]), getattr(self.mixer, "scales", (1.0,)) if q == 1 else (1.0,)
+    def sublayer_scales(self):
+        """Per sublayer the scales of the results that it gives where the streams are kept as the sums that they are."""
+        return [(q, getattr(self.mixer, "scales", (1.0,)) if q == 1 else (1.0,)) for q in self._sublayers()]
 
     def forward(self, x, pending, batch, cache, next_norm=None):
         read, write, mix = self.tables[1]
