@@ -1022,6 +1022,16 @@ def mamba2_scan(xbc, dt, dt_bias, a_log, d_skip, state, slots, cu_seqlens_q, hea
     _need(heads % groups == 0 and n_state <= 256, "groups must divide heads; n_state at most 256")
     B = _sequences(slots, cu_seqlens_q, state, heads * n_state * vdim, "mamba2_scan")
     y = torch.empty((T, heads * vdim), dtype=torch.float32, device=xbc.device)
+    if T and max_q_len >= CHUNKED_FROM and xbc.dtype == torch.bfloat16 and xbc.data_ptr() % 16 == 0:
+        lib = library("mamba2")
+        if lib.q3_mamba2_walk_takes(heads, vdim, n_state, groups):
+            lib.q3_mamba2_walk_workspace.restype = ctypes.c_long
+            work = torch.empty(lib.q3_mamba2_walk_workspace(T, B, heads, vdim, n_state, groups), dtype=torch.float32, device=xbc.device)
+            _check(lib.q3_mamba2_walk(
+                _ptr(xbc), _ptr(dt), ctypes.c_long(stride), _ptr(dt_bias), _ptr(a_log), _ptr(d_skip), _ptr(state),
+                ctypes.c_long(state.stride(0)), _ptr(slots), _ptr(cu_seqlens_q), _ptr(y), _ptr(work), T, B, int(max_q_len),
+                heads, vdim, n_state, groups, _stream()), "mamba2_scan")
+            return y
     if T and max_q_len >= CHUNKED_FROM:
         lib = library("recurrent")
         lib.q3_chunked_workspace.restype = ctypes.c_long
