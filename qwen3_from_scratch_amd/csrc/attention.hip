@@ -1452,7 +1452,7 @@ __global__ __launch_bounds__(64 * DECODE_WAVES) Q3_DECODE_WAVES void attn_short_
     const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, const bf16_t* __restrict__ k_cache,
     const bf16_t* __restrict__ v_cache, int num_pages, const int* __restrict__ block_table, int bt_stride,
     const int* __restrict__ cu_q, const int* __restrict__ kv_lens, int sequences, int Hq, int Hkv, int page,
-    score_scale_t scale_log2, const float* __restrict__ sink) {
+    score_scale_t scale_log2, const float* __restrict__ sink Q3_GATE_PARAM) {
   __shared__ DecodeShared<D, false, D> shared;
   const int G = Hq / Hkv, tokens = 16 / G;
   int tile = blockIdx.y;
@@ -1461,7 +1461,7 @@ __global__ __launch_bounds__(64 * DECODE_WAVES) Q3_DECODE_WAVES void attn_short_
   tile = __builtin_amdgcn_readfirstlane(tile);
   decode_block<D, false, float, true, D, true>(shared, 0, blockIdx.x, b, q, q_stride, out, k_cache, v_cache, num_pages,
                                                block_table, bt_stride, cu_q, kv_lens, Hq, Hkv, page, scale_log2, 0, 1, nullptr,
-                                               nullptr, DecodePrep{}, sink, tile * tokens, tokens);
+                                               nullptr, DecodePrep{}, sink Q3_GATE_PASS, tile * tokens, tokens);
 }
 
 // Both kinds of sequences of a step without a window in one launch: `prompt_blocks` blocks for the prompts (Hkv per key share
@@ -1479,7 +1479,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int* __restrict__ cu_q, const int* __restrict__ kv_lens, int sequences, int Hq, int Hkv, int page,
     score_scale_t scale_log2, int prompts_first, int first_blocks, int tokens_per_block, int key_splits, float* __restrict__ part_acc,
     float* __restrict__ part_ml, int splits, float* __restrict__ ws_acc, float* __restrict__ ws_ml,
-    const float* __restrict__ sink) {
+    const float* __restrict__ sink Q3_GATE_PARAM) {
   __shared__ union {
     DecodeShared<D, false, D> decode;
     PrefillShared<D, TILE, STAGES, D> prompt;
@@ -1494,13 +1494,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     tile = __builtin_amdgcn_readfirstlane(tile);
     prefill_block<D, TILE, STAGES, D>(shared.prompt, id % Hkv, tile * key_splits + share % key_splits, b, q, q_stride, out,
                                       k_cache, v_cache, num_pages, block_table, bt_stride, cu_q, kv_lens, Hq, Hkv, page,
-                                      scale_log2, 0, tokens_per_block, key_splits, part_acc, part_ml, sink);
+                                      scale_log2, 0, tokens_per_block, key_splits, part_acc, part_ml, sink Q3_GATE_PASS);
   } else {
     const int pair = id / splits;
     if (pair >= Hkv * sequences) return;
     decode_block<D, false, float, true, D>(shared.decode, id % splits, pair % Hkv, pair / Hkv, q, q_stride, out, k_cache, v_cache,
                                            num_pages, block_table, bt_stride, cu_q, kv_lens, Hq, Hkv, page, scale_log2, 0,
-                                           splits, ws_acc, ws_ml, DecodePrep{}, sink);
+                                           splits, ws_acc, ws_ml, DecodePrep{}, sink Q3_GATE_PASS);
   }
 }
 #endif
@@ -1606,7 +1606,7 @@ static int launch_fast(const void* q, int q_stride, void* out, const void* k_cac
   if (many && window == 0 && splits == 1 && key_splits == 1 && short_tiles * Hkv <= SHORT_BLOCKS) {
     hipLaunchKernelGGL(attn_short_kernel<D>, dim3(Hkv, (unsigned)short_tiles), dim3(256), 0, stream, (const bf16_t*)q, q_stride,
                        (bf16_t*)out, (const bf16_t*)k_cache, (const bf16_t*)v_cache, num_pages, block_table, bt_stride, cu_q,
-                       kv_lens, B, Hq, Hkv, page, scale_log2, sink);
+                       kv_lens, B, Hq, Hkv, page, scale_log2, sink Q3_GATE_ARG);
     return q3_launch_status();
   }
 #endif
@@ -1622,7 +1622,7 @@ static int launch_fast(const void* q, int q_stride, void* out, const void* k_cac
                        stream, (const bf16_t*)q, q_stride, (bf16_t*)out, (const bf16_t*)k_cache, (const bf16_t*)v_cache,
                        num_pages, block_table, bt_stride, cu_q, kv_lens, B, Hq, Hkv, page, scale_log2, prompts_first ? 1 : 0,
                        (int)(prompts_first ? prompt_blocks : decode_blocks), tokens_per_block, key_splits, part_acc, part_ml,
-                       splits, ws_acc, ws_ml, sink);
+                       splits, ws_acc, ws_ml, sink Q3_GATE_ARG);
 #endif
   if (few && !together) {
 #if !defined(Q3_POOLED) && !defined(Q3_SPAN)
@@ -1663,15 +1663,15 @@ static int launch_decode_prep(const void* qkv, void* out, const void* k_cache, c
     hipLaunchKernelGGL((attn_decode_kernel<D, true, W, true>), dim3(splits, Hkv, B), dim3(256), 0, stream,
                        (const bf16_t*)qkv, (Hq + 2 * Hkv) * D, (bf16_t*)out, (const bf16_t*)k_cache,
                        (const bf16_t*)v_cache, num_pages, block_table, bt_stride, cu_q, kv_lens, Hq, Hkv, page,
-                       scale_log2, window, splits, ws_acc, ws_ml, prep, (const float*)nullptr);
+                       scale_log2, window, splits, ws_acc, ws_ml, prep, (const float*)nullptr Q3_GATE_ARG);
   else
     hipLaunchKernelGGL((attn_decode_kernel<D, true, W, false>), dim3(splits, Hkv, B), dim3(256), 0, stream,
                        (const bf16_t*)qkv, (Hq + 2 * Hkv) * D, (bf16_t*)out, (const bf16_t*)k_cache,
                        (const bf16_t*)v_cache, num_pages, block_table, bt_stride, cu_q, kv_lens, Hq, Hkv, page,
-                       scale_log2, window, splits, ws_acc, ws_ml, prep, (const float*)nullptr);
+                       scale_log2, window, splits, ws_acc, ws_ml, prep, (const float*)nullptr Q3_GATE_ARG);
   if (splits > 1 && merge)
     hipLaunchKernelGGL(attn_decode_reduce_kernel<D>, dim3(Hkv, B), dim3(256), 0, stream, (bf16_t*)out,
-                       (const int*)nullptr, Hq, Hkv, splits, ws_acc, ws_ml, (const float*)nullptr);
+                       (const int*)nullptr, Hq, Hkv, splits, ws_acc, ws_ml, (const float*)nullptr Q3_GATE_ARG);
   return q3_launch_status();
 }
 #endif

@@ -1494,8 +1494,8 @@ def softcap_attention(q, k_cache, v_cache, block_table, cu_seqlens_q, kv_lens, s
         out = paged_attention(q, H, k_cache, v_cache, block_table, cu_seqlens_q, kv_lens, max_q_len, max_kv_len, scale,
                               window=window, min_q_len=min_q_len, max_kv_len_of_many=max_kv_len_of_many, softcap=softcap,
                               sink=sink, runs=runs, sigmoid_bias=sigmoid_bias,
-                              gate=gate if runs is not None or sigmoid_bias is not None else None)
-        if gate is not None and runs is None and sigmoid_bias is None:
+                              gate=gate if runs is not None or sigmoid_bias is not None or softcap > 0 else None)
+        if gate is not None and runs is None and sigmoid_bias is None and softcap <= 0:
             _check(library("softcap").q3_gate_heads(_ptr(out), _ptr(gate), ctypes.c_long(stride), wide, T, H, vdim,
                                                     _DT[q.dtype], _stream()), "gate_heads")
         return out
@@ -1738,9 +1738,9 @@ def paged_attention(q, num_q_heads, k_cache, v_cache, block_table, cu_seqlens_q,
             if chunk or window:
                 visible = min(visible, (chunk or window) + keep)
                 longest = min(longest, (chunk or window) + keep)
-        if not (gate is None or runs is not None or sigmoid_bias is not None or span is not None):
-            raise OperandError("a gate comes with runs, sigmoid weights or spans only")
-        if runs is not None or sigmoid_bias is not None or span is not None:
+        if not (gate is None or kinds):
+            raise OperandError("a gate comes with capped scores, runs, sigmoid weights or spans only")
+        if kinds:
             gate_stride = 0
             if gate is not None:
                 gate_stride = _rows_view(gate, "gate")
