@@ -330,12 +330,35 @@ __global__ void gated_rmsnorm_kernel(const float* __restrict__ y, const TA* __re
 // rows): every number is read, and its gate formed, once, where the kernel above does both twice and in a loop that waits
 // for each number: a part of 4,096 takes 4.8 us for 8 rows (there 14.5) and 17.9 for 2,048 rows (there 27; 67 MB,
 // bound by memory).
+//
+// `moved` (a step of one token a sequence; no rows: none): behind a recurrence whose blocks all read the last three inputs of a short
+// convolution's channels `first` .. `first` + `count`, the block of a row moves them up by that row's.
+template <typename TA>
+struct MovedTail {
+  const TA* rows;      // (T, .), `stride` apart, from the convolution's first channel on
+  long stride;
+  float* tails;        // (slots, 3, channels), `tail_stride` apart
+  long tail_stride;
+  const int *slots, *seq_index;
+  int channels, first, count;
+};
 template <typename TA>
 __global__ void __launch_bounds__(1024) gated_rmsnorm_row_kernel(const float* __restrict__ y, const TA* __restrict__ gate,
                                                                  long gate_stride, const float* __restrict__ weight,
-                                                                 TA* __restrict__ out, int inner, int size, float eps) {
+                                                                 TA* __restrict__ out, int inner, int size, float eps,
+                                                                 MovedTail<TA> moved) {
   __shared__ float scratch[17];
   const int t = blockIdx.x, part = blockIdx.y;
+  if (moved.rows && part == 0) {
+    float* tail = moved.tails + (size_t)moved.slots[moved.seq_index[t]] * moved.tail_stride;
+    for (int c = moved.first + threadIdx.x; c < moved.first + moved.count; c += blockDim.x) {
+      const float one = tail[(size_t)moved.channels + c], two = tail[2 * (size_t)moved.channels + c];
+      const float own = to_float(moved.rows[(size_t)t * moved.stride + c]);
+      tail[c] = one;
+      tail[(size_t)moved.channels + c] = two;
+      tail[2 * (size_t)moved.channels + c] = own;
+    }
+  }
   const bool live = 4 * threadIdx.x < (unsigned)size;
   const size_t at = (size_t)part * size + (live ? 4 * threadIdx.x : 0);
   float v[4], g[4], w[4];
@@ -450,21 +473,43 @@ extern "C" int q3_streams_from_sources(const void* const* at, const float* c, in
   return q3_launch_status();
 }
 
+// Whether a part fits a block whole.
+static bool whole_parts(const float* y, const void* gate, long gate_stride, const float* weight, const void* out, int size, int act_dtype) {
+  const size_t act_quad = act_dtype == Q3_F32 ? 15 : 7;
+  return size % 4 == 0 && size <= 4096 && gate_stride % 4 == 0 && (((size_t)y | (size_t)weight) & 15) == 0 &&
+         (((size_t)gate | (size_t)out) & act_quad) == 0;
+}
+
 extern "C" int q3_gated_rmsnorm(const float* y, const void* gate, long gate_stride, const float* weight, void* out,
                                 int T, int inner, int parts, float eps, int act_dtype, hipStream_t stream) {
   if (T <= 0 || inner <= 0 || parts <= 0 || inner % parts || parts > 65535) return Q3_ERR_BAD_ARGUMENT;
   const int size = inner / parts;
-  const size_t act_quad = act_dtype == Q3_F32 ? 15 : 7;
-  if (size % 4 == 0 && size <= 4096 && gate_stride % 4 == 0 && (((size_t)y | (size_t)weight) & 15) == 0 &&
-      (((size_t)gate | (size_t)out) & act_quad) == 0) {
+  if (whole_parts(y, gate, gate_stride, weight, out, size, act_dtype)) {
     Q3_DISPATCH_DTYPE(act_dtype, TA,
                       hipLaunchKernelGGL(gated_rmsnorm_row_kernel<TA>, dim3(T, parts), dim3((size / 4 + 63) / 64 * 64), 0,
-                                         stream, y, (const TA*)gate, gate_stride, weight, (TA*)out, inner, size, eps));
+                                         stream, y, (const TA*)gate, gate_stride, weight, (TA*)out, inner, size, eps, MovedTail<TA>{}));
     return q3_launch_status();
   }
   Q3_DISPATCH_DTYPE(act_dtype, TA,
                     hipLaunchKernelGGL(gated_rmsnorm_kernel<TA>, dim3(T, parts), dim3(threads_for(size)), 0, stream, y,
                                        (const TA*)gate, gate_stride, weight, (TA*)out, inner, size, eps));
+  return q3_launch_status();
+}
+
+// The same for parts that fit a block whole, moving a convolution's tail up by the way (see MovedTail).
+extern "C" int q3_gated_rmsnorm_moving(const float* y, const void* gate, long gate_stride, const float* weight, void* out, int T,
+                                       int inner, int parts, float eps, const void* rows, long stride, float* tails, long tail_stride,
+                                       const int* slots, const int* seq_index, int channels, int first, int count, int act_dtype,
+                                       hipStream_t stream) {
+  if (T <= 0 || inner <= 0 || parts <= 0 || inner % parts || parts > 65535 || !rows || !tails || !slots || !seq_index || first < 0 ||
+      count < 0 || first + count > channels)
+    return Q3_ERR_BAD_ARGUMENT;
+  const int size = inner / parts;
+  if (!whole_parts(y, gate, gate_stride, weight, out, size, act_dtype)) return Q3_ERR_UNSUPPORTED;
+  Q3_DISPATCH_DTYPE(act_dtype, TA,
+                    hipLaunchKernelGGL(gated_rmsnorm_row_kernel<TA>, dim3(T, parts), dim3((size / 4 + 63) / 64 * 64), 0, stream, y,
+                                       (const TA*)gate, gate_stride, weight, (TA*)out, inner, size, eps,
+                                       MovedTail<TA>{(const TA*)rows, stride, tails, tail_stride, slots, seq_index, channels, first, count}));
   return q3_launch_status();
 }
 

@@ -829,6 +829,88 @@ __global__ void __launch_bounds__(256) mamba2_scan_kernel(
   at.store(mine, N, P, group, column);
 }
 
+// A step of one token a sequence, its convolution of four taps inside: `row` of a sequence holds [x: H P | B: G N | C: G N] before it. A block
+// convolves its own 64 columns of x, whose tail it moves up, and the group's B and C, whose tail its fellow blocks read as well: that one
+// moves in the kernel behind (gated_rmsnorm_row_kernel). The same numbers as causal_conv_kernel and mamba2_scan_kernel, whose pair took
+// 5.2 + 9.1 us for 8 requests of 64 heads of 128 x 64, and this 9.5.
+template <typename TA, int EACH, bool WHOLE>
+__global__ void __launch_bounds__(256) mamba2_token_kernel(
+    const TA* __restrict__ rows, const TA* __restrict__ dt, long stride, const float* __restrict__ conv_w,
+    const float* __restrict__ conv_bias, float* __restrict__ tails, const float* __restrict__ dt_bias, const float* __restrict__ a_log,
+    const float* __restrict__ d_skip, float* __restrict__ state, long state_stride, const int* __restrict__ slots,
+    const int* __restrict__ cu, float* __restrict__ y, int H, int P, int N, int G) {
+  __shared__ float sB[16 * EACH], sC[16 * EACH];
+  __shared__ __attribute__((aligned(16))) float sx[64];
+  __shared__ __attribute__((aligned(16))) float part[4][64];
+  constexpr int ITEMS = (64 + 32 * EACH + 255) / 256;      // numbers that a thread convolves
+  const int tid = threadIdx.x, group = tid >> 4;
+  const int column = blockIdx.x * 64 + 4 * (tid & 15);
+  const int h = blockIdx.y, b = blockIdx.z, g = h / (H / G);
+  const int t = cu[b];
+  if (cu[b + 1] <= t) return;
+  const int C = H * P + 2 * G * N;
+  const size_t slot = (size_t)slots[b] * state_stride;
+  const TA* row = rows + (size_t)t * stride;
+  const float rate = expf(a_log[h]), shift = dt_bias[h], skip = d_skip[h];
+  const TA rd = dt[(size_t)t * stride + h];
+  int channel[ITEMS];
+  TA now[ITEMS];
+  float before[ITEMS][3], base[ITEMS];
+  float4 w[ITEMS];
+#pragma unroll
+  for (int k = 0; k < ITEMS; ++k) {
+    const int i = tid + 256 * k;
+    const int c = i < 64 ? (blockIdx.x * 64 + i < P ? h * P + (int)blockIdx.x * 64 + i : -1)
+                         : i - 64 < N ? H * P + g * N + i - 64 : i - 64 - N < N ? H * P + (G + g) * N + i - 64 - N : -1;
+    channel[k] = c;
+    const int at = c < 0 ? 0 : c;
+    now[k] = row[at];
+    w[k] = *reinterpret_cast<const float4*>(conv_w + 4 * (size_t)at);
+    base[k] = conv_bias[at];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) before[k][j] = tails[slot + (size_t)j * C + at];
+  }
+  float* mine = state + slot + (size_t)h * N * P;
+  StateColumns<EACH, WHOLE> at;
+  at.load(mine, N, P, group, column);
+  if (N < 16 * EACH && tid < 16 * EACH && tid >= N) sB[tid] = sC[tid] = 0.f;
+#pragma unroll
+  for (int k = 0; k < ITEMS; ++k) {
+    const int i = tid + 256 * k;
+    const float own = to_float(now[k]);
+    float acc = base[k];
+    acc += w[k].w * own;
+    acc += w[k].z * before[k][2];
+    acc += w[k].y * before[k][1];
+    acc += w[k].x * before[k][0];
+    const float value = to_float(from_float<TA>(silu_value(acc)));
+    if (i < 64) {
+      sx[i] = channel[k] < 0 ? 0.f : value;
+      if (channel[k] >= 0) {
+        float* tail = tails + slot + channel[k];
+        tail[0] = before[k][1];
+        tail[(size_t)C] = before[k][2];
+        tail[2 * (size_t)C] = own;
+      }
+    } else if (i - 64 < N) {
+      sB[i - 64] = value;
+    } else if (i - 64 - N < N) {
+      sC[i - 64 - N] = value;
+    }
+  }
+  const float step = softplus_value(to_float(rd) + shift);
+  const float decay = expf(-rate * step);
+  __syncthreads();
+  const float4 x4 = *reinterpret_cast<const float4*>(sx + 4 * (tid & 15));
+  const float push[4] = {step * x4.x, step * x4.y, step * x4.z, step * x4.w};
+  at.step(decay, sB, sC, push, N, group, part);
+  __syncthreads();
+  const int own = blockIdx.x * 64 + (tid & 63);
+  if (tid < 64 && own < P)
+    y[((size_t)t * H + h) * P + own] = ((part[0][tid] + part[1][tid]) + (part[2][tid] + part[3][tid])) + skip * sx[tid];
+  at.store(mine, N, P, group, column);
+}
+
 // Rows of the input are [q: H dim | k: H dim | v: H vdim | g: H vdim]. Per token q and k turn by the position (pairs
 // (i, i + half) of their first 2 * half numbers, angle = position * inv_freq[i]), k times k_scale; S = decay S + k v^T,
 // o = S^T q, left as float32 in `raw` (T, H vdim): the division by the head's root mean square and the gate follow in
@@ -1006,6 +1088,81 @@ __global__ void __launch_bounds__(256) block_gates_few_kernel(const float* __res
 #pragma unroll
   for (int k = 0; k < 4; ++k) total += part[k][16 * (o / 4) + t][o % 4];
   out[((size_t)g * T + t0 + t) * width + b * bw + o0 + o] = sigmoid_value(total);
+}
+
+// Both gates and the recurrence of a step of one token a sequence: block_gates_few_kernel's products for the two gates at once, then
+// rglru_scan_kernel's step of the block's 16 tokens and outputs, with their numbers. Launches of their own took 5.1 and 5.0 us for 8 tokens of
+// 8 parts of 256, and this 6.5.
+template <typename TO>
+__global__ void __launch_bounds__(256) rglru_token_kernel(const float* __restrict__ u, const float* __restrict__ w,
+                                                          const float* __restrict__ bias, const float* __restrict__ rate,
+                                                          const float* __restrict__ y, long y_stride, const float* __restrict__ y_bias,
+                                                          float* __restrict__ state, long state_stride, const int* __restrict__ slots,
+                                                          const int* __restrict__ seq_index, TO* __restrict__ out, int T, int width,
+                                                          int bw, int out_tiles) {
+  __shared__ __attribute__((aligned(16))) float part[2][4][64][4];
+  const int t0 = blockIdx.x * 16;
+  const int b = blockIdx.y / out_tiles, o0 = (blockIdx.y % out_tiles) * 16;
+  const int blocks = width / bw;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, grp = lane >> 4;
+  const bool token = t0 + col < T, output = o0 + col < bw;
+  const float* ub = u + (size_t)(token ? t0 + col : 0) * width + b * bw;
+  const float* wb = w + (size_t)b * bw * bw + (output ? o0 + col : 0);
+  const size_t other = (size_t)blocks * bw * bw;      // the second gate's weights lie that much further
+  const bool whole = bw % 4 == 0 && ((size_t)u & 15) == 0;
+  // a thread's own output and token at the end, and all that they need
+  const int t = threadIdx.x >> 4, o = threadIdx.x & 15;
+  const bool mine = t0 + t < T && o0 + o < bw;
+  const int row = mine ? t0 + t : 0, c = b * bw + (mine ? o0 + o : 0);
+  float total[2] = {bias[c], bias[width + c]};
+  float* held = state + (size_t)slots[seq_index[row]] * state_stride + c;
+  float S = *held;
+  const float k = rate[c], z = y[(size_t)row * y_stride + c] + y_bias[c], in = u[(size_t)row * width + c];
+  f32x4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  for (int i0 = 64 * wave; i0 < bw; i0 += 256) {
+    float wv[2][4][4], uv[4][4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int i = i0 + 16 * q + 4 * grp;
+      // inputs past the end: a place that exists, and zeros behind the load
+#pragma unroll
+      for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) wv[g][q][e] = wb[g * other + (size_t)(i + e < bw ? i + e : 0) * bw];
+      if (whole) {
+        const float4 four = *reinterpret_cast<const float4*>(ub + (i < bw ? i : 0));
+        uv[q][0] = four.x, uv[q][1] = four.y, uv[q][2] = four.z, uv[q][3] = four.w;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) uv[q][e] = ub[i + e < bw ? i + e : 0];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int i = i0 + 16 * q + 4 * grp;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+          acc[g] = __builtin_amdgcn_mfma_f32_16x16x4f32(output && i + e < bw ? wv[g][q][e] : 0.f, token && i + e < bw ? uv[q][e] : 0.f,
+                                                        acc[g], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int g = 0; g < 2; ++g) *reinterpret_cast<f32x4_t*>(part[g][wave][lane]) = acc[g];
+  __syncthreads();
+  if (!mine) return;
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) total[g] += part[g][v][16 * (o / 4) + t][o % 4];
+  }
+  const float log_a = -k * sigmoid_value(total[0]);
+  const float a = expf(log_a);
+  S = a * S + sqrtf(-expm1f(2.f * log_a)) * sigmoid_value(total[1]) * in;
+  const float branch = 0.5f * z * (1.f + tanhf(0.79788456080286536f * (z + 0.044715f * z * z * z)));
+  out[(size_t)row * width + c] = from_float<TO>(S * branch);
+  *held = S;
 }
 
 // What the three kernels need of Mamba-2's rows: step = softplus(dt + dt_bias); ld = -exp(A_log) step;
@@ -1372,6 +1529,46 @@ extern "C" int q3_mamba2_scan(const void* xbc, const void* dt, long dt_stride, c
   Q3_DISPATCH_DTYPE(act_dtype, TA, return launch_mamba2<TA>(xbc, dt, dt_stride, dt_bias, a_log, d_skip, state,
                                                             state_stride, slots, cu, y, B, H, P, N, G, stream));
   return 0;
+}
+
+// One token a sequence (T == B, cu's steps of one), four taps: `rows` (T, .) from the column of x on, `dt` the column of dt, rows `stride`
+// apart; `tails` and `state` begin in slot 0, slots `state_stride` apart. conv_w at sixteen bytes.
+extern "C" int q3_mamba2_token(const void* rows, const void* dt, long stride, const float* conv_w, const float* conv_bias, float* tails,
+                               const float* dt_bias, const float* a_log, const float* d_skip, float* state, long state_stride,
+                               const int* slots, const int* cu, float* y, int B, int H, int P, int N, int G, int act_dtype,
+                               hipStream_t stream) {
+  if (B <= 0 || H <= 0 || P <= 0 || N <= 0 || G <= 0 || H % G || H > 65535 || B > 65535 || ((size_t)conv_w & 15)) return Q3_ERR_BAD_ARGUMENT;
+  if (N > 256) return Q3_ERR_UNSUPPORTED;
+  const dim3 grid((P + 63) / 64, H, B);
+  const bool whole = P % 4 == 0 && state_stride % 4 == 0 && ((size_t)state & 15) == 0;
+#define Q3_TOKEN(EACH)                                                                                                              \
+  Q3_DISPATCH_DTYPE(act_dtype, TA,                                                                                                  \
+                    hipLaunchKernelGGL((whole ? mamba2_token_kernel<TA, EACH, true> : mamba2_token_kernel<TA, EACH, false>), grid,  \
+                                       dim3(256), 0, stream, (const TA*)rows, (const TA*)dt, stride, conv_w, conv_bias, tails,      \
+                                       dt_bias, a_log, d_skip, state, state_stride, slots, cu, y, H, P, N, G))
+  if (N <= 32) Q3_TOKEN(2);
+  else if (N <= 64) Q3_TOKEN(4);
+  else if (N <= 128) Q3_TOKEN(8);
+  else Q3_TOKEN(16);
+#undef Q3_TOKEN
+  return q3_launch_status();
+}
+
+// One token a sequence; weights (2, blocks, bw, bw), biases (2, width). Few tokens: see Q3_GATES_FEW.
+extern "C" int q3_rglru_token_takes(int T, int width, int blocks) {
+  return T > 0 && blocks > 0 && width > 0 && width % blocks == 0 && width / blocks <= 1536 && (long)T * width <= Q3_GATES_FEW &&
+         (long)blocks * ((width / blocks + 15) / 16) <= 65535;
+}
+extern "C" int q3_rglru_token(const float* u, const float* w, const float* bias, const float* rate, const float* y, long y_stride,
+                              const float* y_bias, float* state, long state_stride, const int* slots, const int* seq_index, void* out,
+                              int T, int width, int blocks, int out_dtype, hipStream_t stream) {
+  if (!q3_rglru_token_takes(T, width, blocks)) return Q3_ERR_BAD_ARGUMENT;
+  const int bw = width / blocks, out_tiles = (bw + 15) / 16;
+  Q3_DISPATCH_DTYPE(out_dtype, TO,
+                    hipLaunchKernelGGL(rglru_token_kernel<TO>, dim3((T + 15) / 16, blocks * out_tiles), dim3(256), 0, stream, u, w, bias,
+                                       rate, y, y_stride, y_bias, state, state_stride, slots, seq_index, (TO*)out, T, width, bw,
+                                       out_tiles));
+  return q3_launch_status();
 }
 
 extern "C" int q3_block_gates(const float* u, const float* w, const float* bias, float* out, int T, int width, int blocks,

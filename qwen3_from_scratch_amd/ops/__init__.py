@@ -52,6 +52,10 @@ __all__ = [
     "causal_conv",
     "mamba2_scan",
     "gated_rmsnorm",
+    "mamba2_token",
+    "mamba2_token_takes",
+    "rglru_token",
+    "rglru_token_takes",
     "block_gates",
     "rglru_scan",
     "retention_scan",
@@ -1064,6 +1068,72 @@ def gated_rmsnorm(y, gate, weight, groups, eps, out_dtype):
     if T:
         _check(library("hyper").q3_gated_rmsnorm(_ptr(y), _ptr(gate), ctypes.c_long(stride), _ptr(weight), _ptr(out), T, n,
                                                  groups, ctypes.c_float(eps), _DT[out_dtype], _stream()), "gated_rmsnorm")
+    return out
+
+
+def mamba2_token_takes(proj, heads, vdim, n_state, groups, norm_groups, conv_weight, rows, sequences, max_q_len):
+    """Whether `mamba2_token` takes a step: single tokens, one a sequence, four taps, parts of the norm that fit a block."""
+    inner = heads * vdim
+    return (proj.is_cuda and max_q_len == 1 and rows == sequences and rows > 0 and conv_weight.shape[1] == 4 and n_state <= 256
+            and conv_weight.data_ptr() % 16 == 0 and (inner // norm_groups) % 4 == 0 and inner // norm_groups <= 4096
+            and proj.stride(1) == 1 and proj.stride(0) % 4 == 0 and proj.data_ptr() % 16 == 0)
+
+
+def mamba2_token(proj, conv_weight, conv_bias, dt_bias, a_log, d_skip, norm_weight, norm_groups, eps, state, slots, cu_seqlens_q,
+                 seq_index, heads, vdim, n_state, groups):
+    """A Mamba-2 mixer's step of one token a sequence between its two products: `causal_conv` with silu, `mamba2_scan` and
+    `gated_rmsnorm` of proj (T, [z | x | B | C | dt]), whose results these are, in two kernels. state float32 (slots, 3 channels + heads
+    n_state vdim): the convolution's last inputs, then the recurrence's state, both brought up to date. See `mamba2_token_takes`."""
+    _dev(conv_weight, conv_bias, dt_bias, a_log, d_skip, norm_weight, seq_index)
+    inner, channels = heads * vdim, heads * vdim + 2 * groups * n_state
+    T = proj.shape[0]
+    stride = _rows_view(proj, "proj")
+    _need(proj.shape[1] == inner + channels + heads and heads % groups == 0, "proj must be (T, [z | x | B | C | dt])")
+    _f32(conv_weight, (channels, 4), "conv_weight")
+    _f32(conv_bias, (channels,), "conv_bias")
+    for t, what in ((dt_bias, "dt_bias"), (a_log, "a_log"), (d_skip, "d_skip")):
+        _f32(t, (heads,), what)
+    _f32(norm_weight, (inner,), "norm_weight")
+    B = _sequences(slots, cu_seqlens_q, state, 3 * channels + heads * n_state * vdim, "mamba2_token")
+    _need(B == T and seq_index.dtype == torch.int32 and seq_index.shape == (T,), "one token a sequence, seq_index int32 (T,)")
+    xbc, dt, held = proj[:, inner:inner + channels], proj[:, inner + channels:], state[:, 3 * channels:]
+    y = torch.empty((T, inner), dtype=torch.float32, device=proj.device)
+    out = torch.empty((T, inner), dtype=proj.dtype, device=proj.device)
+    _check(library("recurrent").q3_mamba2_token(
+        _ptr(xbc), _ptr(dt), ctypes.c_long(stride), _ptr(conv_weight), _ptr(conv_bias), _ptr(state), _ptr(dt_bias), _ptr(a_log),
+        _ptr(d_skip), _ptr(held), ctypes.c_long(state.stride(0)), _ptr(slots), _ptr(cu_seqlens_q), _ptr(y), B, heads, vdim, n_state,
+        groups, _DT[proj.dtype], _stream()), "mamba2_token")
+    _check(library("hyper").q3_gated_rmsnorm_moving(
+        _ptr(y), _ptr(proj), ctypes.c_long(stride), _ptr(norm_weight), _ptr(out), T, inner, norm_groups, ctypes.c_float(eps), _ptr(xbc),
+        ctypes.c_long(stride), _ptr(state), ctypes.c_long(state.stride(0)), _ptr(slots), _ptr(seq_index), channels, inner,
+        2 * groups * n_state, _DT[proj.dtype], _stream()), "mamba2_token")
+    return out
+
+
+def rglru_token_takes(u, rows, sequences, max_q_len, blocks):
+    """Whether `rglru_token` takes a step: single tokens, one a sequence, and few of them."""
+    return (u.is_cuda and max_q_len == 1 and rows == sequences and rows > 0
+            and bool(library("recurrent").q3_rglru_token_takes(rows, u.shape[1], blocks)))
+
+
+def rglru_token(u, weights, biases, rate, y, y_bias, state, slots, cu_seqlens_q, seq_index, out_dtype):
+    """`block_gates` and `rglru_scan` of a step of one token a sequence, with their results, in one kernel."""
+    _dev(u, weights, biases, rate, y_bias, seq_index)
+    T, width = u.shape
+    blocks, bw = weights.shape[1], weights.shape[2]
+    _f32(u, (T, width), "u")
+    _f32(weights, (2, blocks, bw, bw), "weights")
+    _f32(biases, (2, blocks, bw), "biases")
+    _f32(rate, (width,), "rate")
+    _f32(y_bias, (width,), "y_bias")
+    stride = _rows_view(y, "y")
+    _need(blocks * bw == width and y.shape == (T, width) and y.dtype == torch.float32 and out_dtype in _DT, "y must be float32 (T, width)")
+    B = _sequences(slots, cu_seqlens_q, state, width, "rglru_token")
+    _need(B == T and seq_index.dtype == torch.int32 and seq_index.shape == (T,), "one token a sequence, seq_index int32 (T,)")
+    out = torch.empty((T, width), dtype=out_dtype, device=u.device)
+    _check(library("recurrent").q3_rglru_token(
+        _ptr(u), _ptr(weights), _ptr(biases), _ptr(rate), _ptr(y), ctypes.c_long(stride), _ptr(y_bias), _ptr(state),
+        ctypes.c_long(state.stride(0)), _ptr(slots), _ptr(seq_index), _ptr(out), T, width, blocks, _DT[out_dtype], _stream()), "rglru_token")
     return out
 
 

@@ -76,6 +76,10 @@ class RecurrentUnit(Part):
         u = ops.causal_conv(both[:, w:], self.conv, self.conv_bias, cache.state[:, :tail], batch.state_slots,
                             batch.cu_seqlens_q, batch.seq_index, activation=None, out_dtype=torch.float32,
                             in_bias=self.bias_x, max_q_len=batch.max_q_len)
+        if ops.rglru_token_takes(u, u.shape[0], batch.state_slots.shape[0], batch.max_q_len, self.blocks):
+            return self.w_out.forward(ops.rglru_token(
+                u, self.gate_weights, self.gate_biases, self.decay_rate, both[:, :w], self.bias_y, cache.state[:, tail:],
+                batch.state_slots, batch.cu_seqlens_q, batch.seq_index, self.precision.act))
         gates = ops.block_gates(u, self.gate_weights, self.gate_biases)
         mixed = ops.rglru_scan(u, gates, self.decay_rate, both[:, :w], self.bias_y, cache.state[:, tail:],
                                batch.state_slots, batch.cu_seqlens_q, self.precision.act, max_q_len=batch.max_q_len)
