@@ -121,30 +121,48 @@ __global__ void qk_norm_rope_store_kernel(T* __restrict__ qkv, const W* __restri
 }
 
 // ---------------------------------------------------------------------------
-// The same work for bfloat16 with 16-byte accesses, for head sizes 16, 32, 64,
+// The same work with 16-byte accesses, for head sizes 16, 32, 64,
 // 128 and 256 with full or no rotation: a query or key head is served by D / 16
 // lanes, each holding eight elements of the head's first half and the eight
 // that pair with them in the second half; values are transposed page by page
-// through shared memory by a second kernel.
+// through shared memory by further blocks of the launch. Either type of storage: 336 float32 rows of 16 + 8 + 8 heads of 128 take 5.1 us,
+// 8.8 with a wavefront a head.
 // ---------------------------------------------------------------------------
+// Eight neighbouring numbers as they are stored.
+template <typename T>
+struct Eight {
+  union {
+    uint4 u[sizeof(T) / 2];
+    T e[8];
+  };
+  __device__ __forceinline__ void load(const T* p) {
+#pragma unroll
+    for (unsigned i = 0; i < sizeof(T) / 2; ++i) u[i] = reinterpret_cast<const uint4*>(p)[i];
+  }
+  __device__ __forceinline__ void store(T* p) const {
+#pragma unroll
+    for (unsigned i = 0; i < sizeof(T) / 2; ++i) reinterpret_cast<uint4*>(p)[i] = u[i];
+  }
+};
+
 // grid (T, ceil(heads / heads_per_block)), 256 threads; LPH = D / 16 lanes per head. With
 // STORE_V the value heads are handled here too, element by element into the transposed
 // cache (for steps of few tokens, where a second launch would cost more than it saves).
-template <typename W, int LPH, bool STORE_V>
+template <typename T, typename W, int LPH, bool STORE_V>
 __device__ __forceinline__ void qk_vec_body(
-    int t, int head_block, bf16_t* __restrict__ qkv, const W* __restrict__ q_weight, const W* __restrict__ k_weight,
+    int t, int head_block, T* __restrict__ qkv, const W* __restrict__ q_weight, const W* __restrict__ k_weight,
     float eps, const float* __restrict__ table, int max_pos, const int* __restrict__ positions,
     const int* __restrict__ seq_index, const int* __restrict__ block_table, int bt_stride, int bt_rows,
-    bf16_t* __restrict__ k_cache, bf16_t* __restrict__ v_cache, int page_size, int num_pages, int Hq, int Hkv) {
+    T* __restrict__ k_cache, T* __restrict__ v_cache, int page_size, int num_pages, int Hq, int Hkv) {
   constexpr int D = LPH * 16, HALF = D / 2;
   const int head = head_block * (256 / LPH) + threadIdx.x / LPH;
   const int c = threadIdx.x % LPH;  // which eight of the half
   if (head >= Hq + (STORE_V ? 2 : 1) * Hkv) return;
-  bf16_t* src = qkv + ((size_t)t * (Hq + 2 * Hkv) + head) * D;
+  T* src = qkv + ((size_t)t * (Hq + 2 * Hkv) + head) * D;
   const int pos = positions[t];
-  Half8 x1, x2;
-  x1.u = *reinterpret_cast<const uint4*>(src + 8 * c);
-  x2.u = *reinterpret_cast<const uint4*>(src + HALF + 8 * c);
+  Eight<T> x1, x2;
+  x1.load(src + 8 * c);
+  x2.load(src + HALF + 8 * c);
   if (STORE_V && head >= Hq + Hkv) {
     if (v_cache == nullptr) return;
     const int sq = seq_index[t];
@@ -152,7 +170,7 @@ __device__ __forceinline__ void qk_vec_body(
     if (sq < 0 || sq >= bt_rows || blk >= bt_stride || pos < 0) return;
     const int page = block_table[(size_t)sq * bt_stride + blk];
     if (page < 0 || page >= num_pages) return;
-    bf16_t* o = v_cache + ((size_t)page * Hkv + (head - Hq - Hkv)) * D * page_size + (pos % page_size);
+    T* o = v_cache + ((size_t)page * Hkv + (head - Hq - Hkv)) * D * page_size + (pos % page_size);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       o[(size_t)(8 * c + i) * page_size] = x1.e[i];
@@ -163,8 +181,8 @@ __device__ __forceinline__ void qk_vec_body(
   float a[8], b[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    a[i] = bf16_to_float(x1.e[i]);
-    b[i] = bf16_to_float(x2.e[i]);
+    a[i] = to_float(x1.e[i]);
+    b[i] = to_float(x2.e[i]);
   }
   const W* w = head < Hq ? q_weight : k_weight;
   if (w != nullptr) {
@@ -182,7 +200,7 @@ __device__ __forceinline__ void qk_vec_body(
     load_weights8<float>(table + (size_t)pos * D + HALF + 8 * c, sn);
     pairs_rotate(a, b, cs, sn);
   }
-  bf16_t* dst = src;
+  T* dst = src;
   if (head >= Hq) {
     dst = nullptr;
     if (k_cache != nullptr) {
@@ -198,20 +216,20 @@ __device__ __forceinline__ void qk_vec_body(
   if (dst == nullptr) return;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    x1.e[i] = float_to_bf16(a[i]);
-    x2.e[i] = float_to_bf16(b[i]);
+    x1.e[i] = from_float<T>(a[i]);
+    x2.e[i] = from_float<T>(b[i]);
   }
-  *reinterpret_cast<uint4*>(dst + 8 * c) = x1.u;
-  *reinterpret_cast<uint4*>(dst + HALF + 8 * c) = x2.u;
+  x1.store(dst + 8 * c);
+  x2.store(dst + HALF + 8 * c);
 }
 
-template <typename W, int LPH, bool STORE_V>
+template <typename T, typename W, int LPH, bool STORE_V>
 __global__ __launch_bounds__(256) void qk_norm_rope_store_vec_kernel(
-    bf16_t* __restrict__ qkv, const W* __restrict__ q_weight, const W* __restrict__ k_weight, float eps,
+    T* __restrict__ qkv, const W* __restrict__ q_weight, const W* __restrict__ k_weight, float eps,
     const float* __restrict__ table, int max_pos, const int* __restrict__ positions,
     const int* __restrict__ seq_index, const int* __restrict__ block_table, int bt_stride, int bt_rows,
-    bf16_t* __restrict__ k_cache, bf16_t* __restrict__ v_cache, int page_size, int num_pages, int Hq, int Hkv) {
-  qk_vec_body<W, LPH, STORE_V>(blockIdx.x, blockIdx.y, qkv, q_weight, k_weight, eps, table, max_pos, positions,
+    T* __restrict__ k_cache, T* __restrict__ v_cache, int page_size, int num_pages, int Hq, int Hkv) {
+  qk_vec_body<T, W, LPH, STORE_V>(blockIdx.x, blockIdx.y, qkv, q_weight, k_weight, eps, table, max_pos, positions,
                                seq_index, block_table, bt_stride, bt_rows, k_cache, v_cache, page_size, num_pages,
                                Hq, Hkv);
 }
@@ -221,11 +239,11 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_vec_kernel(
 // `page_size` (<= 64) tokens that fall in the page are staged in shared memory and
 // written as rows of the page, 16 bytes at a time where eight neighbouring slots
 // are all written in this step, element by element otherwise.
-template <int D>
+template <typename T, int D>
 __device__ __forceinline__ void store_values_body(
-    int span_page, int g, int b, bf16_t (*tile)[D + 8], const bf16_t* __restrict__ qkv,
+    int span_page, int g, int b, T (*tile)[D + 16 / sizeof(T)], const T* __restrict__ qkv,
     const int* __restrict__ cu_q, const int* __restrict__ kv_lens, const int* __restrict__ block_table,
-    int bt_stride, bf16_t* __restrict__ v_cache, int page_size, int num_pages, int Hq, int Hkv) {
+    int bt_stride, T* __restrict__ v_cache, int page_size, int num_pages, int Hq, int Hkv) {
   const int q0 = cu_q[b];
   const int q_len = cu_q[b + 1] - q0;
   if (q_len <= 0) return;
@@ -240,22 +258,24 @@ __device__ __forceinline__ void store_values_body(
   const int n = hi - lo;
   for (int idx = threadIdx.x; idx < n * (D / 8); idx += 256) {
     const int r = idx / (D / 8), c = idx % (D / 8);
-    const bf16_t* row = qkv + ((size_t)(q0 + lo - first_pos + r) * heads + Hq + Hkv + g) * D;
-    *reinterpret_cast<uint4*>(&tile[r][8 * c]) = *reinterpret_cast<const uint4*>(row + 8 * c);
+    const T* row = qkv + ((size_t)(q0 + lo - first_pos + r) * heads + Hq + Hkv + g) * D;
+    Eight<T> h;
+    h.load(row + 8 * c);
+    h.store(&tile[r][8 * c]);
   }
   __syncthreads();
   const int slot_lo = lo - blk * page_size;
-  bf16_t* base = v_cache + ((size_t)page * Hkv + g) * D * page_size;
+  T* base = v_cache + ((size_t)page * Hkv + g) * D * page_size;
   const int groups = page_size / 8;  // 16-byte groups of slots per row (page_size is a multiple of 8 here)
   for (int idx = threadIdx.x; idx < D * groups; idx += 256) {
     const int d = idx / groups, s8 = (idx % groups) * 8;
     if (s8 + 8 <= slot_lo || s8 >= slot_lo + n) continue;
-    bf16_t* o = base + (size_t)d * page_size + s8;
+    T* o = base + (size_t)d * page_size + s8;
     if (s8 >= slot_lo && s8 + 8 <= slot_lo + n) {
-      Half8 h;
+      Eight<T> h;
 #pragma unroll
       for (int i = 0; i < 8; ++i) h.e[i] = tile[s8 - slot_lo + i][d];
-      *reinterpret_cast<uint4*>(o) = h.u;
+      h.store(o);
     } else {
       for (int i = 0; i < 8; ++i) {
         const int r = s8 + i - slot_lo;
@@ -269,25 +289,25 @@ __device__ __forceinline__ void store_values_body(
 // (span_pages x Hkv x B of them) transpose values, the others prepare queries and keys. The
 // two touch different parts of qkv and different caches, so they need no order, and a launch
 // of its own for the values, which is short on work per block, would only add its latency.
-template <typename W, int LPH>
+template <typename T, typename W, int LPH>
 __global__ __launch_bounds__(256) void qk_and_values_kernel(
-    bf16_t* __restrict__ qkv, const W* __restrict__ q_weight, const W* __restrict__ k_weight, float eps,
+    T* __restrict__ qkv, const W* __restrict__ q_weight, const W* __restrict__ k_weight, float eps,
     const float* __restrict__ table, int max_pos, const int* __restrict__ positions,
     const int* __restrict__ seq_index, const int* __restrict__ block_table, int bt_stride, int bt_rows,
-    bf16_t* __restrict__ k_cache, bf16_t* __restrict__ v_cache, int page_size, int num_pages, int Hq, int Hkv,
+    T* __restrict__ k_cache, T* __restrict__ v_cache, int page_size, int num_pages, int Hq, int Hkv,
     const int* __restrict__ cu_q, const int* __restrict__ kv_lens, int span_pages, int value_blocks,
     int head_blocks) {
   constexpr int D = LPH * 16;
-  __shared__ bf16_t tile[64][D + 8];
+  __shared__ __attribute__((aligned(16))) T tile[64][D + 16 / sizeof(T)];
   int id = blockIdx.x;
   if (id < value_blocks) {
     const int span_page = id % span_pages, g = (id / span_pages) % Hkv, b = id / (span_pages * Hkv);
-    store_values_body<D>(span_page, g, b, tile, qkv, cu_q, kv_lens, block_table, bt_stride, v_cache, page_size,
+    store_values_body<T, D>(span_page, g, b, tile, qkv, cu_q, kv_lens, block_table, bt_stride, v_cache, page_size,
                          num_pages, Hq, Hkv);
     return;
   }
   id -= value_blocks;
-  qk_vec_body<W, LPH, false>(id / head_blocks, id % head_blocks, qkv, q_weight, k_weight, eps, table, max_pos,
+  qk_vec_body<T, W, LPH, false>(id / head_blocks, id % head_blocks, qkv, q_weight, k_weight, eps, table, max_pos,
                              positions, seq_index, block_table, bt_stride, bt_rows, k_cache, v_cache, page_size,
                              num_pages, Hq, Hkv);
 }
@@ -329,7 +349,7 @@ static int launch_qk(void* qkv, const void* qw, const void* kw, float eps, const
   return q3_launch_status();
 }
 
-template <typename W>
+template <typename T, typename W>
 static int launch_qk_vec(void* qkv, const void* qw, const void* kw, float eps, const float* table, int max_pos,
                          const int* positions, const int* seq_index, const int* block_table, int bt_stride,
                          int bt_rows, void* k_cache, void* v_cache, int page_size, int num_pages, int T_, int Hq,
@@ -346,19 +366,19 @@ static int launch_qk_vec(void* qkv, const void* qw, const void* kw, float eps, c
     if (values_apart) {                                                                                       \
       const long blocks = value_blocks + (long)T_ * head_blocks;                                              \
       if (blocks > 0x7fffffffL) return Q3_ERR_UNSUPPORTED;                                                    \
-      hipLaunchKernelGGL((qk_and_values_kernel<W, LPH>), dim3((unsigned)blocks), dim3(256), 0, stream,        \
-                         (bf16_t*)qkv, (const W*)qw, (const W*)kw, eps, table, max_pos, positions, seq_index, \
-                         block_table, bt_stride, bt_rows, (bf16_t*)k_cache, (bf16_t*)v_cache, page_size,      \
+      hipLaunchKernelGGL((qk_and_values_kernel<T, W, LPH>), dim3((unsigned)blocks), dim3(256), 0, stream,        \
+                         (T*)qkv, (const W*)qw, (const W*)kw, eps, table, max_pos, positions, seq_index, \
+                         block_table, bt_stride, bt_rows, (T*)k_cache, (T*)v_cache, page_size,      \
                          num_pages, Hq, Hkv, cu_q, kv_lens, span_pages, (int)value_blocks, head_blocks);      \
     } else if (few) {                                                                                         \
-      hipLaunchKernelGGL((qk_norm_rope_store_vec_kernel<W, LPH, true>), dim3(T_, head_blocks), dim3(256), 0,  \
-                         stream, (bf16_t*)qkv, (const W*)qw, (const W*)kw, eps, table, max_pos, positions,    \
-                         seq_index, block_table, bt_stride, bt_rows, (bf16_t*)k_cache, (bf16_t*)v_cache,      \
+      hipLaunchKernelGGL((qk_norm_rope_store_vec_kernel<T, W, LPH, true>), dim3(T_, head_blocks), dim3(256), 0,  \
+                         stream, (T*)qkv, (const W*)qw, (const W*)kw, eps, table, max_pos, positions,    \
+                         seq_index, block_table, bt_stride, bt_rows, (T*)k_cache, (T*)v_cache,      \
                          page_size, num_pages, Hq, Hkv);                                                      \
     } else {                                                                                                  \
-      hipLaunchKernelGGL((qk_norm_rope_store_vec_kernel<W, LPH, false>), dim3(T_, head_blocks), dim3(256), 0, \
-                         stream, (bf16_t*)qkv, (const W*)qw, (const W*)kw, eps, table, max_pos, positions,    \
-                         seq_index, block_table, bt_stride, bt_rows, (bf16_t*)k_cache, (bf16_t*)v_cache,      \
+      hipLaunchKernelGGL((qk_norm_rope_store_vec_kernel<T, W, LPH, false>), dim3(T_, head_blocks), dim3(256), 0, \
+                         stream, (T*)qkv, (const W*)qw, (const W*)kw, eps, table, max_pos, positions,    \
+                         seq_index, block_table, bt_stride, bt_rows, (T*)k_cache, (T*)v_cache,      \
                          page_size, num_pages, Hq, Hkv);                                                      \
     }                                                                                                         \
   } while (0)
@@ -391,13 +411,16 @@ extern "C" int q3_qk_norm_rope_store(void* qkv, const void* q_weight, const void
   if (k_cache && (!v_cache || !block_table || page_size <= 0)) return Q3_ERR_BAD_ARGUMENT;
   if ((q_weight == nullptr) != (k_weight == nullptr)) return Q3_ERR_BAD_ARGUMENT;
   const bool pow2_head = D == 16 || D == 32 || D == 64 || D == 128 || D == 256;
-  const bool vec = act_dtype == Q3_BF16 && pow2_head && (!table || rotary_dim == D) &&
+  // (float32 rows, weights and caches that begin off sixteen bytes stay with the general kernel)
+  const bool aligned = act_dtype == Q3_BF16 || (((size_t)qkv | (size_t)q_weight | (size_t)k_weight | (size_t)table | (size_t)k_cache |
+                                                 (size_t)v_cache) & 15) == 0;
+  const bool vec = aligned && pow2_head && (!table || rotary_dim == D) &&
                    (!k_cache || (cu_q && kv_lens && B > 0 && B <= 65535 && max_q_len > 0 && page_size % 8 == 0 &&
                                  page_size <= 64));
   if (vec) {
-    Q3_DISPATCH_DTYPE(w_dtype, WW, return (launch_qk_vec<WW>(
+    Q3_DISPATCH_DTYPE(act_dtype, TT, Q3_DISPATCH_DTYPE(w_dtype, WW, return (launch_qk_vec<TT, WW>(
         qkv, q_weight, k_weight, eps, table, max_pos, positions, seq_index, block_table, bt_stride, bt_rows,
-        k_cache, v_cache, page_size, num_pages, T_, Hq, Hkv, D, cu_q, kv_lens, B, max_q_len, stream)));
+        k_cache, v_cache, page_size, num_pages, T_, Hq, Hkv, D, cu_q, kv_lens, B, max_q_len, stream))));
   }
   Q3_DISPATCH_DTYPE(act_dtype, TT, Q3_DISPATCH_DTYPE(w_dtype, WW, return (launch_qk<TT, WW>(
       qkv, q_weight, k_weight, eps, table, rotary_dim, max_pos, positions, seq_index, block_table,

@@ -1627,7 +1627,7 @@ def qk_norm_rope_store(qkv, num_q_heads, num_kv_heads, head_dim, positions, seq_
     rotation are each skipped when their operand is None. The rotation pairs
     element i with i + R/2 over the first R = table.shape[1] elements.
     `cu_seqlens_q`, `kv_lens` (after this step's write) and `max_q_len`
-    describe the step's sequences; with them, bfloat16 steps use kernels with
+    describe the step's sequences; with them, steps use kernels with
     16-byte accesses that write values page by page. positions must then be
     kv_lens[b] - q_len[b] + i for row i of sequence b, as the step function
     makes them. `max_kv_len`: the step's last position + 1, if the caller knows it;
