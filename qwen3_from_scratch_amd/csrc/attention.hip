@@ -163,14 +163,17 @@ static int launch_general(const void* q, int q_stride, void* out, const void* k_
 //
 //   S^T (keys x rows) = K . Q^T, O^T (d x rows) += V^T . P^T: the row is the lane's low four bits in both.
 //
-// Lane group g holds d = 16 c + 4 g .. + 3 of its key and of its row as one 16-byte load each and step s multiplies
-// the four d = 16 c + 4 g + s; it then has the scores of keys 4 g .. 4 g + 3, which the values' 16-byte loads (the
-// cache is transposed within the page) match in the same way. Nothing passes through shared memory but the
-// eight results at the end.
+// Lane group g holds d = 16 c + 4 g .. + 3 of its key and of its row as 16 bytes each and step s multiplies
+// the four d = 16 c + 4 g + s; it then has the scores of keys 4 g .. 4 g + 3, which the values' 16 bytes (the
+// cache is transposed within the page) match in the same way. So neighbouring lanes hold neighbouring rows, but they load
+// neighbouring pieces of one row, 64 bytes by four lanes, and change places through shared memory, a wavefront for itself: loads
+// whose neighbouring lanes are rows apart kept the CU's address path busy four times as long, and bound the kernel with its eight
+// wavefronts' 24 loads a tile.
 //
-// Bound by the wait for keys and values from the L2 and by the chain from scores to probabilities; the kernel
-// above, 16 rows of one head a block, read two numbers from shared memory per multiply-add. Two prompts of 111 and
-// 222 tokens beside three single tokens behind up to 150, 16 heads over 8 of 128: 177 us there, 22 here.
+// The kernel above, 16 rows of one head a block, read two numbers from shared memory per multiply-add. Two prompts of 111 and
+// 222 tokens beside three single tokens behind up to 150, 16 heads over 8 of 128: 177 us there, 22 with loads in the lanes' order of
+// use, 20.4 here; a prompt of 2,000 308 and 274, four requests over 3,000 96 and 86. What bounds it now is the float32 matrix
+// instruction (64 of them a tile, 32 cycles each) and the chain from scores to probabilities: the next tile on its way ahead gave nothing.
 // ---------------------------------------------------------------------------
 typedef __attribute__((ext_vector_type(4))) float f32_four;
 
@@ -183,7 +186,12 @@ __global__ __launch_bounds__(512) void attn_f32_mma_kernel(
     const int* __restrict__ cu_q, const int* __restrict__ kv_lens, int Hq, int Hkv, int page, float scale, int window,
     const float* __restrict__ sink, int tokens_per_block) {
   constexpr int C = D / 16, LD = D + 4;
-  __shared__ float part[4][16][LD], sh_m[8][16], sh_l[8][16];
+  __shared__ union {
+    float part[4][16][LD];
+    f32_four turn[8][C][64];      // a wavefront's pieces on their way from the lane that loads to the lane that uses
+  } shared;
+  float (&part)[4][16][LD] = shared.part;
+  __shared__ float sh_m[8][16], sh_l[8][16];
   const int b = blockIdx.z, g_kv = blockIdx.y, G = Hq / Hkv;
   const int q0 = cu_q[b], q_len = cu_q[b + 1] - q0;
   const int t0 = blockIdx.x * tokens_per_block;
@@ -195,13 +203,33 @@ __global__ __launch_bounds__(512) void attn_f32_mma_kernel(
   const bool my_row = col < rows;
   const int my_pos = my_row ? first_pos + t0 + col / G : -1;
 
-  f32_four qr[C], acc[C];
+  // piece p of row r is loaded by lane 4 r + p and used by lane 16 p + r; its place keeps eight neighbouring readers in different banks
+  const int from_row = lane >> 2, from_piece = lane & 3;
+  f32_four* put = &shared.turn[wave][0][4 * from_row + ((from_piece + (from_row >> 2)) & 3)];
+  const f32_four* take = &shared.turn[wave][0][4 * col + ((grp + (col >> 2)) & 3)];
+  auto turned = [&](f32_four (&x)[C]) {
 #pragma unroll
-  for (int c = 0; c < C; ++c) {
-    qr[c] = f32_four{0.f, 0.f, 0.f, 0.f};
-    acc[c] = f32_four{0.f, 0.f, 0.f, 0.f};
-    if (my_row)
-      qr[c] = load_four(q + (size_t)(q0 + t0 + col / G) * q_stride + (size_t)(g_kv * G + col % G) * D + 16 * c + 4 * grp);
+    for (int c = 0; c < C; ++c) put[64 * c] = x[c];
+    // (the wavefront's own: its reads follow its writes)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int c = 0; c < C; ++c) x[c] = take[64 * c];
+    __builtin_amdgcn_wave_barrier();
+  };
+  f32_four qr[C], acc[C];
+  {
+    const bool row = from_row < rows;
+    const float* at = q + (size_t)(q0 + t0 + (row ? from_row / G : 0)) * q_stride + (size_t)(g_kv * G + (row ? from_row % G : 0)) * D +
+                      4 * from_piece;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      qr[c] = load_four(at + 16 * c);
+      if (!row) qr[c] = f32_four{0.f, 0.f, 0.f, 0.f};
+      acc[c] = f32_four{0.f, 0.f, 0.f, 0.f};
+    }
+    turned(qr);
   }
   float m_run = -INFINITY, l_run = 0.f;
 
@@ -213,18 +241,20 @@ __global__ __launch_bounds__(512) void attn_f32_mma_kernel(
     const int pg = block_table[(size_t)b * bt_stride + key0 / page];
     const bool there = pg >= 0 && pg < num_pages;   // (a page given back counts as zeros; nobody sees it)
     const size_t base = ((size_t)(there ? pg : 0) * Hkv + g_kv) * page * D;
-    const float* kp = k_cache + base + (size_t)(key0 % page + col) * D + 4 * grp;
-    const float* vp = v_cache + base + (size_t)col * page + key0 % page + 4 * grp;
+    const float* kp = k_cache + base + (size_t)(key0 % page + from_row) * D + 4 * from_piece;
+    const float* vp = v_cache + base + (size_t)from_row * page + key0 % page + 4 * from_piece;
     f32_four kr[C], vr[C];
 #pragma unroll
     for (int c = 0; c < C; ++c) kr[c] = there ? load_four(kp + 16 * c) : f32_four{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int c = 0; c < C; ++c) vr[c] = there ? load_four(vp + (size_t)16 * c * page) : f32_four{0.f, 0.f, 0.f, 0.f};
+    turned(kr);
     f32_four s4 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int c = 0; c < C; ++c)
 #pragma unroll
       for (int i = 0; i < 4; ++i) s4 = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[c][i], qr[c][i], s4, 0, 0, 0);
+    turned(vr);
     const int my_key = key0 + 4 * grp;
     if (key0 + 16 > k_end) {                        // what lies behind the sequence's end may be anything
 #pragma unroll
@@ -263,7 +293,7 @@ __global__ __launch_bounds__(512) void attn_f32_mma_kernel(
     sh_m[wave][col] = m_run;
     sh_l[wave][col] = l_run;
   }
-  __syncthreads();
+  __syncthreads();      // (and no wavefront's pieces are on their way any more)
   float top = sh_m[0][col];
 #pragma unroll
   for (int w = 1; w < 8; ++w) top = fmaxf(top, sh_m[w][col]);
