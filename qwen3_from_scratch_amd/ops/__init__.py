@@ -55,6 +55,9 @@ __all__ = [
     "mamba2_token",
     "mamba2_token_takes",
     "rglru_token",
+    "narrow_gates",
+    "rglru_rows",
+    "rglru_rows_take",
     "rglru_token_takes",
     "block_gates",
     "rglru_scan",
@@ -1134,6 +1137,50 @@ def rglru_token(u, weights, biases, rate, y, y_bias, state, slots, cu_seqlens_q,
     _check(library("recurrent").q3_rglru_token(
         _ptr(u), _ptr(weights), _ptr(biases), _ptr(rate), _ptr(y), ctypes.c_long(stride), _ptr(y_bias), _ptr(state),
         ctypes.c_long(state.stride(0)), _ptr(slots), _ptr(seq_index), _ptr(out), T, width, blocks, _DT[out_dtype], _stream()), "rglru_token")
+    return out
+
+
+def narrow_gates(weights):
+    """The weights of `block_gates`, (2, blocks, in, out) float32 on the GPU, in bfloat16 and in the order in which `rglru_rows` reads them, or
+    None where bfloat16 does not hold them exactly or the parts are of other sizes than it takes."""
+    if not weights.is_cuda or weights.dtype != torch.float32 or weights.shape[2] not in (32, 64, 128, 256):
+        return None
+    copy = weights.to(torch.bfloat16)
+    if bool((weights - copy).any()):          # (an infinity's or a NaN's difference is a NaN)
+        return None
+    g, blocks, bw, _ = weights.shape
+    # (in, out) -> (16 outputs, 32 inputs, [8 inputs, output] = lane, eight inputs)
+    return copy.view(g, blocks, bw // 32, 4, 8, bw // 16, 16).permute(0, 1, 5, 2, 3, 6, 4).contiguous()
+
+
+def rglru_rows_take(u, narrow, max_q_len):
+    """Whether `rglru_rows` takes a step: sequences of more than 64 rows, and weights that `narrow_gates` took."""
+    return narrow is not None and max_q_len > 64 and u.data_ptr() % 16 == 0
+
+
+def rglru_rows(u, narrow, biases, rate, y, y_bias, state, slots, cu_seqlens_q, out_dtype, max_q_len):
+    """`block_gates` and `rglru_scan` of a step of many rows: every segment of 32 rows with its gates in one kernel, joined in a second.
+    `narrow`: the gates' weights as `narrow_gates` gives them."""
+    _dev(u, narrow, biases, rate, y_bias)
+    T, width = u.shape
+    blocks = narrow.shape[1]
+    _f32(u, (T, width), "u")
+    _need(narrow.dtype == torch.bfloat16 and narrow.numel() == 2 * width * (width // blocks), "narrow must be what narrow_gates gives")
+    _f32(biases, (2, blocks, width // blocks), "biases")
+    _f32(rate, (width,), "rate")
+    _f32(y_bias, (width,), "y_bias")
+    stride = _rows_view(y, "y")
+    _need(y.shape == (T, width) and y.dtype == torch.float32 and out_dtype in _DT, "y must be float32 (T, width)")
+    B = _sequences(slots, cu_seqlens_q, state, width, "rglru_rows")
+    out = torch.empty((T, width), dtype=out_dtype, device=u.device)
+    if T:
+        lib = library("rglru")
+        lib.q3_rglru_rows_workspace.restype = ctypes.c_long
+        work = torch.empty(lib.q3_rglru_rows_workspace(T, B, width), dtype=torch.float32, device=u.device)
+        _check(lib.q3_rglru_rows(
+            _ptr(u), _ptr(narrow), _ptr(biases), _ptr(rate), _ptr(y), ctypes.c_long(stride), _ptr(y_bias), _ptr(state),
+            ctypes.c_long(state.stride(0)), _ptr(slots), _ptr(cu_seqlens_q), _ptr(out), _ptr(work), T, B, int(max_q_len), width, blocks,
+            _DT[out_dtype], _stream()), "rglru_rows")
     return out
 
 

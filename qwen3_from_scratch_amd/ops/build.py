@@ -31,7 +31,7 @@ FLAGS = [
     "-Wno-unused-command-line-argument",
 ]
 MODULES = ("elementwise", "norm", "rotary", "attention", "attention_capped", "attention_pooled", "attention_sigmoid", "attention_span", "latent", "moe",
-           "hyper", "recurrent", "mamba2", "mlstm", "delta", "softcap", "gemm", "matmul", "sampling", "probes", "layers", "decode_layers")
+           "hyper", "recurrent", "mamba2", "rglru", "mlstm", "delta", "softcap", "gemm", "matmul", "sampling", "probes", "layers", "decode_layers")
 # A module's further sources, compiled on their own: their kernels are code objects of their own in its library. Where a kernel's
 # code lies decides how long a launch of it takes to get going: with the kernels of these two between those of matmul.hip, the
 # tiled and the weight-streaming product of a step of 64 requests of the 8B shape took 11.7 and 39.9 us with the instructions

@@ -33,7 +33,7 @@ class RecurrentUnit(Part):
                              % (width // blocks, conv))
         self.hidden_size, self.width, self.blocks, self.taps, self.rate = hidden_size, width, blocks, conv, float(rate)
         self.w_in = self.w_out = self.bias_y = self.bias_x = self.conv = self.conv_bias = None
-        self.gate_weights = self.gate_biases = self.decay_rate = None
+        self.gate_weights = self.gate_biases = self.decay_rate = self.narrow_gates = None
 
     def _tail(self):
         return (self.taps - 1) * self.width
@@ -65,6 +65,7 @@ class RecurrentUnit(Part):
         # the gates' matrices as (gate, block, in, out), so that neighbouring threads read neighbouring numbers
         gates = torch.stack((fetch(self._name("ra"), torch.float32), fetch(self._name("ri"), torch.float32)))
         self.gate_weights = gates.transpose(2, 3).contiguous()
+        self.narrow_gates = ops.narrow_gates(self.gate_weights)
         self.gate_biases = torch.stack((fetch(self._name("ra.b"), torch.float32),
                                         fetch(self._name("ri.b"), torch.float32))).contiguous()
         lam = fetch(self._name("lam"), torch.float32).double()
@@ -80,6 +81,10 @@ class RecurrentUnit(Part):
             return self.w_out.forward(ops.rglru_token(
                 u, self.gate_weights, self.gate_biases, self.decay_rate, both[:, :w], self.bias_y, cache.state[:, tail:],
                 batch.state_slots, batch.cu_seqlens_q, batch.seq_index, self.precision.act))
+        if ops.rglru_rows_take(u, self.narrow_gates, batch.max_q_len):
+            return self.w_out.forward(ops.rglru_rows(
+                u, self.narrow_gates, self.gate_biases, self.decay_rate, both[:, :w], self.bias_y, cache.state[:, tail:],
+                batch.state_slots, batch.cu_seqlens_q, self.precision.act, batch.max_q_len))
         gates = ops.block_gates(u, self.gate_weights, self.gate_biases)
         mixed = ops.rglru_scan(u, gates, self.decay_rate, both[:, :w], self.bias_y, cache.state[:, tail:],
                                batch.state_slots, batch.cu_seqlens_q, self.precision.act, max_q_len=batch.max_q_len)
