@@ -55,11 +55,15 @@ class CacheStorage:
         return sum(t.numel() * t.element_size() for t in tensors)
 
     def clear_fresh_slots(self):
-        fresh, self.manager.fresh_slots = self.manager.fresh_slots, []
-        if fresh and self.states:
-            index = torch.tensor(fresh, dtype=torch.long, device=self.device)
-            for t in self.states:
-                t[:, index] = 0
+        """Zeros in the slots handed out since the last call, a fill for each run of neighbouring ones: an index or a zero that came
+        from the host would have the host wait for all that the device still has to do."""
+        fresh, self.manager.fresh_slots = sorted(set(self.manager.fresh_slots)), []
+        first = 0
+        for i, slot in enumerate(fresh):
+            if i + 1 == len(fresh) or fresh[i + 1] != slot + 1:
+                for t in self.states:
+                    t[:, fresh[first]:slot + 1].zero_()
+                first = i + 1
 
     def keep_states(self, slots):
         """Copies of the states in `slots` (a device tensor of slot numbers), to be put back by
