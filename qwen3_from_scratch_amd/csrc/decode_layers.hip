@@ -10,11 +10,12 @@
 // block). The weights of a product's first steps are asked for while the last one's results are on their way, so memory is not idle
 // meanwhile.
 //
-// What it measured (us a step in a graph, the layers' kernels one by one / this): the 0.6B shape, one request over 100 keys 978 / 506,
-// over 1,100 1,014 / 563, over 8,000 1,149 / 753, over 30,000 1,540 / 1,139, four over 1,100 1,134 / 646, eight over 2,000 1,407 / 915,
-// sixteen 1,886 / 1,341, 20 over 770 1,412 / 1,150, 32 over 2,000 2,414 / 2,147; the 8B shape, one over 2,060 3,383 / 2,768, eight
-// 3,926 / 3,331, sixteen 4,818 / 4,171, eight over 8,000 5,043 / 4,423. Faster at each of 39 sizes of these two from 1 to 32 rows (16) and 100 to
-// 30,000 keys, all contexts alike, by 3 percent (32 over 8,000) to 93; uneven ones: `share_out`; other shapes: `rows_most`.
+// What it measured (us a step in a graph, the layers' kernels one by one / this): the 0.6B shape, one request over 100 keys 973 / 504,
+// over 1,100 1,013 / 563, over 8,000 1,137 / 758, over 30,000 1,531 / 1,138, four over 1,100 1,145 / 623, eight over 2,000 1,412 / 876,
+// sixteen 1,921 / 1,273, 20 over 770 1,433 / 990, 32 over 2,000 2,410 / 1,916; the 8B shape, one over 2,060 3,382 / 2,769, eight
+// 3,923 / 3,157, sixteen 4,843 / 3,799, eight over 8,000 5,179 / 4,166, sixteen 6,773 / 5,802. With rows in one piece each (`place_of`) it was
+// faster at each of 39 sizes of these two from 1 to 32 rows (16) and 100 to 30,000 keys, all contexts alike, by 3 percent (32 over 8,000)
+// to 93; uneven ones: `share_out`; other shapes: `rows_most`.
 //
 // What bounds it: one request of the small shape the chain of five or six exchanges a layer; a look that fails costs a second one behind
 // the first, a store holds up the wavefront's next look (they come back in order), and a wavefront alone on its SIMD takes 4 to 5 cycles
@@ -153,6 +154,18 @@ __device__ __forceinline__ float other_half(float v, int lane) {
   return __uint_as_float(lane < 32 ? a[1] : a[0]);
 }
 
+// Where numbers k .. of row `row`, of `width`, lie among what a product multiplies with, in bytes: `turned` rows (1, 2, 4, 8, 16, as many
+// as hold the step's or 16) side by side, a row's eight numbers followed by the next row's, as the lanes of a matrix instruction take
+// them. Neighbouring lanes then look at neighbouring places, where with each row in one piece a look cost a CU's address path up to four
+// times as long, and lines of memory by rows. Rows in one piece each / side by side, us a step: the 0.6B shape over 1,000 keys, two 592 / 577,
+// four 637 / 615, eight 746 / 690, sixteen 919 / 829, 20 1,214 / 1,058, 32 over 2,000 1,953 / 1,726; the 8B shape, four over 1,000
+// 2,888 / 2,842, eight over 2,000 3,179 / 3,005, sixteen over 1,000 3,591 / 3,202.
+__host__ __device__ __forceinline__ int place_of(int turned, int row, int k, int width) {
+  if (turned == 1) return (row * width + k) * 2;
+  const unsigned rest = (unsigned)row % (unsigned)turned;
+  return (row - (int)rest) * width * 2 + (k >> 3) * (16 * turned) + (int)rest * 16 + (k & 7) * 2;
+}
+
 // Until shared memory holds what the block's wavefronts have written (and nothing about memory)
 __device__ __forceinline__ void meet() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
@@ -268,7 +281,7 @@ __device__ __forceinline__ void gave_up(const Args& a) {
   compiler_fence();
 }
 
-template <typename QKW, int GROUPS, bool MANY>
+template <typename QKW, int GROUPS, int TURNED>
 struct Block {
   Shared& sh;
   const Args& a;
@@ -281,6 +294,7 @@ struct Block {
   unsigned rows_inverse;
   int held;                    // the product whose first weights are on their way: four times its layer, and which
   static constexpr int STEPS = CHUNKS / GROUPS;          // kilobytes of weights that a wavefront has on their way
+  static constexpr int STEP_BYTES = 64 * TURNED;            // from a lane's numbers of one step of K to those of the next
   u32x4_t w[STEPS];            // they
 
   // (as a number of its own: what is computed from it is not kept in registers over the whole launch)
@@ -368,12 +382,12 @@ struct Block {
   __device__ __forceinline__ static void look(u32x4_t (&x)[CHUNKS], const Rows& r, int i, int left) {
 #pragma unroll
     for (int g = 0; g < GROUPS; ++g) {
-      const int at = anew(r.at[g] + 64 * i);
+      const int at = anew(r.at[g] + STEP_BYTES * i);
 #pragma unroll
       for (int quarter = 0; quarter < N / 4; ++quarter) {
-        const int from = N < STEPS || quarter == 0 || left > 4 * quarter ? at : NOWHERE;
+        const int from = (N < STEPS || quarter == 0 || left > 4 * quarter ? at : NOWHERE) + 4 * STEP_BYTES * quarter;
 #pragma unroll
-        for (int j = 4 * quarter; j < 4 * quarter + 4; ++j) x[N * g + j] = peek16(r.ex, from + 64 * j, r.src);
+        for (int j = 0; j < 4; ++j) x[N * g + 4 * quarter + j] = peek16(r.ex, from + STEP_BYTES * j, r.src);
       }
       if (left < N && (left == 0 || left & 3)) {
 #pragma unroll
@@ -396,7 +410,7 @@ struct Block {
     // One look at one place first: so many rows asked for again and again hold up those that write them. From four rows on (the 0.6B shape,
     // four over 1,100 keys 638 us, without 663, six over 500 649 and 694; the 8B shape, two 2,829 with it, 2,819 without).
     if (i == 0 && a.rows >= 4 && left > 0) {
-      const int place = __builtin_amdgcn_readfirstlane(r.at[0]) + 64 * (min(left, N) - 1);
+      const int place = __builtin_amdgcn_readfirstlane(r.at[0]) + STEP_BYTES * (min(left, N) - 1);
       for (int n = 0;; ++n) {
         compiler_fence();
         const u32x4_t v = peek16(r.ex, place, r.src);
@@ -406,7 +420,7 @@ struct Block {
     bool have = false;
     for (int n = 0;; ++n) {
       compiler_fence();
-      if (!MANY || !have) {
+      if (TURNED < 8 || !have) {
         look<N>(x, r, i, left);
         have = all_there<N>(x);
       }
@@ -603,7 +617,7 @@ struct Block {
             ss += x[e] * x[e];
             pk.e[e] = (__bf16)(x[e] * w4[e]);
           }
-          put8(ex, dst + (row * width + n) * 2, pk.u);
+          put8(ex, dst + place_of(TURNED, row, n, width), pk.u);
           ss += quad_xor<1>(ss);
           ss += quad_xor<2>(ss);
           if (grp == 0) put4(ex, number(which, DST_SUMS) + (row * (width / 16) + slab) * 4, __float_as_uint(ss), 0x7fc00000u);
@@ -618,7 +632,7 @@ struct Block {
             const float g = (float)(__bf16)acc[2 * e], u = (float)(__bf16)acc[2 * e + 1];
             pk.e[e] = (__bf16)(gate_value<0>(g) * u);
           }
-          put4(ex, dst + (row * width + n / 2) * 2, pk.u.x, 0x7fc07fc0u);
+          put4(ex, dst + place_of(TURNED, row, n / 2, width), pk.u.x, 0x7fc07fc0u);
         } else {
 #pragma unroll
           for (int e = 0; e < 4; ++e) pk.e[e] = (__bf16)acc[e];
@@ -884,7 +898,7 @@ struct Block {
         } pk;
 #pragma unroll
         for (int e = 0; e < 4; ++e) pk.e[e] = (__bf16)(o[e] * inv);
-        put8(ex, a.at_att + ((b * a.heads + g_kv * G + row) * D + d) * 2, pk.u);
+        put8(ex, a.at_att + place_of(TURNED, b, (g_kv * G + row) * D + d, a.heads * D), pk.u);
       } else {
         const int slot = it.n * G + row;
         u32x4_t p;
@@ -958,7 +972,7 @@ struct Block {
       } pk;
 #pragma unroll
       for (int e = 0; e < 4; ++e) pk.e[e] = (__bf16)(o[e] * inv);
-      if (idx < G * (D / 4)) put8(ex, a.at_att + ((b * a.heads + g_kv * G + r) * D + d) * 2, pk.u);
+      if (idx < G * (D / 4)) put8(ex, a.at_att + place_of(TURNED, b, (g_kv * G + r) * D + d, a.heads * D), pk.u);
     }
   }
 
@@ -1016,7 +1030,8 @@ struct Block {
         r.sums = number(which, SUMS);
 #pragma unroll
         for (int g = 0; g < GROUPS; ++g)
-          r.at[g] = col + 16 * g < a.rows ? (col + 16 * g) * number(which, ROW_BYTES) + 64 * number(which, FIRST_STEP) + 16 * (lane >> 4) : NOWHERE;
+          r.at[g] = col + 16 * g >= a.rows ? NOWHERE
+                    : g * 16 * number(which, ROW_BYTES) + STEP_BYTES * number(which, FIRST_STEP) + 16 * (TURNED * (lane >> 4) + col);
         const uint64_t eps = entry(n, EPS);
         r.eps = __uint_as_float((unsigned)(which == 0 ? eps : eps >> 32));
         // (the last layer's down product prepares no rows: its norm is the one behind the layers, of another kernel)
@@ -1077,7 +1092,7 @@ __device__ __forceinline__ void gather(const Args& a, int& rank, int& blocks) {
   }
 }
 
-template <typename QKW, int GROUPS, bool MANY>
+template <typename QKW, int GROUPS, int TURNED>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void decode_layers_kernel(Args a) {
   __shared__ Shared sh;
   if (threadIdx.x == 0) {
@@ -1091,7 +1106,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
   for (int i = threadIdx.x; i < a.count * LAYER_WORDS; i += THREADS) sh.layers[i] = reinterpret_cast<const uint64_t*>(a.layers)[i];
   __syncthreads();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  Block<QKW, GROUPS, MANY> b{sh, a, rank, blocks, wave, (int)threadIdx.x & 63, (int)threadIdx.x, numbers_of(a, rank, blocks, wave, threadIdx.x & 63),
+  Block<QKW, GROUPS, TURNED> b{sh, a, rank, blocks, wave, (int)threadIdx.x & 63, (int)threadIdx.x, numbers_of(a, rank, blocks, wave, threadIdx.x & 63),
                   min(MOST_SLABS, RESULTS / a.rows), a.limit, 1, (1u << 20) / a.rows + 1, -1};
   b.layers();
 }
@@ -1103,7 +1118,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
 struct Entry {
   const float* residual;
   const void* norm;
-  int rows, width, norm_f32;
+  int rows, width, norm_f32, turned;
   char *out, *sums;
 };
 struct Blank {
@@ -1157,7 +1172,8 @@ __global__ __launch_bounds__(256) void decode_layers_begin_kernel(LayerPack pack
       __bf16 e[4];
     } pk;
     pk.e[0] = (__bf16)(x.x * w.x), pk.e[1] = (__bf16)(x.y * w.y), pk.e[2] = (__bf16)(x.z * w.z), pk.e[3] = (__bf16)(x.w * w.w);
-    reinterpret_cast<uint2*>(entry.out)[i] = make_uint2(marked(pk.u.x, 0x7fc07fc0u), marked(pk.u.y, 0x7fc07fc0u));
+    const int to = place_of(entry.turned, (int)(i * 4 / entry.width), n, entry.width);
+    *reinterpret_cast<uint2*>(entry.out + to) = make_uint2(marked(pk.u.x, 0x7fc07fc0u), marked(pk.u.y, 0x7fc07fc0u));
     float ss = x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w;
     ss += __shfl_xor(ss, 1, 64);
     ss += __shfl_xor(ss, 2, 64);
@@ -1174,6 +1190,10 @@ __global__ void decode_layers_shares_kernel(ShareArgs args, int* out) {
 
 inline long up(long n) { return (n + 255) & ~255l; }
 
+// How many rows lie side by side in what a product multiplies with (`place_of`), and for how many there is room.
+inline int turned(int rows) { return rows > 8 ? 16 : rows > 4 ? 8 : rows > 2 ? 4 : rows; }
+inline long rows_held(int rows) { return (long)(rows + turned(rows) - 1) / turned(rows) * turned(rows); }
+
 struct Layout {
   long part, ml, att, mid, mid_sums, hid, out, out_sums, size;
 };
@@ -1182,11 +1202,12 @@ inline Layout layout_of(long rows, long width, long heads, long kv_heads, long i
   l.part = up(rows * (heads + 2 * kv_heads) * HEAD * 2);
   l.ml = l.part + items * (heads / kv_heads) * HEAD * 4;
   l.att = l.ml + up(items * (heads / kv_heads) * 8);
-  l.mid = l.att + up(rows * heads * HEAD * 2);
-  l.mid_sums = l.mid + up(rows * width * 2);
+  const long held = rows_held(rows);
+  l.mid = l.att + up(held * heads * HEAD * 2);
+  l.mid_sums = l.mid + up(held * width * 2);
   l.hid = l.mid_sums + up(rows * (width / 16) * 4);
-  l.out = l.hid + up(rows * inner * 2);
-  l.out_sums = l.out + up(rows * width * 2);
+  l.out = l.hid + up(held * inner * 2);
+  l.out_sums = l.out + up(held * width * 2);
   l.size = l.out_sums + up(rows * (width / 16) * 4);
   return l;
 }
@@ -1220,6 +1241,19 @@ inline bool sizes_fit(int rows, int width, int heads, int kv_heads, int dim, int
   return rows >= 1 && dim == HEAD && heads >= 1 && kv_heads >= 1 && heads % kv_heads == 0 && heads / kv_heads <= 16 &&
          width >= 32 * WAVES && width % 128 == 0 && inner >= 32 * WAVES && inner % 128 == 0 && heads * HEAD >= 32 * WAVES &&
          width <= (1 << 16) && inner <= (1 << 18) && heads <= 512 && rows <= rows_most(width, heads, inner);
+}
+
+// The kernel for as many rows: two groups of sixteen of them, and how many lie side by side.
+template <typename QKW>
+void (*kernel_of(int rows))(Args) {
+  if (rows > 16) return decode_layers_kernel<QKW, 2, 16>;
+  switch (turned(rows)) {
+    case 1: return decode_layers_kernel<QKW, 1, 1>;
+    case 2: return decode_layers_kernel<QKW, 1, 2>;
+    case 4: return decode_layers_kernel<QKW, 1, 4>;
+    case 8: return decode_layers_kernel<QKW, 1, 8>;
+    default: return decode_layers_kernel<QKW, 1, 16>;
+  }
 }
 
 }  // namespace
@@ -1279,7 +1313,7 @@ int q3_decode_layers(const Layer* layers, int count, float* residual, int rows, 
   char *entry_part = (char*)control + 256, *exchange = entry_part + l.size;
   const ShareArgs shares{kv_lens, rows, kv_heads, parts_taken((long)rows * kv_heads, parts), (int)items};
   const Blank to_blank{exchange, l.size, (int)l.part, (int)l.ml, (int)l.att, heads / kv_heads, shares};
-  const Entry entry{residual, layers[0].entry_norm, rows, width, norm_dtype == Q3_F32, entry_part + l.out, entry_part + l.out_sums};
+  const Entry entry{residual, layers[0].entry_norm, rows, width, norm_dtype == Q3_F32, turned(rows), entry_part + l.out, entry_part + l.out_sums};
   for (int first = 0; first < count; first += LAYERS_A_LAUNCH) {
     const int n = count - first < LAYERS_A_LAUNCH ? count - first : LAYERS_A_LAUNCH;
     LayerPack pack{};
@@ -1307,11 +1341,7 @@ int q3_decode_layers(const Layer* layers, int count, float* residual, int rows, 
   a.patience = patience, a.limit = limit;
   a.qk_eps = qk_eps;
   a.scale_log2 = make_score_scale(scale);
-  void (*kernel)(Args);
-  if (qk_dtype == Q3_F32)
-    kernel = rows > 16 ? decode_layers_kernel<float, 2, true> : rows >= 8 ? decode_layers_kernel<float, 1, true> : decode_layers_kernel<float, 1, false>;
-  else
-    kernel = rows > 16 ? decode_layers_kernel<bf16_t, 2, true> : rows >= 8 ? decode_layers_kernel<bf16_t, 1, true> : decode_layers_kernel<bf16_t, 1, false>;
+  auto kernel = qk_dtype == Q3_F32 ? kernel_of<float>(rows) : kernel_of<bf16_t>(rows);
   hipLaunchKernelGGL(kernel, dim3(blocks), dim3(THREADS), 0, stream, a);
   return q3_launch_status();
 }
