@@ -1,5 +1,5 @@
 // All decoder layers of a step of single tokens in one launch: pre-norm layers of softmax attention with grouped heads of 128 and a
-// gated unit, bfloat16, up to 16 rows, 32 of a small model, or 3 to 8 of a wide one. What gemm.hip's few-row products and attention.hip's decoding attention do layer by layer.
+// gated unit, bfloat16, up to 32 rows, of some shapes 24 or 16, or 3 to 8 of a wide one. What gemm.hip's few-row products and attention.hip's decoding attention do layer by layer.
 //
 // A kernel that waits for its predecessor costs 2 us inside a graph if it does nothing and 4 to 4.5 if it loads, reduces and stores a
 // row, and a step of the 0.6B shape was 145 of them: 1,011 us where its bytes take 240. Here a block per compute unit stays for all
@@ -1222,9 +1222,13 @@ inline long items_taken(long pairs, int parts) {
 // Up to how many rows this launch is the faster way (what is slower it does not take). Rows of more than 4,096 numbers, of two groups of
 // sixteen more than 2,048, do not stay in registers from slab to slab and are asked for with each, rows / 16 of what its weights
 // are; a width of that size is where a block has many slabs. The kernels one by one / this, us a step:
-// - two groups, up to a width of 1,024: the 0.6B shape 17 rows over 100 keys 1,149 / 947, 32 over 2,000 2,377 / 2,127; an inner size of 8,192
-//   (16 layers) 17 over 100 785 / 743, 24 over 1,000 1,014 / 957, 32 over 300 899 / 928; 16,384 17 over 300 1,043 / 1,186, 32 1,103 / 1,382;
-//   the 8B shape 20 over 1,000 4,327 / 5,229;
+// - two groups, up to a width of 1,024 (14 layers): the 0.6B shape 17 rows over 300 keys 601 / 399, 32 over 2,000 1,170 / 948; an inner size of
+//   8,192 17 over 300 712 / 525, 24 over 2,000 1,106 / 893. Longer sums, and widths up to 1,536: sixteen rows, and for more the kernels one by one;
+// - two groups from 1,536 to 4,096, inner sizes to 18,944 (with rows in one piece each, `place_of`, the 8B shape took 20 over 1,000 in 4,327 / 5,229):
+//   1,536 and 8,960 (12 layers) 17 over 300 807 / 571, 32 over 8,000 1,339 / 1,060; 2,048 and 6,144 (14) 17 over 300 833 / 591, 32 over
+//   8,000 3,219 / 2,845; 2,560 and 9,728 (12) 17 over 300 1,032 / 916, 32 over 8,000 3,105 / 2,881; the 8B shape 17 over 1,000 4,244 / 3,886,
+//   24 over 2,000 4,937 / 4,430, 32 over 500 4,312 / 4,008, over 2,000 5,210 / 4,892, 10 of its layers 17 over 100 1,061 / 969, 32 1,095 / 1,046, 32 over 8,000
+//   2,833 / 2,656, one over 30,000 and 31 over 500 1,658 / 1,383; 4,096 and 18,944 (8) 17 over 300 1,349 / 1,107, 32 1,295 / 1,195; faster at each of 92 sizes;
 // - one group, up to 4,096: 12 shapes from 512 to 4,096 wide, inner sizes to 18,944, 1 to 16 rows over 300 to 8,000 keys, all the faster
 //   here, by 10 (the 8B shape, sixteen over 8,000) to 80 percent;
 // - wider ones by how evenly the blocks have the slabs of the products into the stream. A last round half full or more: 6,144
@@ -1234,6 +1238,7 @@ inline long items_taken(long pairs, int parts) {
 inline int rows_most(int width, int heads, int inner) {
   if (width > 4096) return width / 16 % 256 == 0 || width / 16 % 256 >= 128 ? 8 : 3;
   const int longest = inner > heads * HEAD ? inner : heads * HEAD;
+  if (width >= 1536) return longest <= 18944 ? MOST_ROWS : 16;
   return width > 1024 || longest > 8192 ? 16 : longest > 4096 ? 24 : MOST_ROWS;
 }
 // Every wavefront of a block has a step of 32 of each product's K at least: the smallest K is 256, from two heads on.

@@ -179,7 +179,7 @@ class DecoderLayers:
         return out, exit_
 
 
-DECODE_ROWS_MOST = 32          # rows of a step of single tokens that `DecodeLayers` takes (of wider models than 1,024: 16, and of very wide ones fewer)
+DECODE_ROWS_MOST = 32          # rows of a step of single tokens that `DecodeLayers` takes (of some shapes 24 or 16, and of very wide models fewer)
 
 
 class _DecodeLayer(ctypes.Structure):

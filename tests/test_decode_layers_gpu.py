@@ -74,6 +74,21 @@ def test_against_the_parts(rows, longest, sizes, page):
         assert (replayed - want).norm() <= 0.02 * want.norm()
 
 
+# rows side by side in ones, twos, fours, eights and sixteens, one less and one more than a group holds, and two groups of wider models
+@pytest.mark.parametrize("rows,sizes", [
+    (2, {}), (3, {}), (4, {}), (6, {}), (7, {}), (10, {}), (15, {}), (18, {}), (31, {}), (17, dict(hidden_size=1536, intermediate_size=2304)),
+    (32, dict(hidden_size=2048, intermediate_size=6144)), (19, dict(hidden_size=4096, num_attention_heads=32, intermediate_size=12288)),
+    (32, dict(hidden_size=2176, intermediate_size=18944))])
+def test_rows_side_by_side(rows, sizes):
+    model = _model(layers=2, **sizes)
+    lengths = [1 + (41 * i) % 150 for i in range(rows)]
+    want = _logits(model, lengths, 2, launch=False)
+    got = _logits(model, lengths, 2)
+    # as in the test above; of each row by itself: one that another's numbers came into would be off by its own size
+    assert ((got - want).norm(dim=-1) <= 0.03 * want.norm(dim=-1)).all()
+    assert not torch.equal(got, want)
+
+
 def test_any_number_of_blocks_gives_the_same_bits(monkeypatch):
     """Fewer blocks than there is work for, one alone, and more than find room at once, where those that are there go on by themselves."""
     from qwen3_from_scratch_amd.ops.layers import DecodeLayers
