@@ -825,7 +825,8 @@ struct PrefillSmem {
 
 // The softmax update of one block of 16 rows for one tile of KB4 16-key blocks: as
 // softmax_step; the probabilities come back as the P operands of the tile's 32-key halves.
-template <int NB, int KB4>
+// (block j of them begins 16 STEP j keys behind key0)
+template <int NB, int KB4, int STEP = 1>
 __device__ __forceinline__ void softmax_tile(const f32x4_t (&s)[KB4], bool full, int key0, int grp, int row_pos,
                                              row_span_t window, score_scale_t scale_log2, float& m_run, float& l_run,
                                              f32x4_t (&acc)[NB], Pack16 (&p)[KB4 / 2]) {
@@ -846,7 +847,7 @@ __device__ __forceinline__ void softmax_tile(const f32x4_t (&s)[KB4], bool full,
     asm volatile("" : "+v"(pos), "+v"(first_key));
 #pragma unroll
     for (int j = 0; j < N; ++j) {
-      const int key = first_key + 16 * (j >> 2) + (j & 3);
+      const int key = first_key + 16 * STEP * (j >> 2) + (j & 3);
       bool seen = key <= pos;
       if (span_hides(window, pos, key)) seen = false;
       if (!seen) v[j] = -INFINITY;
@@ -905,8 +906,11 @@ struct PrefillShared {
   int pages[PREFILL_PAGES];
 };
 
-// A block's work: row tile and keys' share `y` of sequence `b`'s rows for key head `g_kv`.
-template <int D, int TILE, int STAGES, int DV>
+// A block's work: row tile and keys' share `y` of sequence `b`'s rows for key head `g_kv`. A wavefront has 16 QB rows and, of each tile, its KEYS-th
+// part of the keys (every KEYS-th block of 16, as the probabilities' operands pair them): 128 rows a block as (1, 2), 64 as (2, 2), 32 as (2, 1). A block is
+// one chain of tiles, 2.4 us each where a wavefront multiplies its 32 rows by all 64 keys, and with fewer than 128 rows some wavefronts had none: 276 rows
+// of 32 heads over 1,300 keys, 32 a block, 38.6 us so and 25.1 as (2, 1); 64 a block, 31.0 as (2, 2). The halves meet in shared memory at the end.
+template <int D, int TILE, int STAGES, int DV, int KEYS = 1, int QB = 2>
 __device__ __forceinline__ void prefill_block(
     PrefillShared<D, TILE, STAGES, DV>& shared, const int g_kv, const int y, const int b, const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, const bf16_t* __restrict__ k_cache,
     const bf16_t* __restrict__ v_cache, int num_pages, const int* __restrict__ block_table, int bt_stride,
@@ -941,14 +945,16 @@ __device__ __forceinline__ void prefill_block(
   const int lane = tid & 63, wave = tid >> 6;
   const int col = lane & 15, grp = lane >> 4;
   const int first_pos = kv_len - q_len;
-  const int rows_in_block = tokens_per_block * G;  // <= 128
+  const int rows_in_block = tokens_per_block * G;  // <= 64 QB / KEYS
+  constexpr int ROW_WAVES = 4 / KEYS, MINE = KB4 / KEYS, HALVES = KB4 / 2 / KEYS;
+  const int row_wave = KEYS == 1 ? wave : wave % ROW_WAVES, key_wave = KEYS == 1 ? 0 : wave / ROW_WAVES;
 
-  int row_pos[2], row_tok[2], row_head[2];
-  Pack16 qreg[2][D / 32];
+  int row_pos[QB], row_tok[QB], row_head[QB];
+  Pack16 qreg[QB][D / 32];
   int pos_max = -1, pos_min = 0x7fffffff;
 #pragma unroll
-  for (int qb = 0; qb < 2; ++qb) {
-    const int r = wave * 32 + qb * 16 + col;
+  for (int qb = 0; qb < QB; ++qb) {
+    const int r = row_wave * 16 * QB + qb * 16 + col;
     const int tok = tile * tokens_per_block + r / G;
     const bool ok = r < rows_in_block && tok < q_len;
     row_tok[qb] = q0 + tok;
@@ -975,17 +981,19 @@ __device__ __forceinline__ void prefill_block(
   // the same in all lanes: kept as scalars, so that what is decided by them per tile is a scalar branch
   pos_max = __builtin_amdgcn_readfirstlane(pos_max);
   pos_min = __builtin_amdgcn_readfirstlane(pos_min);
-  f32x4_t acc[2][DV / 16];
+  f32x4_t acc[QB][DV / 16];
 #pragma unroll
-  for (int qb = 0; qb < 2; ++qb)
+  for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
     for (int nb = 0; nb < DV / 16; ++nb) acc[qb][nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #ifdef Q3_SIGMOID
-  float m_run[2], l_run[2] = {0.f, 0.f};
+  float m_run[QB], l_run[QB];
 #pragma unroll
-  for (int qb = 0; qb < 2; ++qb) m_run[qb] = -score_bias[row_head[qb]] * 1.4426950408889634f;
+  for (int qb = 0; qb < QB; ++qb) m_run[qb] = -score_bias[row_head[qb]] * 1.4426950408889634f, l_run[qb] = 0.f;
 #else
-  float m_run[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.f, 0.f};
+  float m_run[QB], l_run[QB];
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) m_run[qb] = -INFINITY, l_run[qb] = 0.f;
 #endif
 
   // the block's range of tiles: from the window's start of its first row to its last row's position
@@ -1006,7 +1014,7 @@ __device__ __forceinline__ void prefill_block(
   row_spans_t<2> row_spans;
   row_spans.keep = window.keep;
 #pragma unroll
-  for (int qb = 0; qb < 2; ++qb) row_spans.lo[qb] = span_begin(window, max(row_pos[qb], 0));
+  for (int qb = 0; qb < QB; ++qb) row_spans.lo[qb] = span_begin(window, max(row_pos[qb], 0));
   const int first_seen = span_begin(window, first_pos);                 // of the portion's first row
   const int latest_lo = span_begin(window, max(pos_max, 0));            // of the wavefront's last row
   // the tiles of the first keys, ahead of the others in the sequence of tiles that the splits share out
@@ -1200,11 +1208,11 @@ __device__ __forceinline__ void prefill_block(
   const int k_swz = (col / SM::RPW) % SM::SWZ;
   const int v_lane = (col / SM::VRW) * 256 + (col % SM::VRW) * SM::VPR * 16 + 8 * (grp & 1);
   const int v_swz = (col / SM::VRW) % SM::VPR;
-  int k_read[D / 32], v_read[TILE / 32];
+  int k_read[D / 32], v_read[HALVES];
 #pragma unroll
-  for (int i = 0; i < D / 32; ++i) k_read[i] = k_lane + 16 * ((4 * i + grp) ^ k_swz);
+  for (int i = 0; i < D / 32; ++i) k_read[i] = k_lane + 16 * ((4 * i + grp) ^ k_swz) + 16 * SM::CPR * 16 * key_wave;
 #pragma unroll
-  for (int h = 0; h < TILE / 32; ++h) v_read[h] = v_lane + 16 * ((2 * h + (grp >> 1)) ^ v_swz);
+  for (int h = 0; h < HALVES; ++h) v_read[h] = v_lane + 16 * ((2 * (h + key_wave) + (grp >> 1)) ^ v_swz);
   constexpr int LOADS_PER_TILE = K_TURNS + V_TURNS;  // this thread's loads in flight per tile on its way
 
   // The query rows are used here, before the tile loop, so that the compiler waits for their
@@ -1212,7 +1220,7 @@ __device__ __forceinline__ void prefill_block(
   // would also wait, every time round, for the next tile's copy (the compiler counts loads,
   // and does not know of those it did not issue).
 #pragma unroll
-  for (int qb = 0; qb < 2; ++qb)
+  for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
     for (int i = 0; i < D / 32; ++i) asm volatile("" : "+v"(qreg[qb][i].v));
 
@@ -1245,7 +1253,7 @@ __device__ __forceinline__ void prefill_block(
   kv_len = token_len / runs.pool;
   window = 0;
 #pragma unroll
-  for (int qb = 0; qb < 2; ++qb) row_pos[qb] = runs_seen(token_pos[qb], token_window, runs.pool) - 1;
+  for (int qb = 0; qb < QB; ++qb) row_pos[qb] = runs_seen(token_pos[qb], token_window, runs.pool) - 1;
   pos_max = runs_seen(token_max, token_window, runs.pool) - 1;
   pos_min = token_max >= 0 ? runs_seen(token_min, token_window, runs.pool) - 1 : -1;
   tile_lo = my_lo = run_lo;
@@ -1312,15 +1320,15 @@ __device__ __forceinline__ void prefill_block(
         const unsigned char* ks = smem + stage * SM::STAGE;
         const unsigned char* vs = ks + SM::K_BYTES;
         const int key0 = t * TILE;
-        f32x4_t sc[2][KB4];
+        f32x4_t sc[QB][MINE];
 #pragma unroll
-        for (int kb4 = 0; kb4 < KB4; ++kb4) {
+        for (int kb4 = 0; kb4 < MINE; ++kb4) {
           Pack16 a[D / 32];
 #pragma unroll
           for (int i = 0; i < D / 32; ++i)
-            a[i].u = *reinterpret_cast<const uint4*>(ks + 16 * SM::CPR * 16 * kb4 + k_read[i]);
+            a[i].u = *reinterpret_cast<const uint4*>(ks + 16 * SM::CPR * 16 * KEYS * kb4 + k_read[i]);
 #pragma unroll
-          for (int qb = 0; qb < 2; ++qb) {
+          for (int qb = 0; qb < QB; ++qb) {
             f32x4_t c = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int i = 0; i < D / 32; ++i)
@@ -1336,17 +1344,18 @@ __device__ __forceinline__ void prefill_block(
         const bool full = key0 + TILE - 1 <= pos_min && (window == 0 || pos_max - key0 < window);
         const int tile_span = window;
 #endif
-        Pack16 p[2][KB4 / 2];
+        Pack16 p[QB][HALVES];
 #pragma unroll
-        for (int qb = 0; qb < 2; ++qb)
-          softmax_tile<DV / 16, KB4>(sc[qb], full, key0, grp, row_pos[qb], span_of(tile_span, qb), scale_log2, m_run[qb],
+        for (int qb = 0; qb < QB; ++qb)
+          softmax_tile<DV / 16, MINE, KEYS>(sc[qb], full, key0 + 16 * key_wave, grp, row_pos[qb], span_of(tile_span, qb), scale_log2, m_run[qb],
                                      l_run[qb], acc[qb], p[qb]);
         // the values' operands (keys 4 grp .. 4 grp + 3 of blocks half and half + KB4 / 2) are
         // read one group of output columns ahead of the matrix instructions that use them
-        Pack16 vt[4][KB4 / 2];
-        auto read_values = [&](int nb, Pack16 (&to)[KB4 / 2]) {
+        constexpr int AHEAD = 2 * KEYS, OPERANDS = DV / 16 * HALVES;
+        Pack16 vt[2 * AHEAD][HALVES];
+        auto read_values = [&](int nb, Pack16 (&to)[HALVES]) {
 #pragma unroll
-          for (int half = 0; half < KB4 / 2; ++half)
+          for (int half = 0; half < HALVES; ++half)
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb) {
               // (an empty statement of assembly after each read keeps it a ds_read_b64 of its own: joined by the
@@ -1359,27 +1368,27 @@ __device__ __forceinline__ void prefill_block(
               asm volatile("" ::: "memory");
             }
         };
-        read_values(0, vt[0]);
-        read_values(1, vt[1]);
+#pragma unroll
+        for (int nb = 0; nb < AHEAD && nb < DV / 16; ++nb) read_values(nb, vt[nb]);
 #pragma unroll
         for (int nb = 0; nb < DV / 16; ++nb) {
-          if (nb + 2 < DV / 16) read_values(nb + 2, vt[(nb + 2) & 3]);
+          if (nb + AHEAD < DV / 16) read_values(nb + AHEAD, vt[(nb + AHEAD) % (2 * AHEAD)]);
 #pragma unroll
-          for (int half = 0; half < KB4 / 2; ++half)
+          for (int half = 0; half < HALVES; ++half)
 #pragma unroll
-            for (int qb = 0; qb < 2; ++qb)
+            for (int qb = 0; qb < QB; ++qb)
               acc[qb][nb] =
-                  __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt[nb & 3][half].v, p[qb][half].v, acc[qb][nb], 0, 0, 0);
+                  __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt[nb % (2 * AHEAD)][half].v, p[qb][half].v, acc[qb][nb], 0, 0, 0);
         }
         // the order the compiler is to keep (left to itself it reads each operand right before
         // its use, into the same registers, and waits for it every time): four operands (two reads each) ahead
         __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
 #pragma unroll
-        for (int i = 0; i < (DV / 16) * (KB4 / 2) - 4; ++i) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+        for (int i = 0; i < OPERANDS - 4; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x008, QB, 0);
           __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
         }
-        __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 4 * QB, 0);
       }
       // this wavefront's share of the next tile has landed; the tiles after it may still travel
       wait_for_tile(min(t + STAGES - 1, span_hi - 1) - (t + 1));
@@ -1390,10 +1399,42 @@ __device__ __forceinline__ void prefill_block(
   }
 #endif
 #pragma unroll
-  for (int qb = 0; qb < 2; ++qb) {
+  for (int qb = 0; qb < QB; ++qb) {
+    l_run[qb] += __shfl_xor(l_run[qb], 16, 64);
+    l_run[qb] += __shfl_xor(l_run[qb], 32, 64);
+  }
+#if !defined(Q3_POOLED) && !defined(Q3_SIGMOID) && !defined(Q3_SPAN)
+  if constexpr (KEYS == 2) {
+    // the second half's sums to the first half's wavefronts, through the stages' place; a half without a key for a row weighs nothing
+    constexpr int PLACES = DV / 16 + 1;
+    f32x4_t* sums = reinterpret_cast<f32x4_t*>(smem) + (row_wave * QB * PLACES * 64 + lane);
+    static_assert(ROW_WAVES * QB * PLACES * 64 * 16 <= STAGES * SM::STAGE, "room for them");
+    __syncthreads();
+    if (key_wave == 1) {
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) {
+#pragma unroll
+        for (int nb = 0; nb < DV / 16; ++nb) sums[64 * (qb * PLACES + nb)] = acc[qb][nb];
+        sums[64 * (qb * PLACES + DV / 16)] = f32x4_t{m_run[qb], l_run[qb], 0.f, 0.f};
+      }
+    }
+    __syncthreads();
+    if (key_wave == 1) return;
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) {
+      const f32x4_t ml = sums[64 * (qb * PLACES + DV / 16)];
+      const float m = max_of_numbers(m_run[qb], ml[0]), m_use = m > -INFINITY ? m : 0.f;
+      const float mine = fast_exp2(m_run[qb] - m_use), other = fast_exp2(ml[0] - m_use);
+#pragma unroll
+      for (int nb = 0; nb < DV / 16; ++nb) acc[qb][nb] = acc[qb][nb] * mine + sums[64 * (qb * PLACES + nb)] * other;
+      l_run[qb] = l_run[qb] * mine + ml[1] * other;
+      m_run[qb] = m;
+    }
+  }
+#endif
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
     float l = l_run[qb];
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
     if (row_pos[qb] < 0) continue;
     if (key_splits > 1) {
       const size_t slot = ((size_t)row_tok[qb] * Hq + row_head[qb]) * key_splits + split;
@@ -1429,7 +1470,7 @@ __device__ __forceinline__ void prefill_block(
   }
 }
 
-template <int D, int TILE, int STAGES, int DV = D>
+template <int D, int TILE, int STAGES, int DV = D, int KEYS = 1, int QB = 2>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_prefill_kernel(
     const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, const bf16_t* __restrict__ k_cache,
     const bf16_t* __restrict__ v_cache, int num_pages, const int* __restrict__ block_table, int bt_stride,
@@ -1437,7 +1478,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     span_t window, int tokens_per_block, int key_splits, float* __restrict__ part_acc, float* __restrict__ part_ml,
     const float* __restrict__ sink Q3_BIAS_PARAM Q3_RUNS_PARAM Q3_GATE_PARAM) {
   __shared__ PrefillShared<D, TILE, STAGES, DV> shared;
-  prefill_block<D, TILE, STAGES, DV>(shared, blockIdx.x, blockIdx.y, blockIdx.z, q, q_stride, out, k_cache, v_cache, num_pages,
+  prefill_block<D, TILE, STAGES, DV, KEYS, QB>(shared, blockIdx.x, blockIdx.y, blockIdx.z, q, q_stride, out, k_cache, v_cache, num_pages,
                                      block_table, bt_stride, cu_q, kv_lens, Hq, Hkv, page, scale_log2, window, tokens_per_block,
                                      key_splits, part_acc, part_ml, sink Q3_BIAS_PASS Q3_RUNS_PASS Q3_GATE_PASS);
 }
@@ -1470,13 +1511,12 @@ __device__ __forceinline__ int sequence_of_tile(int& n, const int* __restrict__ 
 
 // A step of few rows in all: 16 of them a block, whatever sequence they are of, as the decoding kernel treats its 16. The prompt
 // kernel's 32 to 128 rows a block walk tiles of 64 keys one after the other through shared memory; here four wavefronts share the keys in
-// tiles of 32, straight from the L2, which every block asks for them anew: the way as long as a CU has two such blocks at most
-// (SHORT_BLOCKS, a little less for the tiles that do not come). Microseconds, prompt kernel / this, 16 and 32 heads over 8 of 128: three
-// prompts of 33, 67 and 101 tokens 10.9 / 7.0 and 11.0 / 9.6; one of 200 11.6 / 8.1 and 13.2 / 10.4; 64 rows over 512 keys 17.7 / 10.4
-// and 17.8 / 10.4; 32 over 1,000 30 / 15, over 1,900 51 / 23 (from 1,985 keys on the prompt kernel shares them out); 440 and 220 over
-// 1,900 (440 blocks each) 52 / 40; 400 over 400 (400 and 800 blocks) 17.6 / 13.2 and 18.1 / 20.9; four prompts of 128
-// (512 and 1,024) 9.7 / 10.3 and 10.2 / 18.4.
-#define SHORT_BLOCKS 448
+// tiles of 32, straight from the L2, which every block asks for them anew: the way as long as there is one such block a CU. Microseconds,
+// prompt kernel / this, groups of two and four heads over 8 of 128 (blocks here): three prompts of 33, 67 and 101 tokens 8.9 / 7.8 (216) and 9.1 / 10.3
+// (416); one of 200 9.6 / 8.7 (200) and 9.7 / 11.2 (400); 64 rows over 512 keys 11.4 / 11.0 and 11.5 / 11.0; 32 over 1,000 19.8 / 15.7, over
+// 1,900 31.6 / 23.3; 220 over 1,900 31.5 / 23.6 (224) and 32.0 / 40.1 (440); 150 over 600 14.1 / 12.1 (152) and 14.2 / 17.7 (304); 300 over 300
+// 11.0 / 11.6 (304); eight prompts of 16 7.4 / 7.5 (256).
+#define SHORT_BLOCKS 256
 template <int D>
 __global__ __launch_bounds__(64 * DECODE_WAVES) Q3_DECODE_WAVES void attn_short_kernel(
     const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, const bf16_t* __restrict__ k_cache,
@@ -1498,11 +1538,13 @@ __global__ __launch_bounds__(64 * DECODE_WAVES) Q3_DECODE_WAVES void attn_short_
 // and row tile, of as many row tiles as the sequences can come to; the last find none), the others for the decoding ones (splits x Hkv x
 // sequences). The decoding ones wait for memory and the prompts' for the matrix cores and the vector unit; a block of either
 // takes half a CU's registers and shared memory, so they run side by side. The kind that comes first (both in multiples of
-// eight blocks, so that a key head's blocks stay on its chiplet) is the prompts', whose chains are longer, where it leaves half of the
-// room, else the decoding one. 23 requests over 150 to 3,000 keys beside a prompt's rows, 32 heads in groups of four, microseconds:
-// one kernel after the other / in one launch, prompts first / decoding first: 512 rows over 512 keys 68 / 48 / 49, over 1,024 80 /
-// 51 / 58, 276 over 1,300 86 / 54 / 65, 512 over 3,584 (512 blocks of them) 109 / 104 / 84; 5 requests beside the first 38 / 27 / 31.
-template <int D, int TILE, int STAGES>
+// eight blocks, so that a key head's blocks stay on its chiplet) is the prompts', whose chains are longer, where there are 128 pairs of decoding
+// sequences and key heads or they leave half of the room, else the decoding one. Prompts first / decoding first, microseconds, 32 heads in groups of
+// four: 23 requests over 150 to 3,000 keys beside 276 rows over 1,300 54.1 / 62.5, 512 over 512 47.8 / 47.7, over 1,536 57.4 / 64.2, over 3,584 92.5 /
+// 106.5, 1,400 over 1,400 58.1 / 65.9; 15 beside 1,000 over 1,000 44.2 / 56.4; 40 over 1,000 beside it 45.9 / 54.9, 40 over 150 to 3,000 beside 276 over
+// 1,300 78.7 / 69.5 (the one size of these that loses much). Ten (80 pairs) beside 512 over 512 (512 blocks) 38.6 / 34.3, over 3,584 86.3 / 81.2; beside 276 over
+// 1,300 (280) 37.7 / 43.5; two beside 512 over 512 19.8 / 21.2. One kernel after the other took 68 beside the second of these, 80 over 1,024 (51 so).
+template <int D, int TILE, int STAGES, int KEYS, int QB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_mixed_kernel(
     const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, const bf16_t* __restrict__ k_cache,
     const bf16_t* __restrict__ v_cache, int num_pages, const int* __restrict__ block_table, int bt_stride,
@@ -1522,7 +1564,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int b = __builtin_amdgcn_readfirstlane(sequence_of_tile<true>(tile, cu_q, sequences, Hq / Hkv, tokens_per_block));
     if (b < 0) return;
     tile = __builtin_amdgcn_readfirstlane(tile);
-    prefill_block<D, TILE, STAGES, D>(shared.prompt, id % Hkv, tile * key_splits + share % key_splits, b, q, q_stride, out,
+    prefill_block<D, TILE, STAGES, D, KEYS, QB>(shared.prompt, id % Hkv, tile * key_splits + share % key_splits, b, q, q_stride, out,
                                       k_cache, v_cache, num_pages, block_table, bt_stride, cu_q, kv_lens, Hq, Hkv, page,
                                       scale_log2, 0, tokens_per_block, key_splits, part_acc, part_ml, sink Q3_GATE_PASS);
   } else {
@@ -1587,11 +1629,46 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(bf16_t* __restr
 // How the rows and keys of a step's long sequences go over blocks. A block owns 128 rows
 // (tokens x heads of a group) and all their keys; with so few rows that the blocks do not fill
 // the chip twice (a portion of 512 tokens of one prompt: 128 blocks, each a chain of as many
-// tiles as the prefix is long), first the keys are split over up to four blocks, from 2,048
-// keys on and as long as a split keeps eight tiles (512 tokens over 3,584 keys: 127 us whole,
-// 97 in two, 88 in four; 256 over 7,936: 224, 141, 97; over 512 keys splitting loses), then a
-// block's rows are halved, down to one wavefront's 32 (its other wavefronts then only help
-// to copy the tiles).
+// tiles as the prefix is long), the keys are split over up to four blocks
+// and a block's rows are halved, down to 32.
+#if !defined(Q3_POOLED) && !defined(Q3_SIGMOID) && !defined(Q3_SPAN)
+// A halved block's wavefronts share its keys (prefill_block's KEYS), so its chain is half as long too and nothing has to be merged
+// behind the kernel: rows first, while there are 288 blocks at most, since two run on a CU at once and a few more behind those are short (2,300 rows of 16
+// heads in pairs, 288 blocks, 64.9, 50.5 halved; 1,100 of 32 in fours, 280, 37.2 and 34.2; with a window, whose chains are short, fewer than 256: 1,100 over
+// 128 of them 17.8 and 25.4, 1,024, 256 blocks, 14.4 and 15.8); from 3,072 keys on
+// first the keys (from 2,560 on as many parts as the least rows leave room for). 32 heads in groups of four, rows of a block * parts of the keys, microseconds,
+// 128*1 / 64*1 / 32*1 / 128*4: 512 over 512 19.9 / 17.0 / 13.0 / 36; over 2,048 52.6 / 41.0 / 34.4 / 45.4; over 4,096 95.2 / 71.8 / 60.2 / 60.2, over
+// 8,000 176 / 131 / 124 / 93; 276 over 1,300 39.4 / 31.0 / 25.1 / 39.0; 1,024 over 1,024 32.3 / 27.6 / 31.6 / 48; 1,000 over 2,000 55 / 47 / 59 / 64; 2,048 of one
+// prompt (512 blocks) 56.4 / 71.8 / 83.3 / 88. 128 over 2,048 in 32*1 25.1, 32*4 31.0, over 4,096 41.8 and 37.9; 256 over 4,096 32*1 55.4, 32*2 44.4.
+// Capped scores, whose tiles take longer, from 2,048 keys on: 2,048 rows of 16 heads in fours over 2,048 keys 46.8 and 12 for the merge in 128*2, 65 in 64*1.
+// Beside the decoding sequences of a mixed launch blocks of many rows leave those more of the CUs: with 128 of their pairs or more the rows are
+// halved below 128 blocks only. 23 requests over 150 to 3,000 keys beside 512 over 512 47.0 in 128 rows, 48.3 in 64, 49.4 in 32; beside 512 over
+// 1,536 56.3, 64.9; beside 276 over 1,300 57.5, 52.8, 57.0 (80, 152 and 296 blocks); 40 over 1,000 beside 512 over 1,536 52.3, 62.9; eight over 1,000 beside
+// 276 over 1,300 40.3, 38.3, 36.1.
+static int prompt_key_splits(int total_tokens, int G, int Hkv, int max_kv_len) {
+  const int key_tiles = (max_kv_len + PF_TILE - 1) / PF_TILE;
+#ifdef Q3_SCORE_CAP
+  constexpr int SOME = 32, MANY = 32;
+#else
+  constexpr int SOME = 40, MANY = 48;
+#endif
+  if (key_tiles < SOME) return 1;
+  const int tpb = (key_tiles < MANY ? 32 : 128) / G, enough = key_tiles < MANY ? 257 : 512;
+  int ks = 1;
+  while (Hkv * ((total_tokens + tpb - 1) / tpb) * ks < enough && ks < 4) ks *= 2;
+  return ks;
+}
+
+static int prompt_tokens_per_block(int total_tokens, int G, int Hkv, int key_splits, int window, long decode_pairs) {
+  int tpb = 128 / G;
+  const int enough = decode_pairs >= 128 ? 128 : window ? 256 : 289;
+  while (Hkv * ((total_tokens + tpb - 1) / tpb) * key_splits < enough && (tpb / 2) * G >= 32) tpb /= 2;
+  return tpb;
+}
+#else
+// The keys come first, from 2,048 on and as long as a split keeps eight tiles (512 tokens over 3,584 keys: 127 us whole,
+// 97 in two, 88 in four; 256 over 7,936: 224, 141, 97; over 512 keys splitting loses). Of a block of fewer than 128 rows some
+// wavefronts only help to copy the tiles.
 static int prompt_key_splits(int total_tokens, int G, int Hkv, int max_kv_len) {
   const int tpb = 128 / G;
   int ks = 1;
@@ -1601,11 +1678,12 @@ static int prompt_key_splits(int total_tokens, int G, int Hkv, int max_kv_len) {
   return ks;
 }
 
-static int prompt_tokens_per_block(int total_tokens, int G, int Hkv, int key_splits) {
+static int prompt_tokens_per_block(int total_tokens, int G, int Hkv, int key_splits, int, long) {
   int tpb = 128 / G;
   while (Hkv * ((total_tokens + tpb - 1) / tpb) * key_splits < 256 && (tpb / 2) * G >= 32) tpb /= 2;
   return tpb;
 }
+#endif
 
 template <int D, int DV = D>
 static int launch_fast(const void* q, int q_stride, void* out, const void* k_cache, const void* v_cache,
@@ -1625,7 +1703,7 @@ static int launch_fast(const void* q, int q_stride, void* out, const void* k_cac
   if (window != 0 || g_score_bias == nullptr || sink != nullptr) return Q3_ERR_BAD_ARGUMENT;
 #endif
   const bool few = min_q_len * G <= 16, many = max_q_len * G > 16;
-  const int tokens_per_block = many ? prompt_tokens_per_block(total_tokens, G, Hkv, key_splits) : 1;
+  const int tokens_per_block = many ? prompt_tokens_per_block(total_tokens, G, Hkv, key_splits, window, few && window == 0 ? (long)Hkv * B : 0) : 1;
   const int tiles = (max_q_len + tokens_per_block - 1) / tokens_per_block;
   if (many && tiles * key_splits > 65535) return Q3_ERR_UNSUPPORTED;
   float* part_acc = prompt_ws;
@@ -1645,14 +1723,23 @@ static int launch_fast(const void* q, int q_stride, void* out, const void* k_cac
   // row tiles of the sequences of many rows: one each beyond whole ones, and as many sequences as there are rows for
   const long row_tiles = total_tokens / tokens_per_block + min(B, total_tokens / (16 / G + 1));
   const long prompt_blocks = (row_tiles * key_splits * Hkv + 7) / 8 * 8, decode_blocks = ((long)splits * Hkv * B + 7) / 8 * 8;
-  const bool prompts_first = (long)((total_tokens + tokens_per_block - 1) / tokens_per_block) * key_splits * Hkv <= 256;
+  const bool prompts_first =
+      (long)Hkv * B >= 128 || (long)((total_tokens + tokens_per_block - 1) / tokens_per_block) * key_splits * Hkv <= 288;
   together = few && many && window == 0 && (prompt_blocks + decode_blocks) * 256 < (1L << 32);
+  const int rows = tokens_per_block * G;
+  const auto prompt_kernel = rows > 64 ? attn_prefill_kernel<D, TILE, PF_STAGES, DV> : rows > 32 ? attn_prefill_kernel<D, TILE, PF_STAGES, DV, 2>
+                                                                                        : attn_prefill_kernel<D, TILE, PF_STAGES, DV, 2, 1>;
+  const auto mixed_kernel = rows > 64   ? attn_mixed_kernel<D, TILE, PF_STAGES, 1, 2>
+                            : rows > 32 ? attn_mixed_kernel<D, TILE, PF_STAGES, 2, 2>
+                                        : attn_mixed_kernel<D, TILE, PF_STAGES, 2, 1>;
   if (together)
-    hipLaunchKernelGGL((attn_mixed_kernel<D, TILE, PF_STAGES>), dim3((unsigned)(prompt_blocks + decode_blocks)), dim3(256), 0,
+    hipLaunchKernelGGL(mixed_kernel, dim3((unsigned)(prompt_blocks + decode_blocks)), dim3(256), 0,
                        stream, (const bf16_t*)q, q_stride, (bf16_t*)out, (const bf16_t*)k_cache, (const bf16_t*)v_cache,
                        num_pages, block_table, bt_stride, cu_q, kv_lens, B, Hq, Hkv, page, scale_log2, prompts_first ? 1 : 0,
                        (int)(prompts_first ? prompt_blocks : decode_blocks), tokens_per_block, key_splits, part_acc, part_ml,
                        splits, ws_acc, ws_ml, sink Q3_GATE_ARG);
+#else
+  const auto prompt_kernel = attn_prefill_kernel<D, TILE, PF_STAGES, DV>;
 #endif
   if (few && !together) {
 #if !defined(Q3_POOLED) && !defined(Q3_SPAN)
@@ -1672,7 +1759,7 @@ static int launch_fast(const void* q, int q_stride, void* out, const void* k_cac
     hipLaunchKernelGGL(attn_decode_reduce_kernel<DV>, dim3(Hkv, B), dim3(256), 0, stream, (bf16_t*)out, cu_q, Hq,
                        Hkv, splits, ws_acc, ws_ml, sink Q3_GATE_ARG);
   if (many && !together)
-    hipLaunchKernelGGL((attn_prefill_kernel<D, TILE, PF_STAGES, DV>), dim3(Hkv, tiles * key_splits, B), dim3(256), 0,
+    hipLaunchKernelGGL(prompt_kernel, dim3(Hkv, tiles * key_splits, B), dim3(256), 0,
                        stream, (const bf16_t*)q, q_stride, (bf16_t*)out, (const bf16_t*)k_cache,
                        (const bf16_t*)v_cache, num_pages, block_table, bt_stride, cu_q, kv_lens, Hq, Hkv, page,
                        scale_log2, span, tokens_per_block, key_splits, part_acc, part_ml, sink Q3_BIAS_ARG Q3_RUNS_ARG Q3_GATE_ARG);

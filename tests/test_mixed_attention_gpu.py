@@ -27,7 +27,7 @@ def _lens(name):
     }[name]
 
 
-def _exact(q, kc, vc, bt, cu, kvl, scale, sink, cap):
+def _exact(q, kc, vc, bt, cu, kvl, scale, sink, cap, window=0):
     """The attention in float64, and of every result the sum of the magnitudes that it adds."""
     Hq, Hkv, page = q.shape[1], kc.shape[1], kc.shape[2]
     result, size = [], []
@@ -38,7 +38,8 @@ def _exact(q, kc, vc, bt, cu, kvl, scale, sink, cap):
         v = vc[pages].double().permute(1, 0, 3, 2).flatten(1, 2)[:, :L].repeat_interleave(Hq // Hkv, dim=0)
         s = torch.matmul(rows.transpose(0, 1), k.transpose(1, 2).contiguous()) * scale
         s = cap * torch.tanh(s / cap) if cap else s
-        s = s.masked_fill(torch.arange(L, device="cuda") > torch.arange(L - n, L, device="cuda")[:, None], float("-inf"))
+        behind = torch.arange(L - n, L, device="cuda")[:, None] - torch.arange(L, device="cuda")
+        s = s.masked_fill((behind < 0) | (behind >= (window or L)), float("-inf"))
         if sink is not None:
             s = torch.cat((s, sink.double()[:, None, None].expand(Hq, n, 1)), dim=2)
         w = torch.softmax(s, dim=2)[:, :, :L]
@@ -93,4 +94,24 @@ def test_few_rows_over_many_keys(Hq, Hkv, D, page, lens, cap):
     q, kc, vc, bt, cu, kvl = _paged_case(torch.bfloat16, len(lens), Hq, Hkv, D, page, q_lens, kv_lens, 34)
     got = ops.paged_attention(q, Hq, kc, vc, bt, cu, kvl, max(q_lens), max(kv_lens), D ** -0.5, min_q_len=min(q_lens), softcap=cap)
     want, size = _exact(q, kc, vc, bt, cu, kvl, D ** -0.5, None, cap)
+    assert bool(((got.double() - want).abs() <= _bound(got, size)).all())
+
+
+# Blocks of 32, 64 and 128 rows, whose wavefronts share the keys or do not: rows and keys at the edges of tiles and of their halves (the first row of a
+# prompt sees no key of the second), keys in parts, a window, a group that does not divide the rows; the last two beside 128 pairs of decoding ones
+@pytest.mark.parametrize("Hq,Hkv,D,page,lens,window", [
+    (8, 2, 128, 16, [(200, 200), (17, 33), (130, 177), (129, 1031)], 0), (8, 2, 64, 16, [(300, 300), (95, 128)], 0),
+    (12, 4, 128, 32, [(260, 260), (100, 640)], 0), (16, 2, 128, 16, [(150, 3300)], 0), (8, 2, 128, 64, [(150, 4100), (40, 40)], 0),
+    (8, 2, 128, 16, [(200, 260), (130, 177)], 40), (8, 8, 64, 16, [(1290, 1300), (1250, 1250)], 0), (6, 2, 128, 16, [(1500, 1500), (1501, 1533)], 0),
+    (8, 8, 128, 16, [(1100, 1100), (1111, 1130)], 300), (8, 8, 64, 16, [(2410, 2433), (2400, 2400)], 0),
+    (16, 8, 128, 16, [(1, 50 * i + 1) for i in range(16)] + [(600, 611)], 0), (16, 8, 64, 16, [(1, 30 * i + 1) for i in range(17)] + [(1300, 1300)], 0)])
+@pytest.mark.parametrize("cap", [0.0, 12.0])
+def test_rows_of_a_block(Hq, Hkv, D, page, lens, window, cap):
+    ops = _ops()
+    q_lens, kv_lens = [q for q, _ in lens], [k for _, k in lens]
+    q, kc, vc, bt, cu, kvl = _paged_case(torch.bfloat16, len(lens), Hq, Hkv, D, page, q_lens, kv_lens, 35)
+    sink = torch.randn(Hq, generator=torch.Generator().manual_seed(36)).cuda()
+    got = ops.paged_attention(q, Hq, kc, vc, bt, cu, kvl, max(q_lens), max(kv_lens), D ** -0.5, window=window, min_q_len=min(q_lens),
+                              max_kv_len_of_many=max(k for q, k in lens if q > 1), sink=sink, softcap=cap)
+    want, size = _exact(q, kc, vc, bt, cu, kvl, D ** -0.5, sink, cap, window)
     assert bool(((got.double() - want).abs() <= _bound(got, size)).all())
