@@ -92,6 +92,26 @@ __device__ inline void store8(float* p, const float (&v)[8]) {
   *reinterpret_cast<float4*>(p + 4) = make_float4(v[4], v[5], v[6], v[7]);
 }
 
+__device__ inline void load4(const float* p, float (&v)[4]) {
+  const float4 x = *reinterpret_cast<const float4*>(p);
+  v[0] = x.x, v[1] = x.y, v[2] = x.z, v[3] = x.w;
+}
+__device__ inline void load4(const bf16_t* p, float (&v)[4]) {
+  const uint2 x = *reinterpret_cast<const uint2*>(p);
+  v[0] = __uint_as_float(x.x << 16), v[1] = __uint_as_float(x.x & 0xffff0000u);
+  v[2] = __uint_as_float(x.y << 16), v[3] = __uint_as_float(x.y & 0xffff0000u);
+}
+__device__ inline void store4(float* p, const float (&v)[4]) { *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]); }
+__device__ inline void store4(bf16_t* p, const float (&v)[4]) {
+  union {
+    uint2 u;
+    bf16_t e[4];
+  } a;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) a.e[i] = float_to_bf16(v[i]);
+  *reinterpret_cast<uint2*>(p) = a.u;
+}
+
 // Eight numbers as they come, made float32 where they are used: made so where they are loaded, each load waits.
 template <typename TI>
 struct Eight;
@@ -115,10 +135,11 @@ struct Eight<float> {
 };
 
 // A thread's tile is Q3_CONV_TILE rows. TAPS 4: that many, and a thread takes its channels' taps straight from memory; 0:
-// up to Q3_TAPS_MOST, through shared memory. Bound by memory and the taps' passage: 2,048 rows of 4,352 bfloat16 channels
-// and 4 taps (36 MB) 22 us, 37 with an input's wait before each next one and taps that 32 lanes read from one bank of
-// shared memory (as they still are for other numbers of taps).
-#define Q3_CONV_TILE 8
+// up to Q3_TAPS_MOST, through shared memory. Bound by memory, the taps' passage and the activation: 2,048 rows of 4,352 bfloat16 channels
+// and 4 taps (36 MB) 18.5 us in tiles of four rows, 18.8 of two, 21.8 of eight (fewer inputs read twice, but two wavefronts a SIMD, of which each
+// waits once and then computes; taps turned in shared memory out of neighbouring pieces 20.0); 37 with an input's wait before each next one and taps that 32 lanes
+// read from one bank of shared memory (as they still are for other numbers of taps).
+#define Q3_CONV_TILE 4
 template <typename TI, typename TO, int TAPS>
 __global__ void __launch_bounds__(64) causal_conv_wide_kernel(const TI* __restrict__ x, long x_stride, const float* __restrict__ in_bias,
                                         const float* __restrict__ w, const float* __restrict__ bias,
@@ -1228,6 +1249,55 @@ __global__ void retention_prepare_kernel(const TA* __restrict__ rows, const floa
   for (int e = threadIdx.x; e < hv; e += blockDim.x) vf[(size_t)t * hv + e] = to_float(row[2 * hd + e]);
 }
 
+// The same four neighbouring numbers at a time, a token's sines and cosines once for all its heads, in shared memory: heads and halves of multiples
+// of four. Bound by memory: 2,048 tokens of 8 heads of 128 with values of 256 (50 MB) 13.7 us by the kernel above, 9.7 here.
+#define Q3_QUADS_HALF_MOST 256
+template <typename TA>
+__global__ void __launch_bounds__(256) retention_prepare_quads_kernel(const TA* __restrict__ rows, const float* __restrict__ inv_freq, int half,
+                                                                      const int* __restrict__ positions, float k_scale,
+                                                                      float* __restrict__ qf, float* __restrict__ kf,
+                                                                      float* __restrict__ vf, int H, int dim, int vdim) {
+  __shared__ __attribute__((aligned(16))) float cosines[Q3_QUADS_HALF_MOST], sines[Q3_QUADS_HALF_MOST];
+  const int t = blockIdx.x;
+  const int hd = H * dim, hv = H * vdim;
+  const TA* row = rows + (size_t)t * (2 * (size_t)hd + 2 * (size_t)hv);
+  const float pos = (float)positions[t];
+  for (int j = threadIdx.x; j < half; j += 256) {
+    const float angle = pos * inv_freq[j];
+    cosines[j] = cosf(angle), sines[j] = sinf(angle);
+  }
+  for (int e = 4 * threadIdx.x; e < hv; e += 1024) {
+    float v[4];
+    load4(row + 2 * hd + e, v);
+    store4(vf + (size_t)t * hv + e, v);
+  }
+  __syncthreads();
+  for (int e = 4 * threadIdx.x; e < hd; e += 1024) {
+    const int j = e % dim;
+    float q[4], k[4];
+    load4(row + e, q);
+    load4(row + hd + e, k);
+    if (j < 2 * half) {
+      const bool first = j < half;
+      const int partner = first ? e + half : e - half;
+      float qp[4], kp[4], c[4], s[4];
+      load4(row + partner, qp);
+      load4(row + hd + partner, kp);
+      load4(cosines + (first ? j : j - half), c);
+      load4(sines + (first ? j : j - half), s);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        q[i] = first ? q[i] * c[i] - qp[i] * s[i] : q[i] * c[i] + qp[i] * s[i];
+        k[i] = first ? k[i] * c[i] - kp[i] * s[i] : k[i] * c[i] + kp[i] * s[i];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) k[i] *= k_scale;
+    store4(qf + (size_t)t * hd + e, q);
+    store4(kf + (size_t)t * hd + e, k);
+  }
+}
+
 // One block per (token, head): o divided by its root mean square over the head's vdim numbers, times silu(g).
 template <typename TA>
 __global__ void retention_finish_kernel(const float* __restrict__ o, const TA* __restrict__ rows, float eps,
@@ -1242,6 +1312,54 @@ __global__ void retention_finish_kernel(const float* __restrict__ o, const TA* _
   const float inv = rsqrtf(block_sum(sq, scratch) / (float)vdim + eps);
   for (int j = threadIdx.x; j < vdim; j += blockDim.x)
     out[(size_t)t * hv + h * vdim + j] = from_float<TA>(src[j] * inv * silu_value(to_float(gate[j])));
+}
+
+// The same by a wavefront per (token, head), four neighbouring numbers a lane and turn, all of a head asked for at once: no barrier, and a
+// quarter of the blocks. Bound by memory: 2,048 tokens of 8 heads of 256 (34 MB) 18.5 us by the kernel above, 11.1 here.
+// Heads of a multiple of four, up to 1,024 numbers, rows that lie at multiples of four of them.
+template <typename TA>
+__global__ void __launch_bounds__(256) retention_finish_quads_kernel(const float* __restrict__ o, const TA* __restrict__ rows, float eps,
+                                                                     TA* __restrict__ out, long heads, int H, int dim, int vdim) {
+  const long head = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (head >= heads) return;
+  const int lane = threadIdx.x & 63, h = (int)(head % H);
+  const size_t t = (size_t)(head / H), hd = (size_t)H * dim, hv = (size_t)H * vdim;
+  const float* src = o + (size_t)head * vdim;
+  const TA* gate = rows + t * (2 * hd + 2 * hv) + 2 * hd + hv + (size_t)h * vdim;
+  float4 x[4];
+  float g[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int j = 256 * i + 4 * lane;
+    x[i] = j < vdim ? *reinterpret_cast<const float4*>(src + j) : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (256 * i + 4 * lane < vdim) load4(gate + 256 * i + 4 * lane, g[i]);
+  float sq = 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) sq += x[i].x * x[i].x + x[i].y * x[i].y + x[i].z * x[i].z + x[i].w * x[i].w;
+  const float inv = rsqrtf(wave_sum(sq) / (float)vdim + eps);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int j = 256 * i + 4 * lane;
+    if (j >= vdim) break;
+    const float of[4] = {x[i].x * inv * silu_value(g[i][0]), x[i].y * inv * silu_value(g[i][1]), x[i].z * inv * silu_value(g[i][2]),
+                         x[i].w * inv * silu_value(g[i][3])};
+    store4(out + t * hv + (size_t)h * vdim + j, of);
+  }
+}
+
+template <typename TA>
+static void launch_retention_finish(const float* o, const TA* rows, float eps, TA* out, int T, int H, int dim, int vdim, hipStream_t stream) {
+  if (vdim % 4 == 0 && vdim <= 1024 && H * dim % 2 == 0 && (size_t)o % 16 == 0 && (size_t)rows % (4 * sizeof(TA)) == 0 &&
+      (size_t)out % (4 * sizeof(TA)) == 0) {
+    const long heads = (long)T * H;
+    hipLaunchKernelGGL(retention_finish_quads_kernel<TA>, dim3((unsigned)((heads + 3) / 4)), dim3(256), 0, stream, o, rows, eps, out, heads, H, dim, vdim);
+    return;
+  }
+  const int threads = vdim >= 256 ? 256 : (vdim >= 128 ? 128 : 64);
+  hipLaunchKernelGGL(retention_finish_kernel<TA>, dim3(T, H), dim3(threads), 0, stream, o, rows, eps, out, H, dim, vdim);
 }
 
 // Floats of workspace for a step of T rows in B sequences: q, k, v, ld, the chunks' sums, decays and raw scores.
@@ -1338,16 +1456,15 @@ extern "C" int q3_retention_chunked(const void* rows, const float* inv_freq, int
   float* vf = kf + (size_t)T * H * dim;
   float* sums = vf + (size_t)T * H * vdim;
   float* decays = sums + (size_t)(T / Q3_CHUNK + B) * H * dim * vdim;
+  const bool quads = dim % 4 == 0 && half % 4 == 0 && half <= Q3_QUADS_HALF_MOST && H * vdim % 4 == 0 && (size_t)workspace % 16 == 0 &&
+                     (size_t)rows % (act_dtype == Q3_F32 ? 16 : 8) == 0;
   Q3_DISPATCH_DTYPE(act_dtype, TA,
-                    hipLaunchKernelGGL(retention_prepare_kernel<TA>, dim3(T), dim3(256), 0, stream, (const TA*)rows,
-                                       inv_freq, half, positions, k_scale, qf, kf, vf, H, dim, vdim));
+                    hipLaunchKernelGGL((quads ? retention_prepare_quads_kernel<TA> : retention_prepare_kernel<TA>), dim3(T), dim3(256), 0,
+                                       stream, (const TA*)rows, inv_freq, half, positions, k_scale, qf, kf, vf, H, dim, vdim));
   const int status = launch_chunks<float>(qf, kf, vf, log_decays, 0, sums, decays, scores, state, state_stride, slots, cu,
                                           scratch_out, B, max_q_len, H, 1, dim, vdim, nullptr, 0, nullptr, stream);
   if (status) return status;
-  const int threads = vdim >= 256 ? 256 : (vdim >= 128 ? 128 : 64);
-  Q3_DISPATCH_DTYPE(act_dtype, TA,
-                    hipLaunchKernelGGL(retention_finish_kernel<TA>, dim3(T, H), dim3(threads), 0, stream, scratch_out,
-                                       (const TA*)rows, eps, (TA*)out, H, dim, vdim));
+  Q3_DISPATCH_DTYPE(act_dtype, TA, launch_retention_finish<TA>(scratch_out, (const TA*)rows, eps, (TA*)out, T, H, dim, vdim, stream));
   return q3_launch_status();
 }
 
@@ -1617,9 +1734,7 @@ static int launch_retention(const void* rows, const float* inv_freq, int half, c
   else if (dim <= 128) Q3_RETENTION(8);
   else Q3_RETENTION(16);
 #undef Q3_RETENTION
-  const int threads = vdim >= 256 ? 256 : (vdim >= 128 ? 128 : 64);
-  hipLaunchKernelGGL(retention_finish_kernel<TA>, dim3(T, H), dim3(threads), 0, stream, raw, (const TA*)rows, eps,
-                     (TA*)out, H, dim, vdim);
+  launch_retention_finish<TA>(raw, (const TA*)rows, eps, (TA*)out, T, H, dim, vdim, stream);
   return q3_launch_status();
 }
 

@@ -166,6 +166,28 @@ def test_retention_scan(dtype, H, dim, vdim, rot, lengths):
     _close(a, b, 1e-4)
 
 
+# rows read four numbers at a time and the forms that are not: heads and halves of fours and not, values of one to four turns of a wavefront, rows
+# that begin between multiples of four, two heads a token beside the last block's
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("H,dim,vdim,rot,off", [(3, 64, 4, 8, 0), (2, 128, 260, 128, 0), (1, 64, 1024, 64, 0), (2, 64, 66, 64, 0), (2, 36, 64, 12, 0),
+                                                (1, 64, 1028, 0, 0), (2, 64, 128, 64, 1), (2, 64, 128, 64, 4), (3, 12, 36, 8, 2)])
+def test_retention_rows_in_fours(dtype, H, dim, vdim, rot, off):
+    g = _gen(H * dim + vdim + off)
+    lengths = [67, 1, 20]
+    T, width = sum(lengths), 2 * H * dim + 2 * H * vdim
+    rows = _rand(g, T * width + off, dtype=dtype)[off:].view(T, width)
+    inv_freq = torch.tensor([10000.0 ** (-2.0 * i / rot) for i in range(rot // 2)], dtype=torch.float32, device=DEV) if rot else None
+    positions = torch.tensor([b * 50 + i for b, n in enumerate(lengths) for i in range(n)], dtype=torch.int32, device=DEV)
+    decay = torch.tensor([0.9, 0.99, 0.5][:H], dtype=torch.float32, device=DEV)
+    cu, _, slots = _step(lengths, [0, 2, 1])
+    a = _rand(g, 3, H * dim * vdim, scale=0.2)
+    b = a.clone()
+    got = ops.retention_scan(rows, H, dim, vdim, inv_freq, positions, decay, dim ** -0.5, 1e-6, a, slots, cu, dtype, max_q_len=max(lengths))
+    want = twin.retention_scan(rows, H, dim, vdim, inv_freq, positions, decay, dim ** -0.5, 1e-6, b, slots, cu, dtype)
+    _close(got, want, _tol(dtype))
+    _close(a, b, 1e-4)
+
+
 def _paged(g, lengths_before, lengths, page, G, dim, vdim, dtype):
     """A cache in which every sequence already holds some tokens, on pages in shuffled order."""
     B = len(lengths)
