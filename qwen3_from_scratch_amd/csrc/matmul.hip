@@ -894,6 +894,12 @@ extern "C" int q3_gemm_tiles(const void* x, const void* w, void* out, int M, int
   return Q3_ERR_BAD_ARGUMENT;
 }
 
+// The tile shape for a product with SwiGLU as its epilogue (q3_gemm_tiles) of a size that its tiles cover in one round, -1 for others.
+extern "C" int q3_swiglu_one_round(int M, int N, int K) {
+  std::lock_guard<std::mutex> hold(g_lock);
+  return g_kernels == KERNELS_BOTH ? tiles::one_round_swiglu(M, N, K) : -1;
+}
+
 // 0: sizes get their kernels by the table and the rules (the default); 1: the tuner times the candidates of
 // every size it first meets outside a capture. Sizes already settled keep their kernel.
 extern "C" int q3_matmul_set_mode(int mode) {
@@ -946,7 +952,7 @@ extern "C" int q3_matmul_table_add(int kind, int rows, int N, int K, int out_dty
   const bool of_groups = own >= GROUPS_FIRST && own < GROUPS_FIRST + groups::NUM_SHAPES && kind != KIND_PLAIN && kind != KIND_ROUND;
   const bool of_rounds = own >= ROUNDS_FIRST + rounds::LEAST && own <= ROUNDS_FIRST + rounds::MOST && kind == KIND_ROUND;
   if (library < 0 || library >= MAX_CANDIDATES || splits < 1 || splits > ((of_groups || of_rounds) ? 1 : 64) ||
-      !(own < tiles::NUM_CONFIGS || of_groups || of_rounds))
+      !(own < tiles::TABLE_CONFIGS || of_groups || of_rounds))
     return Q3_ERR_BAD_ARGUMENT;
   std::lock_guard<std::mutex> hold(g_lock);
   Choice c;

@@ -751,6 +751,24 @@ def test_linear_from_the_tiled_copy(M, N, K):
         torch.testing.assert_close(got.float(), plain.float(), rtol=2e-2, atol=2e-2 * float(plain.float().abs().max()))
 
 
+# one round of tiles of 288 x 192, their last rows and columns cut short; and sizes on the other side of each line of the rule
+@pytest.mark.parametrize("M,N,K,takes", [(535, 22528, 2048, True), (513, 24572, 2112, True), (576, 24576, 2048, True), (288, 49152, 2048, True),
+                                         (257, 46004, 2048, True), (512, 24576, 2048, False), (577, 24576, 2048, False), (535, 20480, 2048, False),
+                                         (535, 24580, 2048, False), (256, 49152, 2048, False), (535, 24576, 1984, False)])
+def test_swiglu_in_one_round(M, N, K, takes):
+    ops = _ops()
+    assert (ops.library("matmul").q3_swiglu_one_round(M, N, K) >= 0) == takes
+    if not takes:
+        return
+    x, w = _rand((M, K), torch.bfloat16, 54), _rand((N, K), torch.bfloat16, 55, scale=0.05)
+    got = ops.linear_swiglu(x, w)
+    product = (x.float() @ w.float().T).to(torch.bfloat16).double()
+    want = torch.nn.functional.silu(product[:, 0::2]) * product[:, 1::2]
+    torch.testing.assert_close(got.double(), want, rtol=3.2e-2, atol=2e-2)         # gate and up are a bfloat16 rounding off at most, each
+    odd = torch.empty(M * K + 1, dtype=torch.bfloat16, device="cuda")[1:].view(M, K).copy_(x)     # (rows that the copies' sixteen bytes do not fit)
+    torch.testing.assert_close(ops.linear_swiglu(odd, w).double(), want, rtol=3.2e-2, atol=2e-2)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("M,I,K", [(1, 12288, 4096), (8, 100, 72), (16, 333, 200), (40, 64, 64)])
 def test_linear_swiglu(dtype, M, I, K):
