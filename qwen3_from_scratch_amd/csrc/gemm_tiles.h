@@ -361,8 +361,8 @@ __global__ __launch_bounds__(256) void tiles_residual_kernel(const float* __rest
   if (threadIdx.x == 0) sums[(size_t)blockIdx.x * sums_stride + m] = total;
 }
 
-// The tile shapes on offer, and those of them that a table may name (the last has a rule of its own, `one_round_swiglu`).
-constexpr int NUM_CONFIGS = 10, TABLE_CONFIGS = 9;
+// The tile shapes on offer: (BM, BN, STAGES).
+constexpr int NUM_CONFIGS = 9;
 
 // `splits` > 1: K is shared out over that many blocks per tile, which leave float32 partial
 // products in `partials` (splits x M x N floats) for a second kernel to add, which also applies
@@ -412,7 +412,7 @@ inline int splits_that_fill(int config, int M, int N, int K) {
   // tile rows, tile columns, blocks resident at once on 256 CUs (what shared memory allows)
   static const int shape[NUM_CONFIGS][3] = {{128, 128, 512}, {128, 128, 256}, {256, 128, 256}, {256, 256, 256},
                                             {256, 256, 256}, {64, 128, 512}, {64, 128, 768}, {64, 256, 512},
-                                            {64, 128, 256}, {288, 192, 256}};
+                                            {64, 128, 256}};
   if (config < 0 || config >= NUM_CONFIGS) return 1;
   const int bm = shape[config][0], bn = shape[config][1], slots = shape[config][2];
   const long tiles = (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
@@ -436,23 +436,8 @@ int launch(int config, const void* x, const void* w, void* out, int M, int N, in
     case 6: return launch_config<OUT, EPI, 64, 128, 1, 4, 2>(x, w, out, M, N, K, splits, partials, stream, scale, keep_partials, splits_used);
     case 7: return launch_config<OUT, EPI, 64, 256, 1, 8, 2>(x, w, out, M, N, K, splits, partials, stream, scale, keep_partials, splits_used);
     case 8: return launch_config<OUT, EPI, 64, 128, 1, 4, 5>(x, w, out, M, N, K, splits, partials, stream, scale, keep_partials, splits_used);
-    case 9: return launch_config<OUT, EPI, 288, 192, 6, 2, 2>(x, w, out, M, N, K, splits, partials, stream, scale, keep_partials, splits_used);
   }
   return Q3_ERR_BAD_ARGUMENT;
-}
-
-// The shape whose tiles cover a product with SwiGLU in one round of blocks where the library's, 256 rows high, need a row of tiles more,
-// else -1. Twelve wavefronts of 48 x 96, three a SIMD, 768 threads: the copies of 288 + 192
-// rows divide evenly. Product and activation, microseconds, the library's with the activation's kernel / this: 535 rows of 24,576 x 2,048, 4,096, 5,120 and
-// 8,192 74.2 / 65.5, 127.0 / 111.9, 160.1 / 134.6 and 225.9 / 205.2, 576 of them 74.7 / 66.4 to 229.0 / 209.3; of 22,528 x 4,096 (85 percent of what 256 such tiles
-// hold) 120.8 / 108.5; 280 of 40,960 x 4,096 (81) 132.9 / 125.1. But 512 of 24,576 x 4,096 (the library's two rows of tiles) 95.9 / 110.2, 576 of 20,480 x 4,096, where
-// its three rows come out even, 85.1 / 110.2; 864 of 16,128 x 4,096 107.3 / 111.2. (192 x 192 in three stages: 535 rows 139.6, 299 77.5 and 78.4 by the library.)
-inline int one_round_swiglu(int M, int N, int K) {
-  constexpr int CONFIG = 9, BM = 288, BN = 192;
-  const long rows = (M + BM - 1) / BM, columns = (N + BN - 1) / BN;
-  if (!(M > 256 && M <= 2 * BM && rows < (M + 255) / 256 && K >= 2048 && K % BK == 0 && N % 4 == 0 && rows * columns <= 256)) return -1;
-  const double share = (double)M * N / (256.0 * BM * BN);
-  return share >= (M <= BM ? 0.81 : 0.84) ? CONFIG : -1;
 }
 
 // Whether the kernel takes a product at all.

@@ -40,6 +40,7 @@
 #include "gemm_stream.h"
 #include "gemm_groups.h"
 #include "gemm_rounds.h"
+#include "gemm_wide.h"
 
 #include <hipblaslt/hipblaslt.h>
 
@@ -49,7 +50,7 @@
 #include <vector>
 
 #define Q3_ERR_LIBRARY 20000   // + the library's status
-#define Q3_DECLINED 1          // q3_tiles_residual: nothing was done, the caller's other way is the one for this size
+#define Q3_DECLINED 1          // q3_tiles_residual, q3_wide_swiglu: nothing was done, the caller's other way is the one for this size
 
 namespace {
 
@@ -894,11 +895,16 @@ extern "C" int q3_gemm_tiles(const void* x, const void* w, void* out, int M, int
   return Q3_ERR_BAD_ARGUMENT;
 }
 
-// The tile shape for a product with SwiGLU as its epilogue (q3_gemm_tiles) of a size that its tiles cover in one round, -1 for others.
-extern "C" int q3_swiglu_one_round(int M, int N, int K) {
-  std::lock_guard<std::mutex> hold(g_lock);
-  return g_kernels == KERNELS_BOTH ? tiles::one_round_swiglu(M, N, K) : -1;
+// Gate and up with the activation (gemm_wide.hip): Q3_DECLINED, and nothing is done, for a size that it is not for.
+extern "C" int q3_wide_swiglu(const void* x, const void* w, void* out, int M, int N, int K, void* stream) {
+  {
+    std::lock_guard<std::mutex> hold(g_lock);
+    if (g_kernels != KERNELS_BOTH) return Q3_DECLINED;
+  }
+  if (!x || !w || !out || !wide::takes(M, N, K) || (((size_t)x | (size_t)w) & 15) || ((size_t)out & 7)) return Q3_DECLINED;
+  return wide::launch(x, w, out, M, N, K, (hipStream_t)stream);
 }
+extern "C" int q3_wide_swiglu_takes(int M, int N, int K) { return wide::takes(M, N, K); }
 
 // 0: sizes get their kernels by the table and the rules (the default); 1: the tuner times the candidates of
 // every size it first meets outside a capture. Sizes already settled keep their kernel.
@@ -952,7 +958,7 @@ extern "C" int q3_matmul_table_add(int kind, int rows, int N, int K, int out_dty
   const bool of_groups = own >= GROUPS_FIRST && own < GROUPS_FIRST + groups::NUM_SHAPES && kind != KIND_PLAIN && kind != KIND_ROUND;
   const bool of_rounds = own >= ROUNDS_FIRST + rounds::LEAST && own <= ROUNDS_FIRST + rounds::MOST && kind == KIND_ROUND;
   if (library < 0 || library >= MAX_CANDIDATES || splits < 1 || splits > ((of_groups || of_rounds) ? 1 : 64) ||
-      !(own < tiles::TABLE_CONFIGS || of_groups || of_rounds))
+      !(own < tiles::NUM_CONFIGS || of_groups || of_rounds))
     return Q3_ERR_BAD_ARGUMENT;
   std::lock_guard<std::mutex> hold(g_lock);
   Choice c;

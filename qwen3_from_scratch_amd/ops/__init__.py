@@ -2366,10 +2366,12 @@ def linear_swiglu(x, weight, tiled=None, unscaled=None, kind="silu", narrow=None
     if unscaled is not None:
         raise OperandError("unscaled rows need bfloat16 and few rows with a tiled weight (few_rows_limit), or 17 to "
                            "128 rows (640 of a small weight, fused_rows_most) with an inner size that is a multiple of 64")
-    if x.dtype == torch.bfloat16 and M > 256 and (x.data_ptr() | weight.data_ptr()) % 16 == 0:
-        shape = library("matmul").q3_swiglu_one_round(M, N, K)
-        if shape >= 0:
-            return gemm_tiles(x, weight, shape, swiglu=True)
+    if x.dtype == torch.bfloat16 and 256 < M <= 576:                  # (what gemm_wide.hip may take)
+        out = torch.empty((M, N // 2), dtype=x.dtype, device=x.device)
+        status = library("matmul").q3_wide_swiglu(_ptr(x), _ptr(weight), _ptr(out), M, N, K, _stream())
+        if status != _DECLINED:
+            _check(status, "linear_swiglu")
+            return out
     if M and library("gemm").q3_linear_is_skinny(M, N, K, _DT[x.dtype]):
         out = torch.empty((M, N // 2), dtype=x.dtype, device=x.device)
         _check(library("gemm").q3_linear_swiglu(_ptr(x), _ptr(weight), _ptr(out), M, N, K, _DT[x.dtype], _stream()),

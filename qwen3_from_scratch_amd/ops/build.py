@@ -33,11 +33,11 @@ FLAGS = [
 MODULES = ("elementwise", "norm", "rotary", "attention", "attention_capped", "attention_pooled", "attention_sigmoid", "attention_span", "latent", "moe",
            "hyper", "recurrent", "mamba2", "rglru", "mlstm", "delta", "softcap", "gemm", "matmul", "sampling", "probes", "layers", "decode_layers")
 # A module's further sources, compiled on their own: their kernels are code objects of their own in its library. Where a kernel's
-# code lies decides how long a launch of it takes to get going: with the kernels of these two between those of matmul.hip, the
+# code lies decides how long a launch of it takes to get going: with the kernels of the first two between those of matmul.hip, the
 # tiled and the weight-streaming product of a step of 64 requests of the 8B shape took 11.7 and 39.9 us with the instructions
 # that had taken 10.9 and 39.1, and take 11.1 and 39.4 so. (As many misses in the instruction cache, but longer ones: 7,440 requests
 # of a weight-streaming launch met one under way, 4,420 before and so.)
-FURTHER = {"matmul": ["gemm_groups.hip", "gemm_rounds.hip"]}
+FURTHER = {"matmul": ["gemm_groups.hip", "gemm_rounds.hip", "gemm_wide.hip"]}
 # what a module links besides the HIP runtime
 LINKS = {"matmul": ["-lhipblaslt"]}
 

@@ -757,7 +757,7 @@ def test_linear_from_the_tiled_copy(M, N, K):
                                          (535, 24580, 2048, False), (256, 49152, 2048, False), (535, 24576, 1984, False)])
 def test_swiglu_in_one_round(M, N, K, takes):
     ops = _ops()
-    assert (ops.library("matmul").q3_swiglu_one_round(M, N, K) >= 0) == takes
+    assert bool(ops.library("matmul").q3_wide_swiglu_takes(M, N, K)) == takes
     if not takes:
         return
     x, w = _rand((M, K), torch.bfloat16, 54), _rand((N, K), torch.bfloat16, 55, scale=0.05)
