@@ -1653,7 +1653,7 @@ static int prompt_key_splits(int total_tokens, int G, int Hkv, int max_kv_len) {
   constexpr int SOME = 40, MANY = 48;
 #endif
   if (key_tiles < SOME) return 1;
-  const int tpb = (key_tiles < MANY ? 32 : 128) / G, enough = key_tiles < MANY ? 257 : 512;
+  const int tpb = max(1, (key_tiles < MANY ? 32 : 128) / G), enough = key_tiles < MANY ? 257 : 512;    // (a group of many heads: one that the kernels do not take)
   int ks = 1;
   while (Hkv * ((total_tokens + tpb - 1) / tpb) * ks < enough && ks < 4) ks *= 2;
   return ks;
