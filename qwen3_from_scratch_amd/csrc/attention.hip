@@ -1515,8 +1515,12 @@ __device__ __forceinline__ int sequence_of_tile(int& n, const int* __restrict__ 
 // prompt kernel / this, groups of two and four heads over 8 of 128 (blocks here): three prompts of 33, 67 and 101 tokens 8.9 / 7.8 (216) and 9.1 / 10.3
 // (416); one of 200 9.6 / 8.7 (200) and 9.7 / 11.2 (400); 64 rows over 512 keys 11.4 / 11.0 and 11.5 / 11.0; 32 over 1,000 19.8 / 15.7, over
 // 1,900 31.6 / 23.3; 220 over 1,900 31.5 / 23.6 (224) and 32.0 / 40.1 (440); 150 over 600 14.1 / 12.1 (152) and 14.2 / 17.7 (304); 300 over 300
-// 11.0 / 11.6 (304); eight prompts of 16 7.4 / 7.5 (256).
+// 11.0 / 11.6 (304); eight prompts of 16 7.4 / 7.5 (256). Nearly two of them where the few rows of one portion stand behind more keys than the
+// decoding requests beside them (20 rows over 820 keys beside 36 requests over 150, 312 blocks, 21.6 / 18.2; 100 over 900 beside 16, groups of
+// four, 328, 21.1 / 18.5), and where uneven prompts would have the prompt kernel launch more blocks than that, most of which find no rows (500 and
+// three of 20, eight single heads, 13.7 / 11.4).
 #define SHORT_BLOCKS 256
+#define SHORT_BLOCKS_MOST 448
 template <int D>
 __global__ __launch_bounds__(64 * DECODE_WAVES) Q3_DECODE_WAVES void attn_short_kernel(
     const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, const bf16_t* __restrict__ k_cache,
@@ -1538,12 +1542,8 @@ __global__ __launch_bounds__(64 * DECODE_WAVES) Q3_DECODE_WAVES void attn_short_
 // and row tile, of as many row tiles as the sequences can come to; the last find none), the others for the decoding ones (splits x Hkv x
 // sequences). The decoding ones wait for memory and the prompts' for the matrix cores and the vector unit; a block of either
 // takes half a CU's registers and shared memory, so they run side by side. The kind that comes first (both in multiples of
-// eight blocks, so that a key head's blocks stay on its chiplet) is the prompts', whose chains are longer, where there are 128 pairs of decoding
-// sequences and key heads or they leave half of the room, else the decoding one. Prompts first / decoding first, microseconds, 32 heads in groups of
-// four: 23 requests over 150 to 3,000 keys beside 276 rows over 1,300 54.1 / 62.5, 512 over 512 47.8 / 47.7, over 1,536 57.4 / 64.2, over 3,584 92.5 /
-// 106.5, 1,400 over 1,400 58.1 / 65.9; 15 beside 1,000 over 1,000 44.2 / 56.4; 40 over 1,000 beside it 45.9 / 54.9, 40 over 150 to 3,000 beside 276 over
-// 1,300 78.7 / 69.5 (the one size of these that loses much). Ten (80 pairs) beside 512 over 512 (512 blocks) 38.6 / 34.3, over 3,584 86.3 / 81.2; beside 276 over
-// 1,300 (280) 37.7 / 43.5; two beside 512 over 512 19.8 / 21.2. One kernel after the other took 68 beside the second of these, 80 over 1,024 (51 so).
+// eight blocks, so that a key head's blocks stay on its chiplet): `plan_prompts`. One kernel after the other, 23 requests over 150 to 3,000 keys beside
+// 512 rows over 512 keys took 68 us, over 1,024 80; in one launch 48 and 51.
 template <int D, int TILE, int STAGES, int KEYS, int QB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_mixed_kernel(
     const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, const bf16_t* __restrict__ k_cache,
@@ -1631,57 +1631,96 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(bf16_t* __restr
 // the chip twice (a portion of 512 tokens of one prompt: 128 blocks, each a chain of as many
 // tiles as the prefix is long), the keys are split over up to four blocks
 // and a block's rows are halved, down to 32.
+static inline int pieces(long n, int each) { return (int)((n + each - 1) / each); }
+struct PromptPlan {
+  int tokens;             // a block's
+  bool prompts_first;     // of a mixed launch
+  bool brief;             // sixteen rows a block instead, of whatever sequence (attn_short_kernel)
+};
 #if !defined(Q3_POOLED) && !defined(Q3_SIGMOID) && !defined(Q3_SPAN)
 // A halved block's wavefronts share its keys (prefill_block's KEYS), so its chain is half as long too and nothing has to be merged
-// behind the kernel: rows first, while there are 288 blocks at most, since two run on a CU at once and a few more behind those are short (2,300 rows of 16
-// heads in pairs, 288 blocks, 64.9, 50.5 halved; 1,100 of 32 in fours, 280, 37.2 and 34.2; with a window, whose chains are short, fewer than 256: 1,100 over
-// 128 of them 17.8 and 25.4, 1,024, 256 blocks, 14.4 and 15.8); from 3,072 keys on
-// first the keys (from 2,560 on as many parts as the least rows leave room for). 32 heads in groups of four, rows of a block * parts of the keys, microseconds,
-// 128*1 / 64*1 / 32*1 / 128*4: 512 over 512 19.9 / 17.0 / 13.0 / 36; over 2,048 52.6 / 41.0 / 34.4 / 45.4; over 4,096 95.2 / 71.8 / 60.2 / 60.2, over
+// behind the kernel: rows first, and from 2,048 keys on as many parts of the keys as the least rows leave room for; from 4,096
+// on the keys first. 32 heads in groups of four, rows of a block * parts of the keys, microseconds, 128*1 / 64*1 / 32*1 / 128*4: 512 over
+// 512 19.9 / 17.0 / 13.0 / 36; over 2,048 52.6 / 41.0 / 34.4 / 45.4; over 4,096 95.2 / 71.8 / 60.2 / 60.2, over
 // 8,000 176 / 131 / 124 / 93; 276 over 1,300 39.4 / 31.0 / 25.1 / 39.0; 1,024 over 1,024 32.3 / 27.6 / 31.6 / 48; 1,000 over 2,000 55 / 47 / 59 / 64; 2,048 of one
-// prompt (512 blocks) 56.4 / 71.8 / 83.3 / 88. 128 over 2,048 in 32*1 25.1, 32*4 31.0, over 4,096 41.8 and 37.9; 256 over 4,096 32*1 55.4, 32*2 44.4.
-// Capped scores, whose tiles take longer, from 2,048 keys on: 2,048 rows of 16 heads in fours over 2,048 keys 46.8 and 12 for the merge in 128*2, 65 in 64*1.
-// Beside the decoding sequences of a mixed launch blocks of many rows leave those more of the CUs: with 128 of their pairs or more the rows are
-// halved below 128 blocks only. 23 requests over 150 to 3,000 keys beside 512 over 512 47.0 in 128 rows, 48.3 in 64, 49.4 in 32; beside 512 over
-// 1,536 56.3, 64.9; beside 276 over 1,300 57.5, 52.8, 57.0 (80, 152 and 296 blocks); 40 over 1,000 beside 512 over 1,536 52.3, 62.9; eight over 1,000 beside
-// 276 over 1,300 40.3, 38.3, 36.1.
+// prompt (512 blocks) 56.4 / 71.8 / 83.3 / 88. 128 over 2,048 in 32*1 25.1, 32*4 31.0, over 4,096 41.8 and 37.9; 256 over 4,096 32*1 55.4, 32*2 44.4; 276 over
+// 2,300, 16 heads in pairs, 32*1 36.7, 32*2 29.3; 276 over 3,100, 32 in fours, 64*4 55.4, 32*1 47.3. 64 over 2,000, 32 in fours, 32*4 28.2, by
+// attn_short_kernel 24.4, 16 in pairs 21.6 and 24.4.
+// Capped scores, whose tiles take longer, keys first from 2,048 on: 2,048 rows of 16 heads in fours over 2,048 keys 46.8 and 12 for the merge in 128*2, 65 in 64*1.
 static int prompt_key_splits(int total_tokens, int G, int Hkv, int max_kv_len) {
-  const int key_tiles = (max_kv_len + PF_TILE - 1) / PF_TILE;
+  const int key_tiles = pieces(max_kv_len, PF_TILE);
 #ifdef Q3_SCORE_CAP
-  constexpr int SOME = 32, MANY = 32;
+  constexpr int MANY = 32;
 #else
-  constexpr int SOME = 40, MANY = 48;
+  constexpr int MANY = 64;
 #endif
-  if (key_tiles < SOME) return 1;
+  // (up to 2,560 keys so few rows are attn_short_kernel's)
+  if (key_tiles < (MANY > 32 && Hkv * pieces(total_tokens, max(1, 16 / G)) <= SHORT_BLOCKS ? 40 : 32)) return 1;
   const int tpb = max(1, (key_tiles < MANY ? 32 : 128) / G), enough = key_tiles < MANY ? 257 : 512;    // (a group of many heads: one that the kernels do not take)
   int ks = 1;
-  while (Hkv * ((total_tokens + tpb - 1) / tpb) * ks < enough && ks < 4) ks *= 2;
+  while (Hkv * pieces(total_tokens, tpb) * ks < enough && ks < 4) ks *= 2;
   return ks;
 }
 
-static int prompt_tokens_per_block(int total_tokens, int G, int Hkv, int key_splits, int window, long decode_pairs) {
-  int tpb = 128 / G;
-  const int enough = decode_pairs >= 128 ? 128 : window ? 256 : 289;
-  while (Hkv * ((total_tokens + tpb - 1) / tpb) * key_splits < enough && (tpb / 2) * G >= 32) tpb /= 2;
-  return tpb;
+// How many blocks rows of `tokens` come to counts what is left over at the end of each prompt, of which there are as many by the host's
+// bounds as there must be if all are as long as the longest. 16 prompts of 70, 32 heads in fours, 128 rows a
+// block (384 blocks, where the rows alone would fill 280) 15.8, 64 (640) 21.6; 16 of 130, 16 in pairs 16.2 and 22.0; eight of 130 15.6 and 19.8.
+// - Rows are halved while half of them hold the longest prompt (64 of 20 tokens, eight single heads, 32 rows a block 10.4, 128 12.8), and while there
+//   are 288 blocks at most, since two run on a CU at once and a few more behind those are short (2,300 rows of 16 heads in pairs, 288 blocks, 64.9, 50.5
+//   halved; 1,100 of 32 in fours, 280, 37.2 and 34.2; 512 of 64 in eights, 256, 21.3 and 19.2). Several prompts with short chains from 128 rows below 256
+//   blocks only (seven of 300, 16 in pairs, 280, 19.6 and 22.1; but from 64 rows eight of 64, 32 in fours, 256, 10.1 and 8.5), and with a window
+//   (1,100 over 128 17.8 and 25.4, 1,024, 256 blocks, 14.4 and 15.8).
+// - In a mixed launch blocks of many rows leave the decoding sequences more of the CUs: with 160 pairs of those and key heads rows are halved below 144
+//   blocks only (28 over 150 to 3,000 keys beside 512 over 512, 32 heads in fours, 128 rows 54.0, 64 74.0; beside 512 over 1,536 59 and 85).
+// - The prompts' blocks, whose chains are longer, come first, prompts first / decoding first: 23 over 150 to 3,000 beside 276 over 1,300
+//   52.1 / 57.7, 28 beside 1,400 over 1,400 61.2 / 71.8, 32 beside 512 over 1,536 60 / 87, 64 over 150 to 2,000 beside it 64 / 93. Not where many
+//   contexts are left whole and the prompts' keys are a fifth of theirs at most, so that the decoding ones are the longer chains: 40 over 150 to 3,000
+//   beside 512 over 512 75.9 / 62.6, 48 82 / 74, 28 beside four prompts of 300 64.3 / 51.7. Nor where more than 512 blocks fill the chip by themselves
+//   and are parts of keys or two thirds as long: 23 beside 512 over 3,584 102 / 84, 32 106 / 102; one over 3,000 beside 15 prompts of 130 34.3 / 27.8; 40 over
+//   150 to 3,000 beside 1,400 over 1,400, 64 heads in eights, 120 / 97 (but 64 over 200 to 1,000 80 / 86).
+// Over 1,375 sizes of six groupings of heads these rules take 2 percent less time than one line for all (289 blocks, 128 of them from 128 pairs
+// on, counted by rows alone) and 2.9 percent more than the best choice at each.
+static PromptPlan plan_prompts(int total_tokens, int B, int G, int Hkv, int key_splits, int splits, int window, int max_q_len, int min_q_len,
+                               int longest, int max_kv_len) {
+  const bool few = min_q_len * G <= 16;
+  const int prompts = window ? 1 : max(1, min(B, pieces(max(0, total_tokens - B), max_q_len))), others = few ? B - prompts : 0;
+  const bool beside_many = window == 0 && (long)Hkv * others >= 160;
+  auto blocks = [&](int tokens) {
+    const int rows = pieces(total_tokens, tokens);
+    return (long)Hkv * key_splits * (prompts > 1 ? max(rows, prompts * pieces(pieces(total_tokens - others, prompts), tokens)) : rows);
+  };
+  auto enough = [&](int tokens) {
+    return beside_many ? 144 : window || (tokens * G > 64 && prompts > 1 && longest < 1000) ? 256 : 289;
+  };
+  PromptPlan plan{128 / G, false, false};
+  auto halved = [&] { return (plan.tokens / 2) * G >= 32; };
+  while (plan.tokens / 2 >= max_q_len && halved()) plan.tokens /= 2;
+  while (blocks(plan.tokens) < enough(plan.tokens) && halved()) plan.tokens /= 2;
+  const long filled = blocks(plan.tokens);
+  plan.prompts_first = !(filled > 512 && (key_splits > 1 || 3L * longest <= 2L * max_kv_len)) &&
+                       !(beside_many && splits == 1 && 5L * longest <= max_kv_len);
+  const long brief_blocks = (max(0, total_tokens - B) / (16 / G) + B) * (long)Hkv;   // (the most that so many tokens of so many sequences come to)
+  const bool outlasts = few ? prompts == 1 && longest >= max_kv_len : (long)Hkv * pieces(max_q_len, plan.tokens) * B > SHORT_BLOCKS_MOST;
+  plan.brief = window == 0 && splits == 1 && key_splits == 1 && brief_blocks <= (outlasts ? SHORT_BLOCKS_MOST : SHORT_BLOCKS);
+  return plan;
 }
 #else
 // The keys come first, from 2,048 on and as long as a split keeps eight tiles (512 tokens over 3,584 keys: 127 us whole,
 // 97 in two, 88 in four; 256 over 7,936: 224, 141, 97; over 512 keys splitting loses). Of a block of fewer than 128 rows some
 // wavefronts only help to copy the tiles.
 static int prompt_key_splits(int total_tokens, int G, int Hkv, int max_kv_len) {
-  const int tpb = 128 / G;
+  const int tpb = max(1, 128 / G);
   int ks = 1;
-  const int key_tiles = (max_kv_len + PF_TILE - 1) / PF_TILE;
-  while (Hkv * ((total_tokens + tpb - 1) / tpb) * ks < 512 && ks < 4 && key_tiles >= 32 && key_tiles / (2 * ks) >= 8)
+  const int key_tiles = pieces(max_kv_len, PF_TILE);
+  while (Hkv * pieces(total_tokens, tpb) * ks < 512 && ks < 4 && key_tiles >= 32 && key_tiles / (2 * ks) >= 8)
     ks *= 2;
   return ks;
 }
 
-static int prompt_tokens_per_block(int total_tokens, int G, int Hkv, int key_splits, int, long) {
-  int tpb = 128 / G;
-  while (Hkv * ((total_tokens + tpb - 1) / tpb) * key_splits < 256 && (tpb / 2) * G >= 32) tpb /= 2;
-  return tpb;
+static PromptPlan plan_prompts(int total_tokens, int, int G, int Hkv, int key_splits, int, int, int, int, int, int) {
+  PromptPlan plan{128 / G, false, false};
+  while ((long)Hkv * pieces(total_tokens, plan.tokens) * key_splits < 256 && (plan.tokens / 2) * G >= 32) plan.tokens /= 2;
+  return plan;
 }
 #endif
 
@@ -1689,8 +1728,8 @@ template <int D, int DV = D>
 static int launch_fast(const void* q, int q_stride, void* out, const void* k_cache, const void* v_cache,
                        int num_pages, const int* block_table, int bt_stride, const int* cu_q, const int* kv_lens,
                        int B, int total_tokens, int Hq, int Hkv, int page, float scale, int window, int max_q_len,
-                       int min_q_len, int splits, float* ws_acc, float* ws_ml, int key_splits, float* prompt_ws,
-                       const float* sink, hipStream_t stream) {
+                       int min_q_len, int max_kv_len, int longest, int splits, float* ws_acc, float* ws_ml, int key_splits,
+                       float* prompt_ws, const float* sink, hipStream_t stream) {
   const int G = Hq / Hkv;
   const score_scale_t scale_log2 = make_score_scale(scale);
   const span_t span = make_span(window);
@@ -1703,16 +1742,17 @@ static int launch_fast(const void* q, int q_stride, void* out, const void* k_cac
   if (window != 0 || g_score_bias == nullptr || sink != nullptr) return Q3_ERR_BAD_ARGUMENT;
 #endif
   const bool few = min_q_len * G <= 16, many = max_q_len * G > 16;
-  const int tokens_per_block = many ? prompt_tokens_per_block(total_tokens, G, Hkv, key_splits, window, few && window == 0 ? (long)Hkv * B : 0) : 1;
+  const PromptPlan plan = many ? plan_prompts(total_tokens, B, G, Hkv, key_splits, splits, window, max_q_len, min_q_len, longest, max_kv_len)
+                               : PromptPlan{1, false, false};
+  const int tokens_per_block = plan.tokens;
   const int tiles = (max_q_len + tokens_per_block - 1) / tokens_per_block;
   if (many && tiles * key_splits > 65535) return Q3_ERR_UNSUPPORTED;
   float* part_acc = prompt_ws;
   float* part_ml = prompt_ws ? prompt_ws + (size_t)total_tokens * Hq * key_splits * DV : nullptr;
 #if !defined(Q3_POOLED) && !defined(Q3_SIGMOID) && !defined(Q3_SPAN)
-  const int chunk_tokens = 16 / G;
-  const long short_tiles = max(0, total_tokens - B) / chunk_tokens + B;   // (the most that so many tokens of so many sequences come to)
-  if (many && window == 0 && splits == 1 && key_splits == 1 && short_tiles * Hkv <= SHORT_BLOCKS) {
-    hipLaunchKernelGGL(attn_short_kernel<D>, dim3(Hkv, (unsigned)short_tiles), dim3(256), 0, stream, (const bf16_t*)q, q_stride,
+  if (plan.brief) {
+    const int short_tiles = max(0, total_tokens - B) / (16 / G) + B;
+    hipLaunchKernelGGL(attn_short_kernel<D>, dim3(Hkv, short_tiles), dim3(256), 0, stream, (const bf16_t*)q, q_stride,
                        (bf16_t*)out, (const bf16_t*)k_cache, (const bf16_t*)v_cache, num_pages, block_table, bt_stride, cu_q,
                        kv_lens, B, Hq, Hkv, page, scale_log2, sink Q3_GATE_ARG);
     return q3_launch_status();
@@ -1723,8 +1763,6 @@ static int launch_fast(const void* q, int q_stride, void* out, const void* k_cac
   // row tiles of the sequences of many rows: one each beyond whole ones, and as many sequences as there are rows for
   const long row_tiles = total_tokens / tokens_per_block + min(B, total_tokens / (16 / G + 1));
   const long prompt_blocks = (row_tiles * key_splits * Hkv + 7) / 8 * 8, decode_blocks = ((long)splits * Hkv * B + 7) / 8 * 8;
-  const bool prompts_first =
-      (long)Hkv * B >= 128 || (long)((total_tokens + tokens_per_block - 1) / tokens_per_block) * key_splits * Hkv <= 288;
   together = few && many && window == 0 && (prompt_blocks + decode_blocks) * 256 < (1L << 32);
   const int rows = tokens_per_block * G;
   const auto prompt_kernel = rows > 64 ? attn_prefill_kernel<D, TILE, PF_STAGES, DV> : rows > 32 ? attn_prefill_kernel<D, TILE, PF_STAGES, DV, 2>
@@ -1735,8 +1773,8 @@ static int launch_fast(const void* q, int q_stride, void* out, const void* k_cac
   if (together)
     hipLaunchKernelGGL(mixed_kernel, dim3((unsigned)(prompt_blocks + decode_blocks)), dim3(256), 0,
                        stream, (const bf16_t*)q, q_stride, (bf16_t*)out, (const bf16_t*)k_cache, (const bf16_t*)v_cache,
-                       num_pages, block_table, bt_stride, cu_q, kv_lens, B, Hq, Hkv, page, scale_log2, prompts_first ? 1 : 0,
-                       (int)(prompts_first ? prompt_blocks : decode_blocks), tokens_per_block, key_splits, part_acc, part_ml,
+                       num_pages, block_table, bt_stride, cu_q, kv_lens, B, Hq, Hkv, page, scale_log2, plan.prompts_first ? 1 : 0,
+                       (int)(plan.prompts_first ? prompt_blocks : decode_blocks), tokens_per_block, key_splits, part_acc, part_ml,
                        splits, ws_acc, ws_ml, sink Q3_GATE_ARG);
 #else
   const auto prompt_kernel = attn_prefill_kernel<D, TILE, PF_STAGES, DV>;
@@ -1832,14 +1870,24 @@ extern "C" int q3_paged_attention_prompt_splits(int T, int Hq, int Hkv, int max_
   return prompt_key_splits(T, Hq / Hkv, Hkv, max_kv_len);
 }
 
-// `splits`, `workspace`: for the sequences of few rows (q3_paged_attention_workspace);
+// How `q3_paged_attention` shares out the rows of a step with sequences of many (see plan_prompts): a block's tokens, plus 256 where a mixed
+// launch has the prompts' blocks first, plus 512 where sixteen rows a block serve instead. Sizes of the fast path only.
+extern "C" int q3_paged_attention_plan(int T, int B, int Hq, int Hkv, int prompt_splits, int splits, int window, int max_q_len, int min_q_len,
+                                       int longest, int max_kv_len) {
+  if (T <= 0 || B <= 0 || Hkv <= 0 || Hq < Hkv || Hq % Hkv || Hq / Hkv > 16 || max_q_len <= 0 || max_q_len * (Hq / Hkv) <= 16) return 0;
+  const PromptPlan plan = plan_prompts(T, B, Hq / Hkv, Hkv, prompt_splits, splits, window, max_q_len, min_q_len, longest, max_kv_len);
+  return plan.tokens + (plan.prompts_first ? 256 : 0) + (plan.brief ? 512 : 0);
+}
+
+// `max_kv_len` bounds the sequences' keys, `longest` those of the ones that bring many rows (both choose between ways of sharing the
+// work out alone). `splits`, `workspace`: for the sequences of few rows (q3_paged_attention_workspace);
 // `prompt_splits` (1, 2 or 4), `prompt_workspace`: for those of many. `sink` (Hq floats, or null):
 // head h's softmax has exp(sink[h]) as one more term of its denominator, unscaled and without a value.
 extern "C" int q3_paged_attention(const void* q, int q_stride, void* out, const void* k_cache,
                                   const void* v_cache, int num_pages, const int* block_table,
                                   int bt_stride, const int* cu_q, const int* kv_lens, int B, int T_, int Hq,
                                   int Hkv, int D, int page, float scale, int window, int max_q_len,
-                                  int min_q_len, int max_kv_len, int dtype, int splits, float* workspace,
+                                  int min_q_len, int max_kv_len, int longest, int dtype, int splits, float* workspace,
                                   int prompt_splits, float* prompt_workspace, const float* sink,
                                   hipStream_t stream) {
   if (B <= 0 || T_ <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv || page <= 0 || max_q_len <= 0 || min_q_len <= 0 ||
@@ -1851,7 +1899,6 @@ extern "C" int q3_paged_attention(const void* q, int q_stride, void* out, const 
     if (splits < 1 || splits > MAX_SPLITS || (splits > 1 && workspace == nullptr)) return Q3_ERR_BAD_ARGUMENT;
     if (prompt_splits < 1 || prompt_splits > 4 || (prompt_splits > 1 && prompt_workspace == nullptr))
       return Q3_ERR_BAD_ARGUMENT;
-    (void)max_kv_len;
     if (!k_cache || !v_cache) return Q3_ERR_BAD_ARGUMENT;    // (tiles without a page read the first one: TileAddr)
     float* ws_acc = workspace;
 #ifdef Q3_SPAN
@@ -1862,8 +1909,8 @@ extern "C" int q3_paged_attention(const void* q, int q_stride, void* out, const 
 #define Q3_SPAN_LAUNCH(KD, VD)                                                                                           \
   if (D == KD && DV == VD)                                                                                               \
   return launch_fast<KD, VD>(q, q_stride, out, k_cache, v_cache, num_pages, block_table, bt_stride, cu_q, kv_lens, B, T_, \
-                             Hq, Hkv, page, scale, window, max_q_len, min_q_len, splits, ws_acc, ws_ml, prompt_splits,    \
-                             prompt_workspace, sink, stream)
+                             Hq, Hkv, page, scale, window, max_q_len, min_q_len, max_kv_len, longest, splits, ws_acc,     \
+                             ws_ml, prompt_splits, prompt_workspace, sink, stream)
     Q3_SPAN_LAUNCH(64, 64);
     Q3_SPAN_LAUNCH(64, 128);
     Q3_SPAN_LAUNCH(96, 64);
@@ -1880,10 +1927,10 @@ extern "C" int q3_paged_attention(const void* q, int q_stride, void* out, const 
     float* ws_ml = workspace ? workspace + (size_t)B * Hkv * splits * 16 * D : nullptr;
     if (D == 64)
       return launch_fast<64>(q, q_stride, out, k_cache, v_cache, num_pages, block_table, bt_stride, cu_q, kv_lens,
-                             B, T_, Hq, Hkv, page, scale, window, max_q_len, min_q_len, splits, ws_acc, ws_ml,
+                             B, T_, Hq, Hkv, page, scale, window, max_q_len, min_q_len, max_kv_len, longest, splits, ws_acc, ws_ml,
                              prompt_splits, prompt_workspace, sink, stream);
     return launch_fast<128>(q, q_stride, out, k_cache, v_cache, num_pages, block_table, bt_stride, cu_q, kv_lens, B,
-                            T_, Hq, Hkv, page, scale, window, max_q_len, min_q_len, splits, ws_acc, ws_ml,
+                            T_, Hq, Hkv, page, scale, window, max_q_len, min_q_len, max_kv_len, longest, splits, ws_acc, ws_ml,
                             prompt_splits, prompt_workspace, sink, stream);
   }
 #if defined(Q3_SCORE_CAP) || defined(Q3_POOLED) || defined(Q3_SIGMOID)

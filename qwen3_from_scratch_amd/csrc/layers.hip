@@ -18,7 +18,7 @@ typedef int (*prepare_t)(void* qkv, const void* q_weight, const void* k_weight, 
                          hipStream_t stream);
 typedef int (*attention_t)(const void* q, int q_stride, void* out, const void* k_cache, const void* v_cache, int num_pages,
                            const int* block_table, int bt_stride, const int* cu_q, const int* kv_lens, int B, int T_, int Hq,
-                           int Hkv, int D, int page, float scale, int window, int max_q_len, int min_q_len, int max_kv_len,
+                           int Hkv, int D, int page, float scale, int window, int max_q_len, int min_q_len, int max_kv_len, int longest,
                            int dtype, int splits, float* workspace, int prompt_splits, float* prompt_workspace,
                            const float* sink, hipStream_t stream);
 
@@ -45,7 +45,7 @@ struct Q3LayerStep {
   const float* table;
   int rotary_dim, max_pos;
   const int *positions, *seq_index, *block_table, *cu_q, *kv_lens;
-  int table_width, sequences, page, num_pages, max_q_len, min_q_len, max_kv_len;
+  int table_width, sequences, page, num_pages, max_q_len, min_q_len, max_kv_len, longest;
   int splits, prompt_splits;
   float *workspace, *prompt_workspace;
   // the stream; the rows that still lack their norm, with `chunks` partial sums of squares a row (`sums_stride` floats apart)
@@ -79,7 +79,7 @@ int q3_decoder_layers(const Q3Layer* layers, int n, const Q3LayerStep* step, int
     if (status) return status;
     status = s.attention(s.qkv_rows, joined, s.attended, l.keys, l.values, s.num_pages, s.block_table, s.table_width, s.cu_q,
                          s.kv_lens, s.sequences, s.rows, s.heads, s.kv_heads, s.dim, s.page, s.scale, s.window, s.max_q_len,
-                         s.min_q_len, s.max_kv_len, Q3_BF16, s.splits, s.workspace, s.prompt_splits, s.prompt_workspace,
+                         s.min_q_len, s.max_kv_len, s.longest, Q3_BF16, s.splits, s.workspace, s.prompt_splits, s.prompt_workspace,
                          nullptr, (hipStream_t)s.stream);
     *failed = 6 * i + 2;
     if (status) return status;

@@ -1874,7 +1874,10 @@ def paged_attention(q, num_q_heads, k_cache, v_cache, block_table, cu_seqlens_q,
                     n = lib.q3_paged_attention_workspace(B, Hkv, vdim, splits)
                     workspace = torch.empty((n,), dtype=torch.float32, device=q.device)
             if max_q_len * (Hq // Hkv) > 16:           # few long sequences over many keys: likewise
-                prompt_splits = lib.q3_paged_attention_prompt_splits(T, Hq, Hkv, int(longest))
+                # (behind a window the keys that a block, of 128 tokens at most, goes through)
+                if window and runs is None and span is None:
+                    longest = min(longest, window + 128)
+                prompt_splits = lib.q3_paged_attention_prompt_splits(T, Hq, Hkv, longest)
                 if prompt_splits > 1:
                     prompt_workspace = torch.empty((T * Hq * prompt_splits * (vdim + 2),), dtype=torch.float32,
                                                    device=q.device)
@@ -1884,7 +1887,7 @@ def paged_attention(q, num_q_heads, k_cache, v_cache, block_table, cu_seqlens_q,
             _ptr(q), q.stride(0), _ptr(out), _ptr(k_cache), _ptr(v_cache), pages,
             _ptr(block_table), block_table.shape[1], _ptr(cu_seqlens_q), _ptr(kv_lens),
             B, T, Hq, Hkv, D, page, ctypes.c_float(scale), int(window), int(max_q_len), int(min_q_len),
-            int(max_kv_len), _DT[q.dtype], splits, _ptr(workspace), prompt_splits, _ptr(prompt_workspace), _ptr(sink),
+            int(max_kv_len), longest, _DT[q.dtype], splits, _ptr(workspace), prompt_splits, _ptr(prompt_workspace), _ptr(sink),
             _stream()),
             "paged_attention")
     return out

@@ -22,7 +22,7 @@ class _Step(ctypes.Structure):
                 + [(n, _I) for n in ("rows", "width", "heads", "kv_heads", "dim", "inner", "norm_dtype", "qk_dtype")]
                 + [("qk_eps", _F), ("scale", _F), ("window", _I), ("table", _P), ("rotary_dim", _I), ("max_pos", _I)]
                 + [(n, _P) for n in ("positions", "seq_index", "block_table", "cu_q", "kv_lens")]
-                + [(n, _I) for n in ("table_width", "sequences", "page", "num_pages", "max_q_len", "min_q_len", "max_kv_len",
+                + [(n, _I) for n in ("table_width", "sequences", "page", "num_pages", "max_q_len", "min_q_len", "max_kv_len", "longest",
                                      "splits", "prompt_splits")]
                 + [(n, _P) for n in ("workspace", "prompt_workspace", "residual_rows", "entry_values", "entry_sums")]
                 + [(n, _I) for n in ("entry_chunks", "sums_stride", "middle_chunks", "exit_chunks")]
@@ -138,9 +138,10 @@ class DecoderLayers:
             if splits > 1:
                 attention.q3_paged_attention_workspace.restype = ctypes.c_long
                 workspace = empty(attention.q3_paged_attention_workspace(B, G, D, splits), dtype=torch.float32)
+        longest = int(max_kv_len if max_kv_len_of_many is None else max_kv_len_of_many)
         if max_q_len * (H // G) > 16:
-            longest = int(max_kv_len if max_kv_len_of_many is None else max_kv_len_of_many)
-            prompt_splits = attention.q3_paged_attention_prompt_splits(T, H, G, longest)
+            prompt_splits = attention.q3_paged_attention_prompt_splits(
+                T, H, G, min(longest, self.window + 128) if self.window else longest)
             if prompt_splits > 1:
                 prompt_workspace = empty(T * H * prompt_splits * (D + 2), dtype=torch.float32)
         out = empty(T, self.width)
@@ -158,7 +159,7 @@ class DecoderLayers:
             norm_dtype=_DT[self.norm_dtype], qk_dtype=_DT[self.qk_dtype], qk_eps=self.qk_eps, scale=self.scale, window=self.window,
             table=at(table), rotary_dim=rotary_dim, max_pos=max_pos, positions=at(positions), seq_index=at(seq_index),
             block_table=at(block_table), cu_q=at(cu_seqlens_q), kv_lens=at(kv_lens), table_width=block_table.shape[1], sequences=B,
-            page=page, num_pages=pages, max_q_len=int(max_q_len), min_q_len=int(min_q_len), max_kv_len=int(max_kv_len),
+            page=page, num_pages=pages, max_q_len=int(max_q_len), min_q_len=int(min_q_len), max_kv_len=int(max_kv_len), longest=longest,
             splits=splits, prompt_splits=prompt_splits, workspace=at(workspace), prompt_workspace=at(prompt_workspace),
             residual_rows=at(stream), entry_values=at(values), entry_sums=at(sums), entry_chunks=sums.shape[0], sums_stride=stride,
             middle_chunks=middle.shape[0], exit_chunks=exit_.shape[0], qkv_rows=at(qkv), attended=at(attended), hidden=at(hidden),
