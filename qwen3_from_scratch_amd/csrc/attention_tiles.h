@@ -80,11 +80,11 @@ static inline float make_score_scale(float scale) { return scale * 1.44269504088
 // maximum stands -bias log2(e), which never moves, so that the argument is formed as an exponent is
 // elsewhere; wherever results are joined every weight is one. `q3_set_sigmoid_bias` names the
 // biases (one per query head) of the launches that follow in the calling thread.
-// The builds with Q3_SCORE_CAP, Q3_POOLED, Q3_SIGMOID or Q3_SPAN also multiply a result by sigmoid(gate) on its way out, where
+// The builds with Q3_CAP_GATED, Q3_POOLED, Q3_SIGMOID or Q3_SPAN also multiply a result by sigmoid(gate) on its way out, where
 // its row is final: `gate` float32, rows `stride` apart, a number per head or (`wide`) one per column;
 // null: no gate. `q3_set_gate` names the gate of the launches that follow in the calling thread. (A kernel of its own behind capped
 // attention took 6 us for 8 rows of 16 heads and 10 for 2,048.)
-#if defined(Q3_POOLED) || defined(Q3_SIGMOID) || defined(Q3_SPAN) || defined(Q3_SCORE_CAP)
+#if defined(Q3_POOLED) || defined(Q3_SIGMOID) || defined(Q3_SPAN) || defined(Q3_CAP_GATED)
 #define Q3_GATED 1
 struct OutGate {
   const float* gate;

@@ -1759,8 +1759,8 @@ def paged_attention(q, num_q_heads, k_cache, v_cache, block_table, cu_seqlens_q,
     softmax, a key counts with sigmoid(s * scale + sigmoid_bias[h]). `span` = (chunk, keep_first): a row at
     position p sees, instead of a window, the keys of its own stretch of `chunk` positions (0: what `window`
     says), and the keys before `keep_first` besides; the values may differ from the keys in size
-    (`span_sizes`). These three are builds of their own as well, and they alone take `gate` float32 (T, Hq) or
-    (T, Hq D), rows possibly apart, whose sigmoid multiplies the result where it is written.
+    (`span_sizes`). These three are builds of their own as well. They and capped scores take `gate` float32 (T, Hq) or
+    (T, Hq D), rows possibly apart, whose sigmoid multiplies the result where it is written (capped scores in a further build).
 
     q is (T, Hq, D) seen through a row stride (a view of the qkv buffer is
     fine). Keys are cached as (pages, Hkv, page, D), values as
@@ -1772,8 +1772,8 @@ def paged_attention(q, num_q_heads, k_cache, v_cache, block_table, cu_seqlens_q,
     `max_q_len` and `min_q_len` bound the sequences' row counts (they choose
     between the kernels for few and for many rows; loose bounds cost time only).
     `max_kv_len_of_many`: the most keys of a sequence that brings many rows, if
-    the caller knows it (it decides whether such sequences' keys are shared out
-    over several blocks; `max_kv_len` stands in).
+    the caller knows it (it decides how such sequences' rows and keys are shared out
+    over blocks; `max_kv_len` stands in).
 
     bfloat16 with head size 64 or 128 and a page size that is a power of two from 16
     runs on the matrix cores, and so do float32 heads of 16, 32, 64 and 128 over pages in steps
@@ -1818,7 +1818,7 @@ def paged_attention(q, num_q_heads, k_cache, v_cache, block_table, cu_seqlens_q,
     if T and B:
         kinds = []
         if softcap > 0 or runs is not None or sigmoid_bias is not None or span is not None:
-            kinds = [kind for kind, on in (("capped", softcap > 0), ("pooled", runs is not None),
+            kinds = [kind for kind, on in (("capped" if gate is None else "capped_gated", softcap > 0), ("pooled", runs is not None),
                                            ("sigmoid", sigmoid_bias is not None), ("span", span is not None)) if on]
         if not (len(kinds) <= 1):
             raise OperandError("capped scores, runs, sigmoid weights and spans exclude each other")
@@ -1857,7 +1857,7 @@ def paged_attention(q, num_q_heads, k_cache, v_cache, block_table, cu_seqlens_q,
                 longest = min(longest, (chunk or window) + keep)
         if not (gate is None or kinds):
             raise OperandError("a gate comes with capped scores, runs, sigmoid weights or spans only")
-        if kinds:
+        if kinds and kinds != ["capped"]:
             gate_stride = 0
             if gate is not None:
                 gate_stride = _rows_view(gate, "gate")

@@ -30,7 +30,7 @@ FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-command-line-argument",
 ]
-MODULES = ("elementwise", "norm", "rotary", "attention", "attention_capped", "attention_pooled", "attention_sigmoid", "attention_span", "latent", "moe",
+MODULES = ("elementwise", "norm", "rotary", "attention", "attention_capped", "attention_capped_gated", "attention_pooled", "attention_sigmoid", "attention_span", "latent", "moe",
            "hyper", "recurrent", "mamba2", "rglru", "mlstm", "delta", "softcap", "gemm", "matmul", "sampling", "probes", "layers", "decode_layers")
 # A module's further sources, compiled on their own: their kernels are code objects of their own in its library. Where a kernel's
 # code lies decides how long a launch of it takes to get going: with the kernels of the first two between those of matmul.hip, the

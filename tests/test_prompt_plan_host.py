@@ -62,10 +62,14 @@ def test_few_rows(heads, lengths, keys, brief):
     assert _plan(heads, lengths, keys)[2] == brief
 
 
-@pytest.mark.parametrize("build", ["attention", "attention_capped", "attention_pooled", "attention_sigmoid", "attention_span"])
+@pytest.mark.parametrize("build", ["attention", "attention_capped", "attention_capped_gated", "attention_pooled", "attention_sigmoid", "attention_span"])
 @pytest.mark.parametrize("group", [1, 16, 33, 64, 129, 500])
 def test_any_group_of_heads_has_an_answer(build, group):
     lib = library(build)
     for keys in (100, 2048, 2600, 5000, 100000):
         assert lib.q3_paged_attention_prompt_splits(700, 2 * group, 2, keys) in (1, 2, 4)
     assert lib.q3_paged_attention_plan(700, 3, 34, 2, 1, 1, 0, 300, 1, 300, 300) == 0      # 17 heads a group: not the fast path's
+
+
+def test_capped_scores_without_a_gate_carry_none():
+    assert not hasattr(library("attention_capped"), "q3_set_gate") and hasattr(library("attention_capped_gated"), "q3_set_gate")
