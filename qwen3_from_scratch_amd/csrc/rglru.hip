@@ -5,7 +5,7 @@
 // upper, middle and lower eight bits of its significand: three v_mfma_f32_16x16x32_bf16 of 16 cycles for 32 inputs, where
 // v_mfma_f32_16x16x4_f32 takes eight of 32, exact products and float32 sums. (Bits below 2^-133 are left out.)
 //
-// 2,048 rows of 8 parts of 256, microseconds: gates 54, segments 18, their carries 11 and results 30 as kernels of recurrent.hip / 37 and 16 here (the second
+// 2,048 rows of 8 parts of 256, microseconds: gates 54, segments 18, their carries 4 and results 30 as kernels of recurrent.hip / 37 and 16 here (the second
 // moves 58 MB).
 #include "common.h"
 
@@ -13,6 +13,10 @@
 
 #define Q3_TILE 64         // rows whose gates a block forms
 #define Q3_SEGMENT 32      // rows that a thread walks
+// Rows of a longest sequence from which a third kernel hands the segments' states on: joined segment by segment, each behind the walk over all before it, and
+// so, microseconds for one prompt of 8 parts of 256: 2,048 rows 50.3 / 53.5, 4,096 92.5 / 93.5, 8,192 199.9 / 178.4, 32,768 1,031 / 812 (1,359 by the
+// kernels of recurrent.hip).
+#define Q3_CARRIED_FROM 4096
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
@@ -22,21 +26,45 @@ union Frag {
 };
 
 __device__ inline float sigmoid_value(float z) { return 1.f / (1.f + expf(-z)); }
-__device__ inline int segments_before(const int* __restrict__ cu, int b) {
+__device__ inline int tiles_before(const int* __restrict__ cu, int b) {
   int n = 0;
-  for (int i = 0; i < b; ++i) n += (cu[i + 1] - cu[i] + Q3_SEGMENT - 1) / Q3_SEGMENT;
+  for (int i = 0; i < b; ++i) n += (cu[i + 1] - cu[i] + Q3_TILE - 1) / Q3_TILE;
   return n;
+}
+// The sequence whose tile of 64 rows is number `n` of the step's, counted sequence by sequence, and in `n` its number there; -1 behind the last. Whole
+// wavefronts call it. (A grid over sequences and the longest one's tiles is mostly blocks that find no rows, each of which has to wait for
+// a compute unit's shared memory first: 2,048 rows beside 40 single ones of 8 parts of 256 894 us so, 90 with the tiles that there are.)
+__device__ inline int sequence_of_tile(int& n, const int* __restrict__ cu, int B) {
+  if (B == 1) return n * Q3_TILE < cu[1] - cu[0] ? 0 : -1;
+  const int lane = threadIdx.x & 63;
+  for (int first = 0; first < B; first += 64) {
+    const int b = first + lane, rows = b < B ? cu[b + 1] - cu[b] : 0, tiles = (rows + Q3_TILE - 1) / Q3_TILE;
+    int upto = tiles;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int below = __shfl_up(upto, off, 64);
+      if (lane >= off) upto += below;
+    }
+    const unsigned long long past = __ballot(upto > n);
+    if (past) {
+      const int at = __ffsll((long long)past) - 1;
+      n = __builtin_amdgcn_readfirstlane(n - __shfl(upto - tiles, at, 64));
+      return __builtin_amdgcn_readfirstlane(first + at);
+    }
+    n -= __shfl(upto, 63, 64);
+  }
+  return -1;
 }
 __device__ inline unsigned upper_halves(float a, float b) {
   return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
 }
 
-// grid (tiles of 64 rows of the longest sequence, blocks, B), 64 KS threads: a tile's rows and one part of 32 KS numbers. u's parts lie in
+// grid (tiles of 64 rows of all sequences, blocks), 64 KS threads: a tile's rows and one part of 32 KS numbers. u's parts lie in
 // shared memory in the lanes' order of the matrix instructions; a wavefront forms two runs of 16 outputs for both gates, all 64
 // rows, and weights come straight from memory in that order (`weights`: gate, block, 16 outputs, 32 inputs, lane, eight numbers). Then
 // log a = -rate r and sqrt(1 - a^2) i take the parts' place, and a thread walks a channel through 32 rows, a segment, from S = 0: `local`
 // (2, T, width) receives the state so far and the product of the a so far, by which the state before the segment joins; the segment's
-// last go to `ends` (2, segment, width), and the states at the sequences' starts to `begins` (B, width).
+// last go to `ends` (2, segment, width; two segments a tile), and the states at the sequences' starts to `begins` (B, width).
 //
 // Bound by the vector unit: a number's two sigmoids, exponentials and square root are some 200 instructions. With four wavefronts, one a SIMD, and
 // 64 rows a thread 84 us, so 37.
@@ -46,13 +74,13 @@ __global__ void __launch_bounds__(64 * KS) rglru_gates_kernel(const float* __res
                                                               const float* __restrict__ state, long state_stride,
                                                               const int* __restrict__ slots, const int* __restrict__ cu,
                                                               float* __restrict__ local, float* __restrict__ ends, long all_segments,
-                                                              float* __restrict__ begins, int T, int width) {
+                                                              float* __restrict__ begins, int T, int B, int width) {
   constexpr int BW = 32 * KS, OUTS = 2, ROW = BW + 4;      // runs of 16 outputs a wavefront; floats of a row of results
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  const int b = blockIdx.z, part = blockIdx.y, blocks = width / BW;
-  const int start = cu[b], left = cu[b + 1] - start - (int)blockIdx.x * Q3_TILE;
-  if (left <= 0) return;
-  const int row0 = start + blockIdx.x * Q3_TILE, len = min(left, Q3_TILE);
+  int tile = blockIdx.x;
+  const int b = sequence_of_tile(tile, cu, B), part = blockIdx.y, blocks = width / BW;
+  if (b < 0) return;
+  const int start = cu[b], row0 = start + tile * Q3_TILE, len = min(cu[b + 1] - row0, Q3_TILE);
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6, col = lane & 15, grp = lane >> 4;
   const float* rows = u + (size_t)row0 * width + part * BW;
   // u: four lanes 64 bytes of a row, sixteen rows a load; piece k of row r goes to lane r + 16 (k / 8) of its operand
@@ -147,7 +175,7 @@ __global__ void __launch_bounds__(64 * KS) rglru_gates_kernel(const float* __res
 #pragma unroll
   for (int r = 0; r < Q3_SEGMENT; ++r) in[r] = rows[(size_t)(r0 + r < len ? r0 + r : 0) * width + c];
   __syncthreads();
-  if (blockIdx.x == 0 && t < BW) begins[(size_t)b * width + channel] = state[(size_t)slots[b] * state_stride + channel];
+  if (tile == 0 && t < BW) begins[(size_t)b * width + channel] = state[(size_t)slots[b] * state_stride + channel];
   if (r0 >= len) return;
   float S = 0.f, sum = 0.f, decay = 1.f;
   float* of_states = local + (size_t)(row0 + r0) * width + channel;
@@ -163,22 +191,53 @@ __global__ void __launch_bounds__(64 * KS) rglru_gates_kernel(const float* __res
       of_decays[(size_t)r * width] = decay;
     }
   }
-  const size_t end = (size_t)(segments_before(cu, b) + 2 * blockIdx.x + t / BW) * width + channel;
+  const size_t end = (size_t)(2 * blockIdx.x + t / BW) * width + channel;
   ends[end] = S;
   ends[(size_t)all_segments * width + end] = decay;
 }
 
-// grid (segments of the longest sequence, width / 256, B), 256 threads, a channel each: the state before the segment from the sequence's
-// start and the ends of the segments before it (all asked for ahead of their chain), then S_t = state so far + decay so far x that state,
-// times gelu_tanh(y + y_bias). The last segment's block writes the state, which nobody reads here.
-template <typename TO>
+// The states before a sequence's segments, one behind the other, in the place of the segments' last ones: grid (width / 64, B), 64 threads, a
+// channel each, 32 segments' numbers asked for at a time.
+__global__ void __launch_bounds__(64) rglru_carry_kernel(float* __restrict__ ends, long all_segments, const float* __restrict__ begins,
+                                                         const int* __restrict__ cu, int width) {
+  const int c = blockIdx.x * 64 + threadIdx.x, b = blockIdx.y;
+  const int segments = (cu[b + 1] - cu[b] + Q3_SEGMENT - 1) / Q3_SEGMENT;
+  if (c >= width || segments <= 0) return;
+  float* at = ends + (size_t)2 * tiles_before(cu, b) * width + c;
+  const float* decays = at + (size_t)all_segments * width;
+  float before = begins[(size_t)b * width + c];
+  for (int s0 = 0; s0 < segments; s0 += 32) {
+    float S[32], by[32];
+#pragma unroll
+    for (int s = 0; s < 32; ++s) {
+      const size_t from = (size_t)min(s0 + s, segments - 1) * width;
+      S[s] = at[from];
+      by[s] = decays[from];
+    }
+#pragma unroll
+    for (int s = 0; s < 32; ++s) {
+      if (s0 + s < segments) {
+        at[(size_t)(s0 + s) * width] = before;
+        before = by[s] * before + S[s];
+      }
+    }
+  }
+}
+
+// grid (segments of all sequences, width / 256), 256 threads, a channel each: the state before the segment, then S_t = state so far + decay so far
+// x that state, times gelu_tanh(y + y_bias). That state: from rglru_carry_kernel (CARRIED), or from the sequence's start and the ends of the segments
+// before it (all asked for ahead of their chain), which saves a launch but reads them all in every segment. The last segment's block writes the
+// state, which nobody reads here.
+template <typename TO, bool CARRIED>
 __global__ void __launch_bounds__(256) rglru_join_kernel(const float* __restrict__ local, const float* __restrict__ ends, long all_segments,
                                                          const float* __restrict__ begins, const float* __restrict__ y, long y_stride,
                                                          const float* __restrict__ y_bias, float* __restrict__ state, long state_stride,
                                                          const int* __restrict__ slots, const int* __restrict__ cu,
-                                                         TO* __restrict__ out, int T, int width) {
+                                                         TO* __restrict__ out, int T, int B, int width) {
   const int c = blockIdx.y * 256 + threadIdx.x;
-  const int b = blockIdx.z, segment = blockIdx.x;
+  int tile = blockIdx.x >> 1;
+  const int b = sequence_of_tile(tile, cu, B), segment = 2 * tile + (blockIdx.x & 1);
+  if (b < 0) return;
   const int start = cu[b], left = cu[b + 1] - start - segment * Q3_SEGMENT;
   if (c >= width || left <= 0) return;
   const int row0 = start + segment * Q3_SEGMENT, len = min(left, Q3_SEGMENT);
@@ -196,9 +255,9 @@ __global__ void __launch_bounds__(256) rglru_join_kernel(const float* __restrict
     }
   };
   load(0);
-  float before = begins[(size_t)b * width + c];
-  const float* of_segment = ends + (size_t)segments_before(cu, b) * width + c;
-  for (int s0 = 0; s0 < segment; s0 += 8) {
+  const float* of_segment = ends + (size_t)((int)blockIdx.x - segment) * width + c;
+  float before = CARRIED ? of_segment[(size_t)segment * width] : begins[(size_t)b * width + c];
+  for (int s0 = 0; s0 < (CARRIED ? 0 : segment); s0 += 8) {
     float S[8], by[8];
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
@@ -232,7 +291,18 @@ extern "C" int q3_rglru_rows_take(int width, int blocks) {
   const int bw = width / blocks;
   return bw == 32 || bw == 64 || bw == 128 || bw == 256;
 }
-extern "C" long q3_rglru_rows_workspace(int T, int B, int width) { return 2L * T * width + 2L * (T / Q3_SEGMENT + B) * width + (long)B * width; }      // floats
+static long tiles_most(int T, int B) { return T / Q3_TILE + (B < T ? B : T); }
+// Whether they are the faster way for T rows in B sequences: a tile costs the same whether it has 64 rows or one, where block_gates and rglru_scan pay by
+// the row. One round of blocks, as many as the compute units' shared memory holds at once, always; for each further one 400 rows. Microseconds, those
+// kernels / these, 8 parts of 256: 65 rows beside 23 single ones (24 tiles, one round) 51.7 / 37.2, beside 40 (two) 53.1 / 57.7; 512 beside 40 67.1 / 60.7,
+// beside 64 (three) 72.7 / 81.1; 1,024 beside 64 (three) 109.8 / 83.7; 2,048 beside 40 132.5 / 89.9; 16 parts of 256: 512 beside 23 (two) 79.6 / 71.4, beside
+// 40 (four) 81.3 / 98.4; 32 parts of 64: 512 beside 40 (two) 57.2 / 56.0.
+extern "C" int q3_rglru_rows_pay(int T, int B, int width, int blocks) {
+  if (T <= 0 || B <= 0 || !q3_rglru_rows_take(width, blocks)) return 0;
+  const long at_once = 256l * (256 / (width / blocks)), rounds = (tiles_most(T, B) * blocks + at_once - 1) / at_once;
+  return T >= 400 * (rounds - 1);
+}
+extern "C" long q3_rglru_rows_workspace(int T, int B, int width) { return 2L * T * width + 4L * tiles_most(T, B) * width + (long)B * width; }      // floats
 
 // u (T, width) at sixteen bytes; weights as rglru_gates_kernel reads them, biases (2, width).
 extern "C" int q3_rglru_rows(const float* u, const void* weights, const float* bias, const float* rate, const float* y, long y_stride,
@@ -240,8 +310,8 @@ extern "C" int q3_rglru_rows(const float* u, const void* weights, const float* b
                              float* workspace, int T, int B, int max_q_len, int width, int blocks, int out_dtype, hipStream_t stream) {
   if (T <= 0 || B <= 0 || B > 65535 || max_q_len <= 0 || !q3_rglru_rows_take(width, blocks)) return Q3_ERR_BAD_ARGUMENT;
   if (((size_t)u | (size_t)weights) & 15) return Q3_ERR_BAD_ARGUMENT;
-  const int bw = width / blocks, segments = (max_q_len + Q3_SEGMENT - 1) / Q3_SEGMENT, tiles = (max_q_len + Q3_TILE - 1) / Q3_TILE;
-  const long all_segments = T / Q3_SEGMENT + B;
+  const int bw = width / blocks, tiles = (int)tiles_most(T, B);
+  const long all_segments = 2L * tiles;
   float* local = workspace;
   float* ends = workspace + 2 * (size_t)T * width;
   float* begins = ends + 2 * (size_t)all_segments * width;
@@ -256,10 +326,14 @@ extern "C" int q3_rglru_rows(const float* u, const void* weights, const float* b
     if (e != hipSuccess) return (int)e;
     done = true;
   }
-  hipLaunchKernelGGL(gates, dim3(tiles, blocks, B), dim3(2 * bw), smem, stream, u, (const uint4*)weights, bias, rate, state, state_stride,
-                     slots, cu, local, ends, all_segments, begins, T, width);
+  hipLaunchKernelGGL(gates, dim3(tiles, blocks), dim3(2 * bw), smem, stream, u, (const uint4*)weights, bias, rate, state, state_stride,
+                     slots, cu, local, ends, all_segments, begins, T, B, width);
+  const bool carried = max_q_len > Q3_CARRIED_FROM;
+  if (carried)
+    hipLaunchKernelGGL(rglru_carry_kernel, dim3((width + 63) / 64, B), dim3(64), 0, stream, ends, all_segments, begins, cu, width);
   Q3_DISPATCH_DTYPE(out_dtype, TO,
-                    hipLaunchKernelGGL(rglru_join_kernel<TO>, dim3(segments, (width + 255) / 256, B), dim3(256), 0, stream, local, ends,
-                                       all_segments, begins, y, y_stride, y_bias, state, state_stride, slots, cu, (TO*)out, T, width));
+                    hipLaunchKernelGGL((carried ? rglru_join_kernel<TO, true> : rglru_join_kernel<TO, false>), dim3(2 * tiles, (width + 255) / 256),
+                                       dim3(256), 0, stream, local, ends, all_segments, begins, y, y_stride, y_bias, state, state_stride, slots,
+                                       cu, (TO*)out, T, B, width));
   return q3_launch_status();
 }

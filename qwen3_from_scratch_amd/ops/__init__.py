@@ -1153,9 +1153,11 @@ def narrow_gates(weights):
     return copy.view(g, blocks, bw // 32, 4, 8, bw // 16, 16).permute(0, 1, 5, 2, 3, 6, 4).contiguous()
 
 
-def rglru_rows_take(u, narrow, max_q_len):
-    """Whether `rglru_rows` takes a step: sequences of more than 64 rows, and weights that `narrow_gates` took."""
-    return narrow is not None and max_q_len > 64 and u.data_ptr() % 16 == 0
+def rglru_rows_take(u, narrow, max_q_len, sequences=1):
+    """Whether `rglru_rows` takes a step: sequences of more than 64 rows, not so many short ones beside them that the kernels one by
+    one are the faster way, and weights that `narrow_gates` took."""
+    return narrow is not None and max_q_len > 64 and u.data_ptr() % 16 == 0 and bool(
+        library("rglru").q3_rglru_rows_pay(u.shape[0], sequences, u.shape[1], narrow.shape[1]))
 
 
 def rglru_rows(u, narrow, biases, rate, y, y_bias, state, slots, cu_seqlens_q, out_dtype, max_q_len):

@@ -81,7 +81,7 @@ class RecurrentUnit(Part):
             return self.w_out.forward(ops.rglru_token(
                 u, self.gate_weights, self.gate_biases, self.decay_rate, both[:, :w], self.bias_y, cache.state[:, tail:],
                 batch.state_slots, batch.cu_seqlens_q, batch.seq_index, self.precision.act))
-        if ops.rglru_rows_take(u, self.narrow_gates, batch.max_q_len):
+        if ops.rglru_rows_take(u, self.narrow_gates, batch.max_q_len, batch.state_slots.shape[0]):
             return self.w_out.forward(ops.rglru_rows(
                 u, self.narrow_gates, self.gate_biases, self.decay_rate, both[:, :w], self.bias_y, cache.state[:, tail:],
                 batch.state_slots, batch.cu_seqlens_q, self.precision.act, batch.max_q_len))
