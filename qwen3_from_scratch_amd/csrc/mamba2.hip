@@ -455,6 +455,16 @@ extern "C" int q3_mamba2_walk_takes(int H, int P, int N, int G) {
   return P > 0 && P % 16 == 0 && (N == 32 || N == 64 || N == 128 || N == 256) && G > 0 && H > 0 && H % G == 0 && 2 * G + (H + 15) / 16 <= 65535 &&
          (long)H * P <= (1l << 24) && (long)H * ((P + 63) / 64) <= 65535;
 }
+// Whether they are the faster way: the walk is one chain of 0.65 to 0.95 us a chunk of the longest sequence, however few columns there are beside it,
+// where the float32 kernels take all chunks at once and pay by what they move, and by the sequence. Chunks up to a number that their fewer launches and
+// passes buy, more the more rows, heads and sequences there are. One prompt, microseconds, those kernels / these: a head of 64 columns, N 128, 2,048 rows
+// 37.4 / 34.6, 4,096 48.8 / 52.9; 8 heads 8,192 100.8 / 107.2, N 64 1,024 29.2 / 27.8, 2,048 36.7 / 40.1, N 256 4,096 84.9 / 80.1; 16 heads 8,192 141.9 / 119.0;
+// 24 heads, N 64 8,192 144 / 135 (N 32 137 / 161); 64 heads 2,048 117 / 62, 8,192 479 / 263; four columns of 32, N 32, 512 24.0 / 23.5, 8,192 69.6 / 137, but
+// 2,048 beside 16 single rows 76 / 60. Of 830 sizes none chosen so takes 4 percent longer than by the float32 kernels (127 of the walk's do).
+extern "C" int q3_mamba2_walk_pays(int T, int B, int max_q_len, int H, int P, int N) {
+  const long chunks = (max_q_len + Q3_CHUNK - 1l) / Q3_CHUNK, bought = N <= 32 ? 6 : N <= 64 ? 12 : 44, each = N <= 32 ? 8 : N <= 64 ? 12 : 14;
+  return 2 * chunks <= 2 * bought + 3 * (B - 1l) + 2 * each * ((long)T * H * P / 1000) / 1000;
+}
 extern "C" long q3_mamba2_walk_workspace(int T, int B, int H, int P, int N, int G) {      // in floats
   const long chunks = T / Q3_CHUNK + B;
   return chunks * ((long)G * Q3_CHUNK * Q3_CHUNK + 5L * H * Q3_CHUNK + (long)H * N * P + (long)G * N * Q3_CHUNK);

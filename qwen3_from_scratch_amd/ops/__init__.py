@@ -1017,7 +1017,8 @@ def mamba2_scan(xbc, dt, dt_bias, a_log, d_skip, state, slots, cu_seqlens_q, hea
     S <- exp(-exp(a_log) step) S + step B x^T, y = S^T C + d_skip x. state float32 (slots,
     heads n_state vdim) laid out (head, n, column), continued and brought up to date. Returns y
     float32 (T, heads vdim). `max_q_len`: the rows of the step's longest sequence; from `CHUNKED_FROM` on
-    the sequences are worked through in chunks of 64 rows, all chunks at once, instead of row by row."""
+    the sequences are worked through in chunks of 64 rows instead of row by row: bfloat16 rows by a walk over the chunks' states
+    where that pays, else all chunks at once."""
     _dev(xbc, dt_bias, a_log, d_skip)
     T = xbc.shape[0]
     _need(xbc.dim() == 2 and xbc.dtype in _DT and xbc.shape[1] == heads * vdim + 2 * groups * n_state,
@@ -1031,7 +1032,7 @@ def mamba2_scan(xbc, dt, dt_bias, a_log, d_skip, state, slots, cu_seqlens_q, hea
     y = torch.empty((T, heads * vdim), dtype=torch.float32, device=xbc.device)
     if T and max_q_len >= CHUNKED_FROM and xbc.dtype == torch.bfloat16 and xbc.data_ptr() % 16 == 0:
         lib = library("mamba2")
-        if lib.q3_mamba2_walk_takes(heads, vdim, n_state, groups):
+        if lib.q3_mamba2_walk_takes(heads, vdim, n_state, groups) and lib.q3_mamba2_walk_pays(T, B, int(max_q_len), heads, vdim, n_state):
             lib.q3_mamba2_walk_workspace.restype = ctypes.c_long
             work = torch.empty(lib.q3_mamba2_walk_workspace(T, B, heads, vdim, n_state, groups), dtype=torch.float32, device=xbc.device)
             _check(lib.q3_mamba2_walk(

@@ -56,7 +56,8 @@ def test_many_rows(H, P, N, G, lengths):
 
 
 def test_rows_that_are_no_numbers():
-    """An infinite x stays one in its own column and head, and the state that it leaves; other columns and sequences stay as they are."""
+    """An infinite x stays one in its own column and head, and the state that it leaves; other columns and sequences stay as they are, and so
+    do the chunks before it. (In its own column the rows before it, in its chunk, may be no numbers: what they multiply it with is zero.)"""
     ops = _ops()
     H, P, N, G, lengths = 2, 32, 64, 1, [70, 12]
     xbc, dt, dt_bias, a_log, skip, state, slots, cu = _inputs(H, P, N, G, lengths, 90)
