@@ -1075,12 +1075,14 @@ def gated_rmsnorm(y, gate, weight, groups, eps, out_dtype):
     return out
 
 
-def mamba2_token_takes(proj, heads, vdim, n_state, groups, norm_groups, conv_weight, rows, sequences, max_q_len):
-    """Whether `mamba2_token` takes a step: single tokens, one a sequence, four taps, parts of the norm that fit a block."""
+def mamba2_token_takes(proj, heads, vdim, n_state, groups, norm_groups, conv_weight, rows, sequences, max_q_len, norm_weight=None):
+    """Whether `mamba2_token` takes a step: single tokens, one a sequence, four taps, parts of the norm that fit a block, and rows and
+    weights that begin where they are read sixteen bytes at a time (`norm_weight`, if given, among them)."""
     inner = heads * vdim
     return (proj.is_cuda and max_q_len == 1 and rows == sequences and rows > 0 and conv_weight.shape[1] == 4 and n_state <= 256
             and conv_weight.data_ptr() % 16 == 0 and (inner // norm_groups) % 4 == 0 and inner // norm_groups <= 4096
-            and proj.stride(1) == 1 and proj.stride(0) % 4 == 0 and proj.data_ptr() % 16 == 0)
+            and proj.stride(1) == 1 and proj.stride(0) % 4 == 0 and proj.data_ptr() % 16 == 0
+            and (norm_weight is None or norm_weight.data_ptr() % 16 == 0))
 
 
 def mamba2_token(proj, conv_weight, conv_bias, dt_bias, a_log, d_skip, norm_weight, norm_groups, eps, state, slots, cu_seqlens_q,
@@ -1100,6 +1102,9 @@ def mamba2_token(proj, conv_weight, conv_bias, dt_bias, a_log, d_skip, norm_weig
     _f32(norm_weight, (inner,), "norm_weight")
     B = _sequences(slots, cu_seqlens_q, state, 3 * channels + heads * n_state * vdim, "mamba2_token")
     _need(B == T and seq_index.dtype == torch.int32 and seq_index.shape == (T,), "one token a sequence, seq_index int32 (T,)")
+    # (before the first of the two kernels moves the state)
+    _need(mamba2_token_takes(proj, heads, vdim, n_state, groups, norm_groups, conv_weight, T, B, 1, norm_weight),
+          "sizes, rows and weights that mamba2_token_takes")
     xbc, dt, held = proj[:, inner:inner + channels], proj[:, inner + channels:], state[:, 3 * channels:]
     y = torch.empty((T, inner), dtype=torch.float32, device=proj.device)
     out = torch.empty((T, inner), dtype=proj.dtype, device=proj.device)

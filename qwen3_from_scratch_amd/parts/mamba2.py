@@ -68,7 +68,7 @@ class Mamba2(Part):
         inner, tail = self.inner, self._tail()
         proj = self.w_in.forward(x)
         if ops.mamba2_token_takes(proj, self.heads, self.vdim, self.state, self.groups, self.norm_groups, self.conv, proj.shape[0],
-                                  batch.state_slots.shape[0], batch.max_q_len):
+                                  batch.state_slots.shape[0], batch.max_q_len, self.norm):
             return self.w_out.forward(ops.mamba2_token(
                 proj, self.conv, self.conv_bias, self.dt_bias, self.a_log, self.skip, self.norm, self.norm_groups, self.eps,
                 cache.state, batch.state_slots, batch.cu_seqlens_q, batch.seq_index, self.heads, self.vdim, self.state, self.groups))
