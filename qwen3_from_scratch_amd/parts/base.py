@@ -200,7 +200,7 @@ class HyperAddend:
     `write` (streams,), both float32 (a multiplier of the residual is part of `write`). A norm that
     takes it as `delta` does this in float32 in the kernel that also reads the streams for the
     next sublayer. Where the streams are kept as the sums that they are, y may come as several results, of which
-    `scales` says by how much each counts."""
+    `scales` says by how much each counts, and is read again by every later norm of the pass: a part does not write over what it returned."""
 
     values: object
     mix: torch.Tensor

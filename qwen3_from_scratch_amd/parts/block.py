@@ -189,12 +189,16 @@ class HyperConnectionBlock(Part):
 
     def sublayer_scales(self):
         """Per sublayer the scales of the results that it gives where the streams are kept as the sums that they are."""
-        return [(q, getattr(self.mixer, "scales", (1.0,)) if q == 1 else (1.0,)) for q in self._sublayers()]
+        return [(q, self.mixer.scales if q == 1 and self._two_sided() else (1.0,)) for q in self._sublayers()]
+
+    def _two_sided(self):
+        """Whether the mixer gives its sides' results apart (`ParallelMixers.forward_sides`), each with one of its `scales`."""
+        return hasattr(self.mixer, "forward_sides")
 
     def forward(self, x, pending, batch, cache, next_norm=None):
         read, write, mix = self.tables[1]
         h = self.mixer_norm.forward(x, delta=pending, read=read)
-        if isinstance(x, torch.Tensor) or not hasattr(self.mixer, "scales"):
+        if isinstance(x, torch.Tensor) or not self._two_sided():
             pending = HyperAddend(self.mixer.forward(h, batch, cache), mix, write)
         else:
             pending = HyperAddend(self.mixer.forward_sides(h, batch, cache), mix, write, self.mixer.scales)
