@@ -225,15 +225,16 @@ __global__ void __launch_bounds__(1024) hyper_norm_row_kernel(float* __restrict_
 }
 
 // The streams as what they are sums of: every stream is a weighted sum of the embedding's rows and of the sublayers' results so
-// far, with weights that the model's tables fix, and so is what a sublayer or the last norm reads of them. While these sources
-// take less memory than the streams (see HyperConnectionBlock.plan) nothing is kept but them:
+// far, with weights that the model's tables fix, and so is what a sublayer or the last norm reads of them. While the results
+// take no more memory than the streams (models/stream_sources.py, `results_most`) nothing is kept but these sources:
 //   u = c[0] float(table[ids[t]]) + sum_j c[1 + j] values[j][t],   out = the layer norm of u as above.
 // SOURCES of them, four columns a thread and the whole row in a block, everything asked for at once. An id outside the table
 // counts as a row of zeros.
 //
 // Bound by memory for many rows and by latency for few. 2,048 rows of 2,048, bfloat16, four streams: the update and read of the streams
-// moves 151 MB (21 to 28 us a sublayer, and 18 for the streams' beginning), this 8.4 MB a source and 8.4 out: two sources 8.7 us, four 9.8,
-// seven 12.5. 8 rows 3.7 to 4.6, where the update and read take 4.7 and the streams' beginning 5.5.
+// moves 151 MB (24 us a sublayer, and 18 for the streams' beginning), this 8.4 MB a source and 8.4 out: two sources 7.6 us, four 8.2,
+// seven 11.4, ten 14.6; the streams out of ten sources 27. In float32 26.6 and, two to six sources, 7.9 to 16.6. 8,192 rows of 1,024 in two
+// streams 27.9, six sources 19.3. 8 rows 3.4 to 3.9, where the update and read take 4.1 and the streams' beginning 5.5.
 #define Q3_SOURCES_MOST 16
 struct Sources {
   const void* at[Q3_SOURCES_MOST];      // the table, then the results
@@ -427,8 +428,6 @@ extern "C" int q3_hyper_norm(float* x, const void* delta, const float* mix, cons
                                          rows, (TA*)out, S, W, eps, write_back));
   return q3_launch_status();
 }
-
-extern "C" int q3_sources_most() { return Q3_SOURCES_MOST; }
 
 // `at` (sources) and `c` (sources) are the host's. W a multiple of four up to 4,096, sixteen-byte rows.
 template <typename TA, int SOURCES = Q3_SOURCES_MOST>

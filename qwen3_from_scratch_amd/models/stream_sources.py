@@ -1,9 +1,9 @@
 """A residual in several streams as the sums that its streams are.
 
 Every stream is a weighted sum of the embedding's rows and of the sublayers' results so far, with weights that follow from the
-layers' `in`, `out` and `mix` tables alone. While those sources take less memory than the streams, a pass keeps the sources and
+layers' `in`, `out` and `mix` tables alone. While the results take no more memory than the streams and the next result would, a pass keeps the sources and
 reads the weighted sum that a norm wants of them in one kernel (`ops.read_sources`); from the first sublayer on for which the
-streams are the smaller, it goes on with them (`ops.streams_from_sources`).
+streams are the smaller, it goes on with them (`ops.streams_from_sources`, for whose length both are there).
 """
 
 import math
@@ -56,6 +56,15 @@ class StreamSources:
         return ops.hyper_norm(self.streams, norm.weight, norm.eps, norm.precision.act, read=read, rows=rows)
 
 
+def results_most(streams, size):
+    """How many sublayers' results, of `size` bytes a number, are kept in the place of `streams` streams of float32 numbers: as many as
+    take the memory of the streams and of the result that joins them next, and no more than 20 bytes a number, since results and streams are both
+    there where one gives way to the other, beside less than what a mixer needs for itself. (By what a sublayer moves it would be twice as many; but
+    a long prompt then needs more memory than with the streams: 24 layers of a width of 1,024 in four streams over 8,192 tokens 369 MB, so 330 as
+    with them.)"""
+    return min(ops.SOURCES_MOST - 3, 4 * streams // size + 1, 20 // size)
+
+
 def stream_plan(model):
     """The plan of a loaded model on the GPU whose residual is in several streams from its embedding to its last norm, or None."""
     order, blocks = model.spec.order, [layer.block for layer in model.layers]
@@ -75,10 +84,9 @@ def stream_plan(model):
     # coefficients of every source in every stream, from the tables' numbers in double precision
     each = [[1.0] * streams]
     reads, until, at_streams = [], 0, None
-    # the streams' update and read moves them twice and a result once, a read of sources each of them once; a sublayer adds up to two
-    most = min(ops.SOURCES_MOST - 2, (2 * 4 * streams + table.element_size()) // table.element_size())
+    most = 1 + results_most(streams, table.element_size())      # (the embedding's rows stay in its table; a sublayer adds up to two)
 
-    def take(weights):
+    def take(weights, most):
         nonlocal until, at_streams
         if at_streams is not None:
             return
@@ -99,12 +107,12 @@ def stream_plan(model):
     for step in order:
         for q, scales in blocks[step.layer].sublayer_scales():
             read, write, mix = numbers[step.layer, q]
-            take(read)
+            take(read, most)
             each = [[sum(c[s] * mix[s][t] for s in range(streams)) for t in range(streams)] for c in each]
             each += [[w * scale for w in write] for scale in scales]
             if at_streams is not None:
                 break
-    take([1.0] * streams)
+    take([1.0] * streams, ops.SOURCES_MOST)      # (nothing follows that streams would serve)
     if until == 0 or not all(math.isfinite(x) and abs(x) < 2.0 ** 127 for row in reads + (at_streams or []) for x in row):
         return None
     if at_streams is not None:

@@ -925,7 +925,7 @@ def hyper_norm(x, weight, eps, out_dtype, read=None, delta=None, mix=None, write
     return out
 
 
-SOURCES_MOST = 16     # that `read_sources` takes
+SOURCES_MOST = 16     # that `read_sources` takes (Q3_SOURCES_MOST of hyper.hip, which refuses more)
 
 
 def _sources(ids, table, values):
