@@ -125,6 +125,7 @@ class _DecodeGraph:
             B, widths, self.host, [storage.spare_page(g) for g in range(len(m.groups))], storage.spare_slot,
             [grp.gives_back for grp in m.groups])
         self.graph = None
+        self.plan = None                   # of the model's streams, that the capture was made with
         self.logits = None
         self.copied = torch.cuda.Event()
 
@@ -168,7 +169,7 @@ class _DecodeGraph:
         with collector_paused():
             with torch.cuda.graph(graph, pool=runner.graph_pool):
                 self.logits = runner.model.forward(batch, runner.storage)
-        self.graph = graph
+        self.graph, self.plan = graph, getattr(runner.model, "stream_plan", None)
 
 
 class ModelRunner:
@@ -276,7 +277,11 @@ class ModelRunner:
         while bucket < longest:
             bucket *= 2
         bucket = min(bucket, self.max_request_tokens)
+        plan = getattr(self.model, "current_stream_plan", lambda: None)()
         graph = self._graphs.pop((rows, bucket), None)
+        if graph is not None and graph.plan is not plan:    # captured with other tables than the model has now
+            graph.retire(self.device)
+            graph = None
         if graph is None:
             if len(self._graphs) >= self.max_graphs:       # drop the one used longest ago, once it is idle
                 self._graphs.pop(next(iter(self._graphs))).retire(self.device)

@@ -113,7 +113,9 @@ class DecoderModel:
         return names
 
     def load(self, source):
-        """Check the source's names and shapes against the model, then load."""
+        """Check the source's names and shapes against the model, then load. Products' weights are laid out for the kernels here, in copies
+        that do not follow them if they are written to afterwards: to change them, load again. The recurrent unit's `gate_weights` and the
+        streams' `tables`, of which copies are kept too, may be changed in place: they are copied anew."""
         check_tensors(source, self.tensors(), ignorable=self.spec.ignorable_tensors)
         kept = {}
 
@@ -139,12 +141,23 @@ class DecoderModel:
         self.stream_plan = stream_plan(self)
         return self
 
+    def current_stream_plan(self):
+        """The plan by which a pass keeps a residual in several streams, or None: made anew when the streams' tables have been changed since
+        (not inside a capture, whose pass then goes on with the streams). A captured pass is good as long as this is the plan that it was captured with."""
+        plan = self.stream_plan
+        if plan is not None and not plan.current():
+            if torch.cuda.is_current_stream_capturing():
+                return None
+            plan = self.stream_plan = stream_plan(self)
+        return plan
+
     @torch.no_grad()
     def forward(self, batch, cache):
         """Logits (R, V) float32 at batch.logits_rows, from batch.token_ids and
         what `cache` holds. `cache.view(plane, writes)` gives a mixer its view."""
-        if self.stream_plan is not None and self.observer is None and batch.token_ids.shape[0]:
-            x = self.stream_plan.start(batch.token_ids, self.embedding.weight)
+        plan = self.current_stream_plan() if self.observer is None and batch.token_ids.shape[0] else None
+        if plan is not None:
+            x = plan.start(batch.token_ids, self.embedding.weight)
         else:
             x = self.position.on_embeddings(self.embedding.forward(batch.token_ids), batch)
         # a model whose passes begin with the embedding's output once more keeps a copy: the stream moves on in place

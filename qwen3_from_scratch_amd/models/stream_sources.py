@@ -11,6 +11,7 @@ import math
 import torch
 
 from .. import ops
+from ..parts.base import writes_to
 from ..parts.block import HyperConnectionBlock
 from ..parts.embedding import TokenEmbedding
 from ..parts.norm import LayerNorm
@@ -20,8 +21,16 @@ class StreamPlan:
     """Per read of a pass (one per sublayer, and the last norm's) the sources' coefficients; `until` reads are made of sources,
     and `streams` (streams, sources) are the coefficients of the streams themselves in front of the read that is not."""
 
-    def __init__(self, reads, until, streams):
+    def __init__(self, reads, until, streams, blocks=()):
         self.reads, self.until, self.streams = reads, until, streams
+        # what the coefficients were made of: per block its tables, and how often each of them had been written
+        self._made_of = [(block, dict(block.tables)) for block in blocks]
+        self._writes = [(t, writes_to(t)) for _, held in self._made_of for of_sublayer in held.values() for t in of_sublayer]
+
+    def current(self):
+        """Whether the tables are still those, and as they were, that the coefficients were made of."""
+        return (all(writes_to(t) == n for t, n in self._writes)
+                and all(block.tables.get(q) is of_sublayer for block, held in self._made_of for q, of_sublayer in held.items()))
 
     def start(self, token_ids, table):
         return StreamSources(self, token_ids, table)
@@ -117,4 +126,4 @@ def stream_plan(model):
         return None
     if at_streams is not None:
         at_streams = torch.tensor(at_streams, dtype=torch.float32, device=model.device)
-    return StreamPlan(reads, until, at_streams)
+    return StreamPlan(reads, until, at_streams, blocks)

@@ -215,6 +215,12 @@ class HyperAddend:
         return ops.scaled_sum(a, alpha, b, beta)
 
 
+def writes_to(tensor):
+    """How often `tensor` has been written in place, for who keeps something that was made of its numbers. (What torch counts: not writes
+    through `.data`, and none to tensors made in inference mode.)"""
+    return 0 if tensor.is_inference() else tensor._version
+
+
 def build_part(spec, prefix, precision, device):
     cls = lookup_part(spec.kind, spec.name)
     return cls(prefix=prefix, precision=precision, device=device, **dict(spec.params))

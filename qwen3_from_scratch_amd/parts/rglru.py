@@ -4,7 +4,7 @@ import torch
 
 from .. import ops
 from ..config.registry import register_part
-from .base import CacheNeed, Part, TensorShape
+from .base import CacheNeed, Part, TensorShape, writes_to
 from .linear import LinearWeight
 
 
@@ -34,6 +34,7 @@ class RecurrentUnit(Part):
         self.hidden_size, self.width, self.blocks, self.taps, self.rate = hidden_size, width, blocks, conv, float(rate)
         self.w_in = self.w_out = self.bias_y = self.bias_x = self.conv = self.conv_bias = None
         self.gate_weights = self.gate_biases = self.decay_rate = self.narrow_gates = None
+        self._narrow_of = (None, 0)      # the gates' weights that `narrow_gates` was made of, and how often they had been written
 
     def _tail(self):
         return (self.taps - 1) * self.width
@@ -65,11 +66,22 @@ class RecurrentUnit(Part):
         # the gates' matrices as (gate, block, in, out), so that neighbouring threads read neighbouring numbers
         gates = torch.stack((fetch(self._name("ra"), torch.float32), fetch(self._name("ri"), torch.float32)))
         self.gate_weights = gates.transpose(2, 3).contiguous()
-        self.narrow_gates = ops.narrow_gates(self.gate_weights)
+        self._narrow()
         self.gate_biases = torch.stack((fetch(self._name("ra.b"), torch.float32),
                                         fetch(self._name("ri.b"), torch.float32))).contiguous()
         lam = fetch(self._name("lam"), torch.float32).double()
         self.decay_rate = (self.rate * torch.nn.functional.softplus(lam)).float().contiguous()
+
+    def _narrow(self):
+        """The gates' weights as `ops.rglru_rows` takes them, made anew once they have been changed (in a capture, where that has no
+        place, None). Steps of single tokens read the weights themselves."""
+        weights, writes = self._narrow_of
+        if weights is not self.gate_weights or writes != writes_to(self.gate_weights):
+            if self.gate_weights.is_cuda and torch.cuda.is_current_stream_capturing():
+                return None
+            self._narrow_of = self.gate_weights, writes_to(self.gate_weights)
+            self.narrow_gates = ops.narrow_gates(self.gate_weights)
+        return self.narrow_gates
 
     def forward(self, x, batch, cache):
         w, tail = self.width, self._tail()
@@ -81,9 +93,10 @@ class RecurrentUnit(Part):
             return self.w_out.forward(ops.rglru_token(
                 u, self.gate_weights, self.gate_biases, self.decay_rate, both[:, :w], self.bias_y, cache.state[:, tail:],
                 batch.state_slots, batch.cu_seqlens_q, batch.seq_index, self.precision.act))
-        if ops.rglru_rows_take(u, self.narrow_gates, batch.max_q_len, batch.state_slots.shape[0]):
+        narrow = self._narrow() if batch.max_q_len > 64 else None
+        if ops.rglru_rows_take(u, narrow, batch.max_q_len, batch.state_slots.shape[0]):
             return self.w_out.forward(ops.rglru_rows(
-                u, self.narrow_gates, self.gate_biases, self.decay_rate, both[:, :w], self.bias_y, cache.state[:, tail:],
+                u, narrow, self.gate_biases, self.decay_rate, both[:, :w], self.bias_y, cache.state[:, tail:],
                 batch.state_slots, batch.cu_seqlens_q, self.precision.act, batch.max_q_len))
         gates = ops.block_gates(u, self.gate_weights, self.gate_biases)
         mixed = ops.rglru_scan(u, gates, self.decay_rate, both[:, :w], self.bias_y, cache.state[:, tail:],
