@@ -47,6 +47,7 @@
 #include <map>
 #include <mutex>
 #include <tuple>
+#include <set>
 #include <vector>
 
 #define Q3_ERR_LIBRARY 20000   // + the library's status
@@ -117,6 +118,7 @@ struct Device {
 std::mutex g_lock;
 std::map<int, Device> g_devices;
 std::map<Key, Choice> g_table;
+std::set<Key> g_given;      // those of its sizes that the program gave an entry for, not the package
 int g_candidates = 16;
 enum { KERNELS_BOTH = 0, KERNELS_LIBRARY = 1, KERNELS_OWN = 2 };
 int g_kernels = KERNELS_BOTH;
@@ -895,16 +897,29 @@ extern "C" int q3_gemm_tiles(const void* x, const void* w, void* out, int M, int
   return Q3_ERR_BAD_ARGUMENT;
 }
 
-// Gate and up with the activation (gemm_wide.hip): Q3_DECLINED, and nothing is done, for a size that it is not for.
+extern "C" int q3_wide_swiglu_takes(int M, int N, int K) { return wide::takes(M, N, K); }
+
+// Whether gate and up with the activation go to gemm_wide.hip: for the sizes of its rule, as long as nobody has said which kernel the plain product
+// of that size is to go to, by a table's entry of the program's own, by the tuner, running now or earlier, or by a choice of kernels.
+extern "C" int q3_wide_swiglu_serves(int M, int N, int K) {
+  if (!wide::takes(M, N, K)) return 0;
+  std::lock_guard<std::mutex> hold(g_lock);
+  if (g_kernels != KERNELS_BOTH || g_mode != MODE_RULE) return 0;
+  for (int kind : {(int)KIND_PLAIN, (int)KIND_ROUND})
+    if (g_given.count(Key(kind, rows_key(kind, M), N, K, Q3_BF16))) return 0;
+  int device = 0;
+  if (g_devices.empty() || hipGetDevice(&device) != hipSuccess) return 1;
+  auto d = g_devices.find(device);
+  if (d == g_devices.end()) return 1;
+  auto p = d->second.plans.find(std::make_tuple(M, N, K, (int)Q3_BF16));
+  return p == d->second.plans.end() || !p->second.timed;
+}
+
+// Gate and up with the activation: Q3_DECLINED, and nothing is done, where q3_wide_swiglu_serves says no or the operands lie elsewhere.
 extern "C" int q3_wide_swiglu(const void* x, const void* w, void* out, int M, int N, int K, void* stream) {
-  {
-    std::lock_guard<std::mutex> hold(g_lock);
-    if (g_kernels != KERNELS_BOTH) return Q3_DECLINED;
-  }
-  if (!x || !w || !out || !wide::takes(M, N, K) || (((size_t)x | (size_t)w) & 15) || ((size_t)out & 7)) return Q3_DECLINED;
+  if (!x || !w || !out || (((size_t)x | (size_t)w) & 15) || ((size_t)out & 7) || !q3_wide_swiglu_serves(M, N, K)) return Q3_DECLINED;
   return wide::launch(x, w, out, M, N, K, (hipStream_t)stream);
 }
-extern "C" int q3_wide_swiglu_takes(int M, int N, int K) { return wide::takes(M, N, K); }
 
 // 0: sizes get their kernels by the table and the rules (the default); 1: the tuner times the candidates of
 // every size it first meets outside a capture. Sizes already settled keep their kernel.
@@ -944,7 +959,9 @@ extern "C" int q3_matmul_set_kernels(int mode) {
 // the SwiGLU activation, 3 a product that is added into the residual stream, 4 a plain product of a size that gemm_rounds.hip takes
 // (q3_matmul_plain_kind); `rows` as q3_matmul_rows_key rounds them; `own` >= 0: the tiled kernel's tile shape with `splits` shares of
 // K, or as q3_matmul_plan and q3_matmul_fused_plan give it, from 16 on (kinds 1 to 3) gemm_groups.hip's, from 32 on (kind 4)
-// gemm_rounds.hip's; own < 0: the library's candidate number `library` (for kind 3: the caller's plain product and separate norm).
+// gemm_rounds.hip's; own < 0: the library's candidate number `library` (for kind 3: the caller's plain product and separate norm). `given`: an entry of the
+// program's own, which also keeps the size's plain product in its place where a kernel with the activation inside would serve it
+// (q3_wide_swiglu_serves); the package's own entries were measured without that kernel.
 extern "C" int q3_matmul_rows_key(int kind, int M) { return rows_key(kind, M); }
 
 // Under which kind a plain product of this size is filed, its operands at multiples of sixteen bytes.
@@ -953,7 +970,7 @@ extern "C" int q3_matmul_plain_kind(int M, int N, int K, int out_dtype) {
   return round_height(KIND_PLAIN, M, N, K, out_dtype, true) ? KIND_ROUND : KIND_PLAIN;
 }
 
-extern "C" int q3_matmul_table_add(int kind, int rows, int N, int K, int out_dtype, int library, int own, int splits) {
+extern "C" int q3_matmul_table_add(int kind, int rows, int N, int K, int out_dtype, int library, int own, int splits, int given) {
   if (kind < KIND_PLAIN || kind >= KINDS || rows < 1 || N < 1 || K < 1) return Q3_ERR_BAD_ARGUMENT;
   const bool of_groups = own >= GROUPS_FIRST && own < GROUPS_FIRST + groups::NUM_SHAPES && kind != KIND_PLAIN && kind != KIND_ROUND;
   const bool of_rounds = own >= ROUNDS_FIRST + rounds::LEAST && own <= ROUNDS_FIRST + rounds::MOST && kind == KIND_ROUND;
@@ -966,12 +983,14 @@ extern "C" int q3_matmul_table_add(int kind, int rows, int N, int K, int out_dty
   c.own = own < 0 ? LIBRARY : own;
   c.splits = splits;
   g_table[Key(kind, rows, N, K, out_dtype)] = c;
+  if (given) g_given.insert(Key(kind, rows, N, K, out_dtype));
   return 0;
 }
 
 extern "C" int q3_matmul_table_clear() {
   std::lock_guard<std::mutex> hold(g_lock);
   g_table.clear();
+  g_given.clear();
   return 0;
 }
 

@@ -161,15 +161,15 @@ def _matmul():
         _table_loaded = True
         if os.path.isfile(TABLE_FILE):
             with open(TABLE_FILE, encoding="utf-8") as fh:
-                _add_to_table(lib, json.load(fh)["entries"])
+                _add_to_table(lib, json.load(fh)["entries"], False)
     return lib
 
 
-def _add_to_table(lib, entries):
+def _add_to_table(lib, entries, given):
     for e in entries:
         out = _DT[getattr(torch, e.get("out", "bfloat16"))]
         _check(lib.q3_matmul_table_add(_KINDS[e["kind"]], int(e["rows"]), int(e["N"]), int(e["K"]), out,
-                                       int(e.get("library", 0)), int(e.get("own", -1)), int(e.get("splits", 1))),
+                                       int(e.get("library", 0)), int(e.get("own", -1)), int(e.get("splits", 1)), 1 if given else 0),
                "matmul_table")
 
 
@@ -184,11 +184,12 @@ def matmul_table(entries, clear=False):
     "rows": rounded rows (`matmul_rows_key`), "N", "K", "out": "bfloat16" | "float32",
     "library": the library's candidate number, or "own": tile shape (as `matmul_plan` and
     `matmul_fused_plan` number them) and "splits": shares of K}. Plain products are filed as `matmul_plain_kind` says.
-    Sizes without an entry follow the rules of thumb. Sizes already met keep their kernel."""
+    Sizes without an entry follow the rules of thumb. Sizes already met keep their kernel. A gate and up product whose plain product has
+    an entry here (or a kernel that the tuner found) goes by it, also where a kernel with the activation inside would serve the size."""
     lib = _matmul()                      # the package's own table first, if it is not in yet
     if clear:
         _check(lib.q3_matmul_table_clear(), "matmul_table")
-    _add_to_table(lib, entries)
+    _add_to_table(lib, entries, True)
 
 
 def matmul_rows_key(kind, M):
@@ -2331,7 +2332,8 @@ def linear_swiglu(x, weight, tiled=None, unscaled=None, kind="silu", narrow=None
     2i + 1 up's): (M, K) x (2I, K) -> (M, I); `kind` names the activation (`GATE_KINDS`). With few
     bfloat16 rows, and with as many as may come unscaled (`fused_rows_most`), the activation is the product kernel's
     epilogue (silu in every kernel, the tanh form of gelu in the few-row and the weight-streaming kernel, the exact gelu
-    nowhere); otherwise it is the product followed by `gated_act`, with the same bits. `unscaled` and `narrow`: as for
+    nowhere); otherwise it is the product followed by `gated_act`, with the same bits. 257 to 288 and 513 to 576 rows of a weight that fills the
+    chip in one round (gemm_wide.h) have silu in the epilogue too, behind sums of another order than the plain product's. `unscaled` and `narrow`: as for
     `linear` (silu is the epilogue of the products with a bfloat16 copy too)."""
     if kind not in GATE_KINDS:
         raise OperandError("kind is one of %s" % ", ".join(sorted(GATE_KINDS)))
@@ -2377,9 +2379,9 @@ def linear_swiglu(x, weight, tiled=None, unscaled=None, kind="silu", narrow=None
     if unscaled is not None:
         raise OperandError("unscaled rows need bfloat16 and few rows with a tiled weight (few_rows_limit), or 17 to "
                            "128 rows (640 of a small weight, fused_rows_most) with an inner size that is a multiple of 64")
-    if x.dtype == torch.bfloat16 and 256 < M <= 576:                  # (what gemm_wide.hip may take)
+    if x.dtype == torch.bfloat16 and 256 < M <= 576 and _matmul().q3_wide_swiglu_serves(M, N, K):      # (what gemm_wide.hip may take)
         out = torch.empty((M, N // 2), dtype=x.dtype, device=x.device)
-        status = library("matmul").q3_wide_swiglu(_ptr(x), _ptr(weight), _ptr(out), M, N, K, _stream())
+        status = _matmul().q3_wide_swiglu(_ptr(x), _ptr(weight), _ptr(out), M, N, K, _stream())
         if status != _DECLINED:
             _check(status, "linear_swiglu")
             return out
