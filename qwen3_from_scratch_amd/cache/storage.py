@@ -55,15 +55,21 @@ class CacheStorage:
         return sum(t.numel() * t.element_size() for t in tensors)
 
     def clear_fresh_slots(self):
-        """Zeros in the slots handed out since the last call, a fill for each run of neighbouring ones: an index or a zero that came
-        from the host would have the host wait for all that the device still has to do."""
+        """Zeros in the slots handed out since the last call: neighbouring ones by a fill, others by an index that goes to the device out of
+        pinned memory (from ordinary memory it, or a zero, would have the host wait for all that the device still has to do). The host's
+        time for three groups of states, one slot 15 us by a fill and 22 by an index, two apart 30 and 21, 32 apart 518 and 21."""
         fresh, self.manager.fresh_slots = sorted(set(self.manager.fresh_slots)), []
-        first = 0
-        for i, slot in enumerate(fresh):
-            if i + 1 == len(fresh) or fresh[i + 1] != slot + 1:
-                for t in self.states:
-                    t[:, fresh[first]:slot + 1].zero_()
-                first = i + 1
+        if not fresh or not self.states:
+            return
+        if fresh[-1] - fresh[0] + 1 == len(fresh):
+            for t in self.states:
+                t[:, fresh[0]:fresh[-1] + 1].zero_()
+            return
+        index = torch.tensor(fresh, dtype=torch.long)
+        if self.states[0].is_cuda:
+            index = index.pin_memory().to(self.states[0].device, non_blocking=True)
+        for t in self.states:
+            t.index_fill_(1, index, 0)
 
     def keep_states(self, slots):
         """Copies of the states in `slots` (a device tensor of slot numbers), to be put back by
