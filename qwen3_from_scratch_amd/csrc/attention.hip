@@ -1674,7 +1674,8 @@ static int prompt_key_splits(int total_tokens, int G, int Hkv, int max_kv_len) {
 //   blocks only (28 over 150 to 3,000 keys beside 512 over 512, 32 heads in fours, 128 rows 54.0, 64 74.0; beside 512 over 1,536 59 and 85).
 // - The prompts' blocks, whose chains are longer, come first, prompts first / decoding first: 23 over 150 to 3,000 beside 276 over 1,300
 //   52.1 / 57.7, 28 beside 1,400 over 1,400 61.2 / 71.8, 32 beside 512 over 1,536 60 / 87, 64 over 150 to 2,000 beside it 64 / 93. Not where many
-//   contexts are left whole and the prompts' keys are a fifth of theirs at most, so that the decoding ones are the longer chains: 40 over 150 to 3,000
+//   contexts are left whole and the prompts' keys are a fifth of theirs at most, so that the decoding ones are the longer chains (and long ones: 48 over 150 beside 20
+//   rows 12.1 / 12.6): 40 over 150 to 3,000
 //   beside 512 over 512 75.9 / 62.6, 48 82 / 74, 28 beside four prompts of 300 64.3 / 51.7. Nor where more than 512 blocks fill the chip by themselves
 //   and are parts of keys or two thirds as long: 23 beside 512 over 3,584 102 / 84, 32 106 / 102; one over 3,000 beside 15 prompts of 130 34.3 / 27.8; 40 over
 //   150 to 3,000 beside 1,400 over 1,400, 64 heads in eights, 120 / 97 (but 64 over 200 to 1,000 80 / 86).
@@ -1698,7 +1699,7 @@ static PromptPlan plan_prompts(int total_tokens, int B, int G, int Hkv, int key_
   while (blocks(plan.tokens) < enough(plan.tokens) && halved()) plan.tokens /= 2;
   const long filled = blocks(plan.tokens);
   plan.prompts_first = !(filled > 512 && (key_splits > 1 || 3L * longest <= 2L * max_kv_len)) &&
-                       !(beside_many && splits == 1 && 5L * longest <= max_kv_len);
+                       !(beside_many && splits == 1 && max_kv_len > 512 && 5L * longest <= max_kv_len);
   const long brief_blocks = (max(0, total_tokens - B) / (16 / G) + B) * (long)Hkv;   // (the most that so many tokens of so many sequences come to)
   const bool outlasts = few ? prompts == 1 && longest >= max_kv_len : (long)Hkv * pieces(max_q_len, plan.tokens) * B > SHORT_BLOCKS_MOST;
   plan.brief = window == 0 && splits == 1 && key_splits == 1 && brief_blocks <= (outlasts ? SHORT_BLOCKS_MOST : SHORT_BLOCKS);

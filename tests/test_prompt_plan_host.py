@@ -43,6 +43,7 @@ def test_prompts(heads, lengths, keys, rows, parts):
     ((32, 8), _spread(23, 150, 3000), [(276, 1300)], 64, True), ((32, 8), _spread(28, 150, 3000), [(1400, 1400)], 128, True),
     ((16, 8), _spread(28, 150, 3000), [(300, 300)] * 4, 128, False), ((32, 8), _spread(23, 150, 3000), [(512, 3584)], None, None),
     ((64, 8), _spread(40, 150, 3000), [(1400, 1400)], 128, False), ((64, 8), _spread(64, 200, 1000), [(1400, 1400)], 128, True),
+    ((16, 8), _spread(30, 150, 500), [(16, 16), (33, 33), (51, 51)], 32, True),
     # one decoding request among prompts is not as many as there are sequences
     ((32, 8), [3000], [(130, 130)] * 15, 128, False), ((32, 8), [150], [(33, 33)] * 30, 128, True), ((16, 8), [150], [(300, 300)] * 7, 128, True)])
 def test_prompts_beside_decoding_requests(heads, singles, portions, rows, first):
