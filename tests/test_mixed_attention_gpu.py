@@ -98,7 +98,7 @@ def test_few_rows_over_many_keys(Hq, Hkv, D, page, lens, cap):
 
 
 # Blocks of 32, 64 and 128 rows, whose wavefronts share the keys or do not: rows and keys at the edges of tiles and of their halves (the first row of a
-# prompt sees no key of the second), keys in parts, a window, a group that does not divide the rows; the last two beside 128 pairs of decoding ones
+# prompt sees no key of the second), keys in parts, a window, a group that does not divide the rows; the last two beside decoding ones
 @pytest.mark.parametrize("Hq,Hkv,D,page,lens,window", [
     (8, 2, 128, 16, [(200, 200), (17, 33), (130, 177), (129, 1031)], 0), (8, 2, 64, 16, [(300, 300), (95, 128)], 0),
     (12, 4, 128, 32, [(260, 260), (100, 640)], 0), (16, 2, 128, 16, [(150, 3300)], 0), (8, 2, 128, 64, [(150, 4100), (40, 40)], 0),
