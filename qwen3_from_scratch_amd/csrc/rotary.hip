@@ -349,16 +349,26 @@ static int launch_qk(void* qkv, const void* qw, const void* kw, float eps, const
   return q3_launch_status();
 }
 
+// How many pages, key heads and sequences blocks that store values page by page go over: `max_q_len` rows of every sequence.
+static int span_of(int max_q_len, int page_size) { return (max_q_len + page_size - 1) / page_size + 1; }
+// Whether values are stored so, not element by element by the lanes that prepare queries and keys: from eight rows a sequence on. float32 steps of many
+// short sequences beside a long one go element by element too: each block that finds no rows costs 0.65 ns, every 128 numbers 0.75 ns more than by
+// page. Pages / elements, microseconds, 16 + 8 + 8 heads of 128: 512 rows 6.5 / 9.6, beside eight single ones 7.6 / 10.5, beside 20 10.0 / 10.6, beside
+// 40 13.7 / 10.6; 100 beside 60 12.0 / 6.3 (6.8 by a wavefront a head); 2,048 beside 23 32.1 / 27.5; 600 in 30 sequences 8.0 / 11.1.
+static bool values_by_page(int T, int B, int max_q_len, int Hkv, int D, int page_size, bool f32) {
+  return max_q_len >= 8 && !(f32 && 128l * span_of(max_q_len, page_size) * B > (long)T * D);
+}
+
 template <typename T, typename W>
 static int launch_qk_vec(void* qkv, const void* qw, const void* kw, float eps, const float* table, int max_pos,
                          const int* positions, const int* seq_index, const int* block_table, int bt_stride,
                          int bt_rows, void* k_cache, void* v_cache, int page_size, int num_pages, int T_, int Hq,
                          int Hkv, int D, const int* cu_q, const int* kv_lens, int B, int max_q_len,
                          hipStream_t stream) {
-  const bool few = max_q_len < 8;  // values element by element by the lanes that prepare queries and keys
+  const bool few = v_cache ? !values_by_page(T_, B, max_q_len, Hkv, D, page_size, sizeof(T) == 4) : max_q_len < 8;
   const bool values_apart = v_cache != nullptr && !few;
   const int nheads = Hq + (few ? 2 : 1) * Hkv;
-  const int span_pages = values_apart ? (max_q_len + page_size - 1) / page_size + 1 : 0;
+  const int span_pages = values_apart ? span_of(max_q_len, page_size) : 0;
   const long value_blocks = values_apart ? (long)span_pages * Hkv * B : 0;
 #define Q3_QKV_LAUNCH(LPH)                                                                                    \
   do {                                                                                                        \
@@ -392,6 +402,10 @@ static int launch_qk_vec(void* qkv, const void* qw, const void* kw, float eps, c
   }
 #undef Q3_QKV_LAUNCH
   return q3_launch_status();
+}
+
+extern "C" int q3_values_by_page(int T, int B, int max_q_len, int Hkv, int D, int page_size, int act_dtype) {
+  return T > 0 && B > 0 && page_size > 0 && values_by_page(T, B, max_q_len, Hkv, D, page_size, act_dtype == Q3_F32);
 }
 
 // `cu_q`, `kv_lens`, `B`, `max_q_len` describe the step's sequences (they may be null / 0: then
