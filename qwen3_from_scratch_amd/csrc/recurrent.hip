@@ -134,13 +134,12 @@ struct Eight<float> {
   }
 };
 
-// A thread's tile is Q3_CONV_TILE rows. TAPS 4: that many, and a thread takes its channels' taps straight from memory; 0:
-// up to Q3_TAPS_MOST, through shared memory. Bound by memory, the taps' passage and the activation: 2,048 rows of 4,352 bfloat16 channels
-// and 4 taps (36 MB) 18.5 us in tiles of four rows, 18.8 of two, 21.8 of eight (fewer inputs read twice, but two wavefronts a SIMD, of which each
-// waits once and then computes; taps turned in shared memory out of neighbouring pieces 20.0); 37 with an input's wait before each next one and taps that 32 lanes
-// read from one bank of shared memory (as they still are for other numbers of taps).
-#define Q3_CONV_TILE 4
-template <typename TI, typename TO, int TAPS>
+// A thread's tile is TILE rows. TAPS 4: that many, and a thread takes its channels' taps straight from memory; 0:
+// up to Q3_TAPS_MOST, through shared memory. Bound by memory, the taps' passage and the activation. Tiles of eight rows read fewer inputs twice, tiles of
+// four are twice as many wavefronts, of which each waits once and then computes (`conv_tile`): 2,048 rows of 4,352 bfloat16 channels
+// and 4 taps with the activation (36 MB) 18.5 us in fours, 21.8 in eights (taps turned in shared memory out of neighbouring pieces 20.0); 37 with an input's
+// wait before each next one and taps that 32 lanes read from one bank of shared memory (as they still are for other numbers of taps).
+template <typename TI, typename TO, int TAPS, int TILE>
 __global__ void __launch_bounds__(64) causal_conv_wide_kernel(const TI* __restrict__ x, long x_stride, const float* __restrict__ in_bias,
                                         const float* __restrict__ w, const float* __restrict__ bias,
                                         const float* __restrict__ state, long state_stride,
@@ -151,8 +150,8 @@ __global__ void __launch_bounds__(64) causal_conv_wide_kernel(const TI* __restri
   const int taps = TAPS ? TAPS : any_taps;
   const int first = blockIdx.y * 64 * 8;
   const int c0 = first + threadIdx.x * 8 < C ? first + threadIdx.x * 8 : first;      // (a thread past the end only helps with the taps)
-  const int t0 = blockIdx.x * Q3_CONV_TILE;
-  const int t1 = t0 + Q3_CONV_TILE < T ? t0 + Q3_CONV_TILE : T;
+  const int t0 = blockIdx.x * TILE;
+  const int t1 = t0 + TILE < T ? t0 + TILE : T;
   const int seq = seq_index[t0], start = cu[seq];
   const bool one_sequence = seq == seq_index[t1 - 1];
   float tap[MOST][8];
@@ -165,10 +164,10 @@ __global__ void __launch_bounds__(64) causal_conv_wide_kernel(const TI* __restri
   }
   // the usual case, all rows of one sequence: every input the rows need is asked for at once, behind
   // no branch, rows t0 - (MOST - 1) .. t1 - 1; rows that do not exist (or precede the sequence) are read as one that does
-  Eight<TI> raw[Q3_CONV_TILE + MOST - 1];
+  Eight<TI> raw[TILE + MOST - 1];
   if (one_sequence) {
 #pragma unroll
-    for (int i = 0; i < Q3_CONV_TILE + MOST - 1; ++i) {
+    for (int i = 0; i < TILE + MOST - 1; ++i) {
       int row = t0 - (MOST - 1) + i;
       row = row < start ? start : (row < t1 ? row : t1 - 1);
       raw[i].load(x + (size_t)row * x_stride + c0);
@@ -200,9 +199,9 @@ __global__ void __launch_bounds__(64) causal_conv_wide_kernel(const TI* __restri
   }
   if (first + (int)threadIdx.x * 8 >= C) return;
   if (one_sequence) {
-    float in[Q3_CONV_TILE + MOST - 1][8];
+    float in[TILE + MOST - 1][8];
 #pragma unroll
-    for (int i = 0; i < Q3_CONV_TILE + MOST - 1; ++i) {
+    for (int i = 0; i < TILE + MOST - 1; ++i) {
       raw[i].get(in[i]);
 #pragma unroll
       for (int e = 0; e < 8; ++e) in[i][e] += add[e];
@@ -219,7 +218,7 @@ __global__ void __launch_bounds__(64) causal_conv_wide_kernel(const TI* __restri
       }
     }
 #pragma unroll
-    for (int r = 0; r < Q3_CONV_TILE; ++r) {
+    for (int r = 0; r < TILE; ++r) {
       if (t0 + r < t1) {
         float acc[8];
 #pragma unroll
@@ -1583,6 +1582,19 @@ extern "C" int q3_rglru_chunked(const float* u, const float* gates, const float*
 
 // ---- launchers ----
 
+// Rows of a tile of causal_conv_wide_kernel: four, or eight where tiles of eight are wavefronts enough, the sooner the less there is to compute for a number
+// that moves and, of other numbers of taps than four, the more taps a tile of whatever size brings into shared memory. Tiles of eight / four, microseconds,
+// 1,024 rows of 1,024 channels (256 wavefronts of eight rows), of 4,096 (1,024), 2,048 of 2,048 (1,024), 8,192 of 4,352 (9,216): float32 without an
+// activation 7.8 / 7.7, 13.0 / 14.3, 12.1 / 14.2, 63.3 / 67.0; bfloat16 to float32 7.9 / 7.7, 12.0 / 12.2, 11.6 / 12.5, 43.8 / 47.9; to bfloat16 9.2 / 8.1, 11.2 /
+// 11.0, 10.8 / 10.6, 36.1 / 38.7; with the activation float32 10.7 / 8.9, 15.8 / 15.7, 14.8 / 16.0, 72.3 / 69.1, bfloat16 12.2 / 9.4, 14.2 / 13.7, 14.0 / 13.2,
+// 51.3 / 47.7. Three taps: 2,048 of 2,048 18.0 / 21.6; eight: 2,048 of 4,352 35.4 / 48.9, 512 of 2,048 12.2 / 12.9, of 512 14.1 / 11.
+static int conv_tile(int T, int C, int taps, int act, bool f32_out) {
+  const long of_eight = (long)((T + 7) / 8) * ((C + 511) / 512);
+  const long enough = taps == 4 ? (act && !f32_out ? 1l << 62 : f32_out && !act ? 512 : 1024) : taps < 4 ? 1024 : 256;
+  return of_eight < enough ? 4 : 8;
+}
+extern "C" int q3_conv_tile(int T, int C, int taps, int act, int out_dtype) { return conv_tile(T, C, taps, act, out_dtype == Q3_F32); }
+
 extern "C" int q3_causal_conv(const void* x, long x_stride, const float* in_bias, const float* w, const float* bias,
                               float* state, long state_stride, const int* slots, const int* cu, const int* seq_index,
                               void* out, int T, int B, int C, int taps, int act, int single_rows, int in_dtype,
@@ -1599,10 +1611,11 @@ extern "C" int q3_causal_conv(const void* x, long x_stride, const float* in_bias
       (x_stride * in_size) % 16 == 0 && (C * out_size) % 16 == 0 && ((size_t)bias % 16) == 0 && ((size_t)w % 16) == 0 &&
       (!in_bias || ((size_t)in_bias % 16) == 0)) {
     const int wide_threads = 64;       // the kernel's shared memory is sized for this
-    const dim3 tiles((T + Q3_CONV_TILE - 1) / Q3_CONV_TILE, (C / 8 + wide_threads - 1) / wide_threads);
+    const int tile = conv_tile(T, C, taps, act, out_dtype == Q3_F32);
+    const dim3 tiles((T + tile - 1) / tile, (C / 8 + wide_threads - 1) / wide_threads);
     Q3_DISPATCH_DTYPE(in_dtype, TI, Q3_DISPATCH_DTYPE(out_dtype, TO, {
-                        hipLaunchKernelGGL((taps == 4 ? causal_conv_wide_kernel<TI, TO, 4>
-                                                      : causal_conv_wide_kernel<TI, TO, 0>),
+                        hipLaunchKernelGGL((taps == 4 ? (tile == 4 ? causal_conv_wide_kernel<TI, TO, 4, 4> : causal_conv_wide_kernel<TI, TO, 4, 8>)
+                                                      : (tile == 4 ? causal_conv_wide_kernel<TI, TO, 0, 4> : causal_conv_wide_kernel<TI, TO, 0, 8>)),
                                            tiles, dim3(wide_threads), 0, stream, (const TI*)x, x_stride, in_bias, w, bias,
                                            state, state_stride, slots, cu, seq_index, (TO*)out, T, C, taps, act);
                       }));
