@@ -1251,6 +1251,7 @@ __global__ void retention_prepare_kernel(const TA* __restrict__ rows, const floa
 // The same four neighbouring numbers at a time, a token's sines and cosines once for all its heads, in shared memory: heads and halves of multiples
 // of four. Bound by memory: 2,048 tokens of 8 heads of 128 with values of 256 (50 MB) 13.7 us by the kernel above, 9.7 here.
 #define Q3_QUADS_HALF_MOST 256
+#define Q3_QUADS_KEYS_LEAST 512      // keys of a row, of which the block's threads have four each: 8,192 tokens of one head of 16 62.0 by this, 59.5 by the kernel above
 template <typename TA>
 __global__ void __launch_bounds__(256) retention_prepare_quads_kernel(const TA* __restrict__ rows, const float* __restrict__ inv_freq, int half,
                                                                       const int* __restrict__ positions, float k_scale,
@@ -1315,7 +1316,9 @@ __global__ void retention_finish_kernel(const float* __restrict__ o, const TA* _
 
 // The same by a wavefront per (token, head), four neighbouring numbers a lane and turn, all of a head asked for at once: no barrier, and a
 // quarter of the blocks. Bound by memory: 2,048 tokens of 8 heads of 256 (34 MB) 18.5 us by the kernel above, 11.1 here.
-// Heads of a multiple of four, up to 1,024 numbers, rows that lie at multiples of four of them.
+// Heads of a multiple of four, up to 1,024 numbers, rows that lie at multiples of four of them; smaller heads leave most of a wavefront idle (retention of 8,192
+// tokens, 16 heads of 32 172 by this and 160 by the kernel above, 32 heads of 64 94 and 90).
+#define Q3_QUADS_VALUES_LEAST 96
 template <typename TA>
 __global__ void __launch_bounds__(256) retention_finish_quads_kernel(const float* __restrict__ o, const TA* __restrict__ rows, float eps,
                                                                      TA* __restrict__ out, long heads, int H, int dim, int vdim) {
@@ -1351,7 +1354,7 @@ __global__ void __launch_bounds__(256) retention_finish_quads_kernel(const float
 
 template <typename TA>
 static void launch_retention_finish(const float* o, const TA* rows, float eps, TA* out, int T, int H, int dim, int vdim, hipStream_t stream) {
-  if (vdim % 4 == 0 && vdim <= 1024 && H * dim % 2 == 0 && (size_t)o % 16 == 0 && (size_t)rows % (4 * sizeof(TA)) == 0 &&
+  if (vdim % 4 == 0 && vdim >= Q3_QUADS_VALUES_LEAST && vdim <= 1024 && H * dim % 2 == 0 && (size_t)o % 16 == 0 && (size_t)rows % (4 * sizeof(TA)) == 0 &&
       (size_t)out % (4 * sizeof(TA)) == 0) {
     const long heads = (long)T * H;
     hipLaunchKernelGGL(retention_finish_quads_kernel<TA>, dim3((unsigned)((heads + 3) / 4)), dim3(256), 0, stream, o, rows, eps, out, heads, H, dim, vdim);
@@ -1455,7 +1458,7 @@ extern "C" int q3_retention_chunked(const void* rows, const float* inv_freq, int
   float* vf = kf + (size_t)T * H * dim;
   float* sums = vf + (size_t)T * H * vdim;
   float* decays = sums + (size_t)(T / Q3_CHUNK + B) * H * dim * vdim;
-  const bool quads = dim % 4 == 0 && half % 4 == 0 && half <= Q3_QUADS_HALF_MOST && H * vdim % 4 == 0 && (size_t)workspace % 16 == 0 &&
+  const bool quads = H * dim >= Q3_QUADS_KEYS_LEAST && dim % 4 == 0 && half % 4 == 0 && half <= Q3_QUADS_HALF_MOST && H * vdim % 4 == 0 && (size_t)workspace % 16 == 0 &&
                      (size_t)rows % (act_dtype == Q3_F32 ? 16 : 8) == 0;
   Q3_DISPATCH_DTYPE(act_dtype, TA,
                     hipLaunchKernelGGL((quads ? retention_prepare_quads_kernel<TA> : retention_prepare_kernel<TA>), dim3(T), dim3(256), 0,
