@@ -1688,14 +1688,24 @@ extern "C" int q3_mamba2_token(const void* rows, const void* dt, long stride, co
 }
 
 // One token a sequence; weights (2, blocks, bw, bw), biases (2, width). Few tokens: see Q3_GATES_FEW.
-extern "C" int q3_rglru_token_takes(int T, int width, int blocks) {
+static bool rglru_token_fits(int T, int width, int blocks) {
   return T > 0 && blocks > 0 && width > 0 && width % blocks == 0 && width / blocks <= 1536 && (long)T * width <= Q3_GATES_FEW &&
          (long)blocks * ((width / blocks + 15) / 16) <= 65535;
+}
+
+// Not where the kernels one by one are the faster way: a block here goes through a part's inputs for both gates, one of theirs for one,
+// and where their two blocks to this one's one all have a compute unit of their own and the parts are wide, the shorter walk is more than
+// a launch. One part, 1 / 16 / 32 tokens, one kernel against two: 512 wide 6.2 / 8.1 / 8.2 against 6.5 / 8.6 / 8.8 us, 640 wide 7.7 / 9.7 /
+// 9.8 against 7.4 / 9.8 / 9.9, 1,024 wide 9.3 / 12.9 / 14.8 against 8.4 / 12.4 / 13.7 (at 33 tokens, 384 of their blocks, 15.5 against
+// 21.2), 1,536 wide 16.2 / 21.3 / 22.0 against 12.8 / 17.5 / 28.4.
+extern "C" int q3_rglru_token_takes(int T, int width, int blocks) {
+  return rglru_token_fits(T, width, blocks) &&
+         (width / blocks <= 512 || 2L * blocks * ((width / blocks + 15) / 16) * ((T + 15) / 16) > 256);
 }
 extern "C" int q3_rglru_token(const float* u, const float* w, const float* bias, const float* rate, const float* y, long y_stride,
                               const float* y_bias, float* state, long state_stride, const int* slots, const int* seq_index, void* out,
                               int T, int width, int blocks, int out_dtype, hipStream_t stream) {
-  if (!q3_rglru_token_takes(T, width, blocks)) return Q3_ERR_BAD_ARGUMENT;
+  if (!rglru_token_fits(T, width, blocks)) return Q3_ERR_BAD_ARGUMENT;
   const int bw = width / blocks, out_tiles = (bw + 15) / 16;
   Q3_DISPATCH_DTYPE(out_dtype, TO,
                     hipLaunchKernelGGL(rglru_token_kernel<TO>, dim3((T + 15) / 16, blocks * out_tiles), dim3(256), 0, stream, u, w, bias,
