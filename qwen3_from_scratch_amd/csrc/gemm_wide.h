@@ -6,6 +6,8 @@
 namespace wide {
 
 // Whether tiles of 288 x 192 cover a product with SwiGLU in one round of blocks where the library's, 256 rows high, need a row of tiles more.
+// A narrow window: 513 to 576 rows of weights of 23,180 (at 513; 20,650 at 576) to 24,576 rows, 257 to 288 rows of 44,620 (39,820 at 288) to 49,152; 299 rows, as any
+// other number, go where they went. Other heights of tile were no faster than the library at those (gemm_wide.hip).
 // Product and activation, microseconds, the library's with the activation's kernel / this: 535 rows of 24,576 x 2,048, 4,096, 5,120 and
 // 8,192 74.2 / 65.5, 127.0 / 111.9, 160.1 / 134.6 and 225.9 / 205.2, 576 of them 74.7 / 66.4 to 229.0 / 209.3; of 22,528 x 4,096 (85 percent of what 256 such
 // tiles hold) 120.8 / 108.5; 280 of 40,960 x 4,096 (81) 132.9 / 125.1. But 512 of 24,576 x 4,096 (the library's two rows of tiles) 95.9 / 110.2, 576 of 20,480 x

@@ -5,7 +5,7 @@
 // upper, middle and lower eight bits of its significand: three v_mfma_f32_16x16x32_bf16 of 16 cycles for 32 inputs, where
 // v_mfma_f32_16x16x4_f32 takes eight of 32, exact products and float32 sums. (Bits below 2^-133 are left out.)
 //
-// 2,048 rows of 8 parts of 256, microseconds: gates 54, segments 18, their carries 4 and results 30 as kernels of recurrent.hip / 37 and 16 here (the second
+// 2,048 rows of 8 parts of 256, microseconds: gates 54, segments 18, their carries 4 and results 30 as kernels of recurrent.hip / 37 and 17 here (the second
 // moves 58 MB).
 #include "common.h"
 
